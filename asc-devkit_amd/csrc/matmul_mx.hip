@@ -17,11 +17,14 @@
 // In every case lane l needs scale byte 2 j + l / 32 of its row's bytes for this K step in sub-step j; a lane holds
 // the bytes of a K step as one dword (8- and 6-bit) or two (4-bit) per row, staged through LDS, and shifts them right
 // by 8 (l / 32) where they are used, so that the byte selector of the instruction is the constant 0 or 2.
-// The element-wise kernel (one lane per output) takes every other shape; a 4-bit operand beside an 8-bit one, or e1m2
-// beside e2m1, is first widened to e4m3, which holds every fp4 value.
+// A 4-bit operand beside an 8-bit one, or e1m2 beside e2m1, is first widened to e4m3, which holds every fp4 value.
+// Few rows, and shapes whose rows or scale rows do not fit these tiles, run matmul_mx_decode.hip; what is left (rows that
+// are no whole number of 16-byte pieces, scale rows that are no whole number of dwords) the element-wise kernel (one
+// lane per output).
 #include <type_traits>
 #include <utility>
 
+#include "matmul_mx.h"
 #include "matmul_w8a8.h"
 
 namespace ascq {
@@ -47,31 +50,6 @@ __device__ __forceinline__ void mx_static_for(F&& f)
 constexpr uint32_t kMxBM = 256, kMxBN = 256, kMxBK = 128;  // BK in bytes of an operand row
 constexpr int kMxThreads = 512;
 constexpr uint32_t kMxScaleBuf = (kMxBM + kMxBN) * 16u;  // 16 scale bytes of every row of a tile's a and b
-
-struct MxParams {
-    const uint8_t* a;
-    const uint8_t* b;
-    const uint8_t* sa;
-    const uint8_t* sb;
-    const float* bias;
-    void* c;
-    uint32_t m, n, k;       // k in elements
-    uint32_t row_bytes;     // bytes of a row of a / b in the tile kernel (both operands have the same width there)
-    uint32_t sk;            // bytes of a scale row
-    uint32_t tiles_m, tiles_n;
-    int32_t a_format, b_format, out_dtype;
-};
-
-__device__ __forceinline__ void mx_store(const MxParams& p, size_t idx, float v)
-{
-    if (p.out_dtype == ASCQ_F32) {
-        static_cast<float*>(p.c)[idx] = v;
-    } else if (p.out_dtype == ASCQ_BF16) {
-        static_cast<uint16_t*>(p.c)[idx] = static_cast<uint16_t>(f32_to_bf16_bits(v));
-    } else {
-        static_cast<uint16_t*>(p.c)[idx] = static_cast<uint16_t>(f32_to_half_bits_sat(v));
-    }
-}
 
 // kFour: both operands 4-bit (e2m1); otherwise both a byte per value in memory, with the instruction's format codes
 // kCa / kCb (0 = e4m3, 1 = e5m2, 2 = e2m3 as written by mx_widen_e1m2_kernel; 4 = e2m1).
@@ -583,6 +561,31 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
 }
 
+// Few rows: whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.  Up to 64 rows it
+// always is (n = k = 8192, e2m1: 13.0 against 42.4 us at 64 rows; e4m3: 19.5 against 76.9); beyond, both times are
+// estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a meets 4-bit b) by
+// 32 columns, each round 1.15 (e2m1 pairs), 1.85 (two 8-bit operands), 2.0 (e1m2, widened in registers) or 0.95 (the
+// 32-row form) per 1024 of k.  Tiles: rounds of 256 x 256 tiles, 1.3 per K step, and the passes that widen 4-bit
+// operands, 1 per 3 MB of their codes.  Crossovers measured at n = k = 8192: about 280 rows for e2m1 and e4m3, 380 for
+// e1m2; at n = 14336, k = 4096: 90, 150 and 250; at n = 1024, k = 14336 past 512 for all.
+bool mx_decode_preferred(const MxParams& p)
+{
+    if (p.m <= 64u) {
+        return true;
+    }
+    const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
+    const bool two4 = p.a_format == ASCQ_QDST_FP4_E2M1 && p.b_format == ASCQ_QDST_FP4_E2M1;
+    const double cus = device_compute_units();
+    auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
+    const uint32_t rows = a8 && !b8 ? 32u : 64u;
+    const double per_k = two4 ? 1.15 : a8 && b8 ? 1.85 : a8 || b8 ? (rows == 32u ? 0.95 : 1.85) : 2.0;
+    const double decode = 4.0 + rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u)) * per_k * p.k / 1024.0;
+    const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
+    const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * 1.3 *
+                                           p.k / (two4 ? 256.0 : 128.0);
+    return decode < tiles;
+}
+
 int mx_validate(const ascq_mx_desc* d, const char* who)
 {
     ASCQ_REQUIRE(d != nullptr, ASCQ_ENULL, "%s: desc is NULL", who);
@@ -652,6 +655,9 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
     const bool tile = mx_tile_shape_ok(d) && aligned16(a) && aligned16(b) && (reinterpret_cast<uintptr_t>(a_scale) & 7u) == 0 &&
                       (reinterpret_cast<uintptr_t>(b_scale) & 7u) == 0 &&
                       (need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned16(workspace)));
+    if (mx_decode_supported(p) && (!tile || mx_decode_preferred(p))) {
+        return launch_mx_decode(p, st);
+    }
     if (!tile) {
         const uint32_t arb = is_fp4(d->a_format) ? d->k / 2u : d->k, brb = is_fp4(d->b_format) ? d->k / 2u : d->k;
         size_t blocks = (static_cast<size_t>(d->m) * d->n + 255u) / 256u;

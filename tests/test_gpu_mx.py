@@ -102,6 +102,27 @@ def test_mx_tile_kernel_scale_rows(m, n, k, sk, fa, fb):
     mx_check(run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, fa, fb), is8(fa, fb))
 
 
+@pytest.mark.parametrize("fa,fb", [(a, b) for a in (E4, E5, F2, F1) for b in (E4, E5, F2, F1)])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 40, 160), (16, 33, 1088), (17, 64, 640), (32, 4112, 256), (33, 100, 2304),
+                                   (64, 48, 4096), (65, 32, 1056)])
+def test_mx_few_rows(m, n, k, fa, fb):
+    """The weight-streaming kernel: every format pair, one to two blocks of rows, one and two column groups per
+    workgroup, less k than there are wavefronts, a last tile and a last batch of k that are not full, scale bytes
+    behind the last block of k that would poison the result (255 is NaN), bias; equal calls give equal bits."""
+    announce("mx few rows", m, n, k, fa, fb)
+    rng = np.random.default_rng(3 * m + n + k + fa * 16 + fb)
+    blocks = (k + 31) // 32
+    a, b, sa, sb, bv = mx_case(rng, m, n, k, fa, fb, sk=(blocks + 7) // 4 * 4, bias=True)
+    sa[:, blocks:] = 255
+    sb[:, blocks:] = 255
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sa.shape[1], a_format=fa, b_format=fb, out_dtype=abi.F32, has_bias=1)
+    orc.set_threads(16)
+    want = orc.matmul_mx(d, a, b, sa, sb, bv)
+    got = run_mx(m, n, k, a, b, sa, sb, fa, fb, bias=bv).cpu().numpy()
+    mx_check(got - bv, want - bv, mx_abs_dot(a, b, sa, sb, k, fa, fb) + np.abs(bv), is8(fa, fb))
+    assert np.array_equal(got, run_mx(m, n, k, a, b, sa, sb, fa, fb, bias=bv).cpu().numpy())
+
+
 @pytest.mark.parametrize("n", [320, 257])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float16])
 def test_mx_sixteen_bit_outputs_and_bias(out, n):
