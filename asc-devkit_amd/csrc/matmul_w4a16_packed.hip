@@ -28,6 +28,7 @@
 
 #include "ascq_common.h"
 #include "ascq_device.h"
+#include "matmul_wq_gemm.h"
 
 namespace ascq {
 namespace {
@@ -37,6 +38,9 @@ constexpr int kBuf = 2;                  // register buffers: one batch in fligh
 constexpr uint32_t kPadTiles = 16;       // tiles of padding behind the last slab of a packed matrix (a batch may read on)
 constexpr uint32_t kMaxSlabs = 8;        // slabs per workgroup
 constexpr uint32_t kMaxRows = 16;        // activation rows per launch
+// More rows than this run the tile GEMM (per-weight form) instead of passes of 16: k = 8192, n = 28672: 99 against 88 us at
+// 40 rows, 131 / 88 at 64, 1035 / 203 at 512; k = n = 4096: 35 / 40, 49 / 40 and 396 / 45 us.
+constexpr uint32_t kMaxPassRows = 48;
 constexpr uint32_t kPool = 152 * 1024;   // LDS of a workgroup: staged activations, parameters, per-wavefront sums
 constexpr uint32_t kXBytes = 72 * 1024;  // at most this much of it for the activations of one pass over k
 constexpr uint32_t kParBytes = 40 * 1024;// and this much for the (scale, offset) pairs of one pass
@@ -788,6 +792,21 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
     while ((1u << p.gs_shift) < g32) ++p.gs_shift;
     p.slabs = (d->n + kSlabCols - 1u) / kSlabCols;
     p.ktiles = d->k / kTileK;
+    // the group-sum form needs whole tiles inside one quantisation group; other group sizes keep the per-weight form
+    const bool sum_form = d->mode == ASCQ_W4A16_GROUP_SUM && p.gs_shift >= 2u;
+    if (!sum_form && d->m > kMaxPassRows) {
+        WqParams w{};
+        w.x = static_cast<const uint16_t*>(x);
+        w.w = static_cast<const uint8_t*>(w_packed);
+        w.scale = p.scale;
+        w.offset = p.offset;
+        w.y = y;
+        w.m = d->m;
+        w.n = d->n;
+        w.k = d->k;
+        w.gs_shift = p.gs_shift;
+        return launch_wq_gemm(w, true, d->has_offset != 0, st);
+    }
     const uint32_t cus = device_compute_units();
     constexpr uint32_t waves = 8u, batch = 4u;  // 16 wavefronts with batches of 4 tiles measured slower (37 against 30 us)
     for (uint32_t m0 = 0; m0 < d->m; m0 += kMaxRows) {
@@ -813,11 +832,10 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
                     default: w4a16_packed_rows_kernel<kOff, 8, kSumF><<<grid, 8 * 64, 0, st>>>(p); break;
                 }
             };
-            const bool rows_sum = d->mode == ASCQ_W4A16_GROUP_SUM && p.gs_shift >= 2u;
             if (d->has_offset) {
-                rows_sum ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+                sum_form ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
             } else {
-                rows_sum ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+                sum_form ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
             }
             continue;
         }
@@ -827,8 +845,6 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
         // slabs if the per-wavefront sums would not fit beside them.
         uint32_t spw = (p.slabs + cus - 1u) / cus;
         spw = spw < 1u ? 1u : (spw > kMaxSlabs ? kMaxSlabs : spw);
-        // the group-sum form needs whole tiles inside one quantisation group; other group sizes keep the per-weight form
-        const bool sum_form = d->mode == ASCQ_W4A16_GROUP_SUM && p.gs_shift >= 2u;
         uint32_t pt = 0, xs_wave = 0, par_wave = 0, red_bytes = 0, sum_wave = 0, par_cw = 1;
         // entries per column of a wavefront's table: the groups its tiles can touch, rounded up to an odd number
         auto par_rows = [&](uint32_t tiles) { return ((((tiles * 4u - 1u) >> p.gs_shift) + 2u) | 1u); };

@@ -16,6 +16,7 @@
 #include <type_traits>
 #include "ascq_common.h"
 #include "ascq_device.h"
+#include "matmul_wq_gemm.h"
 
 namespace ascq {
 namespace {
@@ -481,185 +482,7 @@ __global__ __launch_bounds__(kWaves * 64) void w8a16_nk_stream_kernel(SkParams p
     }
 }
 
-// ---- many activation rows: a half GEMM whose B-tile loader de-quantises.
-// Workgroup = 4 wavefronts (2 x 2) on a 128 x 128 tile, K step 64, two LDS stages of 32 KiB (two workgroups per compute
-// unit).  Both tiles sit in LDS as [row or column][64 k] halves, 128 bytes per line in 8 pieces of 16 bytes, piece c of
-// line r stored at position c ^ ((r >> 1) & 7): a 16-byte access is served 16 lanes (256 bytes, all 64 banks) at a
-// time, two lines fill one 256-byte bank row, so the sixteen neighbouring lines of such a group must put their piece
-// into eight different positions per line parity.  A thread stages 32 bytes of one column of B per K step (registers: load, de-quantise exactly as
-// the decode kernel does, four 16-byte LDS writes) and two 16-byte pieces of A; the global loads of the next K step are
-// issued before the MFMAs of the current one.  v_mfma_f32_32x32x16_f16: lane l holds row (column) l % 32 and the 8
-// consecutive k 8 (l / 32) .. + 7 of a K sub-step, i.e. one 16-byte piece of a line.
-constexpr uint32_t kGM = 128, kGN = 128, kGK = 64;
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-template <bool kHasOffset>
-__global__ __launch_bounds__(256, 2) void w8a16_nk_gemm_kernel(NkParams p, uint32_t tiles_m)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t AS[2][kGM * kGK * 2];
-    __shared__ __attribute__((aligned(16))) uint8_t BS[2][kGN * kGK * 2];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave >> 1, wn = wave & 1u;
-    // an XCD (workgroup id mod 8) takes a contiguous share of the tiles, ordered in bands of 8 row tiles: the
-    // workgroups that run side by side in it share their rows of x and their columns of B in its L2
-    const uint32_t tiles_n = (p.n + kGN - 1u) / kGN;
-    const uint32_t t = xcd_remap(blockIdx.x, tiles_m * tiles_n);
-    if (t == 0xFFFFFFFFu) {
-        return;  // whole workgroup (the launch is rounded up to a multiple of 8)
-    }
-    uint32_t tm, tn;
-    band_order(t, tiles_m, tiles_n, tm, tn);
-    const uint32_t row0 = tm * kGM, col0 = tn * kGN;
-
-    // ---- staging roles
-    // B: thread t stages bytes 32 (t & 1) .. + 31 of column col0 + t / 2 (pieces 4 (t & 1) .. + 3 of its LDS line)
-    const uint32_t bcol_l = tid >> 1, bhalf = tid & 1u;
-    uint32_t bcol = col0 + bcol_l;
-    bcol = bcol < p.n ? bcol : p.n - 1u;
-    const uint8_t* bsrc = p.w + static_cast<size_t>(bcol) * p.k + 32u * bhalf;
-    const uint32_t sb = p.scale ? p.scale[bcol] : p.scale_bits;
-    const uint32_t ob = kHasOffset ? (p.scale ? p.offset[bcol] : p.offset_bits) : 0u;
-    const f16x2_t sc2 = h2_from_bits(sb | (sb << 16)), of2 = h2_from_bits(ob | (ob << 16));
-    // A: thread t stages pieces (t & 7) of rows t / 8 and t / 8 + 32 .. (four rows, 16 bytes each)
-    const uint32_t apiece = tid & 7u, arow_l = tid >> 3;
-    const uint16_t* asrc[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t r = row0 + arow_l + 32u * j;
-        r = r < p.m ? r : p.m - 1u;
-        asrc[j] = p.x + static_cast<size_t>(r) * p.k + 8u * apiece;
-    }
-
-    // Two register sets for the raw data of the next two K steps: the loads of step s + 2 are issued while step s
-    // computes, and the data of step s + 1 is de-quantised and written to the other LDS stage in four parts, one behind
-    // the MFMAs of each K sub-step, so that the vector ALU works while the matrix pipe is busy.
-    struct Raw {
-        u32x4 b[2], a[4];
-    };
-    auto fetch = [&](Raw& raw, uint32_t step) __attribute__((always_inline)) {
-        const uint32_t k0 = step * kGK;
-        raw.b[0] = *reinterpret_cast<const u32x4*>(bsrc + k0);
-        raw.b[1] = *reinterpret_cast<const u32x4*>(bsrc + k0 + 16u);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) raw.a[j] = *reinterpret_cast<const u32x4*>(asrc[j] + k0);
-    };
-    // part q of a step's staging: piece q of the thread's half line of B, piece q of its A pieces
-    auto stage_part = [&](const Raw& raw, uint32_t st, int q) __attribute__((always_inline)) {
-        uint32_t h0, h1, h2, h3;
-        dequant4<kHasOffset>(raw.b[q >> 1][2 * (q & 1)], sc2, of2, h0, h1);
-        dequant4<kHasOffset>(raw.b[q >> 1][2 * (q & 1) + 1], sc2, of2, h2, h3);
-        const uint32_t piece = 4u * bhalf + static_cast<uint32_t>(q);
-        *reinterpret_cast<u32x4*>(&BS[st][bcol_l * 128u + ((piece ^ ((bcol_l >> 1) & 7u)) << 4)]) = u32x4{h0, h1, h2, h3};
-        const uint32_t r = arow_l + 32u * static_cast<uint32_t>(q);
-        *reinterpret_cast<u32x4*>(&AS[st][r * 128u + ((apiece ^ ((r >> 1) & 7u)) << 4)]) = raw.a[q];
-    };
-
-    f32x16_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const uint32_t lrow = lane & 31u, lk = lane >> 5;  // operand line and which 8 k of a sub-step
-    // one K step on LDS stage st; `next` (data of the following step) is staged into the other LDS stage when do_stage
-    auto step_body = [&](uint32_t st, const Raw& next, auto do_stage) __attribute__((always_inline)) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t piece = 2u * ks + lk;
-            f16x8_t af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const uint32_t r = wm * 64u + i * 32u + lrow;
-                af[i] = *reinterpret_cast<const f16x8_t*>(&AS[st][r * 128u + ((piece ^ ((r >> 1) & 7u)) << 4)]);
-                const uint32_t c = wn * 64u + i * 32u + lrow;
-                bf[i] = *reinterpret_cast<const f16x8_t*>(&BS[st][c * 128u + ((piece ^ ((c >> 1) & 7u)) << 4)]);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-            if constexpr (decltype(do_stage)::value) {  // the other stage was last read before the barrier that ended the previous step
-                stage_part(next, st ^ 1u, ks);
-            }
-        }
-    };
-
-    const uint32_t steps = p.k / kGK;
-    const uint32_t last = steps - 1u;
-    Raw r0, r1;
-    fetch(r0, 0);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) stage_part(r0, 0, q);
-    fetch(r1, 1u < last ? 1u : last);  // data of step 1 (clamped: a single-step problem re-reads step 0 and drops it)
-    __syncthreads();
-    // Steps in pairs, an odd last one behind the loop, and nothing in a pair conditional (past the end the fetches
-    // repeat the last step's and the staging fills an LDS stage nobody reads): with a second half that can be skipped
-    // the compiler sees a path on which the first half's fetch is the newest load at the loop's top and waits there
-    // for every load in every pass, which takes the fetches' two-step lead away.
-    uint32_t s = 0;
-    for (; s + 1u < steps; s += 2) {
-        // step s on stage 0: r1 holds step s + 1; fetch step s + 2 into r0
-        fetch(r0, s + 2u < last ? s + 2u : last);
-        step_body(0u, r1, std::true_type{});
-        __syncthreads();
-        fetch(r1, s + 3u < last ? s + 3u : last);
-        step_body(1u, r0, std::true_type{});
-        __syncthreads();
-    }
-    if (s < steps) {
-        step_body(0u, r1, std::false_type{});
-        __syncthreads();
-    }
-
-    // ---- register r of lane l in a 32 x 32 block: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
-    if (!p.out_f32 && p.n % 2u == 0) {
-        // half output: after one swap between neighbouring lanes the even lane holds columns (l, l + 1) of the
-        // wavefront's first block of 32 and the odd lane columns (l - 1, l) of the second: one dword store per lane,
-        // and the 32 lanes of a row write one full 128-byte line
-        const bool odd = (lane & 1u) != 0;
-        const uint32_t colw = col0 + wn * 64u;
-        const uint32_t col = odd ? colw + 32u + (lrow - 1u) : colw + lrow;  // first column of the lane's pair
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + wm * 64u + i * 32u + 8u * (r >> 2) + 4u * lk + (r & 3);
-                const uint32_t h0 = f32_to_half_bits(acc[i][0][r]), h1 = f32_to_half_bits(acc[i][1][r]);
-                const uint32_t recv = static_cast<uint32_t>(
-                    __builtin_amdgcn_mov_dpp(static_cast<int>(odd ? h0 : h1), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-                const uint32_t word = odd ? (recv | (h1 << 16)) : (h0 | (recv << 16));
-                if (row < p.m && col < p.n) {
-                    __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.y) +
-                                                                                  static_cast<size_t>(row) * p.n + col));
-                }
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t col = col0 + wn * 64u + j * 32u + lrow;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + wm * 64u + i * 32u + 8u * (r >> 2) + 4u * lk + (r & 3);
-                if (row < p.m && col < p.n) {
-                    const size_t idx = static_cast<size_t>(row) * p.n + col;
-                    if (p.out_f32) {
-                        static_cast<float*>(p.y)[idx] = acc[i][j][r];
-                    } else {
-                        static_cast<uint16_t*>(p.y)[idx] = static_cast<uint16_t>(f32_to_half_bits(acc[i][j][r]));
-                    }
-                }
-            }
-        }
-    }
-}
+constexpr uint32_t kGK = 64;  // K step of the tile GEMM (matmul_wq_gemm.hip)
 
 // int8 [k, n] -> [n, k] through 64 x 64 tiles in LDS (the tile GEMM wants k-contiguous weights).  k % 64 == 0.
 // kVec: n % 16 == 0 and src 16-byte aligned, so a thread's 16 columns of a row are one load.
@@ -794,17 +617,20 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
     p.groups = per;
     const uint32_t grid = (n_groups + per - 1u) / per;
     if (m > kDecodeRows && k % kGK == 0) {
-        // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 rows
-        p.m = m;
-        p.x = static_cast<const uint16_t*>(x);
-        p.y = y;
-        const uint32_t tiles_m = (m + kGM - 1u) / kGM, tiles_n = (n + kGN - 1u) / kGN;
-        if (has_offset) {
-            w8a16_nk_gemm_kernel<true><<<(tiles_m * tiles_n + 7u) / 8u * 8u, 256, 0, st>>>(p, tiles_m);
-        } else {
-            w8a16_nk_gemm_kernel<false><<<(tiles_m * tiles_n + 7u) / 8u * 8u, 256, 0, st>>>(p, tiles_m);
-        }
-        return launch_status("ascq_matmul_w8a16");
+        // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 or 256 rows
+        WqParams q{};
+        q.x = static_cast<const uint16_t*>(x);
+        q.w = p.w;
+        q.scale = p.scale;
+        q.offset = p.offset;
+        q.y = y;
+        q.m = m;
+        q.n = n;
+        q.k = k;
+        q.out_f32 = p.out_f32;
+        q.scale_bits = scale_bits;
+        q.offset_bits = offset_bits;
+        return launch_wq_gemm(q, false, has_offset, st);
     }
     for (uint32_t m0 = 0; m0 < m; m0 += kRows) {
         p.m = m - m0 < kRows ? m - m0 : kRows;

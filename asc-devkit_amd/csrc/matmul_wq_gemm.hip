@@ -1,0 +1,453 @@
+// Half x quantised weights with many activation rows: a half GEMM whose B-tile loader de-quantises int8 weights kept as
+// [n, k] (W8A16) or int4 weights packed by ascq_pack_weight_w4 (W4A16).
+//
+// What bounds it is the matrix pipe, and with it the power limit: every weight becomes a half once per row tile, which
+// at 256 rows costs the vector ALU about a quarter of the clocks the matrix instructions take, and the two run side by
+// side.  v_mfma_f32_16x16x32_f16 instead of the 32 x 32 x 16 form: on random operands a loop of nothing but matrix
+// instructions reaches 1880 against 1640 TFLOP/s (it moves half the sums per product, and the clock is set by the power),
+// which is 4 to 6 % of this kernel.  k = 8192, n = 28672, before (one pass over the weights per 16 rows; 128 x 128 tiles)
+// and now: int4 512 rows 1035 -> 203 us (1180 TFLOP/s), int8 2048 rows 1120 -> 847 us (1136), 512 rows 310 -> 221 us.  A workgroup is 8
+// wavefronts on a BM x BN tile, K step 64, two LDS stages.  x goes from memory to LDS without registers
+// (global_load_lds_dwordx4); the raw bytes of B take the way through registers (16 or 32 per thread and step, fetched
+// two steps ahead), are de-quantised with the operators' own roundings and written to LDS as halves, one 16-byte piece
+// behind the matrix instructions of each quarter of a step.  Both tiles lie in LDS as lines of 64 halves (128 bytes) whose
+// 16-byte pieces are XOR-swizzled by half the line number, so that 16 lanes reading a piece of 16 neighbouring lines
+// meet all 64 banks, and one piece of a line is the operand of v_mfma_f32_16x16x32_f16 as it lies.  A step's barrier
+// stands before its last quarter, whose operands are in registers by then: behind it the matrix pipe has work while
+// the next step's loads are issued and its first operands read.
+#include <type_traits>
+#include <utility>
+
+#include "ascq_common.h"
+#include "ascq_device.h"
+#include "matmul_wq_gemm.h"
+
+namespace ascq {
+namespace {
+
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef __attribute__((address_space(1))) const void* gptr_t;
+
+constexpr uint32_t kBK = 64;  // halves of a K step
+constexpr int kThreads = 512;
+
+template <class F, int... I>
+__device__ __forceinline__ void wq_for_impl(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void wq_for(F&& f)
+{
+    wq_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ f16x2 as_h2(uint32_t b) { return __builtin_bit_cast(f16x2, b); }
+__device__ __forceinline__ uint32_t as_u32(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ f16x2 both(float v) { return f16x2{static_cast<half_t>(v), static_cast<half_t>(v)}; }
+
+// two weights as exact halves -> with the operators' roundings: one for the offset, one for the scale
+template <bool kOff>
+__device__ __forceinline__ uint32_t finish(f16x2 w, f16x2 sc, f16x2 of)
+{
+    if constexpr (kOff) {
+        w = w + of;
+    }
+    return as_u32(sc * w);
+}
+
+// pair c (of 2) of 4 int8: 0x6400 | (w + 128) is the half 1152 + w
+template <bool kOff>
+__device__ __forceinline__ uint32_t pair_of_i8(uint32_t d, int c, f16x2 sc, f16x2 of)
+{
+    const uint32_t flipped = d ^ 0x80808080u;  // w + 128 as an unsigned byte
+    return finish<kOff>(as_h2(__builtin_amdgcn_perm(0x64646464u, flipped, c ? 0x04030402u : 0x04010400u)) - both(1152.0f), sc, of);
+}
+
+// pair c (of 4) of a dword of packed int4 (u = w + 8, k offsets 0 .. 7 in nibbles 0 4 1 5 2 6 3 7): 0x6400 | u is the
+// half 1024 + u, 0x5400 | 16 u the half 64 + u
+template <bool kOff>
+__device__ __forceinline__ uint32_t pair_of_i4(uint32_t q, int c, f16x2 sc, f16x2 of, const WqMasks& mk)
+{
+    const uint32_t src = c & 2 ? q >> 8 : q;
+    return c & 1 ? finish<kOff>(as_h2((src & mk.odd) | mk.exp_odd) - both(72.0f), sc, of)
+                 : finish<kOff>(as_h2((src & mk.even) | mk.exp_even) - both(1032.0f), sc, of);
+}
+
+// One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
+// wavefront owns BM / kWM rows by 64 columns.
+template <int BM, int BN, bool kInt4, bool kOff>
+__device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32_t n0, char* A0, char* A1, char* B0, char* B1)
+{
+    constexpr int kWN = BN / 64, kWM = 8 / kWN, NA = BM / 16 / kWM, NH = NA / 2, TJ = 4;
+    constexpr int kAInstr = BM * 128 / 1024 / 8;           // direct-to-LDS instructions per wavefront and step
+    constexpr int kParts = BN / 64;                        // 16-byte pieces of the B tile per thread and step
+    static_assert(NH >= 1 && NH * 32 * kWM == BM && kAInstr >= 1 && (kParts == 4 || kParts == 2), "tile shape");
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave / kWN, wn = wave % kWN;
+
+    // ---- A: lane owns LDS slot (instr * 64 + lane) of 16 bytes: line slot / 8, piece position ^ ((line / 2) % 8)
+    const uint32_t row_bytes = p.k * 2u;
+    uint32_t aoff[kAInstr];
+#pragma unroll
+    for (int u = 0; u < kAInstr; ++u) {
+        const uint32_t s = (wave * kAInstr + u) * 64u + lane, r = s >> 3;
+        const uint32_t row = row0 + r < p.m ? r : p.m - 1u - row0;  // rows past the end are never stored
+        aoff[u] = row * row_bytes + (((s & 7u) ^ ((r >> 1) & 7u)) << 4);
+    }
+    const char* Abase = reinterpret_cast<const char*>(p.x) + static_cast<size_t>(row0) * row_bytes;
+    auto issue = [&](uint32_t step, char* As) __attribute__((always_inline)) {
+        // a scalar base plus the lane's 32-bit offset, which the load instruction adds itself
+        const uint64_t v = reinterpret_cast<uint64_t>(Abase + step * 128u);
+        uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+        uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+        asm volatile("" : "+s"(lo), "+s"(hi));
+        const char* ab = reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
+#pragma unroll
+        for (int u = 0; u < kAInstr; ++u) asm volatile("" : "+v"(aoff[u]));
+#pragma unroll
+        for (int u = 0; u < kAInstr; ++u) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(ab + aoff[u]), (lds_ptr_t)(As + (wave * kAInstr + u) * 1024u), 16, 0, 0);
+        }
+    };
+
+    // ---- B: the thread's column of the tile and its first piece (of 8 weights) in the column's line
+    uint32_t bcol, bpiece, boff;
+    if constexpr (kInt4) {
+        // a K step is half a packed tile: 32 lanes of 16 bytes, lane column l % 16, k 32 (l / 16) .. + 31
+        constexpr uint32_t kPer = 4u / kParts;             // threads that share such a lane's 16 bytes
+        const uint32_t s = tid / kPer, l = s & 31u;
+        bcol = (s >> 5) * 16u + (l & 15u);
+        bpiece = 4u * (l >> 4) + (tid % kPer) * kParts;
+        boff = (s >> 5) * (p.k * 8u) + l * 16u + (tid % kPer) * 8u;
+    } else {
+        constexpr uint32_t kPer = 8u / kParts;             // threads that share a column's 64 bytes
+        bcol = tid / kPer;
+        bpiece = (tid % kPer) * kParts;
+        boff = bcol * p.k + bpiece * 8u;
+    }
+    // columns past n fall outside the buffer: zeros arrive (their results are never stored)
+    const uint32_t left = p.n - n0 < BN ? p.n - n0 : BN;
+    const uint64_t wbase = kInt4 ? static_cast<uint64_t>(n0 / 16u) * (p.k * 8u) : static_cast<uint64_t>(n0) * p.k;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(p.w) + wbase, 0, static_cast<int>(kInt4 ? (left + 15u) / 16u * (p.k * 8u) : left * p.k), 0x00020000);
+    const uint32_t gcol = n0 + (bcol < left ? bcol : left - 1u);
+    f16x2 csc = both(0.0f), cof = both(0.0f);              // int8: scale and offset belong to the column
+    if constexpr (!kInt4) {
+        const uint32_t sb = p.scale ? p.scale[gcol] : p.scale_bits;
+        const uint32_t ob = kOff ? (p.scale ? p.offset[gcol] : p.offset_bits) : 0u;
+        csc = as_h2(sb * 0x10001u);
+        cof = as_h2(ob * 0x10001u);
+    }
+    __amdgpu_buffer_rsrc_t rs = rw, ro = rw;               // int4: scale and offset of a group of k and a column
+    uint32_t poff = 0;
+    if constexpr (kInt4) {
+        const int bytes = static_cast<int>((p.k >> (5u + p.gs_shift)) * p.n * 2u);
+        rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.scale), 0, bytes, 0x00020000);
+        ro = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kOff ? p.offset : p.scale), 0, bytes, 0x00020000);
+        poff = gcol * 2u + (p.gs_shift == 0 ? (bpiece >> 2) * p.n * 2u : 0u);
+    }
+    struct Raw {
+        u32x4 b[kInt4 ? 1 : kParts / 2];                   // (BN = 128, int4: half of it)
+        uint32_t sc, of;
+    };
+    const uint32_t last = p.k / kBK - 1u;
+    auto fetch = [&](Raw& raw, uint32_t step) __attribute__((always_inline)) {
+        step = step < last ? step : last;                  // past the end: the last step's, into a stage nobody reads
+        const uint32_t at = kInt4 ? step * 512u : step * kBK;
+        if constexpr (kInt4 && kParts == 2) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rw, boff, at, 0);
+            raw.b[0][0] = v[0];
+            raw.b[0][1] = v[1];
+        } else {
+#pragma unroll
+            for (int i = 0; i < static_cast<int>(sizeof(raw.b) / 16u); ++i) {
+                raw.b[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, boff + 16u * i, at, 0));
+            }
+        }
+        if constexpr (kInt4) {
+            // the group of 32 k 2 step + (0 or 1); the lane's half matters for groups of 32 only
+            const uint32_t pat = ((2u * step) >> p.gs_shift) * p.n * 2u;
+            raw.sc = __builtin_amdgcn_raw_buffer_load_b16(rs, poff, pat, 0);
+            raw.of = kOff ? __builtin_amdgcn_raw_buffer_load_b16(ro, poff, pat, 0) : 0u;
+        }
+    };
+    const uint32_t bline = bcol * 128u, bswz = (bcol >> 1) & 7u;
+    WqMasks mk = p.mk;
+    asm volatile("" : "+v"(mk.exp_even), "+v"(mk.exp_odd));  // (an instruction takes one scalar operand)
+    // pair c of piece q of the thread's share of a step; the finished piece goes to LDS
+    u32x4 piece;
+    auto dequant_pair = [&](const Raw& raw, int q, int c) __attribute__((always_inline)) {
+        if constexpr (kInt4) {
+            piece[c] = pair_of_i4<kOff>(raw.b[0][q], c, as_h2(raw.sc * 0x10001u), as_h2(raw.of * 0x10001u), mk);
+        } else {
+            piece[c] = pair_of_i8<kOff>(raw.b[q >> 1][2 * (q & 1) + (c >> 1)], c & 1, csc, cof);
+        }
+    };
+    auto write_piece = [&](char* Bs, int q) __attribute__((always_inline)) {
+        *reinterpret_cast<u32x4*>(Bs + bline + (((bpiece + q) ^ bswz) << 4)) = piece;
+    };
+
+    f32x4 acc[NA][TJ];
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            asm volatile("" : "+v"(acc[i][j]));
+        }
+
+    // ---- operands: lane l holds line l % 16 of a block of 16 and the 8 k of piece 4 ks + l / 16.  A step is four
+    // quarters: quarter q multiplies half q % 2 of the wavefront's rows with the 32 k of sub-step ks = q / 2.
+    const uint32_t lc = lane & 15u, lq = lane >> 4;
+    uint32_t foff[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) foff[ks] = lc * 128u + (((4u * ks + lq) ^ (lc >> 1)) << 4);
+    f16x8 af[2][NH], bf[2][TJ];
+    auto load_a = [&](const char* As, int q, int i) __attribute__((always_inline)) {
+        af[q & 1][i] = *reinterpret_cast<const f16x8*>(As + wm * (NA * 2048u) + ((q & 1) * NH + i) * 2048u + foff[q >> 1]);
+    };
+    auto load_b = [&](const char* Bs, int ks, int j) __attribute__((always_inline)) {
+        bf[ks][j] = *reinterpret_cast<const f16x8*>(Bs + wn * 8192u + j * 2048u + foff[ks]);
+    };
+    // Matrix instruction number n of quarter q.  Written as an instruction that accumulates in place: left to itself the
+    // compiler gave it another destination than its addend and moved accumulators about, spilling some.  (Its operands
+    // come from LDS reads, which the compiler waits for; no vector instruction touches them or the sums in the loop.)
+    auto mfma = [&](int q, int n) __attribute__((always_inline)) {
+        f32x4& c = acc[(q & 1) * NH + n / TJ][n % TJ];
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(af[q & 1][n / TJ]), "v"(bf[q >> 1][n % TJ]));
+    };
+    // One quarter: its NH * TJ matrix instructions, the LDS reads `read(r)`, r < kReads, one behind each of the first, and
+    // a piece of the next step's weights de-quantised pair by pair behind four later ones.  The order is the one written.
+    constexpr int kM = NH * TJ;
+    auto quarter = [&](auto qq, auto reads, auto&& read, auto part, const Raw& next, char* Bn) __attribute__((always_inline)) {
+        constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value, kPart = decltype(part)::value;
+        constexpr int kPer = (kReads + kM - 1) / kM;
+        wq_for<kM>([&](auto nn) {
+            constexpr int n = decltype(nn)::value;
+            mfma(q, n);
+            wq_for<kPer>([&](auto r) {
+                constexpr int i = n * kPer + decltype(r)::value;
+                if constexpr (i < kReads) read(std::integral_constant<int, i>{});
+            });
+            if constexpr (kPart >= 0) {
+                // pairs behind instructions kM - 5 .. kM - 2 (of at least 4)
+                constexpr int first = kM >= 8 ? kM - 5 : 0;
+                if constexpr (n >= first && n < first + 4) dequant_pair(next, kPart, n - first);
+                if constexpr (n == first + 3) write_piece(Bn, kPart);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // Quarters 0 - 2 of step s in stage (A, B), whose first operands are in registers; pieces 1 .. of step s + 1 go
+    // into stage Bn (kParts == 2: the second of two behind quarter 1).
+    auto head = [&](const char* As, const char* Bs, const Raw& next, char* Bn) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(foff[q]));
+        wq_for<3>([&](auto qq) {
+            constexpr int q = decltype(qq)::value;
+            constexpr int part = kParts == 4 ? q + 1 : q == 1 ? 1 : -1;
+            quarter(qq, std::integral_constant<int, NH + (q < 2 ? 2 : 0)>{}, [&](auto r) __attribute__((always_inline)) {
+                constexpr int i = decltype(r)::value;
+                if constexpr (i < NH) {
+                    load_a(As, q + 1, i);
+                } else {
+                    load_b(Bs, 1, 2 * q + i - NH);
+                }
+            }, std::integral_constant<int, part>{}, next, Bn);
+        });
+    };
+    // Behind the barrier: the last quarter's instructions, the first operands of step s + 1 and piece 0 of step s + 2
+    // (into this step's stage, which everyone has left).
+    auto first_operands = [&](const char* An, const char* Bn, int i) __attribute__((always_inline)) {
+        if (i == 0 || i > NH) {
+            load_b(Bn, 0, i == 0 ? 0 : i - NH);
+        } else {
+            load_a(An, 0, i - 1);
+        }
+    };
+    auto tail = [&](const char* An, const char* Bn, const Raw& next2, char* Bs) __attribute__((always_inline)) {
+        quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
+            first_operands(An, Bn, decltype(r)::value);
+        }, std::integral_constant<int, 0>{}, next2, Bs);
+    };
+    auto clamp = [&](uint32_t step) { return step < last ? step : last; };
+
+    Raw r0, r1;
+    issue(0, A0);
+    fetch(r0, 0);
+    fetch(r1, 1);
+#pragma unroll
+    for (int q = 0; q < kParts; ++q) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) dequant_pair(r0, q, c);
+        write_piece(B0, q);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    issue(clamp(1), A1);
+    fetch(r0, 2);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dequant_pair(r1, 0, c);
+    write_piece(B1, 0);
+#pragma unroll
+    for (int i = 0; i < NH + TJ; ++i) first_operands(A0, B0, i);
+    // At the top of step s (stage x, other stage y): its first operands are in registers, piece 0 of step s + 1 is in
+    // y, the rest of it in raw set (s + 1) % 2, step s + 2's raw bytes are on their way into set s % 2.
+    const uint32_t steps = last + 1u;
+    uint32_t s = 0;
+    for (; s + 1u < steps; s += 2u) {
+        head(A0, B0, r1, B1);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        issue(clamp(s + 2u), A0);
+        fetch(r1, s + 3u);
+        tail(A1, B1, r0, B0);
+        head(A1, B1, r0, B0);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        issue(clamp(s + 3u), A1);
+        fetch(r0, s + 4u);
+        tail(A0, B0, r1, B1);
+    }
+    if (s < steps) {  // an odd last step
+        head(A0, B0, r1, B1);
+#pragma unroll
+        for (int n = 0; n < kM; ++n) mfma(3, n);
+    }
+    // the last sums are on their way through the matrix pipe
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past the end
+
+    // ---- register r of lane l in a 16 x 16 block: row 4 (l / 16) + r, column l % 16
+    const uint32_t colw = n0 + wn * 64u, roww = row0 + wm * (NA * 16u) + 4u * lq;
+    if (!p.out_f32 && p.n % 4u == 0) {
+        // half output: a 4 x 4 transposition inside each four neighbouring lanes (two exchanges of packed pairs) leaves
+        // lane b of the four with columns 4 (l / 4) .. + 3 of block b: one 8-byte store per lane and row, and the 16
+        // lanes of a row write one full 128-byte line
+        const bool b0 = (lane & 1u) != 0, b1 = (lane & 2u) != 0;
+        const uint32_t col = colw + 16u * (lane & 3u) + (lc & 12u);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t row = roww + i * 16u + r;
+                uint32_t h[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) h[j] = f32_to_half_bits(acc[i][j][r]);
+                const uint32_t give = b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16);
+                const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+                const uint32_t lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
+                const uint32_t hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
+                const uint32_t got2 = static_cast<uint32_t>(
+                    __builtin_amdgcn_mov_dpp(static_cast<int>(b1 ? lo : hi), 0x4E, 0xF, 0xF, true));  // lane ^ 2
+                if (row < p.m && col < p.n) {
+                    __builtin_nontemporal_store(b1 ? u32x2{got2, hi} : u32x2{lo, got2},
+                                                reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.y) + static_cast<size_t>(row) * p.n + col));
+                }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const uint32_t col = colw + j * 16u + lc;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t row = roww + i * 16u + r;
+                if (row < p.m && col < p.n) {
+                    const size_t idx = static_cast<size_t>(row) * p.n + col;
+                    if (p.out_f32) {
+                        static_cast<float*>(p.y)[idx] = acc[i][j][r];
+                    } else {
+                        static_cast<uint16_t*>(p.y)[idx] = static_cast<uint16_t>(f32_to_half_bits(acc[i][j][r]));
+                    }
+                }
+            }
+        }
+    }
+}
+
+// 256 x 256: the first p.full tiles are run as they are; each of the others, which would leave part of the last
+// round of the chip idle, is run by two workgroups with 128 x 256 tiles.
+template <int BM, int BN, bool kInt4, bool kOff>
+__global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
+{
+    __shared__ __attribute__((aligned(1024))) char A0[BM * 128];
+    __shared__ __attribute__((aligned(1024))) char A1[BM * 128];
+    __shared__ __attribute__((aligned(1024))) char B0[BN * 128];
+    __shared__ __attribute__((aligned(1024))) char B1[BN * 128];
+    const uint32_t tiles = p.tiles_m * p.tiles_n;
+    uint32_t tm, tn;
+    if (BM == 128 || blockIdx.x < p.full) {
+        const uint32_t t = xcd_remap(blockIdx.x, BM == 128 ? tiles : p.full);
+        if (t == 0xFFFFFFFFu) {
+            return;  // whole workgroup (the launch is rounded up to a multiple of 8)
+        }
+        band_order(t, p.tiles_m, p.tiles_n, tm, tn);
+        wq_tile<BM, BN, kInt4, kOff>(p, tm * BM, tn * BN, A0, A1, B0, B1);
+    } else if constexpr (BM == 256) {
+        const uint32_t t = xcd_remap(blockIdx.x - p.full, 2u * (tiles - p.full));
+        if (t == 0xFFFFFFFFu) {
+            return;
+        }
+        band_order(p.full + t / 2u, p.tiles_m, p.tiles_n, tm, tn);
+        const uint32_t row0 = tm * 256u + (t & 1u) * 128u;
+        if (row0 < p.m) {
+            wq_tile<128, BN, kInt4, kOff>(p, row0, tn * BN, A0, A1, B0, B1);
+        }
+    }
+}
+
+template <int BM, int BN>
+void wq_launch(WqParams p, bool int4, bool has_offset, hipStream_t st)
+{
+    p.tiles_m = (p.m + BM - 1u) / BM;
+    p.tiles_n = (p.n + BN - 1u) / BN;
+    const uint32_t tiles = p.tiles_m * p.tiles_n;
+    const uint32_t blocks = BM == 256 ? p.full + 2u * (tiles - p.full) : tiles;
+    const uint32_t grid = (blocks + 7u) / 8u * 8u;
+    if (int4) {
+        has_offset ? wq_gemm_kernel<BM, BN, true, true><<<grid, kThreads, 0, st>>>(p)
+                   : wq_gemm_kernel<BM, BN, true, false><<<grid, kThreads, 0, st>>>(p);
+    } else {
+        has_offset ? wq_gemm_kernel<BM, BN, false, true><<<grid, kThreads, 0, st>>>(p)
+                   : wq_gemm_kernel<BM, BN, false, false><<<grid, kThreads, 0, st>>>(p);
+    }
+}
+
+}  // namespace
+
+// The tile shape: the one with the smallest estimate of rounds of the chip times a round's time per K step, measured at
+// k = 8192, n = 28672 with every compute unit busy (us): 256 x 256 1.62, 128 x 256 1.11, 128 x 128 1.2 for the two tiles
+// that share a unit and 0.62 for one alone.  256 x 256 tiles that would fill less than about two thirds of the last round
+// are cut in half there (k = 4096, n = 11008, 2048 rows: 204 -> 187 us; where the power limit and not
+// the rounds sets the time it makes no difference, k = 8192, n = 28672, 2048 rows: 847 us either way).
+int launch_wq_gemm(const WqParams& p, bool int4, bool has_offset, hipStream_t st)
+{
+    WqParams q = p;
+    q.mk = WqMasks{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
+    const uint32_t cus = device_compute_units();
+    auto up = [](uint32_t a, uint32_t b) { return (a + b - 1u) / b; };
+    const uint32_t t256 = up(p.m, 256u) * up(p.n, 256u), t128 = up(p.m, 128u) * up(p.n, 256u), tsmall = up(p.m, 128u) * up(p.n, 128u);
+    const uint32_t rounds = t256 / cus, rest = t256 % cus;
+    const double tail = up(2u * rest, cus) * 1.11;
+    const bool halve = rest != 0 && tail < 1.62;
+    const double c256 = rounds * 1.62 + (rest == 0 ? 0.0 : halve ? tail : 1.62);
+    const double c128 = up(t128, cus) * 1.11;
+    const double csmall = tsmall <= cus ? 0.62 : up(tsmall, 2u * cus) * 1.2;
+    if (csmall <= c128 && csmall <= c256) {
+        wq_launch<128, 128>(q, int4, has_offset, st);
+    } else if (c128 < c256) {
+        wq_launch<128, 256>(q, int4, has_offset, st);
+    } else {
+        q.full = halve ? rounds * cus : t256;
+        wq_launch<256, 256>(q, int4, has_offset, st);
+    }
+    return launch_status("half x quantised weights (tile GEMM)");
+}
+
+}  // namespace ascq

@@ -689,7 +689,7 @@ def main():
             r = w8a16(2048, 30, 5, sets=1, b_nk=nk)
             others["w8a16_nk_m2048_k8192_n28672" if nk else "w8a16_m2048_k8192_n28672"] = {
                 "kernel_ms": r["kernel_ms"], "tflops": r["tflops"], "f16_mfma_frac": r["tflops"] / PEAK_F16_TFLOPS,
-                "note": "half GEMM whose B-tile loader de-quantises (w8a16_nk_gemm_kernel)" +
+                "note": "half GEMM whose B-tile loader de-quantises (wq_gemm_kernel)" +
                         ("" if nk else ", after one transposed copy of the [k, n] weights into the workspace")}
             torch.cuda.empty_cache()
         r = group5(max(20, side_steps // 5), 5)

@@ -560,7 +560,8 @@ int ascq_matmul_w4a16_workspace_size(const ascq_w4a16_desc* desc, size_t* bytes)
  * rounding to half) in one launch with no workspace: a workgroup owns whole columns and adds its wavefronts' partial
  * sums in a fixed order, so repeated calls give identical bits.  Up to 4 activation rows (decode) its wavefronts
  * split k and add their sums in LDS; 5 to 16 rows run one wavefront per slab with the activations shared chunk by
- * chunk; more rows take further passes of 16 over the weights.  Requires k % 128 == 0, n % 8 == 0, group_size =
+ * chunk; more rows take further passes of 16 over the weights, and beyond 48 rows the per-weight form runs a half GEMM
+ * whose B-tile loader de-quantises.  Requires k % 128 == 0, n % 8 == 0, group_size =
  * 32 * 2^i (ASCQ_EUNSUPPORTED otherwise: use ascq_matmul_w4a16), and x, w_packed, scale, offset 16-byte aligned.
  */
 int ascq_pack_weight_w4_size(uint32_t k, uint32_t n, size_t* bytes);
@@ -584,8 +585,8 @@ int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* desc, void* y, const void* x
  * workgroup: one launch, no workspace (the size query answers 0), identical bits from call to call; that form needs
  * k % 128 == 0 and 16-byte aligned x and w (other shapes and alignments run a slow kernel with one lane per output
  * element, as they do for [k, n] weights).
- * Many rows (more than 32 on [n, k] weights, more than 96 on [k, n]) run a half GEMM on 128 x 128 tiles whose B-tile
- * loader de-quantises; [k, n] weights are first copied transposed into the workspace (k * n bytes, which the size query
+ * Many rows (more than 32 on [n, k] weights, more than 96 on [k, n]) run a half GEMM whose B-tile loader
+ * de-quantises (tiles of up to 256 x 256); [k, n] weights are first copied transposed into the workspace (k * n bytes, which the size query
  * then asks for; given less, the call falls back to one pass over the weights per 32 rows).
  * workspace: ascq_matmul_w8a16_workspace_size bytes (contents need not be initialised); calls that share a
  * workspace must not overlap.

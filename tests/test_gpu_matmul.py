@@ -706,6 +706,28 @@ def test_w4a16_packed_more_than_four_rows(m, k, n, gs):
     assert torch.equal(y1, y2)
 
 
+@pytest.mark.parametrize("m,k,n,gs", [(49, 128, 8, 32), (128, 256, 248, 64), (129, 384, 264, 128), (257, 640, 520, 128), (300, 128, 1032, 32),
+                                       (1300, 256, 14600, 256)])
+@pytest.mark.parametrize("offset", ["int", "frac", None])
+def test_w4a16_packed_many_rows(m, k, n, gs, offset):
+    """More rows than a few passes: the half GEMM whose B-tile loader de-quantises the packed tiles.  One step of k, odd
+    and even numbers of steps, row and column tails of every tile shape, groups of half a step; the last case has tiles
+    beyond a whole round, which are cut in half (checked on its first, a middle and the last columns)."""
+    announce("w4a16 packed many rows", m, k, n, gs, offset)
+    rng = np.random.default_rng(m + 3 * k + n)
+    x, wp, sc, of = w4_case(rng, m, k, n, gs, offset is not None)
+    if offset == "frac":
+        of = (rng.standard_normal((k // gs, n)) * 3).astype(np.float16)
+    w_gpu = ops.pack_weight_w4(to_dev(wp), k, n)
+    y = torch.full((m, n), 7.0, dtype=torch.float16, device=DEV)
+    ops.matmul_w4a16_packed(y, to_dev(x), w_gpu, to_dev(sc), None if of is None else to_dev(of), gs)
+    d = abi.W4A16Desc(m=m, n=n, k=k, group_size=gs, has_offset=int(of is not None))
+    orc.set_threads(16)
+    for c0, c1 in [(0, n)] if n < 2000 else [(0, 80), (n // 2, n // 2 + 80), (n - 80, n)]:
+        want = orc.matmul_w4a16(d, x, wp, sc, of, cols=(c0, c1))[:, c0:c1]
+        w4_check(np.ascontiguousarray(y.cpu().numpy()[:, c0:c1]), np.ascontiguousarray(want), x)
+
+
 def config4_columns(m, n):
     """The oracle covers every column at M=1 (about 6 s on 16 threads); for more rows three slabs: the first and the last
     512 columns (the kernels' first and last column blocks) and one from the middle."""
@@ -956,6 +978,29 @@ def test_w8a16_trans_b(m, k, n, mode):
     assert np.array_equal(np.asarray(want).view(np.uint8),
                           np.asarray(orc.matmul_w8a16(d, x, np.ascontiguousarray(wt.T), None if per_tensor else of,
                                                       None if per_tensor else sc)).view(np.uint8))
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 128, 7), (128, 256, 248), (129, 384, 264), (257, 640, 521), (300, 128, 1034)])
+@pytest.mark.parametrize("mode", ["vector+offset", "vector", "scalar+offset"])
+@pytest.mark.parametrize("out_f32", [False, True])
+def test_w8a16_trans_b_many_rows(m, k, n, mode, out_f32):
+    """The half GEMM whose B-tile loader de-quantises [n, k] weights: two steps of k and more, row and column tails of
+    every tile shape, column counts that are no multiple of 4 (stored element by element) and of 2."""
+    announce("w8a16 [n, k] many rows", m, k, n, mode, out_f32)
+    rng = np.random.default_rng(m + k + n)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    wt = rng.integers(-128, 128, (n, k)).astype(np.int8)
+    per_tensor, has_offset = mode.startswith("scalar"), "offset" in mode
+    sc = 0.0077 if per_tensor else rng.uniform(1e-3, 1e-2, n).astype(np.float16)
+    of = None if not has_offset else 2.5 if per_tensor else rng.uniform(-9, 9, n).astype(np.float16)
+    y = torch.full((m, n), 7.0, dtype=torch.float32 if out_f32 else torch.float16, device=DEV)
+    ops.matmul_w8a16(y, to_dev(x), to_dev(wt), of if per_tensor or of is None else to_dev(of), sc if per_tensor else to_dev(sc),
+                     workspace=torch.empty(4, device=DEV), trans_b=True)
+    d = abi.W8A16Desc(m=m, n=n, k=k, per_tensor=int(per_tensor), has_offset=int(has_offset), scale=sc if per_tensor else 0.0,
+                      offset=of if per_tensor and has_offset else 0.0, out_dtype=abi.F32 if out_f32 else abi.F16, trans_b=1)
+    orc.set_threads(16)
+    want = orc.matmul_w8a16(d, x, wt, None if per_tensor else of, None if per_tensor else sc)
+    w8a16_check(y.cpu().numpy(), want, x, out_f32)
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
