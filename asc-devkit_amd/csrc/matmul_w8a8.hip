@@ -560,13 +560,13 @@ bool fast_path_ok(const ascq_matmul_desc* d, const void* a, const void* b)
 // Up to this many rows the 128 x 128 direct-to-LDS kernel (K split over workgroups) is used when the shape allows.
 constexpr uint32_t kSkinnyMaxM = 512;
 
-// ascq_matmul_w8a8_packed between 129 and 512 rows: true when the 128 x 128 tiles (no K split: the call has no
-// workspace) are expected to beat the weights-in-registers form.  Both estimates are fits to measurements at
+// Packed weights between 129 and 512 rows: true when the 128 x 128 tiles (`splits` of K, 1 without a workspace) are
+// expected to beat the weights-in-registers form.  Both estimates are fits to measurements at
 // k = 4096, n = 11008 and k = 11008, n = 4096 (the crossovers there: 256 and about 380 rows).  Registers form: the
 // weights once (5 us + 1 us per 4.7 MB), then 0.95 us per 16 rows and 4096 of k, per round of workgroups.  Tiles:
 // 6.5 us per 1024 of k for up to one tile per compute unit, 1.45 times that with two (they share the unit), and in
 // proportion beyond.  Above 512 rows the 256-row tiles always lead.
-bool packed_tiles_faster(const GemmParams& p)
+bool packed_tiles_faster(const GemmParams& p, uint32_t splits)
 {
     const double kk = p.k / 4096.0;
     const double ws_us = 5.0 + static_cast<double>(p.n) * p.k / 4.7e6 +
@@ -575,6 +575,10 @@ bool packed_tiles_faster(const GemmParams& p)
     const double cus = device_compute_units();
     const double load = tiles <= cus ? 1.0 : tiles <= 2.0 * cus ? 1.0 + 0.45 * (tiles - cus) / cus : 1.45 * tiles / (2.0 * cus);
     const double tiles_us = 4.0 + 26.0 * kk * load;
+    if (splits > 1u) {  // a second launch, and the partial tiles written and read back (gemm_dma_small_tiles)
+        const double split_us = 8.0 + 26.0 * kk / splits + static_cast<double>(splits) * p.m * p.n * 8.0 / 5e6;
+        return (split_us < tiles_us ? split_us : tiles_us) < ws_us;
+    }
     return tiles_us < ws_us;
 }
 // Up to this many rows the weight-stream kernel is preferred over those tiles.
@@ -609,14 +613,33 @@ __global__ __launch_bounds__(256) void swiglu_epilogue_kernel(GemmParams p)
     }
 }
 
-// True when the plain matmul of this descriptor runs on the large direct-to-LDS tile kernel, whose epilogue applies
-// SwiGLU in registers (16-bit outputs).
+// Whether the direct-to-LDS tiles take this plain matmul.  A last, partial K step or columns off the tile size cost them
+// a few masked loads (729 rows, k = 4304, n = 1152, quantiser included: 123 us on the register-staged tiles, 28 us here).
+// [n, k] weights with such a k, 33 to 512 rows: only where K is split; otherwise the plan query promises the
+// register-staged tiles (and up to 32 rows those have a K split of their own).
+bool dma_tiles_ok(const ascq_matmul_desc* d, const GemmParams& p)
+{
+    if (d->trans_a || !gemm_dma_supported(p, d->trans_b ? 1 : 0)) {
+        return false;
+    }
+    return !d->trans_b || d->k % 128u == 0 || d->m > kSkinnyMaxM ||
+           (d->m > 32u && gemm_dma_skinny_splits(d->m, d->n, d->k) > 1u);
+}
+
+// Of those, the calls that run 128 x 128 tiles (K split where the caller brings a workspace).
+bool dma_tiles_small(const ascq_matmul_desc* d)
+{
+    return d->m <= kSkinnyMaxM || (d->activation != ASCQ_MM_ACT_SWIGLU && gemm_dma_small_tiles(d->m, d->n, d->k));
+}
+
+// True when the plain matmul of this descriptor runs on the direct-to-LDS tiles without a K split, whose epilogue
+// applies SwiGLU in registers (16-bit outputs).
 bool swiglu_in_tile_kernel(const ascq_matmul_desc* d, const GemmParams& p, const void* a, const void* b)
 {
     if (d->out_dtype != ASCQ_F16 && d->out_dtype != ASCQ_BF16) {
         return false;
     }
-    if (d->m <= kSkinnyMaxM || !gemm_dma_supported(p)) {
+    if (!dma_tiles_ok(d, p) || (d->m <= kSkinnyMaxM && (d->m <= 128u || gemm_dma_skinny_splits(d->m, d->n, d->k) > 1u))) {
         return false;
     }
     return d->b_format == ASCQ_MM_B_NZ || fast_path_ok(d, a, b);
@@ -651,6 +674,11 @@ ascq_matmul_desc raw_accumulator_desc(const ascq_matmul_desc* d)
 
 using namespace ascq;
 
+namespace {
+int matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const void* w_packed, const void* bias,
+                       const void* quant_vector, const void* tok_scale, void* workspace, size_t workspace_bytes, void* stream);
+}  // namespace
+
 extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t* bytes)
 {
     ASCQ_REQUIRE(d != nullptr && bytes != nullptr, ASCQ_ENULL, "ascq_matmul_w8a8_workspace_size: NULL argument");
@@ -684,7 +712,7 @@ extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t
         // (few rows on [n, k] weights with k % 128 == 0 run the whole-column kernel, which needs none)
         *bytes = static_cast<size_t>(d->m) * d->n * sizeof(int32_t);
     }
-    if (d->m <= kSkinnyMaxM && !d->trans_a && d->k % 128 == 0 && d->n % 16 == 0 && !(d->m <= 32 && d->trans_b)) {
+    if (dma_tiles_ok(d, shape) && dma_tiles_small(d) && !(d->m <= 32 && d->trans_b)) {
         const size_t need =
             static_cast<size_t>(gemm_dma_skinny_splits(d->m, d->n, d->k)) * d->m * d->n * sizeof(int32_t);
         if (need > *bytes && need > static_cast<size_t>(d->m) * d->n * sizeof(int32_t)) {
@@ -765,9 +793,10 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
     }
     // Up to 8 rows the weight streams; from 9 rows on the split-K tiles below are faster when the shape allows them
     // (k = 4096, n = 11008: 16.8-17.9 against 17.3-17.6 us up to 8 rows, 18.9 / 23.1 against 17.0 / 17.5 us at 16 / 32)
-    const bool tiles_instead = d->m > kStreamMaxM && gemm_dma_supported(p) && workspace != nullptr &&
-                               aligned16(workspace) &&
-                               workspace_bytes >= static_cast<size_t>(gemm_dma_skinny_splits(d->m, d->n, d->k)) * d->m * d->n * sizeof(int32_t);
+    const bool small_workspace =
+        workspace != nullptr && aligned16(workspace) &&
+        workspace_bytes >= static_cast<size_t>(gemm_dma_skinny_splits(d->m, d->n, d->k)) * d->m * d->n * sizeof(int32_t);
+    const bool tiles_instead = d->m > kStreamMaxM && dma_tiles_ok(d, p) && small_workspace;
     if (!tiles_instead && !d->trans_b && gemm_stream_supported(p) && workspace != nullptr && aligned16(workspace) &&
         workspace_bytes >= gemm_stream_workspace(d->m, d->n, d->k)) {
         return launch_gemm_stream(p, workspace, st);
@@ -781,7 +810,7 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
     if (d->m <= 32 && d->trans_b && !d->trans_a && gemm_nk_supported(p)) {
         return launch_gemm_nk(p, st);
     }
-    if (d->m <= kSkinnyMaxM && !d->trans_a && gemm_dma_supported(p)) {
+    if (dma_tiles_ok(d, p) && dma_tiles_small(d) && (d->m <= kSkinnyMaxM || small_workspace)) {
         return launch_gemm_dma_skinny(p, workspace, workspace_bytes, st, d->trans_b != 0);
     }
     if (d->m <= 32) {
@@ -815,11 +844,8 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
         }
         return d->trans_b ? launch_gemm<TileST, true, false>(p, st) : launch_gemm<TileS, false, false>(p, st);
     }
-    if (d->m > 128 && !d->trans_b && gemm_dma_supported(p)) {
-        return launch_gemm_dma(p, false, st);
-    }
-    if (d->m > 512 && d->trans_b && !d->trans_a && gemm_dma_supported(p)) {
-        return launch_gemm_dma(p, false, st, true);  // B as [n][k]: its tiles are staged and read like A's
+    if (dma_tiles_ok(d, p)) {
+        return launch_gemm_dma(p, false, st, d->trans_b != 0);  // B as [n][k]: its tiles are staged and read like A's
     }
     if (d->m <= 1024) {
         return d->trans_b ? launch_gemm<TileMT, true, false>(p, st) : launch_gemm<TileM, false, false>(p, st);
@@ -832,6 +858,14 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
 // (examples/.../quant_group_matmul_high_performance/scripts/gen_data.py:62-64)
 extern "C" int ascq_matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const void* w_packed,
                                        const void* bias, const void* quant_vector, const void* tok_scale, void* stream)
+{
+    return matmul_w8a8_packed(d, c, a, w_packed, bias, quant_vector, tok_scale, nullptr, 0, stream);
+}
+
+namespace {
+
+int matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const void* w_packed, const void* bias,
+                       const void* quant_vector, const void* tok_scale, void* workspace, size_t workspace_bytes, void* stream)
 {
     ASCQ_REQUIRE(d != nullptr, ASCQ_ENULL, "ascq_matmul_w8a8_packed: desc is NULL");
     int rc = validate_mm(d, "ascq_matmul_w8a8_packed", c, a, w_packed, bias, quant_vector, tok_scale);
@@ -853,17 +887,25 @@ extern "C" int ascq_matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const
     // Many rows: the direct-to-LDS tile kernels read the packed tiles as they lie (one tile per load instruction), so a
     // caller that packed its weights for decode needs no second copy of them for prefill.  (SwiGLU in those kernels'
     // epilogue exists for 16-bit outputs.)
-    const bool tiles_ok = gemm_dma_supported(p) &&
+    const bool tiles_ok = gemm_dma_supported(p, 2) &&
                           (d->activation != ASCQ_MM_ACT_SWIGLU || d->out_dtype == ASCQ_F16 || d->out_dtype == ASCQ_BF16);
-    if (tiles_ok && (d->m > kSkinnyMaxM || (d->m > 128u && packed_tiles_faster(p)))) {
-        return d->m <= kSkinnyMaxM ? launch_gemm_dma_skinny(p, nullptr, 0, static_cast<hipStream_t>(stream), 2)
-                                   : launch_gemm_dma(p, false, static_cast<hipStream_t>(stream), 2);
+    uint32_t splits = gemm_dma_skinny_splits(d->m, d->n, d->k);
+    if (workspace == nullptr || !aligned16(workspace) || d->activation == ASCQ_MM_ACT_SWIGLU ||
+        workspace_bytes < static_cast<size_t>(splits) * d->m * d->n * sizeof(int32_t)) {
+        splits = 1;
+    }
+    if (tiles_ok && (d->m > kSkinnyMaxM || (d->m > 128u && packed_tiles_faster(p, splits)))) {
+        const bool small = d->m <= kSkinnyMaxM || (splits > 1u && gemm_dma_small_tiles(d->m, d->n, d->k));
+        return small ? launch_gemm_dma_skinny(p, workspace, splits > 1u ? workspace_bytes : 0, static_cast<hipStream_t>(stream), 2)
+                     : launch_gemm_dma(p, false, static_cast<hipStream_t>(stream), 2);
     }
     if (gemm_ws_supported(p, false)) {
         return launch_gemm_ws(p, static_cast<hipStream_t>(stream), false);
     }
     return launch_gemm_packed(p, static_cast<hipStream_t>(stream));
 }
+
+}  // namespace
 
 // ref: include/adv_api/matmul/matmul_tilingdata.h:21-72 (TCubeTiling, the reference's host-side plan of a matmul)
 extern "C" int ascq_matmul_w8a8_plan(const ascq_matmul_desc* d, const void* c, const void* a, const void* b,
@@ -1006,7 +1048,9 @@ extern "C" int ascq_linear_w8a8_dynamic_packed(const ascq_matmul_desc* d, int32_
     if (rc != ASCQ_OK) {
         return rc;
     }
-    return ascq_matmul_w8a8_packed(&dd, c, q, w_packed, bias, quant_vector, tok, stream);
+    char* rest = reinterpret_cast<char*>(tok) + round256(static_cast<size_t>(d->m) * sizeof(float));
+    return matmul_w8a8_packed(&dd, c, q, w_packed, bias, quant_vector, tok, rest, workspace_bytes - static_cast<size_t>(rest - ws),
+                              stream);
 }
 
 // ------------------------------------------------------------------------------- the same call without a workspace
@@ -1229,7 +1273,7 @@ extern "C" int ascq_group_matmul_w8a8(const ascq_group_matmul_desc* g, void* y, 
     p.b_nz = d->b_format == ASCQ_MM_B_NZ ? 1u : 0u;
     ASCQ_REQUIRE(d->activation != ASCQ_MM_ACT_SWIGLU || d->out_dtype == ASCQ_F16 || d->out_dtype == ASCQ_BF16,
                  ASCQ_EUNSUPPORTED, "ascq_group_matmul_w8a8: SwiGLU writes half or bfloat16 here");
-    if (gemm_dma_supported(p)) {
+    if (gemm_dma_supported(p) && ((d->k % 128u == 0 && d->n % 16u == 0) || d->activation != ASCQ_MM_ACT_SWIGLU)) {
         return launch_gemm_dma(p, true, st);
     }
     ASCQ_REQUIRE(!p.b_nz, ASCQ_EUNSUPPORTED, "ascq_group_matmul_w8a8: fractal (NZ) weights need the tile kernel's shape");

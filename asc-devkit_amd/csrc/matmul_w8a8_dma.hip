@@ -794,9 +794,18 @@ __global__ __launch_bounds__(256) void splitk_sum_epilogue_kernel(GemmParams p)
 
 }  // namespace
 
-bool gemm_dma_supported(const GemmParams& p)
+// Whole 16-byte pieces along k of both operands ([n, k], packed: its tiles of 64 k) or along n ([k, n], where a last tile
+// moved left to end at n also starts its pieces at 8 bytes; it needs a whole tile's columns then).  A last partial K step
+// is masked where it is loaded.
+bool gemm_dma_supported(const GemmParams& p, int b_layout)
 {
-    return p.k % BK == 0 && p.n % 16 == 0 && p.n >= 16 && aligned16(p.a) && aligned16(p.b);
+    if (p.k % (b_layout == 2 ? 64u : 16u) != 0 || p.n < 16u || !aligned16(p.a) || !aligned16(p.b)) {
+        return false;
+    }
+    if (p.b_nz) {
+        return p.k % BK == 0 && p.n % 32u == 0;
+    }
+    return p.n % 16u == 0 || (p.n % 8u == 0 && (b_layout != 0 || p.n >= 256u));
 }
 
 namespace {
@@ -922,15 +931,31 @@ uint32_t gemm_dma_skinny_splits(uint32_t m, uint32_t n, uint32_t k)
         return 1u;
     }
     uint32_t s = 344u / tiles;
-    const uint32_t steps = k / BK;
+    const uint32_t steps = (k + BK - 1u) / BK;
     if (s > steps) s = steps;
     if (s > 16u) s = 16u;
     return s ? s : 1u;
 }
 
-// M up to a few hundred rows: 128 x 128 tiles, K split over blockIdx.y when a workspace of
-// splits * m * n * 4 bytes (16-byte aligned) is given.  b_layout: 0 [k, n], 1 [n, k], 2 packed (never split: its
-// entry point has no workspace).
+// More than 512 rows: whether the 128 x 128 tiles, K split, are expected ahead of the 256 x 256 ones, which leave most of
+// the chip idle on a narrow matrix.  In us: a 256 x 256 tile takes 1.3 per K step when most units have none; a split
+// of 128 x 128 tiles 0.8 per K step, a launch of 4 and its int32 partial tiles, written and read back at 5 TB/s
+// (729 rows, k = 4352, n = 1152, quantiser included: 52 us on 15 wide tiles, 26 us on 54 split in six; 532 rows, k = 3072,
+// n = 512: 38.5 and 24.4 us).
+bool gemm_dma_small_tiles(uint32_t m, uint32_t n, uint32_t k)
+{
+    const uint32_t wide = ((m + 255u) / 256u) * ((n + 255u) / 256u);
+    const uint32_t splits = gemm_dma_skinny_splits(m, n, k);
+    if (wide > 64u || splits < 2u) {
+        return false;
+    }
+    const uint32_t steps = (k + BK - 1u) / BK;
+    const double split_us = 4.0 + 0.8 * ((steps + splits - 1u) / splits) + static_cast<double>(splits) * m * n * 8.0 / 5e6;
+    return split_us < 1.3 * steps;
+}
+
+// M up to a few hundred rows, or few tiles: 128 x 128 tiles, K split over blockIdx.y when a workspace of
+// splits * m * n * 4 bytes (16-byte aligned) is given.  b_layout: 0 [k, n], 1 [n, k], 2 packed.
 int launch_gemm_dma_skinny(GemmParams& p, void* workspace, size_t workspace_bytes, hipStream_t st, int b_layout)
 {
     p.tiles_m = (p.m + 127u) / 128u;
@@ -938,7 +963,7 @@ int launch_gemm_dma_skinny(GemmParams& p, void* workspace, size_t workspace_byte
     const uint32_t t = (p.tiles_m * p.tiles_n + 7u) / 8u * 8u;
     uint32_t splits = gemm_dma_skinny_splits(p.m, p.n, p.k);
     const size_t need = static_cast<size_t>(splits) * p.m * p.n * sizeof(int32_t);
-    if (splits > 1 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace) || b_layout == 2)) {
+    if (splits > 1 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {
         splits = 1;
     }
     if (plan_recording()) {
@@ -957,11 +982,9 @@ int launch_gemm_dma_skinny(GemmParams& p, void* workspace, size_t workspace_byte
     }
     p.k_splits = splits;
     p.partial = static_cast<int32_t*>(workspace);
-    if (b_layout == 1) {
-        gemm_dma_kernel<128, 128, true, 1><<<dim3(t, splits), kThreads, 0, st>>>(p, 0u);
-    } else {
-        gemm_dma_kernel<128, 128, true><<<dim3(t, splits), kThreads, 0, st>>>(p, 0u);
-    }
+    with_b_layout(b_layout, [&](auto kb) {
+        gemm_dma_kernel<128, 128, true, decltype(kb)::value><<<dim3(t, splits), kThreads, 0, st>>>(p, 0u);
+    });
     int rc = launch_status("ascq_matmul_w8a8 (split-K)");
     if (rc != ASCQ_OK) {
         return rc;

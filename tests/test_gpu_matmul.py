@@ -1114,6 +1114,60 @@ def test_matmul_nz_weights(m, n, k, out):
     assert np.array_equal(bits(c), want)
 
 
+@pytest.mark.parametrize("m", [9, 200, 513, 729])
+@pytest.mark.parametrize("k,n", [(16, 256), (112, 264), (144, 1152), (1040, 280), (4304, 1160)])
+def test_w8a8_ragged_sizes_on_the_tile_kernels(m, k, n):
+    """The direct-to-LDS tiles with a last, partial K step and with columns that are no multiple of 16 (the last tile of
+    [k, n] weights moves left), K split or not, in all weight layouts; SwiGLU; a grouped matmul of the same sizes.
+    Integer sums are exact, the de-quantised outputs have the oracle's bits."""
+    announce("w8a8 ragged tiles", m, k, n)
+    rng = np.random.default_rng(m + 3 * k + n)
+    a, b = rand_i8(rng, (m, k)), rand_i8(rng, (k, n))
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.int64)
+    bt = np.ascontiguousarray(b.T)
+    for trans in (False, True):
+        c, _ = run_mm(m, n, k, a, bt if trans else b, out=torch.int32, trans_b=trans)
+        assert np.array_equal(c.cpu().numpy(), want)
+    cs = rng.uniform(1e-4, 1e-2, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    q, ts = orc.dynamic_quant_per_token(abi.BF16, bits(x))
+    d = abi.MatmulDesc(m=m, n=n, k=k, out_dtype=abi.BF16, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32,
+                       has_tok_scale=1, bias_kind=abi.MM_BIAS_F32_POST)
+    gold = orc.matmul_w8a8(d, q, b, bias, cs, ts)
+    d.activation, d.act_beta = abi.MM_ACT_SWIGLU, 1.0
+    gold_swiglu = orc.matmul_w8a8(d, q, b, bias, cs, ts).view(np.uint16)
+    for trans in (False, True):
+        w = to_dev(bt if trans else b)
+        c = torch.zeros((m, n), dtype=torch.bfloat16, device=DEV)
+        ops.linear_w8a8_dynamic(c, x, w, to_dev(cs), to_dev(bias), abi.MM_ACT_NONE, trans)
+        assert np.array_equal(bits(c), gold)
+        cg = torch.zeros((m, n // 2), dtype=torch.bfloat16, device=DEV)
+        ops.linear_w8a8_dynamic(cg, x, w, to_dev(cs), to_dev(bias), abi.MM_ACT_SWIGLU, trans)
+        swiglu_close(bits(cg), gold_swiglu, "bf16")
+    counts = [m // 3, 0, m - m // 3 - 1]
+    got, ref = run_group(m, k, n, counts, abi.GROUP_LIST_COUNTS, torch.bfloat16, rng, True, abi.MM_ACT_NONE)
+    assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("m", [129, 300, 600])
+@pytest.mark.parametrize("k,n", [(64, 40), (1472, 512), (5888, 520), (4096, 1024)])
+def test_linear_w8a8_dynamic_packed_split_over_k(m, k, n):
+    """Packed weights with too few tiles for the chip: K split over workgroups, the pieces in the call's workspace."""
+    announce("linear dynamic packed, K split", m, k, n)
+    rng = np.random.default_rng(m + k + n)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(DEV).to(torch.float16)
+    w = rand_i8(rng, (k, n))
+    cs = rng.uniform(1e-4, 1e-2, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device=DEV)
+    ops.linear_w8a8_dynamic_packed(c, x, ops.pack_weight_w8(to_dev(w), k, n), n, to_dev(cs), to_dev(bias))
+    q, ts = orc.dynamic_quant_per_token(abi.F16, bits(x))
+    d = abi.MatmulDesc(m=m, n=n, k=k, out_dtype=abi.BF16, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32,
+                       has_tok_scale=1, bias_kind=abi.MM_BIAS_F32_POST)
+    assert np.array_equal(bits(c), orc.matmul_w8a8(d, q, w, bias, cs, ts))
+
+
 @pytest.mark.parametrize("m,kernel", [(1, abi.MM_KERNEL_STREAM), (100, abi.MM_KERNEL_DMA_128),
                                       (700, abi.MM_KERNEL_DMA_256)])
 def test_matmul_plan_then_call(m, kernel):
