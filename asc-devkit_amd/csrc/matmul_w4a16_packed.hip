@@ -692,6 +692,64 @@ __global__ __launch_bounds__(kW * 64) void w4a16_packed_rows_kernel(W4pParams p)
     }
 }
 
+// The same repacking for n % 8 == 0 and dword-aligned weights, where a thread turns 32 k of 8 columns round: four 8 x 8
+// nibble transpositions in registers (exchanges of 16, 8 and 4 bits).  A workgroup reads 256-byte runs of 128 rows and
+// writes whole tiles.  It has to keep pace with memory, because a matmul on [k, n] weights with many rows repacks them
+// on every call.
+__global__ __launch_bounds__(256) void pack_w4_tiles_kernel(const uint32_t* __restrict__ w, u32x4* __restrict__ out, uint32_t k,
+                                                            uint32_t n, uint32_t slabs, uint32_t ktiles, uint32_t col_blocks)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    if (blockIdx.x >= col_blocks * ktiles) {  // padding behind the last slab: w = 0
+        const uint32_t i = (blockIdx.x - col_blocks * ktiles) * 256u + tid;
+        if (i < kPadTiles * 64u) {
+            out[static_cast<size_t>(slabs) * ktiles * 64u + i] = u32x4{0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u};
+        }
+        return;
+    }
+    const uint32_t tile = blockIdx.x / col_blocks, g = lane >> 4;
+    const uint32_t dcol = (blockIdx.x % col_blocks) * 64u + (tid >> 6) * 16u + (lane & 15u);  // dword of 8 columns
+    const uint32_t slab = dcol >> 1, row_dw = n / 8u, k0 = tile * kTileK + g * 32u;
+    if (slab >= slabs) {
+        return;
+    }
+    uint32_t q[32];
+#pragma unroll
+    for (uint32_t e = 0; e < 32u; ++e) {
+        q[e] = k0 + e < k && dcol < row_dw ? w[static_cast<size_t>(k0 + e) * row_dw + dcol] : 0u;
+    }
+    u32x4 v[8];
+#pragma unroll
+    for (uint32_t d = 0; d < 4u; ++d) {
+        // nibble p of a finished dword is k offset 2 p (p < 4) or 2 p - 7
+        uint32_t t[8];
+#pragma unroll
+        for (uint32_t p = 0; p < 8u; ++p) t[p] = q[8u * d + (p < 4u ? 2u * p : 2u * p - 7u)];
+#pragma unroll
+        for (uint32_t p = 0; p < 4u; ++p) {
+            const uint32_t a = t[p], b = t[p + 4u];
+            t[p] = (a & 0xFFFFu) | (b << 16);
+            t[p + 4u] = (a >> 16) | (b & 0xFFFF0000u);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            const uint32_t p = (i & 1u) | ((i & 2u) << 1);
+            const uint32_t a = t[p], b = t[p + 2u];
+            t[p] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+            t[p + 2u] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < 8u; p += 2u) {
+            const uint32_t a = t[p], b = t[p + 1u];
+            v[p][d] = ((a & 0x0F0F0F0Fu) | ((b << 4) & 0xF0F0F0F0u)) ^ 0x88888888u;
+            v[p + 1u][d] = (((a >> 4) & 0x0F0F0F0Fu) | (b & 0xF0F0F0F0u)) ^ 0x88888888u;
+        }
+    }
+    u32x4* const dst = out + (static_cast<size_t>(slab) * ktiles + tile) * 64u + 16u * g + 8u * (dcol & 1u);
+#pragma unroll
+    for (uint32_t c = 0; c < 8u; ++c) dst[c] = v[c];
+}
+
 // ND [k, n / 2] (even column in the low nibble, two's complement) -> packed; one thread per lane of a tile.
 __global__ __launch_bounds__(256) void pack_w4_kernel(const uint8_t* __restrict__ w, u32x4* __restrict__ out, uint32_t k,
                                                       uint32_t n, uint32_t slabs, uint32_t ktiles)
@@ -751,6 +809,12 @@ extern "C" int ascq_pack_weight_w4(const void* w, void* packed, uint32_t k, uint
     const uint32_t slabs = (n + kSlabCols - 1u) / kSlabCols, ktiles = (k + kTileK - 1u) / kTileK;
     const size_t lanes = (static_cast<size_t>(slabs) * ktiles + kPadTiles) * 64u;
     ASCQ_REQUIRE((lanes + 255u) / 256u < (1ull << 31), ASCQ_EINVAL, "ascq_pack_weight_w4: matrix too large");
+    if (n % 8u == 0 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0) {
+        const uint32_t col_blocks = (n / 8u + 63u) / 64u;
+        pack_w4_tiles_kernel<<<col_blocks * ktiles + (kPadTiles * 64u + 255u) / 256u, 256, 0, static_cast<hipStream_t>(stream)>>>(
+            static_cast<const uint32_t*>(w), static_cast<u32x4*>(packed), k, n, slabs, ktiles, col_blocks);
+        return launch_status("ascq_pack_weight_w4");
+    }
     pack_w4_kernel<<<static_cast<uint32_t>((lanes + 255u) / 256u), 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const uint8_t*>(w), static_cast<u32x4*>(packed), k, n, slabs, ktiles);
     return launch_status("ascq_pack_weight_w4");

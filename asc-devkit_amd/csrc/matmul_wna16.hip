@@ -1008,6 +1008,18 @@ bool fast_ok(const ascq_w4a16_desc* d, const void* x, const void* w, const void*
            static_cast<uint64_t>((d->n + kColsPerBlock - 1u) / kColsPerBlock) * (d->k / kChunkRows) < (1ull << 31);
 }
 
+// Many rows: the weights are packed into the workspace and the tile GEMM of the packed form runs on them, instead of a
+// pass over the weights per 32 rows: k = 5632, n = 1408, 1149 rows 1069 -> 68 us; k = 11648, n = 11520, 128 rows 179 ->
+// 142 us.  The line lies where the two meet at k = n = 8192 (96 rows 107 and 103 us; 65 rows 91 and 103 us).
+bool pack_first(const ascq_w4a16_desc* d)
+{
+    const uint32_t g32 = d->group_size / 32u;
+    size_t bytes = 0;
+    return d->m > 96u && d->k % 128u == 0 && d->n % 8u == 0 && d->group_size % 32u == 0 && (g32 & (g32 - 1u)) == 0 &&
+           ascq_pack_weight_w4_size(d->k, d->n, &bytes) == ASCQ_OK && bytes < (1ull << 31) &&
+           static_cast<uint64_t>(d->k / d->group_size) * d->n * 2u < (1ull << 31);
+}
+
 }  // namespace
 }  // namespace ascq
 
@@ -1034,6 +1046,10 @@ extern "C" int ascq_matmul_w4a16_workspace_size(const ascq_w4a16_desc* d, size_t
     if (d->k % kChunkRows == 0) {
         *bytes = workspace_need(d->n, d->k);
     }
+    size_t packed = 0;
+    if (pack_first(d) && ascq_pack_weight_w4_size(d->k, d->n, &packed) == ASCQ_OK && packed > *bytes) {
+        *bytes = packed;  // (a smaller workspace is accepted: the row kernels then pass over the weights)
+    }
     return ASCQ_OK;
 }
 
@@ -1048,6 +1064,18 @@ extern "C" int ascq_matmul_w4a16(const ascq_w4a16_desc* d, void* y, const void* 
     ASCQ_REQUIRE(y && x && w && scale, ASCQ_ENULL, "ascq_matmul_w4a16: y / x / w / scale is NULL");
     ASCQ_REQUIRE(!d->has_offset || offset, ASCQ_ENULL, "ascq_matmul_w4a16: offset is NULL");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    size_t packed = 0;
+    if (pack_first(d) && workspace != nullptr && aligned16(workspace) && aligned16(x) && aligned16(scale) &&
+        (!d->has_offset || aligned16(offset)) && ascq_pack_weight_w4_size(d->k, d->n, &packed) == ASCQ_OK &&
+        workspace_bytes >= packed) {
+        rc = ascq_pack_weight_w4(w, workspace, d->k, d->n, stream);
+        if (rc != ASCQ_OK) {
+            return rc;
+        }
+        ascq_w4a16_desc per_weight = *d;
+        per_weight.mode = ASCQ_W4A16_PER_WEIGHT;
+        return ascq_matmul_w4a16_packed(&per_weight, y, x, workspace, scale, offset, stream);
+    }
     WnParams p{};
     p.x = static_cast<const uint16_t*>(x);
     p.w = static_cast<const uint8_t*>(w);
