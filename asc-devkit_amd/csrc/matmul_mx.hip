@@ -12,8 +12,10 @@
 //   * 4-bit operands: registers 0-3 of lane l hold its row's k = 32 (l / 32) .. + 31 (16 bytes), scaled by the lane's
 //     own scale byte: one read per operand and instruction.
 //   * 6-bit operands (e2m3 codes, what two e1m2 operands are rewritten as): registers 0-5 of lane l hold its row's
-//     k = 32 (l / 32) .. + 31 as little-endian 6-bit fields (24 bytes, padded to 32 in memory), scaled by the lane's
-//     own scale byte: a 16-byte and an 8-byte read per operand and instruction.
+//     k = 32 (l / 32) .. + 31 as little-endian 6-bit fields (24 bytes), scaled by the lane's own scale byte: a 16-byte and
+//     an 8-byte read per operand and instruction, from units of 32 rows x 64 k in lane order.  (What bounds this form is
+//     the rate at which tiles reach the LDS: with each block of 32 k padded to 32 bytes m = n = k = 8192 took 419 us, both
+//     widening passes included, without the padding 365 us; 874 x 2000 x 8960 104 -> 73 us.)
 // In every case lane l needs scale byte 2 j + l / 32 of its row's bytes for this K step in sub-step j; a lane holds
 // the bytes of a K step as one dword (8- and 6-bit) or two (4-bit) per row, staged through LDS, and shifts them right
 // by 8 (l / 32) where they are used, so that the byte selector of the instruction is the constant 0 or 2.
@@ -56,13 +58,14 @@ constexpr uint32_t kMxScaleBuf = (kMxBM + kMxBN) * 16u;  // 16 scale bytes of ev
 template <bool kFour, int kCa, int kCb>
 __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
 {
-    __shared__ __attribute__((aligned(1024))) char A0[kMxBM * kMxBK];
-    __shared__ __attribute__((aligned(1024))) char B0[kMxBN * kMxBK];
-    __shared__ __attribute__((aligned(1024))) char A1[kMxBM * kMxBK];
-    __shared__ __attribute__((aligned(1024))) char B1[kMxBN * kMxBK];
-    __shared__ __attribute__((aligned(1024))) char SC[2 * kMxScaleBuf];  // two buffers of scale bytes, see below
     constexpr int TI = 4, TJ = 2;
-    constexpr bool kSix = !kFour && kCa == 2;  // e2m3 codes, the 24 bytes of every 32 values padded to 32
+    constexpr bool kSix = !kFour && kCa == 2;  // e2m3 codes in units of 32 rows x 64 k (mx_widen_e1m2_kernel)
+    constexpr uint32_t kRowBytes = kSix ? 96u : kMxBK;  // bytes of a row and K step in LDS
+    __shared__ __attribute__((aligned(1024))) char A0[kMxBM * kRowBytes];
+    __shared__ __attribute__((aligned(1024))) char B0[kMxBN * kRowBytes];
+    __shared__ __attribute__((aligned(1024))) char A1[kMxBM * kRowBytes];
+    __shared__ __attribute__((aligned(1024))) char B1[kMxBN * kRowBytes];
+    __shared__ __attribute__((aligned(1024))) char SC[2 * kMxScaleBuf];  // two buffers of scale bytes, see below
     static_assert(!kSix || kCb == 2, "6-bit operands come in pairs");
     constexpr int kSub = kFour ? 4 : 2;       // instructions (64 k each) per K step and block pair
     constexpr int kScaleDw = kFour ? 2 : 1;   // dwords of scale bytes per row and K step
@@ -95,11 +98,20 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
     const uint32_t RB = p.row_bytes;
 
     // ---- DMA sources: 4 A and 4 B instructions per wavefront and K step; lane owns LDS slot (instr * 64 + lane) of
-    // 16 bytes: row slot / 8, position slot % 8, which holds piece position ^ ((row / 2) % 8) of the row's 128 bytes
-    uint32_t aoff[4], boff[4];
+    // 16 bytes: row slot / 8, position slot % 8, which holds piece position ^ ((row / 2) % 8) of the row's 128 bytes.
+    // 6-bit operands: 3 and 3 instructions, the two units of a block of 32 rows as they lie in memory.
+    constexpr int kInstr = kSix ? 3 : 4;
+    uint32_t aoff[kInstr], boff[kInstr];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const uint32_t s = (wave * 4u + u) * 64u + lane;
+    for (int u = 0; u < kInstr; ++u) {
+        const uint32_t s = (wave * kInstr + u) * 64u + lane;
+        if constexpr (kSix) {
+            const uint32_t block = s / 192u, at = s % 192u * 16u;
+            const uint32_t a_last = (p.m + 31u) / 32u - 1u - row0 / 32u, b_last = (p.n + 31u) / 32u - 1u - n0 / 32u;
+            aoff[u] = (block < a_last ? block : a_last) * (RB * 24u) + at;
+            boff[u] = (block < b_last ? block : b_last) * (RB * 24u) + at;
+            continue;
+        }
         const uint32_t r = s >> 3, c = (s & 7u) ^ ((r >> 1) & 7u);
         uint32_t row = row0 + r, col = n0 + r;
         row = row < p.m ? row : p.m - 1u;  // rows and columns past the end are never stored: any valid one will do
@@ -107,8 +119,9 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         aoff[u] = (row - row0) * RB + 16u * c;
         boff[u] = (col - n0) * RB + 16u * c;
     }
-    const uint8_t* Abase = p.a + static_cast<size_t>(row0) * RB;
-    const uint8_t* Bbase = p.b + static_cast<size_t>(n0) * RB;
+    // (a block of 32 rows of 6-bit operands is RB / 64 units of 1536 bytes)
+    const uint8_t* Abase = p.a + (kSix ? static_cast<size_t>(row0 / 32u) * (RB * 24u) : static_cast<size_t>(row0) * RB);
+    const uint8_t* Bbase = p.b + (kSix ? static_cast<size_t>(n0 / 32u) * (RB * 24u) : static_cast<size_t>(n0) * RB);
     // A wavefront-uniform address, pinned to scalar registers: a load's address is then this base plus the lane's
     // 32-bit offset, which the load instruction adds itself (otherwise the compiler folds the lane's offset into
     // 64-bit per-lane addresses: twice the registers and an addition per load).
@@ -120,19 +133,19 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         return reinterpret_cast<const uint8_t*>((static_cast<uint64_t>(hi) << 32) | lo);
     };
     auto issue = [&](uint32_t k0, char* As, char* Bs) __attribute__((always_inline)) {
-        const uint8_t* ab = uniform(Abase + k0);
-        const uint8_t* bb = uniform(Bbase + k0);
+        const uint8_t* ab = uniform(Abase + (kSix ? k0 * 24u : k0));
+        const uint8_t* bb = uniform(Bbase + (kSix ? k0 * 24u : k0));
         // (re-materialised here: widened to 64 bits once, ahead of the loop, the offsets would no longer be seen as
         // 32-bit offsets where the loads are selected)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(aoff[u]), "+v"(boff[u]));
+        for (int u = 0; u < kInstr; ++u) asm volatile("" : "+v"(aoff[u]), "+v"(boff[u]));
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            __builtin_amdgcn_global_load_lds((gptr_t)(ab + aoff[u]), (lds_ptr_t)(As + (wave * 4u + u) * 1024u), 16, 0, 0);
+        for (int u = 0; u < kInstr; ++u) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(ab + aoff[u]), (lds_ptr_t)(As + (wave * kInstr + u) * 1024u), 16, 0, 0);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            __builtin_amdgcn_global_load_lds((gptr_t)(bb + boff[u]), (lds_ptr_t)(Bs + (wave * 4u + u) * 1024u), 16, 0, 0);
+        for (int u = 0; u < kInstr; ++u) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(bb + boff[u]), (lds_ptr_t)(Bs + (wave * kInstr + u) * 1024u), 16, 0, 0);
         }
     };
 
@@ -211,20 +224,26 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
     // ---- fragments: piece q of tile line r sits at r * 128 + ((q ^ ((r / 2) % 8)) * 16).  A lane reads piece
     // kPieceStep u + h (+ 2 for the upper registers of an 8-bit operand) of a line whose number is lrow + a multiple
     // of 32, i.e. at lrow * 128 + (((kPieceStep u) ^ (h ^ swizzle)) * 16) + constants: one register per u.
-    // (6-bit operands, 24 bytes per lane: pieces 4 s + 2 h and the first half of 4 s + 2 h + 1, u = 2 s and 2 s + 1)
+    // (6-bit operands: the lane's 16 bytes of a unit at 16 l, its other 8 at 1024 + 8 l)
     constexpr int kPieceStep = 2;
-    constexpr int kPieces = 4;   // u = 0 .. 3: pieces 0 2 4 6 (+ h)
+    constexpr int kPieces = kSix ? 2 : 4;   // u = 0 .. 3: pieces 0 2 4 6 (+ h)
     uint32_t foff[kPieces];
 #pragma unroll
     for (int u = 0; u < kPieces; ++u) {
-        const uint32_t piece = kSix ? 4u * (u >> 1) + 2u * h + (u & 1) : static_cast<uint32_t>(kPieceStep * u) ^ h;
-        foff[u] = lrow * 128u + ((piece ^ ((lrow >> 1) & 7u)) << 4);
-        if (kSix && (u & 1)) {
-            foff[u] += 8u * (lrow & 1u);  // odd rows keep these 8 bytes in the piece's second half
-        }
+        foff[u] = kSix ? (u == 0 ? lane * 16u : 1024u + lane * 8u)
+                       : lrow * 128u + (((static_cast<uint32_t>(kPieceStep * u) ^ h ^ ((lrow >> 1) & 7u))) << 4);
     }
     auto frag = [&](const char* S, uint32_t line0, int u) __attribute__((always_inline)) {
         return *reinterpret_cast<const i32x4*>(S + line0 * 128u + foff[u]);
+    };
+    auto frag_six = [&](const char* S, uint32_t block, int s) __attribute__((always_inline)) {
+        const char* unit = S + block * 3072u + s * 1536u;
+        const i32x4 lo = *reinterpret_cast<const i32x4*>(unit + foff[0]);
+        const i32x2_t hi = *reinterpret_cast<const i32x2_t*>(unit + foff[1]);
+        v8i t = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 6 registers
+        t[4] = hi[0];
+        t[5] = hi[1];
+        return t;
     };
     struct Frags {
         v8i a[TI], b[TJ];
@@ -238,12 +257,7 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
                 const i32x4 lo = frag(As, line0, s);
                 f.a[i] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 4 registers of a 4-bit operand
             } else if constexpr (kSix) {
-                const i32x4 lo = frag(As, line0, 2 * s);
-                const i32x2_t hi = *reinterpret_cast<const i32x2_t*>(As + line0 * 128u + foff[2 * s + 1]);
-                v8i t = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 6 registers
-                t[4] = hi[0];
-                t[5] = hi[1];
-                f.a[i] = t;
+                f.a[i] = frag_six(As, line0 / 32u, s);
             } else {
                 const i32x4 lo = frag(As, line0, 2 * s), hi = frag(As, line0, 2 * s + 1);
                 f.a[i] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -256,12 +270,7 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
                 const i32x4 lo = frag(Bs, line0, s);
                 f.b[j] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);
             } else if constexpr (kSix) {
-                const i32x4 lo = frag(Bs, line0, 2 * s);
-                const i32x2_t hi = *reinterpret_cast<const i32x2_t*>(Bs + line0 * 128u + foff[2 * s + 1]);
-                v8i t = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 6 registers
-                t[4] = hi[0];
-                t[5] = hi[1];
-                f.b[j] = t;
+                f.b[j] = frag_six(Bs, line0 / 32u, s);
             } else {
                 const i32x4 lo = frag(Bs, line0, 2 * s), hi = frag(Bs, line0, 2 * s + 1);
                 f.b[j] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -511,35 +520,45 @@ __global__ __launch_bounds__(256) void mx_widen_fp4_kernel(const u32x4* __restri
     }
 }
 
-// e1m2 [rows, k / 2 bytes] -> e2m3 codes, 32 values as 24 bytes (little-endian 6-bit fields, the layout the matrix
-// instruction reads from a lane's six registers) followed by 8 unused bytes, so that a row is k bytes like an 8-bit
-// operand's.  An e1m2 value is +-(code / 4), code 0 .. 7, which is the e2m3 value with magnitude bits 2 * code (its
-// subnormals run 0, 1/8 .. 7/8 and its first binade 1, 9/8 .. 15/8).
-// The last 8 of the 24 bytes sit in the first half of the second 16-byte piece in even rows and in its second half in
-// odd rows: an 8-byte LDS read is served 16 lanes at a time, a row and its neighbour keep their pieces at the same
-// position of their 128-byte lines, and the two would meet in the same banks.
-__global__ __launch_bounds__(256) void mx_widen_e1m2_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
-                                                            size_t pieces, uint32_t pieces_per_row)
+// e1m2 [rows, k / 2 bytes] -> e2m3 codes in units of 32 rows x 64 k, k innermost: 1024 bytes that hold bytes 0 - 15 and
+// 512 that hold bytes 16 - 23 of the 24 a lane of the matrix instruction owns (its row's 32 consecutive k as little-endian
+// 6-bit fields), in lane order.  So the tiles of the matmul are contiguous runs, a lane's operand two LDS reads without
+// bank conflicts, and 96 bytes of a row travel per 128 k.  An e1m2 value is +-(code / 4), code 0 .. 7, which is the e2m3 value with magnitude
+// bits 2 * code (its subnormals run 0, 1/8 .. 7/8 and its first binade 1, 9/8 .. 15/8).  Both operands in one launch: a
+// workgroup takes 32 rows x 256 k, whole 128-byte lines of the source.
+struct MxWidenParams {
+    const uint8_t* src[2];
+    uint8_t* dst[2];
+    uint32_t rows[2];
+    uint32_t a_blocks, k_blocks, k;  // workgroups of the first operand; workgroups per block of 32 rows
+};
+
+__global__ __launch_bounds__(256) void mx_widen_e1m2_kernel(MxWidenParams p)
 {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256u + threadIdx.x; i < pieces; i += static_cast<size_t>(gridDim.x) * 256u) {
-        const u32x4 q = __builtin_nontemporal_load(src + i);  // 32 values, value v of a dword in bits 4 v .. 4 v + 3
-        uint64_t c[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            uint64_t t = q[d];
-            t = (t & 0xFFFFull) | ((t & 0xFFFF0000ull) << 8);                              // values 0-3 | 4-7, 24 bits each
-            t = (t & 0x00000000FF0000FFull) | ((t & 0x000000FF0000FF00ull) << 4);          // pairs, 12 bits each
-            t = (t & 0x00000F00F00F00Full) | ((t & 0x0000F00F00F00F0ull) << 2);            // value v in bits 6 v .. 6 v + 3
-            c[d] = ((t & 0x0000208208208208ull) << 2) | ((t & 0x00001C71C71C71C7ull) << 1);  // sign to bit 5, magnitude doubled
-        }
-        const u32x4 lo = {static_cast<uint32_t>(c[0]), static_cast<uint32_t>(c[0] >> 32) | (static_cast<uint32_t>(c[1]) << 16),
-                          static_cast<uint32_t>(c[1] >> 16), static_cast<uint32_t>(c[2])};
-        const uint32_t w4 = static_cast<uint32_t>(c[2] >> 32) | (static_cast<uint32_t>(c[3]) << 16);
-        const uint32_t w5 = static_cast<uint32_t>(c[3] >> 16);
-        const bool upper = ((i / pieces_per_row) & 1u) != 0;
-        dst[2 * i] = lo;
-        dst[2 * i + 1] = upper ? u32x4{0u, 0u, w4, w5} : u32x4{w4, w5, 0u, 0u};
+    const uint32_t which = blockIdx.x < p.a_blocks ? 0u : 1u;
+    const uint32_t id = blockIdx.x - (which ? p.a_blocks : 0u);
+    const uint32_t lane = threadIdx.x & 63u, unit = (id % p.k_blocks) * 4u + (threadIdx.x >> 6), block = id / p.k_blocks;
+    if (unit >= p.k / 64u) {
+        return;
     }
+    uint32_t row = block * 32u + (lane & 31u);
+    row = row < p.rows[which] ? row : p.rows[which] - 1u;  // (rows past the end are never stored by the matmul)
+    const u32x4 q = *reinterpret_cast<const u32x4*>(p.src[which] + static_cast<size_t>(row) * (p.k / 2u) + unit * 32u + (lane >> 5) * 16u);
+    uint64_t c[4];  // 32 values, value v of a dword in bits 4 v .. 4 v + 3
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        uint64_t t = q[d];
+        t = (t & 0xFFFFull) | ((t & 0xFFFF0000ull) << 8);                              // values 0-3 | 4-7, 24 bits each
+        t = (t & 0x00000000FF0000FFull) | ((t & 0x000000FF0000FF00ull) << 4);          // pairs, 12 bits each
+        t = (t & 0x00000F00F00F00Full) | ((t & 0x0000F00F00F00F0ull) << 2);            // value v in bits 6 v .. 6 v + 3
+        c[d] = ((t & 0x0000208208208208ull) << 2) | ((t & 0x00001C71C71C71C7ull) << 1);  // sign to bit 5, magnitude doubled
+    }
+    uint8_t* const out = p.dst[which] + (static_cast<size_t>(block) * (p.k / 64u) + unit) * 1536u;
+    *reinterpret_cast<u32x4*>(out + lane * 16u) =
+        u32x4{static_cast<uint32_t>(c[0]), static_cast<uint32_t>(c[0] >> 32) | (static_cast<uint32_t>(c[1]) << 16),
+              static_cast<uint32_t>(c[1] >> 16), static_cast<uint32_t>(c[2])};
+    *reinterpret_cast<u32x2*>(out + 1024u + lane * 8u) =
+        u32x2{static_cast<uint32_t>(c[2] >> 32) | (static_cast<uint32_t>(c[3]) << 16), static_cast<uint32_t>(c[3] >> 16)};
 }
 
 inline bool is_fp8(int f) { return f == ASCQ_QDST_FP8_E4M3FN || f == ASCQ_QDST_FP8_E5M2; }
@@ -558,6 +577,11 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     bool wa, wb;
     mx_widen_plan(d, wa, wb);
     const bool four = is_fp4(d->a_format) && !wa;  // both e2m1
+    // two e1m2 operands: the 6-bit codes of rows rounded up to 32 must fit the workspace of a byte per value
+    auto fits = [](uint32_t rows) { return (static_cast<uint64_t>(rows) + 31u) / 32u * 24u <= rows; };
+    if (d->a_format == ASCQ_QDST_FP4_E1M2 && d->b_format == ASCQ_QDST_FP4_E1M2 && !(fits(d->m) && fits(d->n))) {
+        return false;
+    }
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
 }
 
@@ -673,21 +697,23 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         const size_t pieces = rows * (d->k / 2u) / 16u;  // k is a multiple of 128 here
         size_t blocks = (pieces + 255u) / 256u;
         if (blocks > 65536u) blocks = 65536u;
-        if (six) {
-            mx_widen_e1m2_kernel<<<static_cast<uint32_t>(blocks), 256, 0, st>>>(reinterpret_cast<const u32x4*>(src),
-                                                                               reinterpret_cast<u32x4*>(ws), pieces, d->k / 32u);
-        } else {
-            mx_widen_fp4_kernel<<<static_cast<uint32_t>(blocks), 256, 0, st>>>(reinterpret_cast<const u32x4*>(src),
-                                                                              reinterpret_cast<u32x4*>(ws), pieces, fmt);
-        }
+        mx_widen_fp4_kernel<<<static_cast<uint32_t>(blocks), 256, 0, st>>>(reinterpret_cast<const u32x4*>(src),
+                                                                          reinterpret_cast<u32x4*>(ws), pieces, fmt);
         src = ws;
         ws += rows * d->k;
         fmt = ASCQ_QDST_FP8_E4M3FN;
     };
-    if (wa) {
+    if (six) {
+        MxWidenParams w{{p.a, p.b}, {ws, ws + static_cast<size_t>(d->m) * d->k}, {d->m, d->n}, 0, (d->k + 255u) / 256u, d->k};
+        w.a_blocks = (d->m + 31u) / 32u * w.k_blocks;
+        mx_widen_e1m2_kernel<<<w.a_blocks + (d->n + 31u) / 32u * w.k_blocks, 256, 0, st>>>(w);
+        p.a = w.dst[0];
+        p.b = w.dst[1];
+        fa = fb = ASCQ_QDST_FP8_E4M3FN;  // (a byte per value as far as the sizes below go)
+    } else if (wa) {
         widen(p.a, fa, d->m);
     }
-    if (wb) {
+    if (wb && !six) {
         widen(p.b, fb, d->n);
     }
     const bool four = is_fp4(fa);  // (after the widening: both e2m1)
