@@ -456,6 +456,99 @@ typedef Tile<2, 4, 2, 2, true> TileMT;
 typedef Tile<1, 2, 1, 4, false> TileS;   // 32 x 256, split-K
 typedef Tile<1, 2, 1, 4, true> TileST;
 
+// [k, n] weights whose rows start at any byte (n no multiple of 8: a vocabulary with added tokens), up to 32 rows.  What
+// bounds it is the weights' trip from memory, so they come as unaligned dwords, a wavefront reading 256 neighbouring columns
+// of a row; four rows of k are turned round in registers (8 byte permutes) into one dword of 4 k per column, which meets
+// the activations' scalar dwords in v_dot4_i32_i8.  A workgroup's 8 wavefronts split its range of k and are added in LDS;
+// workgroups along k add into the zeroed workspace.  4 rows, k = 6784, n = 5805: 1930 us with one lane per output
+// element, 27 us now (32 rows, k = 4096, n = 32003: 2854 and 129 us).
+constexpr uint32_t kOddCols = 256, kOddWaves = 8;
+
+template <int R>
+__global__ __launch_bounds__(kOddWaves * 64) void gemm_odd_kernel(GemmParams p)
+{
+    __shared__ i32x4 sums[kOddWaves][4][64];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col = blockIdx.x * kOddCols + 4u * lane;
+    const uint32_t units = p.k / 16u, parts = gridDim.y * kOddWaves, part = blockIdx.y * kOddWaves + wave;
+    const uint32_t begin = static_cast<uint32_t>(static_cast<uint64_t>(units) * part / parts);
+    const uint32_t end = static_cast<uint32_t>(static_cast<uint64_t>(units) * (part + 1u) / parts);
+    const uint64_t last = static_cast<uint64_t>(p.k) * p.n - 4u;  // of the addresses that start a whole dword
+    i32x4 acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = i32x4{0, 0, 0, 0};
+    // columns past the end run on into the next row (never stored); at the matrix's end the dword is moved back
+    auto fetch = [&](uint32_t k, auto inside) __attribute__((always_inline)) {
+        const uint64_t at = static_cast<uint64_t>(k) * p.n + col;
+        uint32_t v;
+        if constexpr (decltype(inside)::value) {
+            __builtin_memcpy(&v, p.b + static_cast<uint64_t>(k) * p.n + col, 4);
+            return v;
+        }
+        __builtin_memcpy(&v, p.b + (at < last ? at : last), 4);
+        const uint64_t past = at > last ? at - last : 0u;
+        return past < 4u ? v >> (8u * static_cast<uint32_t>(past)) : 0u;
+    };
+    // QN dwords of k from k0: all of them are requested before the first is used
+    auto run = [&](uint32_t k0, auto count, auto inside) __attribute__((always_inline)) {
+        constexpr int QN = decltype(count)::value;
+        uint32_t w[4 * QN], c[4 * QN];
+#pragma unroll
+        for (int i = 0; i < 4 * QN; ++i) w[i] = fetch(k0 + i, inside);
+#pragma unroll
+        for (int q = 0; q < QN; ++q) {
+            const uint32_t* v = w + 4 * q;
+            const uint32_t t0 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u), t1 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u);
+            const uint32_t t2 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u), t3 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
+            c[4 * q] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+            c[4 * q + 1] = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
+            c[4 * q + 2] = __builtin_amdgcn_perm(t3, t2, 0x05040100u);
+            c[4 * q + 3] = __builtin_amdgcn_perm(t3, t2, 0x07060302u);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t row = static_cast<uint32_t>(r) < p.m ? r : p.m - 1u;
+            int x[QN];
+            __builtin_memcpy(x, __builtin_assume_aligned(p.a + static_cast<size_t>(row) * p.k + k0, 4), sizeof(x));
+#pragma unroll
+            for (int q = 0; q < QN; ++q) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[r][j] = __builtin_amdgcn_sdot4(static_cast<int>(c[4 * q + j]), x[q], acc[r][j], false);
+            }
+        }
+    };
+    const uint64_t block_end = static_cast<uint64_t>(blockIdx.x) * kOddCols + kOddCols - 4u;
+    for (uint32_t u = begin; u < end; ++u) {
+        if ((16u * u + 15u) * static_cast<uint64_t>(p.n) + block_end <= last) {  // (the same for the whole workgroup)
+            run(16u * u, std::integral_constant<int, 4>{}, std::true_type{});
+        } else {
+            run(16u * u, std::integral_constant<int, 4>{}, std::false_type{});
+        }
+    }
+    if (part == parts - 1u) {  // what is left of k
+        for (uint32_t k = 16u * units; k < p.k; k += 4u) run(k, std::integral_constant<int, 1>{}, std::false_type{});
+    }
+#pragma unroll
+    for (int r0 = 0; r0 < R; r0 += 4) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[wave][r][lane] = acc[r0 + r];
+        __syncthreads();
+        if (threadIdx.x < 256u) {
+            const uint32_t r = threadIdx.x >> 6, row = r0 + r;
+            i32x4 s = sums[0][r][lane];
+#pragma unroll
+            for (uint32_t o = 1; o < kOddWaves; ++o) s += sums[o][r][lane];
+            if (row < p.m) {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    if (col + j < p.n) atomicAdd(&p.partial[static_cast<size_t>(row) * p.n + col + j], s[j]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
 template <class K>
 int set_lds(K kernel, int bytes)
 {
@@ -780,6 +873,44 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
         p.b_nz = 1;
         return d->m <= kSkinnyMaxM ? launch_gemm_dma_skinny(p, workspace, workspace_bytes, st)
                                    : launch_gemm_dma(p, false, st);
+    }
+    if (!fast_path_ok(d, a, b) && d->m <= 32u && !d->trans_a && !d->trans_b && d->n >= 64u && d->k % 4u == 0 && d->k >= 128u &&
+        (reinterpret_cast<uintptr_t>(a) & 3u) == 0 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 3u) == 0 &&
+        workspace_bytes >= static_cast<size_t>(d->m) * d->n * sizeof(int32_t)) {
+        // about 16 wavefronts per compute unit, each with at least 32 of k
+        const uint32_t cols = (d->n + kOddCols - 1u) / kOddCols;
+        uint32_t parts = (2u * device_compute_units() + cols - 1u) / cols;
+        const uint32_t most = d->k / (32u * kOddWaves);
+        parts = parts < most ? parts : most;
+        const dim3 grid(cols, parts ? parts : 1u);
+        p.partial = static_cast<int32_t*>(workspace);
+        const size_t need = static_cast<size_t>(d->m) * d->n * sizeof(int32_t);
+        if (plan_note(ASCQ_MM_KERNEL_GENERIC, 32, kOddCols, 4, grid.x * grid.y, grid.y, kOddWaves * 4096u, need)) {
+            plan_note(0, 0, 0, 0, 0, 0, 0, 0);  // the zero fill ...
+            plan_note(0, 0, 0, 0, 0, 0, 0, 0);  // ... and the epilogue kernel
+            return ASCQ_OK;
+        }
+        rc = ascq_zero_fill(workspace, need, stream);
+        if (rc != ASCQ_OK) {
+            return rc;
+        }
+        if (d->m <= 4u) {
+            gemm_odd_kernel<4><<<grid, kOddWaves * 64u, 0, st>>>(p);
+        } else if (d->m <= 8u) {
+            gemm_odd_kernel<8><<<grid, kOddWaves * 64u, 0, st>>>(p);
+        } else if (d->m <= 16u) {
+            gemm_odd_kernel<16><<<grid, kOddWaves * 64u, 0, st>>>(p);
+        } else {
+            gemm_odd_kernel<32><<<grid, kOddWaves * 64u, 0, st>>>(p);
+        }
+        rc = launch_status("ascq_matmul_w8a8 (unaligned columns)");
+        if (rc != ASCQ_OK) {
+            return rc;
+        }
+        size_t blocks = (static_cast<size_t>(d->m) * d->n + kThreads - 1) / kThreads;
+        if (blocks > 4096) blocks = 4096;
+        splitk_epilogue_kernel<<<static_cast<uint32_t>(blocks), kThreads, 0, st>>>(p);
+        return launch_status("ascq_matmul_w8a8 (unaligned columns, epilogue)");
     }
     if (!fast_path_ok(d, a, b)) {
         size_t total = static_cast<size_t>(d->m) * d->n;

@@ -728,6 +728,29 @@ def test_w4a16_packed_many_rows(m, k, n, gs, offset):
         w4_check(np.ascontiguousarray(y.cpu().numpy()[:, c0:c1]), np.ascontiguousarray(want), x)
 
 
+@pytest.mark.parametrize("m,k,n,gs", [(97, 128, 8, 32), (98, 384, 40, 128), (130, 256, 528, 64), (200, 640, 1032, 128)])
+@pytest.mark.parametrize("offset", [True, False])
+def test_w4a16_many_rows_packs_the_weights_first(m, k, n, gs, offset):
+    """More than 96 rows on [k, n] weights: the call packs them into its workspace and runs the packed form's tile GEMM,
+    whose bits it has; a workspace that only holds the row kernels' pieces is still accepted."""
+    announce("w4a16 many rows", m, k, n, gs, offset)
+    rng = np.random.default_rng(m + k + n)
+    x, wp, sc, of = w4_case(rng, m, k, n, gs, offset)
+    d = abi.W4A16Desc(m=m, n=n, k=k, group_size=gs, has_offset=int(offset))
+    want = orc.matmul_w4a16(d, x, wp, sc, of)
+    xd, wd, sd, od = to_dev(x), to_dev(wp), to_dev(sc), None if of is None else to_dev(of)
+    y, yp = (torch.zeros((m, n), dtype=torch.float16, device=DEV) for _ in range(2))
+    ops.matmul_w4a16(y, xd, wd, sd, od, gs)
+    w4_check(y.cpu().numpy(), want, x)
+    ops.matmul_w4a16_packed(yp, xd, ops.pack_weight_w4(wd, k, n), sd, od, gs)
+    assert torch.equal(y.view(torch.int16), yp.view(torch.int16))
+    d.m = 32
+    need = C.c_size_t(0)
+    abi.check(abi.load_library().ascq_matmul_w4a16_workspace_size(C.byref(d), C.byref(need)))
+    ops.matmul_w4a16(y, xd, wd, sd, od, gs, workspace=torch.zeros(max(need.value // 4, 4), dtype=torch.float32, device=DEV))
+    w4_check(y.cpu().numpy(), want, x)
+
+
 def config4_columns(m, n):
     """The oracle covers every column at M=1 (about 6 s on 16 threads); for more rows three slabs: the first and the last
     512 columns (the kernels' first and last column blocks) and one from the middle."""
@@ -1148,6 +1171,26 @@ def test_w8a8_ragged_sizes_on_the_tile_kernels(m, k, n):
     counts = [m // 3, 0, m - m // 3 - 1]
     got, ref = run_group(m, k, n, counts, abi.GROUP_LIST_COUNTS, torch.bfloat16, rng, True, abi.MM_ACT_NONE)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("k,n", [(128, 65), (132, 257), (1000, 1023), (6784, 515), (512, 2050)])
+def test_w8a8_few_rows_on_unaligned_columns(m, k, n):
+    """[k, n] weights whose rows start at any byte: int32 sums, and the linear's bits against the oracle."""
+    announce("w8a8 unaligned columns", m, k, n)
+    rng = np.random.default_rng(m + 5 * k + n)
+    a, b = rand_i8(rng, (m, k)), rand_i8(rng, (k, n))
+    c, _ = run_mm(m, n, k, a, b, out=torch.int32)
+    assert np.array_equal(c.cpu().numpy(), a.astype(np.int64) @ b.astype(np.int64))
+    cs = rng.uniform(1e-4, 1e-2, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device=DEV)
+    ops.linear_w8a8_dynamic(c, x, to_dev(b), to_dev(cs), to_dev(bias))
+    q, ts = orc.dynamic_quant_per_token(abi.BF16, bits(x))
+    d = abi.MatmulDesc(m=m, n=n, k=k, out_dtype=abi.BF16, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32,
+                       has_tok_scale=1, bias_kind=abi.MM_BIAS_F32_POST)
+    assert np.array_equal(bits(c), orc.matmul_w8a8(d, q, b, bias, cs, ts))
 
 
 @pytest.mark.parametrize("m", [129, 300, 600])

@@ -102,6 +102,19 @@ def test_mx_tile_kernel_scale_rows(m, n, k, sk, fa, fb):
     mx_check(run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, fa, fb), is8(fa, fb))
 
 
+@pytest.mark.parametrize("m,n,k", [(8200, 1100, 128), (4100, 1128, 384), (4129, 1033, 640), (4096, 1056, 1024)])
+def test_mx_e1m2_pairs_on_the_tile_kernel(m, n, k):
+    """Enough rows for two e1m2 operands to be widened into units of 32 rows x 64 k: one K step, odd and even numbers of
+    them, a widening workgroup that is only partly used, rows and columns that end inside a unit."""
+    announce("mx e1m2 tiles", m, n, k)
+    rng = np.random.default_rng(m + n + k)
+    a, b, sa, sb, _ = mx_case(rng, m, n, k, F1, F1, sk=max(16, (k // 32 + 7) // 8 * 8))
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sa.shape[1], a_format=F1, b_format=F1, out_dtype=abi.F32, has_bias=0)
+    orc.set_threads(16)
+    want = orc.matmul_mx(d, a, b, sa, sb)
+    mx_check(run_mx(m, n, k, a, b, sa, sb, F1, F1).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, F1, F1), False)
+
+
 @pytest.mark.parametrize("fa,fb", [(a, b) for a in (E4, E5, F2, F1) for b in (E4, E5, F2, F1)])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 40, 160), (16, 33, 1088), (17, 64, 640), (32, 4112, 256), (33, 100, 2304),
                                    (64, 48, 4096), (65, 32, 1056)])
