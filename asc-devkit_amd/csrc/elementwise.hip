@@ -587,100 +587,6 @@ __device__ __forceinline__ float antiquant_one(float w, float s, float o, bool h
     return Fmt<kCt>::mul(s, t);
 }
 
-// One lane = 16 consecutive source elements of a row (16 bytes of int8 or 8 bytes of int4), 32 bytes of output.
-// cols % 16 == 0; in the transposed layout additionally group_size % 16 == 0 so that one parameter covers the lane.
-template <int kSrc, int kDst>
-__global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a)
-{
-    const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 16u;
-    if (j >= a.cols) {
-        return;
-    }
-    float s[16], o[16];
-    uint32_t cached_group = 0xFFFFFFFFu;
-    for (uint32_t r0 = blockIdx.y * kRowsInFlight; r0 < a.rows; r0 += gridDim.y * kRowsInFlight) {
-        u32x4 raw[kRowsInFlight];
-#pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
-            if (r0 + u < a.rows) {
-                const size_t e = static_cast<size_t>(r0 + u) * a.cols + j;
-                if constexpr (kSrc == ASCQ_I8) {
-                    raw[u] = *reinterpret_cast<const u32x4*>(static_cast<const int8_t*>(a.src) + e);
-                } else {
-                    u32x2 t = *reinterpret_cast<const u32x2*>(static_cast<const uint8_t*>(a.src) + e / 2);
-                    raw[u] = u32x4{t[0], t[1], 0u, 0u};
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
-            const uint32_t r = r0 + u;
-            if (r >= a.rows) {
-                break;
-            }
-            // parameters: a [groups, cols] row (not transposed) or one scalar per (row, group) (transposed)
-            const uint32_t g = a.per_tensor ? 0u : (a.transpose ? r * a.groups + j / a.group_size : r / a.group_size);
-            if (g != cached_group) {
-                cached_group = g;
-                if (a.per_tensor) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        s[e] = a.sscale;
-                        o[e] = a.soffset;
-                    }
-                } else if (a.transpose) {
-                    const float sv = load1<kDst>(a.scale, g);
-                    const float ov = a.has_offset ? load1<kDst>(a.offset, g) : 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        s[e] = sv;
-                        o[e] = ov;
-                    }
-                } else {
-                    const size_t pi = static_cast<size_t>(g) * a.cols + j;
-                    float t0[8], t1[8];
-                    load8<kDst>(a.scale, pi, t0);
-                    load8<kDst>(a.scale, pi + 8, t1);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        s[e] = t0[e];
-                        s[8 + e] = t1[e];
-                    }
-                    if (a.has_offset) {
-                        load8<kDst>(a.offset, pi, t0);
-                        load8<kDst>(a.offset, pi + 8, t1);
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            o[e] = t0[e];
-                            o[8 + e] = t1[e];
-                        }
-                    }
-                }
-            }
-            float y0[8], y1[8];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                int w;
-                if constexpr (kSrc == ASCQ_I8) {
-                    w = static_cast<int>(static_cast<int8_t>((raw[u][e >> 2] >> (8 * (e & 3))) & 0xFFu));
-                } else {
-                    const uint32_t nib = (raw[u][e >> 3] >> (4 * (e & 7))) & 0xFu;
-                    w = static_cast<int>(nib ^ 8u) - 8;
-                }
-                const float v = antiquant_one<kDst>(static_cast<float>(w), s[e], o[e], a.has_offset != 0);
-                if (e < 8) {
-                    y0[e] = v;
-                } else {
-                    y1[e - 8] = v;
-                }
-            }
-            const size_t oe = static_cast<size_t>(r) * a.cols + j;
-            store8<kDst, true>(a.dst, oe, y0);
-            store8<kDst, true>(a.dst, oe + 8, y1);
-        }
-    }
-}
-
 template <int kSrc, int kDst>
 __global__ __launch_bounds__(kThreads) void antiquant_scalar_kernel(AntiQuantArgs a)
 {
@@ -708,32 +614,45 @@ __global__ __launch_bounds__(kThreads) void antiquant_scalar_kernel(AntiQuantArg
     }
 }
 
-// Fast path int8 -> half, [k, n] layout: bytes become halves through the exponent trick (0x6400 | (b ^ 0x80) is
-// 1024 + b + 128, minus 1152 is b, both exact), then one rounded packed add of the offset and one rounded packed
-// multiply by the scale: about 2.5 VALU operations per element.
-template <bool kHasOffset>
-__global__ __launch_bounds__(kThreads) void antiquant_i8_f16_fast_kernel(AntiQuantArgs a)
+// One lane = 8 consecutive elements of a row: 8 (int8) or 4 (int4) bytes in, one 16-byte store out, so that every store
+// instruction of a wavefront writes 1 KiB of consecutive bytes, 8 rows in flight.  cols % 16 == 0; in the transposed layout
+// additionally group_size % 16 == 0, so that one parameter covers the lane.  The block size is chosen by the host so that the
+// last block of a row is as full as possible.  Memory bounds it: int4 4096 x 11008 to half with a row of parameters per
+// 128 k, 113 MB, 44.0 us with 16 elements per lane (two stores half a line apart, one conversion per element), 22.6 us now.
+// Half outputs: codes become halves through the exponent trick (0x6400 | u is 1024 + u; u = w + 128 or w + 8, taken off
+// again, all exact), then one rounded packed add of the offset and one rounded packed multiply by the scale: about 2.5
+// VALU operations per element.
+template <int kSrc, int kDst, bool kHasOffset, bool kTranspose>
+__global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a)
 {
-    // one lane = 8 columns: 8 bytes in, one 16-byte store out, so that every store instruction of a wavefront writes
-    // 1 KiB of consecutive bytes.  The block size is chosen by the host so that the last block of a row is as full
-    // as possible.
     const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
     if (j >= a.cols) {
         return;
     }
     constexpr int kRows = 2 * kRowsInFlight;
-    const f16x2 k1152 = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
-    f16x2 s[4], o[4];
+    constexpr bool kHalf = kDst == ASCQ_F16;
+    const half_t bias = static_cast<half_t>(kSrc == ASCQ_I8 ? 1152.0f : 1032.0f);
+    f16x2 s[4], o[4];      // half outputs: parameters of column pairs
+    float sf[8], of[8];    // bfloat16 outputs
     uint32_t cached_group = 0xFFFFFFFFu;
-    const int8_t* src = static_cast<const int8_t*>(a.src);
-    uint16_t* dst = static_cast<uint16_t*>(a.dst);
+    const uint32_t jg = kTranspose ? j / a.group_size : 0u;
     for (uint32_t r0 = blockIdx.y * kRows; r0 < a.rows; r0 += gridDim.y * kRows) {
         u32x2 raw[kRows];
+        uint32_t sr[kRows], orr[kRows];  // transposed: the parameters of the rows (a register each: no load waits for another)
 #pragma unroll
         for (int u = 0; u < kRows; ++u) {
             if (r0 + u < a.rows) {
-                raw[u] = __builtin_nontemporal_load(
-                    reinterpret_cast<const u32x2*>(src + static_cast<size_t>(r0 + u) * a.cols + j));
+                const size_t e = static_cast<size_t>(r0 + u) * a.cols + j;
+                if constexpr (kSrc == ASCQ_I8) {
+                    raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const int8_t*>(a.src) + e));
+                } else {
+                    raw[u][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(a.src) + e / 2u));
+                }
+                if (kTranspose && !a.per_tensor) {
+                    const size_t pi = static_cast<size_t>(r0 + u) * a.groups + jg;
+                    sr[u] = static_cast<const uint16_t*>(a.scale)[pi];
+                    orr[u] = kHasOffset ? static_cast<const uint16_t*>(a.offset)[pi] : 0u;
+                }
             }
         }
 #pragma unroll
@@ -742,47 +661,81 @@ __global__ __launch_bounds__(kThreads) void antiquant_i8_f16_fast_kernel(AntiQua
             if (r >= a.rows) {
                 break;
             }
-            const uint32_t g = a.per_tensor ? 0u : r / a.group_size;
+            // parameters: a [groups, cols] row (not transposed) or one scalar per (row, group) (transposed)
+            const uint32_t g = a.per_tensor ? 0u : kTranspose ? r : r / a.group_size;
             if (g != cached_group) {
                 cached_group = g;
-                if (a.per_tensor) {
+                if (a.per_tensor || kTranspose) {
+                    const float sv = a.per_tensor ? a.sscale : __uint_as_float(sr[u] << 16);  // (used by bfloat16 outputs)
+                    const float ov = a.per_tensor ? a.soffset : __uint_as_float(orr[u] << 16);
                     const half_t hs = static_cast<half_t>(a.sscale), ho = static_cast<half_t>(a.soffset);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        s[e] = f16x2{hs, hs};
-                        o[e] = f16x2{ho, ho};
+                        s[e] = a.per_tensor ? f16x2{hs, hs} : h2_from_bits(sr[u] * 0x10001u);
+                        o[e] = a.per_tensor ? f16x2{ho, ho} : h2_from_bits(orr[u] * 0x10001u);
+                        sf[2 * e] = sf[2 * e + 1] = sv;
+                        of[2 * e] = of[2 * e + 1] = ov;
                     }
                 } else {
                     const size_t pi = static_cast<size_t>(g) * a.cols + j;
-                    const u32x4 s0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.scale) + pi);
+                    if constexpr (kHalf) {
+                        const u32x4 s0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.scale) + pi);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) s[e] = h2_from_bits(s0[e]);
-                    if constexpr (kHasOffset) {
-                        const u32x4 o0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.offset) + pi);
+                        for (int e = 0; e < 4; ++e) s[e] = h2_from_bits(s0[e]);
+                        if constexpr (kHasOffset) {
+                            const u32x4 o0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.offset) + pi);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) o[e] = h2_from_bits(o0[e]);
+                            for (int e = 0; e < 4; ++e) o[e] = h2_from_bits(o0[e]);
+                        }
+                    } else {
+                        load8<kDst>(a.scale, pi, sf);
+                        if constexpr (kHasOffset) {
+                            load8<kDst>(a.offset, pi, of);
+                        }
                     }
                 }
             }
-            u32x4 y;
-#pragma unroll
-            for (int d = 0; d < 2; ++d) {
-                const uint32_t x = raw[u][d] ^ 0x80808080u;
-                f16x2 lo = h2_from_bits(__builtin_amdgcn_perm(0x64646464u, x, 0x04010400u)) - k1152;  // bytes 0, 1
-                f16x2 hi = h2_from_bits(__builtin_amdgcn_perm(0x64646464u, x, 0x04030402u)) - k1152;  // bytes 2, 3
-                if constexpr (kHasOffset) {
-                    lo = lo + o[2 * d];
-                    hi = hi + o[2 * d + 1];
-                }
-                lo = s[2 * d] * lo;
-                hi = s[2 * d + 1] * hi;
-                uint32_t blo, bhi;
-                __builtin_memcpy(&blo, &lo, 4);
-                __builtin_memcpy(&bhi, &hi, 4);
-                y[2 * d] = blo;
-                y[2 * d + 1] = bhi;
+            const size_t oe = static_cast<size_t>(r) * a.cols + j;
+            // the codes as bytes w + 128 or w + 8: of columns 0 - 3 and 4 - 7 (int8), of the even and the odd ones (int4)
+            uint32_t b[2];
+            if constexpr (kSrc == ASCQ_I8) {
+                b[0] = raw[u][0] ^ 0x80808080u;
+                b[1] = raw[u][1] ^ 0x80808080u;
+            } else {
+                const uint32_t q = raw[u][0] ^ 0x88888888u;
+                b[0] = q & 0x0F0F0F0Fu;
+                b[1] = (q >> 4) & 0x0F0F0F0Fu;
             }
-            __builtin_nontemporal_store(y, reinterpret_cast<u32x4*>(dst + static_cast<size_t>(r) * a.cols + j));
+            if constexpr (kHalf) {
+                u32x4 y;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {  // columns 2 d and 2 d + 1
+                    uint32_t h;
+                    if constexpr (kSrc == ASCQ_I8) {
+                        h = __builtin_amdgcn_perm(0x64646464u, b[d >> 1], d & 1 ? 0x04030402u : 0x04010400u);
+                    } else {
+                        h = __builtin_amdgcn_perm(b[1], b[0], 0x0C040C00u + 0x00010001u * d) | 0x64006400u;
+                    }
+                    f16x2 v = h2_from_bits(h) - f16x2{bias, bias};
+                    if constexpr (kHasOffset) {
+                        v = v + o[d];
+                    }
+                    v = s[d] * v;
+                    uint32_t bits;
+                    __builtin_memcpy(&bits, &v, 4);
+                    y[d] = bits;
+                }
+                __builtin_nontemporal_store(y, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.dst) + oe));
+            } else {
+                float y[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t byte = kSrc == ASCQ_I8 ? b[e >> 2] >> (8 * (e & 3)) : b[e & 1] >> (8 * (e >> 1));
+                    const float w = static_cast<float>(byte & 0xFFu) - (kSrc == ASCQ_I8 ? 128.0f : 8.0f);
+                    y[e] = antiquant_one<kDst>(w, sf[e], of[e], kHasOffset);
+                }
+                store8<kDst, true>(a.dst, oe, y);
+            }
         }
     }
 }
@@ -792,19 +745,14 @@ int launch_antiquant(const AntiQuantArgs& a, bool vec, hipStream_t st)
 {
     if (vec) {
         // keep the rows of one lane inside as few parameter groups as possible: consecutive row groups per block
-        const RowLaunch rl = row_launch(a.cols / 16, a.rows, kRowsInFlight);
-        if constexpr (kSrc == ASCQ_I8 && kDst == ASCQ_F16) {
-            if (!a.transpose) {
-                const RowLaunch fl = row_launch(a.cols / 8, a.rows, 2 * kRowsInFlight);
-                if (a.has_offset) {
-                    antiquant_i8_f16_fast_kernel<true><<<fl.grid, fl.block, 0, st>>>(a);
-                } else {
-                    antiquant_i8_f16_fast_kernel<false><<<fl.grid, fl.block, 0, st>>>(a);
-                }
-                return launch_status("ascq_antiquant");
-            }
+        const RowLaunch rl = row_launch(a.cols / 8, a.rows, 2 * kRowsInFlight);
+        if (a.transpose) {
+            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, true><<<rl.grid, rl.block, 0, st>>>(a)
+                         : antiquant_vec_kernel<kSrc, kDst, false, true><<<rl.grid, rl.block, 0, st>>>(a);
+        } else {
+            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, false><<<rl.grid, rl.block, 0, st>>>(a)
+                         : antiquant_vec_kernel<kSrc, kDst, false, false><<<rl.grid, rl.block, 0, st>>>(a);
         }
-        antiquant_vec_kernel<kSrc, kDst><<<rl.grid, rl.block, 0, st>>>(a);
     } else {
         size_t total = static_cast<size_t>(a.rows) * a.cols;
         size_t blocks = (total + kThreads - 1) / kThreads;
