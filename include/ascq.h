@@ -380,8 +380,8 @@ int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* desc, size_t* bytes)
  * once.  More rows with k up to 16384 turn the roles round: a workgroup first fetches the weights of its columns into
  * registers and then streams the activations past them, still in one launch.  Every workgroup reads all of the
  * activations there, so from a few hundred rows on (always above 512; between 129 and 512 by an estimate of both
- * times) the call runs the tile kernels of ascq_matmul_w8a8 instead, which read the packed tiles as they lie (n % 16 ==
- * 0 and k % 128 == 0; other shapes stay with the registers form): weights packed for decode serve prefill at the speed
+ * times) the call runs the tile kernels of ascq_matmul_w8a8 instead, which read the packed tiles as they lie (n % 8 ==
+ * 0; other shapes stay with the registers form): weights packed for decode serve prefill at the speed
  * of unpacked ones, without a second copy.  With k above 16384 the rows that do not fit the LDS take one pass over the
  * weights per group that does.  Requires k % 64 == 0 and a, w_packed 16-byte aligned.
  * ref: include/adv_api/matmul/matmul.h:175-185 (the Matmul object and its quant epilogue)
@@ -416,12 +416,12 @@ int ascq_unpack_int4(void* dst, const void* src, size_t elements, void* stream);
 typedef enum ascq_mm_kernel {
     ASCQ_MM_KERNEL_GENERIC = 0,      /* one lane per output element: unaligned or transposed-A inputs */
     ASCQ_MM_KERNEL_STREAM = 1,       /* few rows: weight streams, one per SIMD, then a kernel that adds their pieces */
-    ASCQ_MM_KERNEL_DMA_128 = 2,      /* m <= 512: 128 x 128 direct-to-LDS tiles, K split over workgroups when a
-                                        workspace is given (k_splits > 1: a second kernel adds the partial tiles) */
+    ASCQ_MM_KERNEL_DMA_128 = 2,      /* m <= 512, or few tiles: 128 x 128 direct-to-LDS tiles, K split over workgroups
+                                        when a workspace is given (k_splits > 1: a second kernel adds the partial tiles) */
     ASCQ_MM_KERNEL_DMA_256 = 3,      /* 256 x 256 direct-to-LDS tiles; a last partial round of the chip may be run
                                         by further workgroups of the same launch with 256 x narrow_tile_n tiles */
-    ASCQ_MM_KERNEL_STAGED = 4        /* register-staged tiles: K not a multiple of 128, or n not a multiple of 16
-                                        (a transposed B otherwise runs on the direct-to-LDS kernels like a plain one) */
+    ASCQ_MM_KERNEL_STAGED = 4        /* register-staged tiles: n not a multiple of 8 ([k, n]: of 16 below 256), and a
+                                        transposed B with k off 128, up to 512 rows and without a K split */
 } ascq_mm_kernel;
 
 typedef struct ascq_matmul_plan {
@@ -522,8 +522,9 @@ int ascq_group_matmul_w8a8(const ascq_group_matmul_desc* desc, void* y, const vo
  * x f16 [m, k]; w int4 [k, n] packed along n (n even); scale, offset f16 [k/group_size, n].
  *   wdq[k,j] = f16( scale[k/g][j] * f16( f16(w[k,j]) + offset[k/g][j] ) )     (offset optional)
  *   y[i,j]   = f16( sum_k f32(x[i,k]) * f32(wdq[k,j]) )                       fp32 accumulation
- * workspace: ascq_matmul_w4a16_workspace_size bytes of scratch for the partial sums of the weight streams (contents
- * need not be initialised); calls that share a workspace must not overlap.
+ * workspace: ascq_matmul_w4a16_workspace_size bytes of scratch for the partial sums of the weight streams, with more
+ * than 96 rows also for the weights packed as by ascq_pack_weight_w4 (a smaller one is accepted there; contents need
+ * not be initialised); calls that share a workspace must not overlap.
  */
 typedef enum ascq_w4a16_mode {
     ASCQ_W4A16_PER_WEIGHT = 0, /* wdq rounded to half per weight, the formula above: AscendAntiQuant's own arithmetic */
