@@ -585,24 +585,22 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
 }
 
-// Few rows: whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.  Up to 64 rows it
-// always is (n = k = 8192, e2m1: 13.0 against 42.4 us at 64 rows; e4m3: 19.5 against 76.9); beyond, both times are
-// estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a meets 4-bit b) by
-// 32 columns, each round 1.15 (e2m1 pairs), 1.85 (two 8-bit operands), 2.0 (e1m2, widened in registers) or 0.95 (the
-// 32-row form) per 1024 of k.  Tiles: rounds of 256 x 256 tiles, 1.3 per K step, and the passes that widen 4-bit
-// operands, 1 per 3 MB of their codes.  Crossovers measured at n = k = 8192: about 280 rows for e2m1 and e4m3, 380 for
-// e1m2; at n = 14336, k = 4096: 90, 150 and 250; at n = 1024, k = 14336 past 512 for all.
+// Tile shapes (64 rows and more): whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.
+// Both times are estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
+// meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 4.1 (two 8-bit operands), 2.4 (the
+// 32-row form), 3.1 (4-bit a, 8-bit b), 4.3 (two 4-bit operands, one of them e1m2).  Tiles: rounds of 256 x 256 tiles, 1.3
+// per K step, and the passes that widen 4-bit operands, 1 per 3 MB of their codes.  Measured at n = k = 8192, decode
+// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 37 and 77, e1m2 40 and 94; 128 rows e4m3 70 and 78, e1m2 77 and 98;
+// 256 rows e2m1 41 and 47, e4m3 136 and 85, e1m2 152 and 104; n = 14336, k = 4096, 128 rows: 28 and 26, 75 and 44, 83
+// and 64; n = 1024, k = 14336, 256 rows: 16 and 69, 59 and 147, 66 and 154.
 bool mx_decode_preferred(const MxParams& p)
 {
-    if (p.m <= 64u) {
-        return true;
-    }
     const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
     const bool two4 = p.a_format == ASCQ_QDST_FP4_E2M1 && p.b_format == ASCQ_QDST_FP4_E2M1;
     const double cus = device_compute_units();
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
-    const double per_k = two4 ? 1.15 : a8 && b8 ? 1.85 : a8 || b8 ? (rows == 32u ? 0.95 : 1.85) : 2.0;
+    const double per_k = two4 ? 1.15 : a8 && b8 ? 4.1 : a8 ? 2.4 : b8 ? 3.1 : 4.3;
     const double decode = 4.0 + rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u)) * per_k * p.k / 1024.0;
     const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
     const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * 1.3 *

@@ -9,16 +9,22 @@
 // other is computed, no barrier before the final sum.  The activations travel in the same queue: they are re-read by
 // every workgroup from the L2, m / (16 S) of the weights' bytes, which is why more rows are cut into blocks of 64
 // only up to a few hundred rows (mx_decode_preferred).  n = k = 8192, 16 rows, with one lane per output element before:
-// e2m1 4830 -> 8.9 us a call (4.0 TB/s; the caller's Python is as long as the kernel), e4m3 12.3 us (5.5 TB/s), fp8
-// activations on e2m1 weights 9.6 us; 64 rows on the 256 x 256 tiles before: e2m1 42.4 -> 13.0 us, e4m3 76.9 -> 19.5 us.
-// 32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
+// e2m1 4830 -> 8.9 us a call (4.0 TB/s; the caller's Python is as long as the kernel), e4m3 3870 -> 16.3 us, fp8
+// activations on e2m1 weights 4415 -> 14.8 us; 64 rows on the 256 x 256 tiles before: e2m1 42.4 -> 13.0 us, e4m3 77 ->
+// 37 us.  32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
 // streams half the bytes: n = 1024, k = 14336, e4m3, 9 against 14 us).
 //
-// The matrix instruction is v_mfma_scale_f32_16x16x128_f8f6f4, one scale byte per lane: lane l holds the scale of row
-// l % 16 and block of 32 k number l / 16, an 8-bit operand's registers 0-3 hold k = 16 (l / 16) .. + 15 and registers
-// 4-7 k = 64 + 16 (l / 16) .. + 15, a 4-bit operand's four registers the lane's own block of 32 k.  The two operands'
-// formats are independent, so e2m1 weights meet fp8 activations as they are; e1m2, which the instruction does not
-// know, is widened to e4m3 in registers (exact).
+// Two e2m1 operands run v_mfma_scale_f32_16x16x128_f8f6f4, one scale byte per lane: lane l holds the scale of row l % 16
+// and block of 32 k number l / 16, and in four registers that row's block.  Their products are whole multiples of 1/4 up
+// to 36, which the instruction adds exactly.
+// Every other pair runs v_mfma_f32_16x16x32_bf16 on operands converted in registers (every fp8 and fp4 value is a
+// bfloat16 value, every product of two exact in fp32), one instruction per block of 32 k from zero, whose sums the vector
+// ALU scales and adds: the arithmetic of the kernel with one lane per output element.  The scaled instruction is not good
+// enough for them: it aligns the 128 products of two 8-bit operands to the largest and drops what lies 2^13 below it.
+// Against 64 bits (2-norm, k = 8192, 16 rows, normally distributed e4m3): scaled instruction 1.3e-5, one lane per output
+// 2.2e-7, this 9.2e-8; e2m1 x e4m3 3.0e-7, 1.2e-7 and 6.8e-8.  That arithmetic is also what bounds these pairs from 16
+// rows on: per block of 32 k and 16 x 16 results a multiplication and an addition per sum beside the conversions (e4m3,
+// 16 rows: 16.3 us a call where the scaled instruction took 12.3; 64 rows 37 us and 19.5).
 #include <type_traits>
 #include <utility>
 
@@ -31,10 +37,14 @@ namespace {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* gptr_t;
 typedef int v8i __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 // operand formats: the instruction's codes, and e1m2
 enum { kE4M3 = 0, kE5M2 = 1, kE2M1 = 4, kE1M2 = 5 };
 constexpr bool fmt_is_8bit(int f) { return f == kE4M3 || f == kE5M2; }
+// the pair that the scaled matrix instruction adds up exactly; the others go through bfloat16
+constexpr bool fmt_scaled(int fa, int fb) { return fa == kE2M1 && fb == kE2M1; }
 constexpr uint32_t kPastEnd = 0x7FFFFFF0u;  // an offset every buffer's range check rejects: the load moves no data
 
 // A batch is 128 bytes of a weight column: KB values of k.
@@ -55,21 +65,55 @@ struct MxdShape {
     static_assert(lds <= 158u * 1024u && loads * 2u < 63u, "the ring must fit the LDS and the load counter");
 };
 
-// 16 e1m2 values (two dwords, the even one of a byte in the low nibble) -> 16 e4m3 codes in order.  A magnitude code c
-// is the value c / 4; the eight e4m3 codes are a byte table in two registers that a byte permute looks up.
-__device__ __forceinline__ i32x4 widen_e1m2(uint32_t d0, uint32_t d1)
+// 8 values of a format as bfloat16, every one exact (the scale operand of the conversions is 1).  e1m2 goes by way of
+// e4m3: a magnitude code c is the value c / 4, and the eight e4m3 codes are a byte table in two registers that a byte
+// permute looks up.
+template <int F>
+__device__ __forceinline__ bf16x8_t to_bf16(const typename std::conditional<fmt_is_8bit(F), i32x2_t, uint32_t>::type raw)
 {
-    constexpr uint32_t lut_hi = 0x3E3C3A38u, lut_lo = 0x34302800u;
-    i32x4 out;
+    u32x4 out;
+    auto put = [&](int i, bf16x2_t v) __attribute__((always_inline)) { out[i] = __builtin_bit_cast(uint32_t, v); };
+    if constexpr (F == kE2M1) {
+        put(0, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 0));
+        put(1, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 1));
+        put(2, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 2));
+        put(3, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 3));
+    } else {
+        uint32_t d[2];
+        if constexpr (F == kE1M2) {
+            constexpr uint32_t lut_hi = 0x3E3C3A38u, lut_lo = 0x34302800u;
+            const uint32_t ve = __builtin_amdgcn_perm(lut_hi, lut_lo, raw & 0x07070707u) | ((raw << 4) & 0x80808080u);
+            const uint32_t vo = __builtin_amdgcn_perm(lut_hi, lut_lo, (raw >> 4) & 0x07070707u) | (raw & 0x80808080u);
+            d[0] = __builtin_amdgcn_perm(vo, ve, 0x05010400u);
+            d[1] = __builtin_amdgcn_perm(vo, ve, 0x07030602u);
+        } else {
+            d[0] = static_cast<uint32_t>(raw[0]);
+            d[1] = static_cast<uint32_t>(raw[1]);
+        }
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
-        const uint32_t q = d ? d1 : d0;
-        const uint32_t ve = __builtin_amdgcn_perm(lut_hi, lut_lo, q & 0x07070707u) | ((q << 4) & 0x80808080u);
-        const uint32_t vo = __builtin_amdgcn_perm(lut_hi, lut_lo, (q >> 4) & 0x07070707u) | (q & 0x80808080u);
-        out[2 * d] = static_cast<int>(__builtin_amdgcn_perm(vo, ve, 0x05010400u));
-        out[2 * d + 1] = static_cast<int>(__builtin_amdgcn_perm(vo, ve, 0x07030602u));
+        for (int i = 0; i < 2; ++i) {
+            if constexpr (F == kE5M2) {
+                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(d[i], 1.0f, false));
+                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(d[i], 1.0f, true));
+            } else {
+                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d[i], 1.0f, false));
+                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d[i], 1.0f, true));
+            }
+        }
     }
-    return out;
+    return __builtin_bit_cast(bf16x8_t, out);
+}
+
+// 2^(e - 127) of byte `blk` of a dword of scales, but for e = 0 (the subnormal 2^-127, 0 here) and e = 255 (NaN, infinity
+// here): exact_scale puts those right where a batch has any.
+__device__ __forceinline__ float plain_scale(uint32_t dword, int blk)
+{
+    return __uint_as_float((blk == 3 ? dword >> 1 : dword << (23 - 8 * blk)) & 0x7F800000u);
+}
+__device__ __forceinline__ float exact_scale(float plain)
+{
+    const uint32_t u = __float_as_uint(plain);
+    return __uint_as_float(u == 0u ? 0x00400000u : u == 0x7F800000u ? 0x7FC00000u : u);
 }
 
 // LDS reads are instructions in an asm: one that the compiler knows of makes it wait for every load on its way into LDS.
@@ -85,6 +129,13 @@ __device__ __forceinline__ i32x2_t lds_b64(uint32_t addr)
 {
     i32x2_t v;
     asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(kOff) : "memory");
+    return v;
+}
+template <uint32_t kOff>
+__device__ __forceinline__ uint32_t lds_b32(uint32_t addr)
+{
+    uint32_t v;
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(kOff) : "memory");
     return v;
 }
 template <uint32_t kOff>
@@ -209,88 +260,42 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
         const uint32_t per = row_bytes / 16u;
         return lc * row_bytes + ((piece ^ ((lc / (16u / per)) & (per - 1u))) << 4);
     };
-    // an operand's fragment of tile tt: raw registers, then (behind the wait) the instruction's operand
-    struct Raw {
-        i32x4 lo, hi;
-        i32x2_t h0, h1;
-    };
-    auto read = [&](auto fmt, auto row_bytes, uint32_t base, auto line, auto tt) __attribute__((always_inline)) {
-        constexpr int F = decltype(fmt)::value;
-        constexpr uint32_t rb_ = decltype(row_bytes)::value, off = decltype(line)::value * 16u * rb_;
-        constexpr uint32_t tile = decltype(tt)::value;
-        Raw r;
-        if constexpr (fmt_is_8bit(F)) {
-            r.lo = lds_b128<off>(base + at(rb_, 8u * tile + lq));
-            r.hi = lds_b128<off>(base + at(rb_, 8u * tile + 4u + lq));
-        } else if constexpr (F == kE2M1) {
-            r.lo = lds_b128<off>(base + at(rb_, 4u * tile + lq));
-        } else {
-            r.h0 = lds_b64<off>(base + at(rb_, 4u * tile + (lq >> 1)) + 8u * (lq & 1u));
-            r.h1 = lds_b64<off>(base + at(rb_, 4u * tile + 2u + (lq >> 1)) + 8u * (lq & 1u));
-        }
-        return r;
-    };
-    auto landed = [&](auto fmt, Raw& r) __attribute__((always_inline)) {  // the registers may be used from here on
-        constexpr int F = decltype(fmt)::value;
-        if constexpr (fmt_is_8bit(F)) {
-            asm volatile("" : "+v"(r.lo), "+v"(r.hi));
-        } else if constexpr (F == kE2M1) {
-            asm volatile("" : "+v"(r.lo));
-        } else {
-            asm volatile("" : "+v"(r.h0), "+v"(r.h1));
-        }
-    };
-    auto operand = [&](auto fmt, const Raw& r) __attribute__((always_inline)) {
-        constexpr int F = decltype(fmt)::value;
-        if constexpr (F == kE2M1) {
-            return __builtin_shufflevector(r.lo, r.lo, 0, 1, 2, 3, -1, -1, -1, -1);
-        } else if constexpr (F == kE1M2) {
-            const i32x4 lo = widen_e1m2(static_cast<uint32_t>(r.h0[0]), static_cast<uint32_t>(r.h0[1]));
-            const i32x4 hi = widen_e1m2(static_cast<uint32_t>(r.h1[0]), static_cast<uint32_t>(r.h1[1]));
-            return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        } else {
-            return v8i{r.lo[0], r.lo[1], r.lo[2], r.lo[3], r.hi[0], r.hi[1], r.hi[2], r.hi[3]};
-        }
-    };
-    constexpr std::integral_constant<int, FA> fa{};
-    constexpr std::integral_constant<int, FB> fb{};
     constexpr std::integral_constant<uint32_t, T::arb> arb{};
     constexpr std::integral_constant<uint32_t, T::brb> brb{};
-    constexpr int kCodeA = FA == kE1M2 ? kE4M3 : FA, kCodeB = FB == kE1M2 ? kE4M3 : FB;
-
-    auto step = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
-        if (b >= batches) {
-            return;  // uniform
-        }
-        // loads return in order: everything but the newest batch has landed
+    // loads return in order: everything but the newest batch has landed
+    auto wait_batch = [&]() __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt((T::loads & 15) | ((T::loads >> 4) << 14) | (7 << 4) | (15 << 8));
         asm volatile("" ::: "memory");
+    };
+
+    // Two e2m1 operands: a lane's 16 bytes of a tile are the instruction's operand as they lie.
+    auto step_scaled = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
         const uint32_t abase = ring_addr + slot_off, bbase = abase + T::a_bytes, sbase = bbase + T::b_bytes;
         const uint32_t slane = sbase + lc * (4u * T::sdw) + lq;
-        Raw ar[T::tiles][RT], br[T::tiles][S];
+        i32x4 ar[T::tiles][RT], br[T::tiles][S];
         uint32_t asc[T::tiles][RT], bsc[T::tiles][S];
         mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {
             constexpr uint32_t tl = decltype(tt)::value;
             mxd_for<S>([&](auto j) {
-                br[tl][j] = read(fb, brb, bbase, j, tt);
+                br[tl][j] = lds_b128<decltype(j)::value * 16u * T::brb>(bbase + at(brb, 4u * tl + lq));
                 bsc[tl][j] = lds_u8<(RT + decltype(j)::value) * 64u * T::sdw + 4u * tl>(slane);
             });
             mxd_for<RT>([&](auto i) {
-                ar[tl][i] = read(fa, arb, abase, i, tt);
+                ar[tl][i] = lds_b128<decltype(i)::value * 16u * T::arb>(abase + at(arb, 4u * tl + lq));
                 asc[tl][i] = lds_u8<decltype(i)::value * 64u * T::sdw + 4u * tl>(slane);
             });
         });
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {
+        mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {  // the registers may be used from here on
             mxd_for<S>([&](auto j) {
-                landed(fb, br[tt][j]);
+                i32x4& r = br[tt][j];
                 uint32_t& v = bsc[tt][j];
-                asm volatile("" : "+v"(v));
+                asm volatile("" : "+v"(r), "+v"(v));
             });
             mxd_for<RT>([&](auto i) {
-                landed(fa, ar[tt][i]);
+                i32x4& r = ar[tt][i];
                 uint32_t& v = asc[tt][i];
-                asm volatile("" : "+v"(v));
+                asm volatile("" : "+v"(r), "+v"(v));
             });
         });
         load(b + 2u, ring + slot_off);  // the slot is free again
@@ -300,25 +305,147 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
             if (tile < tb) {  // uniform
                 // blocks past the end of k hold zeros; their scale bytes may be anything, a NaN too
                 const bool in_k = tile * 4u + lq < q.blocks;
-                v8i bo[S];
-                int bs[S];
-#pragma unroll
-                for (int j = 0; j < S; ++j) {
-                    bo[j] = operand(fb, br[tl][j]);
-                    bs[j] = in_k ? static_cast<int>(bsc[tl][j]) : 127;
-                }
+                auto operand = [](const i32x4& r) __attribute__((always_inline)) {
+                    return __builtin_shufflevector(r, r, 0, 1, 2, 3, -1, -1, -1, -1);
+                };
 #pragma unroll
                 for (int i = 0; i < RT; ++i) {
-                    const v8i ao = operand(fa, ar[tl][i]);
-                    const int as = in_k ? static_cast<int>(asc[tl][i]) : 127;
 #pragma unroll
                     for (int j = 0; j < S; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ao, bo[j], acc[i][j], kCodeA, kCodeB, 0,
-                                                                                     as, 0, bs[j]);
+                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            operand(ar[tl][i]), operand(br[tl][j]), acc[i][j], kE2M1, kE2M1, 0,
+                            in_k ? static_cast<int>(asc[tl][i]) : 127, 0, in_k ? static_cast<int>(bsc[tl][j]) : 127);
                     }
                 }
             }
         });
+    };
+
+    // Any other pair: lane l holds k = 32 blk + 8 (l / 16) .. + 7 of row l % 16 for each of a tile's four blocks blk, and
+    // the scale bytes of its four rows of the result (rows 4 (l / 16) .. + 3) and of its column.
+    typedef typename std::conditional<fmt_is_8bit(FA), i32x2_t, uint32_t>::type RawA;
+    typedef typename std::conditional<fmt_is_8bit(FB), i32x2_t, uint32_t>::type RawB;
+    auto step_exact = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
+        const uint32_t abase = ring_addr + slot_off, bbase = abase + T::a_bytes, sbase = bbase + T::b_bytes;
+        RawA ar[T::tiles][4][RT];
+        RawB br[T::tiles][4][S];
+        i32x4 asc[RT][T::sdw];  // dword r of the four rows' T::sdw dwords each, in order
+        typename std::conditional<T::sdw == 2, i32x2_t, uint32_t>::type bsc[S];
+        uint32_t staged[T::s_instr];
+        auto read = [](auto fmt, auto line, auto row_bytes, uint32_t addr) __attribute__((always_inline)) {
+            constexpr uint32_t off = decltype(line)::value * 16u * decltype(row_bytes)::value;
+            if constexpr (fmt_is_8bit(decltype(fmt)::value)) {
+                return lds_b64<off>(addr);
+            } else {
+                return lds_b32<off>(addr);
+            }
+        };
+        // bytes of the lane's 8 values of block blk of tile tl, from the operand's start
+        auto place = [&](auto fmt, auto row_bytes, uint32_t tl, uint32_t blk) __attribute__((always_inline)) {
+            if constexpr (fmt_is_8bit(decltype(fmt)::value)) {
+                return at(row_bytes, 8u * tl + 2u * blk + (lq >> 1)) + 8u * (lq & 1u);
+            } else {
+                return at(row_bytes, 4u * tl + blk) + 4u * lq;
+            }
+        };
+        constexpr std::integral_constant<int, FA> fa{};
+        constexpr std::integral_constant<int, FB> fb{};
+        mxd_for<S>([&](auto j) {
+            constexpr uint32_t off = (RT + decltype(j)::value) * 64u * T::sdw;
+            if constexpr (T::sdw == 2) {
+                bsc[j] = lds_b64<off>(sbase + lc * 8u);
+            } else {
+                bsc[j] = lds_b32<off>(sbase + lc * 4u);
+            }
+        });
+        mxd_for<RT>([&](auto i) {
+            mxd_for<static_cast<int>(T::sdw)>([&](auto h) {
+                asc[i][h] = lds_b128<decltype(i)::value * 64u * T::sdw + decltype(h)::value * 16u>(sbase + lq * (16u * T::sdw));
+            });
+        });
+        mxd_for<static_cast<int>(T::s_instr)>([&](auto u) { staged[u] = lds_b32<decltype(u)::value * 256u>(sbase + lane * 4u); });
+        mxd_for<static_cast<int>(T::tiles) * 4>([&](auto n) {
+            constexpr uint32_t tl = decltype(n)::value / 4, blk = decltype(n)::value % 4;
+            const uint32_t bat = bbase + place(fb, brb, tl, blk), aat = abase + place(fa, arb, tl, blk);
+            mxd_for<S>([&](auto j) { br[tl][blk][j] = read(fb, j, brb, bat); });
+            mxd_for<RT>([&](auto i) { ar[tl][blk][i] = read(fa, i, arb, aat); });
+        });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        auto landed = [](auto& r) __attribute__((always_inline)) { asm volatile("" : "+v"(r)); };  // usable from here on
+        mxd_for<S>([&](auto j) { landed(bsc[j]); });
+        mxd_for<RT>([&](auto i) {
+            mxd_for<static_cast<int>(T::sdw)>([&](auto h) { landed(asc[i][h]); });
+        });
+        mxd_for<static_cast<int>(T::s_instr)>([&](auto u) { landed(staged[u]); });
+        mxd_for<static_cast<int>(T::tiles) * 4>([&](auto n) {
+            mxd_for<S>([&](auto j) { landed(br[n / 4][n % 4][j]); });
+            mxd_for<RT>([&](auto i) { landed(ar[n / 4][n % 4][i]); });
+        });
+        load(b + 2u, ring + slot_off);  // the slot is free again
+        // a byte 0 or 255 among the batch's scales?  (x - 0x01..01 borrows into the top bit of a zero byte)
+        bool odd = false;
+#pragma unroll
+        for (uint32_t u = 0; u < T::s_instr; ++u) {
+            const uint32_t x = staged[u], y = ~x;
+            odd = odd || ((((x - 0x01010101u) & y) | ((y - 0x01010101u) & x)) & 0x80808080u) != 0u;
+        }
+        const bool special = __builtin_amdgcn_ballot_w64(odd) != 0;
+        mxd_for<static_cast<int>(T::tiles) * 4>([&](auto n) {
+            constexpr uint32_t tl = decltype(n)::value / 4, blk = decltype(n)::value % 4;
+            const uint32_t block = (ta + b * T::tiles + tl) * 4u + blk;
+            if (block < tb * 4u && block < q.blocks) {  // uniform; blocks past the end of k may have any scale bytes
+                float sa[RT][4], sb[S];
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    if constexpr (T::sdw == 2) {
+                        sb[j] = plain_scale(static_cast<uint32_t>(bsc[j][tl]), blk);
+                    } else {
+                        sb[j] = plain_scale(bsc[j], blk);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t d = r * T::sdw + tl;
+                        sa[i][r] = plain_scale(static_cast<uint32_t>(asc[i][d / 4u][d % 4u]), blk);
+                    }
+                }
+                if (special) {  // uniform
+#pragma unroll
+                    for (int j = 0; j < S; ++j) sb[j] = exact_scale(sb[j]);
+#pragma unroll
+                    for (int i = 0; i < RT; ++i) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) sa[i][r] = exact_scale(sa[i][r]);
+                    }
+                }
+                bf16x8_t bo[S];
+#pragma unroll
+                for (int j = 0; j < S; ++j) bo[j] = to_bf16<FB>(br[tl][blk][j]);
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    const bf16x8_t ao = to_bf16<FA>(ar[tl][blk][i]);
+#pragma unroll
+                    for (int j = 0; j < S; ++j) {
+                        const f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ao, bo[j], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(part[r], sa[i][r] * sb[j], acc[i][j][r]);
+                    }
+                }
+            }
+        });
+    };
+    auto step = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
+        if (b >= batches) {
+            return;  // uniform
+        }
+        wait_batch();
+        if constexpr (fmt_scaled(FA, FB)) {
+            step_scaled(b, slot_off);
+        } else {
+            step_exact(b, slot_off);
+        }
     };
     load(0, ring);
     load(1, ring + T::slot);

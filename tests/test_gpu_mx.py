@@ -132,8 +132,34 @@ def test_mx_few_rows(m, n, k, fa, fb):
     orc.set_threads(16)
     want = orc.matmul_mx(d, a, b, sa, sb, bv)
     got = run_mx(m, n, k, a, b, sa, sb, fa, fb, bias=bv).cpu().numpy()
-    mx_check(got - bv, want - bv, mx_abs_dot(a, b, sa, sb, k, fa, fb) + np.abs(bv), is8(fa, fb))
+    # exact products and fp32 sums for every pair: the 4e-6 of the terms' magnitudes that mx_check grants additions
+    # are 64 roundings of 2^-24; a result adds 32 products in the matrix core, a wavefront at most 1 + k / 32 / 4 of
+    # those blocks one after the other, then 8 wavefronts and the bias: less than 64 up to k = 2304
+    mx_check(got - bv, want - bv, mx_abs_dot(a, b, sa, sb, k, fa, fb) + np.abs(bv), False)
     assert np.array_equal(got, run_mx(m, n, k, a, b, sa, sb, fa, fb, bias=bv).cpu().numpy())
+
+
+@pytest.mark.parametrize("fa,fb", [(E4, E4), (E5, E4), (E4, F2), (F1, F1), (F2, F2)])
+@pytest.mark.parametrize("m,k", [(16, 512), (40, 1088)])
+def test_mx_few_rows_extreme_scales(fa, fb, m, k):
+    """The ends of the scale bytes' range: 2^-127 (a subnormal float) against 2^127, whose product is 1, and 255, which is
+    NaN and makes its row or column NaN, whatever the values it scales."""
+    announce("mx extreme scales", fa, fb, m, k)
+    rng = np.random.default_rng(k + fa * 16 + fb)
+    n = 64
+    a, b, sa, sb, _ = mx_case(rng, m, n, k, fa, fb, sk=(k // 32 + 7) // 4 * 4, lo=124, hi=131)
+    sa[:, 1], sb[:, 1] = 0, 254
+    sa[:, 7], sb[:, 7] = 254, 0
+    sa[:, k // 32 - 1], sb[:, k // 32 - 1] = 3, 251
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sa.shape[1], a_format=fa, b_format=fb, out_dtype=abi.F32, has_bias=0)
+    want = orc.matmul_mx(d, a, b, sa, sb)
+    mx_check(run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, fa, fb), False)
+    sa[5, 2] = 255
+    sb[33, 9] = 255
+    got = run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy()
+    poisoned = np.zeros((m, n), bool)
+    poisoned[5] = poisoned[:, 33] = True
+    assert np.array_equal(np.isnan(got), poisoned)
 
 
 @pytest.mark.parametrize("n", [320, 257])
