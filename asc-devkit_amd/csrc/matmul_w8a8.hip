@@ -770,9 +770,24 @@ using namespace ascq;
 namespace {
 int matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const void* w_packed, const void* bias,
                        const void* quant_vector, const void* tok_scale, void* workspace, size_t workspace_bytes, void* stream);
+
+// The scratch of a matmul.  kAll: everything the call can use, what the size queries answer.  kRequired: without the
+// partial tiles of a K split of more than 512 rows or of a ragged k or n.  Calls without them run unsplit, so no entry
+// point may insist on them (1024 rows, k = 4096, n = 1024: 24.0 MiB that would not fit the 24 MiB of
+// ascq_linear_w8a8_dynamic_noalloc).  The partial sums of up to 512 regular rows have always been part of what the linear
+// wants, which catches a size that was queried for another shape.
+enum class Scratch { kAll, kRequired };
+int matmul_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes);
+int linear_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes);
 }  // namespace
 
 extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t* bytes)
+{
+    return matmul_scratch(d, Scratch::kAll, bytes);
+}
+
+namespace {
+int matmul_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes)
 {
     ASCQ_REQUIRE(d != nullptr && bytes != nullptr, ASCQ_ENULL, "ascq_matmul_w8a8_workspace_size: NULL argument");
     *bytes = 0;
@@ -789,7 +804,7 @@ extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t
         // scratch of the matmul that produces them.
         const ascq_matmul_desc r = raw_accumulator_desc(d);
         size_t inner = 0;
-        const int rc = ascq_matmul_w8a8_workspace_size(&r, &inner);
+        const int rc = matmul_scratch(&r, which, &inner);
         if (rc != ASCQ_OK) {
             return rc;
         }
@@ -805,7 +820,8 @@ extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t
         // (few rows on [n, k] weights with k % 128 == 0 run the whole-column kernel, which needs none)
         *bytes = static_cast<size_t>(d->m) * d->n * sizeof(int32_t);
     }
-    if (dma_tiles_ok(d, shape) && dma_tiles_small(d) && !(d->m <= 32 && d->trans_b)) {
+    const bool regular = d->m <= kSkinnyMaxM && d->k % 128 == 0 && d->n % 16 == 0;
+    if ((which == Scratch::kAll || regular) && dma_tiles_ok(d, shape) && dma_tiles_small(d) && !(d->m <= 32 && d->trans_b)) {
         const size_t need =
             static_cast<size_t>(gemm_dma_skinny_splits(d->m, d->n, d->k)) * d->m * d->n * sizeof(int32_t);
         if (need > *bytes && need > static_cast<size_t>(d->m) * d->n * sizeof(int32_t)) {
@@ -820,6 +836,7 @@ extern "C" int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* d, size_t
     }
     return ASCQ_OK;
 }
+}  // namespace
 
 // ref: include/adv_api/matmul/matmul.h:175-185 (SetQuantScalar / SetQuantVector), IterateAll: matmul_impl.h:65-92
 extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* a, const void* b, const void* bias,
@@ -842,17 +859,23 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
     if (d->activation == ASCQ_MM_ACT_SWIGLU && !swiglu_in_tile_kernel(d, p, a, b) && !swiglu_in_decode_kernel(d, p, a, b)) {
         // raw accumulators into the workspace, then the pairwise epilogue
         const ascq_matmul_desc r = raw_accumulator_desc(d);
-        size_t inner = 0;
-        rc = ascq_matmul_w8a8_workspace_size(&r, &inner);
+        size_t required = 0, inner = 0;
+        rc = matmul_scratch(&r, Scratch::kRequired, &required);
+        if (rc == ASCQ_OK) {
+            rc = matmul_scratch(&r, Scratch::kAll, &inner);
+        }
         if (rc != ASCQ_OK) {
             return rc;
         }
-        inner = round256(inner);
-        const size_t need = inner + static_cast<size_t>(d->m) * d->n * sizeof(int32_t);
+        const size_t sums = static_cast<size_t>(d->m) * d->n * sizeof(int32_t), need = round256(required) + sums;
         ASCQ_REQUIRE(workspace != nullptr && workspace_bytes >= need, ASCQ_EINVAL,
                      "ascq_matmul_w8a8: SwiGLU at this shape needs a workspace of %zu bytes (see "
                      "ascq_matmul_w8a8_workspace_size)", need);
         ASCQ_REQUIRE(aligned16(workspace), ASCQ_EALIGN, "ascq_matmul_w8a8: workspace must be 16-byte aligned");
+        inner = round256(inner);
+        if (workspace_bytes - sums < inner) {
+            inner = (workspace_bytes - sums) & ~static_cast<size_t>(255u);
+        }
         p.partial = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + inner);
         rc = ascq_matmul_w8a8(&r, p.partial, a, b, r.bias_kind == ASCQ_MM_BIAS_I32_PRE ? bias : nullptr, nullptr, nullptr,
                               inner ? workspace : nullptr, inner, stream);
@@ -1055,11 +1078,17 @@ extern "C" int ascq_matmul_w8a8_plan(const ascq_matmul_desc* d, const void* c, c
 // ---------------------------------------------------------------------------- fused dynamic quantisation + matmul
 extern "C" int ascq_linear_w8a8_dynamic_workspace_size(const ascq_matmul_desc* d, size_t* bytes)
 {
+    return linear_scratch(d, Scratch::kAll, bytes);
+}
+
+namespace {
+int linear_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes)
+{
     ASCQ_REQUIRE(d != nullptr && bytes != nullptr, ASCQ_ENULL, "ascq_linear_w8a8_dynamic_workspace_size: NULL argument");
     size_t mm = 0;
     ascq_matmul_desc dd = *d;
     dd.has_tok_scale = 1;
-    int rc = ascq_matmul_w8a8_workspace_size(&dd, &mm);
+    int rc = matmul_scratch(&dd, which, &mm);
     if (rc != ASCQ_OK) {
         return rc;
     }
@@ -1067,6 +1096,7 @@ extern "C" int ascq_linear_w8a8_dynamic_workspace_size(const ascq_matmul_desc* d
     *bytes = round256(static_cast<size_t>(d->m) * d->k) + round256(static_cast<size_t>(d->m) * sizeof(float)) + mm;
     return ASCQ_OK;
 }
+}  // namespace
 
 // The activation quantiser of a W8A8 linear and the matmul in one call: q, tok = dynamic per-token quantisation of x
 // (ascq_dynamic_quant_per_token), c = matmul(q, b) with the token scales in the epilogue; q and tok live in the
@@ -1091,7 +1121,7 @@ extern "C" int ascq_linear_w8a8_dynamic(const ascq_matmul_desc* d, int32_t x_dty
     ASCQ_REQUIRE(workspace != nullptr, ASCQ_ENULL, "ascq_linear_w8a8_dynamic: workspace is NULL");
     ASCQ_REQUIRE(aligned16(workspace), ASCQ_EALIGN, "ascq_linear_w8a8_dynamic: workspace must be 16-byte aligned");
     size_t need = 0;
-    int rc = ascq_linear_w8a8_dynamic_workspace_size(d, &need);
+    int rc = linear_scratch(d, Scratch::kRequired, &need);
     if (rc != ASCQ_OK) {
         return rc;
     }
@@ -1223,7 +1253,7 @@ extern "C" int ascq_linear_w8a8_dynamic_noalloc(const ascq_matmul_desc* d, int32
                                                 const void* b, const void* bias, const void* quant_vector, void* stream)
 {
     size_t need = 0;
-    int rc = ascq_linear_w8a8_dynamic_workspace_size(d, &need);
+    int rc = linear_scratch(d, Scratch::kRequired, &need);
     if (rc != ASCQ_OK) {
         return rc;
     }
@@ -1308,7 +1338,7 @@ static int validate_w4a4(const ascq_matmul_desc* d)
     return ASCQ_OK;
 }
 
-extern "C" int ascq_matmul_w4a4_workspace_size(const ascq_matmul_desc* d, size_t* bytes)
+static int w4a4_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes)
 {
     int rc = validate_w4a4(d);
     if (rc != ASCQ_OK) {
@@ -1316,13 +1346,18 @@ extern "C" int ascq_matmul_w4a4_workspace_size(const ascq_matmul_desc* d, size_t
     }
     ASCQ_REQUIRE(bytes != nullptr, ASCQ_ENULL, "ascq_matmul_w4a4_workspace_size: bytes is NULL");
     size_t mm = 0;
-    rc = ascq_matmul_w8a8_workspace_size(d, &mm);
+    rc = matmul_scratch(d, which, &mm);
     if (rc != ASCQ_OK) {
         return rc;
     }
     // A and B as int8, then the int8 matmul's own scratch
     *bytes = round256(static_cast<size_t>(d->m) * d->k) + round256(static_cast<size_t>(d->k) * d->n) + mm;
     return ASCQ_OK;
+}
+
+extern "C" int ascq_matmul_w4a4_workspace_size(const ascq_matmul_desc* d, size_t* bytes)
+{
+    return w4a4_scratch(d, Scratch::kAll, bytes);
 }
 
 // Matmul<int4b_t, int4b_t, C>: both operands are widened to int8 in the caller's workspace (exact) and the int8
@@ -1346,7 +1381,7 @@ extern "C" int ascq_matmul_w4a4(const ascq_matmul_desc* d, void* c, const void* 
     ASCQ_REQUIRE(aligned16(workspace) && aligned16(a) && aligned16(b), ASCQ_EALIGN,
                  "ascq_matmul_w4a4: a, b and workspace must be 16-byte aligned");
     size_t need = 0;
-    rc = ascq_matmul_w4a4_workspace_size(d, &need);
+    rc = w4a4_scratch(d, Scratch::kRequired, &need);
     if (rc != ASCQ_OK) {
         return rc;
     }

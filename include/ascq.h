@@ -395,8 +395,8 @@ int ascq_matmul_w8a8_packed(const ascq_matmul_desc* desc, void* c, const void* a
  * Matmul<int4b_t A, int4b_t B, C>: the same descriptor, epilogues and outputs as ascq_matmul_w8a8 with both operands
  * packed two int4 per byte, even element in the low nibble: A [m, k/2] bytes, B [k, n/2] bytes ([n, k/2] with
  * trans_b).  trans_a is not supported (the reference's rule for an int4 A), b_format is ND, k is even, n is even
- * unless trans_b.  Both operands are widened to int8 in the workspace (mandatory; size from the query below), then the
- * int8 matmul runs.  a, b and the workspace are 16-byte aligned.
+ * unless trans_b.  Both operands are widened to int8 in the workspace (mandatory; size from the query below, of which the
+ * partial tiles of a K split of more than 512 rows or of a ragged k or n may be missing), then the int8 matmul runs.  a, b and the workspace are 16-byte aligned.
  * ref: examples/01_simd_cpp_api/04_advanced_api/00_matmul/matmul_int4/matmul_int4.asc:52-58, 155; README.md
  *      ("Constraints"); packing: scripts/gen_data.py:32-42.
  */
@@ -449,7 +449,8 @@ int ascq_matmul_w8a8_plan(const ascq_matmul_desc* desc, const void* c, const voi
  * with exactly those results.  x [m, k] of x_dtype (ASCQ_F16 | ASCQ_BF16 | ASCQ_F32); desc as for ascq_matmul_w8a8 with
  * a dequantising epilogue (quant_mode SCALAR or VECTOR, floating-point out_dtype); desc->has_tok_scale is ignored.
  * The two kernels run one after the other on the stream, with q and tok in the workspace (sized by
- * ascq_linear_w8a8_dynamic_workspace_size; always required, whatever kernel runs).  Decode calls - half or bfloat16 x
+ * ascq_linear_w8a8_dynamic_workspace_size; always required, whatever kernel runs, but for the partial tiles of a K split
+ * of more than 512 rows or of a ragged k or n, which the size includes: with less the matmul runs unsplit).  Decode calls - half or bfloat16 x
  * on weights kept as [n, k] (desc->trans_b), k a multiple of 64, up to 7 rows at k = 4096, 4 at 7168, 2 at 14848 - are
  * one launch: the weight-streaming kernel quantises x itself on its way into LDS (the same bits; the workspace is not
  * touched).  No single reference operator does this: the reference composes it from
@@ -465,8 +466,10 @@ int ascq_linear_w8a8_dynamic_workspace_size(const ascq_matmul_desc* desc, size_t
  * the descriptor may ask for: no trans_a, no NZ, k % 64 == 0; desc->trans_b is ignored).  Results are those
  * of ascq_linear_w8a8_dynamic on the unpacked weights, bit for bit.  Up to 8 rows of half or bfloat16 x are one launch
  * (the packed decode kernel quantises x itself); otherwise the quantiser kernel runs first and
- * ascq_matmul_w8a8_packed after it, with q and the token scales in the workspace.  The workspace holds
- * round256(m * k) + round256(4 * m) bytes; ascq_linear_w8a8_dynamic_workspace_size covers that.
+ * ascq_matmul_w8a8_packed after it, with q and the token scales in the workspace.  The workspace holds at least
+ * round256(m * k) + round256(4 * m) bytes; what lies behind them serves as partial tiles where from 129 rows on a K split
+ * is ahead (a split in s takes s * m * n * 4 bytes; the size that ascq_linear_w8a8_dynamic_workspace_size answers
+ * for [k, n] weights covers it).
  * It has no counterpart in the reference (which composes the linear from ReduceMax / AscendQuant PER_TOKEN and Matmul,
  * ascend_quant_per_group_3510_impl.h:142-178, matmul.h:175-185, on weights it packs offline, gen_data.py:62-64).
  */
@@ -479,8 +482,8 @@ int ascq_linear_w8a8_dynamic_packed(const ascq_matmul_desc* desc, int32_t x_dtyp
  * anything it calls).  It has no counterpart in the reference; it is for callers that cannot allocate device memory:
  * code under stream capture, tight serving loops, harnesses that forbid hipMalloc.  The scratch (quantised
  * activations, token scales, partial sums of the small-m kernels) is a device array of ASCQ_STATIC_SCRATCH_BYTES that
- * is part of the library; every GPU the library runs on holds its own copy until the process ends.  Shapes whose
- * ascq_linear_w8a8_dynamic_workspace_size exceeds that size are rejected with ASCQ_EINVAL (k = 4096, n = 11008 fits
+ * is part of the library; every GPU the library runs on holds its own copy until the process ends.  Shapes that
+ * require more (ascq_linear_w8a8_dynamic; optional partial tiles do not count) are rejected with ASCQ_EINVAL (k = 4096, n = 11008 fits
  * with 1, 16, 128 and 2048 rows; 32 rows need 32 MiB of partial sums and do not).  Results are those of
  * ascq_linear_w8a8_dynamic, bit for bit.  All calls on one GPU share the one array: calls that overlap in time on
  * the same GPU (two streams, two threads) race; serialise them or use the workspace form.  The first call on a device

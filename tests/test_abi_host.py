@@ -437,6 +437,24 @@ def test_linear_dynamic_packed_argument_checks():
     assert need.value >= 4 * 128 + 4 * 4
 
 
+@pytest.mark.parametrize("m,k,n", [(600, 11008, 1024), (729, 11008, 1152), (1024, 8192, 2048), (2048, 4096, 1024), (1024, 4096, 1024),
+                                   (384, 11008, 1000), (512, 14336, 3000)])
+def test_partial_tiles_of_optional_splits_are_not_required(m, k, n):
+    """The K split of more than 512 rows and of a ragged k or n is a matter of speed: its partial tiles are part of the
+    queried size, but the linear runs without them, so it accepts the quantised activations and token scales alone, and
+    the form without a workspace accepts what those leave room for.  (c is NULL, which is looked at behind the size.)"""
+    d = abi.MatmulDesc(m=m, n=n, k=k, out_dtype=abi.BF16, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32)
+    need = C.c_size_t(0)
+    assert L.ascq_linear_w8a8_dynamic_workspace_size(C.byref(d), C.byref(need)) == abi.OK
+    up = lambda v: (v + 255) // 256 * 256
+    least = up(m * k) + up(4 * m)
+    assert need.value > least
+    call = lambda nbytes: L.ascq_linear_w8a8_dynamic(C.byref(d), abi.BF16, None, FAKE, FAKE, None, FAKE, C.c_void_p(0x200000), nbytes, None)
+    assert call(least) == abi.ENULL and call(least - 1) == abi.EINVAL
+    rc = L.ascq_linear_w8a8_dynamic_noalloc(C.byref(d), abi.BF16, None, FAKE, FAKE, None, FAKE, None)
+    assert rc in (abi.ENULL, abi.EHIP)      # (EHIP: no GPU to find the built-in buffer on)
+
+
 def test_tmp_buffer_factor_sizes_known_answers():
     """tests/api/adv_api/tiling/test_tiling.cpp:6549-6553, 6565-6569, 6583-6608, 6621-6625, 6643-6647, 6662-6666,
     6684-6688 of the reference."""

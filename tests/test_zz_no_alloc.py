@@ -52,7 +52,8 @@ def both(m, n, k, seed, with_bias):
 
 @pytest.mark.parametrize("first,second", [((16, 1040, 2048), (3, 528, 1024)),        # weight-stream kernels: partial sums
                                            ((128, 2064, 1024), (40, 528, 512)),        # 128-row tiles, K split over workgroups
-                                           ((600, 528, 640), (300, 272, 512))])        # large tiles: q and token scales only
+                                           ((600, 528, 640), (300, 272, 512)),         # large tiles: q and token scales only
+                                           ((1024, 1024, 4096), (384, 1000, 1104))])   # a K split of many or ragged rows, where it fits
 def test_noalloc_equals_workspace_form_two_calls(first, second):
     for i, (m, n, k) in enumerate((first, second)):
         announce("noalloc", m, n, k)
@@ -99,3 +100,26 @@ def test_noalloc_wrapper_with_swiglu(m, n, k):
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     assert not torch.equal(plain.view(torch.int16), want.view(torch.int16)), "act_beta had no effect"
+
+
+@pytest.mark.parametrize("m,n,k", [(640, 512, 2048), (200, 1000, 1104)])
+def test_w4a4_without_room_for_a_split(m, n, k):
+    """int4 x int4 in a workspace that holds the two widened operands and nothing else: the same bits, unsplit."""
+    announce("w4a4 unsplit", m, n, k)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m)
+    a, b = (torch.randint(0, 256, s, dtype=torch.uint8, device=DEV, generator=g) for s in ((m, k // 2), (k, n // 2)))
+    d = abi.MatmulDesc(m=m, n=n, k=k, out_dtype=abi.I32, quant_mode=abi.MM_QUANT_NONE, scale_format=abi.MM_SCALE_U64)
+    need = C.c_size_t(0)
+    assert L.ascq_matmul_w4a4_workspace_size(C.byref(d), C.byref(need)) == abi.OK
+    least = (m * k + 255) // 256 * 256 + (k * n + 255) // 256 * 256
+    assert need.value > least
+    ws = torch.empty(need.value, dtype=torch.uint8, device=DEV)
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    out = []
+    for nbytes in (need.value, least):
+        c = torch.full((m, n), -1, dtype=torch.int32, device=DEV)
+        rc = L.ascq_matmul_w4a4(C.byref(d), ptr(c), ptr(a), ptr(b), None, None, None, ptr(ws), nbytes, stream)
+        assert rc == abi.OK, L.ascq_last_error().decode()
+        out.append(c)
+    assert torch.equal(*out)
