@@ -791,17 +791,20 @@ int matmul_scratch(const ascq_matmul_desc* d, Scratch which, size_t* bytes)
 {
     ASCQ_REQUIRE(d != nullptr && bytes != nullptr, ASCQ_ENULL, "ascq_matmul_w8a8_workspace_size: NULL argument");
     *bytes = 0;
-    // The size is that for operands aligned to 16 bytes; it cannot see the pointers.  (A SwiGLU call whose misaligned
-    // operands keep it off the tile kernel names the size it needs in its error.)
+    // The size is that for operands aligned to 16 bytes; it cannot see the pointers.  (A SwiGLU call of more than 512 rows
+    // whose misaligned operands keep it off the tile kernel names the size it needs in its error.)
     GemmParams shape{};
     shape.a = shape.b = reinterpret_cast<const int8_t*>(uintptr_t{16});
     shape.m = d->m;
     shape.n = d->n;
     shape.k = d->k;
+    const bool large = d->m > kSkinnyMaxM && d->k % 128 == 0 && d->n % 16 == 0;
     if (d->activation == ASCQ_MM_ACT_SWIGLU && d->quant_mode != ASCQ_MM_QUANT_NONE &&
-        !swiglu_in_tile_kernel(d, shape, shape.a, shape.b) && !swiglu_in_decode_kernel(d, shape, shape.a, shape.b)) {
-        // Shapes outside the large tile kernel keep their int32 accumulators [m][n] in the workspace, behind the
-        // scratch of the matmul that produces them.
+        (!swiglu_in_tile_kernel(d, shape, shape.a, shape.b) || (which == Scratch::kAll && !large)) &&
+        !swiglu_in_decode_kernel(d, shape, shape.a, shape.b)) {
+        // Shapes outside the tile kernels keep their int32 accumulators [m][n] in the workspace, behind the scratch of
+        // the matmul that produces them.  The size for up to 512 rows and for a ragged k or n includes them also where
+        // the tiles take aligned operands, so that misaligned ones find what they need in it.
         const ascq_matmul_desc r = raw_accumulator_desc(d);
         size_t inner = 0;
         const int rc = matmul_scratch(&r, which, &inner);

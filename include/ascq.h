@@ -362,8 +362,9 @@ int ascq_matmul_w8a8(const ascq_matmul_desc* desc, void* c, const void* a, const
                      const void* quant_vector, const void* tok_scale, void* workspace, size_t workspace_bytes,
                      void* stream);
 /* The workspace ascq_matmul_w8a8 needs for this descriptor with operands aligned to 16 bytes (0 for most shapes; the
- * partial sums of the few-row kernels; with ASCQ_MM_ACT_SWIGLU outside the large tile kernel the raw accumulators
- * [m][n]).  A call that needs more than it was given (SwiGLU on misaligned operands) names the size in its error. */
+ * partial sums of the few-row kernels; with ASCQ_MM_ACT_SWIGLU the raw accumulators [m][n], but for more than 512 rows with
+ * k % 128 == 0 and n % 16 == 0).  A call that needs more than it was given (such a one on misaligned operands) names the
+ * size in its error. */
 int ascq_matmul_w8a8_workspace_size(const ascq_matmul_desc* desc, size_t* bytes);
 
 /*

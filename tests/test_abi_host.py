@@ -455,6 +455,20 @@ def test_partial_tiles_of_optional_splits_are_not_required(m, k, n):
     assert rc in (abi.ENULL, abi.EHIP)      # (EHIP: no GPU to find the built-in buffer on)
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 11008, 144), (300, 4096, 1024), (729, 128, 144), (1024, 512, 4304), (2048, 1000, 128)])
+@pytest.mark.parametrize("trans_b", [0, 1])
+def test_swiglu_size_serves_misaligned_operands(m, n, k, trans_b):
+    """Up to 512 rows, and with a ragged k or n, the queried workspace lets a SwiGLU call run whatever its operands'
+    alignment: aligned ones in the tile kernels, others through raw accumulators in the workspace."""
+    d = abi.MatmulDesc(m=m, n=n, k=k, trans_b=trans_b, out_dtype=abi.BF16, quant_mode=abi.MM_QUANT_VECTOR,
+                       scale_format=abi.MM_SCALE_F32, activation=abi.MM_ACT_SWIGLU, act_beta=1.0)
+    need, plan = C.c_size_t(0), abi.MatmulPlan()
+    assert L.ascq_matmul_w8a8_workspace_size(C.byref(d), C.byref(need)) == abi.OK
+    for a, b in ((0x200000, 0x400000), (0x200004, 0x400000), (0x200008, 0x400008), (0x200001, 0x400000)):
+        assert L.ascq_matmul_w8a8_plan(C.byref(d), FAKE, C.c_void_p(a), C.c_void_p(b), None, FAKE, None, C.c_void_p(0x800000),
+                                       need.value, C.byref(plan)) == abi.OK, err()
+
+
 def test_tmp_buffer_factor_sizes_known_answers():
     """tests/api/adv_api/tiling/test_tiling.cpp:6549-6553, 6565-6569, 6583-6608, 6621-6625, 6643-6647, 6662-6666,
     6684-6688 of the reference."""
