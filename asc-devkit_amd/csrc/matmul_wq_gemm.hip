@@ -316,8 +316,15 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
 #pragma unroll
         for (int n = 0; n < kM; ++n) mfma(3, n);
     }
-    // the last sums are on their way through the matrix pipe
+    // The last sums are on their way through the matrix pipe, which the compiler does not know: it sees them changed behind
+    // the wait, so that nothing that reads them can move ahead of it.  (check_matrix_asm.py looks through the machine code
+    // for what this cannot rule out, a copy inside the loop.)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past the end
 
     // ---- register r of lane l in a 16 x 16 block: row 4 (l / 16) + r, column l % 16

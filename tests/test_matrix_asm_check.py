@@ -1,0 +1,39 @@
+"""The build's look through the machine code of matrix instructions in inline assembly, on a few lines of code."""
+import os
+import sys
+
+import pytest
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "asc-devkit_amd", "csrc"))
+import check_matrix_asm as check  # noqa: E402
+
+MFMA = "v_mfma_i32_16x16x64_i8 v[0:3], v[8:11], v[12:15], v[0:3]"
+OTHER = "v_mfma_i32_16x16x64_i8 v[4:7], v[8:11], v[12:15], v[4:7]"
+
+
+def body(*lines):
+    """instructions at addresses 0, 4, ...; 'L: s_branch' forms jump to the line whose number follows '->'"""
+    out = []
+    for n, line in enumerate(lines):
+        text, _, target = line.partition(" -> ")
+        i = check.Instruction(text, 4 * n)
+        i.target = 4 * int(target) if target else None
+        out.append(i)
+    return out
+
+
+@pytest.mark.parametrize("lines,wrong", [
+    ((MFMA, OTHER, MFMA, "s_nop 15", "s_nop 15", "v_cvt_f32_i32_e32 v20, v0", "s_endpgm"), False),
+    ((MFMA, OTHER, "s_nop 7", "v_cvt_f32_i32_e32 v20, v2", "s_endpgm"), True),                 # read too early
+    ((MFMA, "v_mov_b32_e32 v3, v20", "s_endpgm"), True),                                       # overwritten
+    ((MFMA, "global_store_dwordx4 v[20:21], v[0:3], off", "s_endpgm"), True),                  # stored too early
+    ((MFMA, "v_mfma_i32_16x16x64_i8 v[4:7], v[0:3], v[12:15], v[4:7]", "s_endpgm"), True),     # an operand of the next one
+    ((MFMA, "v_mfma_i32_16x16x64_i8 v[4:7], v[8:11], v[12:15], v[0:3]", "s_endpgm"), True),    # added up elsewhere
+    (("v_cvt_f32_i32_e32 v20, v0", "s_nop 15", MFMA, "s_cbranch_scc1 s -> 0", "s_endpgm"), True),   # round the loop
+    (("v_cvt_f32_i32_e32 v20, v0", "s_nop 15", MFMA, "s_nop 15", "s_nop 15", "s_cbranch_scc1 s -> 0", "s_endpgm"), False),
+    (("v_mov_b32_e32 v9, v20", MFMA, "s_nop 15", "s_nop 15", "s_endpgm"), True),               # operand written just before
+    (("v_mov_b32_e32 v9, v20", "s_nop 1", MFMA, "s_endpgm"), False),
+    (("ds_read_b128 v[8:11], v30", "s_waitcnt lgkmcnt(0)", MFMA, "s_endpgm"), False),
+])
+def test_missing_waits_are_found(lines, wrong):
+    assert bool(check.faults(body(*lines))) == wrong
