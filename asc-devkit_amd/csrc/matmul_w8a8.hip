@@ -898,7 +898,7 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
         // only the direct-to-LDS tile kernels address the fractal layout; validate_mm has checked what they need
         p.b_nz = 1;
         return d->m <= kSkinnyMaxM ? launch_gemm_dma_skinny(p, workspace, workspace_bytes, st)
-                                   : launch_gemm_dma(p, false, st);
+                                   : launch_gemm_dma(p, st);
     }
     if (!fast_path_ok(d, a, b) && d->m <= 32u && !d->trans_a && !d->trans_b && d->n >= 64u && d->k % 4u == 0 && d->k >= 128u &&
         (reinterpret_cast<uintptr_t>(a) & 3u) == 0 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 3u) == 0 &&
@@ -1002,7 +1002,7 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
         return d->trans_b ? launch_gemm<TileST, true, false>(p, st) : launch_gemm<TileS, false, false>(p, st);
     }
     if (dma_tiles_ok(d, p)) {
-        return launch_gemm_dma(p, false, st, d->trans_b != 0);  // B as [n][k]: its tiles are staged and read like A's
+        return launch_gemm_dma(p, st, d->trans_b != 0);  // B as [n][k]: its tiles are staged and read like A's
     }
     if (d->m <= 1024) {
         return d->trans_b ? launch_gemm<TileMT, true, false>(p, st) : launch_gemm<TileM, false, false>(p, st);
@@ -1054,7 +1054,7 @@ int matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const 
     if (tiles_ok && (d->m > kSkinnyMaxM || (d->m > 128u && packed_tiles_faster(p, splits)))) {
         const bool small = d->m <= kSkinnyMaxM || (splits > 1u && gemm_dma_small_tiles(d->m, d->n, d->k));
         return small ? launch_gemm_dma_skinny(p, workspace, splits > 1u ? workspace_bytes : 0, static_cast<hipStream_t>(stream), 2)
-                     : launch_gemm_dma(p, false, static_cast<hipStream_t>(stream), 2);
+                     : launch_gemm_dma(p, static_cast<hipStream_t>(stream), 2);
     }
     if (gemm_ws_supported(p, false)) {
         return launch_gemm_ws(p, static_cast<hipStream_t>(stream), false);
@@ -1443,7 +1443,7 @@ extern "C" int ascq_group_matmul_w8a8(const ascq_group_matmul_desc* g, void* y, 
     ASCQ_REQUIRE(d->activation != ASCQ_MM_ACT_SWIGLU || d->out_dtype == ASCQ_F16 || d->out_dtype == ASCQ_BF16,
                  ASCQ_EUNSUPPORTED, "ascq_group_matmul_w8a8: SwiGLU writes half or bfloat16 here");
     if (gemm_dma_supported(p) && ((d->k % 128u == 0 && d->n % 16u == 0) || d->activation != ASCQ_MM_ACT_SWIGLU)) {
-        return launch_gemm_dma(p, true, st);
+        return launch_gemm_dma_group(p, st);
     }
     ASCQ_REQUIRE(!p.b_nz, ASCQ_EUNSUPPORTED, "ascq_group_matmul_w8a8: fractal (NZ) weights need the tile kernel's shape");
     ASCQ_REQUIRE(d->activation != ASCQ_MM_ACT_SWIGLU, ASCQ_EUNSUPPORTED,

@@ -477,6 +477,83 @@ def test_fixpipe_pre_shift_words(m, n, k, trans_b):
         assert np.array_equal(bits(c), want.view(np.uint16) if out == torch.float16 else want), out
 
 
+def gpu_mm(m, n, k, a, b, layout, kind, out, quant, tok, bias):
+    mm = ops.Matmul(m, n, k, trans_b=layout == "nk")
+    mm.set_tensor_a(a)
+    if layout == "packed":
+        mm.set_tensor_b_packed(b)
+    else:
+        mm.set_tensor_b(b)
+    mm.set_quant_vector(quant)
+    mm.set_token_scale(tok)
+    mm.set_bias(bias)
+    mm.set_activation({"gelu": abi.MM_ACT_FASTER_GELU, "swiglu": abi.MM_ACT_SWIGLU}.get(kind, abi.MM_ACT_NONE), 1.0)
+    c = torch.zeros((m, n // 2 if kind == "swiglu" else n), dtype=out, device=DEV)
+    mm.iterate_all(c)
+    return c
+
+
+@pytest.mark.parametrize("k,n,layout", [(3072, 10240, "kn"), (3088, 10008, "kn"), (3200, 10000, "nk"), (3088, 10008, "nk"),
+                                        (3136, 10000, "packed")])
+@pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu", "words", "shifts"])
+def test_w8a8_both_matrix_instructions_agree(k, n, layout, kind):
+    """Long sums in enough 256 x 256 tiles for the 16 x 16 x 64 instruction (5 x 40 of them, the last of 3 rows), against
+    the same rows in two calls of too few tiles for it: equal bits, whole and partial last steps, every weight layout,
+    the activations, quant words with and without the bit that shifts the accumulator.  The plain form also against
+    the sums in 64 bits."""
+    announce("w8a8 both instructions", k, n, layout, kind)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(k + n)
+    m, cut = 1027, 514
+    a = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    b = torch.randint(-127, 128, (n, k) if layout == "nk" else (k, n), dtype=torch.int8, device=DEV, generator=g)
+    w = ops.pack_weight_w8(b, k, n) if layout == "packed" else b
+    tok = torch.rand(m, device=DEV, generator=g) * 0.1 + 1e-3
+    cs = torch.rand(n, device=DEV, generator=g) * 1e-4 + 1e-5
+    bias = torch.randn(n, device=DEV, generator=g)
+    quant, out = cs, torch.bfloat16
+    if kind in ("words", "shifts"):
+        quant = cs.view(torch.int32).to(torch.int64) & 0xFFFFFFFF
+        bias, out = torch.randint(-3000, 3000, (n,), dtype=torch.int32, device=DEV, generator=g), torch.float16
+        if kind == "shifts":
+            pick = torch.randint(0, 32, (n,), device=DEV, generator=g)
+            quant = quant | ((pick & 15) << 32) | ((pick >> 4) << 36)
+    elif kind == "gelu":
+        bias = bias.to(torch.bfloat16)
+    got = gpu_mm(m, n, k, a, w, layout, kind, out, quant, tok, bias)
+    parts = [gpu_mm(hi - lo, n, k, a[lo:hi].clone(), w, layout, kind, out, quant, tok[lo:hi].clone(), bias) for lo, hi in ((0, cut), (cut, m))]
+    assert torch.equal(got.view(torch.int16), torch.cat(parts).view(torch.int16))
+    if kind == "plain":
+        acc = a.double() @ (b.double().t().contiguous() if layout == "nk" else b.double())      # exact: below 2^53
+        want = (acc.float() * cs * tok[:, None] + bias).to(out)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu"])
+def test_group_matmul_both_matrix_instructions_agree(kind):
+    """The grouped matmul at a size for the 16 x 16 x 64 instruction against the plain matmul of each group's rows."""
+    announce("grouped matmul, both instructions", kind)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3)
+    counts, k, n = [513, 0, 300, 260], 3072, 10240
+    m = sum(counts)
+    x = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    w = torch.randint(-127, 128, (len(counts), k, n), dtype=torch.int8, device=DEV, generator=g)
+    tok = torch.rand(m, device=DEV, generator=g) * 0.1 + 1e-3
+    cs = torch.rand((len(counts), n), device=DEV, generator=g) * 1e-4 + 1e-5
+    bias = torch.randn((len(counts), n), device=DEV, generator=g).to(torch.bfloat16)
+    y = torch.zeros((m, n // 2 if kind == "swiglu" else n), dtype=torch.bfloat16, device=DEV)
+    ops.quant_group_matmul(y, x, w, torch.tensor(counts, dtype=torch.int64, device=DEV), cs, tok, bias,
+                           activation={"gelu": abi.MM_ACT_FASTER_GELU, "swiglu": abi.MM_ACT_SWIGLU}.get(kind, abi.MM_ACT_NONE))
+    first = 0
+    for i, c in enumerate(counts):
+        if c:
+            rows = slice(first, first + c)
+            want = gpu_mm(c, n, k, x[rows].clone(), w[i], "kn", kind, torch.bfloat16, cs[i].clone(), tok[rows].clone(), bias[i].clone())
+            assert torch.equal(y[rows].view(torch.int16), want.view(torch.int16)), i
+        first += c
+
+
 def test_post_bias_bf16_and_gelu():
     announce("matmul bf16 bias + token scale + FasterGelu")
     rng = np.random.default_rng(22)
