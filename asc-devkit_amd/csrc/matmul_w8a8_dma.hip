@@ -4,58 +4,6 @@
 namespace ascq {
 namespace {
 
-// The plain matmul: tile number `bid` of the launch (before the XCD remapping), column tiles counted from col_begin,
-// row tiles innermost so that the tiles an XCD runs side by side share their B columns.
-template <int BM, int BN, bool kSplitK, int kB, int kForm>
-__device__ __forceinline__ void gemm_dma_tile(const GemmParams& p, uint32_t col_begin, uint32_t bid, uint32_t bidy,
-                                              char* A0, char* B0, char* A1, char* B1, float* TS)
-{
-    const uint32_t total = p.tiles_m * p.tiles_n;
-    const uint32_t t = xcd_remap(bid, total);
-    if (t >= total) {
-        return;
-    }
-    // bands of 8 row tiles, inside a band column by column (band_order): an XCD's share stays a block of a few columns
-    // by 8 rows whose rows of A and columns of B it reuses from its L2, however many rows the matrix has
-    uint32_t ms, tn;
-    band_order(t, p.tiles_m, p.tiles_n, ms, tn);
-    const TilePlace at{ms * BM, p.m, col_begin + tn * BN, p.b, 0};
-    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, A0, B0, A1, B1, TS);
-}
-
-template <int BM, int BN, bool kSplitK, int kB, int kForm>
-__global__ __launch_bounds__(kThreads, (BM * BK + BK * BN) * 2 <= 65536 ? 2 : 1) void gemm_dma_kernel(
-    GemmParams p, uint32_t col_begin)
-{
-    __shared__ __attribute__((aligned(1024))) char A0[BM * BK];
-    __shared__ __attribute__((aligned(1024))) char B0[BK * BN];
-    __shared__ __attribute__((aligned(1024))) char A1[BM * BK];
-    __shared__ __attribute__((aligned(1024))) char B1[BK * BN];
-    __shared__ __attribute__((aligned(16))) float TS[BM];  // token scales of the tile's rows (1.0f when there are none)
-    gemm_dma_tile<BM, BN, kSplitK, kB, kForm>(p, col_begin, blockIdx.x, blockIdx.y, A0, B0, A1, B1, TS);
-}
-
-// One launch for a matrix whose last round of 256 x 256 tiles would be mostly empty: workgroups [0, wide_wgs) run the
-// 256 x 256 tiles of the first `p.tiles_n` tile columns, the rest 256 x 128 tiles of the remaining columns.  A compute
-// unit that has finished its wide tile takes a narrow one at once, without the drain between two launches.
-template <int kB, int kForm>
-__global__ __launch_bounds__(kThreads, 1) void gemm_dma_dual_kernel(GemmParams p, uint32_t wide_wgs,
-                                                                    uint32_t narrow_tiles_n, uint32_t col_begin)
-{
-    __shared__ __attribute__((aligned(1024))) char A0[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B0[BK * 256];
-    __shared__ __attribute__((aligned(1024))) char A1[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B1[BK * 256];
-    __shared__ __attribute__((aligned(16))) float TS[256];
-    if (blockIdx.x < wide_wgs) {
-        gemm_dma_tile<256, 256, false, kB, kForm>(p, 0u, blockIdx.x, 0u, A0, B0, A1, B1, TS);
-    } else {
-        GemmParams q = p;
-        q.tiles_n = narrow_tiles_n;
-        gemm_dma_tile<256, 128, false, kB, kForm>(q, col_begin, blockIdx.x - wide_wgs, 0u, A0, B0, A1, B1, TS);
-    }
-}
-
 // Second pass of the split-K path: sums the int32 partial tiles [split][m][n] in split order (integer addition: exact in
 // any order) and applies the epilogue.  One lane = four consecutive columns.
 __global__ __launch_bounds__(256) void splitk_sum_epilogue_kernel(GemmParams p)
@@ -104,16 +52,14 @@ bool gemm_dma_supported(const GemmParams& p, int b_layout)
 
 namespace {
 
-// calls f with the B layout (0: [k, n], 1: [n, k], 2: packed by ascq_pack_weight_w8) as a compile-time constant
-template <class F>
-void with_b_layout(int b_layout, F&& f)
+void run_dma(int form, const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t st)
 {
-    if (b_layout == 2) {
-        f(std::integral_constant<int, 2>{});
-    } else if (b_layout == 1) {
-        f(std::integral_constant<int, 1>{});
+    if (form == k32Ragged) {
+        run_dma_ragged(p, l, b_layout, st);
+    } else if (form == k16) {
+        run_dma<k16>(p, l, b_layout, st);
     } else {
-        f(std::integral_constant<int, 0>{});
+        run_dma<k32>(p, l, b_layout, st);
     }
 }
 
@@ -151,6 +97,7 @@ int launch_gemm_dma(GemmParams& p, hipStream_t st, int b_layout)
         }
         return ASCQ_OK;
     }
+    const int form = gemm_dma_form(p);
     if (wide_cols && narrow_cols) {
         // both tile shapes in one launch (narrow_cols is only ever non-zero for the plain matmul)
         const uint32_t col_begin = wide_cols * 256u;
@@ -158,35 +105,17 @@ int launch_gemm_dma(GemmParams& p, hipStream_t st, int b_layout)
         const uint32_t wide_wgs = (p.tiles_m * wide_cols + 7u) / 8u * 8u;
         const uint32_t narrow_wgs = (p.tiles_m * narrow_tiles_n + 7u) / 8u * 8u;
         p.tiles_n = wide_cols;
-        with_b_layout(b_layout, [&](auto kb) {
-            with_form(p, [&](auto form) {
-                gemm_dma_dual_kernel<decltype(kb)::value, decltype(form)::value>
-                    <<<wide_wgs + narrow_wgs, kThreads, 0, st>>>(p, wide_wgs, narrow_tiles_n, col_begin);
-            });
-        });
+        run_dma(form, p, DmaLaunch{DmaLaunch::kBoth, dim3(wide_wgs + narrow_wgs), col_begin, wide_wgs, narrow_tiles_n}, b_layout, st);
         return launch_status("ascq_matmul_w8a8");
     }
     if (wide_cols) {
         p.tiles_n = wide_cols;
         const uint32_t t = p.tiles_m * p.tiles_n;
-        // the wide launch must not touch the narrow region: clip n for its column masks
-        GemmParams q = p;
-        if (narrow_cols) {
-            q.n = p.n;  // row pitch stays n; columns >= wide_cols * 256 are simply not assigned to any tile
-        }
-        with_b_layout(b_layout, [&](auto kb) {
-            with_form(p, [&](auto form) {
-                gemm_dma_kernel<256, 256, false, decltype(kb)::value, decltype(form)::value><<<(t + 7u) / 8u * 8u, kThreads, 0, st>>>(q, 0u);
-            });
-        });
-    }
-    if (narrow_cols) {
-        const uint32_t col_begin = wide_cols * 256u;
-        p.tiles_n = (p.n - col_begin + 127u) / 128u;
+        run_dma(form, p, DmaLaunch{DmaLaunch::kWide, dim3((t + 7u) / 8u * 8u), 0u, 0u, 0u}, b_layout, st);
+    } else {
+        p.tiles_n = (p.n + 127u) / 128u;
         const uint32_t t = p.tiles_m * p.tiles_n;
-        with_b_layout(b_layout, [&](auto kb) {
-            gemm_dma_kernel<256, 128, false, decltype(kb)::value, 32><<<(t + 7u) / 8u * 8u, kThreads, 0, st>>>(p, col_begin);
-        });
+        run_dma(p.k % BK != 0 ? k32Ragged : k32, p, DmaLaunch{DmaLaunch::kNarrow, dim3((t + 7u) / 8u * 8u), 0u, 0u, 0u}, b_layout, st);
     }
     return launch_status("ascq_matmul_w8a8");
 }
@@ -248,17 +177,14 @@ int launch_gemm_dma_skinny(GemmParams& p, void* workspace, size_t workspace_byte
         }
         return ASCQ_OK;
     }
+    const int form = p.k % BK != 0 ? k32Ragged : k32;
     if (splits == 1) {
-        with_b_layout(b_layout, [&](auto kb) {
-            gemm_dma_kernel<128, 128, false, decltype(kb)::value, 32><<<t, kThreads, 0, st>>>(p, 0u);
-        });
+        run_dma(form, p, DmaLaunch{DmaLaunch::kSmall, dim3(t), 0u, 0u, 0u}, b_layout, st);
         return launch_status("ascq_matmul_w8a8");
     }
     p.k_splits = splits;
     p.partial = static_cast<int32_t*>(workspace);
-    with_b_layout(b_layout, [&](auto kb) {
-        gemm_dma_kernel<128, 128, true, decltype(kb)::value, 32><<<dim3(t, splits), kThreads, 0, st>>>(p, 0u);
-    });
+    run_dma(form, p, DmaLaunch{DmaLaunch::kSplit, dim3(t, splits), 0u, 0u, 0u}, b_layout, st);
     int rc = launch_status("ascq_matmul_w8a8 (split-K)");
     if (rc != ASCQ_OK) {
         return rc;

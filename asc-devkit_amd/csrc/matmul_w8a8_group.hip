@@ -30,10 +30,12 @@ __device__ __forceinline__ void group_row_tiles(uint32_t rows, uint32_t& big, ui
 }
 
 // One phase of the grouped kernel's plan (see gemm_dma_group_kernel): the workgroup's ids that fall into it.
+// (tiles of at most 128 rows never run the 16 x 16 x 64 instruction)
 template <uint32_t phase, int kForm>
 __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const uint32_t* PLAN, char* A0, char* B0,
                                                      char* A1, char* B1, float* TS)
 {
+    constexpr int kSmall = kForm == k16 ? k32 : kForm;
     for (uint32_t id = blockIdx.x;; id += gridDim.x) {
         const uint32_t tiles_n = p.tiles_n;
         const uint32_t big_tiles = __builtin_amdgcn_readfirstlane(PLAN[0]);
@@ -89,9 +91,9 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
         } else if constexpr (phase == 1) {
             gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, A0, B0, A1, B1, TS);
         } else if (at.row_end - at.row0 <= 64u) {  // uniform: a remainder of at most 64 rows
-            gemm_dma_tile_at<64, 256, false, true, 0, 32>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, A0, B0, A1, B1, TS);
         } else {
-            gemm_dma_tile_at<128, 256, false, true, 0, 32>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, A0, B0, A1, B1, TS);
         }
         __syncthreads();  // the next tile's loads and token scales overwrite what slower wavefronts may still read
     }
@@ -177,7 +179,14 @@ int launch_gemm_dma_group(GemmParams& p, hipStream_t st)
         plan_note(ASCQ_MM_KERNEL_DMA_256, 256, 256, BK, wgs, 1, 2u * (256u * BK + BK * 256u) + 256u * 4u, 0);
         return ASCQ_OK;
     }
-    with_form(p, [&](auto form) { gemm_dma_group_kernel<decltype(form)::value><<<wgs, kThreads, 0, st>>>(p); });
+    const int form = gemm_dma_form(p);
+    if (form == k32Ragged) {
+        gemm_dma_group_kernel<k32Ragged><<<wgs, kThreads, 0, st>>>(p);
+    } else if (form == k16) {
+        gemm_dma_group_kernel<k16><<<wgs, kThreads, 0, st>>>(p);
+    } else {
+        gemm_dma_group_kernel<k32><<<wgs, kThreads, 0, st>>>(p);
+    }
     return launch_status("ascq_group_matmul_w8a8");
 }
 

@@ -35,6 +35,10 @@ namespace {
 constexpr int kThreads = 512;
 constexpr int BK = 128;
 
+// The forms of a tile: its matrix instruction (gemm_dma_form says which one runs where), and whether k may end inside a
+// step.  Looking for that step costs about 1 % (600 x 4096 x 4096 43.5 -> 43.9 us), so it is a form of its own.
+constexpr int k16 = 16, k32 = 32, k32Ragged = 33;
+
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* gptr_t;
 typedef i32x2_t __attribute__((address_space(3)))* lds_v2_t;
@@ -756,8 +760,7 @@ __device__ __forceinline__ void gemm_dma_body32(const GemmParams& p, const TileP
 
 // kB: how B lies in memory.  0: [k, n] (or the fractal panels); 1: [n, k]; 2: the layout of ascq_pack_weight_w8
 // (slabs of 16 columns, each a run of 1 KiB tiles of 64 k: lane l of a tile owns column l % 16, k 16 (l / 16) .. + 15).
-// kForm: 16 or 32, the matrix instruction (gemm_dma_body16, gemm_dma_body32; gemm_dma_form says which one runs where).
-// k is any multiple of 16 (the pieces of a last, partial step that lie past k arrive as zeros).  With kB = 0 and an n
+// k is a multiple of BK, with k32Ragged of 16 (the pieces of a last, partial step that lie past k arrive as zeros).  With kB = 0 and an n
 // that is no multiple of 16 the last tile is moved left until it ends at n (n >= BN then): the columns it shares with
 // its neighbour are computed twice, with the same values.
 template <int BM, int BN, bool kSplitK, bool kGrouped, int kB, int kForm>
@@ -821,7 +824,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
         // row kb = s / kPieces; the swizzle spreads the 8 rows of a transposing read over half of the banks and, in the
         // 16 x 16 form, the rows 16 further, which are read beside them, over the other half
         const uint32_t kb = s / kPieces;
-        const uint32_t q = (s % kPieces) ^ (BN == 256 ? 2u * (kb & 7u) : 2u * ((kb >> 1) & 3u)) ^ (kForm == 16 ? (kb >> 4) & 1u : 0u);
+        const uint32_t q = (s % kPieces) ^ (BN == 256 ? 2u * (kb & 7u) : 2u * ((kb >> 1) & 3u)) ^ (kForm == k16 ? (kb >> 4) & 1u : 0u);
         uint32_t col = n0 + 16u * q;
         col = col + 16u <= N ? col : N - 16u;      // columns past the end are never stored
         // fractal B: panels of 32 columns, each a contiguous row-major [K][32] block
@@ -829,7 +832,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     }
     const uint32_t ldb = kBT ? 1u : kBP ? 16u : p.b_nz ? 32u : N;  // bytes from one k to the next
     // K range of this workgroup, in steps of BK
-    const uint32_t all_steps = (K + BK - 1u) / BK;
+    const uint32_t all_steps = kForm == k32Ragged ? (K + BK - 1u) / BK : K / BK;
     uint32_t s_begin = 0, steps = all_steps;
     if constexpr (kSplitK) {
         s_begin = steps * bidy / p.k_splits;
@@ -856,7 +859,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
         for (int u = 0; u < kAInstr; ++u) asm volatile("" : "+v"(aoff[u]));
 #pragma unroll
         for (int u = 0; u < kBInstr; ++u) asm volatile("" : "+v"(boff[u]));
-        if (__builtin_expect(step == partial, 0)) {  // uniform, once per tile at most
+        if (kForm == k32Ragged && step == partial) {  // uniform, once per tile at most
             const uint32_t left = K - (s_begin + step) * BK;
             const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(ab), 0, 0x7FFFFF00, 0x00020000);
             const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(bb), 0, 0x7FFFFF00, 0x00020000);
@@ -886,7 +889,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
         }
     };
 
-    if constexpr (kForm == 16) {
+    if constexpr (kForm == k16) {
         static_assert(!kSplitK, "K splits run the other form");
         gemm_dma_body16<BM, BN, kGrouped, kB>(p, at, n0, steps, wave, lane, issue, A0, B0, A1, B1, TS);
     } else {
@@ -904,25 +907,115 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
 //   k = 2048, grouped: 160 41.8 and 42.9, 256 53.8 and 53.4, 512 with SwiGLU 118 and 121, 1024 157 and 154;
 //   k = 1024: 256 22.0 and 21.7, 1024 92.6 and 94.8; k = 512: 256 15.7 and 15.5, 258 21.5 and 22.2.
 // Outputs other than half and bfloat16 are what the other form writes from registers.
-int gemm_dma_form(const GemmParams& p)
+inline int gemm_dma_form(const GemmParams& p)
 {
+    if (p.k % BK != 0) {
+        return k32Ragged;
+    }
     if (p.epi.quant_mode == ASCQ_MM_QUANT_NONE || (p.epi.out_dtype != ASCQ_F16 && p.epi.out_dtype != ASCQ_BF16)) {
-        return 32;
+        return k32;
     }
     const uint64_t tiles = static_cast<uint64_t>((p.m + 255u) / 256u) * ((p.n + 255u) / 256u);
-    return p.k >= 3072u && 4u * tiles >= 3u * device_compute_units() ? 16 : 32;
+    return p.k >= 3072u && 4u * tiles >= 3u * device_compute_units() ? k16 : k32;
 }
 
-// calls f with it as a compile-time constant
-template <class F>
-void with_form(const GemmParams& p, F&& f)
+// The plain matmul: tile number `bid` of the launch (before the XCD remapping), column tiles counted from col_begin,
+// row tiles innermost so that the tiles an XCD runs side by side share their B columns.
+template <int BM, int BN, bool kSplitK, int kB, int kForm>
+__device__ __forceinline__ void gemm_dma_tile(const GemmParams& p, uint32_t col_begin, uint32_t bid, uint32_t bidy,
+                                              char* A0, char* B0, char* A1, char* B1, float* TS)
 {
-    if (gemm_dma_form(p) == 16) {
-        f(std::integral_constant<int, 16>{});
+    const uint32_t total = p.tiles_m * p.tiles_n;
+    const uint32_t t = xcd_remap(bid, total);
+    if (t >= total) {
+        return;
+    }
+    // bands of 8 row tiles, inside a band column by column (band_order): an XCD's share stays a block of a few columns
+    // by 8 rows whose rows of A and columns of B it reuses from its L2, however many rows the matrix has
+    uint32_t ms, tn;
+    band_order(t, p.tiles_m, p.tiles_n, ms, tn);
+    const TilePlace at{ms * BM, p.m, col_begin + tn * BN, p.b, 0};
+    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, A0, B0, A1, B1, TS);
+}
+
+template <int BM, int BN, bool kSplitK, int kB, int kForm>
+__global__ __launch_bounds__(kThreads, (BM * BK + BK * BN) * 2 <= 65536 ? 2 : 1) void gemm_dma_kernel(
+    GemmParams p, uint32_t col_begin)
+{
+    __shared__ __attribute__((aligned(1024))) char A0[BM * BK];
+    __shared__ __attribute__((aligned(1024))) char B0[BK * BN];
+    __shared__ __attribute__((aligned(1024))) char A1[BM * BK];
+    __shared__ __attribute__((aligned(1024))) char B1[BK * BN];
+    __shared__ __attribute__((aligned(16))) float TS[BM];  // token scales of the tile's rows (1.0f when there are none)
+    gemm_dma_tile<BM, BN, kSplitK, kB, kForm>(p, col_begin, blockIdx.x, blockIdx.y, A0, B0, A1, B1, TS);
+}
+
+// One launch for a matrix whose last round of 256 x 256 tiles would be mostly empty: workgroups [0, wide_wgs) run the
+// 256 x 256 tiles of the first `p.tiles_n` tile columns, the rest 256 x 128 tiles of the remaining columns.  A compute
+// unit that has finished its wide tile takes a narrow one at once, without the drain between two launches.
+template <int kB, int kForm>
+__global__ __launch_bounds__(kThreads, 1) void gemm_dma_dual_kernel(GemmParams p, uint32_t wide_wgs,
+                                                                    uint32_t narrow_tiles_n, uint32_t col_begin)
+{
+    __shared__ __attribute__((aligned(1024))) char A0[256 * BK];
+    __shared__ __attribute__((aligned(1024))) char B0[BK * 256];
+    __shared__ __attribute__((aligned(1024))) char A1[256 * BK];
+    __shared__ __attribute__((aligned(1024))) char B1[BK * 256];
+    __shared__ __attribute__((aligned(16))) float TS[256];
+    if (blockIdx.x < wide_wgs) {
+        gemm_dma_tile<256, 256, false, kB, kForm>(p, 0u, blockIdx.x, 0u, A0, B0, A1, B1, TS);
     } else {
-        f(std::integral_constant<int, 32>{});
+        GemmParams q = p;
+        q.tiles_n = narrow_tiles_n;
+        gemm_dma_tile<256, 128, false, kB, kForm>(q, col_begin, blockIdx.x - wide_wgs, 0u, A0, B0, A1, B1, TS);
     }
 }
 
 }  // namespace
+
+// One launch of the plain matmul's kernels.
+struct DmaLaunch {
+    enum Shape { kWide, kNarrow, kBoth, kSmall, kSplit } shape;  // 256 x 256, 256 x 128, both, 128 x 128, those with K split
+    dim3 grid;
+    uint32_t col_begin, wide_wgs, narrow_tiles_n;
+};
+
+namespace {
+
+template <int kB, int kForm>
+void run_dma_layout(const GemmParams& p, const DmaLaunch& l, hipStream_t st)
+{
+    if (l.shape == DmaLaunch::kBoth) {
+        gemm_dma_dual_kernel<kB, kForm><<<l.grid, kThreads, 0, st>>>(p, l.wide_wgs, l.narrow_tiles_n, l.col_begin);
+    } else if (l.shape == DmaLaunch::kWide) {
+        gemm_dma_kernel<256, 256, false, kB, kForm><<<l.grid, kThreads, 0, st>>>(p, l.col_begin);
+    } else if constexpr (kForm != k16) {
+        if (l.shape == DmaLaunch::kNarrow) {
+            gemm_dma_kernel<256, 128, false, kB, kForm><<<l.grid, kThreads, 0, st>>>(p, l.col_begin);
+        } else if (l.shape == DmaLaunch::kSmall) {
+            gemm_dma_kernel<128, 128, false, kB, kForm><<<l.grid, kThreads, 0, st>>>(p, l.col_begin);
+        } else {
+            gemm_dma_kernel<128, 128, true, kB, kForm><<<l.grid, kThreads, 0, st>>>(p, l.col_begin);
+        }
+    }
+}
+
+// b_layout: 0 [k, n], 1 [n, k], 2 packed by ascq_pack_weight_w8
+template <int kForm>
+void run_dma(const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t st)
+{
+    if (b_layout == 2) {
+        run_dma_layout<2, kForm>(p, l, st);
+    } else if (b_layout == 1) {
+        run_dma_layout<1, kForm>(p, l, st);
+    } else {
+        run_dma_layout<0, kForm>(p, l, st);
+    }
+}
+
+}  // namespace
+
+// matmul_w8a8_ragged.hip (a translation unit of its own: the kernels take minutes to compile)
+void run_dma_ragged(const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t st);
+
 }  // namespace ascq
