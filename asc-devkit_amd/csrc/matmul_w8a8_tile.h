@@ -615,6 +615,9 @@ __device__ __forceinline__ void gemm_dma_body32(const GemmParams& p, const TileP
                     bias_pre[j] = static_cast<const int32_t*>(e.bias)[chan_off + col];
                 }
             }
+            // Wait for the conditional loads here: left to itself the compiler waits at each use, and each such wait is one
+            // for the stores before it (2048 x 4096 x 11008, int32 98 -> 105 us).
+            asm volatile("" : "+v"(q[j].s), "+v"(bias_post[j]), "+v"(bias_pre[j]));
         }
         // The uniform choices (post-dequant bias, activation) are made once, outside the element loops, so that each
         // wavefront runs one compact straight-line epilogue.
