@@ -653,26 +653,38 @@ bool fast_path_ok(const ascq_matmul_desc* d, const void* a, const void* b)
 // Up to this many rows the 128 x 128 direct-to-LDS kernel (K split over workgroups) is used when the shape allows.
 constexpr uint32_t kSkinnyMaxM = 512;
 
-// Packed weights between 129 and 512 rows: true when the 128 x 128 tiles (`splits` of K, 1 without a workspace) are
-// expected to beat the weights-in-registers form.  Both estimates are fits to measurements at
-// k = 4096, n = 11008 and k = 11008, n = 4096 (the crossovers there: 256 and about 380 rows).  Registers form: the
-// weights once (5 us + 1 us per 4.7 MB), then 0.95 us per 16 rows and 4096 of k, per round of workgroups.  Tiles:
+// Packed weights between 129 and 512 rows, estimates of the three forms in us.  Registers form: the weights once (5 us +
+// 1 us per 4.7 MB), then 0.95 us per 16 rows and 4096 of k, per round of workgroups.
+double packed_ws_us(const GemmParams& p)
+{
+    return 5.0 + static_cast<double>(p.n) * p.k / 4.7e6 + 0.95 * (p.k / 4096.0) * ((p.m + 15u) / 16u) * gemm_ws_rounds(p);
+}
+
+// True when the 128 x 128 tiles, unsplit, are expected to beat the weights-in-registers form.  Both estimates are fits to
+// measurements at k = 4096, n = 11008 and k = 11008, n = 4096 (the crossovers there: 256 and about 380 rows).  Tiles:
 // 6.5 us per 1024 of k for up to one tile per compute unit, 1.45 times that with two (they share the unit), and in
 // proportion beyond.  Above 512 rows the 256-row tiles always lead.
-bool packed_tiles_faster(const GemmParams& p, uint32_t splits)
+bool packed_tiles_faster(const GemmParams& p)
 {
     const double kk = p.k / 4096.0;
-    const double ws_us = 5.0 + static_cast<double>(p.n) * p.k / 4.7e6 +
-                         0.95 * kk * ((p.m + 15u) / 16u) * gemm_ws_rounds(p);
     const double tiles = static_cast<double>((p.m + 127u) / 128u) * ((p.n + 127u) / 128u);
     const double cus = device_compute_units();
     const double load = tiles <= cus ? 1.0 : tiles <= 2.0 * cus ? 1.0 + 0.45 * (tiles - cus) / cus : 1.45 * tiles / (2.0 * cus);
     const double tiles_us = 4.0 + 26.0 * kk * load;
-    if (splits > 1u) {  // a second launch, and the partial tiles written and read back (gemm_dma_small_tiles)
-        const double split_us = 8.0 + 26.0 * kk / splits + static_cast<double>(splits) * p.m * p.n * 8.0 / 5e6;
-        return (split_us < tiles_us ? split_us : tiles_us) < ws_us;
-    }
-    return tiles_us < ws_us;
+    return tiles_us < packed_ws_us(p);
+}
+
+// Whether those tiles with K split in `splits` are ahead of what runs without a workspace, the registers form or the tiles
+// unsplit (4 us + 4.45 us per 1024 of k: at most 160 of them, a unit for each).  Split: 4.45 us per 1024 of a workgroup's k,
+// two launches, and the partial tiles written and read back at 4.5 TB/s.  Measured, quantiser included: unsplit against
+// split k = n = 4096, 512 rows 27.9 and 32.2; k = n = 2048, 400 rows 16.8 and 22.3; k = 1024, n = 4096, 512 rows 14.5 and 22.8; k =
+// 4096, n = 1024, 512 rows 27.6 and 22.8; k = 11008, n = 4096, 512 rows 60.8 and 54.0; registers form against split k = n =
+// 4096, 192 rows 24.9 and 25.2, 256 rows 28.2 and 26.7; k = 4096, n = 6144, 192 rows 24.6 and 27.1; k = 8192, n = 2048, 300 rows
+// 45.3 and 26.9.
+bool packed_split_faster(const GemmParams& p, uint32_t splits)
+{
+    const double split_us = 9.5 + 4.45 * (p.k / 1024.0) / splits + static_cast<double>(splits) * p.m * p.n * 8.0 / 4.5e6;
+    return split_us < (packed_tiles_faster(p) ? 4.0 + 4.45 * p.k / 1024.0 : packed_ws_us(p) - 0.7);
 }
 // Up to this many rows the weight-stream kernel is preferred over those tiles.
 constexpr uint32_t kStreamMaxM = 8;
@@ -1051,7 +1063,10 @@ int matmul_w8a8_packed(const ascq_matmul_desc* d, void* c, const void* a, const 
         workspace_bytes < static_cast<size_t>(splits) * d->m * d->n * sizeof(int32_t)) {
         splits = 1;
     }
-    if (tiles_ok && (d->m > kSkinnyMaxM || (d->m > 128u && packed_tiles_faster(p, splits)))) {
+    if (splits > 1u && d->m <= kSkinnyMaxM && !packed_split_faster(p, splits)) {
+        splits = 1;
+    }
+    if (tiles_ok && (d->m > kSkinnyMaxM || (d->m > 128u && (splits > 1u || packed_tiles_faster(p))))) {
         const bool small = d->m <= kSkinnyMaxM || (splits > 1u && gemm_dma_small_tiles(d->m, d->n, d->k));
         return small ? launch_gemm_dma_skinny(p, workspace, splits > 1u ? workspace_bytes : 0, static_cast<hipStream_t>(stream), 2)
                      : launch_gemm_dma(p, static_cast<hipStream_t>(stream), 2);

@@ -1270,10 +1270,11 @@ def test_w8a8_few_rows_on_unaligned_columns(m, k, n):
     assert np.array_equal(bits(c), orc.matmul_w8a8(d, q, b, bias, cs, ts))
 
 
-@pytest.mark.parametrize("m", [129, 300, 600])
-@pytest.mark.parametrize("k,n", [(64, 40), (1472, 512), (5888, 520), (4096, 1024)])
+@pytest.mark.parametrize("m", [129, 300, 480, 600])
+@pytest.mark.parametrize("k,n", [(64, 40), (1472, 512), (5888, 520), (4096, 1024), (1024, 2048)])
 def test_linear_w8a8_dynamic_packed_split_over_k(m, k, n):
-    """Packed weights with too few tiles for the chip: K split over workgroups, the pieces in the call's workspace."""
+    """Packed weights with too few tiles for the chip: K split over workgroups, the pieces in the call's workspace, or,
+    where that costs more than it gives (the last shape, up to 512 rows), the tiles as they are."""
     announce("linear dynamic packed, K split", m, k, n)
     rng = np.random.default_rng(m + k + n)
     x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(DEV).to(torch.float16)
