@@ -905,7 +905,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
 // energy per product, and the 16 x 16 x 64 instruction moves half the sums.  Away from that limit it loses: behind a step's
 // barrier it waits for the reads of a 64-k sub-step where the other waits for a 32-k one.  The limit is met by most of
 // the chip's units busy for a good while; in us, 32 x 32 x 32 and 16 x 16 x 64:
-//   k = 4096, plain: 128 tiles 44.9 and 45.6, 172 47.9 and 48.1, 192 50.5 and 49.2, 224 55.9 and 53.9, 256 61.0 and 57.9, 344
+//   k = 4096, plain: 128 tiles 44.9 and 45.6, 172 47.9 and 48.1 (packed weights 53.4 and 51.3), 192 50.5 and 49.2, 224 55.9 and 53.9, 256 61.0 and 57.9, 344
 //   90.6 and 86.2, 688 168 and 163; grouped: 128 67.0 and 67.3, 448 190 and 179, 896 293 and 279;
 //   k = 2048, grouped: 160 41.8 and 42.9, 256 53.8 and 53.4, 512 with SwiGLU 118 and 121, 1024 157 and 154;
 //   k = 1024: 256 22.0 and 21.7, 1024 92.6 and 94.8; k = 512: 256 15.7 and 15.5, 258 21.5 and 22.2.
@@ -919,7 +919,7 @@ inline int gemm_dma_form(const GemmParams& p)
         return k32;
     }
     const uint64_t tiles = static_cast<uint64_t>((p.m + 255u) / 256u) * ((p.n + 255u) / 256u);
-    return p.k >= 3072u && 4u * tiles >= 3u * device_compute_units() ? k16 : k32;
+    return p.k >= 3072u && 3u * tiles >= 2u * device_compute_units() ? k16 : k32;
 }
 
 // The plain matmul: tile number `bid` of the launch (before the XCD remapping), column tiles counted from col_begin,
