@@ -577,9 +577,10 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     bool wa, wb;
     mx_widen_plan(d, wa, wb);
     const bool four = is_fp4(d->a_format) && !wa;  // both e2m1
-    // two e1m2 operands: the 6-bit codes of rows rounded up to 32 must fit the workspace of a byte per value
-    auto fits = [](uint32_t rows) { return (static_cast<uint64_t>(rows) + 31u) / 32u * 24u <= rows; };
-    if (d->a_format == ASCQ_QDST_FP4_E1M2 && d->b_format == ASCQ_QDST_FP4_E1M2 && !(fits(d->m) && fits(d->n))) {
+    // two e1m2 operands: the 6-bit codes of their rows, each rounded up to 32, must fit the workspace of a byte per value
+    // (24 bytes for 32 values; only some pairs of little over 64 rows do not)
+    const uint64_t blocks = (static_cast<uint64_t>(d->m) + 31u) / 32u + (static_cast<uint64_t>(d->n) + 31u) / 32u;
+    if (d->a_format == ASCQ_QDST_FP4_E1M2 && d->b_format == ASCQ_QDST_FP4_E1M2 && blocks * 24u > static_cast<uint64_t>(d->m) + d->n) {
         return false;
     }
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
@@ -702,8 +703,9 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         fmt = ASCQ_QDST_FP8_E4M3FN;
     };
     if (six) {
-        MxWidenParams w{{p.a, p.b}, {ws, ws + static_cast<size_t>(d->m) * d->k}, {d->m, d->n}, 0, (d->k + 255u) / 256u, d->k};
-        w.a_blocks = (d->m + 31u) / 32u * w.k_blocks;
+        const uint32_t a_rows = (d->m + 31u) / 32u;
+        MxWidenParams w{{p.a, p.b}, {ws, ws + static_cast<size_t>(a_rows) * 24u * d->k}, {d->m, d->n}, 0, (d->k + 255u) / 256u, d->k};
+        w.a_blocks = a_rows * w.k_blocks;
         mx_widen_e1m2_kernel<<<w.a_blocks + (d->n + 31u) / 32u * w.k_blocks, 256, 0, st>>>(w);
         p.a = w.dst[0];
         p.b = w.dst[1];
