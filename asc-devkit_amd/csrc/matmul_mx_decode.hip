@@ -14,13 +14,14 @@
 // 37 us.  32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
 // streams half the bytes: n = 1024, k = 14336, e4m3, 9 against 14 us).
 //
-// Two e2m1 operands run v_mfma_scale_f32_16x16x128_f8f6f4, one scale byte per lane: lane l holds the scale of row l % 16
-// and block of 32 k number l / 16, and in four registers that row's block.  Their products are whole multiples of 1/4 up
-// to 36, which the instruction adds exactly.
-// Every other pair runs v_mfma_f32_16x16x32_bf16 on operands converted in registers (every fp8 and fp4 value is a
+// Two 4-bit operands run v_mfma_scale_f32_16x16x128_f8f6f4, one scale byte per lane: lane l holds the scale of row l % 16
+// and block of 32 k number l / 16; an e2m1 operand's four registers hold the lane's own block, e1m2, which the instruction
+// does not know, is widened to e4m3 in registers (exact), whose registers 0-3 hold k = 16 (l / 16) .. + 15 and 4-7 k = 64 +
+// 16 (l / 16) .. + 15.  Their products lie less than 2^8 apart, and the instruction drops none.
+// A pair with fp8 runs v_mfma_f32_16x16x32_bf16 on operands converted in registers (every fp8 and fp4 value is a
 // bfloat16 value, every product of two exact in fp32), one instruction per block of 32 k from zero, whose sums the vector
 // ALU scales and adds: the arithmetic of the kernel with one lane per output element.  The scaled instruction is not good
-// enough for them: it aligns the 128 products of two 8-bit operands to the largest and drops what lies 2^13 below it.
+// enough for them: it aligns the products of fp8 operands to the largest and drops what lies 2^13 below it.
 // Against 64 bits (2-norm, k = 8192, 16 rows, normally distributed e4m3): scaled instruction 1.3e-5, one lane per output
 // 2.2e-7, this 9.2e-8; e2m1 x e4m3 3.0e-7, 1.2e-7 and 6.8e-8.  That arithmetic is also what bounds these pairs from 16
 // rows on: per block of 32 k and 16 x 16 results a multiplication and an addition per sum beside the conversions (e4m3,
@@ -43,8 +44,8 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 // operand formats: the instruction's codes, and e1m2
 enum { kE4M3 = 0, kE5M2 = 1, kE2M1 = 4, kE1M2 = 5 };
 constexpr bool fmt_is_8bit(int f) { return f == kE4M3 || f == kE5M2; }
-// the pair that the scaled matrix instruction adds up exactly; the others go through bfloat16
-constexpr bool fmt_scaled(int fa, int fb) { return fa == kE2M1 && fb == kE2M1; }
+// the pairs whose products the scaled matrix instruction adds up without dropping any; those with fp8 go through bfloat16
+constexpr bool fmt_scaled(int fa, int fb) { return !fmt_is_8bit(fa) && !fmt_is_8bit(fb); }
 constexpr uint32_t kPastEnd = 0x7FFFFFF0u;  // an offset every buffer's range check rejects: the load moves no data
 
 // A batch is 128 bytes of a weight column: KB values of k.
@@ -65,9 +66,18 @@ struct MxdShape {
     static_assert(lds <= 158u * 1024u && loads * 2u < 63u, "the ring must fit the LDS and the load counter");
 };
 
-// 8 values of a format as bfloat16, every one exact (the scale operand of the conversions is 1).  e1m2 goes by way of
-// e4m3: a magnitude code c is the value c / 4, and the eight e4m3 codes are a byte table in two registers that a byte
-// permute looks up.
+// 8 e1m2 values (a dword, the even one of a byte in the low nibble) -> 8 e4m3 codes in order.  A magnitude code c is the
+// value c / 4; the eight e4m3 codes are a byte table in two registers that a byte permute looks up.
+__device__ __forceinline__ i32x2_t widen_e1m2(uint32_t q)
+{
+    constexpr uint32_t lut_hi = 0x3E3C3A38u, lut_lo = 0x34302800u;
+    const uint32_t ve = __builtin_amdgcn_perm(lut_hi, lut_lo, q & 0x07070707u) | ((q << 4) & 0x80808080u);
+    const uint32_t vo = __builtin_amdgcn_perm(lut_hi, lut_lo, (q >> 4) & 0x07070707u) | (q & 0x80808080u);
+    return i32x2_t{static_cast<int>(__builtin_amdgcn_perm(vo, ve, 0x05010400u)),
+                   static_cast<int>(__builtin_amdgcn_perm(vo, ve, 0x07030602u))};
+}
+
+// 8 values of a format as bfloat16, every one exact (the scale operand of the conversions is 1)
 template <int F>
 __device__ __forceinline__ bf16x8_t to_bf16(const typename std::conditional<fmt_is_8bit(F), i32x2_t, uint32_t>::type raw)
 {
@@ -79,25 +89,21 @@ __device__ __forceinline__ bf16x8_t to_bf16(const typename std::conditional<fmt_
         put(2, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 2));
         put(3, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, 1.0f, 3));
     } else {
-        uint32_t d[2];
+        i32x2_t d;
         if constexpr (F == kE1M2) {
-            constexpr uint32_t lut_hi = 0x3E3C3A38u, lut_lo = 0x34302800u;
-            const uint32_t ve = __builtin_amdgcn_perm(lut_hi, lut_lo, raw & 0x07070707u) | ((raw << 4) & 0x80808080u);
-            const uint32_t vo = __builtin_amdgcn_perm(lut_hi, lut_lo, (raw >> 4) & 0x07070707u) | (raw & 0x80808080u);
-            d[0] = __builtin_amdgcn_perm(vo, ve, 0x05010400u);
-            d[1] = __builtin_amdgcn_perm(vo, ve, 0x07030602u);
+            d = widen_e1m2(raw);
         } else {
-            d[0] = static_cast<uint32_t>(raw[0]);
-            d[1] = static_cast<uint32_t>(raw[1]);
+            d = raw;
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
+            const uint32_t v = static_cast<uint32_t>(d[i]);
             if constexpr (F == kE5M2) {
-                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(d[i], 1.0f, false));
-                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(d[i], 1.0f, true));
+                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(v, 1.0f, false));
+                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(v, 1.0f, true));
             } else {
-                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d[i], 1.0f, false));
-                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d[i], 1.0f, true));
+                put(2 * i, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, false));
+                put(2 * i + 1, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, true));
             }
         }
     }
@@ -260,6 +266,8 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
         const uint32_t per = row_bytes / 16u;
         return lc * row_bytes + ((piece ^ ((lc / (16u / per)) & (per - 1u))) << 4);
     };
+    constexpr std::integral_constant<int, FA> fa{};
+    constexpr std::integral_constant<int, FB> fb{};
     constexpr std::integral_constant<uint32_t, T::arb> arb{};
     constexpr std::integral_constant<uint32_t, T::brb> brb{};
     // loads return in order: everything but the newest batch has landed
@@ -268,35 +276,60 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
         asm volatile("" ::: "memory");
     };
 
-    // Two e2m1 operands: a lane's 16 bytes of a tile are the instruction's operand as they lie.
+    // Two 4-bit operands.  e2m1: a lane's 16 bytes of a tile are the instruction's operand as they lie; e1m2, which the
+    // instruction does not know: the two times 8 bytes that widened to e4m3 are the lane's operand of 8 bits.
     auto step_scaled = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
         const uint32_t abase = ring_addr + slot_off, bbase = abase + T::a_bytes, sbase = bbase + T::b_bytes;
         const uint32_t slane = sbase + lc * (4u * T::sdw) + lq;
-        i32x4 ar[T::tiles][RT], br[T::tiles][S];
+        struct Raw {
+            i32x4 v;           // e2m1
+            i32x2_t h0, h1;    // e1m2
+        };
+        auto read = [&](auto fmt, auto line, auto row_bytes, auto tt, uint32_t base) __attribute__((always_inline)) {
+            constexpr uint32_t bytes = decltype(row_bytes)::value, off = decltype(line)::value * 16u * bytes, tl = decltype(tt)::value;
+            Raw r;
+            if constexpr (decltype(fmt)::value == kE2M1) {
+                r.v = lds_b128<off>(base + at(bytes, 4u * tl + lq));
+            } else {
+                r.h0 = lds_b64<off>(base + at(bytes, 4u * tl + (lq >> 1)) + 8u * (lq & 1u));
+                r.h1 = lds_b64<off>(base + at(bytes, 4u * tl + 2u + (lq >> 1)) + 8u * (lq & 1u));
+            }
+            return r;
+        };
+        auto landed = [](auto fmt, Raw& r, uint32_t& scale) __attribute__((always_inline)) {  // usable from here on
+            if constexpr (decltype(fmt)::value == kE2M1) {
+                asm volatile("" : "+v"(r.v), "+v"(scale));
+            } else {
+                asm volatile("" : "+v"(r.h0), "+v"(r.h1), "+v"(scale));
+            }
+        };
+        auto operand = [](auto fmt, const Raw& r) __attribute__((always_inline)) {
+            if constexpr (decltype(fmt)::value == kE2M1) {
+                return __builtin_shufflevector(r.v, r.v, 0, 1, 2, 3, -1, -1, -1, -1);
+            } else {
+                const i32x2_t a = widen_e1m2(static_cast<uint32_t>(r.h0[0])), b = widen_e1m2(static_cast<uint32_t>(r.h0[1]));
+                const i32x2_t c = widen_e1m2(static_cast<uint32_t>(r.h1[0])), d = widen_e1m2(static_cast<uint32_t>(r.h1[1]));
+                return v8i{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+            }
+        };
+        constexpr int kCodeA = FA == kE1M2 ? kE4M3 : FA, kCodeB = FB == kE1M2 ? kE4M3 : FB;
+        Raw ar[T::tiles][RT], br[T::tiles][S];
         uint32_t asc[T::tiles][RT], bsc[T::tiles][S];
         mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {
             constexpr uint32_t tl = decltype(tt)::value;
             mxd_for<S>([&](auto j) {
-                br[tl][j] = lds_b128<decltype(j)::value * 16u * T::brb>(bbase + at(brb, 4u * tl + lq));
+                br[tl][j] = read(fb, j, brb, tt, bbase);
                 bsc[tl][j] = lds_u8<(RT + decltype(j)::value) * 64u * T::sdw + 4u * tl>(slane);
             });
             mxd_for<RT>([&](auto i) {
-                ar[tl][i] = lds_b128<decltype(i)::value * 16u * T::arb>(abase + at(arb, 4u * tl + lq));
+                ar[tl][i] = read(fa, i, arb, tt, abase);
                 asc[tl][i] = lds_u8<decltype(i)::value * 64u * T::sdw + 4u * tl>(slane);
             });
         });
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {  // the registers may be used from here on
-            mxd_for<S>([&](auto j) {
-                i32x4& r = br[tt][j];
-                uint32_t& v = bsc[tt][j];
-                asm volatile("" : "+v"(r), "+v"(v));
-            });
-            mxd_for<RT>([&](auto i) {
-                i32x4& r = ar[tt][i];
-                uint32_t& v = asc[tt][i];
-                asm volatile("" : "+v"(r), "+v"(v));
-            });
+        mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {
+            mxd_for<S>([&](auto j) { landed(fb, br[tt][j], bsc[tt][j]); });
+            mxd_for<RT>([&](auto i) { landed(fa, ar[tt][i], asc[tt][i]); });
         });
         load(b + 2u, ring + slot_off);  // the slot is free again
         mxd_for<static_cast<int>(T::tiles)>([&](auto tt) {
@@ -305,23 +338,27 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
             if (tile < tb) {  // uniform
                 // blocks past the end of k hold zeros; their scale bytes may be anything, a NaN too
                 const bool in_k = tile * 4u + lq < q.blocks;
-                auto operand = [](const i32x4& r) __attribute__((always_inline)) {
-                    return __builtin_shufflevector(r, r, 0, 1, 2, 3, -1, -1, -1, -1);
-                };
+                v8i bo[S];
+                int bs[S];
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    bo[j] = operand(fb, br[tl][j]);
+                    bs[j] = in_k ? static_cast<int>(bsc[tl][j]) : 127;
+                }
 #pragma unroll
                 for (int i = 0; i < RT; ++i) {
+                    const v8i ao = operand(fa, ar[tl][i]);
+                    const int as = in_k ? static_cast<int>(asc[tl][i]) : 127;
 #pragma unroll
                     for (int j = 0; j < S; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            operand(ar[tl][i]), operand(br[tl][j]), acc[i][j], kE2M1, kE2M1, 0,
-                            in_k ? static_cast<int>(asc[tl][i]) : 127, 0, in_k ? static_cast<int>(bsc[tl][j]) : 127);
+                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ao, bo[j], acc[i][j], kCodeA, kCodeB, 0, as, 0, bs[j]);
                     }
                 }
             }
         });
     };
 
-    // Any other pair: lane l holds k = 32 blk + 8 (l / 16) .. + 7 of row l % 16 for each of a tile's four blocks blk, and
+    // A pair with fp8: lane l holds k = 32 blk + 8 (l / 16) .. + 7 of row l % 16 for each of a tile's four blocks blk, and
     // the scale bytes of its four rows of the result (rows 4 (l / 16) .. + 3) and of its column.
     typedef typename std::conditional<fmt_is_8bit(FA), i32x2_t, uint32_t>::type RawA;
     typedef typename std::conditional<fmt_is_8bit(FB), i32x2_t, uint32_t>::type RawB;
@@ -348,8 +385,6 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
                 return at(row_bytes, 4u * tl + blk) + 4u * lq;
             }
         };
-        constexpr std::integral_constant<int, FA> fa{};
-        constexpr std::integral_constant<int, FB> fb{};
         mxd_for<S>([&](auto j) {
             constexpr uint32_t off = (RT + decltype(j)::value) * 64u * T::sdw;
             if constexpr (T::sdw == 2) {
