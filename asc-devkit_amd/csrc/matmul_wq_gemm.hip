@@ -12,7 +12,9 @@
 // two steps ahead), are de-quantised with the operators' own roundings and written to LDS as halves, one 16-byte piece
 // behind the matrix instructions of each quarter of a step.  Both tiles lie in LDS as lines of 64 halves (128 bytes) whose
 // 16-byte pieces are XOR-swizzled by half the line number, so that 16 lanes reading a piece of 16 neighbouring lines
-// meet all 64 banks, and one piece of a line is the operand of v_mfma_f32_16x16x32_f16 as it lies.  A step's barrier
+// meet all 64 banks, and one piece of a line is the operand of v_mfma_f32_16x16x32_f16 as it lies.  (The conflict cycles that
+// are counted, 17.5 % of the LDS cycles, come to 9 for each of the B tile's writes: 33.9 M for 3.7 M of them at 2048 rows of int8.
+// That fits writes that meet 32 banks at a time, where the pieces of a line and its neighbour meet.)  A step's barrier
 // stands before its last quarter, whose operands are in registers by then: behind it the matrix pipe has work while
 // the next step's loads are issued and its first operands read.
 #include <type_traits>

@@ -415,7 +415,10 @@ int ascq_unpack_int4(void* dst, const void* src, size_t elements, void* stream);
  * baseK ~ tile_m / tile_n / tile_k, shareL1Size ~ lds_bytes); here it is informational, the call plans by itself.
  */
 typedef enum ascq_mm_kernel {
-    ASCQ_MM_KERNEL_GENERIC = 0,      /* one lane per output element: unaligned or transposed-A inputs */
+    ASCQ_MM_KERNEL_GENERIC = 0,      /* unaligned or transposed-A inputs: one lane per output element (tile 1 x 1); up to 32
+                                        rows on [k, n] weights with a workspace of m * n * 4 bytes unaligned dwords of the
+                                        weights, K split over workgroups (tile 32 x 256, three launches: the zero fill, the
+                                        sums, the epilogue) */
     ASCQ_MM_KERNEL_STREAM = 1,       /* few rows: weight streams, one per SIMD, then a kernel that adds their pieces */
     ASCQ_MM_KERNEL_DMA_128 = 2,      /* m <= 512, or few tiles: 128 x 128 direct-to-LDS tiles, K split over workgroups
                                         when a workspace is given (k_splits > 1: a second kernel adds the partial tiles) */
@@ -428,7 +431,7 @@ typedef enum ascq_mm_kernel {
 typedef struct ascq_matmul_plan {
     int32_t kernel;             /* ascq_mm_kernel */
     uint32_t tile_m, tile_n;    /* rows x columns of C per workgroup (per wavefront stream for KERNEL_STREAM: the
-                                   rows x columns a stream accumulates at a time); 1 x 1 for KERNEL_GENERIC */
+                                   rows x columns a stream accumulates at a time) */
     uint32_t tile_k;            /* K per main-loop step */
     uint32_t workgroups;        /* workgroups of the main launch */
     uint32_t k_splits;          /* partial sums per output element (1: the main kernel writes C itself) */
