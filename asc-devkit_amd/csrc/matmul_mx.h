@@ -31,8 +31,9 @@ __device__ __forceinline__ void mx_store(const MxParams& p, size_t idx, float v)
     }
 }
 
-// matmul_mx_decode.hip: whole columns per workgroup, wavefronts split k; any m, n
+// matmul_mx_decode.hip: whole columns per workgroup, wavefronts split k; any m, n.  tile_shape: the tiles could take the call,
+// so fp8 operands may have their precision
 bool mx_decode_supported(const MxParams& p);
-int launch_mx_decode(const MxParams& p, hipStream_t st);
+int launch_mx_decode(const MxParams& p, bool tile_shape, hipStream_t st);
 
 }  // namespace ascq

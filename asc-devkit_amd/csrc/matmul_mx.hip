@@ -589,12 +589,12 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
 
 // Tile shapes (64 rows and more): whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.
 // Both times are estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
-// meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 4.1 (two 8-bit operands), 2.4 (the
-// 32-row form), 3.1 (4-bit a, 8-bit b), 2.0 (two 4-bit operands, one of them e1m2).  Tiles: rounds of 256 x 256 tiles, 1.3
+// meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 1.85 (8-bit b), 0.95 (the 32-row
+// form), 2.0 (two 4-bit operands, one of them e1m2).  Tiles: rounds of 256 x 256 tiles, 1.3
 // per K step, and the passes that widen 4-bit operands, 1 per 3 MB of their codes.  Measured at n = k = 8192, decode
-// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 37 and 77, e1m2 20 and 93; 128 rows e4m3 70 and 78, e1m2 36 and 97;
-// 256 rows e2m1 41 and 47, e4m3 136 and 85, e1m2 69 and 103; n = 14336, k = 4096, 128 rows: 28 and 26, 75 and 44, 42
-// and 64; n = 1024, k = 14336, 256 rows: 16 and 69, 59 and 147, 30 and 154.
+// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 20.7 and 78, e1m2 20 and 93; 128 rows e4m3 34 and 79, e1m2 36 and 97; 256
+// rows e2m1 41 and 47, e4m3 64 and 85, e1m2 69 and 103; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44, 42 and 64;
+// n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147, 30 and 154.
 bool mx_decode_preferred(const MxParams& p)
 {
     const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
@@ -602,7 +602,7 @@ bool mx_decode_preferred(const MxParams& p)
     const double cus = device_compute_units();
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
-    const double per_k = two4 ? 1.15 : a8 && b8 ? 4.1 : a8 ? 2.4 : b8 ? 3.1 : 2.0;
+    const double per_k = two4 ? 1.15 : b8 ? 1.85 : a8 ? 0.95 : 2.0;
     const double decode = 4.0 + rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u)) * per_k * p.k / 1024.0;
     const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
     const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * 1.3 *
@@ -680,7 +680,7 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
                       (reinterpret_cast<uintptr_t>(b_scale) & 7u) == 0 &&
                       (need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned16(workspace)));
     if (mx_decode_supported(p) && (!tile || mx_decode_preferred(p))) {
-        return launch_mx_decode(p, st);
+        return launch_mx_decode(p, tile, st);
     }
     if (!tile) {
         const uint32_t arb = is_fp4(d->a_format) ? d->k / 2u : d->k, brb = is_fp4(d->b_format) ? d->k / 2u : d->k;

@@ -11,21 +11,22 @@
 // only up to a few hundred rows (mx_decode_preferred).  n = k = 8192, 16 rows, with one lane per output element before:
 // e2m1 4830 -> 8.9 us a call (4.0 TB/s; the caller's Python is as long as the kernel), e4m3 3870 -> 16.3 us, fp8
 // activations on e2m1 weights 4415 -> 14.8 us; 64 rows on the 256 x 256 tiles before: e2m1 42.4 -> 13.0 us, e4m3 77 ->
-// 37 us.  32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
+// 19.5 us.  32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
 // streams half the bytes: n = 1024, k = 14336, e4m3, 9 against 14 us).
 //
-// Two 4-bit operands run v_mfma_scale_f32_16x16x128_f8f6f4, one scale byte per lane: lane l holds the scale of row l % 16
-// and block of 32 k number l / 16; an e2m1 operand's four registers hold the lane's own block, e1m2, which the instruction
-// does not know, is widened to e4m3 in registers (exact), whose registers 0-3 hold k = 16 (l / 16) .. + 15 and 4-7 k = 64 +
-// 16 (l / 16) .. + 15.  Their products lie less than 2^8 apart, and the instruction drops none.
-// A pair with fp8 runs v_mfma_f32_16x16x32_bf16 on operands converted in registers (every fp8 and fp4 value is a
-// bfloat16 value, every product of two exact in fp32), one instruction per block of 32 k from zero, whose sums the vector
-// ALU scales and adds: the arithmetic of the kernel with one lane per output element.  The scaled instruction is not good
-// enough for them: it aligns the products of fp8 operands to the largest and drops what lies 2^13 below it.
+// v_mfma_scale_f32_16x16x128_f8f6f4 takes one scale byte per lane: lane l holds the scale of row l % 16 and block of 32 k
+// number l / 16; a 4-bit operand's four registers hold the lane's own block, an 8-bit operand's registers 0-3 hold k =
+// 16 (l / 16) .. + 15 and 4-7 k = 64 + 16 (l / 16) .. + 15; e1m2, which the instruction does not know, is widened to e4m3 in
+// registers (exact).  The products of two 4-bit operands lie less than 2^8 apart, and the instruction drops none; those
+// of fp8 operands it aligns to the largest and drops what lies 2^13 below it.  The tiles live with that, so fp8 at the
+// tiles' shapes may run it here too.
+// Elsewhere fp8 runs v_mfma_f32_16x16x32_bf16 on operands converted in registers (every fp8 and fp4 value is a bfloat16
+// value, every product of two exact in fp32), one instruction per block of 32 k from zero, whose sums the vector ALU
+// scales and adds: the arithmetic of the kernel with one lane per output element, which took these calls before.
 // Against 64 bits (2-norm, k = 8192, 16 rows, normally distributed e4m3): scaled instruction 1.3e-5, one lane per output
 // 2.2e-7, this 9.2e-8; e2m1 x e4m3 3.0e-7, 1.2e-7 and 6.8e-8.  That arithmetic is also what bounds these pairs from 16
 // rows on: per block of 32 k and 16 x 16 results a multiplication and an addition per sum beside the conversions (e4m3,
-// 16 rows: 16.3 us a call where the scaled instruction took 12.3; 64 rows 37 us and 19.5).
+// 16 rows: 16.3 us a call where the scaled instruction took 12.3).
 #include <type_traits>
 #include <utility>
 
@@ -44,8 +45,8 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 // operand formats: the instruction's codes, and e1m2
 enum { kE4M3 = 0, kE5M2 = 1, kE2M1 = 4, kE1M2 = 5 };
 constexpr bool fmt_is_8bit(int f) { return f == kE4M3 || f == kE5M2; }
-// the pairs whose products the scaled matrix instruction adds up without dropping any; those with fp8 go through bfloat16
-constexpr bool fmt_scaled(int fa, int fb) { return !fmt_is_8bit(fa) && !fmt_is_8bit(fb); }
+// the pairs whose products the scaled matrix instruction adds up without dropping any
+constexpr bool fmt_lossless(int fa, int fb) { return !fmt_is_8bit(fa) && !fmt_is_8bit(fb); }
 constexpr uint32_t kPastEnd = 0x7FFFFFF0u;  // an offset every buffer's range check rejects: the load moves no data
 
 // A batch is 128 bytes of a weight column: KB values of k.
@@ -172,7 +173,8 @@ struct MxdParams {
     uint32_t row_blocks, col_blocks;
 };
 
-template <int FA, int FB, int RT, int S>
+// kScaled: on the scaled matrix instruction; otherwise in bfloat16
+template <int FA, int FB, int RT, int S, bool kScaled>
 __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_decode_kernel(MxdParams q)
 {
     typedef MxdShape<FA, FB, RT, S> T;
@@ -276,19 +278,22 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
         asm volatile("" ::: "memory");
     };
 
-    // Two 4-bit operands.  e2m1: a lane's 16 bytes of a tile are the instruction's operand as they lie; e1m2, which the
-    // instruction does not know: the two times 8 bytes that widened to e4m3 are the lane's operand of 8 bits.
+    // The scaled instruction.  e2m1: a lane's 16 bytes of a tile are its operand as they lie; fp8: two times 16 bytes; e1m2,
+    // which the instruction does not know: the two times 8 bytes that widened to e4m3 are the lane's operand of 8 bits.
     auto step_scaled = [&](uint32_t b, uint32_t slot_off) __attribute__((always_inline)) {
         const uint32_t abase = ring_addr + slot_off, bbase = abase + T::a_bytes, sbase = bbase + T::b_bytes;
         const uint32_t slane = sbase + lc * (4u * T::sdw) + lq;
         struct Raw {
-            i32x4 v;           // e2m1
+            i32x4 v, w;        // e2m1 (v), fp8
             i32x2_t h0, h1;    // e1m2
         };
         auto read = [&](auto fmt, auto line, auto row_bytes, auto tt, uint32_t base) __attribute__((always_inline)) {
             constexpr uint32_t bytes = decltype(row_bytes)::value, off = decltype(line)::value * 16u * bytes, tl = decltype(tt)::value;
             Raw r;
-            if constexpr (decltype(fmt)::value == kE2M1) {
+            if constexpr (fmt_is_8bit(decltype(fmt)::value)) {
+                r.v = lds_b128<off>(base + at(bytes, 8u * tl + lq));
+                r.w = lds_b128<off>(base + at(bytes, 8u * tl + 4u + lq));
+            } else if constexpr (decltype(fmt)::value == kE2M1) {
                 r.v = lds_b128<off>(base + at(bytes, 4u * tl + lq));
             } else {
                 r.h0 = lds_b64<off>(base + at(bytes, 4u * tl + (lq >> 1)) + 8u * (lq & 1u));
@@ -297,14 +302,18 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
             return r;
         };
         auto landed = [](auto fmt, Raw& r, uint32_t& scale) __attribute__((always_inline)) {  // usable from here on
-            if constexpr (decltype(fmt)::value == kE2M1) {
+            if constexpr (fmt_is_8bit(decltype(fmt)::value)) {
+                asm volatile("" : "+v"(r.v), "+v"(r.w), "+v"(scale));
+            } else if constexpr (decltype(fmt)::value == kE2M1) {
                 asm volatile("" : "+v"(r.v), "+v"(scale));
             } else {
                 asm volatile("" : "+v"(r.h0), "+v"(r.h1), "+v"(scale));
             }
         };
         auto operand = [](auto fmt, const Raw& r) __attribute__((always_inline)) {
-            if constexpr (decltype(fmt)::value == kE2M1) {
+            if constexpr (fmt_is_8bit(decltype(fmt)::value)) {
+                return v8i{r.v[0], r.v[1], r.v[2], r.v[3], r.w[0], r.w[1], r.w[2], r.w[3]};
+            } else if constexpr (decltype(fmt)::value == kE2M1) {
                 return __builtin_shufflevector(r.v, r.v, 0, 1, 2, 3, -1, -1, -1, -1);
             } else {
                 const i32x2_t a = widen_e1m2(static_cast<uint32_t>(r.h0[0])), b = widen_e1m2(static_cast<uint32_t>(r.h0[1]));
@@ -358,7 +367,7 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
         });
     };
 
-    // A pair with fp8: lane l holds k = 32 blk + 8 (l / 16) .. + 7 of row l % 16 for each of a tile's four blocks blk, and
+    // In bfloat16: lane l holds k = 32 blk + 8 (l / 16) .. + 7 of row l % 16 for each of a tile's four blocks blk, and
     // the scale bytes of its four rows of the result (rows 4 (l / 16) .. + 3) and of its column.
     typedef typename std::conditional<fmt_is_8bit(FA), i32x2_t, uint32_t>::type RawA;
     typedef typename std::conditional<fmt_is_8bit(FB), i32x2_t, uint32_t>::type RawB;
@@ -476,7 +485,7 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
             return;  // uniform
         }
         wait_batch();
-        if constexpr (fmt_scaled(FA, FB)) {
+        if constexpr (kScaled) {
             step_scaled(b, slot_off);
         } else {
             step_exact(b, slot_off);
@@ -518,7 +527,7 @@ __global__ __launch_bounds__((MxdShape<FA, FB, RT, S>::waves * 64)) void mx_deco
     }
 }
 
-template <int FA, int FB, int RT, int S>
+template <int FA, int FB, int RT, int S, bool kScaled>
 void mxd_launch(MxdParams q, hipStream_t st)
 {
     typedef MxdShape<FA, FB, RT, S> T;
@@ -526,25 +535,25 @@ void mxd_launch(MxdParams q, hipStream_t st)
     q.col_blocks = (q.p.n + S * 16u - 1u) / (S * 16u);
     const uint32_t per = (q.tiles_k + T::waves - 1u) / T::waves;
     q.tpw = (per + T::tiles - 1u) / T::tiles * T::tiles;
-    mx_decode_kernel<FA, FB, RT, S><<<(q.row_blocks * q.col_blocks + 7u) / 8u * 8u, T::waves * 64u, 0, st>>>(q);
+    mx_decode_kernel<FA, FB, RT, S, kScaled><<<(q.row_blocks * q.col_blocks + 7u) / 8u * 8u, T::waves * 64u, 0, st>>>(q);
 }
 
 template <int FA, int FB>
-void mxd_pick(const MxdParams& q, hipStream_t st)
+void mxd_pick(const MxdParams& q, bool tile_shape, hipStream_t st)
 {
+    constexpr bool kLossless = fmt_lossless(FA, FB);
+    constexpr int kMost = fmt_is_8bit(FA) && !fmt_is_8bit(FB) ? 2 : 4;  // (twice the bytes per row of a: 64 rows do not fit the ring)
     const uint32_t m = q.p.m;
     const bool few_columns = (q.p.n + 31u) / 32u < device_compute_units() / 2u;
-    if (m <= 16u) {
-        few_columns ? mxd_launch<FA, FB, 1, 1>(q, st) : mxd_launch<FA, FB, 1, 2>(q, st);
-        return;
+    if (!kLossless && tile_shape) {
+        mxd_launch<FA, FB, kMost, 2, true>(q, st);
+    } else if (m <= 16u) {
+        few_columns ? mxd_launch<FA, FB, 1, 1, kLossless>(q, st) : mxd_launch<FA, FB, 1, 2, kLossless>(q, st);
+    } else if (m <= 32u || kMost == 2) {
+        mxd_launch<FA, FB, 2, 2, kLossless>(q, st);
+    } else {
+        mxd_launch<FA, FB, kMost, 2, kLossless>(q, st);
     }
-    if constexpr (!(fmt_is_8bit(FA) && !fmt_is_8bit(FB))) {  // (twice the bytes per row of a: 64 rows do not fit the ring)
-        if (m > 32u) {
-            mxd_launch<FA, FB, 4, 2>(q, st);
-            return;
-        }
-    }
-    mxd_launch<FA, FB, 2, 2>(q, st);
 }
 
 inline int code_of(int f)
@@ -566,7 +575,7 @@ bool mx_decode_supported(const MxParams& p)
            static_cast<uint64_t>((p.m + 15u) / 16u) * ((p.n + 15u) / 16u) < (1ull << 31);
 }
 
-int launch_mx_decode(const MxParams& p, hipStream_t st)
+int launch_mx_decode(const MxParams& p, bool tile_shape, hipStream_t st)
 {
     MxdParams q{};
     q.p = p;
@@ -577,7 +586,7 @@ int launch_mx_decode(const MxParams& p, hipStream_t st)
     q.tiles_k = (p.k + 127u) / 128u;
 #define ASCQ_MXD(A, B)                     \
     if (fa == (A) && fb == (B)) {          \
-        mxd_pick<(A), (B)>(q, st);         \
+        mxd_pick<(A), (B)>(q, tile_shape, st); \
     }
     ASCQ_MXD(kE4M3, kE4M3)
     ASCQ_MXD(kE4M3, kE5M2)

@@ -642,9 +642,10 @@ int ascq_matmul_w8a16_workspace_size(const ascq_w8a16_desc* desc, size_t* bytes)
  * query asked for is left alone) and gives the same bits from call to call; it wants rows of a and b that are whole numbers
  * of 16-byte pieces, 16-byte aligned a and b, scale_k % 4 == 0 and 4-byte aligned scales.  Anything else takes a kernel
  * with one lane per output element.
- * Accuracy: exact products and fp32 sums, about 1e-7 from 64 bits (2-norm), except on the tiles with an fp8 operand: there
- * the scaled matrix instruction aligns the products of 64 k to the largest and drops what lies 2^13 below it, which
- * leaves up to 1.3e-5 (2-norm) and single results off by up to 2.3e-4 of their terms' magnitudes.
+ * Accuracy: exact products and fp32 sums, about 1e-7 from 64 bits (2-norm), but for an fp8 operand in a call that the tiles
+ * could take (64 rows and columns and more, the conditions above): there the scaled matrix instruction aligns the
+ * products of an instruction to the largest and drops what lies 2^13 below it, which leaves up to 1.3e-5 (2-norm) and
+ * single results off by up to 2.3e-4 of their terms' magnitudes.
  * ref: include/basic_api/kernel_operator_mm_intf.h:321-340 (MmadMx), examples/01_simd_cpp_api/03_basic_api/
  *      03_matrix_compute/mmad_mx/README.md:5,131-152 and scripts/gen_data.py:52-140 (layouts, golden),
  *      examples/01_simd_cpp_api/05_best_practices/01_matrix_compute/matmul_mxfp4_basic_api_high_performance/
