@@ -57,7 +57,7 @@ void run_dma(int form, const GemmParams& p, const DmaLaunch& l, int b_layout, hi
     if (form == k32Ragged) {
         run_dma_ragged(p, l, b_layout, st);
     } else if (form == k16) {
-        run_dma<k16>(p, l, b_layout, st);
+        run_dma_long(p, l, b_layout, st);
     } else {
         run_dma<k32>(p, l, b_layout, st);
     }

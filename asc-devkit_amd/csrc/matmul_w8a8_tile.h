@@ -1018,7 +1018,9 @@ void run_dma(const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t 
 
 }  // namespace
 
-// matmul_w8a8_ragged.hip (a translation unit of its own: the kernels take minutes to compile)
+// matmul_w8a8_ragged.hip (k32Ragged) and matmul_w8a8_long.hip (k16): translation units of their own, the kernels take
+// minutes to compile
 void run_dma_ragged(const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t st);
+void run_dma_long(const GemmParams& p, const DmaLaunch& l, int b_layout, hipStream_t st);
 
 }  // namespace ascq
