@@ -858,7 +858,7 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
     p.ktiles = d->k / kTileK;
     // the group-sum form needs whole tiles inside one quantisation group; other group sizes keep the per-weight form
     const bool sum_form = d->mode == ASCQ_W4A16_GROUP_SUM && p.gs_shift >= 2u;
-    if (!sum_form && d->m > kMaxPassRows) {
+    if (!sum_form && d->m > kMaxPassRows && d->k <= kWqMaxK) {
         WqParams w{};
         w.x = static_cast<const uint16_t*>(x);
         w.w = static_cast<const uint8_t*>(w_packed);

@@ -536,7 +536,7 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
 // Weights given as [k, n] and many rows: transposed once into the caller's workspace (k * n bytes), then the tile GEMM.
 bool w8a16_kn_gemm_supported(uint32_t m, uint32_t k, const void* x, const void* w)
 {
-    return m > 96u && k % kGK == 0 && aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0;
+    return m > 96u && k % kGK == 0 && k <= kWqMaxK && aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0;
 }
 
 int launch_w8a16_kn_via_transpose(const void* x, const void* w, const void* scale, const void* offset, void* y,
@@ -616,7 +616,7 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
     per = per > kMaxGroups ? kMaxGroups : per;
     p.groups = per;
     const uint32_t grid = (n_groups + per - 1u) / per;
-    if (m > kDecodeRows && k % kGK == 0) {
+    if (m > kDecodeRows && k % kGK == 0 && k <= kWqMaxK) {
         // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 or 256 rows
         WqParams q{};
         q.x = static_cast<const uint16_t*>(x);

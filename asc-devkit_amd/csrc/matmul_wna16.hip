@@ -31,6 +31,7 @@
 
 #include "ascq_common.h"
 #include "ascq_device.h"
+#include "matmul_wq_gemm.h"
 
 namespace ascq {
 namespace {
@@ -1015,7 +1016,7 @@ bool pack_first(const ascq_w4a16_desc* d)
 {
     const uint32_t g32 = d->group_size / 32u;
     size_t bytes = 0;
-    return d->m > 96u && d->k % 128u == 0 && d->n % 8u == 0 && d->group_size % 32u == 0 && (g32 & (g32 - 1u)) == 0 &&
+    return d->m > 96u && d->k <= kWqMaxK && d->k % 128u == 0 && d->n % 8u == 0 && d->group_size % 32u == 0 && (g32 & (g32 - 1u)) == 0 &&
            ascq_pack_weight_w4_size(d->k, d->n, &bytes) == ASCQ_OK && bytes < (1ull << 31) &&
            static_cast<uint64_t>(d->k / d->group_size) * d->n * 2u < (1ull << 31);
 }

@@ -1080,6 +1080,24 @@ def test_w8a16_trans_b(m, k, n, mode):
                                                       None if per_tensor else sc)).view(np.uint8))
 
 
+def test_w8a16_rows_beyond_thirty_two_bit_offsets():
+    """256 rows of x of 16.25 MiB each: the last rows of a tile lie more than 4 GiB behind its first, where a lane's 32-bit
+    offset would wrap round to another row.  x is zero but for a few halves, so every result is an exact integer."""
+    m, n, k = 256, 16, (1 << 23) + (1 << 17)
+    announce("w8a16 long rows", m, n, k)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(1)
+    x = torch.zeros((m, k), dtype=torch.float16, device=DEV)
+    w = torch.randint(-8, 9, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    want = torch.zeros((m, n), dtype=torch.float32, device=DEV)
+    for row, col in ((0, 0), (3, 64), (128, 5), (251, 70), (252, 3), (254, k - 1), (255, 0), (255, 9)):
+        x[row, col] = row % 7 + 1
+        want[row] += (row % 7 + 1) * w[:, col].float()
+    y = torch.full((m, n), -1.0, dtype=torch.float32, device=DEV)
+    ops.matmul_w8a16(y, x, w, None, 1.0, trans_b=True)
+    assert torch.equal(y, want)
+
+
 @pytest.mark.parametrize("m,k,n", [(33, 128, 7), (128, 256, 248), (129, 384, 264), (257, 640, 521), (300, 128, 1034)])
 @pytest.mark.parametrize("mode", ["vector+offset", "vector", "scalar+offset"])
 @pytest.mark.parametrize("out_f32", [False, True])
