@@ -22,7 +22,7 @@ struct WqParams {
     WqMasks mk;
 };
 
-// A lane addresses its row of a tile's 256 by 32 bits: longer rows stay with the passes over the weights.
+// A lane addresses its row of a tile's 128 or 256 by 32 bits: longer rows stay with the passes over the weights.
 constexpr uint32_t kWqMaxK = 1u << 23;
 int launch_wq_gemm(const WqParams& p, bool int4, bool has_offset, hipStream_t st);
 

@@ -1081,16 +1081,16 @@ def test_w8a16_trans_b(m, k, n, mode):
 
 
 def test_w8a16_rows_beyond_thirty_two_bit_offsets():
-    """256 rows of x of 16.25 MiB each: the last rows of a tile lie more than 4 GiB behind its first, where a lane's 32-bit
-    offset would wrap round to another row.  x is zero but for a few halves, so every result is an exact integer."""
-    m, n, k = 256, 16, (1 << 23) + (1 << 17)
+    """128 rows of x of 32.5 MiB each: the last rows of a tile of 128 lie more than 4 GiB behind its first, where a lane's
+    32-bit offset would wrap round to another row.  x is zero but for a few halves, so every result is an exact integer."""
+    m, n, k = 128, 16, (1 << 24) + (1 << 18)
     announce("w8a16 long rows", m, n, k)
     g = torch.Generator(device=DEV)
     g.manual_seed(1)
     x = torch.zeros((m, k), dtype=torch.float16, device=DEV)
     w = torch.randint(-8, 9, (n, k), dtype=torch.int8, device=DEV, generator=g)
     want = torch.zeros((m, n), dtype=torch.float32, device=DEV)
-    for row, col in ((0, 0), (3, 64), (128, 5), (251, 70), (252, 3), (254, k - 1), (255, 0), (255, 9)):
+    for row, col in ((0, 0), (3, 64), (64, 5), (124, 70), (125, 3), (126, k - 1), (127, 0), (127, 9)):
         x[row, col] = row % 7 + 1
         want[row] += (row % 7 + 1) * w[:, col].float()
     y = torch.full((m, n), -1.0, dtype=torch.float32, device=DEV)

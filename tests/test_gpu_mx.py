@@ -74,9 +74,8 @@ def test_mx_reference_example_shape(fa, fb, bias):
 @pytest.mark.parametrize("m,n,k", [(256, 256, 256), (64, 64, 1024), (300, 520, 512), (513, 272, 768), (1024, 256, 2048)])
 @pytest.mark.parametrize("fa,fb", [(E4, E4), (E4, E5), (E5, E4), (E5, E5), (F2, F2), (F1, F1), (F2, F1), (E4, F2), (F1, E5)])
 def test_mx_tile_kernel(m, n, k, fa, fb):
-    """The tile kernel on the scaled matrix instruction: the four 8-bit pairs and e2m1 x e2m1 straight from the given
-    buffers, the other pairs with their 4-bit operands widened to e4m3 first; row and column tails, odd and even
-    numbers of K steps."""
+    """Shapes that the tile kernel could take and the few-row kernel runs, on the scaled matrix instruction: every pair, row
+    and column tails, odd and even numbers of K steps."""
     announce("mx tiles", m, n, k, fa, fb)
     rng = np.random.default_rng(m + n + k + fa * 16 + fb)
     a, b, sa, sb, _ = mx_case(rng, m, n, k, fa, fb)
@@ -90,9 +89,8 @@ def test_mx_tile_kernel(m, n, k, fa, fb):
                                       (256, 256, 1024, 40), (320, 256, 2304, 72), (256, 256, 256, 8)])
 @pytest.mark.parametrize("fa,fb", [(E4, E5), (F2, F2), (F1, E4)])
 def test_mx_tile_kernel_scale_rows(m, n, k, sk, fa, fb):
-    """The tile kernel fetches 16 scale bytes per row for every two K steps and moves the last fetch back to stay inside
-    the row: rows of scale bytes that end in half a fetch, rows longer than k / 32, a single K step, odd numbers of
-    steps; rows shorter than one fetch (the last case) go through the element-wise kernel."""
+    """The same with rows of scale bytes that end in half a fetch of the tile kernel, rows longer than k / 32, a single K
+    step, odd numbers of steps, rows shorter than one fetch (the last case)."""
     announce("mx scale rows", m, n, k, sk, fa, fb)
     rng = np.random.default_rng(m + 3 * n + 5 * k + 7 * sk + fa * 16 + fb)
     a, b, sa, sb, _ = mx_case(rng, m, n, k, fa, fb, sk=sk)
@@ -100,6 +98,27 @@ def test_mx_tile_kernel_scale_rows(m, n, k, sk, fa, fb):
     orc.set_threads(16)
     want = orc.matmul_mx(d, a, b, sa, sb)
     mx_check(run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, fa, fb), is8(fa, fb))
+
+
+@pytest.mark.parametrize("fa,fb", [(E4, E4), (E4, E5), (E5, E4), (E5, E5), (F2, F2), (F2, F1), (E4, F2), (F1, E5)])
+@pytest.mark.parametrize("steps,more", [(1, 0), (3, 8), (5, 0), (8, 8)])
+def test_mx_enough_rows_for_the_tile_kernel(fa, fb, steps, more):
+    """170 tiles, where the few-row kernel would take two or more times as long: the 8-bit pairs and e2m1 x e2m1 straight
+    from the given buffers, the other pairs with their 4-bit operands widened to e4m3 first.  The tile kernel fetches 16
+    scale bytes per row for every two K steps and moves the last fetch back to stay inside the row: one K step, odd and
+    even numbers of them, rows of scale bytes that end in half a fetch, rows longer than k / 32; a last tile of 4 rows and
+    of 40 columns.  The first and last rows and those on either side of a tile's end are compared."""
+    m, n, k = 4100, 2344, steps * (256 if fa == fb == F2 else 128)
+    sk = max(16, (k // 32 + 7) // 8 * 8) + more
+    announce("mx tiles, many rows", fa, fb, k, sk)
+    rng = np.random.default_rng(steps + fa * 16 + fb)
+    a, b, sa, sb, _ = mx_case(rng, m, n, k, fa, fb, sk=sk)
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sk, a_format=fa, b_format=fb, out_dtype=abi.F32, has_bias=0)
+    got = run_mx(m, n, k, a, b, sa, sb, fa, fb).cpu().numpy()
+    orc.set_threads(16)
+    for r0, r1 in ((0, 6), (252, 260), (2040, 2052), (4090, 4100)):
+        want = orc.matmul_mx(d, a, b, sa, sb, rows=(r0, r1))[r0:r1]
+        mx_check(got[r0:r1], want, mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, fa, fb), is8(fa, fb))
 
 
 @pytest.mark.parametrize("m,n,k", [(8200, 1100, 128), (4100, 1128, 384), (4129, 1033, 640), (4096, 1056, 1024)])
