@@ -32,8 +32,8 @@ __device__ __forceinline__ void group_row_tiles(uint32_t rows, uint32_t& big, ui
 // One phase of the grouped kernel's plan (see gemm_dma_group_kernel): the workgroup's ids that fall into it.
 // (tiles of at most 128 rows never run the 16 x 16 x 64 instruction)
 template <uint32_t phase, int kForm>
-__device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const uint32_t* PLAN, char* A0, char* B0,
-                                                     char* A1, char* B1, float* TS)
+__device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const uint32_t* PLAN, const Stage& S0, const Stage& S1,
+                                                     float* TS)
 {
     constexpr int kSmall = kForm == k16 ? k32 : kForm;
     for (uint32_t id = blockIdx.x;; id += gridDim.x) {
@@ -87,13 +87,13 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
             continue;
         }
         if constexpr (phase == 0) {
-            gemm_dma_tile_at<256, 256, false, true, 0, kForm>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<256, 256, false, true, 0, kForm>(p, at, 0u, S0, S1, TS);
         } else if constexpr (phase == 1) {
-            gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, S0, S1, TS);
         } else if (at.row_end - at.row0 <= 64u) {  // uniform: a remainder of at most 64 rows
-            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, S0, S1, TS);
         } else {
-            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, A0, B0, A1, B1, TS);
+            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, S0, S1, TS);
         }
         __syncthreads();  // the next tile's loads and token scales overwrite what slower wavefronts may still read
     }
@@ -114,10 +114,7 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
 template <int kForm>
 __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams p)
 {
-    __shared__ __attribute__((aligned(1024))) char A0[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B0[BK * 256];
-    __shared__ __attribute__((aligned(1024))) char A1[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B1[BK * 256];
+    ASCQ_DMA_STAGES(kForm, 256, 256);
     __shared__ __attribute__((aligned(16))) float TS[256];
     uint32_t n_big = 0, n_small = 0;
     {
@@ -149,9 +146,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams 
     }
     // One loop per phase (a workgroup's ids ascend, so it passes through the phases in order anyway): each loop holds
     // one tile shape's code and registers.
-    gemm_dma_group_phase<0, kForm>(p, PLAN, A0, B0, A1, B1, TS);
-    gemm_dma_group_phase<1, kForm>(p, PLAN, A0, B0, A1, B1, TS);
-    gemm_dma_group_phase<2, kForm>(p, PLAN, A0, B0, A1, B1, TS);
+    gemm_dma_group_phase<0, kForm>(p, PLAN, S0, S1, TS);
+    gemm_dma_group_phase<1, kForm>(p, PLAN, S0, S1, TS);
+    gemm_dma_group_phase<2, kForm>(p, PLAN, S0, S1, TS);
 }
 
 }  // namespace

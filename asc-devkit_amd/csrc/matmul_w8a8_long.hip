@@ -1,4 +1,4 @@
-// The plain int8 matmul on the direct-to-LDS tiles of matmul_w8a8_tile.h, long sums on v_mfma_i32_16x16x64_i8.
+// The plain int8 matmul on the direct-to-LDS tiles of matmul_w8a8_tile.h, half and bfloat16 outputs on v_mfma_i32_16x16x64_i8.
 #include "matmul_w8a8_tile.h"
 
 namespace ascq {

@@ -97,6 +97,13 @@ struct TilePlace {
     size_t chan_off;
 };
 
+// One of the two LDS stages of a tile.  a[0] holds all rows of A, or in the 16x16x64 form those of every wavefront's first
+// half (a[1]: its second half): distinct arrays, like the stages themselves.
+struct Stage {
+    char* a[2];
+    char* b;
+};
+
 constexpr uint32_t kPastEnd = 0x7FFFFFF0u;  // an offset the buffer range check rejects: zeros arrive, nothing is fetched
 
 // The main loop of a tile.  first(A, B): the first operands of a step into registers; head(A, B): everything of a step
@@ -107,8 +114,7 @@ constexpr uint32_t kPastEnd = 0x7FFFFFF0u;  // an offset the buffer range check 
 // burst of LDS reads that follows every barrier.  The loop body never branches between two ways of updating the
 // accumulators (that would make the compiler shuffle all of them): the steady state always has a next step, the last one
 // or two steps are peeled.
-// active: a wavefront whose rows all lie past the end of the tile's group (ragged grouped tiles) skips the matrix work and
-// only keeps the loads and barriers going: its SIMD then runs one wavefront's MFMAs per K step instead of two.
+// active: not a wavefront whose rows all lie past the end of the tile's group.
 template <class Issue, class First, class Head, class Tail, class Last>
 __device__ __forceinline__ void gemm_dma_loop(uint32_t steps, bool active, char* A0, char* B0, char* A1, char* B1, Issue&& issue,
                                               First&& first, Head&& head, Tail&& tail, Last&& last)
@@ -154,11 +160,12 @@ __device__ __forceinline__ void gemm_dma_loop(uint32_t steps, bool active, char*
     }
 }
 
-// The body of a tile on v_mfma_i32_16x16x64_i8, 16-bit outputs only: where the power limit sets the clock.
-// wave, lane: of the workgroup; n0: first column; issue(step, A, B): the loads of a K step into a stage.
-template <int BM, int BN, bool kGrouped, int kB, class Issue>
+// The body of a tile on v_mfma_i32_16x16x64_i8, 16-bit outputs only.
+// wave, lane: of the workgroup; n0: first column; bases(step): where a K step's loads start; load(bases, u, stage): load u
+// of the wavefront's kBLoads + kALoads of a step (B, first half of A's rows, second half).
+template <int BM, int BN, bool kGrouped, int kB, int kALoads, int kBLoads, class Bases, class Load>
 __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TilePlace& at, uint32_t n0, uint32_t steps, uint32_t wave,
-                                                uint32_t lane, Issue&& issue, char* A0, char* B0, char* A1, char* B1, float* TS)
+                                                uint32_t lane, Bases&& bases, Load&& load, const Stage& S0, const Stage& S1, float* TS)
 {
     constexpr bool kBT = kB == 1, kBP = kB == 2;
     constexpr int kWN = BN / 64;            // wavefronts along N
@@ -182,10 +189,10 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     }
 
     // ---- operands of v_mfma_i32_16x16x64_i8: lane l holds row (column) l % 16 of a block of 16 and 16 consecutive k,
-    // 64 ks + 16 (l / 16) .. + 15.  A step is four quarters: quarter q multiplies half q % 2 of the wavefront's rows
-    // with the 64 k of sub-step ks = q / 2.  (This form moves half the sums per product that the 32 x 32 x 32 one
+    // 64 ks + 16 (l / 16) .. + 15.  A step is four quarters: quarter q multiplies half q / 2 of the wavefront's rows
+    // with the 64 k of sub-step ks = q % 2.  (This form moves half the sums per product that the 32 x 32 x 32 one
     // moves: on random operands, where the power limit sets the clock, a loop of nothing but matrix instructions reaches
-    // 4.0 instead of 3.4 POP/s.)
+    // 4.0 instead of 3.3 POP/s.)
     const uint32_t lc = lane & 15u, lq = lane >> 4;
     uint32_t foff[2], b_base[TJ];
 #pragma unroll
@@ -204,16 +211,16 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     i32x4 af[2][NH], bf[2][TJ];
     i32x2_t blo;
     constexpr int kBReads = (kBT || kBP) ? TJ : 2 * TJ;  // LDS reads of a sub-step's columns
-    auto load_a = [&](const char* As, int q, int i) __attribute__((always_inline)) {
-        af[q & 1][i] = *reinterpret_cast<const i32x4*>(As + wm * (NA * 2048u) + ((q & 1) * NH + i) * 2048u + foff[q >> 1]);
+    auto load_a = [&](const Stage& S, int q, int i) __attribute__((always_inline)) {
+        af[q & 1][i] = *reinterpret_cast<const i32x4*>(S.a[q >> 1] + (wm * NH + i) * 2048u + foff[q & 1]);
     };
-    auto load_b = [&](const char* Bs, int ks, int r) __attribute__((always_inline)) {
+    auto load_b = [&](const Stage& S, int ks, int r) __attribute__((always_inline)) {
         if constexpr (kBT) {
-            bf[ks][r] = *reinterpret_cast<const i32x4*>(Bs + wn * 8192u + r * 2048u + foff[ks]);
+            bf[ks][r] = *reinterpret_cast<const i32x4*>(S.b + wn * 8192u + r * 2048u + foff[ks]);
         } else if constexpr (kBP) {
-            bf[ks][r] = *reinterpret_cast<const i32x4*>(Bs + b_base[0] + r * 2048u + ks * 1024u);
+            bf[ks][r] = *reinterpret_cast<const i32x4*>(S.b + b_base[0] + r * 2048u + ks * 1024u);
         } else {
-            const i32x2_t v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2_t)(Bs + b_base[r >> 1] + ks * (64 * BN) + (r & 1) * (8 * BN)));
+            const i32x2_t v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2_t)(S.b + b_base[r >> 1] + ks * (64 * BN) + (r & 1) * (8 * BN)));
             if (r & 1) {
                 bf[ks][r >> 1] = i32x4{blo[0], blo[1], v[0], v[1]};
             } else {
@@ -225,15 +232,18 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     // choice of another destination moves accumulators about).  Its operands come from LDS reads, which the compiler
     // waits for; no vector instruction touches them or the sums inside the loop.
     auto mfma = [&](int q, int n) __attribute__((always_inline)) {
-        i32x4& c = acc[(q & 1) * NH + n / TJ][n % TJ];
-        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(c) : "v"(af[q & 1][n / TJ]), "v"(bf[q >> 1][n % TJ]));
+        i32x4& c = acc[(q >> 1) * NH + n / TJ][n % TJ];
+        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(c) : "v"(af[q & 1][n / TJ]), "v"(bf[q & 1][n % TJ]));
     };
-    // One quarter: its NH * TJ matrix instructions with the LDS reads `read(r)`, r < kReads, spread behind the first ones,
-    // so that the others run while the last reads are on their way.  The order is the one written.
+    // One quarter: its NH * TJ matrix instructions.  The LDS reads `read(r)`, r < kReads, are spread behind the first ones,
+    // so that the others run while the last reads are on their way; the loads `fetch(u)`, u in [kFrom, kTo), behind all.
+    // The order is the one written.
     constexpr int kM = NH * TJ;
-    auto quarter = [&](auto qq, auto reads, auto&& read) __attribute__((always_inline)) {
-        constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value;
+    auto quarter = [&](auto qq, auto reads, auto&& read, auto from, auto to, auto&& fetch) __attribute__((always_inline)) {
+        constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value, kFrom = decltype(from)::value, kCount = decltype(to)::value - kFrom;
         constexpr int kFront = kM >= 8 ? kM / 2 : kM, kPer = (kReads + kFront - 1) / kFront;
+        constexpr int kEvery = kM / (kCount > 0 ? kCount : 1);
+        static_assert(kCount <= kM, "at most one load behind a matrix instruction");
         static_for<kM>([&](auto nn) {
             constexpr int n = decltype(nn)::value;
             mfma(q, n);
@@ -241,12 +251,56 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
                 constexpr int i = n * kPer + decltype(r)::value;
                 if constexpr (i < kReads) read(i);
             });
+            if constexpr (n % kEvery == kEvery - 1 && n / kEvery < kCount) fetch(kFrom + n / kEvery);
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    // Quarters 0-2 of a K step whose first operands are in registers; on return the operands of quarter 3 are on their
-    // way and nothing else of the stage will be read.
-    auto head = [&](const char* As, const char* Bs) __attribute__((always_inline)) {
+    // Behind it all but the newest kLeft loads of every wavefront have landed, and every wavefront has the operands it asked
+    // for in registers.  (Not __syncthreads(): its fence waits for every load.)
+    auto arrive = [&](auto left) __attribute__((always_inline)) {
+        constexpr int kLeft = decltype(left)::value;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kLeft & 15) | ((kLeft >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // the operands that quarter 0 of a K step and quarter 1 read first
+    auto first_operands = [&](const Stage& S, int i) __attribute__((always_inline)) {
+        constexpr int kFirst = kBReads / TJ;  // reads of the first block of columns
+        if (i < kFirst || i >= kFirst + NH) {
+            load_b(S, 0, i < kFirst ? i : i - NH);
+        } else {
+            load_a(S, 0, i - kFirst);
+        }
+    };
+    auto second_operands = [&](const Stage& S, int i) __attribute__((always_inline)) {
+        if (i < kBReads) {
+            load_b(S, 1, i);
+        } else {
+            load_a(S, 1, i - kBReads);
+        }
+    };
+    // A K step in stage X, the next one in Y, the one after it on its way into X where `fetches`.  B and the first half of
+    // A's rows have been read when quarter 1 begins, the second half when quarter 3 begins: a barrier there, and the loads
+    // of the step after next go out behind it.  So a load has one and a half K steps to arrive, and is issued behind a
+    // matrix instruction of its own (all of a step's loads behind one barrier per step: 2048 x 4096 x 11008 with the quantiser 94.7 us, 88.2
+    // like this; 2048 x 8192 x 28672 378 and 361; 256 x 256 tiles on operands of zeros, where the power limit is not met,
+    // 8192 x 4096 x 11008 256 and 238).  The counts are the loads issued behind the one that is waited for.
+    constexpr int kLoads = kBLoads + kALoads, kMid = kBLoads + kALoads / 2;
+    static_assert(kALoads % 2 == 0, "the halves of A's rows are whole loads");
+    auto step = [&](const Stage& X, const Stage& Y, uint32_t fetched, auto fetches, auto more, auto works) __attribute__((always_inline)) {
+        constexpr bool kFetch = decltype(fetches)::value, kMore = decltype(more)::value, kWorks = decltype(works)::value;
+        constexpr std::integral_constant<int, 0> zero{};
+        constexpr std::integral_constant<int, kFetch ? kMid : 0> mid{};
+        constexpr std::integral_constant<int, kFetch ? kLoads : 0> end{};
+        auto work = [&](auto q, auto reads, auto&& read, auto from, auto to, auto&& fetch) __attribute__((always_inline)) {
+            if constexpr (kWorks) {
+                quarter(q, reads, read, from, to, fetch);
+            } else {
+                static_for<decltype(to)::value - decltype(from)::value>([&](auto u) { fetch(decltype(from)::value + decltype(u)::value); });
+            }
+        };
         // Re-materialise the bases inside the loop body: the constant parts of every address then fold into the
         // 16-bit offset field of the DS instructions instead of being hoisted into dozens of registers.
 #pragma unroll
@@ -255,51 +309,65 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
 #pragma unroll
             for (int j = 0; j < (kBP ? 1 : TJ); ++j) asm volatile("" : "+v"(b_base[j]));
         }
-        static_for<3>([&](auto qq) {
-            constexpr int q = decltype(qq)::value;
-            quarter(qq, std::integral_constant<int, NH + (q < 2 ? kBReads / 2 : 0)>{}, [&](int i) __attribute__((always_inline)) {
-                if (i < NH) {
-                    load_a(As, q + 1, i);
-                } else {
-                    load_b(Bs, 1, q * (kBReads / 2) + i - NH);
-                }
-            });
-        });
-    };
-    auto first_operands = [&](const char* As, const char* Bs, int i) __attribute__((always_inline)) {
-        constexpr int kFirst = kBReads / TJ;  // reads of the first block of columns
-        if (i < kFirst || i >= kFirst + NH) {
-            load_b(Bs, 0, i < kFirst ? i : i - NH);
-        } else {
-            load_a(As, 0, i - kFirst);
+        constexpr std::integral_constant<int, NH> half{};
+        constexpr std::integral_constant<int, NH + kBReads> whole{};
+        work(zero, whole, [&](int i) __attribute__((always_inline)) { second_operands(X, i); }, zero, zero, [](int) {});
+        arrive(std::integral_constant<int, kMore ? kLoads : 0>{});
+        const auto from = bases(fetched);
+        auto fetch = [&](int u) __attribute__((always_inline)) { load(from, u, X); };
+        work(std::integral_constant<int, 1>{}, half, [&](int i) __attribute__((always_inline)) { load_a(X, 2, i); }, zero, mid, fetch);
+        work(std::integral_constant<int, 2>{}, half, [&](int i) __attribute__((always_inline)) { load_a(X, 3, i); }, zero, zero, [](int) {});
+        if constexpr (kMore) {
+            arrive(std::integral_constant<int, kFetch ? kLoads : kLoads - kMid>{});
+            work(std::integral_constant<int, 3>{}, whole, [&](int i) __attribute__((always_inline)) { first_operands(Y, i); }, mid, end, fetch);
         }
     };
-    // quarter 3, and the first operands of the next K step (stage An, Bn)
-    auto tail = [&](const char* An, const char* Bn) __attribute__((always_inline)) {
-        quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + kBReads>{},
-                [&](int i) __attribute__((always_inline)) { first_operands(An, Bn, i); });
+    // The loop body never branches between two ways of updating the accumulators (that would make the compiler shuffle all
+    // of them): the steady state always has a next step, the last one or two steps are peeled.  A fetch past the end repeats
+    // the last step into a stage that nobody reads again.
+    const uint32_t last = steps - 1u;
+    auto run_steps = [&](auto works) __attribute__((always_inline)) {
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        uint32_t s = 0;
+        for (; s + 2 < steps; s += 2) {
+            step(S0, S1, s + 2, yes, yes, works);
+            step(S1, S0, s + 3 < last ? s + 3 : last, yes, yes, works);
+        }
+        if (s + 1 < steps) {  // two steps left: this one in stage 0, the last one on its way into stage 1
+            step(S0, S1, last, no, yes, works);
+        }
+        const bool odd = (steps & 1u) != 0;
+        const Stage X{{odd ? S0.a[0] : S1.a[0], odd ? S0.a[1] : S1.a[1]}, odd ? S0.b : S1.b};
+        step(X, X, last, no, no, works);
     };
-
-    gemm_dma_loop(
-        steps, !kGrouped || row0 + wm * (NA * 16u) < row_end, A0, B0, A1, B1, issue,
-        [&](const char* As, const char* Bs) __attribute__((always_inline)) {
+    {
+        const auto from0 = bases(0u), from1 = bases(last < 1u ? last : 1u);
 #pragma unroll
-            for (int i = 0; i < NH + kBReads; ++i) first_operands(As, Bs, i);
-        },
-        head, tail,
-        [&]() __attribute__((always_inline)) {
+        for (int u = 0; u < kLoads; ++u) load(from0, u, S0);
 #pragma unroll
-            for (int n = 0; n < kM; ++n) mfma(3, n);
-            // The last sums are on their way through the matrix pipe, which the compiler does not know: it sees them
-            // changed behind the wait, so that nothing that reads them can move ahead of it.  (check_matrix_asm.py looks
-            // through the machine code for what this cannot rule out, a copy inside the loop.)
-            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        for (int u = 0; u < kLoads; ++u) load(from1, u, S1);
+        arrive(std::integral_constant<int, 2 * kLoads - kMid>{});
+    }
+    // a wavefront whose rows all lie past the end of the tile's group skips the matrix work and only keeps the loads and
+    // barriers going: its SIMD then runs one wavefront's matrix instructions per K step instead of two
+    if (!kGrouped || row0 + wm * (NA * 16u) < row_end) {
 #pragma unroll
-            for (int i = 0; i < NA; ++i) {
+        for (int i = 0; i < NH + kBReads; ++i) first_operands(S0, i);
+        run_steps(std::true_type{});
+        static_for<kM>([&](auto n) { mfma(3, decltype(n)::value); });
+    } else {
+        run_steps(std::false_type{});
+    }
+    // The last sums are on their way through the matrix pipe, which the compiler does not know: it sees them
+    // changed behind the wait, so that nothing that reads them can move ahead of it.  (check_matrix_asm.py looks
+    // through the machine code for what this cannot rule out, a copy inside the loop.)
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-                for (int j = 0; j < TJ; ++j) asm volatile("" : "+v"(acc[i][j]));
-            }
-        });
+    for (int i = 0; i < NA; ++i) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+    }
 
     // ---- epilogue: register r of lane l in a 16 x 16 block is row 4 (l / 16) + r, column l % 16
     const uint32_t colw = n0 + wn * 64u;  // first column of this wavefront
@@ -331,7 +399,7 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
         __syncthreads();  // everyone has left the last stage
     }
     if (by_element) {
-        int32_t* const mine = reinterpret_cast<int32_t*>(B0) + wave * 512u;
+        int32_t* const mine = reinterpret_cast<int32_t*>(S0.b) + wave * 512u;
         auto cell = [](uint32_t row, uint32_t c) __attribute__((always_inline)) { return row * 32u + (c ^ ((row << 2) & 16u)); };
 #pragma unroll 1
         for (uint32_t part = 0; part < NA * 2u; ++part) {
@@ -767,8 +835,8 @@ __device__ __forceinline__ void gemm_dma_body32(const GemmParams& p, const TileP
 // that is no multiple of 16 the last tile is moved left until it ends at n (n >= BN then): the columns it shares with
 // its neighbour are computed twice, with the same values.
 template <int BM, int BN, bool kSplitK, bool kGrouped, int kB, int kForm>
-__device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const TilePlace& at, uint32_t bidy, char* A0,
-                                                 char* B0, char* A1, char* B1, float* TS)
+__device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const TilePlace& at, uint32_t bidy, const Stage& S0,
+                                                 const Stage& S1, float* TS)
 {
     constexpr bool kBT = kB == 1, kBP = kB == 2;
     constexpr int kPieces = BN / 16;        // 16-byte pieces per B row
@@ -801,8 +869,15 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     uint32_t aoff[kAInstr], boff[kBInstr];
 #pragma unroll
     for (int u = 0; u < kAInstr; ++u) {
-        const uint32_t s = a_slot(u);
-        uint32_t row = row0 + (s >> 3);
+        uint32_t s = a_slot(u), line = s >> 3;
+        if constexpr (kForm == k16) {
+            // loads of half h of every wavefront's rows: line r of its LDS array is row r % kRows of that half of wavefront
+            // row r / kRows
+            constexpr uint32_t kPart = kAInstr / 2, kRows = BM * (BN / 64) / 16;
+            s = (wave * kPart + u % kPart) * 64u + lane;
+            line = ((s >> 3) / kRows * 2u + u / kPart) * kRows + (s >> 3) % kRows;
+        }
+        uint32_t row = row0 + line;
         row = row < row_end ? row : row_end - 1;  // rows past the end are never stored: any valid row will do
         aoff[u] = (row - row0) * K + 16u * line_piece(s);
     }
@@ -894,39 +969,48 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
 
     if constexpr (kForm == k16) {
         static_assert(!kSplitK, "K splits run the other form");
-        gemm_dma_body16<BM, BN, kGrouped, kB>(p, at, n0, steps, wave, lane, issue, A0, B0, A1, B1, TS);
+        struct Bases {
+            const int8_t *a, *b;
+        };
+        auto bases = [&](uint32_t step) __attribute__((always_inline)) {
+            return Bases{uniform(Abase + step * BK), uniform(Bbase + static_cast<size_t>(step) * BK * ldb)};
+        };
+        auto load = [&](const Bases& from, int u, const Stage& S) __attribute__((always_inline)) {
+            if (u < kBInstr) {
+                asm volatile("" : "+v"(boff[u]));
+                __builtin_amdgcn_global_load_lds((gptr_t)(from.b + boff[u]), (lds_ptr_t)(S.b + (wave * kBInstr + u) * 1024), 16, 0, 0);
+            } else {
+                constexpr int kPart = kAInstr / 2;
+                const int v = u - kBInstr;
+                asm volatile("" : "+v"(aoff[v]));
+                __builtin_amdgcn_global_load_lds((gptr_t)(from.a + aoff[v]), (lds_ptr_t)(S.a[v / kPart] + (wave * kPart + v % kPart) * 1024), 16, 0, 0);
+            }
+        };
+        gemm_dma_body16<BM, BN, kGrouped, kB, kAInstr, kBInstr>(p, at, n0, steps, wave, lane, bases, load, S0, S1, TS);
     } else {
-        gemm_dma_body32<BM, BN, kSplitK, kGrouped, kB>(p, at, n0, steps, bidy, wave, lane, issue, A0, B0, A1, B1, TS);
+        gemm_dma_body32<BM, BN, kSplitK, kGrouped, kB>(p, at, n0, steps, bidy, wave, lane, issue, S0.a[0], S0.b, S1.a[0], S1.b, TS);
     }
 }
 
-// The matrix instruction of a call's 256-row tiles (smaller ones always run the 32 x 32 x 32 one).  What bounds the large
-// ones is the power limit: on random operands the clock settles near 1.6 GHz whatever the schedule does, so what pays is
-// energy per product, and the 16 x 16 x 64 instruction moves half the sums.  Away from that limit it loses: behind a step's
-// barrier it waits for the reads of a 64-k sub-step where the other waits for a 32-k one.  The limit is met by most of
-// the chip's units busy for a good while; in us, 32 x 32 x 32 and 16 x 16 x 64:
-//   k = 4096, plain: 128 tiles 44.9 and 45.6, 172 47.9 and 48.1 (packed weights 53.4 and 51.3), 192 50.5 and 49.2, 224 55.9 and 53.9, 256 61.0 and 57.9, 344
-//   90.6 and 86.2, 688 168 and 163; grouped: 128 67.0 and 67.3, 448 190 and 179, 896 293 and 279;
-//   k = 2048, grouped: 160 41.8 and 42.9, 256 53.8 and 53.4, 512 with SwiGLU 118 and 121, 1024 157 and 154;
-//   k = 1024: 256 22.0 and 21.7, 1024 92.6 and 94.8; k = 512: 256 15.7 and 15.5, 258 21.5 and 22.2.
-// Outputs other than half and bfloat16 are what the other form writes from registers.
+// The matrix instruction of a call's 256-row tiles (smaller ones always run the 32 x 32 x 32 one): the 16 x 16 x 64 form moves
+// half the sums, which is what counts where the power limit sets the clock, and its loads have longer to arrive.
+// Outputs other than half and bfloat16 are what the other form writes from registers.  In us with the quantiser, 32 x 32 x 32
+// and 16 x 16 x 64: 2048 x 4096 x 11008 98.1 and 88.3; 2048 x 2048 x 5632 38.0 and 36.2; 1024 x 11008 x 4096 (64 tiles) 107.8 and
+// 103.9; 600 x 4096 x 4096 48.5 and 47.3; 4096 x 512 x 4096 21.3 and 21.2; 4096 x 256 x 8192 30.0 and 29.9.
 inline int gemm_dma_form(const GemmParams& p)
 {
     if (p.k % BK != 0) {
         return k32Ragged;
     }
-    if (p.epi.quant_mode == ASCQ_MM_QUANT_NONE || (p.epi.out_dtype != ASCQ_F16 && p.epi.out_dtype != ASCQ_BF16)) {
-        return k32;
-    }
-    const uint64_t tiles = static_cast<uint64_t>((p.m + 255u) / 256u) * ((p.n + 255u) / 256u);
-    return p.k >= 3072u && 3u * tiles >= 2u * device_compute_units() ? k16 : k32;
+    const bool half = p.epi.quant_mode != ASCQ_MM_QUANT_NONE && (p.epi.out_dtype == ASCQ_F16 || p.epi.out_dtype == ASCQ_BF16);
+    return half ? k16 : k32;
 }
 
 // The plain matmul: tile number `bid` of the launch (before the XCD remapping), column tiles counted from col_begin,
 // row tiles innermost so that the tiles an XCD runs side by side share their B columns.
 template <int BM, int BN, bool kSplitK, int kB, int kForm>
 __device__ __forceinline__ void gemm_dma_tile(const GemmParams& p, uint32_t col_begin, uint32_t bid, uint32_t bidy,
-                                              char* A0, char* B0, char* A1, char* B1, float* TS)
+                                              const Stage& S0, const Stage& S1, float* TS)
 {
     const uint32_t total = p.tiles_m * p.tiles_n;
     const uint32_t t = xcd_remap(bid, total);
@@ -938,19 +1022,22 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmParams& p, uint32_t col_
     uint32_t ms, tn;
     band_order(t, p.tiles_m, p.tiles_n, ms, tn);
     const TilePlace at{ms * BM, p.m, col_begin + tn * BN, p.b, 0};
-    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, A0, B0, A1, B1, TS);
+    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, S0, S1, TS);
 }
+
+// The LDS stages S0 and S1 of a kernel (an array that nothing reads takes no space).
+#define ASCQ_DMA_STAGES(kForm, BM, BN)                                                                       \
+    __shared__ __attribute__((aligned(1024))) char A0[BM * BK / (kForm == k16 ? 2 : 1)], A1[sizeof(A0)];      \
+    __shared__ __attribute__((aligned(1024))) char A0h[sizeof(A0)], A1h[sizeof(A0)], B0[BK * BN], B1[BK * BN]; \
+    const Stage S0{{A0, A0h}, B0}, S1{{A1, A1h}, B1}
 
 template <int BM, int BN, bool kSplitK, int kB, int kForm>
 __global__ __launch_bounds__(kThreads, (BM * BK + BK * BN) * 2 <= 65536 ? 2 : 1) void gemm_dma_kernel(
     GemmParams p, uint32_t col_begin)
 {
-    __shared__ __attribute__((aligned(1024))) char A0[BM * BK];
-    __shared__ __attribute__((aligned(1024))) char B0[BK * BN];
-    __shared__ __attribute__((aligned(1024))) char A1[BM * BK];
-    __shared__ __attribute__((aligned(1024))) char B1[BK * BN];
+    ASCQ_DMA_STAGES(kForm, BM, BN);
     __shared__ __attribute__((aligned(16))) float TS[BM];  // token scales of the tile's rows (1.0f when there are none)
-    gemm_dma_tile<BM, BN, kSplitK, kB, kForm>(p, col_begin, blockIdx.x, blockIdx.y, A0, B0, A1, B1, TS);
+    gemm_dma_tile<BM, BN, kSplitK, kB, kForm>(p, col_begin, blockIdx.x, blockIdx.y, S0, S1, TS);
 }
 
 // One launch for a matrix whose last round of 256 x 256 tiles would be mostly empty: workgroups [0, wide_wgs) run the
@@ -960,17 +1047,14 @@ template <int kB, int kForm>
 __global__ __launch_bounds__(kThreads, 1) void gemm_dma_dual_kernel(GemmParams p, uint32_t wide_wgs,
                                                                     uint32_t narrow_tiles_n, uint32_t col_begin)
 {
-    __shared__ __attribute__((aligned(1024))) char A0[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B0[BK * 256];
-    __shared__ __attribute__((aligned(1024))) char A1[256 * BK];
-    __shared__ __attribute__((aligned(1024))) char B1[BK * 256];
+    ASCQ_DMA_STAGES(kForm, 256, 256);
     __shared__ __attribute__((aligned(16))) float TS[256];
     if (blockIdx.x < wide_wgs) {
-        gemm_dma_tile<256, 256, false, kB, kForm>(p, 0u, blockIdx.x, 0u, A0, B0, A1, B1, TS);
+        gemm_dma_tile<256, 256, false, kB, kForm>(p, 0u, blockIdx.x, 0u, S0, S1, TS);
     } else {
         GemmParams q = p;
         q.tiles_n = narrow_tiles_n;
-        gemm_dma_tile<256, 128, false, kB, kForm>(q, col_begin, blockIdx.x - wide_wgs, 0u, A0, B0, A1, B1, TS);
+        gemm_dma_tile<256, 128, false, kB, kForm>(q, col_begin, blockIdx.x - wide_wgs, 0u, S0, S1, TS);
     }
 }
 

@@ -529,6 +529,34 @@ def test_w8a8_both_matrix_instructions_agree(k, n, layout, kind):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("layout", ["kn", "nk", "packed"])
+@pytest.mark.parametrize("m,n,k", [(520, 528, 128), (600, 264, 256), (513, 528, 384), (1000, 272, 512), (520, 1040, 640), (769, 528, 768),
+                                   (2048, 11008, 256)])
+def test_w8a8_large_tiles_with_half_outputs(m, n, k, layout):
+    """256-row tiles whose loads have one and a half K steps to arrive: one to six K steps (prologue, steady state and both
+    peeled ends), row and column remainders; the last size runs 256 x 256 and 256 x 128 tiles in one launch."""
+    announce("half outputs", m, n, k, layout)
+    rng = np.random.default_rng(m + n + k)
+    a, b = rand_i8(rng, (m, k), -128, 127), rand_i8(rng, (k, n), -128, 127)
+    sc, tok = rng.uniform(1e-4, 1e-3, n).astype(np.float32), rng.uniform(5e-3, 2e-2, m).astype(np.float32)
+    mm = ops.Matmul(m, n, k, False, layout == "nk")
+    mm.set_tensor_a(to_dev(a))
+    if layout == "packed":
+        mm.set_tensor_b_packed(ops.pack_weight_w8(to_dev(b), k, n))
+    else:
+        mm.set_tensor_b(to_dev(np.ascontiguousarray(b.T) if layout == "nk" else b))
+    mm.set_quant_vector(to_dev(sc))
+    mm.set_token_scale(to_dev(tok))
+    want = None
+    for out in (torch.bfloat16, torch.float16):
+        c = torch.zeros((m, n), dtype=out, device=DEV)
+        mm.iterate_all(c)
+        # fp32 with one rounding per step, then one to the output (float32 holds every sum of up to 768 products exactly)
+        if want is None:
+            want = (a.astype(np.float32) @ b.astype(np.float32)) * sc * tok[:, None]
+        assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+
+
 @pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu"])
 def test_group_matmul_both_matrix_instructions_agree(kind):
     """The grouped matmul at a size for the 16 x 16 x 64 instruction against the plain matmul of each group's rows."""
