@@ -17,7 +17,7 @@ import sys
 import tempfile
 
 LLVM = os.environ.get("LLVM_BIN", "/opt/rocm/llvm/bin")
-MATRIX = ("v_mfma_i32_16x16x64_i8", "v_mfma_f32_16x16x32_f16")
+MATRIX = ("v_mfma_i32_16x16x64_i8", "v_mfma_f32_16x16x32_f16", "v_mfma_scale_f32_16x16x128_f8f6f4")
 kResult, kOperand = 19, 2
 
 

@@ -36,4 +36,8 @@ __device__ __forceinline__ void mx_store(const MxParams& p, size_t idx, float v)
 bool mx_decode_supported(const MxParams& p);
 int launch_mx_decode(const MxParams& p, bool tile_shape, hipStream_t st);
 
+// matmul_mx_six.hip: two e1m2 operands, k a multiple of 128, on a workspace of mx_six_bytes (16-byte aligned)
+size_t mx_six_bytes(uint32_t m, uint32_t n, uint32_t k);
+int launch_mx_six(const MxParams& p, void* workspace, hipStream_t st);
+
 }  // namespace ascq

@@ -11,15 +11,11 @@
 //     from lanes 32-63: two 16-byte LDS reads per operand and instruction.
 //   * 4-bit operands: registers 0-3 of lane l hold its row's k = 32 (l / 32) .. + 31 (16 bytes), scaled by the lane's
 //     own scale byte: one read per operand and instruction.
-//   * 6-bit operands (e2m3 codes, what two e1m2 operands are rewritten as): registers 0-5 of lane l hold its row's
-//     k = 32 (l / 32) .. + 31 as little-endian 6-bit fields (24 bytes), scaled by the lane's own scale byte: a 16-byte and
-//     an 8-byte read per operand and instruction, from units of 32 rows x 64 k in lane order.  (What bounds this form is
-//     the rate at which tiles reach the LDS: with each block of 32 k padded to 32 bytes m = n = k = 8192 took 419 us, both
-//     widening passes included, without the padding 365 us; 874 x 2000 x 8960 104 -> 73 us.)
 // In every case lane l needs scale byte 2 j + l / 32 of its row's bytes for this K step in sub-step j; a lane holds
-// the bytes of a K step as one dword (8- and 6-bit) or two (4-bit) per row, staged through LDS, and shifts them right
+// the bytes of a K step as one dword (8-bit) or two (4-bit) per row, staged through LDS, and shifts them right
 // by 8 (l / 32) where they are used, so that the byte selector of the instruction is the constant 0 or 2.
-// A 4-bit operand beside an 8-bit one, or e1m2 beside e2m1, is first widened to e4m3, which holds every fp4 value.
+// A 4-bit operand beside an 8-bit one, or e1m2 beside e2m1, is first widened to e4m3, which holds every fp4 value; two e1m2
+// operands run matmul_mx_six.hip.
 // Few rows, and shapes whose rows or scale rows do not fit these tiles, run matmul_mx_decode.hip; what is left (rows that
 // are no whole number of 16-byte pieces, scale rows that are no whole number of dwords) the element-wise kernel (one
 // lane per output).
@@ -54,19 +50,16 @@ constexpr int kMxThreads = 512;
 constexpr uint32_t kMxScaleBuf = (kMxBM + kMxBN) * 16u;  // 16 scale bytes of every row of a tile's a and b
 
 // kFour: both operands 4-bit (e2m1); otherwise both a byte per value in memory, with the instruction's format codes
-// kCa / kCb (0 = e4m3, 1 = e5m2, 2 = e2m3 as written by mx_widen_e1m2_kernel; 4 = e2m1).
+// kCa / kCb (0 = e4m3, 1 = e5m2; 4 = e2m1).
 template <bool kFour, int kCa, int kCb>
 __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
 {
     constexpr int TI = 4, TJ = 2;
-    constexpr bool kSix = !kFour && kCa == 2;  // e2m3 codes in units of 32 rows x 64 k (mx_widen_e1m2_kernel)
-    constexpr uint32_t kRowBytes = kSix ? 96u : kMxBK;  // bytes of a row and K step in LDS
-    __shared__ __attribute__((aligned(1024))) char A0[kMxBM * kRowBytes];
-    __shared__ __attribute__((aligned(1024))) char B0[kMxBN * kRowBytes];
-    __shared__ __attribute__((aligned(1024))) char A1[kMxBM * kRowBytes];
-    __shared__ __attribute__((aligned(1024))) char B1[kMxBN * kRowBytes];
+    __shared__ __attribute__((aligned(1024))) char A0[kMxBM * kMxBK];
+    __shared__ __attribute__((aligned(1024))) char B0[kMxBN * kMxBK];
+    __shared__ __attribute__((aligned(1024))) char A1[kMxBM * kMxBK];
+    __shared__ __attribute__((aligned(1024))) char B1[kMxBN * kMxBK];
     __shared__ __attribute__((aligned(1024))) char SC[2 * kMxScaleBuf];  // two buffers of scale bytes, see below
-    static_assert(!kSix || kCb == 2, "6-bit operands come in pairs");
     constexpr int kSub = kFour ? 4 : 2;       // instructions (64 k each) per K step and block pair
     constexpr int kScaleDw = kFour ? 2 : 1;   // dwords of scale bytes per row and K step
 
@@ -99,19 +92,11 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
 
     // ---- DMA sources: 4 A and 4 B instructions per wavefront and K step; lane owns LDS slot (instr * 64 + lane) of
     // 16 bytes: row slot / 8, position slot % 8, which holds piece position ^ ((row / 2) % 8) of the row's 128 bytes.
-    // 6-bit operands: 3 and 3 instructions, the two units of a block of 32 rows as they lie in memory.
-    constexpr int kInstr = kSix ? 3 : 4;
+    constexpr int kInstr = 4;
     uint32_t aoff[kInstr], boff[kInstr];
 #pragma unroll
     for (int u = 0; u < kInstr; ++u) {
         const uint32_t s = (wave * kInstr + u) * 64u + lane;
-        if constexpr (kSix) {
-            const uint32_t block = s / 192u, at = s % 192u * 16u;
-            const uint32_t a_last = (p.m + 31u) / 32u - 1u - row0 / 32u, b_last = (p.n + 31u) / 32u - 1u - n0 / 32u;
-            aoff[u] = (block < a_last ? block : a_last) * (RB * 24u) + at;
-            boff[u] = (block < b_last ? block : b_last) * (RB * 24u) + at;
-            continue;
-        }
         const uint32_t r = s >> 3, c = (s & 7u) ^ ((r >> 1) & 7u);
         uint32_t row = row0 + r, col = n0 + r;
         row = row < p.m ? row : p.m - 1u;  // rows and columns past the end are never stored: any valid one will do
@@ -119,9 +104,8 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         aoff[u] = (row - row0) * RB + 16u * c;
         boff[u] = (col - n0) * RB + 16u * c;
     }
-    // (a block of 32 rows of 6-bit operands is RB / 64 units of 1536 bytes)
-    const uint8_t* Abase = p.a + (kSix ? static_cast<size_t>(row0 / 32u) * (RB * 24u) : static_cast<size_t>(row0) * RB);
-    const uint8_t* Bbase = p.b + (kSix ? static_cast<size_t>(n0 / 32u) * (RB * 24u) : static_cast<size_t>(n0) * RB);
+    const uint8_t* Abase = p.a + static_cast<size_t>(row0) * RB;
+    const uint8_t* Bbase = p.b + static_cast<size_t>(n0) * RB;
     // A wavefront-uniform address, pinned to scalar registers: a load's address is then this base plus the lane's
     // 32-bit offset, which the load instruction adds itself (otherwise the compiler folds the lane's offset into
     // 64-bit per-lane addresses: twice the registers and an addition per load).
@@ -133,8 +117,8 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         return reinterpret_cast<const uint8_t*>((static_cast<uint64_t>(hi) << 32) | lo);
     };
     auto issue = [&](uint32_t k0, char* As, char* Bs) __attribute__((always_inline)) {
-        const uint8_t* ab = uniform(Abase + (kSix ? k0 * 24u : k0));
-        const uint8_t* bb = uniform(Bbase + (kSix ? k0 * 24u : k0));
+        const uint8_t* ab = uniform(Abase + k0);
+        const uint8_t* bb = uniform(Bbase + k0);
         // (re-materialised here: widened to 64 bits once, ahead of the loop, the offsets would no longer be seen as
         // 32-bit offsets where the loads are selected)
 #pragma unroll
@@ -224,26 +208,15 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
     // ---- fragments: piece q of tile line r sits at r * 128 + ((q ^ ((r / 2) % 8)) * 16).  A lane reads piece
     // kPieceStep u + h (+ 2 for the upper registers of an 8-bit operand) of a line whose number is lrow + a multiple
     // of 32, i.e. at lrow * 128 + (((kPieceStep u) ^ (h ^ swizzle)) * 16) + constants: one register per u.
-    // (6-bit operands: the lane's 16 bytes of a unit at 16 l, its other 8 at 1024 + 8 l)
     constexpr int kPieceStep = 2;
-    constexpr int kPieces = kSix ? 2 : 4;   // u = 0 .. 3: pieces 0 2 4 6 (+ h)
+    constexpr int kPieces = 4;   // u = 0 .. 3: pieces 0 2 4 6 (+ h)
     uint32_t foff[kPieces];
 #pragma unroll
     for (int u = 0; u < kPieces; ++u) {
-        foff[u] = kSix ? (u == 0 ? lane * 16u : 1024u + lane * 8u)
-                       : lrow * 128u + (((static_cast<uint32_t>(kPieceStep * u) ^ h ^ ((lrow >> 1) & 7u))) << 4);
+        foff[u] = lrow * 128u + (((static_cast<uint32_t>(kPieceStep * u) ^ h ^ ((lrow >> 1) & 7u))) << 4);
     }
     auto frag = [&](const char* S, uint32_t line0, int u) __attribute__((always_inline)) {
         return *reinterpret_cast<const i32x4*>(S + line0 * 128u + foff[u]);
-    };
-    auto frag_six = [&](const char* S, uint32_t block, int s) __attribute__((always_inline)) {
-        const char* unit = S + block * 3072u + s * 1536u;
-        const i32x4 lo = *reinterpret_cast<const i32x4*>(unit + foff[0]);
-        const i32x2_t hi = *reinterpret_cast<const i32x2_t*>(unit + foff[1]);
-        v8i t = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 6 registers
-        t[4] = hi[0];
-        t[5] = hi[1];
-        return t;
     };
     struct Frags {
         v8i a[TI], b[TJ];
@@ -256,8 +229,6 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
             if constexpr (kFour) {
                 const i32x4 lo = frag(As, line0, s);
                 f.a[i] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // the instruction reads 4 registers of a 4-bit operand
-            } else if constexpr (kSix) {
-                f.a[i] = frag_six(As, line0 / 32u, s);
             } else {
                 const i32x4 lo = frag(As, line0, 2 * s), hi = frag(As, line0, 2 * s + 1);
                 f.a[i] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -269,8 +240,6 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
             if constexpr (kFour) {
                 const i32x4 lo = frag(Bs, line0, s);
                 f.b[j] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);
-            } else if constexpr (kSix) {
-                f.b[j] = frag_six(Bs, line0 / 32u, s);
             } else {
                 const i32x4 lo = frag(Bs, line0, 2 * s), hi = frag(Bs, line0, 2 * s + 1);
                 f.b[j] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -520,48 +489,6 @@ __global__ __launch_bounds__(256) void mx_widen_fp4_kernel(const u32x4* __restri
     }
 }
 
-// e1m2 [rows, k / 2 bytes] -> e2m3 codes in units of 32 rows x 64 k, k innermost: 1024 bytes that hold bytes 0 - 15 and
-// 512 that hold bytes 16 - 23 of the 24 a lane of the matrix instruction owns (its row's 32 consecutive k as little-endian
-// 6-bit fields), in lane order.  So the tiles of the matmul are contiguous runs, a lane's operand two LDS reads without
-// bank conflicts (the 19.2 M conflict cycles a launch of m = n = k = 8192 counts are those of the scale reads, as in the fp8 form,
-// 43 % of this form's LDS cycles), and 96 bytes of a row travel per 128 k.  An e1m2 value is +-(code / 4), code 0 .. 7, which is the e2m3 value with magnitude
-// bits 2 * code (its subnormals run 0, 1/8 .. 7/8 and its first binade 1, 9/8 .. 15/8).  Both operands in one launch: a
-// workgroup takes 32 rows x 256 k, whole 128-byte lines of the source.
-struct MxWidenParams {
-    const uint8_t* src[2];
-    uint8_t* dst[2];
-    uint32_t rows[2];
-    uint32_t a_blocks, k_blocks, k;  // workgroups of the first operand; workgroups per block of 32 rows
-};
-
-__global__ __launch_bounds__(256) void mx_widen_e1m2_kernel(MxWidenParams p)
-{
-    const uint32_t which = blockIdx.x < p.a_blocks ? 0u : 1u;
-    const uint32_t id = blockIdx.x - (which ? p.a_blocks : 0u);
-    const uint32_t lane = threadIdx.x & 63u, unit = (id % p.k_blocks) * 4u + (threadIdx.x >> 6), block = id / p.k_blocks;
-    if (unit >= p.k / 64u) {
-        return;
-    }
-    uint32_t row = block * 32u + (lane & 31u);
-    row = row < p.rows[which] ? row : p.rows[which] - 1u;  // (rows past the end are never stored by the matmul)
-    const u32x4 q = *reinterpret_cast<const u32x4*>(p.src[which] + static_cast<size_t>(row) * (p.k / 2u) + unit * 32u + (lane >> 5) * 16u);
-    uint64_t c[4];  // 32 values, value v of a dword in bits 4 v .. 4 v + 3
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        uint64_t t = q[d];
-        t = (t & 0xFFFFull) | ((t & 0xFFFF0000ull) << 8);                              // values 0-3 | 4-7, 24 bits each
-        t = (t & 0x00000000FF0000FFull) | ((t & 0x000000FF0000FF00ull) << 4);          // pairs, 12 bits each
-        t = (t & 0x00000F00F00F00Full) | ((t & 0x0000F00F00F00F0ull) << 2);            // value v in bits 6 v .. 6 v + 3
-        c[d] = ((t & 0x0000208208208208ull) << 2) | ((t & 0x00001C71C71C71C7ull) << 1);  // sign to bit 5, magnitude doubled
-    }
-    uint8_t* const out = p.dst[which] + (static_cast<size_t>(block) * (p.k / 64u) + unit) * 1536u;
-    *reinterpret_cast<u32x4*>(out + lane * 16u) =
-        u32x4{static_cast<uint32_t>(c[0]), static_cast<uint32_t>(c[0] >> 32) | (static_cast<uint32_t>(c[1]) << 16),
-              static_cast<uint32_t>(c[1] >> 16), static_cast<uint32_t>(c[2])};
-    *reinterpret_cast<u32x2*>(out + 1024u + lane * 8u) =
-        u32x2{static_cast<uint32_t>(c[2] >> 32) | (static_cast<uint32_t>(c[3]) << 16), static_cast<uint32_t>(c[3] >> 16)};
-}
-
 inline bool is_fp8(int f) { return f == ASCQ_QDST_FP8_E4M3FN || f == ASCQ_QDST_FP8_E5M2; }
 inline bool is_fp4(int f) { return f == ASCQ_QDST_FP4_E2M1 || f == ASCQ_QDST_FP4_E1M2; }
 
@@ -578,10 +505,10 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     bool wa, wb;
     mx_widen_plan(d, wa, wb);
     const bool four = is_fp4(d->a_format) && !wa;  // both e2m1
-    // two e1m2 operands: the 6-bit codes of their rows, each rounded up to 32, must fit the workspace of a byte per value
-    // (24 bytes for 32 values; only some pairs of little over 64 rows do not)
-    const uint64_t blocks = (static_cast<uint64_t>(d->m) + 31u) / 32u + (static_cast<uint64_t>(d->n) + 31u) / 32u;
-    if (d->a_format == ASCQ_QDST_FP4_E1M2 && d->b_format == ASCQ_QDST_FP4_E1M2 && blocks * 24u > static_cast<uint64_t>(d->m) + d->n) {
+    // two e1m2 operands: the 6-bit codes of their rows, each rounded up to 32, and their scales must fit the workspace of a
+    // byte per value (24 bytes for 32 values; only some pairs of little over 64 rows do not)
+    if (d->a_format == ASCQ_QDST_FP4_E1M2 && d->b_format == ASCQ_QDST_FP4_E1M2 &&
+        mx_six_bytes(d->m, d->n, d->k) > (static_cast<uint64_t>(d->m) + d->n) * d->k) {
         return false;
     }
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
@@ -591,21 +518,22 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
 // Both times are estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
 // meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 1.85 (8-bit b), 0.95 (the 32-row
 // form), 2.0 (two 4-bit operands, one of them e1m2).  Tiles: rounds of 256 x 256 tiles, 1.3
-// per K step, and the passes that widen 4-bit operands, 1 per 3 MB of their codes.  Measured at n = k = 8192, decode
-// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 20.7 and 78, e1m2 20 and 93; 128 rows e4m3 34 and 79, e1m2 36 and 97; 256
-// rows e2m1 41 and 47, e4m3 64 and 85, e1m2 69 and 103; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44, 42 and 64;
-// n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147, 30 and 154.
+// per K step (0.85 for two e1m2 operands), and the passes that widen 4-bit operands, 1 per 3 MB of their codes.  Measured at n = k = 8192, decode
+// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 20.7 and 78; 128 rows e4m3 34 and 79; 256 rows e2m1 41 and 47, e4m3 64 and
+// 85; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44; n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147; two e1m2
+// operands: 874 x 2000 x 8960 75 and 63, 200 x 14336 x 4096 56 and 46, 300 x 8192 x 4096 53 and 45.
 bool mx_decode_preferred(const MxParams& p)
 {
     const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
     const bool two4 = p.a_format == ASCQ_QDST_FP4_E2M1 && p.b_format == ASCQ_QDST_FP4_E2M1;
+    const bool six = p.a_format == ASCQ_QDST_FP4_E1M2 && p.b_format == ASCQ_QDST_FP4_E1M2;
     const double cus = device_compute_units();
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
     const double per_k = two4 ? 1.15 : b8 ? 1.85 : a8 ? 0.95 : 2.0;
     const double decode = 4.0 + rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u)) * per_k * p.k / 1024.0;
     const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
-    const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * 1.3 *
+    const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * (six ? 0.85 : 1.3) *
                                            p.k / (two4 ? 256.0 : 128.0);
     return decode < tiles;
 }
@@ -690,8 +618,9 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         return launch_status("ascq_matmul_mx (element-wise)");
     }
     int fa = d->a_format, fb = d->b_format;
-    // two e1m2 operands become e2m3 codes, which the matrix core runs at the 4-bit rate; any other 4-bit operand e4m3
-    const bool six = fa == ASCQ_QDST_FP4_E1M2 && fb == ASCQ_QDST_FP4_E1M2;
+    if (fa == ASCQ_QDST_FP4_E1M2 && fb == ASCQ_QDST_FP4_E1M2) {
+        return launch_mx_six(p, workspace, st);
+    }
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     auto widen = [&](const uint8_t*& src, int& fmt, size_t rows) {
         const size_t pieces = rows * (d->k / 2u) / 16u;  // k is a multiple of 128 here
@@ -703,18 +632,10 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         ws += rows * d->k;
         fmt = ASCQ_QDST_FP8_E4M3FN;
     };
-    if (six) {
-        const uint32_t a_rows = (d->m + 31u) / 32u;
-        MxWidenParams w{{p.a, p.b}, {ws, ws + static_cast<size_t>(a_rows) * 24u * d->k}, {d->m, d->n}, 0, (d->k + 255u) / 256u, d->k};
-        w.a_blocks = a_rows * w.k_blocks;
-        mx_widen_e1m2_kernel<<<w.a_blocks + (d->n + 31u) / 32u * w.k_blocks, 256, 0, st>>>(w);
-        p.a = w.dst[0];
-        p.b = w.dst[1];
-        fa = fb = ASCQ_QDST_FP8_E4M3FN;  // (a byte per value as far as the sizes below go)
-    } else if (wa) {
+    if (wa) {
         widen(p.a, fa, d->m);
     }
-    if (wb && !six) {
+    if (wb) {
         widen(p.b, fb, d->n);
     }
     const bool four = is_fp4(fa);  // (after the widening: both e2m1)
@@ -724,8 +645,6 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
     const uint32_t grid = (p.tiles_m * p.tiles_n + 7u) / 8u * 8u;
     if (four) {
         mx_tile_kernel<true, 4, 4><<<grid, kMxThreads, 0, st>>>(p);
-    } else if (six) {
-        mx_tile_kernel<false, 2, 2><<<grid, kMxThreads, 0, st>>>(p);
     } else if (fa == ASCQ_QDST_FP8_E4M3FN && fb == ASCQ_QDST_FP8_E4M3FN) {
         mx_tile_kernel<false, 0, 0><<<grid, kMxThreads, 0, st>>>(p);
     } else if (fa == ASCQ_QDST_FP8_E4M3FN) {

@@ -134,6 +134,28 @@ def test_mx_e1m2_pairs_on_the_tile_kernel(m, n, k):
     mx_check(run_mx(m, n, k, a, b, sa, sb, F1, F1).cpu().numpy(), want, mx_abs_dot(a, b, sa, sb, k, F1, F1), False)
 
 
+@pytest.mark.parametrize("steps,more", [(1, 0), (2, 8), (5, 0), (6, 0), (7, 8), (8, 0), (9, 0), (11, 0), (12, 8), (13, 0)])
+@pytest.mark.parametrize("n,out", [(2109, torch.float32), (2104, torch.bfloat16), (2104, torch.float16), (2106, torch.bfloat16)])
+def test_mx_e1m2_tiles_step_counts_and_outputs(steps, more, n, out):
+    """Two e1m2 operands on the tiles: the loop takes six K steps at a time, then what is left, one by one; scale rows longer
+    than k / 32; the store of four columns per lane and the one of single elements; bias.  Products are exact and the fp32 sums
+    err by 4e-6 of the terms' magnitudes at most, so a 16-bit result is the golden's rounded or within that of a tie."""
+    m, k = 2100, 128 * steps
+    announce("mx e1m2 steps", steps, n, out)
+    rng = np.random.default_rng(steps * 7 + n)
+    a, b, sa, sb, bv = mx_case(rng, m, n, k, F1, F1, sk=max(16, (k // 32 + 7) // 8 * 8) + more, bias=True)
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sa.shape[1], a_format=F1, b_format=F1, out_dtype=abi.F32, has_bias=1)
+    got = run_mx(m, n, k, a, b, sa, sb, F1, F1, out=out, bias=bv).float().cpu().numpy().astype(np.float64)
+    orc.set_threads(16)
+    for r0, r1 in ((0, 40), (120, 140), (250, 260), (2040, 2100)):
+        want = orc.matmul_mx(d, a, b, sa, sb, bv, rows=(r0, r1))[r0:r1].astype(np.float64)
+        dot = mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, F1, F1)
+        half_ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[out]
+        if out == torch.float16:
+            want = np.clip(want, -65504.0, 65504.0)
+        assert np.all(np.abs(got[r0:r1] - want) <= half_ulp * 1.01 * np.abs(want) + 4e-6 * (dot + np.abs(bv)) + 2.0 ** -24)
+
+
 @pytest.mark.parametrize("fa,fb", [(a, b) for a in (E4, E5, F2, F1) for b in (E4, E5, F2, F1)])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 40, 160), (16, 33, 1088), (17, 64, 640), (32, 4112, 256), (33, 100, 2304),
                                    (64, 48, 4096), (65, 32, 1056)])
