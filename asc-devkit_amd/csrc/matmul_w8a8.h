@@ -219,6 +219,14 @@ __device__ __forceinline__ float load_bias_post(const EpiParams& e, size_t col)
 bool gemm_dma_supported(const GemmParams& p, int b_layout = 0);
 // b_layout: 0 B is [k, n] (or fractal), 1 [n, k], 2 the layout of ascq_pack_weight_w8
 int launch_gemm_dma(GemmParams& p, hipStream_t st, int b_layout = 0);
+// matmul_w8a8_ring.hip: the operands that gemm_dma_supported accepts, any k and every output
+struct RingPlan {
+    int shape;
+    uint32_t bm, bn;
+    double us;  // estimate, quantiser included
+};
+RingPlan gemm_ring_plan(uint32_t m, uint32_t n, uint32_t k, int b_layout);
+int launch_gemm_ring(const GemmParams& p, int shape, int b_layout, hipStream_t st);
 int launch_gemm_dma_group(GemmParams& p, hipStream_t st);  // matmul_w8a8_group.hip
 uint32_t gemm_dma_skinny_splits(uint32_t m, uint32_t n, uint32_t k);
 bool gemm_dma_small_tiles(uint32_t m, uint32_t n, uint32_t k);

@@ -737,6 +737,49 @@ bool dma_tiles_small(const ascq_matmul_desc* d)
     return d->m <= kSkinnyMaxM || (d->activation != ASCQ_MM_ACT_SWIGLU && gemm_dma_small_tiles(d->m, d->n, d->k));
 }
 
+// What a call of more than 32 rows takes without the ring kernel, in us with the quantiser (the constants are fits to
+// measurements; `splits`: the K split that its workspace allows).
+double without_ring_us(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, uint32_t splits)
+{
+    const double cus = device_compute_units(), steps = (d->k + 127u) / 128u;
+    const double raw_sums = d->activation == ASCQ_MM_ACT_SWIGLU && d->m <= kSkinnyMaxM && b_layout != 2 ? 6.0 : 0.0;  // a pass of its own
+    if (b_layout != 0 && d->m <= kSkinnyMaxM && gemm_ws_supported(p, b_layout == 1) && (b_layout == 1 || d->m <= 128u || !packed_tiles_faster(p))) {
+        // the weights held in registers; 16 rows take 0.85 us however short k is (181 x 1152 x 864 as [n, k] 19.9 us)
+        const double short_k = 0.85 - 0.95 * d->k / 4096.0;
+        return packed_ws_us(p) + (short_k > 0.0 ? short_k * ((d->m + 15u) / 16u) * gemm_ws_rounds(p) : 0.0) - (d->m <= 64u ? 2.0 : 0.0);
+    }
+    const bool small = d->m <= kSkinnyMaxM || (splits > 1u && d->activation != ASCQ_MM_ACT_SWIGLU && gemm_dma_small_tiles(d->m, d->n, d->k));
+    if (!small) {
+        const double tiles = static_cast<double>((d->m + 255u) / 256u) * ((d->n + 255u) / 256u);
+        return 8.5 + steps * (tiles <= cus ? 1.15 + 0.25 * tiles / cus : 1.35 * tiles / cus);
+    }
+    if (splits > 1u) {
+        // two launches, 0.8 a step, the partial tiles written and read back at 3.4 TB/s
+        const uint32_t each = (static_cast<uint32_t>(steps) + splits - 1u) / splits;
+        return 12.5 + 0.8 * each + static_cast<double>(splits) * d->m * d->n * 8.0 / 3.4e6 + raw_sums;
+    }
+    const double tiles = static_cast<double>((d->m + 127u) / 128u) * ((d->n + 127u) / 128u);
+    const double load = tiles <= cus ? 1.0 : tiles <= 2.0 * cus ? 1.0 + 0.45 * (tiles - cus) / cus : 1.45 * tiles / (2.0 * cus);
+    return 8.5 + 0.81 * steps * load + raw_sums;
+}
+
+// Whether the ring kernel is expected to be ahead, and with which tile.  In us with the quantiser, without and with it: [k, n]
+// weights 729 x 4304 x 1152 28.0 and 21.0, 256 x 4096 x 4096 29.3 and 16.9, 600 x 4096 x 4096 47.4 and 27.8, 1024 x 11008 x 4096 103 and
+// 64, 130 x 5120 x 5120 27.7 and 20.7; packed 192 x 4096 x 4096 24.2 and 15.2, 128 x 4096 x 11008 21.9 and 19.0; behind: 64 x 11008 x
+// 4096 28.6 and 36.0 (ten splits of K on 32 tiles), 512 x 2048 x 11008 24.5 and 28.3 (more tiles of 128 x 128 than units).
+bool ring_preferred(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, const void* workspace, size_t workspace_bytes, RingPlan& plan)
+{
+    if (d->m <= 32u || d->trans_a || d->b_format == ASCQ_MM_B_NZ || !gemm_dma_supported(p, b_layout)) {
+        return false;
+    }
+    uint32_t splits = gemm_dma_skinny_splits(d->m, d->n, d->k);
+    if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < static_cast<size_t>(splits) * d->m * d->n * sizeof(int32_t)) {
+        splits = 1u;
+    }
+    plan = gemm_ring_plan(d->m, d->n, d->k, b_layout);
+    return plan.us < 0.95 * without_ring_us(d, p, b_layout, splits);
+}
+
 // True when the plain matmul of this descriptor runs on the direct-to-LDS tiles without a K split, whose epilogue
 // applies SwiGLU in registers (16-bit outputs).
 bool swiglu_in_tile_kernel(const ascq_matmul_desc* d, const GemmParams& p, const void* a, const void* b)
@@ -911,6 +954,13 @@ extern "C" int ascq_matmul_w8a8(const ascq_matmul_desc* d, void* c, const void* 
         p.b_nz = 1;
         return d->m <= kSkinnyMaxM ? launch_gemm_dma_skinny(p, workspace, workspace_bytes, st)
                                    : launch_gemm_dma(p, st);
+    }
+    RingPlan ring;
+    if (d->k >= 1024u && fast_path_ok(d, a, b) && ring_preferred(d, p, d->trans_b ? 1 : 0, workspace, workspace_bytes, ring) && ring.shape == 0 &&
+        static_cast<uint64_t>((d->m + 63u) / 64u) * ((d->n + 63u) / 64u) <= device_compute_units()) {
+        // (calls whose tiles of 64 x 64 are one round of the chip; the plan query promises the other tiles for larger ones,
+        // which the linears below send to the ring themselves)
+        return launch_gemm_ring(p, ring.shape, d->trans_b ? 1 : 0, st);
     }
     if (!fast_path_ok(d, a, b) && d->m <= 32u && !d->trans_a && !d->trans_b && d->n >= 64u && d->k % 4u == 0 && d->k >= 128u &&
         (reinterpret_cast<uintptr_t>(a) & 3u) == 0 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 3u) == 0 &&
@@ -1173,6 +1223,19 @@ extern "C" int ascq_linear_w8a8_dynamic(const ascq_matmul_desc* d, int32_t x_dty
     if (rc != ASCQ_OK) {
         return rc;
     }
+    {
+        GemmParams p{};
+        p.a = q;
+        p.b = static_cast<const int8_t*>(b);
+        p.m = d->m;
+        p.n = d->n;
+        p.k = d->k;
+        p.epi = make_epi(&dd, c, bias, quant_vector, tok);
+        RingPlan ring;
+        if (ring_preferred(&dd, p, d->trans_b ? 1 : 0, rest, workspace_bytes - static_cast<size_t>(rest - ws), ring)) {
+            return launch_gemm_ring(p, ring.shape, d->trans_b ? 1 : 0, static_cast<hipStream_t>(stream));
+        }
+    }
     return ascq_matmul_w8a8(&dd, c, q, b, bias, quant_vector, tok, rest,
                             workspace_bytes - static_cast<size_t>(rest - ws), stream);
 }
@@ -1228,6 +1291,20 @@ extern "C" int ascq_linear_w8a8_dynamic_packed(const ascq_matmul_desc* d, int32_
         return rc;
     }
     char* rest = reinterpret_cast<char*>(tok) + round256(static_cast<size_t>(d->m) * sizeof(float));
+    {
+        GemmParams p{};
+        p.a = q;
+        p.b = static_cast<const int8_t*>(w_packed);
+        p.m = d->m;
+        p.n = d->n;
+        p.k = d->k;
+        p.epi = make_epi(&dd, c, bias, quant_vector, tok);
+        RingPlan ring;
+        if (gemm_packed_supported(p) &&
+            ring_preferred(&dd, p, 2, rest, workspace_bytes - static_cast<size_t>(rest - ws), ring)) {
+            return launch_gemm_ring(p, ring.shape, 2, static_cast<hipStream_t>(stream));
+        }
+    }
     return matmul_w8a8_packed(&dd, c, q, w_packed, bias, quant_vector, tok, rest, workspace_bytes - static_cast<size_t>(rest - ws),
                               stream);
 }

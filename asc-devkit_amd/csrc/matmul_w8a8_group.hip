@@ -87,13 +87,13 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
             continue;
         }
         if constexpr (phase == 0) {
-            gemm_dma_tile_at<256, 256, false, true, 0, kForm>(p, at, 0u, S0, S1, TS);
+            gemm_dma_tile_at<256, 256, false, true, 0, kForm>(p, at, 0u, TS, S0, S1);
         } else if constexpr (phase == 1) {
-            gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, S0, S1, TS);
+            gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, TS, S0, S1);
         } else if (at.row_end - at.row0 <= 64u) {  // uniform: a remainder of at most 64 rows
-            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, S0, S1, TS);
+            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, TS, S0, S1);
         } else {
-            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, S0, S1, TS);
+            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, TS, S0, S1);
         }
         __syncthreads();  // the next tile's loads and token scales overwrite what slower wavefronts may still read
     }

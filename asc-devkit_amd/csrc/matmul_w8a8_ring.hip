@@ -1,0 +1,103 @@
+// int8 matmul of medium size: small tiles with a ring of LDS stages.
+//
+// What bounds these calls is the way of the operands into the LDS, and its latency: 256 x 256 tiles leave most of the chip
+// idle, and a loop that waits for all of its loads at every K step takes 0.8 to 1.3 us for one, whatever its size.  Here
+// a workgroup (8 wavefronts, v_mfma_i32_16x16x64_i8) owns a tile small enough for most compute units to have one, and the 128 KiB
+// or so of stages that its loads fill hold 4 to 8 K steps: a load has kStages - 1/2 steps to arrive, and a step waits only for
+// the next one's.  A step's operands are read from the LDS behind the matrix instructions of the step before.  No K split, so no
+// int32 partial tiles and no second launch.  A last, partial K step and the steps past
+// the end are loads whose offset lies past the buffer: zeros arrive.
+// In us with the quantiser, split or large tiles and this: 729 x 4304 x 1152 27.8 and 21.0, 600 x 4096 x 4096 47.4 and 27.8, 1024 x
+// 11008 x 4096 103 and 64.  What is left: a step of 64 x 64 takes 0.19 us without the bytes of its loads (the barrier, ten LDS
+// reads and two loads per wavefront), one of 128 x 128 0.46 with nothing but loads (what is in flight over the latency of an L2 miss).
+#include "matmul_w8a8_tile.h"
+
+namespace ascq {
+namespace {
+
+template <int BM, int BN, int kStages, int kB>
+__global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(GemmParams p)
+{
+    constexpr int kBytes = (BM + BN) * BK, kOther = 16;
+    // (an array per stage: the compiler tells at most eight targets of such loads apart; one that nothing reads takes no space)
+    __shared__ __attribute__((aligned(1024))) char L0[kBytes], L1[kBytes], L2[kBytes], L3[kBytes],
+        L4[kStages > 4 ? kBytes : kOther], L5[kStages > 5 ? kBytes : kOther], L6[kStages > 6 ? kBytes : kOther], L7[kStages > 7 ? kBytes : kOther];
+    __shared__ __attribute__((aligned(16))) float TS[BM];
+    const uint32_t t = xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n);
+    if (t >= p.tiles_m * p.tiles_n) {
+        return;
+    }
+    uint32_t ms, tn;
+    band_order(t, p.tiles_m, p.tiles_n, ms, tn);
+    const TilePlace at{ms * BM, p.m, tn * BN, p.b, 0};
+    char* const all[8] = {L0, L1, L2, L3, L4, L5, L6, L7};
+    char* ring[kStages];
+    static_for<kStages>([&](auto i) { ring[decltype(i)::value] = all[decltype(i)::value]; });
+    gemm_dma_tile_at<BM, BN, false, false, kB, kRing>(p, at, 0u, TS, ring);
+}
+
+template <int BM, int BN, int kStages>
+void run_ring(const GemmParams& p, int b_layout, hipStream_t st)
+{
+    GemmParams q = p;
+    q.tiles_m = (p.m + BM - 1u) / BM;
+    q.tiles_n = (p.n + BN - 1u) / BN;
+    const uint32_t grid = (q.tiles_m * q.tiles_n + 7u) / 8u * 8u;
+    if (b_layout == 2) {
+        gemm_ring_kernel<BM, BN, kStages, 2><<<grid, kThreads, 0, st>>>(q);
+    } else if (b_layout == 1) {
+        gemm_ring_kernel<BM, BN, kStages, 1><<<grid, kThreads, 0, st>>>(q);
+    } else {
+        gemm_ring_kernel<BM, BN, kStages, 0><<<grid, kThreads, 0, st>>>(q);
+    }
+}
+
+}  // namespace
+
+// The tile of a call and its time with the quantiser in front, in us: 8.5, then rounds of the chip times K steps times a step's
+// time, which grows with the part f of the compute units that have a tile (the way to memory is shared).  Measured on 64 to 256 tiles at
+// k = 2048 to 11008, weights packed or as [n, k]: 64 x 64 0.225; 128 x 64 0.29 .. 0.415; 128 x 128 0.44 .. 0.62.  As
+// [k, n], whose rows a tile of 64 columns reads as half lines: 0.30; 0.36 .. 0.48; 0.48 .. 0.66.  (64 x 128 and 256 x 128 were ahead of these nowhere by
+// more than 8 %.)
+RingPlan gemm_ring_plan(uint32_t m, uint32_t n, uint32_t k, int b_layout)
+{
+    struct Shape {
+        uint32_t bm, bn;
+        double start, step[2], fill[2];  // [b_layout == 0]
+    };
+    static constexpr Shape kShapes[] = {{64, 64, 8.5, {0.225, 0.30}, {0.0, 0.0}},
+                                        {128, 64, 8.5, {0.26, 0.33}, {0.155, 0.15}},
+                                        {128, 128, 8.5, {0.38, 0.44}, {0.24, 0.22}}};
+    const uint32_t steps = (k + BK - 1u) / BK, cus = device_compute_units();
+    RingPlan best{0, 64, 64, 1e30};
+    for (int i = 0; i < 3; ++i) {
+        const Shape& s = kShapes[i];
+        const uint64_t tiles = static_cast<uint64_t>((m + s.bm - 1u) / s.bm) * ((n + s.bn - 1u) / s.bn);
+        const double step = s.step[b_layout == 0], fill = s.fill[b_layout == 0], rest = static_cast<double>(tiles % cus) / cus;
+        const double rounds = static_cast<double>(tiles / cus) * (step + fill) + (rest > 0.0 ? step + fill * rest : 0.0);
+        const double us = s.start + steps * rounds * (tiles > cus ? 1.05 : 1.0);
+        if (us < best.us) {
+            best = RingPlan{i, s.bm, s.bn, us};
+        }
+    }
+    return best;
+}
+
+int launch_gemm_ring(const GemmParams& p, int shape, int b_layout, hipStream_t st)
+{
+    if (plan_recording()) {
+        static constexpr uint32_t kTile[3][3] = {{64, 64, 8}, {128, 64, 6}, {128, 128, 4}};
+        const uint32_t bm = kTile[shape][0], bn = kTile[shape][1];
+        plan_note(ASCQ_MM_KERNEL_DMA_128, bm, bn, BK, ((p.m + bm - 1u) / bm * ((p.n + bn - 1u) / bn) + 7u) / 8u * 8u, 1,
+                  kTile[shape][2] * (bm + bn) * BK + bm * 4u, 0);
+        return ASCQ_OK;
+    }
+    switch (shape) {
+    case 0: run_ring<64, 64, 8>(p, b_layout, st); break;
+    case 1: run_ring<128, 64, 6>(p, b_layout, st); break;
+    default: run_ring<128, 128, 4>(p, b_layout, st); break;
+    }
+    return launch_status("ascq_matmul_w8a8 (ring)");
+}
+
+}  // namespace ascq

@@ -37,7 +37,8 @@ constexpr int BK = 128;
 
 // The forms of a tile: its matrix instruction (gemm_dma_form says which one runs where), and whether k may end inside a
 // step.  Looking for that step costs about 1 % (600 x 4096 x 4096 43.5 -> 43.9 us), so it is a form of its own.
-constexpr int k16 = 16, k32 = 32, k32Ragged = 33;
+// kRing: small tiles with a ring of stages (matmul_w8a8_ring.hip).
+constexpr int k16 = 16, k32 = 32, k32Ragged = 33, kRing = 64;
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* gptr_t;
@@ -160,6 +161,15 @@ __device__ __forceinline__ void gemm_dma_loop(uint32_t steps, bool active, char*
     }
 }
 
+// Where piece q of row kb of a [k][BN] B tile lies: at q ^ b_swizzle(kb).  It spreads the 8 rows of a transposing read over half of
+// the banks and, in the 16 x 16 forms, the rows 16 further, which are read beside them, over the other half.
+template <int BN, bool k16x16>
+__device__ __forceinline__ uint32_t b_swizzle(uint32_t kb)
+{
+    const uint32_t rows = BN == 256 ? 2u * (kb & 7u) : BN == 128 ? 2u * ((kb >> 1) & 3u) : 2u * ((kb >> 2) & 1u);
+    return rows ^ (k16x16 ? (kb >> 4) & 1u : 0u);
+}
+
 // The body of a tile on v_mfma_i32_16x16x64_i8, 16-bit outputs only.
 // wave, lane: of the workgroup; n0: first column; bases(step): where a K step's loads start; load(bases, u, stage): load u
 // of the wavefront's kBLoads + kALoads of a step (B, first half of A's rows, second half).
@@ -204,8 +214,7 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
         const uint32_t bsub = lc >> 1, psub = lc & 1u;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
-            const uint32_t swz = (BN == 256 ? 2u * bsub : 2u * (bsub >> 1)) ^ (lq & 1u);
-            b_base[j] = (16u * lq + bsub) * BN + (((4u * wn + j) ^ swz) << 4) + 8u * psub;
+            b_base[j] = (16u * lq + bsub) * BN + (((4u * wn + j) ^ b_swizzle<BN, true>(16u * lq + bsub)) << 4) + 8u * psub;
         }
     }
     i32x4 af[2][NH], bf[2][TJ];
@@ -514,6 +523,209 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     } else {
         run(OutTag<ASCQ_F16>{});
     }
+}
+
+// The body of a small tile: a ring of kStages LDS stages of a K step each, loads that are issued kStages - 1/2 steps ahead
+// (see matmul_w8a8_ring.hip).  load(step, u, stage): load u of the wavefront's kLoads of a step; past the end it brings zeros.
+template <int BM, int BN, int kB, int kStages, int kLoads, class Load>
+__device__ __forceinline__ void gemm_ring_body(const GemmParams& p, const TilePlace& at, uint32_t n0, uint32_t steps, uint32_t wave,
+                                               uint32_t lane, Load&& load, char* const (&L)[kStages], float* TS)
+{
+    constexpr bool kBT = kB == 1, kBP = kB == 2;
+    constexpr int TJ = BN == 64 ? 2 : 4;                       // 16 x 16 blocks per wavefront along N
+    constexpr int kWN = BN / 16 / TJ, kWM = 8 / kWN;           // wavefronts along N and M
+    constexpr int NA = BM / 16 / kWM;                          // blocks along M
+    static_assert(NA >= 1 && NA * 16 * kWM == BM && kWM * kWN == 8, "tile shape does not fit eight wavefronts");
+    const uint32_t wm = wave / kWN, wn = wave % kWN;
+    const uint32_t lc = lane & 15u, lq = lane >> 4;
+
+    i32x4 acc[NA][TJ];
+    static_for<NA * TJ>([&](auto c) {
+        i32x4& v = acc[decltype(c)::value / TJ][decltype(c)::value % TJ];
+        v = i32x4{0, 0, 0, 0};
+        asm volatile("" : "+v"(v));
+    });
+    uint32_t foff[2], b_base[TJ];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) foff[ks] = lc * 128u + (((4u * ks + lq) ^ (lc >> 1)) << 4);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+        // transposing reads: in 16 lanes, rows bsub of 8 and halves psub of the block's 16 columns
+        const uint32_t bsub = lc >> 1, psub = lc & 1u, row = 16u * lq + bsub;
+        b_base[j] = kBP ? wn * (TJ * 2048u) + lane * 16u : row * BN + (((static_cast<uint32_t>(TJ) * wn + j) ^ b_swizzle<BN, true>(row)) << 4) + 8u * psub;
+    }
+    i32x4 af[2][2][NA], bf[2][2][TJ];  // [set][half of the step]: a step's operands arrive while those of the one before are in use
+    i32x2_t blo;
+    constexpr int kBReads = (kBT || kBP) ? TJ : 2 * TJ, kReads = NA + kBReads;  // LDS reads of 64 k
+    auto read = [&](const char* S, int set, int r) __attribute__((always_inline)) {
+        const char* const Bs = S + BM * BK;
+        const int ks = r / kReads;
+        r %= kReads;
+        if (r < NA) {
+            af[set][ks][r] = *reinterpret_cast<const i32x4*>(S + (wm * NA + r) * 2048u + foff[ks]);
+            return;
+        }
+        r -= NA;
+        if constexpr (kBT) {
+            bf[set][ks][r] = *reinterpret_cast<const i32x4*>(Bs + (wn * TJ + r) * 2048u + foff[ks]);
+        } else if constexpr (kBP) {
+            bf[set][ks][r] = *reinterpret_cast<const i32x4*>(Bs + b_base[0] + r * 2048u + ks * 1024u);
+        } else {
+            const i32x2_t v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2_t)(Bs + b_base[r >> 1] + ks * (64 * BN) + (r & 1) * (8 * BN)));
+            if (r & 1) {
+                bf[set][ks][r >> 1] = i32x4{blo[0], blo[1], v[0], v[1]};
+            } else {
+                blo = v;
+            }
+        }
+    };
+    auto arrive = [&](auto left) __attribute__((always_inline)) {
+        constexpr int kLeft = decltype(left)::value;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kLeft & 15) | ((kLeft >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // (not __syncthreads(): its fence waits for every load)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // A step in stage X, the next one in Y.  Its operands are in registers or on their way there: behind the wait (they are there,
+    // the next step has landed, those behind it are on their way) and the barrier every wavefront has read the stage, which
+    // takes the step kStages ahead, and the next step's operands are read behind this one's matrix instructions, in the order written.
+    constexpr int kM = 2 * NA * TJ, kPer = (2 * kReads + kM - 1) / kM, kLoadPer = (kLoads + kM - 1) / kM;
+    auto step = [&](uint32_t s, char* X, const char* Y, auto set) __attribute__((always_inline)) {
+        constexpr int x = decltype(set)::value;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(foff[q]));
+#pragma unroll
+        for (int j = 0; j < (kBP ? 1 : TJ); ++j) asm volatile("" : "+v"(b_base[j]));
+        arrive(std::integral_constant<int, (kStages - 2) * kLoads>{});
+        static_for<kM>([&](auto nn) {
+            constexpr int n = decltype(nn)::value, ks = n / (NA * TJ), i = n / TJ % NA, j = n % TJ;
+            i32x4& c = acc[i][j];
+            asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(c) : "v"(af[x][ks][i]), "v"(bf[x][ks][j]));
+            static_for<kPer>([&](auto r) {
+                constexpr int m = n * kPer + decltype(r)::value;
+                if constexpr (m < 2 * kReads) read(Y, 1 - x, m);
+            });
+            static_for<kLoadPer>([&](auto r) {
+                constexpr int u = n * kLoadPer + decltype(r)::value;
+                if constexpr (u < kLoads) load(s + kStages, u, X);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    static_for<kStages>([&](auto st) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) load(decltype(st)::value, u, L[decltype(st)::value]);
+    });
+    arrive(std::integral_constant<int, (kStages - 1) * kLoads>{});
+#pragma unroll
+    for (int r = 0; r < 2 * kReads; ++r) read(L[0], 0, r);
+    constexpr int kGroup = kStages % 2 ? 2 * kStages : kStages;  // stages and sets
+    uint32_t s = 0;
+    for (; s + kGroup <= steps; s += kGroup) {
+        static_for<kGroup>([&](auto st) {
+            constexpr int i = decltype(st)::value;
+            step(s + i, L[i % kStages], L[(i + 1) % kStages], std::integral_constant<int, i % 2>{});
+        });
+    }
+    bool more = true;  // what is left of the last group (a step without a next one reads what nobody uses)
+    static_for<kGroup - 1>([&](auto st) {
+        constexpr int i = decltype(st)::value;
+        more = more && s + i < steps;
+        if (more) step(s + i, L[i % kStages], L[(i + 1) % kStages], std::integral_constant<int, i % 2>{});
+    });
+    // The last sums are on their way through the matrix pipe, which the compiler does not know; the loads past the end land
+    // before the LDS is given back.
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    static_for<NA * TJ>([&](auto c) {
+        i32x4& v = acc[decltype(c)::value / TJ][decltype(c)::value % TJ];
+        asm volatile("" : "+v"(v));
+    });
+
+    // ---- epilogue: register r of lane l in a 16 x 16 block is row 4 (l / 16) + r, column l % 16
+    const EpiParams& e = p.epi;
+    const uint32_t N = p.n, colw = n0 + wn * (TJ * 16u);
+    ChannelQ q[TJ];
+    float bias_post[TJ];
+    int32_t bias_pre[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+        const uint32_t col = colw + j * 16u + lc;
+        q[j] = ChannelQ{1.0f, 0, 1};
+        bias_post[j] = 0.0f;
+        bias_pre[j] = 0;
+        if (col < N) {
+            q[j] = load_channel_q(e, at.chan_off + col);
+            bias_post[j] = load_bias_post(e, at.chan_off + col);
+            if (e.bias_kind == ASCQ_MM_BIAS_I32_PRE) {
+                bias_pre[j] = static_cast<const int32_t*>(e.bias)[at.chan_off + col];
+            }
+        }
+        asm volatile("" : "+v"(q[j].s), "+v"(bias_post[j]), "+v"(bias_pre[j]));  // (waited for once, not at every store)
+    }
+    bool shifts = false;  // quant words that shift the accumulator first (rare): element by element
+    if (e.scale_format == ASCQ_MM_SCALE_U64) {
+        int any = 0;
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) any |= q[j].ctl;
+        shifts = __builtin_amdgcn_ballot_w64((any & 2) != 0) != 0;
+    }
+    const bool half_out = e.quant_mode != ASCQ_MM_QUANT_NONE && (e.out_dtype == ASCQ_BF16 || e.out_dtype == ASCQ_F16);
+    if (half_out && !shifts && e.activation != ASCQ_MM_ACT_SWIGLU) {
+        const bool b0 = (lane & 1u) != 0, b1 = (lane & 2u) != 0, post = e.bias_kind >= ASCQ_MM_BIAS_F32_POST;
+        const bool gelu = e.activation == ASCQ_MM_ACT_FASTER_GELU, bf16 = e.out_dtype == ASCQ_BF16;
+        static_for<NA>([&](auto ii) {
+            constexpr int i = decltype(ii)::value;
+            const uint32_t lbase = (wm * NA + i) * 16u + 4u * lq;
+            const f32x4 tok4 = *reinterpret_cast<const f32x4*>(&TS[lbase]);
+            static_for<4>([&](auto rr) {
+                constexpr int r = decltype(rr)::value;
+                const uint32_t row = at.row0 + lbase + r;
+                uint32_t h[TJ];
+                static_for<TJ>([&](auto jj) {
+                    constexpr int j = decltype(jj)::value;
+                    float v = static_cast<float>(acc[i][j][r] + bias_pre[j]) * q[j].s;
+                    v = v * tok4[r];  // 1.0f without a token scale: an exact identity
+                    v = post ? v + bias_post[j] : v;
+                    v = gelu ? faster_gelu(v) : v;
+                    h[j] = bf16 ? to_bits16<ASCQ_BF16>(v) : to_bits16<ASCQ_F16>(v);
+                });
+                uint16_t* const out = static_cast<uint16_t*>(e.c) + static_cast<size_t>(row) * e.ldc;
+                if constexpr (TJ == 4) {
+                    // a 4 x 4 transposition inside each four neighbouring lanes (see gemm_dma_body16): 8-byte stores, whole lines
+                    const uint32_t col = colw + 16u * (lane & 3u) + (lc & 12u);
+                    const uint32_t give = b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16);
+                    const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+                    const uint32_t lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
+                    const uint32_t hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
+                    const uint32_t got2 = static_cast<uint32_t>(
+                        __builtin_amdgcn_mov_dpp(static_cast<int>(b1 ? lo : hi), 0x4E, 0xF, 0xF, true));  // lane ^ 2
+                    if (row < at.row_end && col < N) {
+                        __builtin_nontemporal_store(b1 ? u32x2{got2, hi} : u32x2{lo, got2}, reinterpret_cast<u32x2*>(out + col));
+                    }
+                } else {
+                    // after one swap the even lane holds two adjacent columns of the first block, the odd lane two of the second
+                    const uint32_t col = b0 ? colw + 16u + lc - 1u : colw + lc;
+                    const uint32_t got = static_cast<uint32_t>(
+                        __builtin_amdgcn_mov_dpp(static_cast<int>(b0 ? h[0] : h[1]), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+                    if (row < at.row_end && col < N) {
+                        __builtin_nontemporal_store(b0 ? got | (h[1] << 16) : h[0] | (got << 16), reinterpret_cast<uint32_t*>(out + col));
+                    }
+                }
+            });
+        });
+        return;
+    }
+    static_for<NA * TJ>([&](auto c) {
+        constexpr int i = decltype(c)::value / TJ, j = decltype(c)::value % TJ;
+        const uint32_t lbase = (wm * NA + i) * 16u + 4u * lq, col = colw + j * 16u + lc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (at.row0 + lbase + r < at.row_end && col < N) {
+                epilogue_store_lanes(e, at.row0 + lbase + r, col, acc[i][j][r] + bias_pre[j], q[j], TS[lbase + r], bias_post[j]);
+            }
+        }
+    });
 }
 
 // The body of a tile on v_mfma_i32_32x32x32_i8, every output.
@@ -834,9 +1046,9 @@ __device__ __forceinline__ void gemm_dma_body32(const GemmParams& p, const TileP
 // k is a multiple of BK, with k32Ragged of 16 (the pieces of a last, partial step that lie past k arrive as zeros).  With kB = 0 and an n
 // that is no multiple of 16 the last tile is moved left until it ends at n (n >= BN then): the columns it shares with
 // its neighbour are computed twice, with the same values.
-template <int BM, int BN, bool kSplitK, bool kGrouped, int kB, int kForm>
-__device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const TilePlace& at, uint32_t bidy, const Stage& S0,
-                                                 const Stage& S1, float* TS)
+// stages: S0, S1 (kRing: the array of the ring's stages)
+template <int BM, int BN, bool kSplitK, bool kGrouped, int kB, int kForm, class... Stages>
+__device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const TilePlace& at, uint32_t bidy, float* TS, const Stages&... stages)
 {
     constexpr bool kBT = kB == 1, kBP = kB == 2;
     constexpr int kPieces = BN / 16;        // 16-byte pieces per B row
@@ -899,10 +1111,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
             boff[u] = (col - n0) * K + 16u * line_piece(s);
             continue;
         }
-        // row kb = s / kPieces; the swizzle spreads the 8 rows of a transposing read over half of the banks and, in the
-        // 16 x 16 form, the rows 16 further, which are read beside them, over the other half
-        const uint32_t kb = s / kPieces;
-        const uint32_t q = (s % kPieces) ^ (BN == 256 ? 2u * (kb & 7u) : 2u * ((kb >> 1) & 3u)) ^ (kForm == k16 ? (kb >> 4) & 1u : 0u);
+        const uint32_t kb = s / kPieces, q = (s % kPieces) ^ b_swizzle<BN, kForm == k16 || kForm == kRing>(kb);
         uint32_t col = n0 + 16u * q;
         col = col + 16u <= N ? col : N - 16u;      // columns past the end are never stored
         // fractal B: panels of 32 columns, each a contiguous row-major [K][32] block
@@ -910,7 +1119,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     }
     const uint32_t ldb = kBT ? 1u : kBP ? 16u : p.b_nz ? 32u : N;  // bytes from one k to the next
     // K range of this workgroup, in steps of BK
-    const uint32_t all_steps = kForm == k32Ragged ? (K + BK - 1u) / BK : K / BK;
+    const uint32_t all_steps = kForm == k32Ragged || kForm == kRing ? (K + BK - 1u) / BK : K / BK;
     uint32_t s_begin = 0, steps = all_steps;
     if constexpr (kSplitK) {
         s_begin = steps * bidy / p.k_splits;
@@ -986,9 +1195,30 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
                 __builtin_amdgcn_global_load_lds((gptr_t)(from.a + aoff[v]), (lds_ptr_t)(S.a[v / kPart] + (wave * kPart + v % kPart) * 1024), 16, 0, 0);
             }
         };
-        gemm_dma_body16<BM, BN, kGrouped, kB, kAInstr, kBInstr>(p, at, n0, steps, wave, lane, bases, load, S0, S1, TS);
+        gemm_dma_body16<BM, BN, kGrouped, kB, kAInstr, kBInstr>(p, at, n0, steps, wave, lane, bases, load, stages..., TS);
+    } else if constexpr (kForm == kRing) {
+        auto load = [&](uint32_t step, int u, char* S) __attribute__((always_inline)) {
+            // how much of the row's k is left from here on, nothing past the last step; a piece past it brings zeros
+            const uint32_t at_k = step < steps ? step : 0u, left = step < steps ? K - step * BK : 0u;
+            if (u < kAInstr) {
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(uniform(Abase + at_k * BK)), 0, 0x7FFFFF00, 0x00020000);
+                const uint32_t off = 16u * line_piece(a_slot(u)) < left ? aoff[u] : kPastEnd;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(S + (wave * kAInstr + u) * 1024), 16, off, 0, 0, 0);
+            } else {
+                const int v = u - kAInstr;
+                const __amdgpu_buffer_rsrc_t r =
+                    __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(uniform(Bbase + static_cast<size_t>(at_k) * BK * ldb)), 0, 0x7FFFFF00, 0x00020000);
+                const uint32_t k0 = kBT ? 16u * line_piece(b_slot(v)) : kBP ? ((wave * kBInstr + v) & 1u) * 64u : b_slot(v) / kPieces;
+                const uint32_t off = k0 < left ? boff[v] : kPastEnd;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(S + BM * BK + (wave * kBInstr + v) * 1024), 16, off, 0, 0, 0);
+            }
+        };
+        gemm_ring_body<BM, BN, kB, (sizeof(Stages) + ...) / sizeof(char*), kAInstr + kBInstr>(p, at, n0, steps, wave, lane, load, stages..., TS);
     } else {
-        gemm_dma_body32<BM, BN, kSplitK, kGrouped, kB>(p, at, n0, steps, bidy, wave, lane, issue, S0.a[0], S0.b, S1.a[0], S1.b, TS);
+        auto run = [&](const Stage& S0, const Stage& S1) __attribute__((always_inline)) {
+            gemm_dma_body32<BM, BN, kSplitK, kGrouped, kB>(p, at, n0, steps, bidy, wave, lane, issue, S0.a[0], S0.b, S1.a[0], S1.b, TS);
+        };
+        run(stages...);
     }
 }
 
@@ -1022,7 +1252,7 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmParams& p, uint32_t col_
     uint32_t ms, tn;
     band_order(t, p.tiles_m, p.tiles_n, ms, tn);
     const TilePlace at{ms * BM, p.m, col_begin + tn * BN, p.b, 0};
-    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, S0, S1, TS);
+    gemm_dma_tile_at<BM, BN, kSplitK, false, kB, kForm>(p, at, bidy, TS, S0, S1);
 }
 
 // The LDS stages S0 and S1 of a kernel (an array that nothing reads takes no space).

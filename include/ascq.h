@@ -421,7 +421,8 @@ typedef enum ascq_mm_kernel {
                                         sums, the epilogue) */
     ASCQ_MM_KERNEL_STREAM = 1,       /* few rows: weight streams, one per SIMD, then a kernel that adds their pieces */
     ASCQ_MM_KERNEL_DMA_128 = 2,      /* m <= 512, or few tiles: 128 x 128 direct-to-LDS tiles, K split over workgroups
-                                        when a workspace is given (k_splits > 1: a second kernel adds the partial tiles) */
+                                        when a workspace is given (k_splits > 1: a second kernel adds the partial tiles),
+                                        or 64 x 64 tiles with a ring of stages, unsplit */
     ASCQ_MM_KERNEL_DMA_256 = 3,      /* 256 x 256 direct-to-LDS tiles; a last partial round of the chip may be run
                                         by further workgroups of the same launch with 256 x narrow_tile_n tiles */
     ASCQ_MM_KERNEL_STAGED = 4        /* register-staged tiles: n not a multiple of 8 ([k, n]: of 16 below 256), and a

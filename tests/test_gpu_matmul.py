@@ -1335,6 +1335,43 @@ def test_linear_w8a8_dynamic_packed_split_over_k(m, k, n):
     assert np.array_equal(bits(c), orc.matmul_w8a8(d, q, w, bias, cs, ts))
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 16, 264), (65, 144, 520), (130, 400, 1032), (200, 1040, 264), (100, 1152, 1000), (97, 1664, 256), (130, 2192, 272),
+                                   (300, 640, 4400), (290, 1136, 4408), (600, 384, 6400), (520, 1744, 6008)])
+@pytest.mark.parametrize("act", [abi.MM_ACT_NONE, abi.MM_ACT_FASTER_GELU, abi.MM_ACT_SWIGLU])
+def test_linear_w8a8_small_tiles_with_a_ring_of_stages(m, k, n, act):
+    """The linears of medium size, all weight layouts: tiles of 64 x 64, 128 x 64 (from 300 x 640 x 4400 on) and 128 x 128
+    (from 600 x 384 x 6400 on), one K step to eighteen (fewer and more than the ring has stages, whole groups of them and
+    every remainder), a last K step of 16 to 112, rows and columns that end inside a tile, a last [k, n] tile moved left."""
+    announce("ring", m, k, n, act)
+    rng = np.random.default_rng(m + k + n)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    w = rand_i8(rng, (k, n))
+    cs = rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    q, ts = orc.dynamic_quant_per_token(abi.BF16, bits(x))
+    sums = (q.astype(np.float64) @ w.astype(np.float64)).astype(np.int32)      # exact
+    v = sums.astype(np.float32) * cs * ts[:, None] + bias                      # one rounding per step, like the epilogue
+    forms = [("kn", to_dev(w)), ("nk", to_dev(np.ascontiguousarray(w.T)))]
+    if k % 64 == 0:
+        forms.append(("packed", ops.pack_weight_w8(to_dev(w), k, n)))
+    for out in (torch.bfloat16, torch.float16, torch.float32):
+        for layout, wd in forms:
+            c = torch.zeros((m, n // 2 if act == abi.MM_ACT_SWIGLU else n), dtype=out, device=DEV)
+            if layout == "packed":
+                ops.linear_w8a8_dynamic_packed(c, x, wd, n, to_dev(cs), to_dev(bias), act)
+            else:
+                ops.linear_w8a8_dynamic(c, x, wd, to_dev(cs), to_dev(bias), act, layout == "nk")
+            if act == abi.MM_ACT_NONE:
+                assert torch.equal(c.cpu(), torch.from_numpy(v).to(out)), layout
+                continue
+            # the activations' exponentials (of arguments up to 2^5) and quotients are approximations of about one fp32 ulp
+            t = v.astype(np.float64)
+            want = t / (1.0 + np.exp(-1.702 * t)) if act == abi.MM_ACT_FASTER_GELU else t[:, 0::2] * t[:, 1::2] / (1.0 + np.exp(-t[:, 1::2]))
+            ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[out]
+            got = c.double().cpu().numpy()
+            assert np.all(np.abs(got - want) <= (ulp + 2.0 ** -18) * np.abs(want) + 1e-6), layout
+
+
 @pytest.mark.parametrize("m,kernel", [(1, abi.MM_KERNEL_STREAM), (100, abi.MM_KERNEL_DMA_128),
                                       (700, abi.MM_KERNEL_DMA_256)])
 def test_matmul_plan_then_call(m, kernel):
