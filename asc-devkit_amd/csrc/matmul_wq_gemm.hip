@@ -78,8 +78,13 @@ __device__ __forceinline__ uint32_t pair_of_i4(uint32_t q, int c, f16x2 sc, f16x
 
 // One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
 // wavefront owns BM / kWM rows by 64 columns.
+struct WqStage {
+    char* a[2];  // the first and the second half of every wavefront's rows: distinct arrays, like the stages
+    char* b;
+};
+
 template <int BM, int BN, bool kInt4, bool kOff>
-__device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32_t n0, char* A0, char* A1, char* B0, char* B1)
+__device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32_t n0, const WqStage& S0, const WqStage& S1)
 {
     constexpr int kWN = BN / 64, kWM = 8 / kWN, NA = BM / 16 / kWM, NH = NA / 2, TJ = 4;
     constexpr int kAInstr = BM * 128 / 1024 / 8;           // direct-to-LDS instructions per wavefront and step
@@ -89,29 +94,34 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / kWN, wn = wave % kWN;
 
-    // ---- A: lane owns LDS slot (instr * 64 + lane) of 16 bytes: line slot / 8, piece position ^ ((line / 2) % 8)
+    // ---- A: lane owns LDS slot (instr * 64 + lane) of 16 bytes of a half's array: line slot / 8, piece position ^ ((line / 2) % 8);
+    // line r is row r % kRows of that half of wavefront row r / kRows
+    constexpr int kHalf = kAInstr / 2;                     // instructions per half
+    constexpr uint32_t kRows = NH * 16u;
+    static_assert(kAInstr % 2 == 0, "the halves are whole instructions");
     const uint32_t row_bytes = p.k * 2u;
     uint32_t aoff[kAInstr];
 #pragma unroll
     for (int u = 0; u < kAInstr; ++u) {
-        const uint32_t s = (wave * kAInstr + u) * 64u + lane, r = s >> 3;
+        const uint32_t s = (wave * kHalf + u % kHalf) * 64u + lane, line = s >> 3;
+        const uint32_t r = (line / kRows * 2u + u / kHalf) * kRows + line % kRows;
         const uint32_t row = row0 + r < p.m ? r : p.m - 1u - row0;  // rows past the end are never stored
-        aoff[u] = row * row_bytes + (((s & 7u) ^ ((r >> 1) & 7u)) << 4);
+        aoff[u] = row * row_bytes + (((s & 7u) ^ ((line >> 1) & 7u)) << 4);
     }
     const char* Abase = reinterpret_cast<const char*>(p.x) + static_cast<size_t>(row0) * row_bytes;
-    auto issue = [&](uint32_t step, char* As) __attribute__((always_inline)) {
-        // a scalar base plus the lane's 32-bit offset, which the load instruction adds itself
-        const uint64_t v = reinterpret_cast<uint64_t>(Abase + step * 128u);
+    const uint32_t last = p.k / kBK - 1u;
+    // a scalar base plus the lane's 32-bit offset, which the load instruction adds itself; past the end the last step's, into
+    // a stage nobody reads
+    auto a_base = [&](uint32_t step) __attribute__((always_inline)) {
+        const uint64_t v = reinterpret_cast<uint64_t>(Abase + (step < last ? step : last) * 128u);
         uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
         uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
         asm volatile("" : "+s"(lo), "+s"(hi));
-        const char* ab = reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
-#pragma unroll
-        for (int u = 0; u < kAInstr; ++u) asm volatile("" : "+v"(aoff[u]));
-#pragma unroll
-        for (int u = 0; u < kAInstr; ++u) {
-            __builtin_amdgcn_global_load_lds((gptr_t)(ab + aoff[u]), (lds_ptr_t)(As + (wave * kAInstr + u) * 1024u), 16, 0, 0);
-        }
+        return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
+    };
+    auto load_rows = [&](const char* base, int u, const WqStage& S) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(aoff[u]));
+        __builtin_amdgcn_global_load_lds((gptr_t)(base + aoff[u]), (lds_ptr_t)(S.a[u / kHalf] + (wave * kHalf + u % kHalf) * 1024u), 16, 0, 0);
     };
 
     // ---- B: the thread's column of the tile and its first piece (of 8 weights) in the column's line
@@ -150,29 +160,31 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
         ro = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kOff ? p.offset : p.scale), 0, bytes, 0x00020000);
         poff = gcol * 2u + (p.gs_shift == 0 ? (bpiece >> 2) * p.n * 2u : 0u);
     }
+    // Raw bytes of a step: two parts of two pieces each, fetched apart (BN = 128: one part).
+    constexpr int kFetches = kParts / 2;
     struct Raw {
-        u32x4 b[kInt4 ? 1 : kParts / 2];                   // (BN = 128, int4: half of it)
+        u32x4 b[kInt4 ? 1 : kFetches];
         uint32_t sc, of;
     };
-    const uint32_t last = p.k / kBK - 1u;
-    auto fetch = [&](Raw& raw, uint32_t step) __attribute__((always_inline)) {
+    // part `which`: its weights, with the last part the parameters
+    constexpr int kPartLoads = 1, kParamLoads = kInt4 ? (kOff ? 2 : 1) : 0;
+    auto fetch = [&](Raw& raw, uint32_t step, int which) __attribute__((always_inline)) {
         step = step < last ? step : last;                  // past the end: the last step's, into a stage nobody reads
         const uint32_t at = kInt4 ? step * 512u : step * kBK;
-        if constexpr (kInt4 && kParts == 2) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rw, boff, at, 0);
-            raw.b[0][0] = v[0];
-            raw.b[0][1] = v[1];
+        if constexpr (kInt4) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rw, boff + 8u * which, at, 0);
+            raw.b[0][2 * which] = v[0];
+            raw.b[0][2 * which + 1] = v[1];
         } else {
-#pragma unroll
-            for (int i = 0; i < static_cast<int>(sizeof(raw.b) / 16u); ++i) {
-                raw.b[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, boff + 16u * i, at, 0));
-            }
+            raw.b[which] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, boff + 16u * which, at, 0));
         }
         if constexpr (kInt4) {
-            // the group of 32 k 2 step + (0 or 1); the lane's half matters for groups of 32 only
-            const uint32_t pat = ((2u * step) >> p.gs_shift) * p.n * 2u;
-            raw.sc = __builtin_amdgcn_raw_buffer_load_b16(rs, poff, pat, 0);
-            raw.of = kOff ? __builtin_amdgcn_raw_buffer_load_b16(ro, poff, pat, 0) : 0u;
+            if (which == kFetches - 1) {
+                // the group of 32 k 2 step + (0 or 1); the lane's half matters for groups of 32 only
+                const uint32_t pat = ((2u * step) >> p.gs_shift) * p.n * 2u;
+                raw.sc = __builtin_amdgcn_raw_buffer_load_b16(rs, poff, pat, 0);
+                raw.of = kOff ? __builtin_amdgcn_raw_buffer_load_b16(ro, poff, pat, 0) : 0u;
+            }
         }
     };
     const uint32_t bline = bcol * 128u, bswz = (bcol >> 1) & 7u;
@@ -201,31 +213,32 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
         }
 
     // ---- operands: lane l holds line l % 16 of a block of 16 and the 8 k of piece 4 ks + l / 16.  A step is four
-    // quarters: quarter q multiplies half q % 2 of the wavefront's rows with the 32 k of sub-step ks = q / 2.
+    // quarters: quarter q multiplies half q / 2 of the wavefront's rows with the 32 k of sub-step ks = q % 2.
     const uint32_t lc = lane & 15u, lq = lane >> 4;
     uint32_t foff[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) foff[ks] = lc * 128u + (((4u * ks + lq) ^ (lc >> 1)) << 4);
     f16x8 af[2][NH], bf[2][TJ];
-    auto load_a = [&](const char* As, int q, int i) __attribute__((always_inline)) {
-        af[q & 1][i] = *reinterpret_cast<const f16x8*>(As + wm * (NA * 2048u) + ((q & 1) * NH + i) * 2048u + foff[q >> 1]);
+    auto load_a = [&](const WqStage& S, int q, int i) __attribute__((always_inline)) {
+        af[q & 1][i] = *reinterpret_cast<const f16x8*>(S.a[q >> 1] + (wm * NH + i) * 2048u + foff[q & 1]);
     };
-    auto load_b = [&](const char* Bs, int ks, int j) __attribute__((always_inline)) {
-        bf[ks][j] = *reinterpret_cast<const f16x8*>(Bs + wn * 8192u + j * 2048u + foff[ks]);
+    auto load_b = [&](const WqStage& S, int ks, int j) __attribute__((always_inline)) {
+        bf[ks][j] = *reinterpret_cast<const f16x8*>(S.b + wn * 8192u + j * 2048u + foff[ks]);
     };
     // Matrix instruction number n of quarter q.  Written as an instruction that accumulates in place: left to itself the
     // compiler gave it another destination than its addend and moved accumulators about, spilling some.  (Its operands
     // come from LDS reads, which the compiler waits for; no vector instruction touches them or the sums in the loop.)
     auto mfma = [&](int q, int n) __attribute__((always_inline)) {
-        f32x4& c = acc[(q & 1) * NH + n / TJ][n % TJ];
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(af[q & 1][n / TJ]), "v"(bf[q >> 1][n % TJ]));
+        f32x4& c = acc[(q >> 1) * NH + n / TJ][n % TJ];
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(af[q & 1][n / TJ]), "v"(bf[q & 1][n % TJ]));
     };
-    // One quarter: its NH * TJ matrix instructions, the LDS reads `read(r)`, r < kReads, one behind each of the first, and
-    // a piece of the next step's weights de-quantised pair by pair behind four later ones.  The order is the one written.
+    // One quarter: its NH * TJ matrix instructions, the LDS reads `read(r)`, r < kReads, one behind each of the first, loads
+    // `load(u)`, u < kLoads, behind the odd ones, and a piece of weights de-quantised pair by pair behind four later ones.
+    // The order is the one written.
     constexpr int kM = NH * TJ;
-    auto quarter = [&](auto qq, auto reads, auto&& read, auto part, const Raw& next, char* Bn) __attribute__((always_inline)) {
-        constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value, kPart = decltype(part)::value;
-        constexpr int kPer = (kReads + kM - 1) / kM;
+    auto quarter = [&](auto qq, auto reads, auto&& read, auto part, const Raw& raw, char* Bs, auto loads, auto&& load) __attribute__((always_inline)) {
+        constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value, kPart = decltype(part)::value, kLoads = decltype(loads)::value;
+        constexpr int kPer = (kReads + kM - 1) / kM, kLoadPer = (2 * kLoads + kM - 1) / kM;
         wq_for<kM>([&](auto nn) {
             constexpr int n = decltype(nn)::value;
             mfma(q, n);
@@ -233,90 +246,136 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
                 constexpr int i = n * kPer + decltype(r)::value;
                 if constexpr (i < kReads) read(std::integral_constant<int, i>{});
             });
+            if constexpr (n % 2 == 1) {
+                wq_for<kLoadPer>([&](auto r) {
+                    constexpr int u = n / 2 * kLoadPer + decltype(r)::value;
+                    if constexpr (u < kLoads) load(u);
+                });
+            }
             if constexpr (kPart >= 0) {
                 // pairs behind instructions kM - 5 .. kM - 2 (of at least 4)
                 constexpr int first = kM >= 8 ? kM - 5 : 0;
-                if constexpr (n >= first && n < first + 4) dequant_pair(next, kPart, n - first);
-                if constexpr (n == first + 3) write_piece(Bn, kPart);
+                if constexpr (n >= first && n < first + 4) dequant_pair(raw, kPart, n - first);
+                if constexpr (n == first + 3) write_piece(Bs, kPart);
             }
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    // Quarters 0 - 2 of step s in stage (A, B), whose first operands are in registers; pieces 1 .. of step s + 1 go
-    // into stage Bn (kParts == 2: the second of two behind quarter 1).
-    auto head = [&](const char* As, const char* Bs, const Raw& next, char* Bn) __attribute__((always_inline)) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(foff[q]));
-        wq_for<3>([&](auto qq) {
-            constexpr int q = decltype(qq)::value;
-            constexpr int part = kParts == 4 ? q + 1 : q == 1 ? 1 : -1;
-            quarter(qq, std::integral_constant<int, NH + (q < 2 ? 2 : 0)>{}, [&](auto r) __attribute__((always_inline)) {
-                constexpr int i = decltype(r)::value;
-                if constexpr (i < NH) {
-                    load_a(As, q + 1, i);
-                } else {
-                    load_b(Bs, 1, 2 * q + i - NH);
-                }
-            }, std::integral_constant<int, part>{}, next, Bn);
-        });
-    };
-    // Behind the barrier: the last quarter's instructions, the first operands of step s + 1 and piece 0 of step s + 2
-    // (into this step's stage, which everyone has left).
-    auto first_operands = [&](const char* An, const char* Bn, int i) __attribute__((always_inline)) {
+    auto first_operands = [&](const WqStage& S, int i) __attribute__((always_inline)) {
         if (i == 0 || i > NH) {
-            load_b(Bn, 0, i == 0 ? 0 : i - NH);
+            load_b(S, 0, i == 0 ? 0 : i - NH);
         } else {
-            load_a(An, 0, i - 1);
+            load_a(S, 0, i - 1);
         }
     };
-    auto tail = [&](const char* An, const char* Bn, const Raw& next2, char* Bs) __attribute__((always_inline)) {
-        quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
-            first_operands(An, Bn, decltype(r)::value);
-        }, std::integral_constant<int, 0>{}, next2, Bs);
+    auto arrive = [&](auto left) __attribute__((always_inline)) {
+        constexpr int kLeft = decltype(left)::value;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kLeft & 15) | ((kLeft >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // (not __syncthreads(): its fence waits for every load)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
     };
-    auto clamp = [&](uint32_t step) { return step < last ? step : last; };
+    // Step s in stage X, step s + 1 in Y; `next` holds the raw bytes of step s + 1, `next2` those of s + 2.  When quarter 1
+    // begins, every wavefront has read X's weights and the first half of its rows, when quarter 3 begins, the second half,
+    // and Y's weights are written: a barrier there, and what was freed takes the loads of step s + 2, what was used up of
+    // the raw bytes those of step s + 3.  So the loads have one and a half steps to arrive (int4's parameters one), where one wait for all of
+    // them at a step's end left them one.  The waits count the loads behind the ones that are needed: before quarter 1 the second
+    // half of this step's rows and the last raw bytes of step s + 1 (behind them all of a step's loads), before quarter 3 the
+    // first half of the next step's rows and the first raw bytes of step s + 2, with int4 its parameters.  (Without a count of its own
+    // for the raw bytes the compiler waits for everything where they cross the loop's end.)
+    // (BN = 128, two small workgroups on a unit: a quarter is four matrix instructions, and one barrier, before quarter 3, is better: 100 x
+    // 4096 x 4096 int4 40.0 us, 42.4 with two.)
+    constexpr bool kMid = kFetches == 2;
+    constexpr int kPartAll = kFetches * kPartLoads + kParamLoads, kLate = kPartLoads + kParamLoads;  // fetches of a step; behind quarter 3
+    constexpr int kEarly = kPartAll - kLate, kRowsLate = kMid ? kHalf : kAInstr;                      // fetches, rows behind quarter 1 / 3
+    auto step = [&](uint32_t s, const WqStage& X, const WqStage& Y, Raw& next, Raw& next2, auto steady) __attribute__((always_inline)) {
+        constexpr bool kSteady = decltype(steady)::value;
+        constexpr std::integral_constant<int, kSteady && kMid ? kHalf + kEarly : 0> early{};
+        constexpr std::integral_constant<int, kSteady ? kRowsLate + 1 : 0> late{};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(foff[q]));
+        const char* const base = a_base(s + 2u);
+        quarter(std::integral_constant<int, 0>{}, std::integral_constant<int, TJ + NH>{}, [&](auto r) __attribute__((always_inline)) {
+            constexpr int i = decltype(r)::value;
+            if constexpr (i < TJ) {
+                load_b(X, 1, i);
+            } else {
+                load_a(X, 1, i - TJ);
+            }
+        }, std::integral_constant<int, kSteady && kParts == 4 ? 1 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
+        if constexpr (kMid) arrive(std::integral_constant<int, kSteady ? kAInstr + kPartAll : 0>{});
+        quarter(std::integral_constant<int, 1>{}, std::integral_constant<int, NH>{}, [&](auto r) __attribute__((always_inline)) {
+            load_a(X, 2, decltype(r)::value);
+        }, std::integral_constant<int, !kSteady ? -1 : kParts == 4 ? 2 : 1>{}, next, Y.b, early, [&](int u) __attribute__((always_inline)) {
+            if (u < kHalf) {
+                load_rows(base, u, X);
+            } else {
+                fetch(next, s + 3u, 0);  // (its first part was used up by quarter 0)
+            }
+        });
+        quarter(std::integral_constant<int, 2>{}, std::integral_constant<int, NH>{}, [&](auto r) __attribute__((always_inline)) {
+            load_a(X, 3, decltype(r)::value);
+        }, std::integral_constant<int, kSteady && kParts == 4 ? 3 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
+        if constexpr (kSteady) {
+            arrive(std::integral_constant<int, !kMid ? 0 : kInt4 ? kHalf + kEarly : kAInstr + kPartAll>{});
+            quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
+                first_operands(Y, decltype(r)::value);
+            }, std::integral_constant<int, 0>{}, next2, X.b, late, [&](int u) __attribute__((always_inline)) {
+                if (u < kRowsLate) {
+                    load_rows(base, kAInstr - kRowsLate + u, X);
+                } else {
+                    fetch(next, s + 3u, kFetches - 1);
+                }
+            });
+        } else {
+            wq_for<kM>([&](auto n) { mfma(3, decltype(n)::value); });
+        }
+    };
 
+    // The loads in the order in which the loop would have issued them.
     Raw r0, r1;
-    issue(0, A0);
-    fetch(r0, 0);
-    fetch(r1, 1);
 #pragma unroll
-    for (int q = 0; q < kParts; ++q) {
+    for (int w = 0; w < kFetches; ++w) fetch(r0, 0, w);
+    auto prologue_rows = [&](uint32_t st, int h, const WqStage& S) __attribute__((always_inline)) {
+        const char* const base = a_base(st);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) dequant_pair(r0, q, c);
-        write_piece(B0, q);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    issue(clamp(1), A1);
-    fetch(r0, 2);
+        for (int u = 0; u < kHalf; ++u) load_rows(base, h * kHalf + u, S);
+    };
+    prologue_rows(0, 0, S0);
+    if constexpr (kEarly != 0) fetch(r1, 1, 0);
+    prologue_rows(0, 1, S0);
+    fetch(r1, 1, kFetches - 1);
+    wq_for<kParts>([&](auto q) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) dequant_pair(r0, decltype(q)::value, c);
+        write_piece(S0.b, decltype(q)::value);
+    });
+    prologue_rows(1, 0, S1);
+    if constexpr (kEarly != 0) fetch(r0, 2, 0);
+    arrive(std::integral_constant<int, kMid ? kEarly + kHalf + kLate + kHalf + kEarly : kHalf>{});
+    prologue_rows(1, 1, S1);
+    fetch(r0, 2, kFetches - 1);
 #pragma unroll
     for (int c = 0; c < 4; ++c) dequant_pair(r1, 0, c);
-    write_piece(B1, 0);
+    write_piece(S1.b, 0);
 #pragma unroll
-    for (int i = 0; i < NH + TJ; ++i) first_operands(A0, B0, i);
-    // At the top of step s (stage x, other stage y): its first operands are in registers, piece 0 of step s + 1 is in
-    // y, the rest of it in raw set (s + 1) % 2, step s + 2's raw bytes are on their way into set s % 2.
+    for (int i = 0; i < NH + TJ; ++i) first_operands(S0, i);
+    // At the top of step s (stage X, other stage Y): its first operands are in registers, piece 0 of step s + 1 is in Y, the
+    // rest of it in raw set (s + 1) % 2, step s + 2's raw bytes are on their way into set s % 2.
     const uint32_t steps = last + 1u;
     uint32_t s = 0;
-    for (; s + 1u < steps; s += 2u) {
-        head(A0, B0, r1, B1);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        issue(clamp(s + 2u), A0);
-        fetch(r1, s + 3u);
-        tail(A1, B1, r0, B0);
-        head(A1, B1, r0, B0);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        issue(clamp(s + 3u), A1);
-        fetch(r0, s + 4u);
-        tail(A0, B0, r1, B1);
+    for (; s + 2u < steps; s += 2u) {
+        step(s, S0, S1, r1, r0, std::true_type{});
+        step(s + 1u, S1, S0, r0, r1, std::true_type{});
     }
-    if (s < steps) {  // an odd last step
-        head(A0, B0, r1, B1);
-#pragma unroll
-        for (int n = 0; n < kM; ++n) mfma(3, n);
+    if (s + 1u < steps) {
+        step(s, S0, S1, r1, r0, std::true_type{});
+    }
+    {
+        const bool odd = (steps & 1u) != 0;
+        const WqStage X{{odd ? S0.a[0] : S1.a[0], odd ? S0.a[1] : S1.a[1]}, odd ? S0.b : S1.b};
+        step(last, X, X, r1, r0, std::false_type{});
     }
     // The last sums are on their way through the matrix pipe, which the compiler does not know: it sees them changed behind
     // the wait, so that nothing that reads them can move ahead of it.  (check_matrix_asm.py looks through the machine code
@@ -385,10 +444,8 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
 template <int BM, int BN, bool kInt4, bool kOff>
 __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
 {
-    __shared__ __attribute__((aligned(1024))) char A0[BM * 128];
-    __shared__ __attribute__((aligned(1024))) char A1[BM * 128];
-    __shared__ __attribute__((aligned(1024))) char B0[BN * 128];
-    __shared__ __attribute__((aligned(1024))) char B1[BN * 128];
+    __shared__ __attribute__((aligned(1024))) char A0[BM * 64], A0h[BM * 64], A1[BM * 64], A1h[BM * 64], B0[BN * 128], B1[BN * 128];
+    const WqStage S0{{A0, A0h}, B0}, S1{{A1, A1h}, B1};
     const uint32_t tiles = p.tiles_m * p.tiles_n;
     uint32_t tm, tn;
     if (BM == 128 || blockIdx.x < p.full) {
@@ -397,7 +454,7 @@ __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
             return;  // whole workgroup (the launch is rounded up to a multiple of 8)
         }
         band_order(t, p.tiles_m, p.tiles_n, tm, tn);
-        wq_tile<BM, BN, kInt4, kOff>(p, tm * BM, tn * BN, A0, A1, B0, B1);
+        wq_tile<BM, BN, kInt4, kOff>(p, tm * BM, tn * BN, S0, S1);
     } else if constexpr (BM == 256) {
         const uint32_t t = xcd_remap(blockIdx.x - p.full, 2u * (tiles - p.full));
         if (t == 0xFFFFFFFFu) {
@@ -406,7 +463,7 @@ __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
         band_order(p.full + t / 2u, p.tiles_m, p.tiles_n, tm, tn);
         const uint32_t row0 = tm * 256u + (t & 1u) * 128u;
         if (row0 < p.m) {
-            wq_tile<128, BN, kInt4, kOff>(p, row0, tn * BN, A0, A1, B0, B1);
+            wq_tile<128, BN, kInt4, kOff>(p, row0, tn * BN, S0, S1);
         }
     }
 }
