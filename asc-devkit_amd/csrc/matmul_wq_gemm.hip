@@ -6,17 +6,16 @@
 // side.  v_mfma_f32_16x16x32_f16 instead of the 32 x 32 x 16 form: on random operands a loop of nothing but matrix
 // instructions reaches 1880 against 1640 TFLOP/s (it moves half the sums per product, and the clock is set by the power),
 // which is 4 to 6 % of this kernel.  k = 8192, n = 28672, before (one pass over the weights per 16 rows; 128 x 128 tiles)
-// and now: int4 512 rows 1035 -> 203 us (1180 TFLOP/s), int8 2048 rows 1120 -> 847 us (1136), 512 rows 310 -> 221 us.  A workgroup is 8
+// and now: int4 512 rows 1035 -> 207 us (1160 TFLOP/s), int8 2048 rows 1120 -> 810 us (1190), 512 rows 310 -> 216 us.  A workgroup is 8
 // wavefronts on a BM x BN tile, K step 64, two LDS stages.  x goes from memory to LDS without registers
 // (global_load_lds_dwordx4); the raw bytes of B take the way through registers (16 or 32 per thread and step, fetched
 // two steps ahead), are de-quantised with the operators' own roundings and written to LDS as halves, one 16-byte piece
-// behind the matrix instructions of each quarter of a step.  Both tiles lie in LDS as lines of 64 halves (128 bytes) whose
-// 16-byte pieces are XOR-swizzled by half the line number, so that 16 lanes reading a piece of 16 neighbouring lines
-// meet all 64 banks, and one piece of a line is the operand of v_mfma_f32_16x16x32_f16 as it lies.  (The conflict cycles that
-// are counted, 17.5 % of the LDS cycles, come to 9 for each of the B tile's writes: 33.9 M for 3.7 M of them at 2048 rows of int8.
-// That fits writes that meet 32 banks at a time, where the pieces of a line and its neighbour meet.)  A step's barrier
-// stands before its last quarter, whose operands are in registers by then: behind it the matrix pipe has work while
-// the next step's loads are issued and its first operands read.
+// behind the matrix instructions of each quarter of a step.  Both tiles lie in LDS as lines of 64 halves (128 bytes), one
+// 16-byte piece of which is the operand of v_mfma_f32_16x16x32_f16 as it lies; neither reads nor writes meet a bank twice
+// (wq_swizzle; with pieces swizzled by half the line number alone every write of the B tile cost 9 cycles more, 21 % of the
+// LDS cycles: 2048 x 8192 x 28672 813 -> 809 us, 300 x 4096 x 11008 64 -> 62).  The barriers stand before a step's second and last quarter, whose operands are in registers by
+// then: behind them the matrix pipe has work while loads are issued and operands read.  At 2048 rows of int8 the matrix
+// pipe works in 69 % of the clocks, which the power limit holds at 1.64 GHz.
 #include <type_traits>
 #include <utility>
 
@@ -76,6 +75,10 @@ __device__ __forceinline__ uint32_t pair_of_i4(uint32_t q, int c, f16x2 sc, f16x
                  : finish<kOff>(as_h2((src & mk.even) | mk.exp_even) - both(1032.0f), sc, of);
 }
 
+// Where piece q of a line of 128 bytes lies: at q ^ wq_swizzle(line).  16 neighbouring lines meet all 64 banks in a 16-byte
+// read of one piece, and four neighbouring lines all 32 banks that a write sees at a time in two pieces four apart.
+__device__ __forceinline__ uint32_t wq_swizzle(uint32_t line) { return ((line >> 1) & 7u) ^ ((line & 1u) << 1); }
+
 // One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
 // wavefront owns BM / kWM rows by 64 columns.
 struct WqStage {
@@ -94,7 +97,7 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / kWN, wn = wave % kWN;
 
-    // ---- A: lane owns LDS slot (instr * 64 + lane) of 16 bytes of a half's array: line slot / 8, piece position ^ ((line / 2) % 8);
+    // ---- A: lane owns LDS slot (instr * 64 + lane) of 16 bytes of a half's array: line slot / 8, piece position ^ wq_swizzle(line);
     // line r is row r % kRows of that half of wavefront row r / kRows
     constexpr int kHalf = kAInstr / 2;                     // instructions per half
     constexpr uint32_t kRows = NH * 16u;
@@ -106,7 +109,7 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
         const uint32_t s = (wave * kHalf + u % kHalf) * 64u + lane, line = s >> 3;
         const uint32_t r = (line / kRows * 2u + u / kHalf) * kRows + line % kRows;
         const uint32_t row = row0 + r < p.m ? r : p.m - 1u - row0;  // rows past the end are never stored
-        aoff[u] = row * row_bytes + (((s & 7u) ^ ((line >> 1) & 7u)) << 4);
+        aoff[u] = row * row_bytes + (((s & 7u) ^ wq_swizzle(line)) << 4);
     }
     const char* Abase = reinterpret_cast<const char*>(p.x) + static_cast<size_t>(row0) * row_bytes;
     const uint32_t last = p.k / kBK - 1u;
@@ -129,7 +132,8 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     if constexpr (kInt4) {
         // a K step is half a packed tile: 32 lanes of 16 bytes, lane column l % 16, k 32 (l / 16) .. + 31
         constexpr uint32_t kPer = 4u / kParts;             // threads that share such a lane's 16 bytes
-        const uint32_t s = tid / kPer, l = s & 31u;
+        // (neighbouring threads take both halves of a column's 64 k, so that eight of them write eight pieces apart)
+        const uint32_t s = tid / kPer, l = kParts == 4 ? ((s >> 1) & 15u) | (s & 1u) << 4 : s & 31u;
         bcol = (s >> 5) * 16u + (l & 15u);
         bpiece = 4u * (l >> 4) + (tid % kPer) * kParts;
         boff = (s >> 5) * (p.k * 8u) + l * 16u + (tid % kPer) * 8u;
@@ -187,7 +191,7 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
             }
         }
     };
-    const uint32_t bline = bcol * 128u, bswz = (bcol >> 1) & 7u;
+    const uint32_t bline = bcol * 128u, bswz = wq_swizzle(bcol);
     WqMasks mk = p.mk;
     asm volatile("" : "+v"(mk.exp_even), "+v"(mk.exp_odd));  // (an instruction takes one scalar operand)
     // pair c of piece q of the thread's share of a step; the finished piece goes to LDS
@@ -217,7 +221,7 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     const uint32_t lc = lane & 15u, lq = lane >> 4;
     uint32_t foff[2];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) foff[ks] = lc * 128u + (((4u * ks + lq) ^ (lc >> 1)) << 4);
+    for (int ks = 0; ks < 2; ++ks) foff[ks] = lc * 128u + (((4u * ks + lq) ^ wq_swizzle(lc)) << 4);
     f16x8 af[2][NH], bf[2][TJ];
     auto load_a = [&](const WqStage& S, int q, int i) __attribute__((always_inline)) {
         af[q & 1][i] = *reinterpret_cast<const f16x8*>(S.a[q >> 1] + (wm * NH + i) * 2048u + foff[q & 1]);
