@@ -30,12 +30,10 @@ __device__ __forceinline__ void group_row_tiles(uint32_t rows, uint32_t& big, ui
 }
 
 // One phase of the grouped kernel's plan (see gemm_dma_group_kernel): the workgroup's ids that fall into it.
-// (tiles of at most 128 rows never run the 16 x 16 x 64 instruction)
-template <uint32_t phase, int kForm>
+template <uint32_t phase, int kForm>  // (kForm: of the phase's tiles)
 __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const uint32_t* PLAN, const Stage& S0, const Stage& S1,
                                                      float* TS)
 {
-    constexpr int kSmall = kForm == k16 ? k32 : kForm;
     for (uint32_t id = blockIdx.x;; id += gridDim.x) {
         const uint32_t tiles_n = p.tiles_n;
         const uint32_t big_tiles = __builtin_amdgcn_readfirstlane(PLAN[0]);
@@ -91,9 +89,9 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
         } else if constexpr (phase == 1) {
             gemm_dma_tile_at<256, 128, false, true, 0, kForm>(p, at, 0u, TS, S0, S1);
         } else if (at.row_end - at.row0 <= 64u) {  // uniform: a remainder of at most 64 rows
-            gemm_dma_tile_at<64, 256, false, true, 0, kSmall>(p, at, 0u, TS, S0, S1);
+            gemm_dma_tile_at<64, 256, false, true, 0, kForm>(p, at, 0u, TS, S0, S1);
         } else {
-            gemm_dma_tile_at<128, 256, false, true, 0, kSmall>(p, at, 0u, TS, S0, S1);
+            gemm_dma_tile_at<128, 256, false, true, 0, kForm>(p, at, 0u, TS, S0, S1);
         }
         __syncthreads();  // the next tile's loads and token scales overwrite what slower wavefronts may still read
     }
@@ -111,7 +109,7 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
 // run side by side.  The group sizes are known only on the device, so a launch sized by the host for the worst case
 // would consist mostly of workgroups with nothing to do; the loop has none.  gridDim.x must be a multiple of 8;
 // p.tiles_n = 256-wide tile columns of the whole matrix.
-template <int kForm>
+template <int kForm, int kSmall>
 __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams p)
 {
     ASCQ_DMA_STAGES(kForm, 256, 256);
@@ -148,7 +146,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams 
     // one tile shape's code and registers.
     gemm_dma_group_phase<0, kForm>(p, PLAN, S0, S1, TS);
     gemm_dma_group_phase<1, kForm>(p, PLAN, S0, S1, TS);
-    gemm_dma_group_phase<2, kForm>(p, PLAN, S0, S1, TS);
+    gemm_dma_group_phase<2, kSmall>(p, PLAN, S0, S1, TS);
 }
 
 }  // namespace
@@ -176,13 +174,20 @@ int launch_gemm_dma_group(GemmParams& p, hipStream_t st)
         plan_note(ASCQ_MM_KERNEL_DMA_256, 256, 256, BK, wgs, 1, 2u * (256u * BK + BK * 256u) + 256u * 4u, 0);
         return ASCQ_OK;
     }
+    // The 16 x 16 x 64 form, whose loads have one and a half K steps to arrive, for the remainders too from k = 3072 on; with fewer steps
+    // a small tile's start, two stages of loads, counts for more.  In us, remainders in the 32 x 32 x 32 and the 16 x 16 x 64 form: 16 experts,
+    // 303 tokens, k = 3712, n = 1408 30.1 and 25.7; 8 experts, 4096 tokens, k = 4096, n = 14336 279 and 273; 16 experts, 500 tokens, k =
+    // 2048, n = 4096 28.1 and 30.0; 32 experts, 1000 tokens, k = 1024, n = 4096 39.6 and 42.6.  (Few rows per group: hardly a big tile,
+    // and the kernel without that form's code is 1 to 2 % ahead.)
     const int form = gemm_dma_form(p);
     if (form == k32Ragged) {
-        gemm_dma_group_kernel<k32Ragged><<<wgs, kThreads, 0, st>>>(p);
-    } else if (form == k16) {
-        gemm_dma_group_kernel<k16><<<wgs, kThreads, 0, st>>>(p);
+        gemm_dma_group_kernel<k32Ragged, k32Ragged><<<wgs, kThreads, 0, st>>>(p);
+    } else if (form == k16 && p.k >= 3072u) {
+        gemm_dma_group_kernel<k16, k16><<<wgs, kThreads, 0, st>>>(p);
+    } else if (form == k16 && p.m > 128u * p.groups) {
+        gemm_dma_group_kernel<k16, k32><<<wgs, kThreads, 0, st>>>(p);
     } else {
-        gemm_dma_group_kernel<k32><<<wgs, kThreads, 0, st>>>(p);
+        gemm_dma_group_kernel<k32, k32><<<wgs, kThreads, 0, st>>>(p);
     }
     return launch_status("ascq_group_matmul_w8a8");
 }

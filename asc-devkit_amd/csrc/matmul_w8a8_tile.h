@@ -251,8 +251,8 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     auto quarter = [&](auto qq, auto reads, auto&& read, auto from, auto to, auto&& fetch) __attribute__((always_inline)) {
         constexpr int q = decltype(qq)::value, kReads = decltype(reads)::value, kFrom = decltype(from)::value, kCount = decltype(to)::value - kFrom;
         constexpr int kFront = kM >= 8 ? kM / 2 : kM, kPer = (kReads + kFront - 1) / kFront;
-        constexpr int kEvery = kM / (kCount > 0 ? kCount : 1);
-        static_assert(kCount <= kM, "at most one load behind a matrix instruction");
+        constexpr int kAtOnce = kCount > kM ? (kCount + kM - 1) / kM : 1, kTimes = kCount > 0 ? (kCount + kAtOnce - 1) / kAtOnce : 1;
+        constexpr int kEvery = kM / kTimes;
         static_for<kM>([&](auto nn) {
             constexpr int n = decltype(nn)::value;
             mfma(q, n);
@@ -260,7 +260,12 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
                 constexpr int i = n * kPer + decltype(r)::value;
                 if constexpr (i < kReads) read(i);
             });
-            if constexpr (n % kEvery == kEvery - 1 && n / kEvery < kCount) fetch(kFrom + n / kEvery);
+            if constexpr (n % kEvery == kEvery - 1) {
+                static_for<kAtOnce>([&](auto r) {
+                    constexpr int u = n / kEvery * kAtOnce + decltype(r)::value;
+                    if constexpr (u < kCount) fetch(kFrom + u);
+                });
+            }
             __builtin_amdgcn_sched_barrier(0);
         });
     };
@@ -1078,16 +1083,20 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     auto a_slot = [&](int u) __attribute__((always_inline)) { return (wave * kAInstr + u) * 64u + lane; };
     auto b_slot = [&](int u) __attribute__((always_inline)) { return (wave * kBInstr + u) * 64u + lane; };
     auto line_piece = [](uint32_t s) __attribute__((always_inline)) { return (s & 7u) ^ ((s >> 4) & 7u); };  // of slot s of a [line][128] tile
-    uint32_t aoff[kAInstr], boff[kBInstr];
+    // 16x16x64 form: instructions of a half of A's rows, per wavefront (64 rows: four in all, issued by two wavefronts each,
+    // so that every wavefront counts the same loads)
+    constexpr int kHalfAll = BM * BK / 2048, kHalfInstr = kHalfAll >= 8 ? kHalfAll / 8 : 1;
+    constexpr int kALoads = kForm == k16 ? 2 * kHalfInstr : kAInstr;
+    uint32_t aoff[kALoads], boff[kBInstr];
 #pragma unroll
-    for (int u = 0; u < kAInstr; ++u) {
+    for (int u = 0; u < kALoads; ++u) {
         uint32_t s = a_slot(u), line = s >> 3;
         if constexpr (kForm == k16) {
             // loads of half h of every wavefront's rows: line r of its LDS array is row r % kRows of that half of wavefront
             // row r / kRows
-            constexpr uint32_t kPart = kAInstr / 2, kRows = BM * (BN / 64) / 16;
-            s = (wave * kPart + u % kPart) * 64u + lane;
-            line = ((s >> 3) / kRows * 2u + u / kPart) * kRows + (s >> 3) % kRows;
+            constexpr uint32_t kRows = BM * (BN / 64) / 16;
+            s = (wave * kHalfInstr + u % kHalfInstr) % kHalfAll * 64u + lane;
+            line = ((s >> 3) / kRows * 2u + u / kHalfInstr) * kRows + (s >> 3) % kRows;
         }
         uint32_t row = row0 + line;
         row = row < row_end ? row : row_end - 1;  // rows past the end are never stored: any valid row will do
@@ -1189,13 +1198,13 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
                 asm volatile("" : "+v"(boff[u]));
                 __builtin_amdgcn_global_load_lds((gptr_t)(from.b + boff[u]), (lds_ptr_t)(S.b + (wave * kBInstr + u) * 1024), 16, 0, 0);
             } else {
-                constexpr int kPart = kAInstr / 2;
                 const int v = u - kBInstr;
                 asm volatile("" : "+v"(aoff[v]));
-                __builtin_amdgcn_global_load_lds((gptr_t)(from.a + aoff[v]), (lds_ptr_t)(S.a[v / kPart] + (wave * kPart + v % kPart) * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr_t)(from.a + aoff[v]),
+                                                 (lds_ptr_t)(S.a[v / kHalfInstr] + (wave * kHalfInstr + v % kHalfInstr) % kHalfAll * 1024), 16, 0, 0);
             }
         };
-        gemm_dma_body16<BM, BN, kGrouped, kB, kAInstr, kBInstr>(p, at, n0, steps, wave, lane, bases, load, stages..., TS);
+        gemm_dma_body16<BM, BN, kGrouped, kB, kALoads, kBInstr>(p, at, n0, steps, wave, lane, bases, load, stages..., TS);
     } else if constexpr (kForm == kRing) {
         auto load = [&](uint32_t step, int u, char* S) __attribute__((always_inline)) {
             // how much of the row's k is left from here on, nothing past the last step; a piece past it brings zeros

@@ -582,6 +582,29 @@ def test_group_matmul_both_matrix_instructions_agree(kind):
         first += c
 
 
+@pytest.mark.parametrize("k", [256, 384, 3072, 3200])
+@pytest.mark.parametrize("nz", [False, True])
+@pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 256, 16, 480, 385]])
+def test_group_matmul_remainders_in_both_forms(counts, nz, k):
+    """Remainders of 64 and of 128 rows, and big tiles whose second wavefront row is empty, partly filled or full; from k =
+    3072 on in the form whose loads are spread over a step and a half; even and odd numbers of K steps."""
+    announce("group remainders", counts, nz, k)
+    rng = np.random.default_rng(k + len(counts) + nz)
+    g, m, n = len(counts), sum(counts), 544
+    x, w = rand_i8(rng, (m, k)), rand_i8(rng, (g, k, n))
+    sc, tok = rng.uniform(1e-4, 1e-3, (g, n)).astype(np.float32), rng.uniform(5e-3, 2e-2, m).astype(np.float32)
+    y = torch.zeros((m, n), dtype=torch.float16, device=DEV)
+    wd = to_dev(w)
+    ops.quant_group_matmul(y, to_dev(x), ops.pack_weight_nz(wd) if nz else wd, torch.tensor(counts, dtype=torch.int64, device=DEV),
+                           to_dev(sc), to_dev(tok), weight_nz=nz)
+    want, r = np.zeros((m, n), np.float32), 0
+    for i, c in enumerate(counts):      # (float64 holds the sums exactly; one fp32 rounding per step of the epilogue)
+        sums = (x[r:r + c].astype(np.float64) @ w[i].astype(np.float64)).astype(np.float32)
+        want[r:r + c] = sums * sc[i] * tok[r:r + c, None]
+        r += c
+    assert torch.equal(y.cpu(), torch.from_numpy(want).to(torch.float16))
+
+
 def test_post_bias_bf16_and_gelu():
     announce("matmul bf16 bias + token scale + FasterGelu")
     rng = np.random.default_rng(22)
