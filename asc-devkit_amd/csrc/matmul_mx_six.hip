@@ -13,10 +13,10 @@
 //
 // The tile kernel: 8 wavefronts as 2 x 4, each 128 x 64 of the tile: 8 x 4 blocks of v_mfma_scale_f32_16x16x128_f8f6f4, which
 // on random operands, where the power limit sets the clock, reaches 6.2 PFLOP/s against 5.6 of the 32x32x64 form.  Three LDS stages of a step
-// each (48 KiB), filled by direct-to-LDS loads that are issued two steps ahead, one behind every other matrix instruction, so that the way
+// each (48 KiB), filled by direct-to-LDS loads that are issued two steps ahead, one behind every fourth matrix instruction or so, so that the way
 // from the L2 is never idle: with two stages and all loads waited for at every step the loads arrived at 11 TB/s over
 // the chip, a loop of nothing but loads with a stage always on its way reaches 26.  m = n = k = 8192: tiles 330 -> 264 us, the call
-// with the widening launch 375 -> 306 (operands of zeros, where the power limit is not met: 301 -> 215); 512 x 8192 x 8192 88 -> 69;
+// with the widening launch 365 -> 290 (operands of zeros, where the power limit is not met: 301 -> 215); 512 x 8192 x 8192 88 -> 69;
 // 4096 x 4096 x 4096 66 -> 56.  What is left: 24 + 2 LDS reads for 32 matrix instructions of a wavefront, the power limit.
 #include <type_traits>
 #include <utility>
@@ -259,11 +259,13 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
     };
     constexpr int kFirst = 14, kSecond = 12;
 
-    // ---- one step, in stage X with operand set `set`; the next one is in Y, the loads go to the stage of the step before.
+    // ---- one step, in stage X with operand set `set`; the next one is in Y, the one behind it on its way into Z.
     // The first half of its matrix instructions takes units 0-3 of a and reads the rest of the step's operands behind them; then the wait
     // (the next step's stage has landed, only the seven loads of the step behind it are on their way; every
-    // wavefront has read this stage) and the barrier; the second half reads the next step's first operands, and the loads of the step three
-    // ahead go into this stage.
+    // wavefront has read this stage) and the barrier; the second half reads the next step's first operands.  The loads of the step
+    // three ahead go into this stage: four of them in this step's second half, the others in the next one's first, each
+    // behind a fourth matrix instruction (all in the second half, behind every other one: m = n = k = 8192 300 us, so 292).
+    constexpr int kNow = 4, kEvery = 4;
     auto half = [&](auto hh, auto set, auto&& behind) __attribute__((always_inline)) {
         constexpr int h = decltype(hh)::value, x = decltype(set)::value;
         six_static_for<16>([&](auto nn) {
@@ -281,16 +283,19 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto step = [&](uint32_t s, const Stage& X, const Stage& Y, auto set) __attribute__((always_inline)) {
+    auto step = [&](uint32_t s, const Stage& X, const Stage& Y, const Stage& Z, auto set) __attribute__((always_inline)) {
+        auto due = [](int n, int count) { return n % kEvery == kEvery - 1 && n / kEvery < count; };
+        const Sources behind = sources(s + 2u);
         asm volatile("" : "+v"(lane16), "+v"(lane8), "+v"(lane4));
         half(std::integral_constant<int, 0>{}, set, [&](auto n) __attribute__((always_inline)) {
             if constexpr (decltype(n)::value < kSecond) second_read(X, n);
+            if (due(decltype(n)::value, kLoads - kNow)) load(behind, kNow + decltype(n)::value / kEvery, Z);
         });
         arrive(std::integral_constant<int, kLoads>{});
-        const Sources from = sources(s + 3u);
+        const Sources ahead = sources(s + 3u);
         half(std::integral_constant<int, 1>{}, set, [&](auto n) __attribute__((always_inline)) {
             if constexpr (decltype(n)::value < kFirst) first_read(Y, std::integral_constant<int, 1 - decltype(set)::value>{}, n);
-            if constexpr (decltype(n)::value % 2 == 1 && decltype(n)::value / 2 < kLoads) load(from, decltype(n)::value / 2, X);
+            if (due(decltype(n)::value, kNow)) load(ahead, decltype(n)::value / kEvery, X);
         });
     };
     const Stage T0{L0, L0 + kOperand, C0}, T1{L1, L1 + kOperand, C1}, T2{L2, L2 + kOperand, C2};
@@ -301,9 +306,9 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) load(f1, u, T1);
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) load(f2, u, T2);
+        for (int u = 0; u < kNow; ++u) load(f2, u, T2);
     }
-    arrive(std::integral_constant<int, 2 * kLoads>{});
+    arrive(std::integral_constant<int, kLoads + kNow>{});
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
     six_static_for<kFirst>([&](auto r) { first_read(T0, even, r); });
@@ -311,23 +316,23 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
     // stage that holds the last step again, or still an older one; nobody uses what it read.)
     uint32_t s = 0;
     for (; s + 6u <= steps; s += 6u) {
-        step(s, T0, T1, even);
-        step(s + 1u, T1, T2, odd);
-        step(s + 2u, T2, T0, even);
-        step(s + 3u, T0, T1, odd);
-        step(s + 4u, T1, T2, even);
-        step(s + 5u, T2, T0, odd);
+        step(s, T0, T1, T2, even);
+        step(s + 1u, T1, T2, T0, odd);
+        step(s + 2u, T2, T0, T1, even);
+        step(s + 3u, T0, T1, T2, odd);
+        step(s + 4u, T1, T2, T0, even);
+        step(s + 5u, T2, T0, T1, odd);
     }
     if (s < steps) {
-        step(s, T0, T1, even);
+        step(s, T0, T1, T2, even);
         if (s + 1u < steps) {
-            step(s + 1u, T1, T2, odd);
+            step(s + 1u, T1, T2, T0, odd);
             if (s + 2u < steps) {
-                step(s + 2u, T2, T0, even);
+                step(s + 2u, T2, T0, T1, even);
                 if (s + 3u < steps) {
-                    step(s + 3u, T0, T1, odd);
+                    step(s + 3u, T0, T1, T2, odd);
                     if (s + 4u < steps) {
-                        step(s + 4u, T1, T2, even);
+                        step(s + 4u, T1, T2, T0, even);
                     }
                 }
             }
