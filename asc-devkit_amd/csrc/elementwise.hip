@@ -7,6 +7,7 @@
 // launch (per-channel scale / offset) are loaded once per lane and reused for all its rows.
 #include "ascq_common.h"
 #include "ascq_device.h"
+#include "matmul_w8a8.h"
 
 namespace ascq {
 namespace {
@@ -347,7 +348,7 @@ __device__ __forceinline__ float block_max(float v, float* lds)
 // two, 4.5 against 4.7 us per launch at 2048 rows of 4096 bfloat16 (a conversion without the reduction: 3.7 us).
 template <int kSrc, int kVecs, int kBlock = kThreads>
 __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q, float* __restrict__ ts,
-                                                          const void* __restrict__ x, uint32_t n)
+                                                          const void* __restrict__ x, uint32_t n, uint32_t ldq)
 {
     constexpr int kThreads = kBlock;  // (shadows the file's constant inside this kernel)
     __shared__ float lds[kThreads / 64];
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
             u32x2 out;
             out[0] = __builtin_amdgcn_perm(u[1], u[0], 0x0c0c0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000c0cu);
             out[1] = __builtin_amdgcn_perm(u[5], u[4], 0x0c0c0400u) | __builtin_amdgcn_perm(u[7], u[6], 0x04000c0cu);
-            *reinterpret_cast<u32x2*>(q + static_cast<size_t>(row) * n + j) = out;
+            *reinterpret_cast<u32x2*>(q + static_cast<size_t>(row) * ldq + j) = out;
         }
     }
 }
@@ -395,7 +396,7 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
 // Any n / alignment: two passes over the row (the second one hits in L2).
 template <int kSrc>
 __global__ __launch_bounds__(kThreads) void dynq_generic_kernel(int8_t* __restrict__ q, float* __restrict__ ts,
-                                                                const void* __restrict__ x, uint32_t n)
+                                                                const void* __restrict__ x, uint32_t n, uint32_t ldq)
 {
     __shared__ float lds[kThreads / 64];
     const size_t base = static_cast<size_t>(blockIdx.x) * n;
@@ -410,28 +411,28 @@ __global__ __launch_bounds__(kThreads) void dynq_generic_kernel(int8_t* __restri
         ts[blockIdx.x] = zero ? 1.0f : amax / 127.0f;
     }
     for (uint32_t j = threadIdx.x; j < n; j += kThreads) {
-        q[base + j] = static_cast<int8_t>(round_sat8<true>(load1<kSrc>(x, base + j) * inv, 0));
+        q[static_cast<size_t>(blockIdx.x) * ldq + j] = static_cast<int8_t>(round_sat8<true>(load1<kSrc>(x, base + j) * inv, 0));
     }
 }
 
 template <int kSrc>
-int launch_dynq(uint32_t m, uint32_t n, void* q, void* ts, const void* x, hipStream_t st)
+int launch_dynq(uint32_t m, uint32_t n, void* q, uint32_t ldq, void* ts, const void* x, hipStream_t st)
 {
     int8_t* qq = static_cast<int8_t*>(q);
     float* tt = static_cast<float*>(ts);
-    const bool vec = (n % 8 == 0) && aligned16(x) && ((reinterpret_cast<uintptr_t>(q) & 7u) == 0);
+    const bool vec = (n % 8 == 0) && (ldq % 8 == 0) && aligned16(x) && ((reinterpret_cast<uintptr_t>(q) & 7u) == 0);
     if (vec && n <= 1024) {
-        dynq_row_kernel<kSrc, 1, 128><<<m, 128, 0, st>>>(qq, tt, x, n);
+        dynq_row_kernel<kSrc, 1, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
     } else if (vec && n <= 2048) {
-        dynq_row_kernel<kSrc, 2, 128><<<m, 128, 0, st>>>(qq, tt, x, n);
+        dynq_row_kernel<kSrc, 2, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
     } else if (vec && n <= 4096) {
-        dynq_row_kernel<kSrc, 4, 128><<<m, 128, 0, st>>>(qq, tt, x, n);
+        dynq_row_kernel<kSrc, 4, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
     } else if (vec && n <= 8192) {
-        dynq_row_kernel<kSrc, 4><<<m, kThreads, 0, st>>>(qq, tt, x, n);
+        dynq_row_kernel<kSrc, 4><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
     } else if (vec && n <= 16384) {
-        dynq_row_kernel<kSrc, 8><<<m, kThreads, 0, st>>>(qq, tt, x, n);
+        dynq_row_kernel<kSrc, 8><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
     } else {
-        dynq_generic_kernel<kSrc><<<m, kThreads, 0, st>>>(qq, tt, x, n);
+        dynq_generic_kernel<kSrc><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
     }
     return launch_status("ascq_dynamic_quant_per_token");
 }
@@ -1116,11 +1117,15 @@ extern "C" int ascq_dynamic_quant_per_token(int32_t src_dtype, uint32_t m, uint3
     if (m == 0) {
         return ASCQ_OK;
     }
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    return dynamic_quant_rows(src_dtype, m, n, q, n, tok_scale, x, static_cast<hipStream_t>(stream));
+}
+
+int ascq::dynamic_quant_rows(int32_t src_dtype, uint32_t m, uint32_t n, void* q, uint32_t ldq, void* tok_scale, const void* x, hipStream_t st)
+{
     switch (src_dtype) {
-        case ASCQ_F16: return launch_dynq<ASCQ_F16>(m, n, q, tok_scale, x, st);
-        case ASCQ_BF16: return launch_dynq<ASCQ_BF16>(m, n, q, tok_scale, x, st);
-        case ASCQ_F32: return launch_dynq<ASCQ_F32>(m, n, q, tok_scale, x, st);
+        case ASCQ_F16: return launch_dynq<ASCQ_F16>(m, n, q, ldq, tok_scale, x, st);
+        case ASCQ_BF16: return launch_dynq<ASCQ_BF16>(m, n, q, ldq, tok_scale, x, st);
+        case ASCQ_F32: return launch_dynq<ASCQ_F32>(m, n, q, ldq, tok_scale, x, st);
         default: return fail(ASCQ_EUNSUPPORTED, "ascq_dynamic_quant_per_token: src dtype %d", src_dtype);
     }
 }

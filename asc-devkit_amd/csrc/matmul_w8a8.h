@@ -20,6 +20,7 @@ struct GemmParams {
     const int8_t* a;
     const int8_t* b;
     uint32_t m, n, k;
+    uint32_t lda;   // bytes from one row of A to the next where they are not k (ring tiles only); 0: k
     uint32_t b_nz;  // B is in the fractal layout [n/32][k][32] (direct-to-LDS tile kernels only)
     uint32_t tiles_m, tiles_n;
     uint32_t k_splits, k_per_split;  // split-K: bytes of K per grid.z slice (multiple of kBK)
@@ -225,6 +226,8 @@ struct RingPlan {
     uint32_t bm, bn;
     double us;  // estimate, quantiser included
 };
+// The per-token quantiser of elementwise.hip, rows of q ldq bytes apart.
+int dynamic_quant_rows(int32_t src_dtype, uint32_t m, uint32_t n, void* q, uint32_t ldq, void* tok_scale, const void* x, hipStream_t st);
 RingPlan gemm_ring_plan(uint32_t m, uint32_t n, uint32_t k, int b_layout);
 int launch_gemm_ring(const GemmParams& p, int shape, int b_layout, hipStream_t st);
 int launch_gemm_dma_group(GemmParams& p, hipStream_t st);  // matmul_w8a8_group.hip

@@ -7,7 +7,7 @@
 // the next one's.  A step's operands are read from the LDS behind the matrix instructions of the step before.  No K split, so no
 // int32 partial tiles and no second launch.  A last, partial K step and the steps past
 // the end are loads whose offset lies past the buffer: zeros arrive.
-// In us with the quantiser, split or large tiles and this: 729 x 4304 x 1152 27.8 and 21.0, 600 x 4096 x 4096 47.4 and 27.8, 1024 x
+// In us with the quantiser, split or large tiles and this: 729 x 4304 x 1152 27.8 and 19.2, 600 x 4096 x 4096 47.4 and 27.8, 1024 x
 // 11008 x 4096 103 and 64.  What is left: a step of 64 x 64 takes 0.19 us without the bytes of its loads (the barrier, ten LDS
 // reads and two loads per wavefront), one of 128 x 128 0.46 with nothing but loads (what is in flight over the latency of an L2 miss).
 #include "matmul_w8a8_tile.h"

@@ -1061,7 +1061,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     constexpr int kBInstr = BK * BN / 1024 / 8;  // B DMA instructions per wavefront and K step
     static_assert(kAInstr >= 1 && kBInstr >= 1, "tile shape does not fit eight wavefronts");
 
-    const uint32_t K = p.k, N = p.n;
+    const uint32_t K = p.k, N = p.n, lda = kForm == kRing && p.lda != 0u ? p.lda : K;
     const uint32_t row0 = at.row0, row_end = at.row_end;
     const uint32_t n0 = kB == 0 && N % 16u != 0 && at.n0 + BN > N ? N - BN : at.n0;
     const int8_t* Bmat = at.b;
@@ -1100,7 +1100,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
         }
         uint32_t row = row0 + line;
         row = row < row_end ? row : row_end - 1;  // rows past the end are never stored: any valid row will do
-        aoff[u] = (row - row0) * K + 16u * line_piece(s);
+        aoff[u] = (row - row0) * lda + 16u * line_piece(s);
     }
 #pragma unroll
     for (int u = 0; u < kBInstr; ++u) {
@@ -1135,7 +1135,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
         steps = steps * (bidy + 1u) / p.k_splits - s_begin;
     }
     const uint32_t partial = K % BK != 0 ? all_steps - 1u - s_begin : 0xFFFFFFFFu;  // the step with less than BK of k
-    const int8_t* Abase = p.a + static_cast<size_t>(row0) * K + static_cast<size_t>(s_begin) * BK;
+    const int8_t* Abase = p.a + static_cast<size_t>(row0) * lda + static_cast<size_t>(s_begin) * BK;
     const int8_t* Bbase = Bmat + (kBT ? static_cast<size_t>(n0) * K : kBP ? static_cast<size_t>(n0 >> 4) * K * 16u : p.b_nz ? 0u : n0) +
                           static_cast<size_t>(s_begin) * BK * ldb;
     // A wavefront-uniform address, pinned to scalar registers: a load's address is then this base plus the lane's
