@@ -769,7 +769,9 @@ double without_ring_us(const ascq_matmul_desc* d, const GemmParams& p, int b_lay
 // 4096 28.6 and 36.0 (ten splits of K on 32 tiles), 512 x 2048 x 11008 24.5 and 28.3 (more tiles of 128 x 128 than units).
 bool ring_preferred(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, const void* workspace, size_t workspace_bytes, RingPlan& plan)
 {
-    if (d->m <= 32u || d->trans_a || d->b_format == ASCQ_MM_B_NZ || !gemm_dma_supported(p, b_layout)) {
+    // (a lane addresses its row or column of a tile by 31 bits)
+    constexpr uint32_t kMost = 1u << 23;
+    if (d->m <= 32u || d->k > kMost || d->n > kMost || d->trans_a || d->b_format == ASCQ_MM_B_NZ || !gemm_dma_supported(p, b_layout)) {
         return false;
     }
     uint32_t splits = gemm_dma_skinny_splits(d->m, d->n, d->k);

@@ -1395,6 +1395,15 @@ def test_linear_w8a8_small_tiles_with_a_ring_of_stages(m, k, n, act):
             assert np.all(np.abs(got - want) <= (ulp + 2.0 ** -18) * np.abs(want) + 1e-6), layout
 
 
+@pytest.mark.parametrize("m,n,k", [(100, 272, 1040), (130, 528, 1152), (257, 1000, 1280)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_matmul_outputs_of_the_ring_tiles(m, n, k, trans_b):
+    """The plain matmul where 64 x 64 tiles with a ring of stages are one round of the chip: raw int32 sums, and quant words
+    with and without the pre-shift to every output type."""
+    test_int32_accumulators_bit_exact(m, n, k, trans_b)
+    test_fixpipe_pre_shift_words(m, n, k, trans_b)
+
+
 @pytest.mark.parametrize("m,kernel", [(1, abi.MM_KERNEL_STREAM), (100, abi.MM_KERNEL_DMA_128),
                                       (700, abi.MM_KERNEL_DMA_256)])
 def test_matmul_plan_then_call(m, kernel):
