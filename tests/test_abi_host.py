@@ -304,6 +304,19 @@ def test_inline_assembly_kernels_have_no_scratch_frame():
         assert k["vgprs"] + k["agprs"] <= 512 and k["lds_bytes"] <= 160 * 1024, k
 
 
+def test_tile_kernels_with_counted_waits_are_guarded():
+    """Every kernel whose matrix instructions are inline assembly (the objects the Makefile names in MATRIX_ASM) and that keeps its
+    tiles in LDS counts its loads by hand: each is on the list that may not spill."""
+    import json
+    import re
+    makefile = open(os.path.join(ROOT, "asc-devkit_amd", "csrc", "Makefile")).read()
+    files = {o.replace(".o", ".hip") for o in re.search(r"^MATRIX_ASM := (.*)$", makefile, re.M).group(1).split()}
+    rec = json.load(open(os.path.join(ROOT, "asc-devkit_amd", "lib", "kernel_resources.json")))
+    tiles = [k for k in rec["kernels"] if k["file"] in files and k["lds_bytes"] >= 48 << 10]
+    assert {k["file"] for k in tiles} == files
+    assert not [k["name"] for k in tiles if not k["guarded"]]
+
+
 def test_resource_checker_rejects_a_guarded_kernel_with_scratch(tmp_path):
     import subprocess
     import sys
