@@ -8,6 +8,8 @@ instruction.  For every such instruction, on every path that follows it, this pr
   * no instruction that reads or writes its result within kResult wait states (an instruction is one, s_nop n is
     n + 1), but for matrix instructions that accumulate in the same registers, and
   * no vector instruction that writes one of its operands within kOperand wait states before it.
+In the kernels of COUNTED a step loads one operand into LDS and the other into registers, and its counted waits rest on both:
+between two barriers either both kinds of loads are issued or none (the compiler drops a register load that nobody uses).
 """
 import os
 import re
@@ -19,6 +21,7 @@ import tempfile
 LLVM = os.environ.get("LLVM_BIN", "/opt/rocm/llvm/bin")
 MATRIX = ("v_mfma_i32_16x16x64_i8", "v_mfma_f32_16x16x32_f16", "v_mfma_scale_f32_16x16x128_f8f6f4")
 kResult, kOperand = 19, 2
+COUNTED = ("wq_gemm_kernel",)
 
 
 def registers(operand):
@@ -115,6 +118,21 @@ def faults(body):
     return bad
 
 
+def dropped_loads(body):
+    bad, lds, reg = [], 0, 0
+    for i in body:
+        if i.name.startswith(("global_load_lds", "buffer_load")) or i.name.startswith("global_load"):
+            if "_lds" in i.name or i.text.endswith(" lds"):
+                lds += 1
+            else:
+                reg += 1
+        elif i.name == "s_barrier":
+            if lds and not reg:
+                bad.append("%d loads into LDS and none into registers before the barrier at %x" % (lds, i.address))
+            lds = reg = 0
+    return bad
+
+
 def main(paths):
     status = 0
     for path in paths:
@@ -123,6 +141,8 @@ def main(paths):
             count = sum(i.matrix for i in body)
             seen += count
             bad = faults(body) if count else []
+            if any(c in name for c in COUNTED):
+                bad += dropped_loads(body)
             for b in bad[:10]:
                 sys.stderr.write("check_matrix_asm: %s: %s\n" % (name, b))
             status |= bool(bad)

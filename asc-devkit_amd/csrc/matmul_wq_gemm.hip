@@ -288,13 +288,15 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     // half of this step's rows and the last raw bytes of step s + 1 (behind them all of a step's loads), before quarter 3 the
     // first half of the next step's rows and the first raw bytes of step s + 2, with int4 its parameters.  (Without a count of its own
     // for the raw bytes the compiler waits for everything where they cross the loop's end.)
+    // `ahead`: how many steps follow, 2 for two or more.  The last step but one issues no loads: nobody would use what they bring, so the
+    // compiler may leave those into registers out, and a count that includes them would no longer hold the waits back.
     // (BN = 128, two small workgroups on a unit: a quarter is four matrix instructions, and one barrier, before quarter 3, is better: 100 x
     // 4096 x 4096 int4 40.0 us, 42.4 with two.)
     constexpr bool kMid = kFetches == 2;
     constexpr int kPartAll = kFetches * kPartLoads + kParamLoads, kLate = kPartLoads + kParamLoads;  // fetches of a step; behind quarter 3
     constexpr int kEarly = kPartAll - kLate, kRowsLate = kMid ? kHalf : kAInstr;                      // fetches, rows behind quarter 1 / 3
-    auto step = [&](uint32_t s, const WqStage& X, const WqStage& Y, Raw& next, Raw& next2, auto steady) __attribute__((always_inline)) {
-        constexpr bool kSteady = decltype(steady)::value;
+    auto step = [&](uint32_t s, const WqStage& X, const WqStage& Y, Raw& next, Raw& next2, auto ahead) __attribute__((always_inline)) {
+        constexpr bool kSteady = decltype(ahead)::value == 2, kMore = decltype(ahead)::value != 0;
         constexpr std::integral_constant<int, kSteady && kMid ? kHalf + kEarly : 0> early{};
         constexpr std::integral_constant<int, kSteady ? kRowsLate + 1 : 0> late{};
 #pragma unroll
@@ -307,11 +309,11 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
             } else {
                 load_a(X, 1, i - TJ);
             }
-        }, std::integral_constant<int, kSteady && kParts == 4 ? 1 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
-        if constexpr (kMid) arrive(std::integral_constant<int, kSteady ? kAInstr + kPartAll : 0>{});
+        }, std::integral_constant<int, kMore && kParts == 4 ? 1 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
+        if constexpr (kMid) arrive(std::integral_constant<int, kMore ? kAInstr + kPartAll : 0>{});
         quarter(std::integral_constant<int, 1>{}, std::integral_constant<int, NH>{}, [&](auto r) __attribute__((always_inline)) {
             load_a(X, 2, decltype(r)::value);
-        }, std::integral_constant<int, !kSteady ? -1 : kParts == 4 ? 2 : 1>{}, next, Y.b, early, [&](int u) __attribute__((always_inline)) {
+        }, std::integral_constant<int, !kMore ? -1 : kParts == 4 ? 2 : 1>{}, next, Y.b, early, [&](int u) __attribute__((always_inline)) {
             if (u < kHalf) {
                 load_rows(base, u, X);
             } else {
@@ -320,12 +322,12 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
         });
         quarter(std::integral_constant<int, 2>{}, std::integral_constant<int, NH>{}, [&](auto r) __attribute__((always_inline)) {
             load_a(X, 3, decltype(r)::value);
-        }, std::integral_constant<int, kSteady && kParts == 4 ? 3 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
-        if constexpr (kSteady) {
-            arrive(std::integral_constant<int, !kMid ? 0 : kInt4 ? kHalf + kEarly : kAInstr + kPartAll>{});
+        }, std::integral_constant<int, kMore && kParts == 4 ? 3 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
+        if constexpr (kMore) {
+            arrive(std::integral_constant<int, !kMid ? 0 : !kSteady ? kHalf + kPartAll : kInt4 ? kHalf + kEarly : kAInstr + kPartAll>{});
             quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
                 first_operands(Y, decltype(r)::value);
-            }, std::integral_constant<int, 0>{}, next2, X.b, late, [&](int u) __attribute__((always_inline)) {
+            }, std::integral_constant<int, kSteady ? 0 : -1>{}, next2, X.b, late, [&](int u) __attribute__((always_inline)) {
                 if (u < kRowsLate) {
                     load_rows(base, kAInstr - kRowsLate + u, X);
                 } else {
@@ -346,20 +348,30 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
 #pragma unroll
         for (int u = 0; u < kHalf; ++u) load_rows(base, h * kHalf + u, S);
     };
+    auto in_order = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };  // the waits count them
+    in_order();
     prologue_rows(0, 0, S0);
+    in_order();
     if constexpr (kEarly != 0) fetch(r1, 1, 0);
+    in_order();
     prologue_rows(0, 1, S0);
+    in_order();
     fetch(r1, 1, kFetches - 1);
+    in_order();
     wq_for<kParts>([&](auto q) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) dequant_pair(r0, decltype(q)::value, c);
         write_piece(S0.b, decltype(q)::value);
     });
+    in_order();
     prologue_rows(1, 0, S1);
+    in_order();
     if constexpr (kEarly != 0) fetch(r0, 2, 0);
     arrive(std::integral_constant<int, kMid ? kEarly + kHalf + kLate + kHalf + kEarly : kHalf>{});
     prologue_rows(1, 1, S1);
+    in_order();
     fetch(r0, 2, kFetches - 1);
+    in_order();
 #pragma unroll
     for (int c = 0; c < 4; ++c) dequant_pair(r1, 0, c);
     write_piece(S1.b, 0);
@@ -368,18 +380,19 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
     // At the top of step s (stage X, other stage Y): its first operands are in registers, piece 0 of step s + 1 is in Y, the
     // rest of it in raw set (s + 1) % 2, step s + 2's raw bytes are on their way into set s % 2.
     const uint32_t steps = last + 1u;
+    constexpr std::integral_constant<int, 2> two{};
     uint32_t s = 0;
     for (; s + 2u < steps; s += 2u) {
-        step(s, S0, S1, r1, r0, std::true_type{});
-        step(s + 1u, S1, S0, r0, r1, std::true_type{});
+        step(s, S0, S1, r1, r0, two);
+        step(s + 1u, S1, S0, r0, r1, two);
     }
     if (s + 1u < steps) {
-        step(s, S0, S1, r1, r0, std::true_type{});
+        step(s, S0, S1, r1, r0, std::integral_constant<int, 1>{});
     }
     {
         const bool odd = (steps & 1u) != 0;
         const WqStage X{{odd ? S0.a[0] : S1.a[0], odd ? S0.a[1] : S1.a[1]}, odd ? S0.b : S1.b};
-        step(last, X, X, r1, r0, std::false_type{});
+        step(last, X, X, r1, r0, std::integral_constant<int, 0>{});
     }
     // The last sums are on their way through the matrix pipe, which the compiler does not know: it sees them changed behind
     // the wait, so that nothing that reads them can move ahead of it.  (check_matrix_asm.py looks through the machine code

@@ -838,9 +838,9 @@ def test_w4a16_packed_more_than_four_rows(m, k, n, gs):
                                        (1300, 256, 14600, 256)])
 @pytest.mark.parametrize("offset", ["int", "frac", None])
 def test_w4a16_packed_many_rows(m, k, n, gs, offset):
-    """More rows than a few passes: the half GEMM whose B-tile loader de-quantises the packed tiles.  One step of k, odd
-    and even numbers of steps, row and column tails of every tile shape, groups of half a step; the last case has tiles
-    beyond a whole round, which are cut in half (checked on its first, a middle and the last columns)."""
+    """More rows than a few passes: the half GEMM whose B-tile loader de-quantises the packed tiles.  Two steps of k and more, row
+    and column tails, groups of half a step, on tiles of 128 x 128; the last case runs 256 x 256 ones, those beyond a whole
+    round cut in half (checked on its first, a middle and the last columns)."""
     announce("w4a16 packed many rows", m, k, n, gs, offset)
     rng = np.random.default_rng(m + 3 * k + n)
     x, wp, sc, of = w4_case(rng, m, k, n, gs, offset is not None)
@@ -1153,8 +1153,8 @@ def test_w8a16_rows_beyond_thirty_two_bit_offsets():
 @pytest.mark.parametrize("mode", ["vector+offset", "vector", "scalar+offset"])
 @pytest.mark.parametrize("out_f32", [False, True])
 def test_w8a16_trans_b_many_rows(m, k, n, mode, out_f32):
-    """The half GEMM whose B-tile loader de-quantises [n, k] weights: two steps of k and more, row and column tails of
-    every tile shape, column counts that are no multiple of 4 (stored element by element) and of 2."""
+    """The half GEMM whose B-tile loader de-quantises [n, k] weights, on tiles of 128 x 128: two steps of k and more, row and
+    column tails, column counts that are no multiple of 4 (stored element by element) and of 2."""
     announce("w8a16 [n, k] many rows", m, k, n, mode, out_f32)
     rng = np.random.default_rng(m + k + n)
     x = rng.standard_normal((m, k)).astype(np.float16)
@@ -1170,6 +1170,39 @@ def test_w8a16_trans_b_many_rows(m, k, n, mode, out_f32):
     orc.set_threads(16)
     want = orc.matmul_w8a16(d, x, wt, None if per_tensor else of, None if per_tensor else sc)
     w8a16_check(y.cpu().numpy(), want, x, out_f32)
+
+
+@pytest.mark.parametrize("m,n", [(300, 24600), (384, 20480), (1300, 14600)])
+@pytest.mark.parametrize("kind,k", [("int8", k) for k in (64, 128, 192, 256, 320, 448)] + [("int4", k) for k in (128, 256, 384, 512)])
+@pytest.mark.parametrize("offset", [True, False])
+def test_half_gemm_on_tiles_of_256_columns(m, n, kind, k, offset):
+    """The half GEMM's tiles of 256 columns, whose loads go out in halves behind two counted waits a step: 256 x 256, 128 x 256, and
+    256 x 256 with the tiles beyond a whole round cut in half; one to eight K steps of 64 (prologue, steady state, the last step but one
+    and the last); row and column tails.  Whole numbers: the de-quantised weights are exact halves and every sum an exact float, so
+    the order of the sums does not matter and every element is compared, float and half outputs."""
+    announce("half GEMM, 256 columns", m, n, kind, k, offset)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + k)
+    x = torch.randint(-4, 5, (m, k), device=DEV, generator=g).to(torch.float16)
+    lo, hi = (-8, 7) if kind == "int4" else (-100, 100)
+    w = torch.randint(lo, hi + 1, (k, n), dtype=torch.int8, device=DEV, generator=g)
+    of = torch.randint(-3, 4, (n,), device=DEV, generator=g).to(torch.float16)
+    sc = torch.randint(1, 3, (n,), device=DEV, generator=g).to(torch.float16) * 0.5
+    # at most 512 * 4 * 103 in magnitude, in halves: exact in fp32
+    want = (x.double() @ ((w.double() + (of.double() if offset else 0.0)) * sc.double())).float()
+    outs = (torch.float16,) if kind == "int4" else (torch.float16, torch.float32)
+    for out in outs:
+        y = torch.full((m, n), 7.0, dtype=out, device=DEV)
+        if kind == "int4":
+            nibbles = (w & 15).to(torch.uint8).view(k, n // 2, 2)
+            packed = ops.pack_weight_w4((nibbles[..., 0] | (nibbles[..., 1] << 4)).contiguous(), k, n)
+            groups = k // 128
+            ops.matmul_w4a16_packed(y, x, packed, sc.expand(groups, n).contiguous(), of.expand(groups, n).contiguous() if offset else None, 128)
+        elif k % 128 == 0:
+            ops.matmul_w8a16(y, x, w.t().contiguous(), of if offset else None, sc, trans_b=True)
+        else:                        # ([n, k] weights take steps of 128; [k, n] ones are turned round and run the same tiles)
+            ops.matmul_w8a16(y, x, w, of if offset else None, sc)
+        assert torch.equal(y, want.clamp(-65504, 65504).to(out) if out == torch.float16 else want)
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])

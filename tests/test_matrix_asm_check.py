@@ -37,3 +37,13 @@ def body(*lines):
 ])
 def test_missing_waits_are_found(lines, wrong):
     assert bool(check.faults(body(*lines))) == wrong
+
+
+def test_loads_that_the_compiler_dropped_are_found():
+    """A counted wait of the half GEMM rests on a step's loads into LDS and into registers: a stretch between two barriers with
+    the first kind alone means that the compiler has left the second out."""
+    step = ["global_load_lds_dwordx4 v1, s[0:1]", "buffer_load_dwordx4 v[4:7], v2, s[4:7], 0 offen", "s_waitcnt vmcnt(6)", "s_barrier"]
+    assert check.dropped_loads(body(*step, *step, *step[2:])) == []          # whole steps, and one that loads nothing
+    assert len(check.dropped_loads(body(*step, *step[:1], *step[2:]))) == 1
+    # (a buffer load into LDS counts as such)
+    assert len(check.dropped_loads(body("buffer_load_dwordx4 v1, s[4:7], 0 offen lds", "s_barrier"))) == 1
