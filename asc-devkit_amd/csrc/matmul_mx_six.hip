@@ -301,10 +301,13 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
     const Stage T0{L0, L0 + kOperand, C0}, T1{L1, L1 + kOperand, C1}, T2{L2, L2 + kOperand, C2};
     {
         const Sources f0 = sources(0), f1 = sources(1), f2 = sources(2);
+        // (stage by stage: the waits count the loads behind the ones they are for)
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) load(f0, u, T0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) load(f1, u, T1);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < kNow; ++u) load(f2, u, T2);
     }

@@ -357,10 +357,17 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
     };
     {
         const auto from0 = bases(0u), from1 = bases(last < 1u ? last : 1u);
+        // (in this order: the waits count the loads behind the ones they are for)
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) load(from0, u, S0);
+        for (int u = 0; u < kLoads; ++u) {
+            load(from0, u, S0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) load(from1, u, S1);
+        for (int u = 0; u < kLoads; ++u) {
+            load(from1, u, S1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         arrive(std::integral_constant<int, 2 * kLoads - kMid>{});
     }
     // a wavefront whose rows all lie past the end of the tile's group skips the matrix work and only keeps the loads and
@@ -618,9 +625,10 @@ __device__ __forceinline__ void gemm_ring_body(const GemmParams& p, const TilePl
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    static_for<kStages>([&](auto st) {
+    static_for<kStages>([&](auto st) {  // (in this order: the waits count the loads behind the ones they are for)
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) load(decltype(st)::value, u, L[decltype(st)::value]);
+        __builtin_amdgcn_sched_barrier(0);
     });
     arrive(std::integral_constant<int, (kStages - 1) * kLoads>{});
 #pragma unroll
