@@ -179,7 +179,7 @@ int launch_gemm_dma_group(GemmParams& p, hipStream_t st)
     // 303 tokens, k = 3712, n = 1408 30.1 and 25.7; 8 experts, 4096 tokens, k = 4096, n = 14336 279 and 273; 16 experts, 500 tokens, k =
     // 2048, n = 4096 28.1 and 30.0; 32 experts, 1000 tokens, k = 1024, n = 4096 39.6 and 42.6.  (Few rows per group: hardly a big tile,
     // and the kernel without that form's code is 1 to 2 % ahead.)
-    const int form = gemm_dma_form(p);
+    const int form = p.k % BK != 0 ? k32Ragged : gemm_half_output(p) ? k16 : k32;
     if (form == k32Ragged) {
         gemm_dma_group_kernel<k32Ragged, k32Ragged><<<wgs, kThreads, 0, st>>>(p);
     } else if (form == k16 && p.k >= 3072u) {

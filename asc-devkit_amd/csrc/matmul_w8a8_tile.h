@@ -1239,18 +1239,27 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     }
 }
 
-// The matrix instruction of a call's 256-row tiles (smaller ones always run the 32 x 32 x 32 one): the 16 x 16 x 64 form moves
-// half the sums, which is what counts where the power limit sets the clock, and its loads have longer to arrive.
-// Outputs other than half and bfloat16 are what the other form writes from registers.  In us with the quantiser, 32 x 32 x 32
-// and 16 x 16 x 64: 2048 x 4096 x 11008 98.1 and 88.3; 2048 x 2048 x 5632 38.0 and 36.2; 1024 x 11008 x 4096 (64 tiles) 107.8 and
-// 103.9; 600 x 4096 x 4096 48.5 and 47.3; 4096 x 512 x 4096 21.3 and 21.2; 4096 x 256 x 8192 30.0 and 29.9.
+inline bool gemm_half_output(const GemmParams& p)
+{
+    return p.epi.quant_mode != ASCQ_MM_QUANT_NONE && (p.epi.out_dtype == ASCQ_F16 || p.epi.out_dtype == ASCQ_BF16);
+}
+
+// The matrix instruction of the plain matmul's 256-row tiles (its smaller ones run the 32 x 32 x 32 one, the ring tiles the other; grouped
+// tiles: launch_gemm_dma_group).  The 16 x 16 x 64 form moves half the sums, which is what counts where the power limit sets the
+// clock, and its loads have longer to arrive; but a tile starts with two stages of loads where the other form waits for one, and
+// its epilogue holds more code.  Time of the 16 x 16 x 64 form over the other's, geometric means of random calls of 513 to 8192 rows with
+// up to 64 / 65 to 512 / more tiles: k = 128 1.06 / 1.05 / 1.08, 512 1.03 / 1.00 / 1.03, 768 1.01 / 1.00 / 1.05, 896 1.01 / 0.98 /
+// 0.98, 1024 1.00 / 0.98 / 1.01, 1280 1.00 / 0.97 / 1.00, 1536 0.99 / 0.98 / 0.94, 2048 1.00 / 0.95, 4096 0.99 / 0.93 / 0.89.  In us
+// with the quantiser: 2048 x 4096 x 11008 98.1 and 88.3; 1024 x 11008 x 4096 (64 tiles) 107.8 and 103.9.  Outputs other than half and
+// bfloat16 are what the 32 x 32 x 32 form writes from registers.
 inline int gemm_dma_form(const GemmParams& p)
 {
     if (p.k % BK != 0) {
         return k32Ragged;
     }
-    const bool half = p.epi.quant_mode != ASCQ_MM_QUANT_NONE && (p.epi.out_dtype == ASCQ_F16 || p.epi.out_dtype == ASCQ_BF16);
-    return half ? k16 : k32;
+    const uint64_t tiles = static_cast<uint64_t>((p.m + 255u) / 256u) * ((p.n + 255u) / 256u), cus = device_compute_units();
+    const bool middle = 4u * tiles > cus && tiles <= 2u * cus;
+    return gemm_half_output(p) && p.k >= (middle ? 896u : 1536u) ? k16 : k32;
 }
 
 // The plain matmul: tile number `bid` of the launch (before the XCD remapping), column tiles counted from col_begin,

@@ -497,10 +497,10 @@ def gpu_mm(m, n, k, a, b, layout, kind, out, quant, tok, bias):
                                         (3136, 10000, "packed")])
 @pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu", "words", "shifts"])
 def test_w8a8_both_matrix_instructions_agree(k, n, layout, kind):
-    """Long sums in enough 256 x 256 tiles for the 16 x 16 x 64 instruction (5 x 40 of them, the last of 3 rows), against
-    the same rows in two calls of too few tiles for it: equal bits, whole and partial last steps, every weight layout,
-    the activations, quant words with and without the bit that shifts the accumulator.  The plain form also against
-    the sums in 64 bits."""
+    """Sums long enough for the 16 x 16 x 64 instruction in 256 x 256 tiles (5 x 40 of them, the last of 3 rows) to a 16-bit type,
+    against a float output, which the 32 x 32 x 32 instruction writes, rounded to that type: equal bits, whole and partial last
+    steps, every weight layout, the activations, quant words (those with the bit that shifts the accumulator: only against the
+    same rows in two calls).  The plain form also against the sums in 64 bits."""
     announce("w8a8 both instructions", k, n, layout, kind)
     g = torch.Generator(device=DEV)
     g.manual_seed(k + n)
@@ -523,6 +523,9 @@ def test_w8a8_both_matrix_instructions_agree(k, n, layout, kind):
     got = gpu_mm(m, n, k, a, w, layout, kind, out, quant, tok, bias)
     parts = [gpu_mm(hi - lo, n, k, a[lo:hi].clone(), w, layout, kind, out, quant, tok[lo:hi].clone(), bias) for lo, hi in ((0, cut), (cut, m))]
     assert torch.equal(got.view(torch.int16), torch.cat(parts).view(torch.int16))
+    if kind != "shifts":                     # (a half output rounds a shifted sum once more)
+        wide = gpu_mm(m, n, k, a, w, layout, kind, torch.float32, quant, tok, bias)
+        assert torch.equal(got.view(torch.int16), wide.to(out).view(torch.int16))
     if kind == "plain":
         acc = a.double() @ (b.double().t().contiguous() if layout == "nk" else b.double())      # exact: below 2^53
         want = (acc.float() * cs * tok[:, None] + bias).to(out)
@@ -555,6 +558,28 @@ def test_w8a8_large_tiles_with_half_outputs(m, n, k, layout):
         if want is None:
             want = (a.astype(np.float32) @ b.astype(np.float32)) * sc * tok[:, None]
         assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+
+
+@pytest.mark.parametrize("layout", ["kn", "nk", "packed"])
+@pytest.mark.parametrize("m,n,k", [(1030, 3344, 768), (1030, 3344, 896), (1030, 3344, 1024), (520, 528, 1408), (520, 528, 1536), (600, 264, 1664),
+                                   (2304, 14600, 1408), (2304, 14600, 1536)])
+def test_w8a8_half_outputs_on_both_sides_of_the_instruction_rule(m, n, k, layout):
+    """256-row tiles to half: 70 of them change to the 16 x 16 x 64 instruction at seven K steps, few (6) and many (more than
+    two rounds of the chip) at twelve; even and odd numbers of steps of both, against the sums in 64 bits."""
+    announce("instruction rule", m, n, k, layout)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n + k)
+    a = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    b = torch.randint(-127, 128, (n, k) if layout == "nk" else (k, n), dtype=torch.int8, device=DEV, generator=g)
+    w = ops.pack_weight_w8(b, k, n) if layout == "packed" else b
+    tok = torch.rand(m, device=DEV, generator=g) * 0.1 + 1e-3
+    cs = torch.rand(n, device=DEV, generator=g) * 1e-4 + 1e-5
+    bias = torch.randn(n, device=DEV, generator=g)
+    acc = a.double() @ (b.double().t().contiguous() if layout == "nk" else b.double())      # exact: below 2^53
+    want = acc.float() * cs * tok[:, None] + bias                                           # one rounding per step
+    for out in (torch.bfloat16, torch.float16):
+        got = gpu_mm(m, n, k, a, w, layout, "plain", out, cs, tok, bias)
+        assert torch.equal(got.view(torch.int16), want.to(out).view(torch.int16))
 
 
 @pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu"])
