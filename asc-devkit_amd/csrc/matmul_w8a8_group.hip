@@ -30,7 +30,7 @@ __device__ __forceinline__ void group_row_tiles(uint32_t rows, uint32_t& big, ui
 }
 
 // One phase of the grouped kernel's plan (see gemm_dma_group_kernel): the workgroup's ids that fall into it.
-template <uint32_t phase, int kForm>  // (kForm: of the phase's tiles)
+template <uint32_t phase, int kForm>
 __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const uint32_t* PLAN, const Stage& S0, const Stage& S1,
                                                      float* TS)
 {
@@ -109,7 +109,7 @@ __device__ __forceinline__ void gemm_dma_group_phase(const GemmParams& p, const 
 // run side by side.  The group sizes are known only on the device, so a launch sized by the host for the worst case
 // would consist mostly of workgroups with nothing to do; the loop has none.  gridDim.x must be a multiple of 8;
 // p.tiles_n = 256-wide tile columns of the whole matrix.
-template <int kForm, int kSmall>
+template <int kForm>
 __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams p)
 {
     ASCQ_DMA_STAGES(kForm, 256, 256);
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams 
     // one tile shape's code and registers.
     gemm_dma_group_phase<0, kForm>(p, PLAN, S0, S1, TS);
     gemm_dma_group_phase<1, kForm>(p, PLAN, S0, S1, TS);
-    gemm_dma_group_phase<2, kSmall>(p, PLAN, S0, S1, TS);
+    gemm_dma_group_phase<2, kForm>(p, PLAN, S0, S1, TS);
 }
 
 }  // namespace
@@ -174,20 +174,19 @@ int launch_gemm_dma_group(GemmParams& p, hipStream_t st)
         plan_note(ASCQ_MM_KERNEL_DMA_256, 256, 256, BK, wgs, 1, 2u * (256u * BK + BK * 256u) + 256u * 4u, 0);
         return ASCQ_OK;
     }
-    // The 16 x 16 x 64 form, whose loads have one and a half K steps to arrive, for the remainders too from k = 3072 on; with fewer steps
-    // a small tile's start, two stages of loads, counts for more.  In us, remainders in the 32 x 32 x 32 and the 16 x 16 x 64 form: 16 experts,
-    // 303 tokens, k = 3712, n = 1408 30.1 and 25.7; 8 experts, 4096 tokens, k = 4096, n = 14336 279 and 273; 16 experts, 500 tokens, k =
-    // 2048, n = 4096 28.1 and 30.0; 32 experts, 1000 tokens, k = 1024, n = 4096 39.6 and 42.6.  (Few rows per group: hardly a big tile,
-    // and the kernel without that form's code is 1 to 2 % ahead.)
-    const int form = p.k % BK != 0 ? k32Ragged : gemm_half_output(p) ? k16 : k32;
-    if (form == k32Ragged) {
-        gemm_dma_group_kernel<k32Ragged, k32Ragged><<<wgs, kThreads, 0, st>>>(p);
-    } else if (form == k16 && p.k >= 3072u) {
-        gemm_dma_group_kernel<k16, k16><<<wgs, kThreads, 0, st>>>(p);
-    } else if (form == k16 && p.m > 128u * p.groups) {
-        gemm_dma_group_kernel<k16, k32><<<wgs, kThreads, 0, st>>>(p);
+    // The 16 x 16 x 64 form's loads have one and a half K steps to arrive, but a tile starts with two stages of them: it
+    // takes long sums, shorter ones the more rows a group has.  Time of the 16 x 16 x 64 kernel over the 32 x 32 x 32 one's,
+    // geometric means of random calls with up to 128 / 129 to 256 / more rows per group: k = 256 1.14 / 1.05 / 1.05, 1024 1.05 / 1.03 /
+    // 0.99, 1280 1.02 / 1.02 / 0.98, 1408 1.02 / 0.98 / 0.99, 1536 1.03 / 0.98 / 0.96, 2048 0.99 / 0.97 / 0.95, 2560 0.94 / 0.95 / 0.94,
+    // 3584 0.90 / 0.89 / 0.91.  (Big tiles in the one form and remainders in the other were ahead of both nowhere by more than 1 %.)
+    const uint64_t rows = p.m, groups = p.groups;
+    const uint32_t long_k = rows > 256u * groups ? 1280u : rows > 128u * groups ? 1408u : 2560u;
+    if (p.k % BK != 0) {
+        gemm_dma_group_kernel<k32Ragged><<<wgs, kThreads, 0, st>>>(p);
+    } else if (gemm_half_output(p) && p.k >= long_k) {
+        gemm_dma_group_kernel<k16><<<wgs, kThreads, 0, st>>>(p);
     } else {
-        gemm_dma_group_kernel<k32, k32><<<wgs, kThreads, 0, st>>>(p);
+        gemm_dma_group_kernel<k32><<<wgs, kThreads, 0, st>>>(p);
     }
     return launch_status("ascq_group_matmul_w8a8");
 }

@@ -584,7 +584,8 @@ def test_w8a8_half_outputs_on_both_sides_of_the_instruction_rule(m, n, k, layout
 
 @pytest.mark.parametrize("kind", ["plain", "gelu", "swiglu"])
 def test_group_matmul_both_matrix_instructions_agree(kind):
-    """The grouped matmul at a size for the 16 x 16 x 64 instruction against the plain matmul of each group's rows."""
+    """The grouped matmul at a size for the 16 x 16 x 64 instruction against the plain matmul of each group's rows to a float
+    output, which the 32 x 32 x 32 instruction writes, rounded to the grouped one's type."""
     announce("grouped matmul, both instructions", kind)
     g = torch.Generator(device=DEV)
     g.manual_seed(3)
@@ -602,17 +603,18 @@ def test_group_matmul_both_matrix_instructions_agree(kind):
     for i, c in enumerate(counts):
         if c:
             rows = slice(first, first + c)
-            want = gpu_mm(c, n, k, x[rows].clone(), w[i], "kn", kind, torch.bfloat16, cs[i].clone(), tok[rows].clone(), bias[i].clone())
-            assert torch.equal(y[rows].view(torch.int16), want.view(torch.int16)), i
+            want = gpu_mm(c, n, k, x[rows].clone(), w[i], "kn", kind, torch.float32, cs[i].clone(), tok[rows].clone(), bias[i].clone())
+            assert torch.equal(y[rows].view(torch.int16), want.to(torch.bfloat16).view(torch.int16)), i
         first += c
 
 
-@pytest.mark.parametrize("k", [256, 384, 3072, 3200])
+@pytest.mark.parametrize("k", [256, 384, 1280, 1408, 2432, 2560, 3072, 3200])
 @pytest.mark.parametrize("nz", [False, True])
-@pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 256, 16, 480, 385]])
+@pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 256, 16, 480, 385], [257, 512, 64, 384]])
 def test_group_matmul_remainders_in_both_forms(counts, nz, k):
-    """Remainders of 64 and of 128 rows, and big tiles whose second wavefront row is empty, partly filled or full; from k =
-    3072 on in the form whose loads are spread over a step and a half; even and odd numbers of K steps."""
+    """Remainders of 64 and of 128 rows, and big tiles whose second wavefront row is empty, partly filled or full, on both
+    sides of the rule that names the instruction: from k = 2560, 1408 and 1280 on (84, 216 and 304 rows per group) the form
+    whose loads are spread over a step and a half; even and odd numbers of K steps."""
     announce("group remainders", counts, nz, k)
     rng = np.random.default_rng(k + len(counts) + nz)
     g, m, n = len(counts), sum(counts), 544
