@@ -120,6 +120,11 @@ __global__ __launch_bounds__(256) void mx_widen_e1m2_kernel(MxWidenParams p)
     }
 }
 
+// How a tile is stored: 16-bit or float rows of a multiple of 4 values, anything else.  A kernel each, and a loop for each 16-bit type: the
+// epilogue runs once per tile, so the way of its instructions from memory is part of its time.  (One kernel, both 16-bit
+// conversions in one loop: 2048 x 2048 x 512 to bfloat16 15.4 us, 14.2 like this, to half 18.7 and 16.3.)
+constexpr int kStoreHalf = 0, kStoreFloat = 1, kStoreAny = 2;
+
 struct MxSixParams {
     const uint8_t *a, *b, *sa, *sb;  // as written by mx_widen_e1m2_kernel
     MxParams out;                    // c, bias, m, n, k, tiles, output type
@@ -147,6 +152,7 @@ __device__ __forceinline__ void six_mfma(f32x4& d, const v6i& a, const v6i& b, u
                  : "v"(a), "v"(b), "v"(sa), "v"(sb), "n"(al), "n"(bl), "n"(ah), "n"(bh));
 }
 
+template <int kStore>
 __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
 {
     const MxParams& p = q.out;
@@ -357,30 +363,97 @@ __global__ __launch_bounds__(512, 1) void mx_six_kernel(MxSixParams q)
         const uint32_t col = colw + j * 16u + lc;
         bias[j] = (p.bias != nullptr && col < p.n) ? p.bias[col] : 0.0f;
     }
-    if (p.out_dtype != ASCQ_F32 && p.n % 4u == 0) {
-        // A 4 x 4 transposition inside each four neighbouring lanes (two exchanges of packed pairs) leaves lane b of the four with
-        // columns 4 (l / 4) .. + 3 of block b: one 8-byte store per lane and row, a full 128-byte line per 16 lanes.
-        const bool b0 = (lane & 1u) != 0, b1 = (lane & 2u) != 0, bf16 = p.out_dtype == ASCQ_BF16;
-        const uint32_t col = colw + 16u * (lane & 3u) + (lc & 12u);
+    // Rows of an even number of values: transpositions inside neighbouring lanes.  After one exchange a lane has two adjacent columns
+    // of blocks l % 2 (`lo`) and 2 + l % 2 (`hi`) each, after a second one, n a multiple of 4, lane b of four has columns 4 (l / 4)
+    // .. + 3 of block b, and the 16 lanes of a row store whole lines of its 64 columns.  (A wavefront's 128 stores of single elements take
+    // 13 us: 2048 x 2050 x 512 to bfloat16 32.3 -> 16.4 us, 636 x 3728 x 1024 to float 31.8 -> 17.0.)
+    const bool b0 = (lane & 1u) != 0, b1 = (lane & 2u) != 0, bf16 = p.out_dtype == ASCQ_BF16;
+    const uint32_t col4 = colw + 16u * (lane & 3u) + (lc & 12u), col2 = colw + 16u * (lane & 1u) + (lc & 14u);
+    auto exchange = [](uint32_t give, auto by) __attribute__((always_inline)) {  // with lane ^ by
+        return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(give), decltype(by)::value == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true));
+    };
+    constexpr std::integral_constant<int, 1> by1{};
+    constexpr std::integral_constant<int, 2> by2{};
+    auto each_row = [&](auto&& store) __attribute__((always_inline)) {  // store(row, the row's sum in block j, j = 0 .. 3)
         six_static_for<32>([&](auto c) {
             constexpr int i = decltype(c)::value / 4, r = decltype(c)::value % 4;
-            const uint32_t row = row0 + (wm * 8u + i) * 16u + 4u * lq + r;
-            uint32_t h[4];
-            six_static_for<4>([&](auto jj) {
-                constexpr int j = decltype(jj)::value;
-                const float v = acc[i][j][r] + bias[j];
-                h[j] = bf16 ? f32_to_bf16_bits(v) : f32_to_half_bits_sat(v);
+            store(row0 + (wm * 8u + i) * 16u + 4u * lq + r, [&](int j) __attribute__((always_inline)) { return acc[i][j][r] + bias[j]; });
+        });
+    };
+    auto half_pairs = [&](auto to_bf16, auto&& value, uint32_t& lo, uint32_t& hi) __attribute__((always_inline)) {
+        uint32_t h[4];
+        six_static_for<4>([&](auto jj) {
+            constexpr int j = decltype(jj)::value;
+            const float v = value(j);
+            h[j] = decltype(to_bf16)::value ? f32_to_bf16_bits(v) : f32_to_half_bits_sat(v);
+        });
+        const uint32_t got = exchange(b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16), by1);
+        lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
+        hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
+    };
+    auto float_pairs = [&](auto&& value, u32x2& lo, u32x2& hi) __attribute__((always_inline)) {
+        uint32_t w[4];
+        six_static_for<4>([&](auto jj) { w[decltype(jj)::value] = __builtin_bit_cast(uint32_t, value(decltype(jj)::value)); });
+        const uint32_t got0 = exchange(b0 ? w[0] : w[1], by1), got1 = exchange(b0 ? w[2] : w[3], by1);
+        lo = b0 ? u32x2{got0, w[1]} : u32x2{w[0], got0};
+        hi = b0 ? u32x2{got1, w[3]} : u32x2{w[2], got1};
+    };
+    uint16_t* const half_out = static_cast<uint16_t*>(p.c);
+    float* const float_out = static_cast<float*>(p.c);
+    if constexpr (kStore == kStoreHalf) {
+        auto store_all = [&](auto to_bf16) __attribute__((always_inline)) {
+            each_row([&](uint32_t row, auto&& value) __attribute__((always_inline)) {
+                uint32_t lo, hi;
+                half_pairs(to_bf16, value, lo, hi);
+                const uint32_t got = exchange(b1 ? lo : hi, by2);
+                if (row < p.m && col4 < p.n) {
+                    __builtin_nontemporal_store(b1 ? u32x2{got, hi} : u32x2{lo, got},
+                                                reinterpret_cast<u32x2*>(half_out + static_cast<size_t>(row) * p.n + col4));
+                }
             });
-            const uint32_t give = b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16);
-            const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-            const uint32_t lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
-            const uint32_t hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
-            const uint32_t got2 = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(b1 ? lo : hi), 0x4E, 0xF, 0xF, true));  // lane ^ 2
-            if (row < p.m && col < p.n) {
-                __builtin_nontemporal_store(b1 ? u32x2{got2, hi} : u32x2{lo, got2},
-                                            reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.c) + static_cast<size_t>(row) * p.n + col));
+        };
+        if (bf16) {
+            store_all(std::true_type{});
+        } else {
+            store_all(std::false_type{});
+        }
+        return;
+    }
+    if constexpr (kStore == kStoreFloat) {
+        each_row([&](uint32_t row, auto&& value) __attribute__((always_inline)) {
+            u32x2 lo, hi;
+            float_pairs(value, lo, hi);
+            const uint32_t got0 = exchange(b1 ? lo[0] : hi[0], by2), got1 = exchange(b1 ? lo[1] : hi[1], by2);
+            if (row < p.m && col4 < p.n) {
+                __builtin_nontemporal_store(b1 ? u32x4{got0, got1, hi[0], hi[1]} : u32x4{lo[0], lo[1], got0, got1},
+                                            reinterpret_cast<u32x4*>(float_out + static_cast<size_t>(row) * p.n + col4));
             }
         });
+        return;
+    }
+    if (p.n % 2u == 0) {
+        auto store = [&](uint32_t row, auto* out, auto lo, auto hi) __attribute__((always_inline)) {
+            auto* const at = out + static_cast<size_t>(row) * p.n + col2;
+            if (row < p.m && col2 < p.n) __builtin_nontemporal_store(lo, reinterpret_cast<decltype(lo)*>(at));
+            if (row < p.m && col2 + 32u < p.n) __builtin_nontemporal_store(hi, reinterpret_cast<decltype(hi)*>(at + 32));
+        };
+        if (p.out_dtype == ASCQ_F32) {
+            each_row([&](uint32_t row, auto&& value) __attribute__((always_inline)) {
+                u32x2 lo, hi;
+                float_pairs(value, lo, hi);
+                store(row, float_out, lo, hi);
+            });
+        } else {
+            each_row([&](uint32_t row, auto&& value) __attribute__((always_inline)) {
+                uint32_t lo, hi;
+                if (bf16) {
+                    half_pairs(std::true_type{}, value, lo, hi);
+                } else {
+                    half_pairs(std::false_type{}, value, lo, hi);
+                }
+                store(row, half_out, lo, hi);
+            });
+        }
         return;
     }
     six_static_for<128>([&](auto c) {
@@ -426,7 +499,14 @@ int launch_mx_six(const MxParams& p, void* workspace, hipStream_t st)
     MxSixParams q{w.dst[0], w.dst[1], w.scale_dst[0], w.scale_dst[1], p};
     q.out.tiles_m = (p.m + 255u) / 256u;
     q.out.tiles_n = (p.n + 255u) / 256u;
-    mx_six_kernel<<<(q.out.tiles_m * q.out.tiles_n + 7u) / 8u * 8u, 512, 0, st>>>(q);
+    const uint32_t grid = (q.out.tiles_m * q.out.tiles_n + 7u) / 8u * 8u;
+    if (p.n % 4u != 0) {
+        mx_six_kernel<kStoreAny><<<grid, 512, 0, st>>>(q);
+    } else if (p.out_dtype == ASCQ_F32) {
+        mx_six_kernel<kStoreFloat><<<grid, 512, 0, st>>>(q);
+    } else {
+        mx_six_kernel<kStoreHalf><<<grid, 512, 0, st>>>(q);
+    }
     return launch_status("ascq_matmul_mx (e1m2)");
 }
 

@@ -156,6 +156,25 @@ def test_mx_e1m2_tiles_step_counts_and_outputs(steps, more, n, out):
         assert np.all(np.abs(got[r0:r1] - want) <= half_ulp * 1.01 * np.abs(want) + 4e-6 * (dot + np.abs(bv)) + 2.0 ** -24)
 
 
+@pytest.mark.parametrize("n", [2104, 2106, 2108, 2110])
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16, torch.float16])
+def test_mx_e1m2_tiles_store_every_row_length(n, out):
+    """Rows of a multiple of four values, and of two, stored four and two at a time: the bits of the same columns of a product
+    with one more, which is stored one by one (and compared with the golden above).  Large scales: halves saturate."""
+    m, k, more = 2100, 384, 2111
+    announce("mx e1m2 stores", n, out)
+    rng = np.random.default_rng(n)
+    a, b, sa, sb, bv = mx_case(rng, m, more, k, F1, F1, sk=16, bias=True)
+    if out == torch.float16:
+        sb[::5] = np.maximum(sb[::5], 140)
+    want = run_mx(m, more, k, a, b, sa, sb, F1, F1, bias=bv)[:, :n]
+    if out == torch.float16:
+        assert (want.abs() > 65504.0).any()
+        want = want.clamp(-65504.0, 65504.0)
+    got = run_mx(m, n, k, a, np.ascontiguousarray(b[:n]), sa, np.ascontiguousarray(sb[:n]), F1, F1, out=out, bias=np.ascontiguousarray(bv[:n]))
+    assert torch.equal(got, want.to(out))
+
+
 @pytest.mark.parametrize("fa,fb", [(a, b) for a in (E4, E5, F2, F1) for b in (E4, E5, F2, F1)])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 40, 160), (16, 33, 1088), (17, 64, 640), (32, 4112, 256), (33, 100, 2304),
                                    (64, 48, 4096), (65, 32, 1056)])
