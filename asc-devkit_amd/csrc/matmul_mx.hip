@@ -517,11 +517,14 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
 // Tile shapes (64 rows and more): whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.
 // Both times are estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
 // meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 1.85 (8-bit b), 0.95 (the 32-row
-// form), 2.0 (two 4-bit operands, one of them e1m2).  Tiles: rounds of 256 x 256 tiles, 1.3
-// per K step (0.85 for two e1m2 operands), and the passes that widen 4-bit operands, 1 per 3 MB of their codes.  Measured at n = k = 8192, decode
+// form), 2.0 (e1m2 beside e2m1).  Tiles: rounds of 256 x 256 tiles, 1.3 per K step, and the passes that widen 4-bit operands, 1 per 3 MB
+// of their codes.  Measured at n = k = 8192, decode
 // against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 20.7 and 78; 128 rows e4m3 34 and 79; 256 rows e2m1 41 and 47, e4m3 64 and
-// 85; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44; n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147; two e1m2
-// operands: 874 x 2000 x 8960 75 and 63, 200 x 14336 x 4096 56 and 46, 300 x 8192 x 4096 53 and 45.
+// 85; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44; n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147.
+// Two e1m2 operands have constants of their own, fits to 500 random calls of 64 to 3000 rows (decode and tiles within 7 and 11 % for eight in ten): a
+// round of decode workgroups also takes 3.6 to start and store, a K step of tiles 0.6 and as much again as the chip fills up; rows of an odd number
+// of values are stored one by one, 16.5 a round (636 x 3729 x 1024 26.6 and 34.7, 636 x 3728 x 1024 26.1 and 17.6; 165 x
+// 12032 x 640 25.4 and 16.3; 874 x 2000 x 8960 75 and 63).
 bool mx_decode_preferred(const MxParams& p)
 {
     const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
@@ -530,11 +533,17 @@ bool mx_decode_preferred(const MxParams& p)
     const double cus = device_compute_units();
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
+    const double decode_rounds = rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u));
+    const double blocks = static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN);
+    if (six) {
+        const double filled = blocks < cus ? blocks / cus : 1.0, store = p.n % 2u != 0 ? 16.5 : 0.0;
+        return 1.7 + decode_rounds * (1.73 * p.k / 1024.0 + 3.6) <
+               11.9 + 0.137e-6 * (static_cast<double>(p.m) + p.n) * p.k + rounds(blocks) * (0.6 * (1.0 + filled) * p.k / 128.0 + store);
+    }
     const double per_k = two4 ? 1.15 : b8 ? 1.85 : a8 ? 0.95 : 2.0;
-    const double decode = 4.0 + rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u)) * per_k * p.k / 1024.0;
+    const double decode = 4.0 + decode_rounds * per_k * p.k / 1024.0;
     const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
-    const double tiles = 5.0 + widen + rounds(static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN)) * (six ? 0.85 : 1.3) *
-                                           p.k / (two4 ? 256.0 : 128.0);
+    const double tiles = 5.0 + widen + rounds(blocks) * 1.3 * p.k / (two4 ? 256.0 : 128.0);
     return decode < tiles;
 }
 

@@ -156,6 +156,21 @@ def test_mx_e1m2_tiles_step_counts_and_outputs(steps, more, n, out):
         assert np.all(np.abs(got[r0:r1] - want) <= half_ulp * 1.01 * np.abs(want) + 4e-6 * (dot + np.abs(bv)) + 2.0 ** -24)
 
 
+@pytest.mark.parametrize("m,n,k", [(636, 3729, 1024), (636, 3728, 1024), (165, 12032, 640), (100, 4096, 512), (924, 1793, 1408)])
+def test_mx_e1m2_pairs_on_both_sides_of_the_estimate(m, n, k):
+    """Sizes whose time the few-row kernel and the tiles share out by an estimate: an odd number of columns more or less, few
+    rows with a short k, both against the golden's first, middle and last rows."""
+    announce("mx e1m2 estimate", m, n, k)
+    rng = np.random.default_rng(m + n + k)
+    a, b, sa, sb, _ = mx_case(rng, m, n, k, F1, F1, sk=max(16, (k // 32 + 7) // 8 * 8))
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sa.shape[1], a_format=F1, b_format=F1, out_dtype=abi.F32, has_bias=0)
+    got = run_mx(m, n, k, a, b, sa, sb, F1, F1).cpu().numpy()
+    orc.set_threads(16)
+    for r0, r1 in ((0, 6), (60, 68), (m - 5, m)):
+        want = orc.matmul_mx(d, a, b, sa, sb, rows=(r0, r1))[r0:r1]
+        mx_check(got[r0:r1], want, mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, F1, F1), False)
+
+
 @pytest.mark.parametrize("n", [2104, 2106, 2108, 2110])
 @pytest.mark.parametrize("out", [torch.float32, torch.bfloat16, torch.float16])
 def test_mx_e1m2_tiles_store_every_row_length(n, out):
