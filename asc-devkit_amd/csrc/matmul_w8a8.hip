@@ -123,8 +123,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int8_t* __r
         bptr = B + static_cast<size_t>(kb * 16u) * N + col;
     }
 
-    // kFull: the whole 128-byte K step is inside [k_begin, k_end): plain loads.  Otherwise loads are clamped to the
-    // last valid 16 bytes / row and the out-of-range part is replaced by zeros (selects, no branches).
+    // kFull: the whole 128-byte K step is inside [k_begin, k_end): plain loads.  Otherwise what lies past k_end is read
+    // from the start of its row / from row 0 (k may be as short as 16, so not even the first step has to hold it) and
+    // replaced by zeros (selects, no branches).
     auto load_global = [&](uint32_t k0, auto full_tag) {
         constexpr bool kFull = decltype(full_tag)::value;
 #pragma unroll
@@ -134,7 +135,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int8_t* __r
                 areg[i] = *reinterpret_cast<const u32x4*>(aptr[i] + k0);
             } else {
                 const bool ok = kk < k_end;
-                u32x4 v = *reinterpret_cast<const u32x4*>(aptr[i] + (ok ? k0 : 0u));
+                u32x4 v = *reinterpret_cast<const u32x4*>(aptr[i] - (kk - k0) + (ok ? kk : 0u));
                 areg[i] = ok ? v : u32x4{0u, 0u, 0u, 0u};
             }
         }
@@ -146,7 +147,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int8_t* __r
                     bregT[i] = *reinterpret_cast<const u32x4*>(bptrT[i] + k0);
                 } else {
                     const bool ok = kk < k_end;
-                    u32x4 v = *reinterpret_cast<const u32x4*>(bptrT[i] + (ok ? k0 : 0u));
+                    u32x4 v = *reinterpret_cast<const u32x4*>(bptrT[i] - (kk - k0) + (ok ? kk : 0u));
                     bregT[i] = ok ? v : u32x4{0u, 0u, 0u, 0u};
                 }
             }
@@ -155,12 +156,11 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int8_t* __r
             for (int i = 0; i < 16; ++i) {
                 const uint32_t kk = k0 + kb * 16u + i;
                 bool ok = true;
-                size_t roff = static_cast<size_t>(k0 + i) * N;
+                const int8_t* src = bptr + static_cast<size_t>(k0 + i) * N;
                 if constexpr (!kFull) {
                     ok = kk < k_end;
-                    roff = ok ? roff : 0;   // row kb*16 of the first step: always valid memory
+                    src = bptr - static_cast<size_t>(kb * 16u) * N + (ok ? static_cast<size_t>(kk) * N : 0u);
                 }
-                const int8_t* src = bptr + roff;
                 if constexpr (T::kCols == 8) {
                     u32x2 v = *reinterpret_cast<const u32x2*>(src);
                     breg[i][0] = ok ? v[0] : 0u;

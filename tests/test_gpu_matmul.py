@@ -1379,6 +1379,36 @@ def test_w8a8_ragged_sizes_on_the_tile_kernels(m, k, n):
     assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("k", [16, 48, 112, 144])
+@pytest.mark.parametrize("m,n,layout", [(33, 1376, "nk"), (300, 640, "nk"), (16, 1376, "nk"), (40, 248, "kn"), (600, 24, "kn"), (17, 136, "kn"), (24, 40, "group")])
+def test_staged_kernel_reads_nothing_past_its_operands(m, n, k, layout):
+    """The register-staged kernel with a k below, or just above, its K step of 128: both operands end where their allocation
+    ends (whole multiples of 2 MiB), so a piece past k must not be fetched from behind the last row."""
+    announce("staged, short k", m, n, k, layout)
+    def at_the_end(t):
+        room = torch.zeros(32 << 20, dtype=torch.int8, device=DEV)
+        tail = room[room.numel() - t.numel():].view(t.shape)
+        tail.copy_(t)
+        return tail
+    rng = np.random.default_rng(m + n + k)
+    a, b = rand_i8(rng, (m, k)), rand_i8(rng, (k, n))
+    if a.size % 16 or b.size % 16:
+        pytest.skip("the operands would not be 16-byte aligned")
+    want = (a.astype(np.int64) @ b.astype(np.int64)).astype(np.int32)
+    if layout == "group":
+        w = at_the_end(torch.from_numpy(b).view(1, k, n))
+        y = torch.zeros((m, n), dtype=torch.float32, device=DEV)
+        ops.quant_group_matmul(y, at_the_end(torch.from_numpy(a)), w, torch.tensor([m], dtype=torch.int64, device=DEV), torch.ones((1, n), device=DEV))
+        assert np.array_equal(y.cpu().numpy(), want.astype(np.float32))
+        return
+    mm = ops.Matmul(m, n, k, trans_b=layout == "nk")
+    mm.set_tensor_a(at_the_end(torch.from_numpy(a)))
+    mm.set_tensor_b(at_the_end(torch.from_numpy(np.ascontiguousarray(b.T) if layout == "nk" else b)))
+    c = torch.zeros((m, n), dtype=torch.int32, device=DEV)
+    mm.iterate_all(c)
+    assert np.array_equal(c.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("m", [1, 4, 5, 16, 17, 32])
 @pytest.mark.parametrize("k,n", [(128, 65), (132, 257), (1000, 1023), (6784, 515), (512, 2050)])
 def test_w8a8_few_rows_on_unaligned_columns(m, k, n):
