@@ -79,13 +79,14 @@ __device__ __forceinline__ uint32_t pair_of_i4(uint32_t q, int c, f16x2 sc, f16x
 // read of one piece, and four neighbouring lines all 32 banks that a write sees at a time in two pieces four apart.
 __device__ __forceinline__ uint32_t wq_swizzle(uint32_t line) { return ((line >> 1) & 7u) ^ ((line & 1u) << 1); }
 
-// One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
-// wavefront owns BM / kWM rows by 64 columns.
+// One of the two LDS stages of a tile.
 struct WqStage {
     char* a[2];  // the first and the second half of every wavefront's rows: distinct arrays, like the stages
     char* b;
 };
 
+// One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
+// wavefront owns BM / kWM rows by 64 columns.
 template <int BM, int BN, bool kInt4, bool kOff>
 __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32_t n0, const WqStage& S0, const WqStage& S1)
 {
@@ -325,15 +326,22 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
         }, std::integral_constant<int, kMore && kParts == 4 ? 3 : -1>{}, next, Y.b, std::integral_constant<int, 0>{}, [](int) {});
         if constexpr (kMore) {
             arrive(std::integral_constant<int, !kMid ? 0 : !kSteady ? kHalf + kPartAll : kInt4 ? kHalf + kEarly : kAInstr + kPartAll>{});
-            quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
-                first_operands(Y, decltype(r)::value);
-            }, std::integral_constant<int, kSteady ? 0 : -1>{}, next2, X.b, late, [&](int u) __attribute__((always_inline)) {
+            auto late_load = [&](int u) __attribute__((always_inline)) {
                 if (u < kRowsLate) {
                     load_rows(base, kAInstr - kRowsLate + u, X);
                 } else {
                     fetch(next, s + 3u, kFetches - 1);
                 }
-            });
+            };
+            // (BN = 128: a step is as long as its loads' way from memory, so they all go out at once.  One behind every other matrix
+            // instruction: w8a16 108 x 8064 x 18496 97.6 -> 106.3 us, 1509 x 10752 x 1664 105.7 -> 116.8, int4 49 x 6272 x 20480 70.5 -> 76.7)
+            constexpr int kAtOnce = kMid ? 0 : decltype(late)::value;
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) late_load(u);
+            __builtin_amdgcn_sched_barrier(0);
+            quarter(std::integral_constant<int, 3>{}, std::integral_constant<int, NH + TJ>{}, [&](auto r) __attribute__((always_inline)) {
+                first_operands(Y, decltype(r)::value);
+            }, std::integral_constant<int, kSteady ? 0 : -1>{}, next2, X.b, std::integral_constant<int, decltype(late)::value - kAtOnce>{}, late_load);
         } else {
             wq_for<kM>([&](auto n) { mfma(3, decltype(n)::value); });
         }
