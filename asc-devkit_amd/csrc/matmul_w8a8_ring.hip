@@ -15,7 +15,7 @@
 namespace ascq {
 namespace {
 
-template <int BM, int BN, int kStages, int kB>
+template <int BM, int BN, int kStages, int kB, int kForm>
 __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(GemmParams p)
 {
     constexpr int kBytes = (BM + BN) * BK, kOther = 16;
@@ -33,7 +33,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(GemmParams p)
     char* const all[8] = {L0, L1, L2, L3, L4, L5, L6, L7};
     char* ring[kStages];
     static_for<kStages>([&](auto i) { ring[decltype(i)::value] = all[decltype(i)::value]; });
-    gemm_dma_tile_at<BM, BN, false, false, kB, kRing>(p, at, 0u, TS, ring);
+    gemm_dma_tile_at<BM, BN, false, false, kB, kForm>(p, at, 0u, TS, ring);
+}
+
+template <int BM, int BN, int kStages, int kB>
+void run_ring(const GemmParams& q, uint32_t grid, hipStream_t st)
+{
+    if (gemm_half_output(q) && q.epi.activation != ASCQ_MM_ACT_SWIGLU && q.epi.scale_format == ASCQ_MM_SCALE_F32) {
+        gemm_ring_kernel<BM, BN, kStages, kB, kRingHalf><<<grid, kThreads, 0, st>>>(q);
+    } else {
+        gemm_ring_kernel<BM, BN, kStages, kB, kRing><<<grid, kThreads, 0, st>>>(q);
+    }
 }
 
 template <int BM, int BN, int kStages>
@@ -44,11 +54,11 @@ void run_ring(const GemmParams& p, int b_layout, hipStream_t st)
     q.tiles_n = (p.n + BN - 1u) / BN;
     const uint32_t grid = (q.tiles_m * q.tiles_n + 7u) / 8u * 8u;
     if (b_layout == 2) {
-        gemm_ring_kernel<BM, BN, kStages, 2><<<grid, kThreads, 0, st>>>(q);
+        run_ring<BM, BN, kStages, 2>(q, grid, st);
     } else if (b_layout == 1) {
-        gemm_ring_kernel<BM, BN, kStages, 1><<<grid, kThreads, 0, st>>>(q);
+        run_ring<BM, BN, kStages, 1>(q, grid, st);
     } else {
-        gemm_ring_kernel<BM, BN, kStages, 0><<<grid, kThreads, 0, st>>>(q);
+        run_ring<BM, BN, kStages, 0>(q, grid, st);
     }
 }
 

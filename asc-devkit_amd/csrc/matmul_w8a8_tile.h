@@ -37,8 +37,10 @@ constexpr int BK = 128;
 
 // The forms of a tile: its matrix instruction (gemm_dma_form says which one runs where), and whether k may end inside a
 // step.  Looking for that step costs about 1 % (600 x 4096 x 4096 43.5 -> 43.9 us), so it is a form of its own.
-// kRing: small tiles with a ring of stages (matmul_w8a8_ring.hip).
-constexpr int k16 = 16, k32 = 32, k32Ragged = 33, kRing = 64;
+// kRing: small tiles with a ring of stages (matmul_w8a8_ring.hip), every output; kRingHalf: those to half or bfloat16, one value per
+// column and no quant words (a tile is short enough to notice what else its kernel holds: 729 x 4304 x 1152 20.0 us with every output's code).
+constexpr int k16 = 16, k32 = 32, k32Ragged = 33, kRing = 64, kRingHalf = 65;
+constexpr bool ring_form(int form) { return form == kRing || form == kRingHalf; }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* gptr_t;
@@ -539,7 +541,8 @@ __device__ __forceinline__ void gemm_dma_body16(const GemmParams& p, const TileP
 
 // The body of a small tile: a ring of kStages LDS stages of a K step each, loads that are issued kStages - 1/2 steps ahead
 // (see matmul_w8a8_ring.hip).  load(step, u, stage): load u of the wavefront's kLoads of a step; past the end it brings zeros.
-template <int BM, int BN, int kB, int kStages, int kLoads, class Load>
+// kHalf: see kRingHalf.
+template <int BM, int BN, int kB, int kStages, int kLoads, bool kHalf, class Load>
 __device__ __forceinline__ void gemm_ring_body(const GemmParams& p, const TilePlace& at, uint32_t n0, uint32_t steps, uint32_t wave,
                                                uint32_t lane, Load&& load, char* const (&L)[kStages], float* TS)
 {
@@ -677,53 +680,117 @@ __device__ __forceinline__ void gemm_ring_body(const GemmParams& p, const TilePl
         asm volatile("" : "+v"(q[j].s), "+v"(bias_post[j]), "+v"(bias_pre[j]));  // (waited for once, not at every store)
     }
     bool shifts = false;  // quant words that shift the accumulator first (rare): element by element
-    if (e.scale_format == ASCQ_MM_SCALE_U64) {
+    if (!kHalf && e.scale_format == ASCQ_MM_SCALE_U64) {
         int any = 0;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) any |= q[j].ctl;
         shifts = __builtin_amdgcn_ballot_w64((any & 2) != 0) != 0;
     }
-    const bool half_out = e.quant_mode != ASCQ_MM_QUANT_NONE && (e.out_dtype == ASCQ_BF16 || e.out_dtype == ASCQ_F16);
-    if (half_out && !shifts && e.activation != ASCQ_MM_ACT_SWIGLU) {
+    const bool quantised = kHalf || e.quant_mode != ASCQ_MM_QUANT_NONE, half_out = kHalf || (quantised && (e.out_dtype == ASCQ_BF16 || e.out_dtype == ASCQ_F16));
+    const bool wide_out = !quantised || e.out_dtype == ASCQ_F32;  // four bytes: raw sums or floats
+    if (kHalf || (!shifts && (half_out || wide_out))) {
+        // (Element by element, a lane's choices made at run time, 364 x 1024 x 7000 with SwiGLU to float took 21.0 us and 829 x 592 x
+        // 5120 to float 31.9; 14.0 and 18.4 like this.)
         const bool b0 = (lane & 1u) != 0, b1 = (lane & 2u) != 0, post = e.bias_kind >= ASCQ_MM_BIAS_F32_POST;
         const bool gelu = e.activation == ASCQ_MM_ACT_FASTER_GELU, bf16 = e.out_dtype == ASCQ_BF16;
-        static_for<NA>([&](auto ii) {
-            constexpr int i = decltype(ii)::value;
-            const uint32_t lbase = (wm * NA + i) * 16u + 4u * lq;
-            const f32x4 tok4 = *reinterpret_cast<const f32x4*>(&TS[lbase]);
-            static_for<4>([&](auto rr) {
-                constexpr int r = decltype(rr)::value;
-                const uint32_t row = at.row0 + lbase + r;
-                uint32_t h[TJ];
-                static_for<TJ>([&](auto jj) {
-                    constexpr int j = decltype(jj)::value;
-                    float v = static_cast<float>(acc[i][j][r] + bias_pre[j]) * q[j].s;
-                    v = v * tok4[r];  // 1.0f without a token scale: an exact identity
-                    v = post ? v + bias_post[j] : v;
-                    v = gelu ? faster_gelu(v) : v;
-                    h[j] = bf16 ? to_bits16<ASCQ_BF16>(v) : to_bits16<ASCQ_F16>(v);
+        const bool pairs = !kHalf && quantised && e.activation == ASCQ_MM_ACT_SWIGLU;
+        auto value = [&](int i, int j, int r, float tok) __attribute__((always_inline)) {
+            float v = static_cast<float>(acc[i][j][r] + bias_pre[j]) * q[j].s;
+            v = v * tok;  // 1.0f without a token scale: an exact identity
+            return post ? v + bias_post[j] : v;
+        };
+        auto bits16 = [&](float v) __attribute__((always_inline)) { return bf16 ? to_bits16<ASCQ_BF16>(v) : to_bits16<ASCQ_F16>(v); };
+        auto swap1 = [](uint32_t v) __attribute__((always_inline)) { return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xF, 0xF, true)); };  // lane ^ 1
+        auto swap2 = [](uint32_t v) __attribute__((always_inline)) { return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xF, 0xF, true)); };  // lane ^ 2
+        // every 4 rows of the wavefront's blocks: block row i, register r, its row of the matrix, its token scale
+        auto rows = [&](auto&& each) __attribute__((always_inline)) {
+            static_for<NA>([&](auto ii) {
+                constexpr int i = decltype(ii)::value;
+                const uint32_t lbase = (wm * NA + i) * 16u + 4u * lq;
+                each(ii, at.row0 + lbase, *reinterpret_cast<const f32x4*>(&TS[lbase]));
+            });
+        };
+        if (half_out && !pairs) {
+            rows([&](auto ii, uint32_t row0, const f32x4& tok4) __attribute__((always_inline)) {
+                constexpr int i = decltype(ii)::value;
+                static_for<4>([&](auto rr) {
+                    constexpr int r = decltype(rr)::value;
+                    const uint32_t row = row0 + r;
+                    uint32_t h[TJ];
+                    static_for<TJ>([&](auto jj) {
+                        constexpr int j = decltype(jj)::value;
+                        const float v = value(i, j, r, tok4[r]);
+                        h[j] = bits16(gelu ? faster_gelu(v) : v);
+                    });
+                    uint16_t* const out = static_cast<uint16_t*>(e.c) + static_cast<size_t>(row) * e.ldc;
+                    if constexpr (TJ == 4) {
+                        // a 4 x 4 transposition inside each four neighbouring lanes (see gemm_dma_body16): 8-byte stores, whole lines
+                        const uint32_t col = colw + 16u * (lane & 3u) + (lc & 12u);
+                        const uint32_t got = swap1(b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16));
+                        const uint32_t lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
+                        const uint32_t hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
+                        const uint32_t got2 = swap2(b1 ? lo : hi);
+                        if (row < at.row_end && col < N) {
+                            __builtin_nontemporal_store(b1 ? u32x2{got2, hi} : u32x2{lo, got2}, reinterpret_cast<u32x2*>(out + col));
+                        }
+                    } else {
+                        // after one swap the even lane holds two adjacent columns of the first block, the odd lane two of the second
+                        const uint32_t col = b0 ? colw + 16u + lc - 1u : colw + lc;
+                        const uint32_t got = swap1(b0 ? h[0] : h[1]);
+                        if (row < at.row_end && col < N) {
+                            __builtin_nontemporal_store(b0 ? got | (h[1] << 16) : h[0] | (got << 16), reinterpret_cast<uint32_t*>(out + col));
+                        }
+                    }
                 });
-                uint16_t* const out = static_cast<uint16_t*>(e.c) + static_cast<size_t>(row) * e.ldc;
-                if constexpr (TJ == 4) {
-                    // a 4 x 4 transposition inside each four neighbouring lanes (see gemm_dma_body16): 8-byte stores, whole lines
-                    const uint32_t col = colw + 16u * (lane & 3u) + (lc & 12u);
-                    const uint32_t give = b0 ? h[0] | (h[2] << 16) : h[1] | (h[3] << 16);
-                    const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-                    const uint32_t lo = b0 ? (got & 0xFFFFu) | (h[1] << 16) : h[0] | (got << 16);
-                    const uint32_t hi = b0 ? (got >> 16) | (h[3] << 16) : h[2] | (got & 0xFFFF0000u);
-                    const uint32_t got2 = static_cast<uint32_t>(
-                        __builtin_amdgcn_mov_dpp(static_cast<int>(b1 ? lo : hi), 0x4E, 0xF, 0xF, true));  // lane ^ 2
-                    if (row < at.row_end && col < N) {
-                        __builtin_nontemporal_store(b1 ? u32x2{got2, hi} : u32x2{lo, got2}, reinterpret_cast<u32x2*>(out + col));
+            });
+            return;
+        }
+        if (pairs) {
+            // Adjacent lanes hold the two columns of a pair.  After one swap the even lane owns the pair of the first of two blocks, the
+            // odd lane that of the second; after another one, of two rows, lanes l and l ^ 2 hold two adjacent outputs of a row each.
+            rows([&](auto ii, uint32_t row0, const f32x4& tok4) __attribute__((always_inline)) {
+                static_for<TJ>([&](auto cc) {
+                    constexpr int i = decltype(ii)::value, j = decltype(cc)::value / 2 * 2, r = decltype(cc)::value % 2 * 2;
+                    float o[2];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const float v0 = value(i, j, r + t, tok4[r + t]), v1 = value(i, j + 1, r + t, tok4[r + t]);
+                        const float got = __int_as_float(static_cast<int>(swap1(static_cast<uint32_t>(__float_as_int(b0 ? v0 : v1)))));
+                        o[t] = swiglu(b0 ? got : v0, b0 ? v1 : got, e.act_beta);
                     }
-                } else {
-                    // after one swap the even lane holds two adjacent columns of the first block, the odd lane two of the second
-                    const uint32_t col = b0 ? colw + 16u + lc - 1u : colw + lc;
-                    const uint32_t got = static_cast<uint32_t>(
-                        __builtin_amdgcn_mov_dpp(static_cast<int>(b0 ? h[0] : h[1]), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-                    if (row < at.row_end && col < N) {
-                        __builtin_nontemporal_store(b0 ? got | (h[1] << 16) : h[0] | (got << 16), reinterpret_cast<uint32_t*>(out + col));
+                    const uint32_t row = row0 + r + (b1 ? 1u : 0u), col = colw + 16u * j + (b0 ? 16u : 0u) + (lc & 12u);
+                    const size_t to = static_cast<size_t>(row) * e.ldc + (col >> 1);
+                    if (half_out) {
+                        const uint32_t h0 = bits16(o[0]), h1 = bits16(o[1]), got = swap2(b1 ? h0 : h1);
+                        if (row < at.row_end && col < N) {
+                            __builtin_nontemporal_store(b1 ? got | (h1 << 16) : h0 | (got << 16), reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(e.c) + to));
+                        }
+                    } else {
+                        const uint32_t h0 = static_cast<uint32_t>(__float_as_int(o[0])), h1 = static_cast<uint32_t>(__float_as_int(o[1]));
+                        const uint32_t got = swap2(b1 ? h0 : h1);
+                        if (row < at.row_end && col < N) {
+                            __builtin_nontemporal_store(b1 ? u32x2{got, h1} : u32x2{h0, got}, reinterpret_cast<u32x2*>(static_cast<uint32_t*>(e.c) + to));
+                        }
                     }
+                });
+            });
+            return;
+        }
+        rows([&](auto ii, uint32_t row0, const f32x4& tok4) __attribute__((always_inline)) {
+            static_for<2 * TJ>([&](auto cc) {
+                // two blocks of a row: after one swap the even lane holds two adjacent columns of the first, the odd lane two of the second
+                constexpr int i = decltype(ii)::value, r = decltype(cc)::value % 4, j = decltype(cc)::value / 4 * 2;
+                uint32_t h[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    float v = value(i, j + t, r, tok4[r]);
+                    v = gelu ? faster_gelu(v) : v;
+                    h[t] = quantised ? static_cast<uint32_t>(__float_as_int(v)) : static_cast<uint32_t>(acc[i][j + t][r] + bias_pre[j + t]);
+                }
+                const uint32_t row = row0 + r, col = b0 ? colw + 16u * j + 16u + lc - 1u : colw + 16u * j + lc, got = swap1(b0 ? h[0] : h[1]);
+                if (row < at.row_end && col < N) {
+                    __builtin_nontemporal_store(b0 ? u32x2{got, h[1]} : u32x2{h[0], got},
+                                                reinterpret_cast<u32x2*>(static_cast<uint32_t*>(e.c) + static_cast<size_t>(row) * e.ldc + col));
                 }
             });
         });
@@ -1069,7 +1136,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     constexpr int kBInstr = BK * BN / 1024 / 8;  // B DMA instructions per wavefront and K step
     static_assert(kAInstr >= 1 && kBInstr >= 1, "tile shape does not fit eight wavefronts");
 
-    const uint32_t K = p.k, N = p.n, lda = kForm == kRing && p.lda != 0u ? p.lda : K;
+    const uint32_t K = p.k, N = p.n, lda = ring_form(kForm) && p.lda != 0u ? p.lda : K;
     const uint32_t row0 = at.row0, row_end = at.row_end;
     const uint32_t n0 = kB == 0 && N % 16u != 0 && at.n0 + BN > N ? N - BN : at.n0;
     const int8_t* Bmat = at.b;
@@ -1128,7 +1195,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
             boff[u] = (col - n0) * K + 16u * line_piece(s);
             continue;
         }
-        const uint32_t kb = s / kPieces, q = (s % kPieces) ^ b_swizzle<BN, kForm == k16 || kForm == kRing>(kb);
+        const uint32_t kb = s / kPieces, q = (s % kPieces) ^ b_swizzle<BN, kForm == k16 || ring_form(kForm)>(kb);
         uint32_t col = n0 + 16u * q;
         col = col + 16u <= N ? col : N - 16u;      // columns past the end are never stored
         // fractal B: panels of 32 columns, each a contiguous row-major [K][32] block
@@ -1136,7 +1203,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
     }
     const uint32_t ldb = kBT ? 1u : kBP ? 16u : p.b_nz ? 32u : N;  // bytes from one k to the next
     // K range of this workgroup, in steps of BK
-    const uint32_t all_steps = kForm == k32Ragged || kForm == kRing ? (K + BK - 1u) / BK : K / BK;
+    const uint32_t all_steps = kForm == k32Ragged || ring_form(kForm) ? (K + BK - 1u) / BK : K / BK;
     uint32_t s_begin = 0, steps = all_steps;
     if constexpr (kSplitK) {
         s_begin = steps * bidy / p.k_splits;
@@ -1213,7 +1280,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
             }
         };
         gemm_dma_body16<BM, BN, kGrouped, kB, kALoads, kBInstr>(p, at, n0, steps, wave, lane, bases, load, stages..., TS);
-    } else if constexpr (kForm == kRing) {
+    } else if constexpr (ring_form(kForm)) {
         auto load = [&](uint32_t step, int u, char* S) __attribute__((always_inline)) {
             // how much of the row's k is left from here on, nothing past the last step; a piece past it brings zeros
             const uint32_t at_k = step < steps ? step : 0u, left = step < steps ? K - step * BK : 0u;
@@ -1230,7 +1297,7 @@ __device__ __forceinline__ void gemm_dma_tile_at(const GemmParams& p, const Tile
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(S + BM * BK + (wave * kBInstr + v) * 1024), 16, off, 0, 0, 0);
             }
         };
-        gemm_ring_body<BM, BN, kB, (sizeof(Stages) + ...) / sizeof(char*), kAInstr + kBInstr>(p, at, n0, steps, wave, lane, load, stages..., TS);
+        gemm_ring_body<BM, BN, kB, (sizeof(Stages) + ...) / sizeof(char*), kAInstr + kBInstr, kForm == kRingHalf>(p, at, n0, steps, wave, lane, load, stages..., TS);
     } else {
         auto run = [&](const Stage& S0, const Stage& S1) __attribute__((always_inline)) {
             gemm_dma_body32<BM, BN, kSplitK, kGrouped, kB>(p, at, n0, steps, bidy, wave, lane, issue, S0.a[0], S0.b, S1.a[0], S1.b, TS);
