@@ -737,66 +737,7 @@ bool dma_tiles_small(const ascq_matmul_desc* d)
     return d->m <= kSkinnyMaxM || (d->activation != ASCQ_MM_ACT_SWIGLU && gemm_dma_small_tiles(d->m, d->n, d->k));
 }
 
-// What a call of more than 32 rows takes without the ring kernel, in us with the quantiser (the constants are fits to
-// measurements; `splits`: the K split that its workspace allows).
-double without_ring_us(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, uint32_t splits)
-{
-    const double cus = device_compute_units(), steps = (d->k + 127u) / 128u;
-    const double raw_sums = d->activation == ASCQ_MM_ACT_SWIGLU && d->m <= kSkinnyMaxM && b_layout != 2 ? 6.0 : 0.0;  // a pass of its own
-    if (b_layout != 0 && d->m <= kSkinnyMaxM && gemm_ws_supported(p, b_layout == 1) && (b_layout == 1 || d->m <= 128u || !packed_tiles_faster(p))) {
-        // the weights held in registers; 16 rows take 0.85 us however short k is (181 x 1152 x 864 as [n, k] 19.9 us)
-        const double short_k = 0.85 - 0.95 * d->k / 4096.0;
-        return packed_ws_us(p) + (short_k > 0.0 ? short_k * ((d->m + 15u) / 16u) * gemm_ws_rounds(p) : 0.0) - (d->m <= 64u ? 2.0 : 0.0);
-    }
-    const bool small = d->m <= kSkinnyMaxM || (splits > 1u && d->activation != ASCQ_MM_ACT_SWIGLU && gemm_dma_small_tiles(d->m, d->n, d->k));
-    if (!small) {
-        const double tiles = static_cast<double>((d->m + 255u) / 256u) * ((d->n + 255u) / 256u);
-        return 8.5 + steps * (tiles <= cus ? 1.15 + 0.25 * tiles / cus : 1.35 * tiles / cus);
-    }
-    if (splits > 1u) {
-        // two launches, 0.8 a step, the partial tiles written and read back at 3.4 TB/s
-        const uint32_t each = (static_cast<uint32_t>(steps) + splits - 1u) / splits;
-        return 12.5 + 0.8 * each + static_cast<double>(splits) * d->m * d->n * 8.0 / 3.4e6 + raw_sums;
-    }
-    const double tiles = static_cast<double>((d->m + 127u) / 128u) * ((d->n + 127u) / 128u);
-    const double load = tiles <= cus ? 1.0 : tiles <= 2.0 * cus ? 1.0 + 0.45 * (tiles - cus) / cus : 1.45 * tiles / (2.0 * cus);
-    return 8.5 + 0.81 * steps * load + raw_sums;
-}
-
-// Whether the ring kernel is expected to be ahead, and with which tile.  In us with the quantiser, without and with it: [k, n]
-// weights 729 x 4304 x 1152 28.0 and 21.0, 256 x 4096 x 4096 29.3 and 16.9, 600 x 4096 x 4096 47.4 and 27.8, 1024 x 11008 x 4096 103 and
-// 64, 130 x 5120 x 5120 27.7 and 20.7; packed 192 x 4096 x 4096 24.2 and 15.2, 128 x 4096 x 11008 21.9 and 19.0; behind: 64 x 11008 x
-// 4096 28.6 and 36.0 (ten splits of K on 32 tiles), 512 x 2048 x 11008 24.5 and 28.3 (more tiles of 128 x 128 than units).
-bool ring_preferred(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, const void* workspace, size_t workspace_bytes, RingPlan& plan)
-{
-    // (a lane addresses its row or column of a tile by 31 bits)
-    constexpr uint32_t kMost = 1u << 23;
-    if (d->m <= 32u || d->k > kMost || d->n > kMost || d->trans_a || d->b_format == ASCQ_MM_B_NZ || !gemm_dma_supported(p, b_layout)) {
-        return false;
-    }
-    uint32_t splits = gemm_dma_skinny_splits(d->m, d->n, d->k);
-    if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < static_cast<size_t>(splits) * d->m * d->n * sizeof(int32_t)) {
-        splits = 1u;
-    }
-    plan = gemm_ring_plan(d->m, d->n, d->k, b_layout);
-    return plan.us < 0.95 * without_ring_us(d, p, b_layout, splits);
-}
-
 inline size_t round256(size_t v) { return (v + 255u) & ~static_cast<size_t>(255u); }
-
-// A linear on the ring kernel: x quantised into the workspace, then the tiles.  Rows of a k off 128 lie a multiple of 128 apart
-// where the workspace has the room, so that the tiles' 128-byte pieces of a row are whole lines (729 x 4304 x 1152 20.9 -> 19.2 us).
-// The caller has checked the workspace for rows of k bytes.
-int linear_on_ring(GemmParams& p, const RingPlan& ring, int b_layout, int32_t x_dtype, const void* x, char* ws, size_t workspace_bytes, hipStream_t st)
-{
-    const uint32_t apart = (p.k + 127u) / 128u * 128u;
-    p.lda = round256(static_cast<size_t>(p.m) * apart) + static_cast<size_t>(p.m) * sizeof(float) <= workspace_bytes ? apart : p.k;
-    float* const tok = reinterpret_cast<float*>(ws + round256(static_cast<size_t>(p.m) * p.lda));
-    p.a = reinterpret_cast<const int8_t*>(ws);
-    p.epi.tok_scale = tok;
-    const int rc = dynamic_quant_rows(x_dtype, p.m, p.k, ws, p.lda, tok, x, st);
-    return rc != ASCQ_OK ? rc : launch_gemm_ring(p, ring.shape, b_layout, st);
-}
 
 // True when the plain matmul of this descriptor runs on the direct-to-LDS tiles without a K split, whose epilogue
 // applies SwiGLU in registers (16-bit outputs).
@@ -819,6 +760,91 @@ bool swiglu_in_decode_kernel(const ascq_matmul_desc* d, const GemmParams& p, con
         return false;
     }
     return (d->m <= gemm_packed_pass_rows(p) && gemm_packed_nk_supported(p)) || gemm_ws_supported(p, true);
+}
+
+// What a call of more than 32 rows takes without the ring kernel, in us with the quantiser: the time of the kernel that the
+// dispatch below (matmul_w8a8_packed for packed weights) picks for it.  The constants are fits to measurements; `splits`: the K split that
+// its workspace allows; `ring`: the ring tile that it is compared with.
+double without_ring_us(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, uint32_t splits, int ring)
+{
+    const double cus = device_compute_units(), steps = (d->k + 127u) / 128u;
+    const bool pairs = d->activation == ASCQ_MM_ACT_SWIGLU;
+    const bool raw = pairs && b_layout != 2 && !swiglu_in_tile_kernel(d, p, p.a, p.b) && !swiglu_in_decode_kernel(d, p, p.a, p.b);
+    // a pass of its own over the int32 sums, which are written and read back at 5 TB/s
+    const double pass = raw ? 6.0 + static_cast<double>(d->m) * d->n * 8.0 / 5e6 : 0.0;
+    auto registers = [&]() {
+        // the weights held in registers; 16 rows take 0.85 us however short k is (181 x 1152 x 864 as [n, k] 19.9 us)
+        const double short_k = 0.85 - 0.95 * d->k / 4096.0;
+        return packed_ws_us(p) + (short_k > 0.0 ? short_k * ((d->m + 15u) / 16u) * gemm_ws_rounds(p) : 0.0) - (d->m <= 64u ? 2.0 : 0.0);
+    };
+    bool small;  // tiles of 128 x 128 and not of 256 x 256
+    if (b_layout == 2) {
+        if (pairs || (splits > 1u && d->m <= kSkinnyMaxM && !packed_split_faster(p, splits))) {
+            splits = 1u;
+        }
+        const bool tiles_ok = !pairs || d->out_dtype == ASCQ_F16 || d->out_dtype == ASCQ_BF16;
+        if (!tiles_ok || (d->m <= kSkinnyMaxM && (d->m <= 128u || (splits == 1u && !packed_tiles_faster(p))))) {
+            // (where they do not fit the registers: a trip over them per 16 rows)
+            return gemm_ws_supported(p, false) ? registers() : (d->m + 15u) / 16u * (5.0 + static_cast<double>(d->n) * d->k / 4.7e6);
+        }
+        small = d->m <= kSkinnyMaxM || (splits > 1u && gemm_dma_small_tiles(d->m, d->n, d->k));
+    } else {
+        if (b_layout == 1 && gemm_ws_supported(p, true)) {
+            return registers();
+        }
+        if (!dma_tiles_ok(d, p)) {
+            // register-staged tiles of 128 x 256 (300 x 4112 x 11008 as [n, k] 82 us, 434 x 2192 x 18688 108)
+            const double tiles = static_cast<double>((d->m + 127u) / 128u) * ((d->n + 255u) / 256u);
+            return 29.0 + 1.5 * steps * (tiles <= cus ? 1.0 : 1.7 * static_cast<double>(static_cast<uint64_t>((tiles + cus - 1.0) / cus))) + pass;
+        }
+        small = d->m <= kSkinnyMaxM || ((raw || !pairs) && splits > 1u && gemm_dma_small_tiles(d->m, d->n, d->k));
+    }
+    if (!small) {
+        const double tiles = static_cast<double>((d->m + 255u) / 256u) * ((d->n + 255u) / 256u);
+        return 8.5 + steps * (tiles <= cus ? 1.15 + 0.25 * tiles / cus : 1.35 * tiles / cus) + pass;
+    }
+    if (splits > 1u) {
+        // two launches, 0.8 a step, the partial tiles written and read back at 3.4 TB/s
+        const uint32_t each = (static_cast<uint32_t>(steps) + splits - 1u) / splits;
+        return 12.5 + 0.8 * each + static_cast<double>(splits) * d->m * d->n * 8.0 / 3.4e6 + pass;
+    }
+    // (2.1 us off against ring tiles of the same size, which start with four stages of loads: 257 x 512 x 7696 9.5 us, on the ring 12.7)
+    const double tiles = static_cast<double>((d->m + 127u) / 128u) * ((d->n + 127u) / 128u);
+    const double load = tiles <= cus ? 1.0 : tiles <= 2.0 * cus ? 1.0 + 0.45 * (tiles - cus) / cus : 1.45 * tiles / (2.0 * cus);
+    return 8.5 + 0.81 * steps * load + pass - (ring == 2 ? 2.1 : 0.0);
+}
+
+// Whether the ring kernel is expected to be ahead, and with which tile.  In us with the quantiser, without and with it: [k, n]
+// weights 729 x 4304 x 1152 28.0 and 19.2, 256 x 4096 x 4096 29.3 and 16.9, 600 x 4096 x 4096 47.4 and 27.8, 1024 x 11008 x 4096 103 and
+// 64, 130 x 5120 x 5120 27.7 and 20.7; packed 192 x 4096 x 4096 24.2 and 15.2, 128 x 4096 x 11008 21.9 and 19.0; behind: 64 x 11008 x
+// 4096 28.6 and 36.0 (ten splits of K on 32 tiles), 512 x 2048 x 11008 24.5 and 28.3 (more tiles of 128 x 128 than units).
+bool ring_preferred(const ascq_matmul_desc* d, const GemmParams& p, int b_layout, const void* workspace, size_t workspace_bytes, RingPlan& plan)
+{
+    // (a lane addresses its row or column of a tile by 31 bits)
+    constexpr uint32_t kMost = 1u << 23;
+    if (d->m <= 32u || d->k > kMost || d->n > kMost || d->trans_a || d->b_format == ASCQ_MM_B_NZ || !gemm_dma_supported(p, b_layout)) {
+        return false;
+    }
+    uint32_t splits = gemm_dma_skinny_splits(d->m, d->n, d->k);
+    if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < static_cast<size_t>(splits) * d->m * d->n * sizeof(int32_t)) {
+        splits = 1u;
+    }
+    plan = gemm_ring_plan(d->m, d->n, d->k, b_layout);
+    return plan.us < 0.95 * without_ring_us(d, p, b_layout, splits, plan.shape);
+}
+
+// A linear on the ring kernel: x quantised into the workspace, then the tiles.  Rows of a k off 128 lie a multiple of 128 apart
+// where the workspace has the room, so that the tiles' 128-byte pieces of a row are whole lines (729 x 4304 x 1152 20.9 -> 19.2 us).
+// The caller has checked the workspace for rows of k bytes.
+int linear_on_ring(GemmParams& p, const RingPlan& ring, int b_layout, int32_t x_dtype, const void* x, char* ws, size_t workspace_bytes, hipStream_t st)
+{
+    const uint32_t apart = (p.k + 127u) / 128u * 128u;
+    p.lda = round256(static_cast<size_t>(p.m) * apart) + static_cast<size_t>(p.m) * sizeof(float) <= workspace_bytes ? apart : p.k;
+    float* const tok = reinterpret_cast<float*>(ws + round256(static_cast<size_t>(p.m) * p.lda));
+    p.a = reinterpret_cast<const int8_t*>(ws);
+    p.epi.tok_scale = tok;
+    const int rc = dynamic_quant_rows(x_dtype, p.m, p.k, ws, p.lda, tok, x, st);
+    return rc != ASCQ_OK ? rc : launch_gemm_ring(p, ring.shape, b_layout, st);
 }
 
 // the matmul that leaves raw accumulators: same operands, no quantisation, at most the pre-dequant bias

@@ -1485,11 +1485,58 @@ def test_linear_w8a8_small_tiles_with_a_ring_of_stages(m, k, n, act):
             assert np.all(np.abs(got - want) <= (ulp + 2.0 ** -18) * np.abs(want) + 1e-6), layout
 
 
+def ring_tiles(call):
+    """The tiles of the ring kernel that `call` launches, by the kernel names that the profiler saw: {(rows, columns)}."""
+    import re
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    found = [re.search(r"gemm_ring_kernel(?:ILi(\d+)ELi(\d+)|<(\d+), (\d+))", e.key) for e in prof.key_averages()]
+    return {tuple(int(g) for g in f.groups() if g) for f in found if f}
+
+
+@pytest.mark.parametrize("m,k,n,tile", [(65, 144, 520, (64, 64)), (200, 1040, 264, (64, 64)), (130, 2192, 272, (64, 64)), (300, 640, 4400, (128, 64)),
+                                        (290, 1136, 4408, (128, 64)), (600, 384, 6400, (128, 128)), (520, 1744, 6008, (128, 128))])
+def test_linears_reach_every_tile_of_the_ring(m, k, n, tile):
+    """The sizes of the test above that stand for a tile shape run it, with and without SwiGLU: its comparisons are of that kernel."""
+    announce("ring tiles", m, k, n, tile)
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device=DEV)
+    cs = torch.ones(n, device=DEV)
+    for trans_b in (False, True):
+        w = torch.zeros((n, k) if trans_b else (k, n), dtype=torch.int8, device=DEV)
+        for act in (abi.MM_ACT_NONE, abi.MM_ACT_SWIGLU):
+            c = torch.zeros((m, n // 2 if act == abi.MM_ACT_SWIGLU else n), dtype=torch.bfloat16, device=DEV)
+            assert ring_tiles(lambda: ops.linear_w8a8_dynamic(c, x, w, cs, None, act, trans_b)) == {tile}, (trans_b, act)
+
+
+@pytest.mark.parametrize("m,k,n", [(300, 4112, 11008), (434, 2192, 18688), (131, 9136, 18048)])
+def test_linears_of_ragged_k_leave_the_register_staged_tiles(m, k, n):
+    """[n, k] weights with a k off 128 and tiles enough for the chip: the plain matmul runs register-staged tiles, which the ring is
+    twice as fast as, so the linear takes the ring; sampled columns against exact sums."""
+    announce("ring or staged", m, k, n)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + k)
+    x = torch.randn((m, k), device=DEV, generator=g).to(torch.bfloat16)
+    w = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    cs = torch.rand(n, device=DEV, generator=g) * 1e-3 + 1e-4
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device=DEV)
+    assert ring_tiles(lambda: ops.linear_w8a8_dynamic(c, x, w, cs, trans_b=True)) != set()
+    q, ts = ops.dynamic_quant_per_token(x)
+    cols = torch.tensor([0, 1, 63, 64, 127, 128, n // 2, n - 9, n - 1], device=DEV)
+    want = (q.double() @ w[cols].double().t().contiguous()).float() * cs[cols] * ts[:, None]      # exact sums, one rounding per step
+    assert torch.equal(c[:, cols], want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("m,n,k", [(100, 272, 1040), (130, 528, 1152), (257, 1000, 1280)])
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_matmul_outputs_of_the_ring_tiles(m, n, k, trans_b):
     """The plain matmul where 64 x 64 tiles with a ring of stages are one round of the chip: raw int32 sums, and quant words
     with and without the pre-shift to every output type."""
+    mm = ops.Matmul(m, n, k, trans_b=trans_b)
+    mm.set_tensor_a(torch.zeros((m, k), dtype=torch.int8, device=DEV))
+    mm.set_tensor_b(torch.zeros((n, k) if trans_b else (k, n), dtype=torch.int8, device=DEV))
+    plan = mm.plan(torch.zeros((m, n), dtype=torch.int32, device=DEV))
+    assert (plan.tile_m, plan.tile_n) == (64, 64)
     test_int32_accumulators_bit_exact(m, n, k, trans_b)
     test_fixpipe_pre_shift_words(m, n, k, trans_b)
 
