@@ -86,8 +86,8 @@ struct WqStage {
 };
 
 // One BM x BN tile of rows from row0 and columns from n0.  BN = 256: wavefronts 2 (M) x 4 (N); BN = 128: 4 x 2.  A
-// wavefront owns BM / kWM rows by 64 columns.
-template <int BM, int BN, bool kInt4, bool kOff>
+// wavefront owns BM / kWM rows by 64 columns.  kOnce: a step's loads go out at once (BN = 128, see launch_wq_gemm).
+template <int BM, int BN, bool kInt4, bool kOff, bool kOnce>
 __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32_t n0, const WqStage& S0, const WqStage& S1)
 {
     constexpr int kWN = BN / 64, kWM = 8 / kWN, NA = BM / 16 / kWM, NH = NA / 2, TJ = 4;
@@ -333,9 +333,8 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
                     fetch(next, s + 3u, kFetches - 1);
                 }
             };
-            // (BN = 128: a step is as long as its loads' way from memory, so they all go out at once.  One behind every other matrix
-            // instruction: w8a16 108 x 8064 x 18496 97.6 -> 106.3 us, 1509 x 10752 x 1664 105.7 -> 116.8, int4 49 x 6272 x 20480 70.5 -> 76.7)
-            constexpr int kAtOnce = kMid ? 0 : decltype(late)::value;
+            static_assert(!kOnce || !kMid, "one barrier per step");
+            constexpr int kAtOnce = kOnce ? decltype(late)::value : 0;
 #pragma unroll
             for (int u = 0; u < kAtOnce; ++u) late_load(u);
             __builtin_amdgcn_sched_barrier(0);
@@ -466,7 +465,7 @@ __device__ __forceinline__ void wq_tile(const WqParams& p, uint32_t row0, uint32
 
 // 256 x 256: the first p.full tiles are run as they are; each of the others, which would leave part of the last
 // round of the chip idle, is run by two workgroups with 128 x 256 tiles.
-template <int BM, int BN, bool kInt4, bool kOff>
+template <int BM, int BN, bool kInt4, bool kOff, bool kOnce>
 __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
 {
     __shared__ __attribute__((aligned(1024))) char A0[BM * 64], A0h[BM * 64], A1[BM * 64], A1h[BM * 64], B0[BN * 128], B1[BN * 128];
@@ -479,7 +478,7 @@ __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
             return;  // whole workgroup (the launch is rounded up to a multiple of 8)
         }
         band_order(t, p.tiles_m, p.tiles_n, tm, tn);
-        wq_tile<BM, BN, kInt4, kOff>(p, tm * BM, tn * BN, S0, S1);
+        wq_tile<BM, BN, kInt4, kOff, kOnce>(p, tm * BM, tn * BN, S0, S1);
     } else if constexpr (BM == 256) {
         const uint32_t t = xcd_remap(blockIdx.x - p.full, 2u * (tiles - p.full));
         if (t == 0xFFFFFFFFu) {
@@ -488,12 +487,12 @@ __global__ __launch_bounds__(kThreads) void wq_gemm_kernel(WqParams p)
         band_order(p.full + t / 2u, p.tiles_m, p.tiles_n, tm, tn);
         const uint32_t row0 = tm * 256u + (t & 1u) * 128u;
         if (row0 < p.m) {
-            wq_tile<128, BN, kInt4, kOff>(p, row0, tn * BN, S0, S1);
+            wq_tile<128, BN, kInt4, kOff, kOnce>(p, row0, tn * BN, S0, S1);
         }
     }
 }
 
-template <int BM, int BN>
+template <int BM, int BN, bool kOnce = false>
 void wq_launch(WqParams p, bool int4, bool has_offset, hipStream_t st)
 {
     p.tiles_m = (p.m + BM - 1u) / BM;
@@ -502,11 +501,11 @@ void wq_launch(WqParams p, bool int4, bool has_offset, hipStream_t st)
     const uint32_t blocks = BM == 256 ? p.full + 2u * (tiles - p.full) : tiles;
     const uint32_t grid = (blocks + 7u) / 8u * 8u;
     if (int4) {
-        has_offset ? wq_gemm_kernel<BM, BN, true, true><<<grid, kThreads, 0, st>>>(p)
-                   : wq_gemm_kernel<BM, BN, true, false><<<grid, kThreads, 0, st>>>(p);
+        has_offset ? wq_gemm_kernel<BM, BN, true, true, kOnce><<<grid, kThreads, 0, st>>>(p)
+                   : wq_gemm_kernel<BM, BN, true, false, kOnce><<<grid, kThreads, 0, st>>>(p);
     } else {
-        has_offset ? wq_gemm_kernel<BM, BN, false, true><<<grid, kThreads, 0, st>>>(p)
-                   : wq_gemm_kernel<BM, BN, false, false><<<grid, kThreads, 0, st>>>(p);
+        has_offset ? wq_gemm_kernel<BM, BN, false, true, kOnce><<<grid, kThreads, 0, st>>>(p)
+                   : wq_gemm_kernel<BM, BN, false, false, kOnce><<<grid, kThreads, 0, st>>>(p);
     }
 }
 
@@ -514,9 +513,10 @@ void wq_launch(WqParams p, bool int4, bool has_offset, hipStream_t st)
 
 // The tile shape: the one with the smallest estimate of rounds of the chip times a round's time per K step, measured at
 // k = 8192, n = 28672 with every compute unit busy (us): 256 x 256 1.62, 128 x 256 1.11, 128 x 128 1.2 for the two tiles
-// that share a unit and 0.62 for one alone.  256 x 256 tiles that would fill less than about two thirds of the last round
+// that share a unit and 0.62 for one alone; since then the loads of all three are spread better and take 3 to 8 % less, which
+// leaves the choice where it was.  256 x 256 tiles that would fill less than about two thirds of the last round
 // are cut in half there (k = 4096, n = 11008, 2048 rows: 204 -> 187 us; where the power limit and not
-// the rounds sets the time it makes no difference, k = 8192, n = 28672, 2048 rows: 847 us either way).
+// the rounds sets the time it makes no difference, k = 8192, n = 28672, 2048 rows).
 int launch_wq_gemm(const WqParams& p, bool int4, bool has_offset, hipStream_t st)
 {
     WqParams q = p;
@@ -531,7 +531,15 @@ int launch_wq_gemm(const WqParams& p, bool int4, bool has_offset, hipStream_t st
     const double c128 = up(t128, cus) * 1.11;
     const double csmall = tsmall <= cus ? 0.62 : up(tsmall, 2u * cus) * 1.2;
     if (csmall <= c128 && csmall <= c256) {
-        wq_launch<128, 128>(q, int4, has_offset, st);
+        // From half a million on (tiles times k): a step is as long as its loads' way from memory, and they all go out at once
+        // behind its barrier.  Less: each goes out behind a matrix instruction of its own.  In us, one behind every other
+        // instruction and at once: w8a16 108 x 8064 x 18496 106.8 and 98.1, 1509 x 10752 x 1664 121.1 and 106.7, int4 49 x 6272 x
+        // 20480 76.7 and 70.7; w8a16 54 x 5888 x 1440 52.1 and 55.7, int4 68 x 2176 x 2304 21.6 and 23.5.
+        if (static_cast<uint64_t>(tsmall) * p.k >= 500000u) {
+            wq_launch<128, 128, true>(q, int4, has_offset, st);
+        } else {
+            wq_launch<128, 128>(q, int4, has_offset, st);
+        }
     } else if (c128 < c256) {
         wq_launch<128, 256>(q, int4, has_offset, st);
     } else {

@@ -1232,6 +1232,14 @@ def test_half_gemm_on_tiles_of_256_columns(m, n, kind, k, offset):
         assert torch.equal(y, want.clamp(-65504, 65504).to(out) if out == torch.float16 else want)
 
 
+@pytest.mark.parametrize("kind,k", [("int8", 4224), ("int8", 4352), ("int8", 4416), ("int8", 4480), ("int4", 4224), ("int4", 4352), ("int4", 4480)])
+@pytest.mark.parametrize("offset", [True, False])
+def test_half_gemm_on_both_sides_of_the_load_rule(kind, k, offset):
+    """115 tiles of 128 x 128: below 4348 of k each load of a step goes out behind a matrix instruction, from there on all at once; even
+    and odd numbers of K steps, exact sums as above."""
+    test_half_gemm_on_tiles_of_256_columns(100, 14600, kind, k, offset)
+
+
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("k,n", [(128, 16), (256, 256), (512, 1040), (384, 30), (2048, 520), (8192, 144)])
 @pytest.mark.parametrize("mode", ["vector+offset", "vector", "scalar+offset", "scalar"])
