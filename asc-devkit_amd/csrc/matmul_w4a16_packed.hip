@@ -788,6 +788,23 @@ __global__ __launch_bounds__(256) void pack_w4_kernel(const uint8_t* __restrict_
     out[i] = v;
 }
 
+// Wavefronts per workgroup of w4a16_packed_rows_kernel: as many as give every compute unit a workgroup (7 at n = 28672 on 256
+// units), between 4 and 8.
+uint32_t rows_waves(uint32_t slabs, uint32_t cus)
+{
+    const uint32_t kw = (slabs + cus - 1u) / cus;
+    return kw < 4u ? 4u : (kw > 8u ? 8u : kw);
+}
+
+// us that passes of 16 rows are expected to take (90 random calls, nine tenths within 20 %): a launch, and per 1024 k a time that
+// grows with the wavefronts that share a compute unit.
+double passes_estimate(uint32_t m, uint32_t slabs, uint32_t k, bool sum_form, uint32_t cus)
+{
+    const uint32_t kw = rows_waves(slabs, cus), grid = (slabs + kw - 1u) / kw;
+    const double steps = static_cast<double>((grid + cus - 1u) / cus) * ((k + 1023u) / 1024u);
+    return ((m + kMaxRows - 1u) / kMaxRows) * (sum_form ? 3.25 + steps * (0.47 * kw - 0.12) : 2.95 + steps * (0.68 * kw - 0.71));
+}
+
 }  // namespace
 }  // namespace ascq
 
@@ -858,7 +875,9 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
     p.ktiles = d->k / kTileK;
     // the group-sum form needs whole tiles inside one quantisation group; other group sizes keep the per-weight form
     const bool sum_form = d->mode == ASCQ_W4A16_GROUP_SUM && p.gs_shift >= 2u;
-    if (!sum_form && d->m > kMaxPassRows && d->k <= kWqMaxK) {
+    const uint32_t cus = device_compute_units();
+    const bool tiles = !sum_form && d->m > kMaxPassRows && d->k <= kWqMaxK;
+    if (d->m > 4u) {
         WqParams w{};
         w.x = static_cast<const uint16_t*>(x);
         w.w = static_cast<const uint8_t*>(w_packed);
@@ -869,9 +888,13 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
         w.n = d->n;
         w.k = d->k;
         w.gs_shift = p.gs_shift;
-        return launch_wq_gemm(w, true, d->has_offset != 0, st);
+        if (wq_rows_ahead(w, true, sum_form, d->has_offset != 0, tiles ? wq_gemm_estimate(d->m, d->n, d->k) : passes_estimate(d->m, p.slabs, d->k, sum_form, cus), st)) {
+            return launch_status("ascq_matmul_w4a16_packed");
+        }
+        if (tiles) {
+            return launch_wq_gemm(w, true, d->has_offset != 0, st);
+        }
     }
-    const uint32_t cus = device_compute_units();
     constexpr uint32_t waves = 8u, batch = 4u;  // 16 wavefronts with batches of 4 tiles measured slower (37 against 30 us)
     for (uint32_t m0 = 0; m0 < d->m; m0 += kMaxRows) {
         p.m = d->m - m0 < kMaxRows ? d->m - m0 : kMaxRows;
@@ -880,10 +903,8 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
         p.y = static_cast<uint16_t*>(y) + static_cast<size_t>(m0) * d->n;
         const uint32_t groups = d->k / d->group_size;
         if (p.m > 4u && groups <= kRowsMaxGroups) {
-            // one wavefront per slab, the activations shared chunk by chunk: as many wavefronts per workgroup as give
-            // every compute unit a workgroup (7 at n = 28672 on 256 units), between 4 and 8
-            uint32_t kw = (p.slabs + cus - 1u) / cus;
-            kw = kw < 4u ? 4u : (kw > 8u ? 8u : kw);
+            // one wavefront per slab, the activations shared chunk by chunk
+            const uint32_t kw = rows_waves(p.slabs, cus);
             p.par_pitch = groups | 1u;
             const uint32_t grid = (p.slabs + kw - 1u) / kw;
             auto go = [&](auto has_offset, auto sum_form) {

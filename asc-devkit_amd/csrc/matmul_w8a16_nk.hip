@@ -616,8 +616,8 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
     per = per > kMaxGroups ? kMaxGroups : per;
     p.groups = per;
     const uint32_t grid = (n_groups + per - 1u) / per;
-    if (m > kDecodeRows && k % kGK == 0 && k <= kWqMaxK) {
-        // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 or 256 rows
+    const bool tiles = m > kDecodeRows && k % kGK == 0 && k <= kWqMaxK;
+    if (k % kGK == 0) {
         WqParams q{};
         q.x = static_cast<const uint16_t*>(x);
         q.w = p.w;
@@ -630,7 +630,16 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
         q.out_f32 = p.out_f32;
         q.scale_bits = scale_bits;
         q.offset_bits = offset_bits;
-        return launch_wq_gemm(q, false, has_offset, st);
+        // passes of 16 rows (51 random calls, nine tenths within 15 %): a launch, and per 1024 k a time that grows with the columns
+        const double runs = static_cast<double>((grid + cus - 1u) / cus) * ((k + 1023u) / 1024u);
+        const double passes = ((m + kRows - 1u) / kRows) * (3.25 + runs * (0.31 + 0.875 * per));
+        if (wq_rows_ahead(q, false, false, has_offset, tiles ? wq_gemm_estimate(m, n, k) : passes, st)) {
+            return launch_status("ascq_matmul_w8a16");
+        }
+        // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 or 256 rows
+        if (tiles) {
+            return launch_wq_gemm(q, false, has_offset, st);
+        }
     }
     for (uint32_t m0 = 0; m0 < m; m0 += kRows) {
         p.m = m - m0 < kRows ? m - m0 : kRows;

@@ -883,6 +883,78 @@ def test_w4a16_packed_many_rows(m, k, n, gs, offset):
         w4_check(np.ascontiguousarray(y.cpu().numpy()[:, c0:c1]), np.ascontiguousarray(want), x)
 
 
+@pytest.mark.parametrize("m,k,n,gs", [(36, 4096, 1032, 64), (21, 1152, 3336, 128), (129, 1152, 1544, 32), (40, 1280, 3336, 128),
+                                       (60, 2176, 5128, 64), (85, 1408, 13320, 128), (5, 128, 8, 128), (17, 384, 24, 32)])
+@pytest.mark.parametrize("offset", ["frac", None])
+@pytest.mark.parametrize("mode", [abi.W4A16_PER_WEIGHT, abi.W4A16_GROUP_SUM])
+def test_w4a16_packed_whole_k_tiles(m, k, n, gs, offset, mode):
+    """Rows and columns that leave the large tiles' chip idle: one case per tile of 16 x 16 to 64 x 64 (row and column tails, k that the
+    eight wavefronts cannot share evenly, a half-filled last stage), and calls shorter than the wavefronts' smallest share.
+    (Groups that are no multiple of 128 run the per-weight form.)  Two calls give identical bits, past the last row nothing is written."""
+    announce("w4a16 packed whole-k tiles", m, k, n, gs, offset, mode)
+    rng = np.random.default_rng(m + 5 * k + n)
+    x, wp, sc, of = w4_case(rng, m, k, n, gs, offset is not None)
+    if offset == "frac":
+        of = (rng.standard_normal((k // gs, n)) * 3).astype(np.float16)
+    w_gpu = ops.pack_weight_w4(to_dev(wp), k, n)
+    xd, sd, od = to_dev(x), to_dev(sc), None if of is None else to_dev(of)
+    # (the outputs begin 2 bytes off an 8-byte line: no wide stores)
+    buf = [torch.full(((m + 1) * n + 1,), 7.0, dtype=torch.float16, device=DEV) for _ in range(2)]
+    ys = [b[j:j + m * n].view(m, n) for j, b in enumerate(buf)]
+    for y in ys:
+        ops.matmul_w4a16_packed(y, xd, w_gpu, sd, od, gs, mode=mode)
+    assert torch.equal(ys[0].reshape(-1).view(torch.int16), ys[1].reshape(-1).view(torch.int16))
+    assert all(bool((b[j + m * n:] == 7.0).all()) for j, b in enumerate(buf))
+    d = abi.W4A16Desc(m=m, n=n, k=k, group_size=gs, has_offset=int(of is not None))
+    orc.set_threads(16)
+    for c0, c1 in [(0, n)] if n < 4000 else [(0, 80), (n // 2, n // 2 + 80), (n - 80, n)]:
+        want = np.ascontiguousarray(orc.matmul_w4a16(d, x, wp, sc, of, cols=(c0, c1))[:, c0:c1])
+        got = np.ascontiguousarray(ys[0].cpu().numpy()[:, c0:c1])
+        if mode == abi.W4A16_GROUP_SUM:
+            w4_group_sum_gate(got, want)
+        else:
+            w4_check(got, want, x)
+
+
+@pytest.mark.parametrize("m", [36, 140, 700])
+def test_w4a16_group_sum_whole_k_tiles_are_the_real_number_value(m):
+    """The group-sum form with more rows than a pass: on inputs whose products and sums are exact in fp32 (as above, at most
+    2^23 in units of 2^-6 with k = 1024) it gives the exact value."""
+    k, n, gs = 1024, 1032, 256
+    announce("w4a16 packed group sum, many rows, exact", m, k, n)
+    rng = np.random.default_rng(78 + m)
+    x = rng.integers(-4, 5, (m, k)).astype(np.float16)
+    w = rng.integers(-8, 8, (k, n)).astype(np.int8)
+    sc = (2.0 ** rng.integers(-6, -2, (k // gs, n))).astype(np.float16)
+    of = rng.integers(-8, 8, (k // gs, n)).astype(np.float16)
+    y = torch.zeros((m, n), dtype=torch.float16, device=DEV)
+    ops.matmul_w4a16_packed(y, to_dev(x), ops.pack_weight_w4(to_dev(pack_int4(w)), k, n), to_dev(sc), to_dev(of), gs,
+                            mode=abi.W4A16_GROUP_SUM)
+    xg = x.astype(np.float64).reshape(m, k // gs, gs)
+    wg = w.astype(np.float64).reshape(k // gs, gs, n)
+    want = sum((xg[:, g] @ wg[g] + xg[:, g].sum(axis=1)[:, None] * of[g].astype(np.float64)[None]) * sc[g].astype(np.float64)[None]
+               for g in range(k // gs))
+    assert np.array_equal(y.cpu().numpy(), want.astype(np.float16))
+
+
+@pytest.mark.parametrize("m,k,n,gs", [(8, 1152, 18064, 128), (12, 640, 26400, 64), (6, 5248, 28720, 128)])
+@pytest.mark.parametrize("mode", [abi.W4A16_PER_WEIGHT, abi.W4A16_GROUP_SUM])
+def test_w4a16_packed_rows_kernel_wide(m, k, n, gs, mode):
+    """5 to 16 rows and as many columns as give every compute unit a full workgroup: the kernel with one wavefront per slab (chunks of
+    1024 k with a short last one, a last workgroup with idle wavefronts)."""
+    announce("w4a16 packed rows, wide", m, k, n, gs, mode)
+    rng = np.random.default_rng(m * 131 + k + n)
+    x, wp, sc, of = w4_case(rng, m, k, n, gs, True)
+    y = torch.full((m, n), 7.0, dtype=torch.float16, device=DEV)
+    ops.matmul_w4a16_packed(y, to_dev(x), ops.pack_weight_w4(to_dev(wp), k, n), to_dev(sc), to_dev(of), gs, mode=mode)
+    d = abi.W4A16Desc(m=m, n=n, k=k, group_size=gs, has_offset=1)
+    orc.set_threads(16)
+    for c0, c1 in [(0, 80), (n // 2, n // 2 + 80), (n - 80, n)]:
+        want = np.ascontiguousarray(orc.matmul_w4a16(d, x, wp, sc, of, cols=(c0, c1))[:, c0:c1])
+        got = np.ascontiguousarray(y.cpu().numpy()[:, c0:c1])
+        w4_group_sum_gate(got, want) if mode == abi.W4A16_GROUP_SUM else w4_check(got, want, x)
+
+
 @pytest.mark.parametrize("m,k,n,gs", [(97, 128, 8, 32), (98, 384, 40, 128), (130, 256, 528, 64), (200, 640, 1032, 128)])
 @pytest.mark.parametrize("offset", [True, False])
 def test_w4a16_many_rows_packs_the_weights_first(m, k, n, gs, offset):
@@ -1156,6 +1228,28 @@ def test_w8a16_trans_b(m, k, n, mode):
     assert np.array_equal(np.asarray(want).view(np.uint8),
                           np.asarray(orc.matmul_w8a16(d, x, np.ascontiguousarray(wt.T), None if per_tensor else of,
                                                       None if per_tensor else sc)).view(np.uint8))
+
+
+@pytest.mark.parametrize("m,k,n", [(9, 8448, 1280), (28, 2176, 2573), (70, 3072, 1551), (100, 1152, 2055), (40, 2048, 5000), (300, 1152, 2059),
+                                   (85, 1152, 6913), (5, 128, 3), (16, 1664, 23264)])
+@pytest.mark.parametrize("mode", ["vector+offset", "scalar"])
+@pytest.mark.parametrize("out_f32", [True, False])
+def test_w8a16_trans_b_whole_k_tiles(m, k, n, mode, out_f32):
+    """Rows and columns that leave the large tiles' chip idle: one case per tile of 16 x 16 to 64 x 64, row and column tails (odd widths), k
+    that the eight wavefronts cannot share evenly or at all; the last case stays with the passes of 16 rows."""
+    announce("w8a16 [n, k] whole-k tiles", m, k, n, mode, out_f32)
+    rng = np.random.default_rng(m * 7 + k + n)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    wt = rng.integers(-128, 128, (n, k)).astype(np.int8)
+    per_tensor, has_offset = mode == "scalar", mode.endswith("offset")
+    sc, of = (0.0077, None) if per_tensor else (rng.uniform(1e-3, 1e-2, n).astype(np.float16), rng.uniform(-9, 9, n).astype(np.float16))
+    y = torch.full((m + 1, n), 7.0, dtype=torch.float32 if out_f32 else torch.float16, device=DEV)
+    ops.matmul_w8a16(y[:m], to_dev(x), to_dev(wt), of if per_tensor else to_dev(of), sc if per_tensor else to_dev(sc), trans_b=True)
+    assert bool((y[m] == 7.0).all())
+    d = abi.W8A16Desc(m=m, n=n, k=k, per_tensor=int(per_tensor), has_offset=int(has_offset), scale=sc if per_tensor else 0.0, offset=0.0,
+                      out_dtype=abi.F32 if out_f32 else abi.F16, trans_b=1)
+    orc.set_threads(16)
+    w8a16_check(y[:m].cpu().numpy(), orc.matmul_w8a16(d, x, wt, None if per_tensor else of, None if per_tensor else sc), x, out_f32)
 
 
 def test_w8a16_rows_beyond_thirty_two_bit_offsets():
