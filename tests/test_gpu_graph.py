@@ -149,3 +149,25 @@ def test_grouped_and_whole_column_kernels_replay_like_eager():
         torch.cuda.synchronize()
         for o, e in zip(outs, eager):
             assert torch.equal(o.view(torch.int16), e.view(torch.int16))
+
+
+def test_stream_handle_is_the_current_streams():
+    """The handle that the wrappers pass on: the default stream, a side stream, an external one and a capturing one."""
+    announce("current stream's handle")
+    same = lambda: ops._stream() == torch.cuda.current_stream().cuda_stream  # noqa: E731
+    assert same()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert same() and ops._stream() == side.cuda_stream
+        with torch.cuda.stream(torch.cuda.default_stream()):
+            assert same()
+        with torch.cuda.stream(torch.cuda.ExternalStream(side.cuda_stream)):
+            assert same() and ops._stream() == side.cuda_stream
+    seen, t = [], torch.ones(64, device=DEV)
+
+    def step():
+        t.add_(1.0)
+        seen.append(same())
+
+    _capture(step)
+    assert all(seen) and len(seen) == 2 and same()
