@@ -47,6 +47,8 @@ __device__ __forceinline__ void mx_static_for(F&& f)
 
 constexpr uint32_t kMxBM = 256, kMxBN = 256, kMxBK = 128;  // BK in bytes of an operand row
 constexpr int kMxThreads = 512;
+constexpr uint32_t kMxBufferCols = 1u << 20;  // columns up to which a tile's offsets in c fit 31 bits
+constexpr int kMxNt = 2;                      // cache policy of the stores: non-temporal (c is written once)
 constexpr uint32_t kMxScaleBuf = (kMxBM + kMxBN) * 16u;  // 16 scale bytes of every row of a tile's a and b
 
 // kFour: both operands 4-bit (e2m1); otherwise both a byte per value in memory, with the instruction's format codes
@@ -370,29 +372,55 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         const uint32_t col = n0 + (wn * TJ + j) * 32u + lrow;
         bias[j] = (p.bias != nullptr && col < p.n) ? p.bias[col] : 0.0f;
     }
-    if (p.out_dtype != ASCQ_F32 && p.n % 2u == 0) {
+    // Stores through a buffer that ends with the tile's last row: a scalar row offset and the lane's place in a row (past the end
+    // for columns that do not exist), no comparison or 64-bit product per value.  (With those and a choice of the type per
+    // value a float tile took 20 us to store: 854 x 3584 x 2048, e2m1, 33.3 us.)
+    constexpr uint32_t kNoColumn = 0x7FFFFFF0u;
+    const bool f32 = p.out_dtype == ASCQ_F32, bf = p.out_dtype == ASCQ_BF16;
+    const uint32_t size = f32 ? 4u : 2u, rows_left = p.m - row0 < kMxBM ? p.m - row0 : kMxBM;
+    const uint32_t off_line = reinterpret_cast<uintptr_t>(p.c) & 3u;
+    if (p.n > kMxBufferCols || (off_line & (size - 1u)) != 0) {  // offsets in a tile beyond 31 bits, values off their own size
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const uint32_t col = n0 + (wn * TJ + j) * 32u + lrow;
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = row0 + (wm * TI + i) * 32u + 8u * (r >> 2) + 4u * h + (r & 3);
+                    if (row < p.m && col < p.n) {
+                        mx_store(p, static_cast<size_t>(row) * p.n + col, acc[i][j][r] + bias[j]);
+                    }
+                }
+            }
+        }
+        return;
+    }
+    const uint32_t row_size = p.n * size;
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        static_cast<char*>(p.c) + static_cast<size_t>(row0) * row_size, 0, static_cast<int>(rows_left * row_size), 0x00020000);
+    uint32_t row_lo = wm * (TI * 32u) * row_size;
+    asm volatile("" : "+s"(row_lo));  // (or 64 offsets are computed ahead, and spilled)
+    auto row_at = [&](int i, int r) __attribute__((always_inline)) { return row_lo + (i * 32u + 8u * (r >> 2) + (r & 3)) * row_size; };
+    if (!f32 && p.n % 2u == 0 && off_line == 0) {
         // 16-bit outputs: after one swap between neighbouring lanes the even lane holds columns (l, l + 1) of the
         // wavefront's first block of 32 and the odd lane columns (l - 1, l) of the second: one dword store per lane,
         // and the 32 lanes of a row write one full 128-byte line
         const bool odd = (lane & 1u) != 0;
-        const bool bf = p.out_dtype == ASCQ_BF16;
         const uint32_t colw = n0 + wn * (TJ * 32u);
         const uint32_t col = odd ? colw + 32u + (lrow - 1u) : colw + lrow;  // first column of the lane's pair
+        const uint32_t at = col < p.n ? 4u * h * row_size + col * 2u : kNoColumn;
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + (wm * TI + i) * 32u + 8u * (r >> 2) + 4u * h + (r & 3);
                 const float v0 = acc[i][0][r] + bias[0], v1 = acc[i][1][r] + bias[1];
                 const uint32_t h0 = bf ? f32_to_bf16_bits(v0) : f32_to_half_bits_sat(v0);
                 const uint32_t h1 = bf ? f32_to_bf16_bits(v1) : f32_to_half_bits_sat(v1);
                 const uint32_t recv = static_cast<uint32_t>(
                     __builtin_amdgcn_mov_dpp(static_cast<int>(odd ? h0 : h1), 0xB1, 0xF, 0xF, true));  // lane ^ 1
                 const uint32_t word = odd ? (recv | (h1 << 16)) : (h0 | (recv << 16));
-                if (row < p.m && col < p.n) {
-                    __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.c) +
-                                                                                  static_cast<size_t>(row) * p.n + col));
-                }
+                __builtin_amdgcn_raw_buffer_store_b32(word, rc, at, row_at(i, r), kMxNt);
             }
         }
         return;
@@ -400,13 +428,23 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
         const uint32_t col = n0 + (wn * TJ + j) * 32u + lrow;
+        const uint32_t at = col < p.n ? 4u * h * row_size + col * size : kNoColumn;
+        if (f32) {
 #pragma unroll
-        for (int i = 0; i < TI; ++i) {
+            for (int i = 0; i < TI; ++i) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + (wm * TI + i) * 32u + 8u * (r >> 2) + 4u * h + (r & 3);
-                if (row < p.m && col < p.n) {
-                    mx_store(p, static_cast<size_t>(row) * p.n + col, acc[i][j][r] + bias[j]);
+                for (int r = 0; r < 16; ++r) {
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r] + bias[j]), rc, at, row_at(i, r), kMxNt);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float v = acc[i][j][r] + bias[j];
+                    const uint16_t bits = static_cast<uint16_t>(bf ? f32_to_bf16_bits(v) : f32_to_half_bits_sat(v));
+                    __builtin_amdgcn_raw_buffer_store_b16(bits, rc, at, row_at(i, r), 0);
                 }
             }
         }

@@ -237,6 +237,35 @@ def test_mx_few_rows_extreme_scales(fa, fb, m, k):
     assert np.array_equal(np.isnan(got), poisoned)
 
 
+@pytest.mark.parametrize("f", [E4, F2])
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16, torch.float16])
+def test_mx_tiles_store_every_row_length(f, out):
+    """256 x 256 tiles with a last one of 52 rows and 63 columns or fewer: floats, 16-bit values in pairs, one by one (odd rows; an output
+    that begins 2 bytes off a dword), every form the rounded bits of the float product's columns, which are compared with the
+    golden; past the last row nothing is written.  Large scales: halves saturate."""
+    m, k, more = 4148, 512, 2111
+    announce("mx tile stores", f, out)
+    rng = np.random.default_rng(f)
+    a, b, sa, sb, bv = mx_case(rng, m, more, k, f, f, sk=16, bias=True)
+    if out == torch.float16:
+        sb[::5] = np.maximum(sb[::5], 140)
+    want = run_mx(m, more, k, a, b, sa, sb, f, f, bias=bv)
+    d = abi.MxDesc(m=m, n=more, k=k, scale_k=16, a_format=f, b_format=f, out_dtype=abi.F32, has_bias=1)
+    orc.set_threads(16)
+    for r0, r1 in ((0, 3), (254, 258), (4144, 4148)):
+        gold = orc.matmul_mx(d, a, b, sa, sb, bv, rows=(r0, r1))[r0:r1]
+        mx_check(want[r0:r1].cpu().numpy(), gold, mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, f, f) + np.abs(bv), is8(f, f))
+    if out == torch.float16:
+        assert (want.abs() > 65504.0).any()
+        want = want.clamp(-65504.0, 65504.0)
+    ad, bd, sad, sbd, bvd = to_dev(a), to_dev(b), to_dev(sa), to_dev(sb), to_dev(bv)
+    for n, off in ((2111, 0), (2110, 0), (2110, 1), (2108, 0)):
+        buf = torch.full((off + (m + 1) * n,), 7.0, dtype=out, device=DEV)
+        c = buf[off:off + m * n].view(m, n)
+        ops.matmul_mx(c, ad, bd[:n], sad, sbd[:n], f, f, k, bvd[:n])
+        assert torch.equal(c, want[:, :n].to(out)) and bool((buf[off + m * n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("n", [320, 257])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float16])
 def test_mx_sixteen_bit_outputs_and_bias(out, n):
