@@ -52,13 +52,28 @@ struct QuantArgs {
     int dst_format;  // ascq_quant_dst
 };
 
+// What a launch of the vector kernel stores: the formats a program quantises to have a kernel each, whose code holds
+// nothing of the others; the rest share one.
+enum QuantKind { kQuantI8Rint, kQuantE4M3, kQuantE5M2, kQuantE2M1Rint, kQuantOther };
+
+inline int quant_kind(const QuantArgs& a)
+{
+    const bool rint = a.round_mode == ASCQ_CAST_RINT || a.round_mode == ASCQ_CAST_NONE;
+    switch (a.dst_format) {
+        case ASCQ_QDST_I8: return rint ? kQuantI8Rint : kQuantOther;
+        case ASCQ_QDST_FP8_E4M3FN: return kQuantE4M3;
+        case ASCQ_QDST_FP8_E5M2: return kQuantE5M2;
+        case ASCQ_QDST_FP4_E2M1: return rint ? kQuantE2M1Rint : kQuantOther;
+        default: return kQuantOther;
+    }
+}
+
 // the last step: int8 with the requested rounding, hifloat8 (ties away from zero, saturating), or an 8-bit float
 // (always half-even, saturating)
-template <bool kRint>
 __device__ __forceinline__ int quant_final(float t, const QuantArgs& a)
 {
     if (a.dst_format == ASCQ_QDST_I8) {
-        return round_sat8<kRint>(t, a.round_mode);
+        return round_sat8<false>(t, a.round_mode);
     }
     if (a.dst_format == ASCQ_QDST_HIF8) {
         return static_cast<int>(f32_to_hif8_sat(t));
@@ -70,6 +85,57 @@ __device__ __forceinline__ int quant_final(float t, const QuantArgs& a)
                                                                    : f32_to_fp4_sat<false>(b, a.round_mode));
     }
     return a.dst_format == ASCQ_QDST_FP8_E5M2 ? f32_to_fp8_sat<true>(t) : f32_to_fp8_sat<false>(t);
+}
+
+// The same for eight values, packed.  The machine's converters round half to even; what lies past the largest finite
+// value is brought there first, and NaN becomes +0 (about four operations per element; f32_to_fp8_sat takes 25).
+template <int kKind>
+__device__ __forceinline__ u32x2 quant_final8(const float (&t)[8], const QuantArgs& a)
+{
+    u32x2 out = {0u, 0u};
+    if constexpr (kKind == kQuantE4M3 || kKind == kQuantE5M2) {
+        constexpr float kMax = kKind == kQuantE4M3 ? 448.0f : 57344.0f;
+        float c[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e] = t[e] != t[e] ? 0.0f : __builtin_amdgcn_fmed3f(t[e], -kMax, kMax);
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            int w = 0;
+            if constexpr (kKind == kQuantE4M3) {
+                w = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d], c[4 * d + 1], w, false);
+                w = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d + 2], c[4 * d + 3], w, true);
+            } else {
+                w = __builtin_amdgcn_cvt_pk_bf8_f32(c[4 * d], c[4 * d + 1], w, false);
+                w = __builtin_amdgcn_cvt_pk_bf8_f32(c[4 * d + 2], c[4 * d + 3], w, true);
+            }
+            out[d] = static_cast<uint32_t>(w);
+        }
+    } else if constexpr (kKind == kQuantE2M1Rint) {
+        float c[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float b = bf16_bits_to_f32(f32_to_bf16_bits(t[e]));
+            c[e] = b != b ? 0.0f : __builtin_amdgcn_fmed3f(b, -6.0f, 6.0f);
+        }
+        uint32_t w = 0u;
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, c[0], c[1], 1.0f, 0);
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, c[2], c[3], 1.0f, 1);
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, c[4], c[5], 1.0f, 2);
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, c[6], c[7], 1.0f, 3);
+        out[0] = w;
+    } else {
+        int q[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = kKind == kQuantI8Rint ? round_sat8<true>(t[e], 0) : quant_final(t[e], a);
+        if (kKind == kQuantOther && (a.dst_format == ASCQ_QDST_FP4_E2M1 || a.dst_format == ASCQ_QDST_FP4_E1M2)) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out[0] |= static_cast<uint32_t>(q[e]) << (4 * e);
+        } else {
+            out[0] = pack4_i8(q[0], q[1], q[2], q[3]);
+            out[1] = pack4_i8(q[4], q[5], q[6], q[7]);
+        }
+    }
+    return out;
 }
 
 template <int kPar>
@@ -112,25 +178,31 @@ __device__ __forceinline__ float quant_param1(const QuantArgs& a, const void* ba
     }
 }
 
-// One lane = 8 consecutive columns; blockIdx.y walks groups of kRowsInFlight rows.  Requires n % 8 == 0 and
-// 16-byte aligned tensors.
-template <int kSrc, int kPar, int kCt, bool kRint>
+// One lane = 8 consecutive columns; blockIdx.y walks groups of kRows rows.  Requires n % 8 == 0 and 16-byte aligned
+// tensors.  Memory bounds it, on a few rows the chain of one row: a launch of few rows takes one at a time, and a row's
+// own parameter (per token, per group along the row) is asked for with the row itself.
+// One kernel per stored format, against one that chooses the format per element: half to e5m2 per group, 4117 x 3328, 21.5 ->
+// 11.4 us; bfloat16 to e2m1, 4000 x 4096, 33.0 -> 11.3; float to e4m3 per token 28.0 -> 18.5; bfloat16 to int8 18.9 -> 11.5
+// (49 MB: 4.3 TB/s, and a copy reaches 4.6).
+template <int kSrc, int kPar, int kCt, int kKind, int kRows>
 __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
 {
     const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
     if (j >= a.n) {
         return;
     }
-    const bool row_params = (a.policy == ASCQ_PER_TOKEN || a.policy == ASCQ_PER_GROUP);
-    const bool has_off = a.offset_kind != ASCQ_OFFSET_NONE;
+    const bool along = a.policy == ASCQ_PER_GROUP && a.k_dim == 1;
+    const bool row_scalar = a.policy == ASCQ_PER_TOKEN || along;      // one parameter for the lane's 8 columns of a row
+    const bool row_params = a.policy == ASCQ_PER_GROUP && !along;     // eight of them, others every group_size rows
+    const bool has_off = a.offset_kind != ASCQ_OFFSET_NONE, off_tensor = a.offset_kind == ASCQ_OFFSET_TENSOR;
+    const uint32_t per_row = along ? a.params_per_row : 1u, jg = along ? j / a.group_size : 0u;
     float s[8], o[8];
-    if (!row_params) {
-        quant_params8<kPar>(a, a.scale, a.sscale, 0, j, s);
-        if (a.offset_kind == ASCQ_OFFSET_TENSOR) {
-            quant_params8<kPar>(a, a.offset, a.soffset, 0, j, o);
-        } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = a.soffset;
+    for (int e = 0; e < 8; ++e) o[e] = Fmt<kCt>::cvt(a.soffset);
+    if (!row_scalar && !row_params) {
+        quant_params8<kPar>(a, a.scale, a.sscale, 0, j, s);
+        if (off_tensor) {
+            quant_params8<kPar>(a, a.offset, a.soffset, 0, j, o);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -138,27 +210,35 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
             o[e] = Fmt<kCt>::cvt(o[e]);
         }
     }
-    for (uint32_t r0 = blockIdx.y * kRowsInFlight; r0 < a.rows; r0 += gridDim.y * kRowsInFlight) {
-        float x[kRowsInFlight][8];
+    for (uint32_t r0 = blockIdx.y * kRows; r0 < a.rows; r0 += gridDim.y * kRows) {
+        float x[kRows][8], rs[kRows], ro[kRows];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kRows; ++u) {
             if (r0 + u < a.rows) {
                 load8<kSrc, true>(a.src, static_cast<size_t>(r0 + u) * a.n + j, x[u]);  // read once: non-temporal
+                if (row_scalar) {
+                    const size_t pi = static_cast<size_t>(r0 + u) * per_row + jg;
+                    rs[u] = load1<kPar>(a.scale, pi);
+                    ro[u] = off_tensor ? load1<kPar>(a.offset, pi) : a.soffset;
+                }
             }
         }
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kRows; ++u) {
             const uint32_t r = r0 + u;
             if (r >= a.rows) {
                 break;
             }
-            if (row_params) {
-                quant_params8<kPar>(a, a.scale, a.sscale, r, j, s);
-                if (a.offset_kind == ASCQ_OFFSET_TENSOR) {
-                    quant_params8<kPar>(a, a.offset, a.soffset, r, j, o);
-                } else {
+            if (row_scalar) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = a.soffset;
+                for (int e = 0; e < 8; ++e) {
+                    s[e] = Fmt<kCt>::cvt(rs[u]);
+                    o[e] = Fmt<kCt>::cvt(ro[u]);
+                }
+            } else if (row_params) {
+                quant_params8<kPar>(a, a.scale, a.sscale, r, j, s);
+                if (off_tensor) {
+                    quant_params8<kPar>(a, a.offset, a.soffset, r, j, o);
                 }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -166,28 +246,24 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
                     o[e] = Fmt<kCt>::cvt(o[e]);
                 }
             }
-            int q[8];
+            float t[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float t = Fmt<kCt>::mul(Fmt<kCt>::cvt(x[u][e]), s[e]);
+                t[e] = Fmt<kCt>::mul(Fmt<kCt>::cvt(x[u][e]), s[e]);
                 if (has_off) {
-                    t = Fmt<kCt>::add(t, o[e]);
+                    t[e] = Fmt<kCt>::add(t[e], o[e]);
                 }
-                q[e] = quant_final<kRint>(t, a);
             }
-            if (a.dst_format == ASCQ_QDST_FP4_E2M1 || a.dst_format == ASCQ_QDST_FP4_E1M2) {
+            const u32x2 out = quant_final8<kKind>(t, a);
+            const size_t at = static_cast<size_t>(r) * a.n + j;
+            if (kKind == kQuantE2M1Rint ||
+                (kKind == kQuantOther && (a.dst_format == ASCQ_QDST_FP4_E2M1 || a.dst_format == ASCQ_QDST_FP4_E1M2))) {
                 // two codes per byte, the even element in the low nibble: 8 columns are one dword
-                uint32_t out = 0;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) out |= static_cast<uint32_t>(q[e]) << (4 * e);
-                __builtin_nontemporal_store(
-                    out, reinterpret_cast<uint32_t*>(a.dst + (static_cast<size_t>(r) * a.n + j) / 2u));
-                continue;
+                const uint32_t word = out[0];
+                __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(a.dst + at / 2u));
+            } else {
+                __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(a.dst + at));
             }
-            u32x2 out;
-            out[0] = pack4_i8(q[0], q[1], q[2], q[3]);
-            out[1] = pack4_i8(q[4], q[5], q[6], q[7]);
-            __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(a.dst + static_cast<size_t>(r) * a.n + j));
         }
     }
 }
@@ -208,7 +284,7 @@ __global__ __launch_bounds__(kThreads) void quant_scalar_kernel(QuantArgs a)
                                                             : a.soffset;
             t = Fmt<kCt>::add(t, Fmt<kCt>::cvt(o));
         }
-        a.dst[e] = static_cast<int8_t>(quant_final<false>(t, a));
+        a.dst[e] = static_cast<int8_t>(quant_final(t, a));
     }
 }
 
@@ -291,26 +367,39 @@ __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
     }
 }
 
+template <int kSrc, int kPar, int kCt, int kKind>
+void launch_quant_vec(const QuantArgs& a, hipStream_t st)
+{
+    // Up to 2048 wavefronts of single rows are resident at once and take the time of one row (27 x 2272 half to e4m3 8.7 us ->
+    // below the 5.3 us that the host needs per call); beyond, several rows per lane keep more bytes in flight.
+    const bool few = static_cast<uint64_t>(a.rows) * a.n <= 2048u * 64u * 8u;
+    const RowLaunch rl = row_launch(a.n / 8, a.rows, few ? 1 : kRowsInFlight);
+    if (few) {
+        quant_vec_kernel<kSrc, kPar, kCt, kKind, 1><<<rl.grid, rl.block, 0, st>>>(a);
+    } else {
+        quant_vec_kernel<kSrc, kPar, kCt, kKind, kRowsInFlight><<<rl.grid, rl.block, 0, st>>>(a);
+    }
+}
+
 template <int kSrc, int kPar, int kCt>
 int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
 {
     if (vec) {
-        const RowLaunch rl = row_launch(a.n / 8, a.rows, kRowsInFlight);
-        const dim3 grid = rl.grid;
-        const uint32_t block = rl.block;
-        const bool rint = a.round_mode == ASCQ_CAST_RINT || a.round_mode == ASCQ_CAST_NONE;
+        const int kind = quant_kind(a);
         if constexpr (kSrc == ASCQ_F16 && kCt == ASCQ_F16) {
             // fp16 contract on a half source: scale / offset are half tensors or scalars
-            if (rint && a.dst_format == ASCQ_QDST_I8 &&
-                (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
-                quant_f16_fast_kernel<<<grid, block, 0, st>>>(a);
+            if (kind == kQuantI8Rint && (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
+                const RowLaunch rl = row_launch(a.n / 8, a.rows, kRowsInFlight);
+                quant_f16_fast_kernel<<<rl.grid, rl.block, 0, st>>>(a);
                 return launch_status("ascq_quant");
             }
         }
-        if (rint) {
-            quant_vec_kernel<kSrc, kPar, kCt, true><<<grid, block, 0, st>>>(a);
-        } else {
-            quant_vec_kernel<kSrc, kPar, kCt, false><<<grid, block, 0, st>>>(a);
+        switch (kind) {
+            case kQuantI8Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantI8Rint>(a, st); break;
+            case kQuantE4M3: launch_quant_vec<kSrc, kPar, kCt, kQuantE4M3>(a, st); break;
+            case kQuantE5M2: launch_quant_vec<kSrc, kPar, kCt, kQuantE5M2>(a, st); break;
+            case kQuantE2M1Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantE2M1Rint>(a, st); break;
+            default: launch_quant_vec<kSrc, kPar, kCt, kQuantOther>(a, st); break;
         }
     } else {
         size_t total = static_cast<size_t>(a.rows) * a.n;

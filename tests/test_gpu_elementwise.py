@@ -194,6 +194,34 @@ def test_quant_fp8(fmt, pair, policy):
             assert np.any((got[:cal] & 0x7F) == top_code)          # saturation was exercised
 
 
+@pytest.mark.parametrize("fmt", [abi.QDST_I8, abi.QDST_FP8_E4M3FN, abi.QDST_FP8_E5M2, abi.QDST_FP4_E2M1])
+@pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16])
+@pytest.mark.parametrize("rows", [32, 544])
+def test_quant_every_16_bit_value_to_the_packed_formats(fmt, src_dt, rows):
+    """Every half / bfloat16 value (infinities, NaN, subnormals, the midpoints of every grid) with scales that are powers
+    of two, so that midpoints stay midpoints, and with a few that are not; few rows (one per lane) and more than 2^20
+    elements (several rows per lane).  int8 leaves NaN out: it is outside the operator's domain."""
+    n = 2048
+    announce("quant every value", fmt, src_dt, rows)
+    x = np.resize(np.arange(65536, dtype=np.uint32).astype(np.uint16), (rows, n))
+    if fmt == abi.QDST_I8:
+        x = np.where((x & 0x7FFF) > (0x7C00 if src_dt == abi.F16 else 0x7F80), np.uint16(0x3F80), x)
+    xs = x.view(np.float16) if src_dt == abi.F16 else x
+    s = np.exp2(np.arange(rows * (n // 32)) % 9 - 4.0).astype(np.float32).reshape(rows, n // 32)
+    s[::3] *= np.float32(1.37)
+    para = ops.AscendQuantParam(m=rows, n=n, cal_count=rows * n, group_size=32)
+    dst = torch.zeros((rows, n // 2) if fmt == abi.QDST_FP4_E2M1 else (rows, n), dtype=torch.uint8 if fmt == abi.QDST_FP4_E2M1 else
+                      FP8.get(fmt, torch.int8), device=DEV)
+    cfg = ops.AscendQuantConfig(has_offset=False, k_dim=1, round_mode=abi.CAST_RINT)
+    ops.ascend_quant_policy(dst, to_dev(x, "bf16" if src_dt == abi.BF16 else "f16"), to_dev(s), None, para, abi.PER_GROUP, cfg, dst_format=fmt)
+    d = abi.QuantDesc(policy=abi.PER_GROUP, src_dtype=src_dt, scale_dtype=abi.F32, compute=abi.COMPUTE_SCALE_T,
+                      round_mode=abi.CAST_RINT, k_dim=1, m=rows, n=n, cal_count=rows * n, group_size=32, dst_format=fmt,
+                      offset_kind=abi.OFFSET_NONE)
+    want = orc.quant(d, xs, s).view(np.uint8)
+    got = dst.view(torch.uint8).cpu().numpy()
+    assert np.array_equal(got.reshape(-1), want.reshape(-1))
+
+
 @pytest.mark.parametrize("pair", PAIRS)
 @pytest.mark.parametrize("policy", ["token", "group0", "group1", "channel", "tensor"])
 def test_quant_hifloat8(pair, policy):
