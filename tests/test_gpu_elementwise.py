@@ -626,6 +626,32 @@ def test_antiquant_fp4_sources(fmt, dst_dt, mode):
         assert not got[rows:].any()
 
 
+@pytest.mark.parametrize("fmt", [abi.QDST_I8, abi.QDST_FP8_E4M3FN, abi.QDST_FP8_E5M2, abi.QDST_HIF8, abi.QDST_FP4_E2M1, abi.QDST_FP4_E1M2])
+@pytest.mark.parametrize("dst_dt", [abi.F16, abi.BF16])
+@pytest.mark.parametrize("along_n", [True, False])
+def test_antiquant_policy_more_than_2_to_the_20_elements(fmt, dst_dt, along_n):
+    """Several rows per lane, the last lanes with fewer: 517 rows of 2080, every code among them."""
+    m, n, gs = 517, 2080, 32
+    announce("antiquant policy, many rows", fmt, dst_dt, along_n)
+    rng = np.random.default_rng(m + fmt)
+    fp4 = fmt in (abi.QDST_FP4_E2M1, abi.QDST_FP4_E1M2)
+    src = np.resize(np.arange(256, dtype=np.uint8), (m, n // 2 if fp4 else n))
+    if fmt in (abi.QDST_FP8_E4M3FN, abi.QDST_FP8_E5M2):
+        src = np.where((src & 0x7F) > 0x7B, np.uint8(0x31), src)        # finite codes
+    sshape = (m, n // gs) if along_n else (-(-m // gs), n)
+    sc = rng.integers(100, 150, sshape).astype(np.uint8) if fp4 else rng.uniform(-2, 2, sshape).astype(np.float32)
+    of = None if fp4 else rng.uniform(-3, 3, sshape).astype(np.float32)
+    dst = torch.zeros((m, n), dtype=TDT[dst_dt], device=DEV)
+    cfg = ops.AscendAntiQuantConfig(has_offset=not fp4, k_dim=int(along_n))
+    para = ops.AscendAntiQuantParam(m=m, n=n, cal_count=m * n, group_size=gs)
+    srcd = to_dev(src) if fp4 else to_dev(src).view(B8[fmt])
+    ops.ascend_antiquant_policy(dst, srcd, to_dev(sc), None if fp4 else to_dev(of), para, abi.PER_GROUP, cfg, src_format=fmt)
+    d = abi.AntiQuantPolicyDesc(policy=abi.PER_GROUP, src_format=fmt, scale_dtype=abi.E8M0 if fp4 else abi.F32, dst_dtype=dst_dt,
+                                compute=abi.COMPUTE_SCALE_T, has_offset=int(not fp4), k_dim=int(along_n), m=m, n=n,
+                                cal_count=m * n, group_size=gs)
+    assert np.array_equal(bits(dst), orc.antiquant_policy(d, src, sc, of).view(np.uint16))
+
+
 def test_antiquant_fp4_rejects():
     announce("antiquant fp4 rejects")
     src = torch.zeros((4, 32), dtype=torch.uint8, device=DEV)
