@@ -218,42 +218,52 @@ struct Elem<ASCQ_I32> {
     static __device__ __forceinline__ float to_f32(int32_t v) { return static_cast<float>(v); }  // RNE
 };
 
-// 16-byte load / store with or without the non-temporal cache policy (data that is touched once per call).
-template <bool kNT>
+// 16-byte load / store: aligned, aligned and non-temporal (data that is touched once per call), or from any address (rows of
+// a width that is not a multiple of the vector; the machine takes such an access as one instruction).
+enum Access { kAligned = 0, kNonTemporal = 1, kAnyAddress = 2 };
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+template <int kAccess>
 __device__ __forceinline__ u32x4 ld16(const void* p)
 {
-    if constexpr (kNT) {
+    if constexpr (kAccess == kNonTemporal) {
         return __builtin_nontemporal_load(static_cast<const u32x4*>(p));
+    } else if constexpr (kAccess == kAnyAddress) {
+        return *static_cast<const u32x4_any*>(p);
     } else {
         return *static_cast<const u32x4*>(p);
     }
 }
-template <bool kNT, class V>
+template <int kAccess, class V>
 __device__ __forceinline__ void st16(void* p, V v)
 {
-    if constexpr (kNT) {
+    if constexpr (kAccess == kNonTemporal) {
         __builtin_nontemporal_store(v, static_cast<V*>(p));
+    } else if constexpr (kAccess == kAnyAddress) {
+        typedef V V_any __attribute__((aligned(1)));
+        *static_cast<V_any*>(p) = v;
     } else {
         *static_cast<V*>(p) = v;
     }
 }
 
-// Load 8 consecutive elements (16-byte aligned group for 2-byte types) widened to fp32.
-template <int kDt, bool kNT = false>
+// Load 8 consecutive elements (16-byte aligned group for 2-byte types, or any address) widened to fp32.
+template <int kDt, int kAccess = kAligned>
 __device__ __forceinline__ void load8(const void* base, size_t idx, float (&out)[8])
 {
     typedef typename Elem<kDt>::type T;
     const T* p = static_cast<const T*>(base) + idx;
     if constexpr (sizeof(T) == 2) {
-        u32x4 v = ld16<kNT>(p);
+        u32x4 v = ld16<kAccess>(p);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             out[2 * i] = Elem<kDt>::to_f32(static_cast<uint16_t>(v[i] & 0xFFFFu));
             out[2 * i + 1] = Elem<kDt>::to_f32(static_cast<uint16_t>(v[i] >> 16));
         }
     } else if constexpr (sizeof(T) == 4) {
-        u32x4 a = ld16<kNT>(reinterpret_cast<const u32x4*>(p));
-        u32x4 b = ld16<kNT>(reinterpret_cast<const u32x4*>(p) + 1);
+        u32x4 a = ld16<kAccess>(p);
+        u32x4 b = ld16<kAccess>(p + 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t ua = a[i], ub = b[i];
@@ -264,6 +274,7 @@ __device__ __forceinline__ void load8(const void* base, size_t idx, float (&out)
             out[4 + i] = Elem<kDt>::to_f32(tb);
         }
     } else {
+        static_assert(kAccess != kAnyAddress, "64-bit parameters are read aligned");
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             u32x4 v = reinterpret_cast<const u32x4*>(p)[i];
@@ -281,13 +292,13 @@ __device__ __forceinline__ float load1(const void* base, size_t idx)
 }
 
 // Store 8 fp32 values as the destination type (rounded once).
-template <int kDt, bool kNT = false>
+template <int kDt, int kAccess = kAligned>
 __device__ __forceinline__ void store8(void* base, size_t idx, const float (&v)[8])
 {
     if constexpr (kDt == ASCQ_F32) {
         f32x4* p = reinterpret_cast<f32x4*>(static_cast<float*>(base) + idx);
-        st16<kNT>(p, f32x4{v[0], v[1], v[2], v[3]});
-        st16<kNT>(p + 1, f32x4{v[4], v[5], v[6], v[7]});
+        st16<kAccess>(p, f32x4{v[0], v[1], v[2], v[3]});
+        st16<kAccess>(p + 1, f32x4{v[4], v[5], v[6], v[7]});
     } else {
         u32x4 o;
 #pragma unroll
@@ -302,7 +313,7 @@ __device__ __forceinline__ void store8(void* base, size_t idx, const float (&v)[
             }
             o[i] = lo | (hi << 16);
         }
-        st16<kNT>(static_cast<uint16_t*>(base) + idx, o);
+        st16<kAccess>(static_cast<uint16_t*>(base) + idx, o);
     }
 }
 

@@ -146,19 +146,19 @@ __device__ __forceinline__ u32x2 quant_final8(const float (&t)[8], const QuantAr
     return out;
 }
 
-template <int kPar>
+template <int kPar, int kAccess>
 __device__ __forceinline__ void quant_params8(const QuantArgs& a, const void* base, float scalar, uint32_t i,
                                               uint32_t j, float (&p)[8])
 {
     float s = scalar;
     switch (a.policy) {
-        case ASCQ_PER_CHANNEL: load8<kPar>(base, j, p); return;
+        case ASCQ_PER_CHANNEL: load8<kPar, kAccess>(base, j, p); return;
         case ASCQ_PER_TOKEN: s = load1<kPar>(base, i); break;
         case ASCQ_PER_GROUP:
             if (a.k_dim == 1) {
                 s = load1<kPar>(base, static_cast<size_t>(i) * a.params_per_row + j / a.group_size);
             } else {
-                load8<kPar>(base, static_cast<size_t>(i / a.group_size) * a.n + j, p);
+                load8<kPar, kAccess>(base, static_cast<size_t>(i / a.group_size) * a.n + j, p);
                 return;
             }
             break;
@@ -186,16 +186,25 @@ __device__ __forceinline__ float quant_param1(const QuantArgs& a, const void* ba
     }
 }
 
+// The columns of a lane, at a row's end moved back so that they end with the row: in rows of an odd width the last two lanes
+// share columns and store the same values there.
+template <bool kAny>
+__device__ __forceinline__ uint32_t lane_columns(uint32_t n)
+{
+    const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
+    return kAny && j < n && j + 8u > n ? n - 8u : j;
+}
+
 // One lane = 8 consecutive columns; blockIdx.y walks groups of kRows rows.  Requires n % 8 == 0 and 16-byte aligned
-// tensors.  Memory bounds it, on a few rows the chain of one row: a launch of few rows takes one at a time, and a row's
+// tensors, or, kAny, n >= 8 (parameters per group or token: n % 8 == 0).  Memory bounds it, on a few rows the chain of one row: a launch of few rows takes one at a time, and a row's
 // own parameter (per token, per group along the row) is asked for with the row itself.
 // One kernel per stored format, against one that chooses the format per element: half to e5m2 per group, 4117 x 3328, 21.5 ->
 // 11.4 us; bfloat16 to e2m1, 4000 x 4096, 33.0 -> 11.3; float to e4m3 per token 28.0 -> 18.5; bfloat16 to int8 18.9 -> 11.5
 // (49 MB: 4.3 TB/s, and a copy reaches 4.6).
-template <int kSrc, int kPar, int kCt, int kKind, int kRows>
+template <int kSrc, int kPar, int kCt, int kKind, int kRows, bool kAny>
 __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
 {
-    const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
+    const uint32_t j = lane_columns<kAny>(a.n);
     if (j >= a.n) {
         return;
     }
@@ -208,9 +217,9 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = Fmt<kCt>::cvt(a.soffset);
     if (!row_scalar && !row_params) {
-        quant_params8<kPar>(a, a.scale, a.sscale, 0, j, s);
+        quant_params8<kPar, kAny ? kAnyAddress : kAligned>(a, a.scale, a.sscale, 0, j, s);
         if (off_tensor) {
-            quant_params8<kPar>(a, a.offset, a.soffset, 0, j, o);
+            quant_params8<kPar, kAny ? kAnyAddress : kAligned>(a, a.offset, a.soffset, 0, j, o);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
 #pragma unroll
         for (int u = 0; u < kRows; ++u) {
             if (r0 + u < a.rows) {
-                load8<kSrc, true>(a.src, static_cast<size_t>(r0 + u) * a.n + j, x[u]);  // read once: non-temporal
+                load8<kSrc, kAny ? kAnyAddress : kNonTemporal>(a.src, static_cast<size_t>(r0 + u) * a.n + j, x[u]);  // read once: non-temporal
                 if (row_scalar) {
                     const size_t pi = static_cast<size_t>(r0 + u) * per_row + jg;
                     rs[u] = load1<kPar>(a.scale, pi);
@@ -244,9 +253,9 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
                     o[e] = Fmt<kCt>::cvt(ro[u]);
                 }
             } else if (row_params) {
-                quant_params8<kPar>(a, a.scale, a.sscale, r, j, s);
+                quant_params8<kPar, kAny ? kAnyAddress : kAligned>(a, a.scale, a.sscale, r, j, s);
                 if (off_tensor) {
-                    quant_params8<kPar>(a, a.offset, a.soffset, r, j, o);
+                    quant_params8<kPar, kAny ? kAnyAddress : kAligned>(a, a.offset, a.soffset, r, j, o);
                 }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -269,6 +278,8 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
                 // two codes per byte, the even element in the low nibble: 8 columns are one dword
                 const uint32_t word = out[0];
                 __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(a.dst + at / 2u));
+            } else if constexpr (kAny) {
+                *reinterpret_cast<u32x2_any*>(a.dst + at) = out;
             } else {
                 __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(a.dst + at));
             }
@@ -276,7 +287,7 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
     }
 }
 
-// Any shape / alignment: one element per lane.
+// Rows of fewer than 8 columns: one element per lane.
 template <int kSrc, int kPar, int kCt>
 __global__ __launch_bounds__(kThreads) void quant_scalar_kernel(QuantArgs a)
 {
@@ -321,15 +332,17 @@ __device__ __forceinline__ uint32_t quant_h2x2_to_i8x4(f16x2 a, f16x2 b)
     return __builtin_amdgcn_perm(ub, ua, 0x06040200u);  // low bytes of the four 16-bit integers
 }
 
+template <bool kAny>
 __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
 {
-    const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
+    constexpr int kParAccess = kAny ? kAnyAddress : kAligned;
+    const uint32_t j = lane_columns<kAny>(a.n);
     if (j >= a.n) {
         return;
     }
     f16x2 s[4], o[4];
     if (a.policy == ASCQ_PER_CHANNEL) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.scale) + j);
+        const u32x4 v = ld16<kParAccess>(static_cast<const uint16_t*>(a.scale) + j);
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[e] = h2_from_bits(v[e]);
     } else {
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
         for (int e = 0; e < 4; ++e) s[e] = f16x2{hs, hs};
     }
     if (a.offset_kind == ASCQ_OFFSET_TENSOR) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.offset) + j);
+        const u32x4 v = ld16<kParAccess>(static_cast<const uint16_t*>(a.offset) + j);
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = h2_from_bits(v[e]);
     } else {
@@ -353,8 +366,7 @@ __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
 #pragma unroll
         for (int u = 0; u < kRowsInFlight; ++u) {
             if (r0 + u < a.rows) {
-                x[u] = __builtin_nontemporal_load(
-                    reinterpret_cast<const u32x4*>(src + static_cast<size_t>(r0 + u) * a.n + j));
+                x[u] = ld16<kAny ? kAnyAddress : kNonTemporal>(src + static_cast<size_t>(r0 + u) * a.n + j);
             }
         }
 #pragma unroll
@@ -369,7 +381,12 @@ __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
                 u32x2 out;
                 out[0] = quant_h2x2_to_i8x4(t[0], t[1]);
                 out[1] = quant_h2x2_to_i8x4(t[2], t[3]);
-                __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(a.dst + static_cast<size_t>(r0 + u) * a.n + j));
+                int8_t* to = a.dst + static_cast<size_t>(r0 + u) * a.n + j;
+                if constexpr (kAny) {
+                    *reinterpret_cast<u32x2_any*>(to) = out;
+                } else {
+                    __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(to));
+                }
             }
         }
     }
@@ -381,37 +398,47 @@ void launch_quant_vec(const QuantArgs& a, hipStream_t st)
     const bool few = few_rows(a.rows, a.n);
     const RowLaunch rl = row_launch(a.n / 8, a.rows, few ? 1 : kRowsInFlight);
     if (few) {
-        quant_vec_kernel<kSrc, kPar, kCt, kKind, 1><<<rl.grid, rl.block, 0, st>>>(a);
+        quant_vec_kernel<kSrc, kPar, kCt, kKind, 1, false><<<rl.grid, rl.block, 0, st>>>(a);
     } else {
-        quant_vec_kernel<kSrc, kPar, kCt, kKind, kRowsInFlight><<<rl.grid, rl.block, 0, st>>>(a);
+        quant_vec_kernel<kSrc, kPar, kCt, kKind, kRowsInFlight, false><<<rl.grid, rl.block, 0, st>>>(a);
     }
 }
 
 template <int kSrc, int kPar, int kCt>
 int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
 {
-    if (vec) {
-        const int kind = quant_kind(a);
-        if constexpr (kSrc == ASCQ_F16 && kCt == ASCQ_F16) {
-            // fp16 contract on a half source: scale / offset are half tensors or scalars
-            if (kind == kQuantI8Rint && (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
-                const RowLaunch rl = row_launch(a.n / 8, a.rows, kRowsInFlight);
-                quant_f16_fast_kernel<<<rl.grid, rl.block, 0, st>>>(a);
-                return launch_status("ascq_quant");
-            }
-        }
-        switch (kind) {
-            case kQuantI8Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantI8Rint>(a, st); break;
-            case kQuantE4M3: launch_quant_vec<kSrc, kPar, kCt, kQuantE4M3>(a, st); break;
-            case kQuantE5M2: launch_quant_vec<kSrc, kPar, kCt, kQuantE5M2>(a, st); break;
-            case kQuantE2M1Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantE2M1Rint>(a, st); break;
-            default: launch_quant_vec<kSrc, kPar, kCt, kQuantOther>(a, st); break;
-        }
-    } else {
+    const int kind = quant_kind(a);
+    const bool per_row = a.policy == ASCQ_PER_TOKEN || a.policy == ASCQ_PER_GROUP;
+    const bool any = !vec && a.n >= 8 && (a.n % 8 == 0 || !per_row);
+    if (!vec && !any) {
         size_t total = static_cast<size_t>(a.rows) * a.n;
         size_t blocks = (total + kThreads - 1) / kThreads;
         if (blocks > 65536) blocks = 65536;
         quant_scalar_kernel<kSrc, kPar, kCt><<<static_cast<uint32_t>(blocks), kThreads, 0, st>>>(a);
+        return launch_status("ascq_quant");
+    }
+    const RowLaunch rl = row_launch((a.n + 7) / 8, a.rows, kRowsInFlight);
+    if constexpr (kSrc == ASCQ_F16 && kCt == ASCQ_F16) {
+        // fp16 contract on a half source: scale / offset are half tensors or scalars
+        if (kind == kQuantI8Rint && (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
+            any ? quant_f16_fast_kernel<true><<<rl.grid, rl.block, 0, st>>>(a)
+                : quant_f16_fast_kernel<false><<<rl.grid, rl.block, 0, st>>>(a);
+            return launch_status("ascq_quant");
+        }
+    }
+    if (any) {
+        // rows of any width and alignment: bfloat16 4000 x 4099 per channel 13.3 us, 47.0 with one
+        // element per lane
+        kind == kQuantI8Rint ? quant_vec_kernel<kSrc, kPar, kCt, kQuantI8Rint, kRowsInFlight, true><<<rl.grid, rl.block, 0, st>>>(a)
+                             : quant_vec_kernel<kSrc, kPar, kCt, kQuantOther, kRowsInFlight, true><<<rl.grid, rl.block, 0, st>>>(a);
+        return launch_status("ascq_quant");
+    }
+    switch (kind) {
+        case kQuantI8Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantI8Rint>(a, st); break;
+        case kQuantE4M3: launch_quant_vec<kSrc, kPar, kCt, kQuantE4M3>(a, st); break;
+        case kQuantE5M2: launch_quant_vec<kSrc, kPar, kCt, kQuantE5M2>(a, st); break;
+        case kQuantE2M1Rint: launch_quant_vec<kSrc, kPar, kCt, kQuantE2M1Rint>(a, st); break;
+        default: launch_quant_vec<kSrc, kPar, kCt, kQuantOther>(a, st); break;
     }
     return launch_status("ascq_quant");
 }
@@ -438,10 +465,13 @@ __device__ __forceinline__ float block_max(float v, float* lds)
 }
 
 // One workgroup per row; the row stays in registers between the abs-max reduction (wavefront shuffles, then LDS
-// across the wavefronts) and the quantisation, so it is read from HBM once.  n % 8 == 0, n <= 8 * kBlock * kVecs.
+// across the wavefronts) and the quantisation, so it is read from HBM once.  n <= 8 * kBlock * kVecs; n % 8 == 0 and aligned
+// tensors or, kAny, n >= 8 (the last lane's columns then end with the row and overlap its neighbour's: the same maximum, the
+// same codes).  bfloat16 4000 x 4099: 10.7 us, 21.3 with the two passes of
+// dynq_generic_kernel.
 // Rows of up to 4096 elements run on two wavefronts with up to four vectors per lane: against four wavefronts with
 // two, 4.5 against 4.7 us per launch at 2048 rows of 4096 bfloat16 (a conversion without the reduction: 3.7 us).
-template <int kSrc, int kVecs, int kBlock = kThreads>
+template <int kSrc, bool kAny, int kVecs, int kBlock = kThreads>
 __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q, float* __restrict__ ts,
                                                           const void* __restrict__ x, uint32_t n, uint32_t ldq)
 {
@@ -452,9 +482,10 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
     float amax = 0.0f;
 #pragma unroll
     for (int k = 0; k < kVecs; ++k) {
-        const uint32_t j = (k * kThreads + threadIdx.x) * 8u;
+        uint32_t j = (k * kThreads + threadIdx.x) * 8u;
         if (j < n) {
-            load8<kSrc>(x, static_cast<size_t>(row) * n + j, v[k]);
+            if (kAny && j + 8u > n) j = n - 8u;
+            load8<kSrc, kAny ? kAnyAddress : kAligned>(x, static_cast<size_t>(row) * n + j, v[k]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[k][e]));
         }
@@ -472,8 +503,9 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
     // permute per pair gathers the low bytes.
 #pragma unroll
     for (int k = 0; k < kVecs; ++k) {
-        const uint32_t j = (k * kThreads + threadIdx.x) * 8u;
+        uint32_t j = (k * kThreads + threadIdx.x) * 8u;
         if (j < n) {
+            if (kAny && j + 8u > n) j = n - 8u;
             uint32_t u[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -483,12 +515,17 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
             u32x2 out;
             out[0] = __builtin_amdgcn_perm(u[1], u[0], 0x0c0c0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000c0cu);
             out[1] = __builtin_amdgcn_perm(u[5], u[4], 0x0c0c0400u) | __builtin_amdgcn_perm(u[7], u[6], 0x04000c0cu);
-            *reinterpret_cast<u32x2*>(q + static_cast<size_t>(row) * ldq + j) = out;
+            int8_t* to = q + static_cast<size_t>(row) * ldq + j;
+            if constexpr (kAny) {
+                *reinterpret_cast<u32x2_any*>(to) = out;
+            } else {
+                *reinterpret_cast<u32x2*>(to) = out;
+            }
         }
     }
 }
 
-// Any n / alignment: two passes over the row (the second one hits in L2).
+// Rows of fewer than 8 or more than 16384 columns: two passes over the row (the second one hits in L2).
 template <int kSrc>
 __global__ __launch_bounds__(kThreads) void dynq_generic_kernel(int8_t* __restrict__ q, float* __restrict__ ts,
                                                                 const void* __restrict__ x, uint32_t n, uint32_t ldq)
@@ -510,24 +547,34 @@ __global__ __launch_bounds__(kThreads) void dynq_generic_kernel(int8_t* __restri
     }
 }
 
+template <int kSrc, bool kAny>
+void launch_dynq_row(uint32_t m, uint32_t n, int8_t* q, uint32_t ldq, float* ts, const void* x, hipStream_t st)
+{
+    if (n <= 1024) {
+        dynq_row_kernel<kSrc, kAny, 1, 128><<<m, 128, 0, st>>>(q, ts, x, n, ldq);
+    } else if (n <= 2048) {
+        dynq_row_kernel<kSrc, kAny, 2, 128><<<m, 128, 0, st>>>(q, ts, x, n, ldq);
+    } else if (n <= 4096) {
+        dynq_row_kernel<kSrc, kAny, 4, 128><<<m, 128, 0, st>>>(q, ts, x, n, ldq);
+    } else if (n <= 8192) {
+        dynq_row_kernel<kSrc, kAny, 4><<<m, kThreads, 0, st>>>(q, ts, x, n, ldq);
+    } else {
+        dynq_row_kernel<kSrc, kAny, 8><<<m, kThreads, 0, st>>>(q, ts, x, n, ldq);
+    }
+}
+
 template <int kSrc>
 int launch_dynq(uint32_t m, uint32_t n, void* q, uint32_t ldq, void* ts, const void* x, hipStream_t st)
 {
     int8_t* qq = static_cast<int8_t*>(q);
     float* tt = static_cast<float*>(ts);
     const bool vec = (n % 8 == 0) && (ldq % 8 == 0) && aligned16(x) && ((reinterpret_cast<uintptr_t>(q) & 7u) == 0);
-    if (vec && n <= 1024) {
-        dynq_row_kernel<kSrc, 1, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
-    } else if (vec && n <= 2048) {
-        dynq_row_kernel<kSrc, 2, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
-    } else if (vec && n <= 4096) {
-        dynq_row_kernel<kSrc, 4, 128><<<m, 128, 0, st>>>(qq, tt, x, n, ldq);
-    } else if (vec && n <= 8192) {
-        dynq_row_kernel<kSrc, 4><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
-    } else if (vec && n <= 16384) {
-        dynq_row_kernel<kSrc, 8><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
-    } else {
+    if (n < 8 || n > 16384) {
         dynq_generic_kernel<kSrc><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
+    } else if (vec) {
+        launch_dynq_row<kSrc, false>(m, n, qq, ldq, tt, x, st);
+    } else {
+        launch_dynq_row<kSrc, true>(m, n, qq, ldq, tt, x, st);
     }
     return launch_status("ascq_dynamic_quant_per_token");
 }
@@ -584,7 +631,7 @@ __global__ __launch_bounds__(kThreads) void dequant_vec_kernel(DequantArgs a)
 #pragma unroll
         for (int u = 0; u < kRowsInFlight; ++u) {
             if (r0 + u < a.rows) {
-                load8<kSrc, true>(a.src, static_cast<size_t>(r0 + u) * a.n + j, x[u]);  // read once: non-temporal
+                load8<kSrc, kNonTemporal>(a.src, static_cast<size_t>(r0 + u) * a.n + j, x[u]);  // read once: non-temporal
             }
         }
 #pragma unroll
@@ -602,7 +649,7 @@ __global__ __launch_bounds__(kThreads) void dequant_vec_kernel(DequantArgs a)
             float y[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = x[u][e] * s[e];
-            store8<kDst, true>(a.dst, static_cast<size_t>(r) * a.dst_stride + j, y);
+            store8<kDst, kNonTemporal>(a.dst, static_cast<size_t>(r) * a.dst_stride + j, y);
         }
     }
 }
@@ -718,10 +765,14 @@ __global__ __launch_bounds__(kThreads) void antiquant_scalar_kernel(AntiQuantArg
 // Half outputs: codes become halves through the exponent trick (0x6400 | u is 1024 + u; u = w + 128 or w + 8, taken off
 // again, all exact), then one rounded packed add of the offset and one rounded packed multiply by the scale: about 2.5
 // VALU operations per element.
-template <int kSrc, int kDst, bool kHasOffset, bool kTranspose>
+// kAny (not transposed): cols >= 8 and any alignment; int8 5504 x 5564 with 43 groups to half 16.1 us (92 MB:
+// 5.7 TB/s), 50.6 with one element per lane.
+template <int kSrc, int kDst, bool kHasOffset, bool kTranspose, bool kAny>
 __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a)
 {
-    const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
+    static_assert(!(kTranspose && kAny), "a transposed row has one parameter per lane");
+    constexpr int kParAccess = kAny ? kAnyAddress : kAligned;
+    const uint32_t j = lane_columns<kAny>(a.cols);
     if (j >= a.cols) {
         return;
     }
@@ -739,8 +790,12 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
         for (int u = 0; u < kRows; ++u) {
             if (r0 + u < a.rows) {
                 const size_t e = static_cast<size_t>(r0 + u) * a.cols + j;
-                if constexpr (kSrc == ASCQ_I8) {
+                if constexpr (kSrc == ASCQ_I8 && kAny) {
+                    raw[u] = *reinterpret_cast<const u32x2_any*>(static_cast<const int8_t*>(a.src) + e);
+                } else if constexpr (kSrc == ASCQ_I8) {
                     raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const int8_t*>(a.src) + e));
+                } else if constexpr (kAny) {
+                    raw[u][0] = *reinterpret_cast<const u32_any*>(static_cast<const uint8_t*>(a.src) + e / 2u);
                 } else {
                     raw[u][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(a.src) + e / 2u));
                 }
@@ -775,18 +830,18 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
                 } else {
                     const size_t pi = static_cast<size_t>(g) * a.cols + j;
                     if constexpr (kHalf) {
-                        const u32x4 s0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.scale) + pi);
+                        const u32x4 s0 = ld16<kParAccess>(static_cast<const uint16_t*>(a.scale) + pi);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) s[e] = h2_from_bits(s0[e]);
                         if constexpr (kHasOffset) {
-                            const u32x4 o0 = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.offset) + pi);
+                            const u32x4 o0 = ld16<kParAccess>(static_cast<const uint16_t*>(a.offset) + pi);
 #pragma unroll
                             for (int e = 0; e < 4; ++e) o[e] = h2_from_bits(o0[e]);
                         }
                     } else {
-                        load8<kDst>(a.scale, pi, sf);
+                        load8<kDst, kParAccess>(a.scale, pi, sf);
                         if constexpr (kHasOffset) {
-                            load8<kDst>(a.offset, pi, of);
+                            load8<kDst, kParAccess>(a.offset, pi, of);
                         }
                     }
                 }
@@ -821,7 +876,7 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
                     __builtin_memcpy(&bits, &v, 4);
                     y[d] = bits;
                 }
-                __builtin_nontemporal_store(y, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.dst) + oe));
+                st16<kAny ? kAnyAddress : kNonTemporal>(static_cast<uint16_t*>(a.dst) + oe, y);
             } else {
                 float y[8];
 #pragma unroll
@@ -830,7 +885,7 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
                     const float w = static_cast<float>(byte & 0xFFu) - (kSrc == ASCQ_I8 ? 128.0f : 8.0f);
                     y[e] = antiquant_one<kDst>(w, sf[e], of[e], kHasOffset);
                 }
-                store8<kDst, true>(a.dst, oe, y);
+                store8<kDst, kAny ? kAnyAddress : kNonTemporal>(a.dst, oe, y);
             }
         }
     }
@@ -839,15 +894,18 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
 template <int kSrc, int kDst>
 int launch_antiquant(const AntiQuantArgs& a, bool vec, hipStream_t st)
 {
-    if (vec) {
+    if (vec || (!a.transpose && a.cols >= 8)) {
         // keep the rows of one lane inside as few parameter groups as possible: consecutive row groups per block
-        const RowLaunch rl = row_launch(a.cols / 8, a.rows, 2 * kRowsInFlight);
-        if (a.transpose) {
-            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, true><<<rl.grid, rl.block, 0, st>>>(a)
-                         : antiquant_vec_kernel<kSrc, kDst, false, true><<<rl.grid, rl.block, 0, st>>>(a);
+        const RowLaunch rl = row_launch((a.cols + 7) / 8, a.rows, 2 * kRowsInFlight);
+        if (!vec) {
+            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, false, true><<<rl.grid, rl.block, 0, st>>>(a)
+                         : antiquant_vec_kernel<kSrc, kDst, false, false, true><<<rl.grid, rl.block, 0, st>>>(a);
+        } else if (a.transpose) {
+            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, true, false><<<rl.grid, rl.block, 0, st>>>(a)
+                         : antiquant_vec_kernel<kSrc, kDst, false, true, false><<<rl.grid, rl.block, 0, st>>>(a);
         } else {
-            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, false><<<rl.grid, rl.block, 0, st>>>(a)
-                         : antiquant_vec_kernel<kSrc, kDst, false, false><<<rl.grid, rl.block, 0, st>>>(a);
+            a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, false, false><<<rl.grid, rl.block, 0, st>>>(a)
+                         : antiquant_vec_kernel<kSrc, kDst, false, false, false><<<rl.grid, rl.block, 0, st>>>(a);
         }
     } else {
         size_t total = static_cast<size_t>(a.rows) * a.cols;
@@ -989,7 +1047,7 @@ __global__ __launch_bounds__(kThreads) void antiquant_policy_vec_kernel(AntiQuan
                 t = Fmt<kCt>::mul(t, Fmt<kCt>::cvt(s[e]));
                 v[e] = kCt == kDst ? t : aqp_saturate<kDst>(t);
             }
-            store8<kDst, true>(a.dst, static_cast<size_t>(r) * a.n + j, v);
+            store8<kDst, kNonTemporal>(a.dst, static_cast<size_t>(r) * a.n + j, v);
         }
     }
 }
@@ -1041,7 +1099,6 @@ template <int kDst, bool kE1M2, int kRows>
 __global__ __launch_bounds__(kThreads) void antiquant_fp4_kernel(AntiQuantPolicyArgs a)
 {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef u32x2 u32x2_any __attribute__((aligned(1)));  // (the scales may lie anywhere)
     const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
     if (j >= a.n) {
         return;
@@ -1095,7 +1152,7 @@ __global__ __launch_bounds__(kThreads) void antiquant_fp4_kernel(AntiQuantPolicy
                 const float p = v[e] * s[e];
                 v[e] = kDst == ASCQ_F16 ? aqp_saturate<ASCQ_F16>(p) : p;
             }
-            store8<kDst, true>(a.dst, static_cast<size_t>(r) * a.n + j, v);
+            store8<kDst, kNonTemporal>(a.dst, static_cast<size_t>(r) * a.n + j, v);
         }
     }
 }

@@ -748,3 +748,61 @@ def test_config2c_full_size_antiquant():
                           scale_width=11008, offset_height=1, offset_width=11008)
     orc.set_threads(16)
     assert np.array_equal(bits(dst), orc.antiquant(d, w, of, sc).view(np.uint16))
+
+
+# ------------------------------------------------------------------ rows of any width, tensors at any element
+@pytest.mark.parametrize("n", [7, 8, 9, 15, 17, 1023, 1025, 2049, 4099, 8191, 9661, 16383, 16385])
+@pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16, abi.F32])
+def test_quantisers_of_odd_widths_off_the_vector_alignment(n, src_dt):
+    """Widths on both sides of the vector's 8 columns and of the row kernels' limits, inputs and outputs one element past a
+    16-byte boundary; the bytes around the outputs stay as they are."""
+    m = 13
+    announce("quant odd widths", n, src_dt)
+    rng = np.random.default_rng(n)
+    x, _ = src_array(rng, (m, n), src_dt, 3.0)
+    xd = to_dev(np.concatenate([x.reshape(-1)[:1], x.reshape(-1)]), "bf16" if src_dt == abi.BF16 else None)[1:].view(m, n)
+    room = torch.full((m * n + 16,), 55, dtype=torch.int8, device=DEV)
+    q, ts = room[1:1 + m * n].view(m, n), torch.empty(m, dtype=torch.float32, device=DEV)
+    ops.dynamic_quant_per_token(xd, q, ts)
+    wq, wts = orc.dynamic_quant_per_token(src_dt, x)
+    assert np.array_equal(q.cpu().numpy(), wq) and np.array_equal(ts.cpu().numpy(), wts)
+    assert room[0] == 55 and (room[1 + m * n:] == 55).all()
+    s, _ = src_array_uniform(rng, (n,), src_dt, 5, 40)
+    sd = to_dev(np.concatenate([s[:1], s]), "bf16" if src_dt == abi.BF16 else None)[1:]
+    room.fill_(55)
+    ops.ascend_quant(q, xd, sd, 2.5)
+    d = abi.QuantDesc(policy=abi.PER_CHANNEL, src_dtype=src_dt, scale_dtype=src_dt, compute=abi.COMPUTE_F16,
+                      offset_kind=abi.OFFSET_SCALAR, offset=2.5, round_mode=abi.CAST_RINT, n=n,
+                      cal_count=m * n)
+    assert np.array_equal(q.cpu().numpy(), orc.quant(d, x, s))
+    assert room[0] == 55 and (room[1 + m * n:] == 55).all()
+
+
+@pytest.mark.parametrize("n", [7, 8, 10, 22, 24, 1030, 4098])
+@pytest.mark.parametrize("int4", [False, True])
+@pytest.mark.parametrize("dst_dt", [abi.F16, abi.BF16])
+@pytest.mark.parametrize("has_offset", [True, False])
+def test_antiquant_of_odd_widths_off_the_vector_alignment(n, int4, dst_dt, has_offset):
+    """The same for AscendAntiQuant: sources, parameters and outputs one element past a 16-byte boundary."""
+    if int4:
+        n += n % 2
+    k, g = 30, 3
+    announce("antiquant odd widths", n, int4, dst_dt, has_offset)
+    rng = np.random.default_rng(n)
+    w = rng.integers(-8, 8, (k, n)).astype(np.int8) if int4 else rng.integers(-128, 128, (k, n)).astype(np.int8)
+    sc, _ = src_array_uniform(rng, (g, n), dst_dt, -2, 2)
+    of, _ = src_array_uniform(rng, (g, n), dst_dt, -9, 9)
+    kind = "bf16" if dst_dt == abi.BF16 else None
+
+    def off(a, kd=None):
+        return to_dev(np.concatenate([a.reshape(-1)[:1], a.reshape(-1)]), kd)[1:].view(*a.shape)
+    src = pack_int4(w) if int4 else w
+    room = torch.zeros(k * n + 16, dtype=TDT[dst_dt], device=DEV)
+    dst = room[1:1 + k * n].view(k, n)
+    info = ops.AntiQuantShapeInfo(g, n, g, n)
+    ops.ascend_antiquant(dst, off(src), off(of, kind) if has_offset else None, off(sc, kind), k, info, int4=int4)
+    d = abi.AntiQuantDesc(src_dtype=abi.I4 if int4 else abi.I8, dst_dtype=dst_dt, has_offset=int(has_offset), k=k, n=n,
+                          scale_height=g, scale_width=n, offset_height=g, offset_width=n)
+    want = orc.antiquant(d, src, of if has_offset else None, sc)
+    assert np.array_equal(bits(dst), want.view(np.uint16))
+    assert room[0] == 0 and not room[1 + k * n:].any()
