@@ -806,6 +806,15 @@ double passes_estimate(uint32_t m, uint32_t slabs, uint32_t k, bool sum_form, ui
 }
 
 }  // namespace
+
+double w4a16_packed_estimate(uint32_t m, uint32_t n, uint32_t k)
+{
+    const double other = m > kMaxPassRows && k <= kWqMaxK ? wq_gemm_estimate(m, n, k)
+                                                          : passes_estimate(m, (n + kSlabCols - 1u) / kSlabCols, k, false, device_compute_units());
+    const double rows = wq_rows_estimate(m, n, k, true);
+    return k <= kWqMaxK && rows < other ? rows : other;
+}
+
 }  // namespace ascq
 
 using namespace ascq;

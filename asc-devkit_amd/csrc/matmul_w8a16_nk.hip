@@ -534,9 +534,43 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
                     bool channel_sum);
 
 // Weights given as [k, n] and many rows: transposed once into the caller's workspace (k * n bytes), then the tile GEMM.
-bool w8a16_kn_gemm_supported(uint32_t m, uint32_t k, const void* x, const void* w)
+// us of passes of 16 rows (51 random calls, nine tenths within 15 %): a launch, and per 1024 k a time that grows with the columns
+static double passes_estimate(uint32_t m, uint32_t n, uint32_t k)
 {
-    return m > 96u && k % kGK == 0 && k <= kWqMaxK && aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0;
+    const uint32_t cus = device_compute_units(), n_groups = (n + 15u) / 16u;
+    uint32_t per = (n_groups + cus - 1u) / cus;
+    per = per > kMaxGroups ? kMaxGroups : per;
+    const uint32_t grid = (n_groups + per - 1u) / per;
+    const double runs = static_cast<double>((grid + cus - 1u) / cus) * ((k + 1023u) / 1024u);
+    return ((m + kRows - 1u) / kRows) * (3.25 + runs * (0.31 + 0.875 * per));
+}
+
+static bool tiles_apply(uint32_t m, uint32_t k) { return m > kDecodeRows && k % kGK == 0 && k <= kWqMaxK; }
+
+double w8a16_nk_estimate(uint32_t m, uint32_t n, uint32_t k)
+{
+    const double other = tiles_apply(m, k) ? wq_gemm_estimate(m, n, k) : passes_estimate(m, n, k);
+    const double rows = wq_rows_estimate(m, n, k, false);
+    return k % kGK == 0 && k <= kWqMaxK && rows < other ? rows : other;
+}
+
+// Weights as [k, n]: whether they are transposed first.  Above 96 rows always; from 17 on where the transposition (3 us and
+// 0.55 us per MB of weights) and the [n, k] form are expected to be ahead of a pass over the weights per 32 rows (14 us, another
+// 12 once the weights are some 16 MB, and 0.2 per MB; fits to 45 random calls): 65 x 2048 x 3328 58 against 15 us,
+// 64 x 6400 x 1632 57 and 23, 24 x 9472 x 3136 33 and 33, 17 x 5248 x 11712 34 and 57.
+bool w8a16_kn_transposed(uint32_t m, uint32_t n, uint32_t k)
+{
+    if (k % kGK != 0 || k > kWqMaxK) {
+        return false;
+    }
+    const double mb = 1e-6 * k * n;
+    return m > 96u || (m > 16u && k % kRun == 0 && 3.0 + 0.55 * mb + w8a16_nk_estimate(m, n, k) <
+                                                   0.9 * ((m + 31u) / 32u) * (14.0 + 12.0 * (1.0 - __builtin_exp(-mb / 8.0)) + 0.2 * mb));
+}
+
+bool w8a16_kn_gemm_supported(uint32_t m, uint32_t n, uint32_t k, const void* x, const void* w)
+{
+    return w8a16_kn_transposed(m, n, k) && aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0;
 }
 
 int launch_w8a16_kn_via_transpose(const void* x, const void* w, const void* scale, const void* offset, void* y,
@@ -616,7 +650,7 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
     per = per > kMaxGroups ? kMaxGroups : per;
     p.groups = per;
     const uint32_t grid = (n_groups + per - 1u) / per;
-    const bool tiles = m > kDecodeRows && k % kGK == 0 && k <= kWqMaxK;
+    const bool tiles = tiles_apply(m, k);
     if (k % kGK == 0) {
         WqParams q{};
         q.x = static_cast<const uint16_t*>(x);
@@ -630,10 +664,7 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
         q.out_f32 = p.out_f32;
         q.scale_bits = scale_bits;
         q.offset_bits = offset_bits;
-        // passes of 16 rows (51 random calls, nine tenths within 15 %): a launch, and per 1024 k a time that grows with the columns
-        const double runs = static_cast<double>((grid + cus - 1u) / cus) * ((k + 1023u) / 1024u);
-        const double passes = ((m + kRows - 1u) / kRows) * (3.25 + runs * (0.31 + 0.875 * per));
-        if (wq_rows_ahead(q, false, false, has_offset, tiles ? wq_gemm_estimate(m, n, k) : passes, st)) {
+        if (wq_rows_ahead(q, false, false, has_offset, tiles ? wq_gemm_estimate(m, n, k) : passes_estimate(m, n, k), st)) {
             return launch_status("ascq_matmul_w8a16");
         }
         // more rows than a few passes of the decode kernel: the tile GEMM reads the weights once per 128 or 256 rows

@@ -1009,16 +1009,30 @@ bool fast_ok(const ascq_w4a16_desc* d, const void* x, const void* w, const void*
            static_cast<uint64_t>((d->n + kColsPerBlock - 1u) / kColsPerBlock) * (d->k / kChunkRows) < (1ull << 31);
 }
 
-// Many rows: the weights are packed into the workspace and the tile GEMM of the packed form runs on them, instead of a
-// pass over the weights per 32 rows: k = 5632, n = 1408, 1149 rows 1069 -> 68 us; k = 11648, n = 11520, 128 rows 179 ->
-// 142 us.  The line lies where the two meet at k = n = 8192 (96 rows 107 and 103 us; 65 rows 91 and 103 us).
+// Many rows: the weights are packed into the workspace and the kernels of the packed form run on them, instead of a
+// pass over the weights per 32 rows: k = 5632, n = 1408, 1149 rows 1069 -> 68 us.  Above 96 rows always; from 5 on where the
+// repacking (4.5 us and 0.42 us per MB of weights) and the packed form are expected to be ahead of the passes (up to 16 rows 9.5 us and
+// 0.3 per row, above 17; another 8 or 12 once the weights are some 10 MB, and 0.32 or 0.3 per MB; fits to 45 random calls): 64 x 1792 x
+// 22496 76 against 34 us, 33 x 2304 x 1152 32 and 11, 16 x 8448 x 1920 32 and 19, 8 x 4864 x 4288 22 and 21, 12 x 8448 x 13088 37 and 52.
+bool packed_ahead(const ascq_w4a16_desc* d)
+{
+    if (d->m > 96u) {
+        return true;
+    }
+    const double mb = 0.5e-6 * d->k * d->n, filled = 1.0 - __builtin_exp(-mb / 5.0);
+    const double pass = d->m <= kTileRows ? 9.5 + 0.3 * d->m + 8.0 * filled + 0.32 * mb : 17.0 + 12.0 * filled + 0.3 * mb;
+    // (more than 128 groups along k: the passes over packed weights do not take every shape)
+    return d->m > 4u && d->k / d->group_size <= 128u && 4.5 + 0.42 * mb + w4a16_packed_estimate(d->m, d->n, d->k) <
+                            0.9 * ((d->m + 2u * kTileRows - 1u) / (2u * kTileRows)) * pass;
+}
+
 bool pack_first(const ascq_w4a16_desc* d)
 {
     const uint32_t g32 = d->group_size / 32u;
     size_t bytes = 0;
-    return d->m > 96u && d->k <= kWqMaxK && d->k % 128u == 0 && d->n % 8u == 0 && d->group_size % 32u == 0 && (g32 & (g32 - 1u)) == 0 &&
+    return d->k <= kWqMaxK && d->k % 128u == 0 && d->n % 8u == 0 && d->group_size % 32u == 0 && (g32 & (g32 - 1u)) == 0 &&
            ascq_pack_weight_w4_size(d->k, d->n, &bytes) == ASCQ_OK && bytes < (1ull << 31) &&
-           static_cast<uint64_t>(d->k / d->group_size) * d->n * 2u < (1ull << 31);
+           static_cast<uint64_t>(d->k / d->group_size) * d->n * 2u < (1ull << 31) && packed_ahead(d);
 }
 
 }  // namespace
@@ -1165,7 +1179,8 @@ bool w8a16_nk_supported(uint32_t k, const void* x, const void* w);
 int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void* offset, void* y, uint32_t m, uint32_t n,
                     uint32_t k, bool has_offset, bool out_f32, uint32_t scale_bits, uint32_t offset_bits, hipStream_t st,
                     bool channel_sum);
-bool w8a16_kn_gemm_supported(uint32_t m, uint32_t k, const void* x, const void* w);
+bool w8a16_kn_transposed(uint32_t m, uint32_t n, uint32_t k);
+bool w8a16_kn_gemm_supported(uint32_t m, uint32_t n, uint32_t k, const void* x, const void* w);
 int launch_w8a16_kn_via_transpose(const void* x, const void* w, const void* scale, const void* offset, void* y,
                                   uint32_t m, uint32_t n, uint32_t k, bool has_offset, bool out_f32, uint32_t scale_bits,
                                   uint32_t offset_bits, void* workspace, hipStream_t st);
@@ -1207,7 +1222,7 @@ extern "C" int ascq_matmul_w8a16_workspace_size(const ascq_w8a16_desc* d, size_t
         return ASCQ_OK;
     }
     *bytes = (d->n % 16 == 0 && d->k % kChunkRows == 0) ? w8a16_workspace_need(d->n, d->k) : 0;
-    if (d->m > 96u && d->k % 64u == 0) {
+    if (w8a16_kn_transposed(d->m, d->n, d->k)) {
         // many rows: the weights are transposed into the workspace once and a tile GEMM runs on them (a smaller
         // workspace is accepted and the weight-stream kernel then passes over the weights once per 32 rows)
         const size_t need = static_cast<size_t>(d->k) * d->n;
@@ -1263,7 +1278,7 @@ extern "C" int ascq_matmul_w8a16(const ascq_w8a16_desc* d, void* y, const void* 
         return launch_w8a16_nk(x, w, p.scale, p.offset, y, d->m, d->n, d->k, d->has_offset != 0, d->out_dtype == ASCQ_F32,
                                p.scale_bits, p.offset_bits, st, d->mode == ASCQ_W8A16_CHANNEL_SUM);
     }
-    if (w8a16_kn_gemm_supported(d->m, d->k, x, w) && workspace != nullptr && aligned16(workspace) &&
+    if (w8a16_kn_gemm_supported(d->m, d->n, d->k, x, w) && workspace != nullptr && aligned16(workspace) &&
         workspace_bytes >= static_cast<size_t>(d->k) * d->n) {
         return launch_w8a16_kn_via_transpose(x, w, p.scale, p.offset, y, d->m, d->n, d->k, d->has_offset != 0,
                                              d->out_dtype == ASCQ_F32, p.scale_bits, p.offset_bits, workspace, st);

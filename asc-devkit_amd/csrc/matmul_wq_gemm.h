@@ -69,5 +69,12 @@ double wq_gemm_estimate(uint32_t m, uint32_t n, uint32_t k);
 // Whole-k tiles of 16 to 64 rows and columns (matmul_wq_rows.hip): runs the call and returns true where they are expected to
 // beat `other_us`, what the caller would do instead.  sum: int4 in group-sum form (group_size a multiple of 128).
 bool wq_rows_ahead(const WqParams& p, bool int4, bool sum, bool has_offset, double other_us, hipStream_t st);
+// us that the best of those tiles is expected to take
+double wq_rows_estimate(uint32_t m, uint32_t n, uint32_t k, bool int4);
+
+// us that a call on packed int4 (per weight) or [n, k] int8 weights is expected to take with 5 rows and more: for callers that
+// would have to bring their weights into that form first
+double w4a16_packed_estimate(uint32_t m, uint32_t n, uint32_t k);
+double w8a16_nk_estimate(uint32_t m, uint32_t n, uint32_t k);
 
 }  // namespace ascq

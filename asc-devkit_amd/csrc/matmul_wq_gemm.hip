@@ -483,7 +483,7 @@ void wq_launch(WqParams p, bool int4, bool has_offset, hipStream_t st)
 // the rounds sets the time it makes no difference, k = 8192, n = 28672, 2048 rows).
 struct WqShape {
     double c256, c128, csmall;  // us per K step of each tile shape
-    uint32_t t256, tsmall, rounds;
+    uint32_t t256, t128, tsmall, rounds;
     bool halve;
 };
 static WqShape wq_shape(uint32_t m, uint32_t n)
@@ -493,22 +493,28 @@ static WqShape wq_shape(uint32_t m, uint32_t n)
     WqShape s{};
     s.t256 = up(m, 256u) * up(n, 256u);
     s.tsmall = up(m, 128u) * up(n, 128u);
-    const uint32_t t128 = up(m, 128u) * up(n, 256u), rest = s.t256 % cus;
+    s.t128 = up(m, 128u) * up(n, 256u);
+    const uint32_t rest = s.t256 % cus;
     s.rounds = s.t256 / cus;
     const double tail = up(2u * rest, cus) * 1.11;
     s.halve = rest != 0 && tail < 1.62;
     s.c256 = s.rounds * 1.62 + (rest == 0 ? 0.0 : s.halve ? tail : 1.62);
-    s.c128 = up(t128, cus) * 1.11;
+    s.c128 = up(s.t128, cus) * 1.11;
     s.csmall = s.tsmall <= cus ? 0.62 : up(s.tsmall, 2u * cus) * 1.2;
     return s;
 }
 
 // 3.5 us and 0.91 of the estimate above (214 random calls of 33 rows and more that leave the chip partly idle, half of them within 5 %,
-// nine tenths within 20 %).
+// nine tenths within 20 %).  One round of 128 x 256 tiles on at most three quarters of the compute units has their share of the way to
+// memory as well, and takes 0.77 of it: int4 641 x 6272 x 6656 79 us (102 without that factor, and the whole-k tiles that were then
+// taken needed 88), 403 x 8064 x 12032 102 (131), 493 x 4096 x 12160 55 (68); at 236 tiles of 256 the estimate holds.
 double wq_gemm_estimate(uint32_t m, uint32_t n, uint32_t k)
 {
     const WqShape s = wq_shape(m, n);
-    const double c = s.c256 < s.c128 ? s.c256 : s.c128;
+    double c = s.c256 < s.c128 ? s.c256 : s.c128;
+    if (s.t128 <= device_compute_units() * 3u / 4u) {
+        c *= 0.77;
+    }
     return 3.5 + 0.91 * (s.csmall < c ? s.csmall : c) * (k / kBK);
 }
 

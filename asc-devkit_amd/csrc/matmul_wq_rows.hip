@@ -331,29 +331,45 @@ struct RowsShape {
 constexpr RowsShape kShapes[] = {{16, 16, 3.00, 0.880, 4.48, 1.34}, {32, 16, 2.20, 0.745, 2.86, 1.06}, {32, 32, 2.80, 0.990, 4.00, 1.53},
                                  {64, 16, 1.75, 0.620, 2.44, 0.82}, {64, 32, 2.30, 0.745, 3.31, 1.05}, {64, 64, 3.30, 1.100, 5.13, 1.51}};
 
+// the shape that is expected to be fastest; its time
+int best_shape(uint32_t m, uint32_t n, uint32_t k, bool int4, double& us)
+{
+    const uint32_t cus = device_compute_units(), unit = int4 ? 2u : 1u;
+    auto up = [](uint64_t a, uint64_t b) { return (a + b - 1u) / b; };
+    int at = 0;
+    us = 1e30;
+    for (int i = 0; i < static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+        const RowsShape& s = kShapes[i];
+        const uint64_t tiles = up(m, s.bm) * up(n, s.bn);
+        const uint64_t stages = up(up(k / 64u / unit, kWaves) * unit, 64u / s.bm);
+        const double t = up(tiles, cus) * (int4 ? s.round4 + s.stage4 * stages : s.round8 + s.stage8 * stages);
+        if (tiles < (1ull << 31) - 8u && t < us) {
+            us = t;
+            at = i;
+        }
+    }
+    us += int4 ? 1.35 : 1.0;
+    return at;
+}
+
 }  // namespace
+
+double wq_rows_estimate(uint32_t m, uint32_t n, uint32_t k, bool int4)
+{
+    double us;
+    best_shape(m, n, k, int4, us);
+    return us;
+}
 
 bool wq_rows_ahead(const WqParams& p, bool int4, bool sum, bool has_offset, double other_us, hipStream_t st)
 {
     if (p.k > kWqMaxK) {
         return false;
     }
-    const uint32_t cus = device_compute_units(), unit = int4 ? 2u : 1u;
-    auto up = [](uint64_t a, uint64_t b) { return (a + b - 1u) / b; };
-    double best = 1e30;
-    int at = 0;
-    for (int i = 0; i < static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
-        const RowsShape& s = kShapes[i];
-        const uint64_t tiles = up(p.m, s.bm) * up(p.n, s.bn);
-        const uint64_t stages = up(up(p.k / 64u / unit, kWaves) * unit, 64u / s.bm);
-        const double us = up(tiles, cus) * (int4 ? s.round4 + s.stage4 * stages : s.round8 + s.stage8 * stages);
-        if (tiles < (1ull << 31) - 8u && us < best) {
-            best = us;
-            at = i;
-        }
-    }
+    double us;
+    const int at = best_shape(p.m, p.n, p.k, int4, us);
     // (5 % ahead, or the two are as good as each other)
-    if (best + (int4 ? 1.35 : 1.0) > 0.95 * other_us) {
+    if (us > 0.95 * other_us) {
         return false;
     }
     WqParams q = p;

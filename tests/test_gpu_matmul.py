@@ -823,6 +823,33 @@ def test_w4a16_packed_small(m, k, n, gs, offset):
     w4_check(y.cpu().numpy(), orc.matmul_w4a16(d, x, wp, sc, of), x)
 
 
+@pytest.mark.parametrize("m,k,n,gs", [(5, 1024, 1152, 64), (16, 1408, 264, 128), (17, 1792, 1440, 32), (33, 2304, 1152, 128), (64, 1152, 2976, 64),
+                                       (96, 1280, 96, 128), (48, 4224, 32, 32)])
+@pytest.mark.parametrize("offset", [True, False])
+def test_w4a16_few_rows_repacked_or_in_passes(m, k, n, gs, offset):
+    """[k, n / 2] weights that are repacked into the workspace first and, with a workspace that has no room for that, passes over
+    them (n a multiple of 32; (48, 4224, 32, 32) has more groups than the repacked form is taken for): the oracle's values both ways."""
+    import ctypes as C
+    announce("w4a16 few rows", m, k, n, gs, offset)
+    rng = np.random.default_rng(m + k + n)
+    x, wp, sc, of = w4_case(rng, m, k, n, gs, offset)
+    d = abi.W4A16Desc(m=m, n=n, k=k, group_size=gs, has_offset=int(offset))
+    want = orc.matmul_w4a16(d, x, wp, sc, of)
+    need, packed = C.c_size_t(0), C.c_size_t(0)
+    lib = ops.load_library()
+    assert lib.ascq_matmul_w4a16_workspace_size(C.byref(d), C.byref(need)) == abi.OK
+    assert lib.ascq_pack_weight_w4_size(k, n, C.byref(packed)) == abi.OK
+    for room in [need.value] + ([packed.value - 16] if n % 32 == 0 else []):
+        y = torch.zeros((m, n), dtype=torch.float16, device=DEV)
+        ws = torch.zeros(room, dtype=torch.uint8, device=DEV)
+        xd, wd, sd, od = to_dev(x), to_dev(wp), to_dev(sc), to_dev(of) if offset else None
+        rc = lib.ascq_matmul_w4a16(C.byref(d), ops._ptr(y), ops._ptr(xd), ops._ptr(wd), ops._ptr(sd), ops._ptr(od), ops._ptr(ws), room, ops._stream())
+        if rc == abi.EINVAL and room < need.value:
+            continue      # too small for the passes as well: refused
+        assert rc == abi.OK
+        w4_check(y.cpu().numpy(), want, x)
+
+
 def test_w4a16_packed_multi_pass_and_repeatable():
     """k too long for one pass of staged activations (several passes per wavefront), and two calls give identical bits."""
     m, k, n, gs = 4, 24576, 256, 128
@@ -1268,6 +1295,29 @@ def test_w8a16_rows_beyond_thirty_two_bit_offsets():
     y = torch.full((m, n), -1.0, dtype=torch.float32, device=DEV)
     ops.matmul_w8a16(y, x, w, None, 1.0, trans_b=True)
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 1280, 1040), (24, 1408, 36), (33, 2304, 1152), (65, 1024, 2688), (96, 128, 7)])
+@pytest.mark.parametrize("offset", [True, False])
+def test_w8a16_few_rows_transposed_first(m, k, n, offset):
+    """[k, n] weights that are transposed into the workspace first: the value in 64 bits, and the call on [n, k] weights; columns
+    that are no multiple of 16 among them."""
+    announce("w8a16 few rows on [k, n]", m, k, n, offset)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + k + n)
+    x = torch.randn((m, k), device=DEV, generator=g).half()
+    w = torch.randint(-128, 128, (k, n), device=DEV, dtype=torch.int8, generator=g)
+    sc = (torch.rand(n, device=DEV, generator=g) * 0.01 + 0.001).half()
+    of = (torch.rand(n, device=DEV, generator=g) * 16 - 8).half() if offset else None
+    y0, y1 = torch.zeros((m, n), dtype=torch.float16, device=DEV), torch.zeros((m, n), dtype=torch.float16, device=DEV)
+    ops.matmul_w8a16(y0, x, w, of, sc)
+    ops.matmul_w8a16(y1, x, w.t().contiguous(), of, sc, trans_b=True)
+    wf = w.half() + of if offset else w.half()
+    want = x.double().cpu() @ (wf * sc).double().cpu()
+    # two roundings of a result in half, fp32 sums: 2^-11 of the value and 1e-6 of the sum of magnitudes
+    room = 2.0 ** -11 * want.abs() + 1e-6 * (x.double().abs().cpu() @ (wf * sc).double().abs().cpu()) + 1e-7
+    assert ((y0.double().cpu() - want).abs() <= room).all()
+    assert torch.allclose(y0.float(), y1.float(), rtol=2.0 ** -10, atol=1e-3)
 
 
 @pytest.mark.parametrize("m,k,n", [(33, 128, 7), (128, 256, 248), (129, 384, 264), (257, 640, 521), (300, 128, 1034)])
