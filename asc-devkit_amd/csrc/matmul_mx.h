@@ -36,6 +36,10 @@ __device__ __forceinline__ void mx_store(const MxParams& p, size_t idx, float v)
 bool mx_decode_supported(const MxParams& p);
 int launch_mx_decode(const MxParams& p, bool tile_shape, hipStream_t st);
 
+// matmul_mx_ring.hip: tiles of 64 x 64 (shape 0), 128 x 64 and 128 x 128 for medium sizes; formats as the matrix instruction's codes (0
+// e4m3, 1 e5m2, 4 e2m1, that as b beside an 8-bit a or as both), k a multiple of 128, of 256 with a 4-bit operand
+int launch_mx_ring(const MxParams& p, int shape, int code_a, int code_b, hipStream_t st);
+
 // matmul_mx_six.hip: two e1m2 operands, k a multiple of 128, on a workspace of mx_six_bytes (16-byte aligned)
 size_t mx_six_bytes(uint32_t m, uint32_t n, uint32_t k);
 int launch_mx_six(const MxParams& p, void* workspace, hipStream_t st);

@@ -552,37 +552,90 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
 }
 
-// Tile shapes (64 rows and more): whether the kernel of matmul_mx_decode.hip is expected to be ahead of the tile kernel.
-// Both times are estimated, in us.  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
-// meets 4-bit b) by 32 columns, each round so much per 1024 of k: 1.15 (e2m1 pairs), 1.85 (8-bit b), 0.95 (the 32-row
-// form), 2.0 (e1m2 beside e2m1).  Tiles: rounds of 256 x 256 tiles, 1.3 per K step, and the passes that widen 4-bit operands, 1 per 3 MB
-// of their codes.  Measured at n = k = 8192, decode
-// against tiles: 64 rows e2m1 13.0 and 42.4, e4m3 20.7 and 78; 128 rows e4m3 34 and 79; 256 rows e2m1 41 and 47, e4m3 64 and
-// 85; n = 14336, k = 4096, 128 rows: 28 and 26, 36 and 44; n = 1024, k = 14336, 256 rows: 16 and 69, 29 and 147.
+// us that a call of the tiles' shapes is expected to take: in the kernel of matmul_mx_decode.hip, on 256 x 256 tiles, on the smaller ones of
+// matmul_mx_ring.hip (and the best of their shapes).
+struct MxPlan {
+    double decode, tiles, ring;
+    int shape;
+};
+
+// whether the ring tiles take a call; and whether they take its operands as they are
+inline bool mx_ring_supported(const MxParams& p)
+{
+    const uint32_t size = p.out_dtype == ASCQ_F32 ? 4u : 2u;
+    return p.k <= 1u << 23 && p.n <= kMxBufferCols && (reinterpret_cast<uintptr_t>(p.c) & (size - 1u)) == 0 &&
+           !(p.a_format == ASCQ_QDST_FP4_E1M2 && p.b_format == ASCQ_QDST_FP4_E1M2);
+}
+inline bool mx_ring_mixed(const MxParams& p) { return is_fp8(p.a_format) && p.b_format == ASCQ_QDST_FP4_E2M1 && p.k % 256u == 0; }
+
+// All are fits to 370 random calls of 64 to 4096 rows, k and n of 1024 to 14336 (ring tiles within 4 to 7 % for nine in ten, the others within 6
+// to 20 %).  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a meets 4-bit b) by 32 columns, each
+// with a part of its own and one per 1024 of k.  Tiles of 256 x 256: so much per round and per K step, which takes longer the more of the
+// chip has a tile, and the passes that widen 4-bit operands.  Ring: the same for each shape (tiles that share the chip with
+// few others wait less for memory).  Measured, in us, tiles, decode and the three ring shapes:
+//   e4m3 152 x 3680 x 2816   29.2, 15.6,  9.4, 10.8, 13.3      e2m1 378 x 2016 x 3584  21.6, 13.5,  7.7,  9.2, 11.9
+//   e4m3 441 x 4032 x 1792   26.9, 24.7, 13.2,  9.1, 10.5      e2m1 999 x 1856 x 3328  27.2, 26.0, 13.5,  9.7, 11.7
+//   e4m3 1370 x 2800 x 8448  89.2, 144, 77.5, 52.4, 39.0       e2m1 470 x 5888 x 11520 63.4, 74.6, 45.5, 41.4, 31.6
+//   e4m3 66 x 2512 x 7936    73.9, 15.4, 18.3, 21.3, 27.2      e2m1 64 x 4064 x 6912   35.3,  9.9, 10.5, 13.1, 18.1
+//   e4m3 3300 x 8192 x 1024  45.5, 236, 110, 70.7, 59.9        e4m3 x e2m1 507 x 6896 x 7936 104, 111, 54.7, 41.4, 31.1
 // Two e1m2 operands have constants of their own, fits to 500 random calls of 64 to 3000 rows (decode and tiles within 7 and 11 % for eight in ten): a
 // round of decode workgroups also takes 3.6 to start and store, a K step of tiles 0.6 and as much again as the chip fills up; rows of an odd number
 // of values are stored one by one, 16.5 a round (636 x 3729 x 1024 26.6 and 34.7, 636 x 3728 x 1024 26.1 and 17.6; 165 x
 // 12032 x 640 25.4 and 16.3; 874 x 2000 x 8960 75 and 63).
-bool mx_decode_preferred(const MxParams& p)
+MxPlan mx_plan(const MxParams& p)
 {
     const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
     const bool two4 = p.a_format == ASCQ_QDST_FP4_E2M1 && p.b_format == ASCQ_QDST_FP4_E2M1;
     const bool six = p.a_format == ASCQ_QDST_FP4_E1M2 && p.b_format == ASCQ_QDST_FP4_E1M2;
     const double cus = device_compute_units();
+    MxPlan plan{0.0, 0.0, 1e30, 0};
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
     const double decode_rounds = rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u));
     const double blocks = static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN);
     if (six) {
         const double filled = blocks < cus ? blocks / cus : 1.0, store = p.n % 2u != 0 ? 16.5 : 0.0;
-        return 1.7 + decode_rounds * (1.73 * p.k / 1024.0 + 3.6) <
-               11.9 + 0.137e-6 * (static_cast<double>(p.m) + p.n) * p.k + rounds(blocks) * (0.6 * (1.0 + filled) * p.k / 128.0 + store);
+        plan.decode = 1.7 + decode_rounds * (1.73 * p.k / 1024.0 + 3.6);
+        plan.tiles = 11.9 + 0.137e-6 * (static_cast<double>(p.m) + p.n) * p.k + rounds(blocks) * (0.6 * (1.0 + filled) * p.k / 128.0 + store);
+        return plan;
     }
-    const double per_k = two4 ? 1.15 : b8 ? 1.85 : a8 ? 0.95 : 2.0;
-    const double decode = 4.0 + decode_rounds * per_k * p.k / 1024.0;
-    const double widen = two4 ? 0.0 : ((a8 ? 0.0 : static_cast<double>(p.m) * p.k) + (b8 ? 0.0 : static_cast<double>(p.n) * p.k)) / 6e6;
-    const double tiles = 5.0 + widen + rounds(blocks) * 1.3 * p.k / (two4 ? 256.0 : 128.0);
-    return decode < tiles;
+    // 8-bit pairs; e2m1 pairs; 8-bit a with e2m1 b
+    const bool mixed = mx_ring_mixed(p);
+    const int kind = two4 ? 1 : mixed ? 2 : 0;
+    const double k1024 = p.k / 1024.0, steps = p.k / (two4 ? 256.0 : 128.0);
+    if (!a8 && !b8 && !two4) {  // e1m2 beside e2m1
+        plan.decode = 4.0 + decode_rounds * 2.0 * k1024;
+    } else {
+        static constexpr double kDecode[3][3] = {{1.3, 1.60, 2.9}, {1.6, 0.83, 3.2}, {1.6, 0.84, 2.3}};
+        const double* const c = kDecode[two4 ? 1 : a8 && !b8 ? 2 : 0];
+        plan.decode = c[0] + decode_rounds * (c[1] * k1024 + c[2]);
+    }
+    const double widen_a = two4 || a8 ? 0.0 : static_cast<double>(p.m) * p.k / 6e6, widen_b = two4 || b8 ? 0.0 : static_cast<double>(p.n) * p.k / 6e6;
+    const double widen = widen_a + widen_b == 0.0 ? 0.0 : 5.0 + 1.9 * (widen_a + widen_b), filled = blocks < cus ? blocks / cus : 1.0;
+    plan.tiles = 8.0 + widen + rounds(blocks) * steps * (1.08 + (two4 ? 0.91 : 0.5) * filled) + 9.0 * (rounds(blocks) - 1.0);
+    if (mx_ring_supported(p)) {
+        struct Shape {
+            uint32_t bm, bn;
+            double start, step, fill, round;
+        };
+        static constexpr Shape kShapes[3][3] = {
+            {{64, 64, 3.8, 0.225, 0.04, 2.2}, {128, 64, 4.1, 0.27, 0.085, 2.5}, {128, 128, 4.7, 0.357, 0.155, 4.0}},
+            {{64, 64, 3.8, 0.23, 0.068, 2.1}, {128, 64, 4.2, 0.29, 0.15, 2.5}, {128, 128, 4.7, 0.47, 0.215, 3.2}},
+            {{64, 64, 3.8, 0.27, 0.10, 2.1}, {128, 64, 4.1, 0.45, 0.16, 2.4}, {128, 128, 5.0, 0.70, 0.245, 3.7}}};
+        const double ring_steps = mixed ? p.k / 256.0 : steps;
+        for (int i = 0; i < 3; ++i) {
+            const Shape& s = kShapes[kind][i];
+            const double tiles = static_cast<double>((p.m + s.bm - 1u) / s.bm) * ((p.n + s.bn - 1u) / s.bn);
+            const double whole = __builtin_floor(tiles / cus), rest = tiles / cus - whole;
+            const double us = s.start + (mixed ? 0.0 : widen) + s.round * (rounds(tiles) - 1.0) +
+                              ring_steps * (whole * (s.step + s.fill) + (rest > 0.0 ? s.step + s.fill * rest : 0.0));
+            if (us < plan.ring) {
+                plan.ring = us;
+                plan.shape = i;
+            }
+        }
+    }
+    return plan;
 }
 
 int mx_validate(const ascq_mx_desc* d, const char* who)
@@ -654,7 +707,8 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
     const bool tile = mx_tile_shape_ok(d) && aligned16(a) && aligned16(b) && (reinterpret_cast<uintptr_t>(a_scale) & 7u) == 0 &&
                       (reinterpret_cast<uintptr_t>(b_scale) & 7u) == 0 &&
                       (need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned16(workspace)));
-    if (mx_decode_supported(p) && (!tile || mx_decode_preferred(p))) {
+    const MxPlan plan = tile ? mx_plan(p) : MxPlan{};
+    if (mx_decode_supported(p) && (!tile || (plan.decode < plan.tiles && plan.decode < plan.ring))) {
         return launch_mx_decode(p, tile, st);
     }
     if (!tile) {
@@ -679,11 +733,16 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         ws += rows * d->k;
         fmt = ASCQ_QDST_FP8_E4M3FN;
     };
+    const bool ring = plan.ring < plan.tiles;
     if (wa) {
         widen(p.a, fa, d->m);
     }
-    if (wb) {
+    if (wb && !(ring && mx_ring_mixed(p))) {
         widen(p.b, fb, d->n);
+    }
+    if (ring) {
+        auto code = [](int f) { return f == ASCQ_QDST_FP8_E4M3FN ? 0 : f == ASCQ_QDST_FP8_E5M2 ? 1 : 4; };
+        return launch_mx_ring(p, plan.shape, code(fa), code(fb), st);
     }
     const bool four = is_fp4(fa);  // (after the widening: both e2m1)
     p.row_bytes = four ? d->k / 2u : d->k;

@@ -121,6 +121,37 @@ def test_mx_enough_rows_for_the_tile_kernel(fa, fb, steps, more):
         mx_check(got[r0:r1], want, mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, fa, fb), is8(fa, fb))
 
 
+@pytest.mark.parametrize("fa,fb", [(E4, E4), (E4, E5), (E5, E4), (E5, E5), (F2, F2), (E4, F2), (E5, F2), (F2, E4), (E4, F1)])
+@pytest.mark.parametrize("m,n", [(131, 2801), (449, 2530), (700, 2999)])
+@pytest.mark.parametrize("steps,more,out", [(1, 0, torch.float32), (2, 8, torch.bfloat16), (3, 0, torch.float16), (6, 8, torch.float32), (9, 0, torch.bfloat16),
+                                            (17, 0, torch.float32)])
+def test_mx_ring_tiles(fa, fb, m, n, steps, more, out):
+    """Tiles of 64 x 64, 128 x 64 and 128 x 128 (one size each): fewer K steps than LDS stages, odd and even numbers of them, the last fetch of
+    16 scale bytes moved back inside the row and not, ragged rows and columns, every output type (16-bit ones in pairs and, odd n, one by
+    one), a bias.  An e2m1 b beside an 8-bit a is taken as it is where k is a multiple of 256, widened otherwise.  All columns of
+    the rows at the tiles' ends; past the last row nothing is written."""
+    k = steps * (256 if fa == fb == F2 else 128)
+    sk = max(16, (k // 32 + 7) // 8 * 8) + more
+    announce("mx ring tiles", fa, fb, m, n, k, sk, out)
+    rng = np.random.default_rng(m + steps + fa * 16 + fb)
+    a, b, sa, sb, bias = mx_case(rng, m, n, k, fa, fb, sk=sk, bias=True, lo=122, hi=133)
+    room = torch.zeros((m + 1) * n, dtype=out, device=DEV)
+    c = room[:m * n].view(m, n)
+    ops.matmul_mx(c, to_dev(a), to_dev(b), to_dev(sa), to_dev(sb), fa, fb, k, to_dev(bias))
+    assert not room[m * n:].any()
+    d = abi.MxDesc(m=m, n=n, k=k, scale_k=sk, a_format=fa, b_format=fb, out_dtype=abi.F32, has_bias=1)
+    got = c.float().cpu().numpy()
+    orc.set_threads(16)
+    for r0, r1 in ((0, 3), (62, 66), (126, 130), (m - 2, m)):
+        want = orc.matmul_mx(d, a, b, sa, sb, bias, rows=(r0, r1))[r0:r1].astype(np.float64)
+        absdot = mx_abs_dot(a[r0:r1], b, sa[r0:r1], sb, k, fa, fb) + np.abs(bias)
+        g = got[r0:r1].astype(np.float64)
+        if out == torch.float16:
+            want = np.clip(want, -65504.0, 65504.0)          # the reference's saturating cast
+        eps = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[out]     # one rounding of the result
+        assert np.all(np.abs(g - want) <= (1e-3 if is8(fa, fb) else 4e-6) * absdot + eps * np.abs(want) + 1e-7)
+
+
 @pytest.mark.parametrize("m,n,k", [(8200, 1100, 128), (4100, 1128, 384), (4129, 1033, 640), (4096, 1056, 1024)])
 def test_mx_e1m2_pairs_on_the_tile_kernel(m, n, k):
     """Enough rows for two e1m2 operands to be widened into units of 32 rows x 64 k: one K step, odd and even numbers of
