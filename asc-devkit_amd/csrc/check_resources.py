@@ -19,7 +19,7 @@ import sys
 GUARDED = ("gemm_nkl_kernel", "w8a16_nk_stream_kernel", "w4a16_gemv_kernel", "w4a16_tile_kernel", "w8a16_tile_kernel", "gemm_stream_kernel", "gemm_dma_kernel",
            "gemm_dma_dual_kernel", "gemm_dma_group_kernel", "w4a16_packed_kernel", "w4a16_packed_rows_kernel",
            "gemm_packed_kernel", "gemm_packed_dyn_kernel", "gemm_ws_kernel", "mx_tile_kernel", "mx_decode_kernel", "wq_gemm_kernel",
-           "gemm_ring_kernel", "mx_six_kernel", "mx_ring_kernel", "wq_rows_kernel")
+           "gemm_ring_kernel", "gemm_group_ring_kernel", "mx_six_kernel", "mx_ring_kernel", "wq_rows_kernel")
 
 FIELDS = {
     "TotalSGPRs": "sgprs", "VGPRs": "vgprs", "AGPRs": "agprs", "ScratchSize [bytes/lane]": "scratch_bytes_per_lane",

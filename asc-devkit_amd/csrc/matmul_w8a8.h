@@ -231,6 +231,8 @@ int dynamic_quant_rows(int32_t src_dtype, uint32_t m, uint32_t n, void* q, uint3
 RingPlan gemm_ring_plan(uint32_t m, uint32_t n, uint32_t k, int b_layout);
 int launch_gemm_ring(const GemmParams& p, int shape, int b_layout, hipStream_t st);
 int launch_gemm_dma_group(GemmParams& p, hipStream_t st);  // matmul_w8a8_group.hip
+int gemm_group_ring_shape(const GemmParams& p);            // matmul_w8a8_ring.hip: tiles of 64 x 64, 64 x 128 and 128 x 128 (shape 0, 1, 2; -1: none)
+int launch_gemm_group_ring(const GemmParams& p, int shape, hipStream_t st);
 uint32_t gemm_dma_skinny_splits(uint32_t m, uint32_t n, uint32_t k);
 bool gemm_dma_small_tiles(uint32_t m, uint32_t n, uint32_t k);
 bool gemm_stream_supported(const GemmParams& p);

@@ -153,6 +153,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_dma_group_kernel(GemmParams 
 
 int launch_gemm_dma_group(GemmParams& p, hipStream_t st)
 {
+    const int ring = gemm_group_ring_shape(p);
+    if (ring >= 0) {
+        return launch_gemm_group_ring(p, ring, st);
+    }
     const uint32_t tiles_n = (p.n + 255u) / 256u;
     // The group sizes are on the device; the kernel plans its tiles there.  One persistent workgroup per compute
     // unit (a multiple of 8, so that a workgroup's id mod 8 is its XCD), fewer when no group list over m rows

@@ -608,6 +608,48 @@ def test_group_matmul_both_matrix_instructions_agree(kind):
         first += c
 
 
+@pytest.mark.parametrize("k", [128, 384, 1408, 2560])
+@pytest.mark.parametrize("nz", [False, True])
+@pytest.mark.parametrize("n", [544, 1632, 2080, 2720])
+@pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 0, 16, 480, 5], [1] * 7 + [0] * 57, [3] * 70])
+@pytest.mark.parametrize("act", ["none", "swiglu"])
+def test_group_matmul_tile_shapes_by_width(counts, n, nz, k, act):
+    """The widths on both sides of the rule that names the tiles (64 x 64, 64 x 128, 128 x 128 with a ring of stages, and those of 256 rows): fewer K
+    steps than stages and more, groups without rows, one to 300 rows, 64 groups and more than the ring's kernel scans; counts
+    and prefix sums of more rows than there are give the same."""
+    announce("grouped, shapes by width", counts[:8], n, nz, k, act)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(k + n)
+    gr, m = len(counts), sum(counts)
+    x = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    w = torch.randint(-127, 128, (gr, k, n), dtype=torch.int8, device=DEV, generator=g)
+    tok = torch.rand(m, device=DEV, generator=g) * 0.02 + 5e-3
+    cs = torch.rand((gr, n), device=DEV, generator=g) * 1e-3 + 1e-4
+    wd = ops.pack_weight_nz(w) if nz else w
+    code = abi.MM_ACT_SWIGLU if act == "swiglu" else abi.MM_ACT_NONE
+    out = n // 2 if act == "swiglu" else n
+    room = torch.zeros((m + 1) * out, dtype=torch.float16, device=DEV)
+    y = room[:m * out].view(m, out)
+    ops.quant_group_matmul(y, x, wd, torch.tensor(counts, dtype=torch.int64, device=DEV), cs, tok, activation=code, weight_nz=nz)
+    assert not room[m * out:].any()
+    r = 0
+    for i, c in enumerate(counts):       # (float64 holds the sums exactly; one fp32 rounding per step of the epilogue)
+        if c and (gr < 20 or i % 9 == 0):
+            v = (x[r:r + c].double() @ w[i].double()).float() * cs[i] * tok[r:r + c, None]
+            if act == "swiglu":
+                a, b = v[:, 0::2].double(), v[:, 1::2].double()
+                want = a * (b / (1.0 + torch.exp(-b)))
+                assert ((y[r:r + c].double() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-4).all(), i
+            else:
+                assert torch.equal(y[r:r + c], v.half()), i
+        r += c
+    y2 = torch.zeros_like(y)
+    big = torch.tensor(counts, dtype=torch.int64, device=DEV).cumsum(0)
+    big[-1] += 1000
+    ops.quant_group_matmul(y2, x, wd, big, cs, tok, activation=code, weight_nz=nz, group_list_kind=abi.GROUP_LIST_PREFIX_SUM)
+    assert torch.equal(y2.view(torch.int16), y.view(torch.int16))
+
+
 @pytest.mark.parametrize("k", [256, 384, 1280, 1408, 2432, 2560, 3072, 3200])
 @pytest.mark.parametrize("nz", [False, True])
 @pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 256, 16, 480, 385], [257, 512, 64, 384]])
