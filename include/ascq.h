@@ -531,8 +531,9 @@ int ascq_group_matmul_w8a8(const ascq_group_matmul_desc* desc, void* y, const vo
  *   wdq[k,j] = f16( scale[k/g][j] * f16( f16(w[k,j]) + offset[k/g][j] ) )     (offset optional)
  *   y[i,j]   = f16( sum_k f32(x[i,k]) * f32(wdq[k,j]) )                       fp32 accumulation
  * workspace: ascq_matmul_w4a16_workspace_size bytes of scratch for the partial sums of the weight streams, with more
- * than 96 rows also for the weights packed as by ascq_pack_weight_w4 (a smaller one is accepted there; contents need
- * not be initialised); calls that share a workspace must not overlap.
+ * than 96 rows, or fewer where that is expected to be faster (5 rows and more), also for the weights packed as by
+ * ascq_pack_weight_w4 (a smaller one is accepted there; contents need not be initialised); calls that share a
+ * workspace must not overlap.
  */
 typedef enum ascq_w4a16_mode {
     ASCQ_W4A16_PER_WEIGHT = 0, /* wdq rounded to half per weight, the formula above: AscendAntiQuant's own arithmetic */
@@ -569,8 +570,9 @@ int ascq_matmul_w4a16_workspace_size(const ascq_w4a16_desc* desc, size_t* bytes)
  * rounding to half) in one launch with no workspace: a workgroup owns whole columns and adds its wavefronts' partial
  * sums in a fixed order, so repeated calls give identical bits.  Up to 4 activation rows (decode) its wavefronts
  * split k and add their sums in LDS; 5 to 16 rows run one wavefront per slab with the activations shared chunk by
- * chunk; more rows take further passes of 16 over the weights, and beyond 48 rows the per-weight form runs a half GEMM
- * whose B-tile loader de-quantises.  Requires k % 128 == 0, n % 8 == 0, group_size =
+ * chunk; more rows take further passes of 16 over the weights, tiles of 16 x 16 to 64 x 64 over all of k that de-quantise in
+ * registers or, beyond 48 rows in the per-weight form, a half GEMM whose B-tile loader de-quantises, whichever is expected to be
+ * fastest.  Requires k % 128 == 0, n % 8 == 0, group_size =
  * 32 * 2^i (ASCQ_EUNSUPPORTED otherwise: use ascq_matmul_w4a16), and x, w_packed, scale, offset 16-byte aligned.
  */
 int ascq_pack_weight_w4_size(uint32_t k, uint32_t n, size_t* bytes);
@@ -594,8 +596,8 @@ int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* desc, void* y, const void* x
  * workgroup: one launch, no workspace (the size query answers 0), identical bits from call to call; that form needs
  * k % 128 == 0 and 16-byte aligned x and w (other shapes and alignments run a slow kernel with one lane per output
  * element, as they do for [k, n] weights).
- * Many rows (more than 32 on [n, k] weights, more than 96 on [k, n]) run a half GEMM whose B-tile loader
- * de-quantises (tiles of up to 256 x 256); [k, n] weights are first copied transposed into the workspace (k * n bytes, which the size query
+ * Many rows (more than 32 on [n, k] weights; on [k, n] more than 96, or fewer where that is expected to be faster, 17 rows and more)
+ * run a half GEMM that de-quantises in its tile loader or in registers (tiles of 16 x 16 to 256 x 256); [k, n] weights are first copied transposed into the workspace (k * n bytes, which the size query
  * then asks for; given less, the call falls back to one pass over the weights per 32 rows).
  * workspace: ascq_matmul_w8a16_workspace_size bytes (contents need not be initialised); calls that share a
  * workspace must not overlap.
@@ -636,8 +638,8 @@ int ascq_matmul_w8a16_workspace_size(const ascq_w8a16_desc* desc, size_t* bytes)
  * product rounded to the output type, compared at rtol = atol = 1e-3.
  * a_format / b_format: ASCQ_QDST_FP8_E4M3FN | ASCQ_QDST_FP8_E5M2 | ASCQ_QDST_FP4_E2M1 | ASCQ_QDST_FP4_E1M2.
  * Two 8-bit operands, or two e2m1 operands, with k % 128 == 0 (8-bit) / k % 256 == 0 (4-bit), 16-byte aligned a, b and
- * scale_k % 8 == 0, scale_k >= 16 run v_mfma_scale_f32_32x32x64_f8f6f4 on 256 x 256 tiles straight from the given buffers.  Other
- * format pairs first widen their 4-bit operands in the workspace (two e1m2 operands to 6-bit e2m3 codes, anything else
+ * scale_k % 8 == 0, scale_k >= 16 run the scaled matrix instruction on tiles of 64 x 64 to 256 x 256 straight from the given buffers
+ * (as do an 8-bit a and an e2m1 b with k % 256 == 0 where the smaller tiles take the call).  Other format pairs first widen their 4-bit operands in the workspace (two e1m2 operands to 6-bit e2m3 codes, anything else
  * to e4m3; both exact).  Few rows (always below 64, up to a few hundred where an estimate says so) and shapes outside
  * the tiles' run a weight-streaming kernel that takes every format pair as it lies, needs no workspace (one that the size
  * query asked for is left alone) and gives the same bits from call to call; it wants rows of a and b that are whole numbers
