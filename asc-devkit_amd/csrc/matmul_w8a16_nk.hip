@@ -484,30 +484,59 @@ __global__ __launch_bounds__(kWaves * 64) void w8a16_nk_stream_kernel(SkParams p
 
 constexpr uint32_t kGK = 64;  // K step of the tile GEMM (matmul_wq_gemm.hip)
 
-// int8 [k, n] -> [n, k] through 64 x 64 tiles in LDS (the tile GEMM wants k-contiguous weights).  k % 64 == 0.
-// kVec: n % 16 == 0 and src 16-byte aligned, so a thread's 16 columns of a row are one load.
-template <bool kVec>
-__global__ __launch_bounds__(256) void transpose_i8_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                           uint32_t k, uint32_t n)
+// int8 [k, n] -> [n, k] (the kernels want k-contiguous weights) for n % 16 == 0 and 16-byte aligned src; k % 64 == 0.  A workgroup turns 128 x 128
+// round: whole lines in and out, a thread's 4 rows of 16 columns become 16 dwords of 4 k by byte permutes, which meet in the LDS: dword d of
+// column c lies in piece (d / 4) ^ (c / 16 % 8) of its 128 bytes, so that writes meet a bank twice and the 16-byte reads none.  Memory bounds it:
+// 110 MB of weights 65.9 us through 64 x 64 tiles and bytes, 48.7 us now (4.5 TB/s read and written), 31 MB 23.3 and 17.5, 5 MB 5.5 and 5.2.
+__global__ __launch_bounds__(256) void transpose_i8_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t k, uint32_t n)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t T[128 * 32];
+    const uint32_t tiles_n = (n + 127u) / 128u;
+    const uint32_t k0 = (blockIdx.x / tiles_n) * 128u, n0 = (blockIdx.x % tiles_n) * 128u;
+    const uint32_t t = threadIdx.x, r = t >> 3, c = t & 7u;
+    const bool here = n0 + 16u * c < n && k0 + 4u * r < k;
+    u32x4 v[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        v[i] = u32x4{0u, 0u, 0u, 0u};
+        if (here) {
+            v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + static_cast<size_t>(k0 + 4u * r + i) * n + n0 + 16u * c));
+        }
+    }
+    const uint32_t place = (((r >> 2) ^ c) << 2) + (r & 3u);
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {  // a 4 x 4 block of bytes: columns 16 c + 4 w .. + 3
+        const uint32_t a = __builtin_amdgcn_perm(v[1][w], v[0][w], 0x05010400u), b = __builtin_amdgcn_perm(v[3][w], v[2][w], 0x05010400u);
+        const uint32_t e = __builtin_amdgcn_perm(v[1][w], v[0][w], 0x07030602u), f = __builtin_amdgcn_perm(v[3][w], v[2][w], 0x07030602u);
+        uint32_t* const to = T + (16u * c + 4u * w) * 32u + place;
+        to[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        to[32] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        to[64] = __builtin_amdgcn_perm(f, e, 0x05040100u);
+        to[96] = __builtin_amdgcn_perm(f, e, 0x07060302u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t col = i * 32u + r;
+        if (n0 + col < n && k0 + 16u * c < k) {
+            *reinterpret_cast<u32x4*>(dst + static_cast<size_t>(n0 + col) * k + k0 + 16u * c) =
+                *reinterpret_cast<const u32x4*>(T + col * 32u + ((c ^ ((col >> 4) & 7u)) << 2));
+        }
+    }
+}
+
+// The same for any n and alignment, through 64 x 64 tiles.
+__global__ __launch_bounds__(256) void transpose_i8_any_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t k, uint32_t n)
 {
     __shared__ __attribute__((aligned(16))) uint8_t T[64][68];
     const uint32_t tiles_n = (n + 63u) / 64u;
     const uint32_t k0 = (blockIdx.x / tiles_n) * 64u, n0 = (blockIdx.x % tiles_n) * 64u;
     const uint32_t t = threadIdx.x, r = t >> 2, c = (t & 3u) * 16u;
     const uint8_t* row = src + static_cast<size_t>(k0 + r) * n;
-    if constexpr (kVec) {
-        u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        if (n0 + c < n) {
-            v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + n0 + c));
-        }
 #pragma unroll
-        for (uint32_t w = 0; w < 4; ++w) *reinterpret_cast<uint32_t*>(&T[r][c + 4u * w]) = v[w];
-    } else {
-#pragma unroll
-        for (uint32_t i = 0; i < 16; ++i) {
-            const uint32_t col = n0 + c + i;
-            T[r][c + i] = row[col < n ? col : n - 1u];
-        }
+    for (uint32_t i = 0; i < 16; ++i) {
+        const uint32_t col = n0 + c + i;
+        T[r][c + i] = row[col < n ? col : n - 1u];
     }
     __syncthreads();
     if (n0 + r < n) {
@@ -554,17 +583,17 @@ double w8a16_nk_estimate(uint32_t m, uint32_t n, uint32_t k)
     return k % kGK == 0 && k <= kWqMaxK && rows < other ? rows : other;
 }
 
-// Weights as [k, n]: whether they are transposed first.  Above 96 rows always; from 17 on where the transposition (3 us and
-// 0.55 us per MB of weights) and the [n, k] form are expected to be ahead of a pass over the weights per 32 rows (14 us, another
+// Weights as [k, n]: whether they are transposed first.  Above 96 rows always; from 17 on where the transposition (4 us and
+// 0.39 us per MB of weights) and the [n, k] form are expected to be ahead of a pass over the weights per 32 rows (14 us, another
 // 12 once the weights are some 16 MB, and 0.2 per MB; fits to 45 random calls): 65 x 2048 x 3328 58 against 15 us,
-// 64 x 6400 x 1632 57 and 23, 24 x 9472 x 3136 33 and 33, 17 x 5248 x 11712 34 and 57.
+// 64 x 6400 x 1632 57 and 23, 24 x 9472 x 3136 33 and 29, 17 x 5248 x 11712 34 and 50.
 bool w8a16_kn_transposed(uint32_t m, uint32_t n, uint32_t k)
 {
     if (k % kGK != 0 || k > kWqMaxK) {
         return false;
     }
     const double mb = 1e-6 * k * n;
-    return m > 96u || (m > 16u && k % kRun == 0 && 3.0 + 0.55 * mb + w8a16_nk_estimate(m, n, k) <
+    return m > 96u || (m > 16u && k % kRun == 0 && 4.0 + 0.39 * mb + w8a16_nk_estimate(m, n, k) <
                                                    0.9 * ((m + 31u) / 32u) * (14.0 + 12.0 * (1.0 - __builtin_exp(-mb / 8.0)) + 0.2 * mb));
 }
 
@@ -577,11 +606,12 @@ int launch_w8a16_kn_via_transpose(const void* x, const void* w, const void* scal
                                   uint32_t m, uint32_t n, uint32_t k, bool has_offset, bool out_f32, uint32_t scale_bits,
                                   uint32_t offset_bits, void* workspace, hipStream_t st)
 {
-    const uint32_t tiles = (k / 64u) * ((n + 63u) / 64u);
+    const uint8_t* const from = static_cast<const uint8_t*>(w);
+    uint8_t* const to = static_cast<uint8_t*>(workspace);
     if (n % 16u == 0 && aligned16(w)) {
-        transpose_i8_kernel<true><<<tiles, 256, 0, st>>>(static_cast<const uint8_t*>(w), static_cast<uint8_t*>(workspace), k, n);
+        transpose_i8_kernel<<<(k + 127u) / 128u * ((n + 127u) / 128u), 256, 0, st>>>(from, to, k, n);
     } else {
-        transpose_i8_kernel<false><<<tiles, 256, 0, st>>>(static_cast<const uint8_t*>(w), static_cast<uint8_t*>(workspace), k, n);
+        transpose_i8_any_kernel<<<(k / 64u) * ((n + 63u) / 64u), 256, 0, st>>>(from, to, k, n);
     }
     return launch_w8a16_nk(x, workspace, scale, offset, y, m, n, k, has_offset, out_f32, scale_bits, offset_bits, st,
                            false);
