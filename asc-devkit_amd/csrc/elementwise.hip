@@ -8,6 +8,7 @@
 #include "ascq_common.h"
 #include "ascq_device.h"
 #include "matmul_w8a8.h"
+#include "row_walk.h"
 
 namespace ascq {
 namespace {
@@ -15,28 +16,14 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRowsInFlight = 4;
 
-// Launch shape of the row-wise vector kernels: blockIdx.x walks the lanes of a row, blockIdx.y groups of rows.  The
-// block size (256, 128 or 64) is the one that leaves the fewest idle lanes in a row's last block: 11008 columns at 8
-// per lane are 10.75 blocks of 128 but 5.4 of 256, and that mostly empty sixth block cost 8 % of the kernel's time.
 struct RowLaunch {
     dim3 grid;
     uint32_t block;
 };
 inline RowLaunch row_launch(uint32_t lanes, uint32_t rows, uint32_t rows_per_group)
 {
-    uint32_t block = kThreads;
-    for (uint32_t b = kThreads / 2; b >= 64u; b /= 2) {
-        if ((lanes + b - 1) / b * b < (lanes + block - 1) / block * block) {
-            block = b;
-        }
-    }
-    RowLaunch r{dim3((lanes + block - 1) / block, 1), block};
-    const uint32_t row_groups = (rows + rows_per_group - 1) / rows_per_group;
-    // enough blocks to fill 256 CUs several times over, but no more row groups than exist
-    const uint32_t want = (8192u * (kThreads / block) + r.grid.x - 1) / r.grid.x;
-    r.grid.y = row_groups < want ? row_groups : want;
-    if (r.grid.y > 65535u) r.grid.y = 65535u;
-    return r;
+    const RowWalk w = row_walk(lanes, rows, rows_per_group, kThreads);
+    return {dim3(w.grid_x, w.grid_y), w.block};
 }
 
 // Up to 2048 wavefronts of single rows (8 elements a lane) are resident at once and take the time of one row; beyond,
@@ -186,13 +173,12 @@ __device__ __forceinline__ float quant_param1(const QuantArgs& a, const void* ba
     }
 }
 
-// The columns of a lane, at a row's end moved back so that they end with the row: in rows of an odd width the last two lanes
-// share columns and store the same values there.
+// The columns of a lane: in rows of an odd width the last two lanes share columns and store the same values there.
 template <bool kAny>
 __device__ __forceinline__ uint32_t lane_columns(uint32_t n)
 {
     const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) * 8u;
-    return kAny && j < n && j + 8u > n ? n - 8u : j;
+    return kAny ? whole_columns(j, n) : j;
 }
 
 // One lane = 8 consecutive columns; blockIdx.y walks groups of kRows rows.  Requires n % 8 == 0 and 16-byte aligned
@@ -417,7 +403,7 @@ int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
         quant_scalar_kernel<kSrc, kPar, kCt><<<static_cast<uint32_t>(blocks), kThreads, 0, st>>>(a);
         return launch_status("ascq_quant");
     }
-    const RowLaunch rl = row_launch((a.n + 7) / 8, a.rows, kRowsInFlight);
+    const RowLaunch rl = row_launch(row_lanes(a.n), a.rows, kRowsInFlight);
     if constexpr (kSrc == ASCQ_F16 && kCt == ASCQ_F16) {
         // fp16 contract on a half source: scale / offset are half tensors or scalars
         if (kind == kQuantI8Rint && (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
@@ -896,7 +882,7 @@ int launch_antiquant(const AntiQuantArgs& a, bool vec, hipStream_t st)
 {
     if (vec || (!a.transpose && a.cols >= 8)) {
         // keep the rows of one lane inside as few parameter groups as possible: consecutive row groups per block
-        const RowLaunch rl = row_launch((a.cols + 7) / 8, a.rows, 2 * kRowsInFlight);
+        const RowLaunch rl = row_launch(row_lanes(a.cols), a.rows, 2 * kRowsInFlight);
         if (!vec) {
             a.has_offset ? antiquant_vec_kernel<kSrc, kDst, true, false, true><<<rl.grid, rl.block, 0, st>>>(a)
                          : antiquant_vec_kernel<kSrc, kDst, false, false, true><<<rl.grid, rl.block, 0, st>>>(a);
