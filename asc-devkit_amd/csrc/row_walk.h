@@ -1,5 +1,5 @@
 // How the row-wise kernels of elementwise.hip share out a matrix: integers only, for the device and for a host compiler alone.
-// Every count of 32 bits is in range, also the last ones, where a sum such as n + 7 does not fit.
+// Every count of 32 bits is in range, also the last ones, where a sum such as n + 7 or r0 + 8 does not fit.
 #pragma once
 #include <cstdint>
 
@@ -18,6 +18,16 @@ ASCQ_HD inline uint32_t row_lanes(uint32_t n) { return ceil_div(n, 8u); }
 
 // The first of a lane's 8 columns, at a row's end moved back so that they end with the row (n >= 8).
 ASCQ_HD inline uint32_t whole_columns(uint32_t j, uint32_t n) { return j < n && n - j < 8u ? n - 8u : j; }
+
+// On to the next rows of a workgroup, `step` further; false where there are none.
+ASCQ_HD inline bool next_rows(uint32_t& r0, uint32_t step, uint32_t rows)
+{
+    if (rows - r0 <= step) {
+        return false;
+    }
+    r0 += step;
+    return true;
+}
 
 // Launch shape of the row-wise vector kernels: grid_x walks the lanes of a row, grid_y groups of rows.  The
 // block size (threads, half or a quarter of them) is the one that leaves the fewest idle lanes in a row's last block: 11008 columns at 8
