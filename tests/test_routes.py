@@ -1,0 +1,23 @@
+"""The kernels that calls choose, without a GPU (tests/routes.py): the sizes at which a rule was measured keep the faster side."""
+import pytest
+
+from ascq import _abi as abi
+from routes import route
+
+DST, SRC, SCALE, OFFSET = 1 << 44, 1 << 20, 1 << 42, 1 << 43      # apart, aligned, never read
+
+
+def quant(rows, n, src=abi.BF16, par=abi.BF16, fmt=abi.QDST_I8, mode=abi.CAST_RINT, policy=abi.PER_CHANNEL, compute=abi.COMPUTE_F32, src_at=SRC):
+    d = dict(policy=policy, src_dtype=src, scale_dtype=par, compute=compute, round_mode=mode, offset_kind=abi.OFFSET_NONE, k_dim=1, m=rows, n=n,
+             cal_count=rows * n, group_size=32, dst_format=fmt)
+    launch, = route("ascq_quant", ("QuantDesc", d), DST, src_at, None if policy == abi.PER_TENSOR else SCALE, None, None)
+    return launch
+
+
+@pytest.mark.parametrize("rows,n", [(4000, 4096), (100000, 32), (40000, 128), (4000, 1024)])
+@pytest.mark.parametrize("fmt,mode", [(abi.QDST_I8, abi.CAST_FLOOR), (abi.QDST_HIF8, abi.CAST_ROUND)])
+def test_formats_without_a_kernel_of_their_own_hold_two_rows_per_lane(rows, n, fmt, mode):
+    """quant_vec_kernel<source, parameters, arithmetic, kind, rows per lane, any address>: four rows cost two of seven wavefronts."""
+    assert quant(rows, n, fmt=fmt, mode=mode).args[3:] == ("4", "2", "false")
+    assert quant(100, n, fmt=fmt, mode=mode).args[3:] == ("4", "1", "false")
+    assert quant(rows, n).args[3:] == ("0", "4", "false")
