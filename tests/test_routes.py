@@ -21,3 +21,14 @@ def test_formats_without_a_kernel_of_their_own_hold_two_rows_per_lane(rows, n, f
     assert quant(rows, n, fmt=fmt, mode=mode).args[3:] == ("4", "2", "false")
     assert quant(100, n, fmt=fmt, mode=mode).args[3:] == ("4", "1", "false")
     assert quant(rows, n).args[3:] == ("0", "4", "false")
+
+
+@pytest.mark.parametrize("rows,n,per_lane", [(8192, 32, "1"), (8193, 32, "4"), (30000, 32, "4"), (4000, 32, "1"), (16000, 64, "4"), (2047, 512, "1"), (2049, 512, "4"),
+                                             (1024, 1024, "1"), (1025, 1024, "4"), (1, 2 ** 20, "1")])
+def test_narrow_rows_come_one_to_a_lane_up_to_8192_wavefronts(rows, n, per_lane):
+    """Up to 2^20 elements a lane holds one row, unless the rows are that many wavefronts: quantisers and dequantisation policies."""
+    assert quant(rows, n).args[4] == per_lane
+    d = dict(policy=abi.PER_TOKEN, src_format=abi.QDST_FP8_E4M3FN, scale_dtype=abi.BF16, dst_dtype=abi.BF16, compute=abi.COMPUTE_SCALE_T,
+             k_dim=1, m=rows, n=n, cal_count=rows * n, group_size=32)
+    launch, = route("ascq_antiquant_policy", ("AntiQuantPolicyDesc", d), DST, SRC, SCALE, None, None)
+    assert launch.name == "antiquant_policy_vec_kernel" and launch.args[4] == per_lane
