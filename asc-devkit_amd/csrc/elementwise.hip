@@ -774,21 +774,19 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
     if (j >= a.cols) {
         return;
     }
-    constexpr uint32_t kRows = 2 * kRowsInFlight;
+    constexpr int kRows = 2 * kRowsInFlight;
     constexpr bool kHalf = kDst == ASCQ_F16;
     const half_t bias = static_cast<half_t>(kSrc == ASCQ_I8 ? 1152.0f : 1032.0f);
     f16x2 s[4], o[4];      // half outputs: parameters of column pairs
     float sf[8], of[8];    // bfloat16 outputs
     uint32_t cached_group = 0xFFFFFFFFu;
     const uint32_t jg = kTranspose ? j / a.group_size : 0u;
-    uint32_t r0 = blockIdx.y * kRows;
-    do {
-        const uint32_t left = a.rows - r0;  // (up to 2^32 - 1 rows: neither r0 + u nor the next r0 need fit 32 bits)
+    for (uint32_t r0 = blockIdx.y * kRows; r0 < a.rows; r0 += gridDim.y * kRows) {
         u32x2 raw[kRows];
         uint32_t sr[kRows], orr[kRows];  // transposed: the parameters of the rows (a register each: no load waits for another)
 #pragma unroll
-        for (uint32_t u = 0; u < kRows; ++u) {
-            if (u < left) {
+        for (int u = 0; u < kRows; ++u) {
+            if (r0 + u < a.rows) {
                 const size_t e = static_cast<size_t>(r0 + u) * a.cols + j;
                 if constexpr (kSrc == ASCQ_I8 && kAny) {
                     raw[u] = *reinterpret_cast<const u32x2_any*>(static_cast<const int8_t*>(a.src) + e);
@@ -807,9 +805,9 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
             }
         }
 #pragma unroll
-        for (uint32_t u = 0; u < kRows; ++u) {
+        for (int u = 0; u < kRows; ++u) {
             const uint32_t r = r0 + u;
-            if (u >= left) {
+            if (r >= a.rows) {
                 break;
             }
             // parameters: a [groups, cols] row (not transposed) or one scalar per (row, group) (transposed)
@@ -888,13 +886,14 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
                 store8<kDst, kAny ? kAnyAddress : kNonTemporal>(a.dst, oe, y);
             }
         }
-    } while (next_rows(r0, gridDim.y * kRows, a.rows));
+    }
 }
 
 template <int kSrc, int kDst>
 int launch_antiquant(const AntiQuantArgs& a, bool vec, hipStream_t st)
 {
-    if (vec || (!a.transpose && a.cols >= 8)) {
+    // (rows whose walk passes 2^32 run one element per lane, which counts in 64 bits)
+    if (walk_fits(a.rows, 2 * kRowsInFlight) && (vec || (!a.transpose && a.cols >= 8))) {
         // keep the rows of one lane inside as few parameter groups as possible: consecutive row groups per block
         const RowLaunch rl = row_launch(row_lanes(a.cols), a.rows, 2 * kRowsInFlight);
         if (!vec) {

@@ -1,5 +1,5 @@
 // How the row-wise kernels of elementwise.hip share out a matrix: integers only, for the device and for a host compiler alone.
-// Every count of 32 bits is in range, also the last ones, where a sum such as n + 7 or r0 + 8 does not fit.
+// Every count of 32 bits is in range, also the last ones, where a sum such as n + 7 does not fit.
 #pragma once
 #include <cstdint>
 
@@ -18,16 +18,6 @@ ASCQ_HD inline uint32_t row_lanes(uint32_t n) { return ceil_div(n, 8u); }
 
 // The first of a lane's 8 columns, at a row's end moved back so that they end with the row (n >= 8).
 ASCQ_HD inline uint32_t whole_columns(uint32_t j, uint32_t n) { return j < n && n - j < 8u ? n - 8u : j; }
-
-// On to the next rows of a workgroup, `step` further; false where there are none.
-ASCQ_HD inline bool next_rows(uint32_t& r0, uint32_t step, uint32_t rows)
-{
-    if (rows - r0 <= step) {
-        return false;
-    }
-    r0 += step;
-    return true;
-}
 
 // Launch shape of the row-wise vector kernels: grid_x walks the lanes of a row, grid_y groups of rows.  The
 // block size (threads, half or a quarter of them) is the one that leaves the fewest idle lanes in a row's last block: 11008 columns at 8
@@ -50,5 +40,8 @@ inline RowWalk row_walk(uint32_t lanes, uint32_t rows, uint32_t rows_per_group, 
     r.grid_y = r.grid_y < 65535u ? r.grid_y : 65535u;
     return r;
 }
+
+// Whether the rows r0 of every workgroup's walk, r0 += grid_y * rows_per_group up to the first past the end, fit 32 bits.
+inline bool walk_fits(uint32_t rows, uint32_t rows_per_group) { return rows <= 0xFFFFFFFFu - 65535u * rows_per_group; }
 
 }  // namespace ascq

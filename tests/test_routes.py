@@ -32,3 +32,12 @@ def test_narrow_rows_come_one_to_a_lane_up_to_8192_wavefronts(rows, n, per_lane)
              k_dim=1, m=rows, n=n, cal_count=rows * n, group_size=32)
     launch, = route("ascq_antiquant_policy", ("AntiQuantPolicyDesc", d), DST, SRC, SCALE, None, None)
     assert launch.name == "antiquant_policy_vec_kernel" and launch.args[4] == per_lane
+
+
+@pytest.mark.parametrize("cols", [9, 16])
+def test_rows_whose_walk_passes_32_bits_run_one_element_per_lane(cols):
+    last = 2 ** 32 - 1 - 65535 * 8
+    for rows, kernel in ((last, "antiquant_vec_kernel"), (last + 1, "antiquant_scalar_kernel"), (2 ** 32 - 1, "antiquant_scalar_kernel")):
+        d = dict(src_dtype=abi.I8, dst_dtype=abi.F16, has_offset=0, per_tensor=1, k=rows, n=cols)
+        launch, = route("ascq_antiquant", ("AntiQuantDesc", d), 1 << 52, SRC, None, None, None)
+        assert launch.name == kernel and launch.grid_y >= 1

@@ -20,8 +20,7 @@ def walk(tmp_path_factory):
     src.write_text('#include "row_walk.h"\n'
                    'extern "C" {\n'
                    'uint32_t lanes(uint32_t n) { return ascq::row_lanes(n); }\n'
-                   'uint32_t rounds(uint32_t r0, uint32_t step, uint32_t rows, uint32_t* last)\n'
-                   '{ uint32_t n = 0; do { *last = r0; ++n; } while (n < (1u << 20) && ascq::next_rows(r0, step, rows)); return n; }\n'
+                   'uint32_t fits(uint32_t rows, uint32_t per) { return ascq::walk_fits(rows, per); }\n'
                    'uint32_t columns(uint32_t j, uint32_t n) { return ascq::whole_columns(j, n); }\n'
                    'void shape(uint32_t lanes, uint32_t rows, uint32_t per, uint32_t* out)\n'
                    '{ auto w = ascq::row_walk(lanes, rows, per, 256); out[0] = w.grid_x; out[1] = w.grid_y; out[2] = w.block; }\n'
@@ -30,9 +29,9 @@ def walk(tmp_path_factory):
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-o", lib, "-I",
                            os.path.join(ROOT, "asc-devkit_amd", "csrc"), str(src)])
     lib = C.CDLL(lib)
-    lib.lanes.restype = lib.columns.restype = lib.rounds.restype = C.c_uint32
+    lib.lanes.restype = lib.columns.restype = lib.fits.restype = C.c_uint32
     lib.lanes.argtypes, lib.columns.argtypes = [C.c_uint32], [C.c_uint32] * 2
-    lib.rounds.argtypes = [C.c_uint32] * 3 + [C.POINTER(C.c_uint32)]
+    lib.fits.argtypes = [C.c_uint32] * 2
     lib.shape.argtypes = [C.c_uint32] * 3 + [C.POINTER(C.c_uint32)]
     return lib
 
@@ -57,11 +56,11 @@ def test_every_row_count_has_groups(walk, rows):
     out = (C.c_uint32 * 3)()
     walk.shape(2, rows, 8, out)
     assert 1 <= out[1] <= min(65535, -(-rows // 8))
-    # a workgroup's walk over the groups ends, behind the last one that is its own
-    groups, last = out[1], C.c_uint32()
-    for y in {0, groups // 2, groups - 1}:
-        own = range(8 * y, rows, 8 * groups)
-        assert walk.rounds(8 * y, 8 * groups, rows, C.byref(last)) == len(own) and last.value == own[-1]
+    # a workgroup's walk: the first row past the end fits 32 bits, or the rows are refused
+    groups = out[1]
+    past = [8 * y + -(-(rows - 8 * y) // (8 * groups)) * 8 * groups for y in {0, groups // 2, groups - 1}]
+    assert not walk.fits(rows, 8) or max(past) < TOP
+    assert walk.fits(rows, 8) == (rows <= TOP - 1 - 65535 * 8)
 
 
 CHILD = """
