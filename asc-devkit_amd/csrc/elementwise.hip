@@ -35,6 +35,14 @@ inline bool few_rows(uint32_t rows, uint32_t n)
     return static_cast<uint64_t>(rows) * n <= 2048u * 64u * 8u && rows * ceil_div(n, 512u) <= 8192u;
 }
 
+// Whether rows of any width and alignment run the vector kernels or one element per lane.  The vectors waste the lanes of a wavefront
+// that a narrow row has no columns for, and a call of few elements is over in the one load, product and store of the other kernel:
+// measured at 0.7 to 12 million elements in rows of 9 to 8195, the vectors are ahead from `width` columns and `elements` on.
+inline bool any_address_ahead(uint32_t rows, uint32_t n, uint32_t width, uint64_t elements)
+{
+    return n >= width && static_cast<uint64_t>(rows) * n >= elements;
+}
+
 // ===================================================================== AscendQuant
 struct QuantArgs {
     int8_t* dst;
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(kThreads) void quant_vec_kernel(QuantArgs a)
     }
 }
 
-// Rows of fewer than 8 columns: one element per lane.
+// Rows off the vectors' width or alignment where they are narrow or few (any_address_ahead): one element per lane.
 template <int kSrc, int kPar, int kCt>
 __global__ __launch_bounds__(kThreads) void quant_scalar_kernel(QuantArgs a)
 {
@@ -410,7 +418,16 @@ int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
 {
     const int kind = quant_kind(a);
     const bool per_row = a.policy == ASCQ_PER_TOKEN || a.policy == ASCQ_PER_GROUP;
-    const bool any = !vec && a.n >= 8 && (a.n % 8 == 0 || !per_row);
+    // fp16 contract on a half source: scale / offset are half tensors or scalars
+    const bool half = kSrc == ASCQ_F16 && kCt == ASCQ_F16 && kind == kQuantI8Rint &&
+                      (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16));
+    // In us with one element per lane and as vectors: half to int8 4000 x 33 2.3 and 3.4, 10769 x 65 3.8 and 3.6; bfloat16 to int8 5426 x 129
+    // 3.8 and 4.5, 1000 x 515 3.2 and 3.6, 5440 x 193 4.6 and 4.5, 2007 x 523 4.6 and 4.3, 1333333 x 9 33 and 270; to e4m3 (the kernel
+    // of all formats) 1369 x 511 3.6 and 5.0, 11673 x 257 8.9 and 9.4, 5736 x 523 8.9 and 8.8, 7792 x 385 9.0 and 7.7.
+    const bool any = !vec && (a.n % 8 == 0 || !per_row) &&
+                     (half                   ? any_address_ahead(a.rows, a.n, 64u, 0u)
+                      : kind == kQuantI8Rint ? any_address_ahead(a.rows, a.n, 192u, 1u << 20)
+                                             : any_address_ahead(a.rows, a.n, 384u, 3u << 20));
     if (!vec && !any) {
         size_t total = static_cast<size_t>(a.rows) * a.n;
         size_t blocks = (total + kThreads - 1) / kThreads;
@@ -419,8 +436,7 @@ int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
         return launch_status("ascq_quant");
     }
     if constexpr (kSrc == ASCQ_F16 && kCt == ASCQ_F16) {
-        // fp16 contract on a half source: scale / offset are half tensors or scalars
-        if (kind == kQuantI8Rint && (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16))) {
+        if (half) {
             const RowLaunch rl = row_launch(row_lanes(a.n), a.rows, kRowsInFlight);
             any ? quant_f16_fast_kernel<true><<<rl.grid, rl.block, 0, st>>>(a)
                 : quant_f16_fast_kernel<false><<<rl.grid, rl.block, 0, st>>>(a);
@@ -892,8 +908,13 @@ __global__ __launch_bounds__(kThreads) void antiquant_vec_kernel(AntiQuantArgs a
 template <int kSrc, int kDst>
 int launch_antiquant(const AntiQuantArgs& a, bool vec, hipStream_t st)
 {
+    // In us with one element per lane and as vectors: int8 to half 3626 x 193 3.3 and 3.4, 5440 x 193 4.0 and 3.5; to bfloat16 2676 x 523 4.7 and
+    // 5.2, 10362 x 193 6.0 and 5.6; one parameter for all, half 1014 x 1035 3.4 and 3.5, 1365 x 1035 3.9 and 3.7, bfloat16 2600 x 769 4.8
+    // and 5.1, 3901 x 769 6.4 and 5.3; 1333333 x 9 to bfloat16 26 and 180.
+    const uint64_t from = kDst == ASCQ_F16 ? 1u << 20 : 2u << 20;
+    const bool any = !a.transpose && any_address_ahead(a.rows, a.cols, 192u, a.per_tensor ? from + from / 2u : from);
     // (rows whose walk passes 2^32 run one element per lane, which counts in 64 bits)
-    if (walk_fits(a.rows, 2 * kRowsInFlight) && (vec || (!a.transpose && a.cols >= 8))) {
+    if (walk_fits(a.rows, 2 * kRowsInFlight) && (vec || any)) {
         // keep the rows of one lane inside as few parameter groups as possible: consecutive row groups per block
         const RowLaunch rl = row_launch(row_lanes(a.cols), a.rows, 2 * kRowsInFlight);
         if (!vec) {

@@ -29,25 +29,34 @@ class Launch(NamedTuple):
         return tuple(a.strip() for a in self.kernel.partition("<")[2].rstrip(">").split(","))
 
 
-def routes(calls):
-    """calls: [(entry point, [argument, ...])], an argument being a number, None, or (descriptor class name, {field: value}).
-    Returns [(status, [Launch, ...])]."""
-    assert os.path.exists(LOG), "tests/cpp/launch_log.so is not built: run __graft_entry__.build()"
-    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", PYTHONPATH=os.path.join(ROOT, "asc-devkit_amd"))
-    r = subprocess.run([sys.executable, os.path.abspath(__file__)], input=json.dumps(calls), env=env, capture_output=True, text=True,
-                       timeout=300)
-    assert r.returncode == 0, r.stderr[-2000:]
-    return [(status, [Launch(n, int(x), int(y), int(b)) for n, x, y, b in launches]) for status, launches in json.loads(r.stdout)]
+class Calls:
+    """The child process; it ends with this one."""
 
+    def __init__(self):
+        assert os.path.exists(LOG), "tests/cpp/launch_log.so is not built: run __graft_entry__.build()"
+        env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", PYTHONPATH=os.path.join(ROOT, "asc-devkit_amd"))
+        self.child = subprocess.Popen([sys.executable, os.path.abspath(__file__)], env=env, stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
 
-def route(entry, *args):
-    """the kernels of one call that is accepted"""
-    return _route(entry, json.dumps(args))
+    def __call__(self, entry, args):
+        self.child.stdin.write(json.dumps([entry, args]) + "\n")
+        self.child.stdin.flush()
+        status, lines = json.loads(self.child.stdout.readline())
+        return status, [Launch(n, int(x), int(y), int(b)) for n, x, y, b in lines]
 
 
 @functools.lru_cache(maxsize=None)
-def _route(entry, args):
-    (status, launches), = routes([(entry, json.loads(args))])
+def _calls():
+    return Calls()
+
+
+def call(entry, *args):
+    """(status, [Launch, ...]) of one call; an argument is a number, None, or (descriptor class name, {field: value})."""
+    return _calls()(entry, args)
+
+
+def route(entry, *args):
+    """The kernels of one call that is accepted."""
+    status, launches = call(entry, *args)
     assert status == 0, (entry, args, status)
     return launches
 
@@ -57,15 +66,13 @@ def _child():
     log = C.CDLL(LOG, mode=C.RTLD_GLOBAL)
     log.launch_log_take.restype = C.c_char_p
     lib = C.CDLL(abi.LIB_PATH)
-    out = []
-    for entry, args in json.load(sys.stdin):
+    for line in sys.stdin:
+        entry, args = json.loads(line)
         fn = getattr(lib, entry)
         fn.restype, fn.argtypes = abi.SIGNATURES[entry]
         held = [getattr(abi, a[0])(**a[1]) if isinstance(a, list) else a for a in args]
         status = fn(*[C.byref(h) if isinstance(h, C.Structure) else h for h in held])
-        lines = log.launch_log_take().decode().splitlines()
-        out.append((status, [line.rsplit(";", 3) for line in lines]))
-    json.dump(out, sys.stdout)
+        print(json.dumps([status, [text.rsplit(";", 3) for text in log.launch_log_take().decode().splitlines()]]), flush=True)
 
 
 if __name__ == "__main__":

@@ -753,11 +753,14 @@ def test_config2c_full_size_antiquant():
 # ------------------------------------------------------------------ rows of any width, tensors at any element
 @pytest.mark.parametrize("n", [7, 8, 9, 15, 17, 1023, 1025, 2049, 4099, 8191, 9661, 16383, 16385])
 @pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16, abi.F32])
-def test_quantisers_of_odd_widths_off_the_vector_alignment(n, src_dt):
+@pytest.mark.parametrize("elements", [0, 3 << 20])
+def test_quantisers_of_odd_widths_off_the_vector_alignment(n, src_dt, elements):
     """Widths on both sides of the vector's 8 columns and of the row kernels' limits, inputs and outputs one element past a
-    16-byte boundary; the bytes around the outputs stay as they are."""
-    m = 13
-    announce("quant odd widths", n, src_dt)
+    16-byte boundary; the bytes around the outputs stay as they are.  Few rows, and (wide ones) as many as the vectors take."""
+    if elements and n < 1023:
+        pytest.skip("narrow rows run one element per lane in any number")
+    m = max(13, -(-elements // n))
+    announce("quant odd widths", n, src_dt, m)
     rng = np.random.default_rng(n)
     x, _ = src_array(rng, (m, n), src_dt, 3.0)
     xd = to_dev(np.concatenate([x.reshape(-1)[:1], x.reshape(-1)]), "bf16" if src_dt == abi.BF16 else None)[1:].view(m, n)
@@ -776,18 +779,37 @@ def test_quantisers_of_odd_widths_off_the_vector_alignment(n, src_dt):
                       cal_count=m * n)
     assert np.array_equal(q.cpu().numpy(), orc.quant(d, x, s))
     assert room[0] == 55 and (room[1 + m * n:] == 55).all()
+    # the kernel that the other formats share, and all of the tensor as one row of an odd length
+    para = ops.AscendQuantParam(m=m, n=n, cal_count=m * n)
+    for fmt, mode in ((abi.QDST_HIF8, abi.CAST_ROUND), (abi.QDST_FP8_E4M3FN, abi.CAST_RINT), (abi.QDST_I8, abi.CAST_FLOOR)):
+        room.fill_(55)
+        cfg = ops.AscendQuantConfig(round_mode=mode)
+        ops.quantize(q.view(torch.uint8) if fmt == abi.QDST_HIF8 else q, xd, sd, None, para, abi.PER_CHANNEL, cfg, dst_format=fmt)
+        d = abi.QuantDesc(policy=abi.PER_CHANNEL, src_dtype=src_dt, scale_dtype=src_dt, compute=abi.COMPUTE_F32, round_mode=mode,
+                          offset_kind=abi.OFFSET_NONE, m=m, n=n, cal_count=m * n, dst_format=fmt)
+        assert np.array_equal(q.cpu().numpy().view(np.uint8).reshape(-1), orc.quant(d, x, s).view(np.uint8).reshape(-1)), fmt
+        assert room[0] == 55 and (room[1 + m * n:] == 55).all()
+    room.fill_(55)
+    ops.ascend_quant(q, xd, 4.5, -1.25)
+    d = abi.QuantDesc(policy=abi.PER_TENSOR, src_dtype=src_dt, scale_dtype=src_dt, compute=abi.COMPUTE_F16, scale=4.5, offset=-1.25,
+                      offset_kind=abi.OFFSET_SCALAR, round_mode=abi.CAST_RINT, cal_count=m * n)
+    assert np.array_equal(q.cpu().numpy().reshape(-1), orc.quant(d, x, None).reshape(-1))
+    assert room[0] == 55 and (room[1 + m * n:] == 55).all()
 
 
 @pytest.mark.parametrize("n", [7, 8, 10, 22, 24, 1030, 4098])
 @pytest.mark.parametrize("int4", [False, True])
 @pytest.mark.parametrize("dst_dt", [abi.F16, abi.BF16])
 @pytest.mark.parametrize("has_offset", [True, False])
-def test_antiquant_of_odd_widths_off_the_vector_alignment(n, int4, dst_dt, has_offset):
+@pytest.mark.parametrize("elements", [0, 2 << 20])
+def test_antiquant_of_odd_widths_off_the_vector_alignment(n, int4, dst_dt, has_offset, elements):
     """The same for AscendAntiQuant: sources, parameters and outputs one element past a 16-byte boundary."""
+    if elements and n < 1023:
+        pytest.skip("narrow rows run one element per lane in any number")
     if int4:
         n += n % 2
-    k, g = 30, 3
-    announce("antiquant odd widths", n, int4, dst_dt, has_offset)
+    k, g = 3 * max(10, -(-elements // (3 * n))), 3
+    announce("antiquant odd widths", n, int4, dst_dt, has_offset, k)
     rng = np.random.default_rng(n)
     w = rng.integers(-8, 8, (k, n)).astype(np.int8) if int4 else rng.integers(-128, 128, (k, n)).astype(np.int8)
     sc, _ = src_array_uniform(rng, (g, n), dst_dt, -2, 2)

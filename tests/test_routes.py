@@ -34,10 +34,43 @@ def test_narrow_rows_come_one_to_a_lane_up_to_8192_wavefronts(rows, n, per_lane)
     assert launch.name == "antiquant_policy_vec_kernel" and launch.args[4] == per_lane
 
 
-@pytest.mark.parametrize("cols", [9, 16])
+@pytest.mark.parametrize("cols", [193, 16])
 def test_rows_whose_walk_passes_32_bits_run_one_element_per_lane(cols):
-    last = 2 ** 32 - 1 - 65535 * 8
+    last = 2 ** 32 - 1 - 65535 * 8                # (a width off 16 is as wide as the vectors take it)
     for rows, kernel in ((last, "antiquant_vec_kernel"), (last + 1, "antiquant_scalar_kernel"), (2 ** 32 - 1, "antiquant_scalar_kernel")):
         d = dict(src_dtype=abi.I8, dst_dtype=abi.F16, has_offset=0, per_tensor=1, k=rows, n=cols)
         launch, = route("ascq_antiquant", ("AntiQuantDesc", d), 1 << 52, SRC, None, None, None)
         assert launch.name == kernel and launch.grid_y >= 1
+
+
+# widths and numbers of elements from which rows off the vectors' width or alignment are vectors all the same
+@pytest.mark.parametrize("src,par,compute,fmt,width,elements,scalar_name", [
+    (abi.F16, abi.F16, abi.COMPUTE_F16, abi.QDST_I8, 64, 0, "quant_f16_fast_kernel"),
+    (abi.BF16, abi.BF16, abi.COMPUTE_F16, abi.QDST_I8, 192, 1 << 20, "quant_vec_kernel"),
+    (abi.F32, abi.F32, abi.COMPUTE_F32, abi.QDST_I8, 192, 1 << 20, "quant_vec_kernel"),
+    (abi.BF16, abi.BF16, abi.COMPUTE_F32, abi.QDST_FP8_E4M3FN, 384, 3 << 20, "quant_vec_kernel"),
+    (abi.F32, abi.F32, abi.COMPUTE_F32, abi.QDST_HIF8, 384, 3 << 20, "quant_vec_kernel")])
+def test_quantisers_of_odd_widths_are_vectors_where_wide_and_many(src, par, compute, fmt, width, elements, scalar_name):
+    mode = abi.CAST_ROUND if fmt == abi.QDST_HIF8 else abi.CAST_RINT
+    for n in (9, width - 1, width + 1, 2051):
+        for rows in (13, -(-elements // n) - 1, -(-elements // n)):
+            for policy in (abi.PER_CHANNEL, abi.PER_TENSOR):
+                if rows < 1:
+                    continue
+                cols = rows * n if policy == abi.PER_TENSOR else n        # one row, or rows of 2048
+                if cols % 8 == 0:
+                    continue
+                launch = quant(rows, n, src, par, fmt, mode, policy, compute)
+                assert launch.name == (scalar_name if cols >= width and rows * n >= elements else "quant_scalar_kernel"), (rows, n, policy)
+    # a width of whole vectors off their alignment
+    assert quant(7, 2048, src, par, fmt, mode, compute=compute, src_at=SRC + 4).name == (scalar_name if elements == 0 else "quant_scalar_kernel")
+
+
+@pytest.mark.parametrize("int4", [False, True])
+@pytest.mark.parametrize("dst,per_tensor,elements", [(abi.F16, 0, 1 << 20), (abi.F16, 1, 3 << 19), (abi.BF16, 0, 2 << 20), (abi.BF16, 1, 3 << 20)])
+def test_antiquant_of_odd_widths_is_vectors_where_wide_and_many(dst, per_tensor, elements, int4):
+    for n in (10, 190, 194, 2050):
+        for rows in (13, -(-elements // n) - 1, -(-elements // n)):
+            d = dict(src_dtype=abi.I4 if int4 else abi.I8, dst_dtype=dst, has_offset=1, per_tensor=per_tensor, k=rows, n=n)
+            launch, = route("ascq_antiquant", ("AntiQuantDesc", d), DST, SRC, OFFSET, SCALE, None)
+            assert launch.name == ("antiquant_vec_kernel" if n >= 192 and rows * n >= elements else "antiquant_scalar_kernel"), (rows, n)
