@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
         ts[row] = zero ? 1.0f : amax / 127.0f;
     }
     // |v * inv| <= 127 (1 + 2^-23) by construction, so the product needs no clamp for finite inputs (the median keeps
-    // infinities inside int8; NaN becomes -128).  Adding 1.5 * 2^23 rounds the fp32 product to the nearest integer, ties
+    // infinities inside int8; NaN becomes -128, or, kAny, 0 as in dynq_generic_kernel).  Adding 1.5 * 2^23 rounds the fp32 product to the nearest integer, ties
     // to even, exactly as rint does (the sum's spacing is 1 and the constant is even), and leaves that integer in two's
     // complement in the low mantissa bits: one add replaces rint, the conversion and the sign handling, and one byte
     // permute per pair gathers the low bytes.
@@ -523,7 +523,8 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
             uint32_t u[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float t = __builtin_amdgcn_fmed3f(v[k][e] * inv, -128.0f, 127.0f);
+                const float p = v[k][e] * inv;
+                const float t = kAny && p != p ? 0.0f : __builtin_amdgcn_fmed3f(p, -128.0f, 127.0f);
                 u[e] = __float_as_uint(t + 12582912.0f);
             }
             u32x2 out;

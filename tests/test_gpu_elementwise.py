@@ -828,3 +828,28 @@ def test_antiquant_of_odd_widths_off_the_vector_alignment(n, int4, dst_dt, has_o
     want = orc.antiquant(d, src, of if has_offset else None, sc)
     assert np.array_equal(bits(dst), want.view(np.uint16))
     assert room[0] == 0 and not room[1 + k * n:].any()
+
+
+@pytest.mark.parametrize("n", [7, 9, 1025, 2049, 4099, 8191, 16383, 16385])
+@pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16, abi.F32])
+def test_rows_of_odd_widths_quantise_nan_to_zero(n, src_dt):
+    """The dynamic quantiser in rows of any width: NaN counts for nothing in a row's maximum and becomes 0, a row that holds an infinity
+    has a scale of infinity and codes of 0 (every product is 0 or NaN), a row of NaN alone a scale of 1."""
+    m = 6
+    announce("dynamic quant, NaN", n, src_dt)
+    rng = np.random.default_rng(n)
+    plain = rng.standard_normal((m, n)).astype(np.float32)
+    bad = np.zeros((m, n), dtype=bool)
+    bad[0, [0, n - 1]] = bad[1, n // 2] = bad[2] = True
+    plain[bad] = 0.0
+    x = np.where(bad, np.float32(np.nan), plain)
+    x[3, n - 2], x[4, 0] = np.inf, -np.inf
+    x[4, n - 1] = np.nan
+
+    def as_src(a):
+        return a if src_dt == abi.F32 else a.astype(np.float16) if src_dt == abi.F16 else (a.view(np.uint32) >> 16).astype(np.uint16)
+    q, ts = ops.dynamic_quant_per_token(to_dev(as_src(x), "bf16" if src_dt == abi.BF16 else None))
+    wq, wts = orc.dynamic_quant_per_token(src_dt, as_src(plain))
+    wq[3:5], wts[3:5] = 0, np.inf
+    assert np.array_equal(ts.cpu().numpy(), wts)
+    assert np.array_equal(q.cpu().numpy(), wq)
