@@ -304,8 +304,8 @@ __global__ __launch_bounds__(kThreads) void quant_scalar_kernel(QuantArgs a)
 
 // Fast path of the fp16 contract for half sources (per tensor / per channel): the arithmetic stays in packed half
 // registers - v_pk_mul_f16, v_pk_add_f16 (one rounding each), v_rndne_f16, packed clamp, v_cvt_i16_f16 - about five
-// VALU operations per element instead of the generic path's conversions through fp32.  NaN inputs give an
-// unspecified int8 here (they are outside the operator's defined domain).
+// VALU operations per element instead of the generic path's conversions through fp32.  NaN gives an unspecified int8 in aligned
+// rows (it is outside the operator's defined domain) and, kNanZero, 0 in rows of any width, as with one element per lane.
 __device__ __forceinline__ f16x2 h2_from_bits(uint32_t b)
 {
     f16x2 r;
@@ -313,14 +313,25 @@ __device__ __forceinline__ f16x2 h2_from_bits(uint32_t b)
     return r;
 }
 
-__device__ __forceinline__ uint32_t quant_h2x2_to_i8x4(f16x2 a, f16x2 b)
+template <bool kNanZero>
+__device__ __forceinline__ f16x2 quant_h2_clamp(f16x2 a)
 {
     const f16x2 lo = {static_cast<half_t>(-128.0f), static_cast<half_t>(-128.0f)};
     const f16x2 hi = {static_cast<half_t>(127.0f), static_cast<half_t>(127.0f)};
-    a = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_elementwise_rint(a), lo), hi);
-    b = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_elementwise_rint(b), lo), hi);
-    const s16x2 ia = __builtin_convertvector(a, s16x2);
-    const s16x2 ib = __builtin_convertvector(b, s16x2);
+    a = __builtin_elementwise_rint(a);
+    if constexpr (kNanZero) {  // the larger and the smaller of NaN and 0 are 0: the positive part and the negative one
+        const f16x2 zero = {static_cast<half_t>(0.0f), static_cast<half_t>(0.0f)};
+        return __builtin_elementwise_min(__builtin_elementwise_max(a, zero), hi) + __builtin_elementwise_max(__builtin_elementwise_min(a, zero), lo);
+    } else {
+        return __builtin_elementwise_min(__builtin_elementwise_max(a, lo), hi);
+    }
+}
+
+template <bool kNanZero>
+__device__ __forceinline__ uint32_t quant_h2x2_to_i8x4(f16x2 a, f16x2 b)
+{
+    const s16x2 ia = __builtin_convertvector(quant_h2_clamp<kNanZero>(a), s16x2);
+    const s16x2 ib = __builtin_convertvector(quant_h2_clamp<kNanZero>(b), s16x2);
     uint32_t ua, ub;
     __builtin_memcpy(&ua, &ia, 4);
     __builtin_memcpy(&ub, &ib, 4);
@@ -374,8 +385,8 @@ __global__ __launch_bounds__(kThreads) void quant_f16_fast_kernel(QuantArgs a)
                     t[e] = t[e] + o[e];                    // one rounding
                 }
                 u32x2 out;
-                out[0] = quant_h2x2_to_i8x4(t[0], t[1]);
-                out[1] = quant_h2x2_to_i8x4(t[2], t[3]);
+                out[0] = quant_h2x2_to_i8x4<kAny>(t[0], t[1]);
+                out[1] = quant_h2x2_to_i8x4<kAny>(t[2], t[3]);
                 int8_t* to = a.dst + static_cast<size_t>(r0 + u) * a.n + j;
                 if constexpr (kAny) {
                     *reinterpret_cast<u32x2_any*>(to) = out;
@@ -421,11 +432,11 @@ int launch_quant(const QuantArgs& a, bool vec, hipStream_t st)
     // fp16 contract on a half source: scale / offset are half tensors or scalars
     const bool half = kSrc == ASCQ_F16 && kCt == ASCQ_F16 && kind == kQuantI8Rint &&
                       (a.policy == ASCQ_PER_TENSOR || (a.policy == ASCQ_PER_CHANNEL && kPar == ASCQ_F16));
-    // In us with one element per lane and as vectors: half to int8 4000 x 33 2.3 and 3.4, 10769 x 65 3.8 and 3.6; bfloat16 to int8 5426 x 129
+    // In us with one element per lane and as vectors: half to int8 4000 x 33 2.3 and 3.4, 27 x 2271 2.3 and 2.4, 4000 x 129 3.2 and 2.7; bfloat16 to int8 5426 x 129
     // 3.8 and 4.5, 1000 x 515 3.2 and 3.6, 5440 x 193 4.6 and 4.5, 2007 x 523 4.6 and 4.3, 1333333 x 9 33 and 270; to e4m3 (the kernel
     // of all formats) 1369 x 511 3.6 and 5.0, 11673 x 257 8.9 and 9.4, 5736 x 523 8.9 and 8.8, 7792 x 385 9.0 and 7.7.
     const bool any = !vec && (a.n % 8 == 0 || !per_row) &&
-                     (half                   ? any_address_ahead(a.rows, a.n, 64u, 0u)
+                     (half                   ? any_address_ahead(a.rows, a.n, 96u, 1u << 17)
                       : kind == kQuantI8Rint ? any_address_ahead(a.rows, a.n, 192u, 1u << 20)
                                              : any_address_ahead(a.rows, a.n, 384u, 3u << 20));
     if (!vec && !any) {

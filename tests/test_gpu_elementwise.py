@@ -853,3 +853,31 @@ def test_rows_of_odd_widths_quantise_nan_to_zero(n, src_dt):
     wq[3:5], wts[3:5] = 0, np.inf
     assert np.array_equal(ts.cpu().numpy(), wts)
     assert np.array_equal(q.cpu().numpy(), wq)
+
+
+@pytest.mark.parametrize("n,elements", [(9, 0), (2051, 0), (97, 1 << 17), (2051, 1 << 17), (4099, 1 << 17)])
+@pytest.mark.parametrize("per_channel", [True, False])
+@pytest.mark.parametrize("offset", [0.0, 2.5])
+def test_half_rows_of_odd_widths_quantise_nan_to_zero(n, elements, per_channel, offset):
+    """Half per channel and per tensor in rows of any width: NaN, whether it comes in or arises from an infinity times 0, becomes 0,
+    infinities the end of the range on their side; everything else is the oracle's.  One element per lane and as vectors."""
+    m = max(5, -(-elements // n))
+    announce("half quant, NaN", n, per_channel, offset)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((m, n)).astype(np.float16)
+    s = rng.uniform(5, 40, n).astype(np.float16)
+    x[0, [0, n - 1]], x[1, n // 2], x[2] = np.nan, -np.nan, np.nan
+    x[3, 1], x[3, n - 2], x[4, n // 3] = np.inf, -np.inf, np.inf
+    if per_channel:
+        s[n // 3] = 0.0
+    special = ~np.isfinite(x)
+    q = torch.full((m, n), 77, dtype=torch.int8, device=DEV)
+    ops.ascend_quant(q, to_dev(x), to_dev(s) if per_channel else 7.5, offset)
+    d = abi.QuantDesc(policy=abi.PER_CHANNEL if per_channel else abi.PER_TENSOR, src_dtype=abi.F16, scale_dtype=abi.F16, compute=abi.COMPUTE_F16,
+                      scale=0.0 if per_channel else 7.5, offset_kind=abi.OFFSET_SCALAR, offset=offset, round_mode=abi.CAST_RINT, n=n,
+                      cal_count=m * n)
+    want = orc.quant(d, np.where(special, np.float16(0.0), x), s if per_channel else None).reshape(m, n)
+    with np.errstate(invalid="ignore"):
+        product = x * (s if per_channel else np.float16(7.5))
+    want = np.where(special, np.where(np.isnan(product), 0, np.where(product > 0, 127, -128)), want)
+    assert np.array_equal(q.cpu().numpy(), want)

@@ -45,7 +45,7 @@ def test_rows_whose_walk_passes_32_bits_run_one_element_per_lane(cols):
 
 # widths and numbers of elements from which rows off the vectors' width or alignment are vectors all the same
 @pytest.mark.parametrize("src,par,compute,fmt,width,elements,scalar_name", [
-    (abi.F16, abi.F16, abi.COMPUTE_F16, abi.QDST_I8, 64, 0, "quant_f16_fast_kernel"),
+    (abi.F16, abi.F16, abi.COMPUTE_F16, abi.QDST_I8, 96, 1 << 17, "quant_f16_fast_kernel"),
     (abi.BF16, abi.BF16, abi.COMPUTE_F16, abi.QDST_I8, 192, 1 << 20, "quant_vec_kernel"),
     (abi.F32, abi.F32, abi.COMPUTE_F32, abi.QDST_I8, 192, 1 << 20, "quant_vec_kernel"),
     (abi.BF16, abi.BF16, abi.COMPUTE_F32, abi.QDST_FP8_E4M3FN, 384, 3 << 20, "quant_vec_kernel"),
@@ -63,7 +63,8 @@ def test_quantisers_of_odd_widths_are_vectors_where_wide_and_many(src, par, comp
                 launch = quant(rows, n, src, par, fmt, mode, policy, compute)
                 assert launch.name == (scalar_name if cols >= width and rows * n >= elements else "quant_scalar_kernel"), (rows, n, policy)
     # a width of whole vectors off their alignment
-    assert quant(7, 2048, src, par, fmt, mode, compute=compute, src_at=SRC + 4).name == (scalar_name if elements == 0 else "quant_scalar_kernel")
+    for rows in (7, 2048):
+        assert quant(rows, 2048, src, par, fmt, mode, compute=compute, src_at=SRC + 4).name == (scalar_name if rows == 2048 else "quant_scalar_kernel")
 
 
 @pytest.mark.parametrize("int4", [False, True])
