@@ -10,6 +10,9 @@ instruction.  For every such instruction, on every path that follows it, this pr
   * no vector instruction that writes one of its operands within kOperand wait states before it.
 In the kernels of COUNTED a step loads one operand into LDS and the other into registers, and its counted waits rest on both:
 between two barriers either both kinds of loads are issued or none (the compiler drops a register load that nobody uses).
+In the kernels of STAGED a stage's loads into LDS go out in one run, those into registers behind them, and the counted wait ahead of
+a stage's LDS reads leaves the next stage's loads on their way: on every path to such a wait, its count is at most the
+number of loads from the start of the last run on.  (Their matrix instructions are the compiler's own: it knows what they need.)
 """
 import os
 import re
@@ -22,6 +25,7 @@ LLVM = os.environ.get("LLVM_BIN", "/opt/rocm/llvm/bin")
 MATRIX = ("v_mfma_i32_16x16x64_i8", "v_mfma_f32_16x16x32_f16", "v_mfma_scale_f32_16x16x128_f8f6f4")
 kResult, kOperand = 19, 2
 COUNTED = ("wq_gemm_kernel",)
+STAGED = ("wq_rows_kernel",)
 
 
 def registers(operand):
@@ -133,6 +137,41 @@ def dropped_loads(body):
     return bad
 
 
+def loose_waits(body):
+    where = {i.address: n for n, i in enumerate(body)}
+
+    def guards(n):
+        """the count of a wait with LDS reads behind it (no other access or matrix instruction in between)"""
+        m = re.search(r"vmcnt\((\d+)\)", body[n].text) if body[n].name == "s_waitcnt" else None
+        for i in body[n + 1:] if m else ():
+            if i.name.startswith("ds_read"):
+                return int(m[1])
+            if i.name.startswith(("ds_", "buffer_", "global_", "v_mfma", "s_waitcnt", "s_barrier", "s_branch", "s_cbranch", "s_endpgm")):
+                break
+        return None
+
+    bad, seen, work = [], set(), [(0, 0, False)]               # instruction, loads since the last run's start, still in the run
+    while work:
+        n, loads, run = work.pop()
+        while n < len(body) and (n, loads, run) not in seen:
+            seen.add((n, loads, run))
+            i = body[n]
+            if i.name.startswith(("buffer_load", "global_load")):
+                lds = "_lds" in i.name or i.text.endswith(" lds")
+                loads, run = (1 if lds and not run else min(loads + 1, 64)), lds
+            left = guards(n)
+            if left is not None and left > loads:
+                bad.append("%s at %x leaves more than the %d loads since the last run into LDS began" % (i.text, i.address, loads))
+            if i.target is not None:
+                work.append((where[i.target], loads, run))
+                if i.name == "s_branch":
+                    break
+            if i.name in ("s_endpgm", "s_setpc_b64"):
+                break
+            n += 1
+    return sorted(set(bad))
+
+
 def main(paths):
     status = 0
     for path in paths:
@@ -140,7 +179,8 @@ def main(paths):
         for name, body in kernels(path):
             count = sum(i.matrix for i in body)
             seen += count
-            bad = faults(body) if count else []
+            staged = any(c in name for c in STAGED)
+            bad = loose_waits(body) if staged else faults(body) if count else []
             if any(c in name for c in COUNTED):
                 bad += dropped_loads(body)
             for b in bad[:10]:

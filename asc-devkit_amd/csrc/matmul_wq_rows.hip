@@ -38,13 +38,27 @@ __device__ __forceinline__ uint32_t sum_place(uint32_t row, uint32_t col)
     return (row * BN + col) ^ (((row >> 2) & 3u) << 4);
 }
 
+// The loads of an even (0) or odd (1) stage.
+template <int BM, int BN, int kKind, bool kOff>
+struct StageLoads {
+    // Whether a sub-step fetches parameters: with int8 none does; in the sum form those at the end of 128 k (loads that nobody uses the
+    // compiler leaves out, and a count that includes them would not hold a wait back).
+    static constexpr bool params(int parity, int s) { return kKind == kInt4Weight || (kKind == kInt4Sum && ((parity * (64 / BM) + s) & 1) != 0); }
+    static constexpr int count(int parity)
+    {
+        int n = kALoads + 64 / BM * (BN / 16);
+        for (int s = 0; s < 64 / BM; ++s) n += params(parity, s) ? BN / 16 * (kOff ? 2 : 1) : 0;
+        return n;
+    }
+};
+
 template <int BM, int BN, int kKind, bool kOff>
 __global__ __launch_bounds__(kWaves * 64, 2) void wq_rows_kernel(WqParams p)
 {
     constexpr bool kInt4 = kKind != kInt8Weight, kSum = kKind == kInt4Sum;
     constexpr int NI = BM / 16, NJ = BN / 16, SUB = 64 / BM;  // a stage: SUB times BM rows x 64 k
     constexpr int kParams = kInt4 ? SUB * NJ : 1;
-    constexpr int kBLoads = SUB * NJ + (kInt4 ? SUB * NJ * (kOff ? 2 : 1) : 0);
+    using Loads = StageLoads<BM, BN, kKind, kOff>;
     constexpr uint32_t kUnit = kInt4 ? 2u : 1u;               // a wavefront's share of k is a multiple of this many 64 k
     static_assert(NI * 16 == BM && NJ * 16 == BN && SUB * BM == 64, "tile shape");
     __shared__ __attribute__((aligned(1024))) char A0[kWaves * kStageBytes], A1[kWaves * kStageBytes];
@@ -107,24 +121,27 @@ __global__ __launch_bounds__(kWaves * 64, 2) void wq_rows_kernel(WqParams p)
         u32x4 w[SUB][NJ];                                     // int4: the first two
         uint32_t sc[kParams], of[kParams];
     };
-    auto fetch_one = [&](Raw& raw, uint32_t stage, int s, int j) __attribute__((always_inline)) {
+    auto fetch_one = [&](Raw& raw, uint32_t stage, int s, int j, auto parity) __attribute__((always_inline)) {
+        constexpr int kPar = decltype(parity)::value;
         const uint32_t sub = sub0 + stage * SUB + s;
         if constexpr (kInt4) {
             const uint32_t pat = ((2u * sub) >> p.gs_shift) * p.n * 2u;
             const auto v = __builtin_amdgcn_raw_buffer_load_b64(rw, boff, sub * 512u + j * bslab, 0);
             raw.w[s][j][0] = v[0];
             raw.w[s][j][1] = v[1];
-            raw.sc[s * NJ + j] = __builtin_amdgcn_raw_buffer_load_b16(rs, poff + j * 32u, pat, 0);
-            if constexpr (kOff) raw.of[s * NJ + j] = __builtin_amdgcn_raw_buffer_load_b16(ro, poff + j * 32u, pat, 0);
+            if (Loads::params(kPar, s)) {
+                raw.sc[s * NJ + j] = __builtin_amdgcn_raw_buffer_load_b16(rs, poff + j * 32u, pat, 0);
+                if constexpr (kOff) raw.of[s * NJ + j] = __builtin_amdgcn_raw_buffer_load_b16(ro, poff + j * 32u, pat, 0);
+            }
         } else {
             raw.w[s][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, boff, sub * 64u + j * bslab, 0));
         }
     };
-    auto fetch = [&](Raw& raw, uint32_t stage) __attribute__((always_inline)) {
+    auto fetch = [&](Raw& raw, uint32_t stage, auto parity) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < SUB; ++s)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) fetch_one(raw, stage, s, j);
+            for (int j = 0; j < NJ; ++j) fetch_one(raw, stage, s, j, parity);
     };
     f16x2 csc[NJ], cof[NJ];                                   // int8: scale and offset belong to the column
     if constexpr (!kInt4) {
@@ -172,8 +189,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void wq_rows_kernel(WqParams p)
 
     // Stage `stage` lies in S and raw.
     auto step = [&](char* S, Raw& raw, uint32_t stage, auto parity) __attribute__((always_inline)) {
-        // everything but the next stage's loads has arrived
-        constexpr int kLeft = kALoads + kBLoads;
+        // everything but the next stage's loads has arrived (the build looks the loads and counts over: check_matrix_asm.py)
+        constexpr int kLeft = Loads::count(1 - decltype(parity)::value);
         __builtin_amdgcn_s_waitcnt(0x0F70 | (kLeft & 15) | ((kLeft >> 4) << 14));
         asm volatile("" ::: "memory");
         f16x8 af[SUB][2][NI];
@@ -232,20 +249,25 @@ __global__ __launch_bounds__(kWaves * 64, 2) void wq_rows_kernel(WqParams p)
                 }
             }
         }
-        fetch(raw, stage + 2u);
+        fetch(raw, stage + 2u, parity);
         __builtin_amdgcn_sched_barrier(0);
     };
 
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
     Raw r0, r1;
+    __builtin_amdgcn_sched_barrier(0);                        // (the first waits count these loads in this order)
     load_x(A0, 0);
-    fetch(r0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(r0, 0, even);
     __builtin_amdgcn_sched_barrier(0);
     load_x(A1, 1);
-    fetch(r1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(r1, 1, odd);
     __builtin_amdgcn_sched_barrier(0);
     for (uint32_t i = 0; i < stages; i += 2u) {
-        step(A0, r0, i, std::integral_constant<int, 0>{});
-        step(A1, r1, i + 1u, std::integral_constant<int, 1>{});
+        step(A0, r0, i, even);
+        step(A1, r1, i + 1u, odd);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);                       // the loads past the end
     asm volatile("" ::: "memory");

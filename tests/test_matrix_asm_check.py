@@ -47,3 +47,22 @@ def test_loads_that_the_compiler_dropped_are_found():
     assert len(check.dropped_loads(body(*step, *step[:1], *step[2:]))) == 1
     # (a buffer load into LDS counts as such)
     assert len(check.dropped_loads(body("buffer_load_dwordx4 v1, s[4:7], 0 offen lds", "s_barrier"))) == 1
+
+
+def test_waits_that_count_more_loads_than_there_are_are_found():
+    """The whole-k tiles: a stage is a run of loads into LDS and the loads into registers behind it; the wait ahead of a stage's LDS reads
+    leaves the next stage on its way.  Too large a count, a load between those of the run, and both only on one path."""
+    lds, reg, read = "buffer_load_dwordx4 v1, s[4:7], s9 offen lds", "buffer_load_dwordx2 v[4:5], v2, s[8:11], s9 offen", "ds_read_b128 v[8:11], v3"
+    stage = [lds, lds, reg]
+
+    def loop(count, prologue, steady=stage):
+        start = len(prologue)
+        step = ["s_waitcnt vmcnt(%d)" % count, read, *steady]
+        return body(*prologue, *step, *step, "s_cbranch_scc1 s -> %d" % start, "s_waitcnt vmcnt(0)", "s_endpgm")
+    assert check.loose_waits(loop(3, stage + stage)) == []
+    assert check.loose_waits(loop(4, stage + stage))                               # a load that is counted and not issued
+    assert check.loose_waits(loop(3, [lds, reg, lds] * 2))                         # the last of the run behind a register load
+    assert check.loose_waits(loop(3, stage + [reg, lds, lds]))                     # the run behind the register loads
+    assert check.loose_waits(loop(3, stage + stage, [lds, lds]))                   # a register load dropped from the steps
+    assert check.loose_waits(body(*stage, "s_cbranch_scc1 s -> 5", reg, "s_nop 0", "s_waitcnt vmcnt(4)", read, "s_endpgm"))  # on one path
+    assert check.loose_waits(body(*stage, *stage, "s_waitcnt vmcnt(9)", "v_mfma_f32_16x16x32_f16 v[0:3], v[4:7], v[8:11], v[0:3]", "s_endpgm")) == []
