@@ -1013,7 +1013,9 @@ bool fast_ok(const ascq_w4a16_desc* d, const void* x, const void* w, const void*
 // pass over the weights per 32 rows: k = 5632, n = 1408, 1149 rows 1069 -> 68 us.  Above 96 rows always; from 5 on where the
 // repacking (4.5 us and 0.42 us per MB of weights) and the packed form are expected to be ahead of the passes (up to 16 rows 9.5 us and
 // 0.3 per row, above 17; another 8 or 12 once the weights are some 10 MB, and 0.32 or 0.3 per MB; fits to 45 random calls): 64 x 1792 x
-// 22496 76 against 34 us, 33 x 2304 x 1152 32 and 11, 16 x 8448 x 1920 32 and 19, 8 x 4864 x 4288 22 and 21, 12 x 8448 x 13088 37 and 52.
+// 22496 76 against 34 us, 33 x 2304 x 1152 32 and 11, 16 x 8448 x 1920 32 and 19, 8 x 3072 x 13920 21 and 27, 12 x 8448 x 13088 37 and 52.
+// Ahead is less than 0.72 of the passes up to 16 rows and 0.8 above: the estimate of the passes is up to a fifth above, the other up to as
+// much below what they take, and from 0.9 on 51 of 620 random calls were slower than in passes, by up to 20 %.
 bool packed_ahead(const ascq_w4a16_desc* d)
 {
     if (d->m > 96u) {
@@ -1023,7 +1025,7 @@ bool packed_ahead(const ascq_w4a16_desc* d)
     const double pass = d->m <= kTileRows ? 9.5 + 0.3 * d->m + 8.0 * filled + 0.32 * mb : 17.0 + 12.0 * filled + 0.3 * mb;
     // (more than 128 groups along k: the passes over packed weights do not take every shape)
     return d->m > 4u && d->k / d->group_size <= 128u && 4.5 + 0.42 * mb + w4a16_packed_estimate(d->m, d->n, d->k) <
-                            0.9 * ((d->m + 2u * kTileRows - 1u) / (2u * kTileRows)) * pass;
+                            (d->m <= kTileRows ? 0.72 : 0.8) * ((d->m + 2u * kTileRows - 1u) / (2u * kTileRows)) * pass;
 }
 
 bool pack_first(const ascq_w4a16_desc* d)

@@ -39,7 +39,9 @@ void __hipRegisterFunction(void**, const void* host, char*, const char* name, un
     for (const char* part : {"(anonymous namespace)::", "ascq::", "void "}) {
         for (size_t at; (at = s.find(part)) != std::string::npos;) s.erase(at, std::char_traits<char>::length(part));
     }
-    kernels()[host] = s.substr(0, s.rfind('('));
+    size_t end = 0;  // of the name: the first bracket outside the template arguments
+    for (int depth = 0; end < s.size() && (depth > 0 || s[end] != '('); ++end) depth += s[end] == '<' ? 1 : s[end] == '>' ? -1 : 0;
+    kernels()[host] = s.substr(0, end);
 }
 int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t shared, void* stream)
 {

@@ -75,3 +75,29 @@ def test_antiquant_of_odd_widths_is_vectors_where_wide_and_many(dst, per_tensor,
             d = dict(src_dtype=abi.I4 if int4 else abi.I8, dst_dtype=dst, has_offset=1, per_tensor=per_tensor, k=rows, n=n)
             launch, = route("ascq_antiquant", ("AntiQuantDesc", d), DST, SRC, OFFSET, SCALE, None)
             assert launch.name == ("antiquant_vec_kernel" if n >= 192 and rows * n >= elements else "antiquant_scalar_kernel"), (rows, n)
+
+
+def half_matmul(entry, m, k, n, **kw):
+    x, w, scale, offset, ws = 1 << 30, 1 << 36, 1 << 38, 1 << 39, 1 << 40
+    if entry == "ascq_matmul_w8a16":
+        d = ("W8A16Desc", dict(m=m, n=n, k=k, has_offset=1, out_dtype=abi.F16, **kw))
+        return route(entry, d, 1 << 42, x, w, offset, scale, ws, 1 << 35, None)
+    d = ("W4A16Desc", dict(m=m, n=n, k=k, has_offset=1, **kw))
+    if entry == "ascq_matmul_w4a16":
+        return route(entry, d, 1 << 42, x, w, scale, offset, ws, 1 << 35, None)
+    return route(entry, d, 1 << 42, x, w, scale, offset, None)
+
+
+@pytest.mark.parametrize("m,k,n,whole_k", [(5, 4736, 8064, False), (6, 5376, 14336, False), (8, 4736, 7488, False), (10, 5376, 3424, False),
+                                           (9, 3072, 1280, False), (9, 7808, 3312, True), (14, 8448, 1376, True), (16, 8448, 1920, True), (30, 1920, 5312, True)])
+def test_int8_passes_of_few_rows_stay_where_they_are_ahead(m, k, n, whole_k):
+    first, *_ = half_matmul("ascq_matmul_w8a16", m, k, n, trans_b=1)
+    assert first.name == ("wq_rows_kernel" if whole_k else "w8a16_nk_kernel")
+
+
+@pytest.mark.parametrize("m,k,n,packed", [(8, 3072, 13920, False), (9, 3456, 9728, False), (5, 2944, 15104, False), (12, 6272, 6272, False),
+                                          (17, 9600, 7744, False), (12, 8448, 13088, False), (16, 8448, 1920, True), (33, 2304, 1152, True),
+                                          (64, 1792, 22496, True), (97, 4096, 27392, True)])
+def test_int4_passes_of_few_rows_stay_where_they_are_ahead(m, k, n, packed):
+    first, *_ = half_matmul("ascq_matmul_w4a16", m, k, n, group_size=128)
+    assert first.name == ("pack_w4_tiles_kernel" if packed else "w4a16_tile_kernel")
