@@ -897,7 +897,13 @@ extern "C" int ascq_matmul_w4a16_packed(const ascq_w4a16_desc* d, void* y, const
         w.n = d->n;
         w.k = d->k;
         w.gs_shift = p.gs_shift;
-        if (wq_rows_ahead(w, true, sum_form, d->has_offset != 0, tiles ? wq_gemm_estimate(d->m, d->n, d->k) : passes_estimate(d->m, p.slabs, d->k, sum_form, cus), st)) {
+        double other = tiles ? wq_gemm_estimate(d->m, d->n, d->k) : passes_estimate(d->m, p.slabs, d->k, sum_form, cus);
+        if (!tiles && d->k / d->group_size > kRowsMaxGroups) {
+            // (passes of the kernel for up to 4 rows, which takes less than the estimate with few more: 15 of 62 random calls with 5 rows, and
+            // 4 of 206 with 7 or 8, were slower off it, 5 x 13568 x 8544 in groups of 64 24.9 us and 31.8)
+            other = d->m <= 5u ? 0.0 : 0.94 * other;
+        }
+        if (wq_rows_ahead(w, true, sum_form, d->has_offset != 0, other, st)) {
             return launch_status("ascq_matmul_w4a16_packed");
         }
         if (tiles) {

@@ -101,3 +101,10 @@ def test_int8_passes_of_few_rows_stay_where_they_are_ahead(m, k, n, whole_k):
 def test_int4_passes_of_few_rows_stay_where_they_are_ahead(m, k, n, packed):
     first, *_ = half_matmul("ascq_matmul_w4a16", m, k, n, group_size=128)
     assert first.name == ("pack_w4_tiles_kernel" if packed else "w4a16_tile_kernel")
+
+
+@pytest.mark.parametrize("m,k,n,group,passes", [(5, 13568, 8544, 64, True), (5, 6784, 5680, 32, True), (8, 13440, 8800, 64, True), (8, 6784, 5680, 32, False),
+                                                (16, 13440, 4000, 64, False), (5, 6784, 5680, 128, False)])
+def test_packed_int4_in_many_groups_stays_in_passes_with_the_fewest_rows(m, k, n, group, passes):
+    first, *_ = half_matmul("ascq_matmul_w4a16_packed", m, k, n, group_size=group)
+    assert first.name == ("w4a16_packed_kernel" if passes else "wq_rows_kernel")
