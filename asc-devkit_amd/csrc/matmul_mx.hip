@@ -48,7 +48,7 @@ __device__ __forceinline__ void mx_static_for(F&& f)
 constexpr uint32_t kMxBM = 256, kMxBN = 256, kMxBK = 128;  // BK in bytes of an operand row
 constexpr int kMxThreads = 512;
 constexpr uint32_t kMxBufferCols = 1u << 20;  // columns up to which a tile's offsets in c fit 31 bits
-constexpr int kMxNt = 2;                      // cache policy of the stores: non-temporal (c is written once)
+constexpr int kMxNt = 2;                      // cache policy of stores of whole lines: non-temporal (c is written once)
 constexpr uint32_t kMxScaleBuf = (kMxBM + kMxBN) * 16u;  // 16 scale bytes of every row of a tile's a and b
 
 // kFour: both operands 4-bit (e2m1); otherwise both a byte per value in memory, with the instruction's format codes
@@ -397,6 +397,9 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         return;
     }
     const uint32_t row_size = p.n * size;
+    // Rows of whole lines bypass the caches; others leave parts of lines for the next store to fill: bfloat16 1792 x 7424 x 1024 13.6 us and 15.7
+    // through the caches, 1792 x 7504 x 1024 17.0 and 15.8 (16.5 before the buffer).
+    const bool whole_lines = row_size % 128u == 0 && (reinterpret_cast<uintptr_t>(p.c) & 127u) == 0;
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         static_cast<char*>(p.c) + static_cast<size_t>(row0) * row_size, 0, static_cast<int>(rows_left * row_size), 0x00020000);
     uint32_t row_lo = wm * (TI * 32u) * row_size;
@@ -411,7 +414,7 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
         const uint32_t colw = n0 + wn * (TJ * 32u);
         const uint32_t col = odd ? colw + 32u + (lrow - 1u) : colw + lrow;  // first column of the lane's pair
         const uint32_t at = col < p.n ? 4u * h * row_size + col * 2u : kNoColumn;
-        auto store_all = [&](auto to_bf16) __attribute__((always_inline)) {
+        auto store_all = [&](auto to_bf16, auto policy) __attribute__((always_inline)) {
             constexpr bool kBf16 = decltype(to_bf16)::value;
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
@@ -423,14 +426,21 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
                     const uint32_t recv = static_cast<uint32_t>(
                         __builtin_amdgcn_mov_dpp(static_cast<int>(odd ? h0 : h1), 0xB1, 0xF, 0xF, true));  // lane ^ 1
                     const uint32_t word = odd ? (recv | (h1 << 16)) : (h0 | (recv << 16));
-                    __builtin_amdgcn_raw_buffer_store_b32(word, rc, at, row_at(i, r), kMxNt);
+                    __builtin_amdgcn_raw_buffer_store_b32(word, rc, at, row_at(i, r), decltype(policy)::value);
                 }
             }
         };
-        if (bf) {
-            store_all(std::true_type{});
+        auto store_as = [&](auto policy) __attribute__((always_inline)) {
+            if (bf) {
+                store_all(std::true_type{}, policy);
+            } else {
+                store_all(std::false_type{}, policy);
+            }
+        };
+        if (whole_lines) {
+            store_as(std::integral_constant<int, kMxNt>{});
         } else {
-            store_all(std::false_type{});
+            store_as(std::integral_constant<int, 0>{});
         }
         return;
     }
@@ -438,14 +448,19 @@ __global__ __launch_bounds__(kMxThreads, 1) void mx_tile_kernel(MxParams p)
     for (int j = 0; j < TJ; ++j) {
         const uint32_t col = n0 + (wn * TJ + j) * 32u + lrow;
         const uint32_t at = col < p.n ? 4u * h * row_size + col * size : kNoColumn;
-        if (f32) {
+        auto store_f32 = [&](auto policy) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r] + bias[j]), rc, at, row_at(i, r), kMxNt);
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r] + bias[j]), rc, at, row_at(i, r), decltype(policy)::value);
                 }
             }
+        };
+        if (f32 && whole_lines) {
+            store_f32(std::integral_constant<int, kMxNt>{});
+        } else if (f32) {
+            store_f32(std::integral_constant<int, 0>{});
         } else {
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
