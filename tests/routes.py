@@ -50,7 +50,7 @@ def _calls():
 
 
 def call(entry, *args):
-    """(status, [Launch, ...]) of one call; an argument is a number, None, or (descriptor class name, {field: value})."""
+    """(status, [Launch, ...]) of one call; an argument is a number, None, or (descriptor class name, {field: value}), fields likewise."""
     return _calls()(entry, args)
 
 
@@ -63,6 +63,10 @@ def route(entry, *args):
 
 def _child():
     from ascq import _abi as abi
+
+    def held(a):
+        return getattr(abi, a[0])(**{field: held(v) for field, v in a[1].items()}) if isinstance(a, list) else a
+
     log = C.CDLL(LOG, mode=C.RTLD_GLOBAL)
     log.launch_log_take.restype = C.c_char_p
     lib = C.CDLL(abi.LIB_PATH)
@@ -70,8 +74,7 @@ def _child():
         entry, args = json.loads(line)
         fn = getattr(lib, entry)
         fn.restype, fn.argtypes = abi.SIGNATURES[entry]
-        held = [getattr(abi, a[0])(**a[1]) if isinstance(a, list) else a for a in args]
-        status = fn(*[C.byref(h) if isinstance(h, C.Structure) else h for h in held])
+        status = fn(*[C.byref(h) if isinstance(h, C.Structure) else h for h in map(held, args)])
         print(json.dumps([status, [text.rsplit(";", 3) for text in log.launch_log_take().decode().splitlines()]]), flush=True)
 
 

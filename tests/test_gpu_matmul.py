@@ -650,16 +650,22 @@ def test_group_matmul_tile_shapes_by_width(counts, n, nz, k, act):
     assert torch.equal(y2.view(torch.int16), y.view(torch.int16))
 
 
+# counts, and the k from which on they run the form whose loads are spread over a step and a half
+GROUP_REMAINDERS = [([300, 64, 1, 130, 0, 96, 65, 17], 2560), ([33, 128, 256, 16, 480, 385], 1408), ([257, 512, 64, 384], 1280)]
+GROUP_WIDE = 2592      # columns, wide enough for tiles of 256 rows (544: tiles of 64 x 64 with a ring of stages)
+
+
 @pytest.mark.parametrize("k", [256, 384, 1280, 1408, 2432, 2560, 3072, 3200])
 @pytest.mark.parametrize("nz", [False, True])
-@pytest.mark.parametrize("counts", [[300, 64, 1, 130, 0, 96, 65, 17], [33, 128, 256, 16, 480, 385], [257, 512, 64, 384]])
-def test_group_matmul_remainders_in_both_forms(counts, nz, k):
+@pytest.mark.parametrize("counts", [counts for counts, _ in GROUP_REMAINDERS])
+@pytest.mark.parametrize("n", [544, GROUP_WIDE])
+def test_group_matmul_remainders_in_both_forms(counts, nz, k, n):
     """Remainders of 64 and of 128 rows, and big tiles whose second wavefront row is empty, partly filled or full, on both
     sides of the rule that names the instruction: from k = 2560, 1408 and 1280 on (84, 216 and 304 rows per group) the form
-    whose loads are spread over a step and a half; even and odd numbers of K steps."""
-    announce("group remainders", counts, nz, k)
+    whose loads are spread over a step and a half; even and odd numbers of K steps.  The narrow width runs the ring's tiles."""
+    announce("group remainders", counts, nz, k, n)
     rng = np.random.default_rng(k + len(counts) + nz)
-    g, m, n = len(counts), sum(counts), 544
+    g, m = len(counts), sum(counts)
     x, w = rand_i8(rng, (m, k)), rand_i8(rng, (g, k, n))
     sc, tok = rng.uniform(1e-4, 1e-3, (g, n)).astype(np.float32), rng.uniform(5e-3, 2e-2, m).astype(np.float32)
     y = torch.zeros((m, n), dtype=torch.float16, device=DEV)
@@ -711,14 +717,18 @@ def run_group(m, k, n, counts, kind, out, rng, with_bias, act, rows_cap=None):
     return bits(y), (want.view(np.uint16) if want.dtype == np.float16 else want)
 
 
+GROUP_EDGES = [[30, 0, 1, 45, 12], [256, 256], [0, 0, 700, 0], [1, 1, 1, 1, 1, 1, 1, 1], [513, 255, 0, 256]]
+GROUP_EDGES_WIDE = 6664      # columns, wide enough for tiles of 256 rows (520: the ring's tiles)
+
+
 @pytest.mark.parametrize("kind", [abi.GROUP_LIST_COUNTS, abi.GROUP_LIST_PREFIX_SUM])
-@pytest.mark.parametrize("counts", [[30, 0, 1, 45, 12], [256, 256], [0, 0, 700, 0], [1, 1, 1, 1, 1, 1, 1, 1],
-                                    [513, 255, 0, 256]])
-def test_group_matmul_edge_cases(kind, counts):
-    announce("grouped matmul", kind, counts)
+@pytest.mark.parametrize("counts", GROUP_EDGES)
+@pytest.mark.parametrize("n", [520, GROUP_EDGES_WIDE])
+def test_group_matmul_edge_cases(kind, counts, n):
+    announce("grouped matmul", kind, counts, n)
     rng = np.random.default_rng(sum(counts) + len(counts))
     m = sum(counts) + 8                                         # 8 rows belong to no group and stay untouched
-    got, want = run_group(m, 256, 520, counts, kind, torch.bfloat16, rng, True, abi.MM_ACT_NONE)
+    got, want = run_group(m, 256, n, counts, kind, torch.bfloat16, rng, True, abi.MM_ACT_NONE)
     assert np.array_equal(got, want)
     assert np.all(got[sum(counts):] == 0x7E7E)
 
@@ -869,8 +879,9 @@ def test_w4a16_packed_small(m, k, n, gs, offset):
                                        (96, 1280, 96, 128), (48, 4224, 32, 32)])
 @pytest.mark.parametrize("offset", [True, False])
 def test_w4a16_few_rows_repacked_or_in_passes(m, k, n, gs, offset):
-    """[k, n / 2] weights that are repacked into the workspace first and, with a workspace that has no room for that, passes over
-    them (n a multiple of 32; (48, 4224, 32, 32) has more groups than the repacked form is taken for): the oracle's values both ways."""
+    """[k, n / 2] weights of which some are repacked into the workspace first and some run as passes (5 rows; (48, 4224, 32, 32) has
+    more groups than the repacked form is taken for): the oracle's values; a workspace too small for the passes is refused where
+    the repacked weights do not fit it either.  (A workspace for the passes and not for the repacked weights: a test below.)"""
     import ctypes as C
     announce("w4a16 few rows", m, k, n, gs, offset)
     rng = np.random.default_rng(m + k + n)
@@ -930,13 +941,17 @@ def test_w4a16_packed_more_than_four_rows(m, k, n, gs):
     assert torch.equal(y1, y2)
 
 
-@pytest.mark.parametrize("m,k,n,gs", [(49, 128, 8, 32), (128, 256, 248, 64), (129, 384, 264, 128), (257, 640, 520, 128), (300, 128, 1032, 32),
-                                       (1300, 256, 14600, 256)])
+W4_MANY_ROWS = {"wq_rows_kernel": [(49, 128, 8, 32), (128, 256, 248, 64), (129, 384, 264, 128), (257, 640, 520, 128)],
+                "wq_gemm_kernel<128, 128, ": [(300, 128, 1032, 32), (69, 128, 2312, 32), (129, 384, 5128, 64), (257, 640, 6152, 32), (1030, 1152, 2056, 128)],
+                "wq_gemm_kernel<256, 256, ": [(1300, 256, 14600, 256)]}
+
+
+@pytest.mark.parametrize("m,k,n,gs", [s for sizes in W4_MANY_ROWS.values() for s in sizes])
 @pytest.mark.parametrize("offset", ["int", "frac", None])
 def test_w4a16_packed_many_rows(m, k, n, gs, offset):
     """More rows than a few passes: the half GEMM whose B-tile loader de-quantises the packed tiles.  Two steps of k and more, row
     and column tails, groups of half a step, on tiles of 128 x 128; the last case runs 256 x 256 ones, those beyond a whole
-    round cut in half (checked on its first, a middle and the last columns)."""
+    round cut in half (wide ones are checked on their first, a middle and the last columns); few rows or columns run whole-k tiles."""
     announce("w4a16 packed many rows", m, k, n, gs, offset)
     rng = np.random.default_rng(m + 3 * k + n)
     x, wp, sc, of = w4_case(rng, m, k, n, gs, offset is not None)
@@ -952,12 +967,17 @@ def test_w4a16_packed_many_rows(m, k, n, gs, offset):
         w4_check(np.ascontiguousarray(y.cpu().numpy()[:, c0:c1]), np.ascontiguousarray(want), x)
 
 
-@pytest.mark.parametrize("m,k,n,gs", [(36, 4096, 1032, 64), (21, 1152, 3336, 128), (129, 1152, 1544, 32), (40, 1280, 3336, 128),
-                                       (60, 2176, 5128, 64), (85, 1408, 13320, 128), (5, 128, 8, 128), (17, 384, 24, 32)])
+W4_WHOLE_K = {(16, 16): [(36, 4096, 1032, 64), (12, 4224, 1032, 128)], (32, 16): [(21, 1152, 3336, 128), (5, 128, 8, 128), (17, 384, 24, 32)],
+              (32, 32): [(129, 1152, 1544, 32), (30, 1920, 5320, 128)], (64, 16): [(40, 1280, 3336, 128)],
+              (64, 32): [(60, 2176, 5128, 64), (40, 1280, 6504, 128)], (64, 64): [(100, 1152, 7208, 32), (85, 1152, 6920, 64), (80, 1152, 7400, 128)],
+              (): [(85, 1408, 13320, 128)]}  # (per weight 128 x 128, as group sums 64 x 64)
+
+
+@pytest.mark.parametrize("m,k,n,gs", [s for sizes in W4_WHOLE_K.values() for s in sizes])
 @pytest.mark.parametrize("offset", ["frac", None])
 @pytest.mark.parametrize("mode", [abi.W4A16_PER_WEIGHT, abi.W4A16_GROUP_SUM])
 def test_w4a16_packed_whole_k_tiles(m, k, n, gs, offset, mode):
-    """Rows and columns that leave the large tiles' chip idle: one case per tile of 16 x 16 to 64 x 64 (row and column tails, k that the
+    """Rows and columns that leave the large tiles' chip idle: every tile of 16 x 16 to 64 x 64 in both forms (row and column tails, k that the
     eight wavefronts cannot share evenly, a half-filled last stage), and calls shorter than the wavefronts' smallest share.
     (Groups that are no multiple of 128 run the per-weight form.)  Two calls give identical bits, past the last row nothing is written."""
     announce("w4a16 packed whole-k tiles", m, k, n, gs, offset, mode)
@@ -1024,11 +1044,15 @@ def test_w4a16_packed_rows_kernel_wide(m, k, n, gs, mode):
         w4_group_sum_gate(got, want) if mode == abi.W4A16_GROUP_SUM else w4_check(got, want, x)
 
 
-@pytest.mark.parametrize("m,k,n,gs", [(97, 128, 8, 32), (98, 384, 40, 128), (130, 256, 528, 64), (200, 640, 1032, 128)])
+W4_PACKED_FIRST = {"wq_rows_kernel": [(97, 128, 8, 32), (98, 384, 40, 128), (130, 256, 528, 64), (200, 640, 1032, 128)],
+                   "wq_gemm_kernel<128, 128, ": [(140, 256, 4104, 32), (300, 640, 5000, 128)]}
+
+
+@pytest.mark.parametrize("m,k,n,gs", [s for sizes in W4_PACKED_FIRST.values() for s in sizes])
 @pytest.mark.parametrize("offset", [True, False])
 def test_w4a16_many_rows_packs_the_weights_first(m, k, n, gs, offset):
-    """More than 96 rows on [k, n] weights: the call packs them into its workspace and runs the packed form's tile GEMM,
-    whose bits it has; a workspace that only holds the row kernels' pieces is still accepted."""
+    """More than 96 rows on [k, n] weights: the call packs them into its workspace and runs the packed form (whole-k tiles or tiles
+    of 128 x 128), whose bits it has; the workspace that a call of 32 rows asks for is accepted."""
     announce("w4a16 many rows", m, k, n, gs, offset)
     rng = np.random.default_rng(m + k + n)
     x, wp, sc, of = w4_case(rng, m, k, n, gs, offset)
@@ -1045,6 +1069,49 @@ def test_w4a16_many_rows_packs_the_weights_first(m, k, n, gs, offset):
     abi.check(abi.load_library().ascq_matmul_w4a16_workspace_size(C.byref(d), C.byref(need)))
     ops.matmul_w4a16(y, xd, wd, sd, od, gs, workspace=torch.zeros(max(need.value // 4, 4), dtype=torch.float32, device=DEV))
     w4_check(y.cpu().numpy(), want, x)
+
+
+# calls whose weights would be packed or turned round first, in a workspace that holds the passes' pieces (128 MiB) and not the weights
+SMALL_WORKSPACE = [("w4a16", 33, 8960, 32576), ("w4a16", 97, 3328, 80672), ("w8a16", 48, 8704, 15584), ("w8a16", 136, 8576, 15680)]
+
+
+def passes_workspace(kind, m, k, n):
+    """(bytes that the passes need, bytes that the call asks for)"""
+    lib, need = abi.load_library(), []
+    for rows in (4, m):                  # (4 rows run in passes)
+        size = C.c_size_t(0)
+        if kind == "w4a16":
+            abi.check(lib.ascq_matmul_w4a16_workspace_size(C.byref(abi.W4A16Desc(m=rows, n=n, k=k, group_size=128, has_offset=1)), C.byref(size)))
+        else:
+            abi.check(lib.ascq_matmul_w8a16_workspace_size(C.byref(abi.W8A16Desc(m=rows, n=n, k=k, has_offset=1, out_dtype=abi.F16)), C.byref(size)))
+        need.append(size.value)
+    return need
+
+
+@pytest.mark.parametrize("kind,m,k,n", SMALL_WORKSPACE)
+def test_half_matmul_in_a_workspace_too_small_for_the_weights(kind, m, k, n):
+    """Weights that are brought into another form first and, where the workspace has no room for that, passes over them as they are:
+    whole numbers (exact halves, exact fp32 sums), so both give the value itself."""
+    announce("small workspace", kind, m, k, n)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + k)
+    x = torch.randint(-4, 5, (m, k), device=DEV, generator=g).to(torch.float16)
+    w = torch.randint(-8, 8, (k, n), dtype=torch.int8, device=DEV, generator=g)
+    of = torch.randint(-3, 4, (n,), device=DEV, generator=g).to(torch.float16)
+    sc = torch.randint(1, 3, (n,), device=DEV, generator=g).to(torch.float16) * 0.5
+    want = torch.cat([x.double() @ ((w[:, c:c + 8192].double() + of[c:c + 8192].double()) * sc[c:c + 8192].double()) for c in range(0, n, 8192)], 1)
+    small, whole = passes_workspace(kind, m, k, n)
+    assert small < whole                 # sums of at most 2^23 halves: exact in fp32
+    for room in (whole, small):
+        y = torch.zeros((m, n), dtype=torch.float16, device=DEV)
+        ws = torch.empty(room // 4, dtype=torch.float32, device=DEV)
+        if kind == "w4a16":
+            nibbles = (w & 15).to(torch.uint8).view(k, n // 2, 2)
+            ops.matmul_w4a16(y, x, (nibbles[..., 0] | (nibbles[..., 1] << 4)).contiguous(), sc.expand(k // 128, n).contiguous(),
+                             of.expand(k // 128, n).contiguous(), 128, workspace=ws)
+        else:
+            ops.matmul_w8a16(y, x, w, of, sc, workspace=ws)
+        assert torch.equal(y, want.clamp(-65504, 65504).half()), room
 
 
 def config4_columns(m, n):
@@ -1299,13 +1366,17 @@ def test_w8a16_trans_b(m, k, n, mode):
                                                       None if per_tensor else sc)).view(np.uint8))
 
 
-@pytest.mark.parametrize("m,k,n", [(9, 8448, 1280), (28, 2176, 2573), (70, 3072, 1551), (100, 1152, 2055), (40, 2048, 5000), (300, 1152, 2059),
-                                   (85, 1152, 6913), (5, 128, 3), (16, 1664, 23264)])
+W8_WHOLE_K = {(16, 16): [(14, 8448, 1379)], (32, 16): [(28, 2176, 2573), (20, 768, 11)], (32, 32): [(30, 1920, 5317)],
+              (64, 16): [(70, 3072, 1551), (22, 128, 51)], (64, 32): [(100, 1152, 2055), (40, 2048, 5000)], (64, 64): [(300, 1152, 2059), (85, 1152, 6913)],
+              (): [(9, 8448, 1280), (5, 128, 3), (16, 1664, 23264)]}  # passes of 16 rows
+
+
+@pytest.mark.parametrize("m,k,n", [s for sizes in W8_WHOLE_K.values() for s in sizes])
 @pytest.mark.parametrize("mode", ["vector+offset", "scalar"])
 @pytest.mark.parametrize("out_f32", [True, False])
 def test_w8a16_trans_b_whole_k_tiles(m, k, n, mode, out_f32):
-    """Rows and columns that leave the large tiles' chip idle: one case per tile of 16 x 16 to 64 x 64, row and column tails (odd widths), k
-    that the eight wavefronts cannot share evenly or at all; the last case stays with the passes of 16 rows."""
+    """Rows and columns that leave the large tiles' chip idle: every tile of 16 x 16 to 64 x 64, row and column tails (odd widths), k
+    that the eight wavefronts cannot share evenly or at all; the last three stay with the passes of 16 rows."""
     announce("w8a16 [n, k] whole-k tiles", m, k, n, mode, out_f32)
     rng = np.random.default_rng(m * 7 + k + n)
     x = rng.standard_normal((m, k)).astype(np.float16)
@@ -1362,12 +1433,16 @@ def test_w8a16_few_rows_transposed_first(m, k, n, offset):
     assert torch.allclose(y0.float(), y1.float(), rtol=2.0 ** -10, atol=1e-3)
 
 
-@pytest.mark.parametrize("m,k,n", [(33, 128, 7), (128, 256, 248), (129, 384, 264), (257, 640, 521), (300, 128, 1034)])
+W8_MANY_ROWS = {"wq_rows_kernel": [(33, 128, 7), (128, 256, 248), (129, 384, 264), (257, 640, 521)],
+                "wq_gemm_kernel<128, 128, ": [(300, 128, 1034), (69, 128, 2307), (700, 384, 3001), (640, 640, 3080), (1030, 640, 2056)]}
+
+
+@pytest.mark.parametrize("m,k,n", [s for sizes in W8_MANY_ROWS.values() for s in sizes])
 @pytest.mark.parametrize("mode", ["vector+offset", "vector", "scalar+offset"])
 @pytest.mark.parametrize("out_f32", [False, True])
 def test_w8a16_trans_b_many_rows(m, k, n, mode, out_f32):
     """The half GEMM whose B-tile loader de-quantises [n, k] weights, on tiles of 128 x 128: two steps of k and more, row and
-    column tails, column counts that are no multiple of 4 (stored element by element) and of 2."""
+    column tails, column counts that are no multiple of 4 (stored element by element) and of 2; few rows or columns run whole-k tiles."""
     announce("w8a16 [n, k] many rows", m, k, n, mode, out_f32)
     rng = np.random.default_rng(m + k + n)
     x = rng.standard_normal((m, k)).astype(np.float16)
@@ -1418,12 +1493,18 @@ def test_half_gemm_on_tiles_of_256_columns(m, n, kind, k, offset):
         assert torch.equal(y, want.clamp(-65504, 65504).to(out) if out == torch.float16 else want)
 
 
-@pytest.mark.parametrize("kind,k", [("int8", 4224), ("int8", 4352), ("int8", 4416), ("int8", 4480), ("int4", 4224), ("int4", 4352), ("int4", 4480)])
+# m, n, kind, k: whether all loads of a step go out at once
+LOAD_RULE = {False: [(200, 8440, "int8", 3648), (200, 8440, "int8", 3712), (200, 8440, "int8", 3776), (200, 8440, "int4", 3712)],
+             True: [(200, 8440, "int8", 3840), (200, 8440, "int8", 3904), (200, 8440, "int8", 3968), (200, 8440, "int4", 3840)],
+             None: [(100, 14600, "int8", k) for k in (4224, 4352, 4416, 4480)] + [(100, 14600, "int4", k) for k in (4224, 4352, 4480)]}
+
+
+@pytest.mark.parametrize("m,n,kind,k", [s for sizes in LOAD_RULE.values() for s in sizes])
 @pytest.mark.parametrize("offset", [True, False])
-def test_half_gemm_on_both_sides_of_the_load_rule(kind, k, offset):
-    """115 tiles of 128 x 128: below 4348 of k each load of a step goes out behind a matrix instruction, from there on all at once; even
-    and odd numbers of K steps, exact sums as above."""
-    test_half_gemm_on_tiles_of_256_columns(100, 14600, kind, k, offset)
+def test_half_gemm_on_both_sides_of_the_load_rule(m, n, kind, k, offset):
+    """132 tiles of 128 x 128: below 3788 of k each load of a step goes out behind a matrix instruction, from there on all at once; even
+    and odd numbers of K steps, exact sums as above.  (100 rows run whole-k tiles of 64 x 64.)"""
+    test_half_gemm_on_tiles_of_256_columns(m, n, kind, k, offset)
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])

@@ -74,8 +74,8 @@ def test_mx_reference_example_shape(fa, fb, bias):
 @pytest.mark.parametrize("m,n,k", [(256, 256, 256), (64, 64, 1024), (300, 520, 512), (513, 272, 768), (1024, 256, 2048)])
 @pytest.mark.parametrize("fa,fb", [(E4, E4), (E4, E5), (E5, E4), (E5, E5), (F2, F2), (F1, F1), (F2, F1), (E4, F2), (F1, E5)])
 def test_mx_tile_kernel(m, n, k, fa, fb):
-    """Shapes that the tile kernel could take and the few-row kernel runs, on the scaled matrix instruction: every pair, row
-    and column tails, odd and even numbers of K steps."""
+    """Shapes that the tile kernel could take and the few-row kernel or ring tiles run, on the scaled matrix instruction: every
+    pair, row and column tails, odd and even numbers of K steps."""
     announce("mx tiles", m, n, k, fa, fb)
     rng = np.random.default_rng(m + n + k + fa * 16 + fb)
     a, b, sa, sb, _ = mx_case(rng, m, n, k, fa, fb)
@@ -129,13 +129,13 @@ def test_mx_ring_tiles(fa, fb, m, n, steps, more, out):
     """Tiles of 64 x 64, 128 x 64 and 128 x 128 (one size each): fewer K steps than LDS stages, odd and even numbers of them, the last fetch of
     16 scale bytes moved back inside the row and not, ragged rows and columns, every output type (16-bit ones in pairs and, odd n, one by
     one), a bias.  An e2m1 b beside an 8-bit a is taken as it is where k is a multiple of 256, widened otherwise.  All columns of
-    the rows at the tiles' ends; past the last row nothing is written."""
+    the rows at the tiles' ends; in a whole tile past the last row nothing is written."""
     k = steps * (256 if fa == fb == F2 else 128)
     sk = max(16, (k // 32 + 7) // 8 * 8) + more
     announce("mx ring tiles", fa, fb, m, n, k, sk, out)
     rng = np.random.default_rng(m + steps + fa * 16 + fb)
     a, b, sa, sb, bias = mx_case(rng, m, n, k, fa, fb, sk=sk, bias=True, lo=122, hi=133)
-    room = torch.zeros((m + 1) * n, dtype=out, device=DEV)
+    room = torch.zeros((m + 128) * n, dtype=out, device=DEV)
     c = room[:m * n].view(m, n)
     ops.matmul_mx(c, to_dev(a), to_dev(b), to_dev(sa), to_dev(sb), fa, fb, k, to_dev(bias))
     assert not room[m * n:].any()
@@ -150,6 +150,24 @@ def test_mx_ring_tiles(fa, fb, m, n, steps, more, out):
             want = np.clip(want, -65504.0, 65504.0)          # the reference's saturating cast
         eps = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[out]     # one rounding of the result
         assert np.all(np.abs(g - want) <= (1e-3 if is8(fa, fb) else 4e-6) * absdot + eps * np.abs(want) + 1e-7)
+
+
+RING_AND_TILES = {(64, 64): 131, (128, 64): 449, (128, 128): 1100}      # rows on each of the ring's tiles with 2344 columns
+
+
+@pytest.mark.parametrize("fa,fb", [(E4, E4), (E5, E4), (E5, E5), (F2, F2)])
+@pytest.mark.parametrize("steps", [1, 2, 5, 8])
+def test_mx_ring_tiles_have_the_bits_of_the_large_tiles(fa, fb, steps):
+    """4100 rows run 256 x 256 tiles, the first of them in a call of their own tiles with a ring of stages: the same instruction window
+    and order of the sums, so the same bits (8-bit products below the window are dropped; another window would show)."""
+    n, k = 2344, steps * (256 if fa == fb == F2 else 128)
+    announce("mx ring and tiles", fa, fb, k)
+    rng = np.random.default_rng(steps + fa * 16 + fb)
+    a, b, sa, sb, bias = mx_case(rng, 4100, n, k, fa, fb, sk=max(16, (k // 32 + 7) // 8 * 8), bias=True)
+    whole = run_mx(4100, n, k, a, b, sa, sb, fa, fb, bias=bias)
+    for m in RING_AND_TILES.values():
+        got = run_mx(m, n, k, a[:m], b, sa[:m], sb, fa, fb, bias=bias)
+        assert torch.equal(got.view(torch.int32), whole[:m].view(torch.int32)), m
 
 
 @pytest.mark.parametrize("m,n,k", [(8200, 1100, 128), (4100, 1128, 384), (4129, 1033, 640), (4096, 1056, 1024)])
@@ -273,7 +291,7 @@ def test_mx_few_rows_extreme_scales(fa, fb, m, k):
 def test_mx_tiles_store_every_row_length(f, out):
     """256 x 256 tiles with a last one of 52 rows and 63 columns or fewer: floats, 16-bit values in pairs, one by one (odd rows; an output
     that begins 2 bytes off a dword), every form the rounded bits of the float product's columns, which are compared with the
-    golden; past the last row nothing is written.  Large scales: halves saturate."""
+    golden; in a whole tile past the last row nothing is written.  Large scales: halves saturate."""
     m, k, more = 4148, 512, 2111
     announce("mx tile stores", f, out)
     rng = np.random.default_rng(f)
@@ -291,7 +309,7 @@ def test_mx_tiles_store_every_row_length(f, out):
         want = want.clamp(-65504.0, 65504.0)
     ad, bd, sad, sbd, bvd = to_dev(a), to_dev(b), to_dev(sa), to_dev(sb), to_dev(bv)
     for n, off in ((2111, 0), (2110, 0), (2110, 1), (2108, 0)):
-        buf = torch.full((off + (m + 1) * n,), 7.0, dtype=out, device=DEV)
+        buf = torch.full((off + (m + 256) * n,), 7.0, dtype=out, device=DEV)
         c = buf[off:off + m * n].view(m, n)
         ops.matmul_mx(c, ad, bd[:n], sad, sbd[:n], f, f, k, bvd[:n])
         assert torch.equal(c, want[:, :n].to(out)) and bool((buf[off + m * n:] == 7.0).all())

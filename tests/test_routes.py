@@ -1,6 +1,8 @@
 """The kernels that calls choose, without a GPU (tests/routes.py): the sizes at which a rule was measured keep the faster side."""
 import pytest
 
+import test_gpu_matmul as sizes
+import test_gpu_mx as mx_sizes
 from ascq import _abi as abi
 from routes import route
 
@@ -77,14 +79,14 @@ def test_antiquant_of_odd_widths_is_vectors_where_wide_and_many(dst, per_tensor,
             assert launch.name == ("antiquant_vec_kernel" if n >= 192 and rows * n >= elements else "antiquant_scalar_kernel"), (rows, n)
 
 
-def half_matmul(entry, m, k, n, **kw):
+def half_matmul(entry, m, k, n, room=1 << 35, **kw):
     x, w, scale, offset, ws = 1 << 30, 1 << 36, 1 << 38, 1 << 39, 1 << 40
     if entry == "ascq_matmul_w8a16":
         d = ("W8A16Desc", dict(m=m, n=n, k=k, has_offset=1, out_dtype=abi.F16, **kw))
-        return route(entry, d, 1 << 42, x, w, offset, scale, ws, 1 << 35, None)
+        return route(entry, d, 1 << 42, x, w, offset, scale, ws, room, None)
     d = ("W4A16Desc", dict(m=m, n=n, k=k, has_offset=1, **kw))
     if entry == "ascq_matmul_w4a16":
-        return route(entry, d, 1 << 42, x, w, scale, offset, ws, 1 << 35, None)
+        return route(entry, d, 1 << 42, x, w, scale, offset, ws, room, None)
     return route(entry, d, 1 << 42, x, w, scale, offset, None)
 
 
@@ -108,3 +110,120 @@ def test_int4_passes_of_few_rows_stay_where_they_are_ahead(m, k, n, packed):
 def test_packed_int4_in_many_groups_stays_in_passes_with_the_fewest_rows(m, k, n, group, passes):
     first, *_ = half_matmul("ascq_matmul_w4a16_packed", m, k, n, group_size=group)
     assert first.name == ("w4a16_packed_kernel" if passes else "wq_rows_kernel")
+
+
+# ---- the sizes of the GPU tests run the kernels that those tests name
+def each(groups):
+    return [(kernel, size) for kernel, members in groups.items() for size in members]
+
+
+@pytest.mark.parametrize("kernel,size", each(sizes.W4_MANY_ROWS))
+def test_packed_int4_tests_of_many_rows_run_the_tiles_they_name(kernel, size):
+    launch, = half_matmul("ascq_matmul_w4a16_packed", *size[:3], group_size=size[3])
+    assert launch.kernel.startswith(kernel)
+
+
+@pytest.mark.parametrize("kernel,size", each(sizes.W4_PACKED_FIRST))
+def test_int4_tests_of_many_rows_pack_and_run_the_tiles_they_name(kernel, size):
+    first, then = half_matmul("ascq_matmul_w4a16", *size[:3], group_size=size[3])
+    assert first.name == "pack_w4_tiles_kernel" and then.kernel.startswith(kernel)
+
+
+@pytest.mark.parametrize("kernel,size", each(sizes.W8_MANY_ROWS))
+def test_int8_tests_of_many_rows_run_the_tiles_they_name(kernel, size):
+    launch, = half_matmul("ascq_matmul_w8a16", *size, trans_b=1)
+    assert launch.kernel.startswith(kernel)
+
+
+@pytest.mark.parametrize("tile,size", each(sizes.W4_WHOLE_K))
+def test_int4_tests_of_whole_k_tiles_run_the_tiles_they_name(tile, size):
+    """wq_rows_kernel<rows, columns, kind, offset>: kind 0 int4 per weight, 1 group sums (groups of whole 128 k), 2 int8"""
+    for mode in (abi.W4A16_PER_WEIGHT, abi.W4A16_GROUP_SUM):
+        launch, = half_matmul("ascq_matmul_w4a16_packed", *size[:3], group_size=size[3], mode=mode)
+        kind = 1 if mode == abi.W4A16_GROUP_SUM and size[3] % 128 == 0 else 0
+        if not tile and kind == 0:
+            assert launch.kernel.startswith("wq_gemm_kernel<128, 128, ")
+        else:
+            assert launch.kernel.startswith("wq_rows_kernel<%d, %d, %d, " % ((tile or (64, 64)) + (kind,)))
+
+
+def test_int4_tests_of_whole_k_tiles_cover_every_tile_in_both_forms():
+    for per_weight in (True, False):
+        reached = {tile for tile, size in each(sizes.W4_WHOLE_K) if per_weight or size[3] % 128 == 0}
+        assert {(16, 16), (32, 16), (32, 32), (64, 16), (64, 32), (64, 64)} <= reached
+
+
+@pytest.mark.parametrize("tile,size", each(sizes.W8_WHOLE_K))
+def test_int8_tests_of_whole_k_tiles_run_the_tiles_they_name(tile, size):
+    first, *_ = half_matmul("ascq_matmul_w8a16", *size, trans_b=1)
+    assert first.kernel.startswith("wq_rows_kernel<%d, %d, 2, " % tile if tile else "w8a16_nk_kernel")
+
+
+@pytest.mark.parametrize("at_once,size", each(sizes.LOAD_RULE))
+def test_load_rule_tests_run_the_form_they_name(at_once, size):
+    m, n, kind, k = size
+    if kind == "int4":
+        last, = half_matmul("ascq_matmul_w4a16_packed", m, k, n, group_size=128)
+    else:
+        *_, last = half_matmul("ascq_matmul_w8a16", m, k, n, trans_b=int(k % 128 == 0))
+    if at_once is None:
+        assert last.kernel.startswith("wq_rows_kernel<64, 64, ")
+    else:
+        assert last.kernel.startswith("wq_gemm_kernel<128, 128, ") and last.args[4] == str(at_once).lower()
+
+
+@pytest.mark.parametrize("kind,m,k,n", sizes.SMALL_WORKSPACE)
+def test_workspaces_too_small_for_the_weights_run_passes(kind, m, k, n):
+    small, whole = sizes.passes_workspace(kind, m, k, n)
+    entry, kw = "ascq_matmul_" + kind, {"group_size": 128} if kind == "w4a16" else {}
+    for room, kernels in ((whole, {"pack_w4_tiles_kernel", "transpose_i8_kernel"}), (small, {"w4a16_tile_kernel", "w8a16_tile_kernel"})):
+        first, *_ = half_matmul(entry, m, k, n, room=room, **kw)
+        assert first.name in kernels
+
+
+def group_matmul(counts, k, n, nz=False, spare=0, out=abi.F16):
+    mm = dict(m=sum(counts) + spare, n=n, k=k, out_dtype=out, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32, has_tok_scale=1,
+              b_format=abi.MM_B_NZ if nz else abi.MM_B_ND)
+    d = ("GroupMatmulDesc", dict(mm=("MatmulDesc", mm), groups=len(counts), group_list_kind=abi.GROUP_LIST_COUNTS))
+    launch, = route("ascq_group_matmul_w8a8", d, 1 << 42, 1 << 30, 1 << 36, None, 1 << 38, 1 << 39, 1 << 40, None)
+    return launch
+
+
+@pytest.mark.parametrize("counts,long_k", sizes.GROUP_REMAINDERS)
+@pytest.mark.parametrize("nz", [False, True])
+def test_group_remainder_tests_cross_the_rule_that_names_the_instruction(counts, long_k, nz):
+    forms = {above: {group_matmul(counts, k, sizes.GROUP_WIDE, nz).kernel for k in (256, 384, 1280, 1408, 2432, 2560, 3072, 3200) if (k >= long_k) == above}
+             for above in (False, True)}
+    assert len(forms[False]) == len(forms[True]) == 1 and forms[False] != forms[True]
+    assert all(kernel.startswith("gemm_dma_group_kernel<") for kernel, in forms.values())
+    assert group_matmul(counts, 1408, 544, nz).name == "gemm_group_ring_kernel"
+
+
+@pytest.mark.parametrize("counts", sizes.GROUP_EDGES)
+def test_group_edge_tests_run_both_kernels(counts):
+    for n, kernel in ((520, "gemm_group_ring_kernel"), (sizes.GROUP_EDGES_WIDE, "gemm_dma_group_kernel")):
+        assert group_matmul(counts, 256, n, spare=8, out=abi.BF16).name == kernel
+
+
+def mx_matmul(m, n, k, fa, fb, scale_k, out=abi.F32):
+    d = ("MxDesc", dict(m=m, n=n, k=k, scale_k=scale_k, a_format=fa, b_format=fb, out_dtype=out, has_bias=0))
+    return route("ascq_matmul_mx", d, 1 << 42, 1 << 30, 1 << 33, 1 << 36, 1 << 37, None, 1 << 44, 1 << 40, None)[-1]
+
+
+@pytest.mark.parametrize("fa,fb", [(mx_sizes.E4, mx_sizes.E4), (mx_sizes.E5, mx_sizes.E4), (mx_sizes.E5, mx_sizes.E5), (mx_sizes.F2, mx_sizes.F2)])
+@pytest.mark.parametrize("steps", [1, 2, 5, 8])
+def test_mx_comparisons_of_ring_and_large_tiles_run_both(fa, fb, steps):
+    k = steps * (256 if fa == mx_sizes.F2 else 128)
+    scale_k = max(16, (k // 32 + 7) // 8 * 8)
+    assert mx_matmul(4100, 2344, k, fa, fb, scale_k).name == "mx_tile_kernel"
+    for tile, m in mx_sizes.RING_AND_TILES.items():
+        assert mx_matmul(m, 2344, k, fa, fb, scale_k).kernel.startswith("mx_ring_kernel<%d, %d, " % tile)
+
+
+# rows, columns: the tile of test_mx_ring_tiles (k is 128 or 256 times 1 to 17)
+@pytest.mark.parametrize("m,n,tile", [(131, 2801, (64, 64)), (449, 2530, (128, 64)), (700, 2999, (128, 128))])
+def test_mx_ring_tests_run_the_tiles_they_name(m, n, tile):
+    for fa, fb in ((mx_sizes.E4, mx_sizes.E5), (mx_sizes.F2, mx_sizes.F2)):
+        for steps in (1, 2, 3, 6, 9, 17):
+            k = steps * (256 if fa == mx_sizes.F2 else 128)
+            assert mx_matmul(m, n, k, fa, fb, max(16, (k // 32 + 7) // 8 * 8)).kernel.startswith("mx_ring_kernel<%d, %d, " % tile)
