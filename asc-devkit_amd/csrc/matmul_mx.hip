@@ -576,10 +576,11 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
     return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
 }
 
-// us that a call of the tiles' shapes is expected to take: in the kernel of matmul_mx_decode.hip, on 256 x 256 tiles, on the smaller ones of
+// Which kernel runs a call of the tiles' shapes: that of matmul_mx_decode.hip, the 256 x 256 tiles, or the smaller ones of
 // matmul_mx_ring.hip (and the best of their shapes).
+enum MxPath { kMxDecode, kMxTiles, kMxRing };
 struct MxPlan {
-    double decode, tiles, ring;
+    MxPath path;
     int shape;
 };
 
@@ -592,74 +593,80 @@ inline bool mx_ring_supported(const MxParams& p)
 }
 inline bool mx_ring_mixed(const MxParams& p) { return is_fp8(p.a_format) && p.b_format == ASCQ_QDST_FP4_E2M1 && p.k % 256u == 0; }
 
-// All are fits to 370 random calls of 64 to 4096 rows, k and n of 1024 to 14336 (ring tiles within 4 to 7 % for nine in ten, the others within 6
-// to 20 %).  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a meets 4-bit b) by 32 columns, each
-// with a part of its own and one per 1024 of k.  Tiles of 256 x 256: so much per round and per K step, which takes longer the more of the
-// chip has a tile, and the passes that widen 4-bit operands.  Ring: the same for each shape (tiles that share the chip with
-// few others wait less for memory).  Measured, in us, tiles, decode and the three ring shapes:
+// All are fits to random calls of 64 to 4096 rows, k and n of 256 to 14336 (370, the 4-bit operands widened or beside an 8-bit one 3800; half of
+// them within 4 %, nine in ten within 6 to 16 %).  Decode: rounds of workgroups (one per compute unit) of 64 rows (32 where 8-bit a
+// meets 4-bit b) by 32 columns, each with a part of its own and one per 1024 of k.  Tiles of 256 x 256: so much per round and per K step, which
+// takes longer the more of the chip has a tile.  Ring: the same for each shape (tiles that share the chip with few others wait less for
+// memory).  Widening 4-bit operands takes 1.7 us a launch and, for 0.25, 1, 3, 15 and 100 million values, about 0.3, 1, 3, 10 and 24 more.
+// Measured, in us, tiles, decode and the three ring shapes:
 //   e4m3 152 x 3680 x 2816   29.2, 15.6,  9.4, 10.8, 13.3      e2m1 378 x 2016 x 3584  21.6, 13.5,  7.7,  9.2, 11.9
 //   e4m3 441 x 4032 x 1792   26.9, 24.7, 13.2,  9.1, 10.5      e2m1 999 x 1856 x 3328  27.2, 26.0, 13.5,  9.7, 11.7
 //   e4m3 1370 x 2800 x 8448  89.2, 144, 77.5, 52.4, 39.0       e2m1 470 x 5888 x 11520 63.4, 74.6, 45.5, 41.4, 31.6
 //   e4m3 66 x 2512 x 7936    73.9, 15.4, 18.3, 21.3, 27.2      e2m1 64 x 4064 x 6912   35.3,  9.9, 10.5, 13.1, 18.1
 //   e4m3 3300 x 8192 x 1024  45.5, 236, 110, 70.7, 59.9        e4m3 x e2m1 507 x 6896 x 7936 104, 111, 54.7, 41.4, 31.1
+//   e1m2 x e2m1 2005 x 9032 x 256 25.6, 159, 53.9, 37.4, 29.7  e1m2 x e2m1 511 x 1228 x 8960 105, 32.5, 34.4, 38.6, 46.6
+//   e2m1 x e4m3 952 x 558 x 3328 39.0, 12.3, 14.9, 17.8, 20.4  e4m3 x e1m2 326 x 7783 x 2560 46.6, 57.8, 40.1, 35.7, 30.2
+// With a 4-bit a decode is taken up to 3 % behind the others' estimates, and the large tiles up to 4 % behind the ring's: where they are that
+// close, they were ahead.
 // Two e1m2 operands have constants of their own, fits to 500 random calls of 64 to 3000 rows (decode and tiles within 7 and 11 % for eight in ten): a
 // round of decode workgroups also takes 3.6 to start and store, a K step of tiles 0.6 and as much again as the chip fills up; rows of an odd number
 // of values are stored one by one, 16.5 a round (636 x 3729 x 1024 26.6 and 34.7, 636 x 3728 x 1024 26.1 and 17.6; 165 x
 // 12032 x 640 25.4 and 16.3; 874 x 2000 x 8960 75 and 63).
 MxPlan mx_plan(const MxParams& p)
 {
-    const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format);
+    const bool a8 = is_fp8(p.a_format), b8 = is_fp8(p.b_format), decode_ok = mx_decode_supported(p);
     const bool two4 = p.a_format == ASCQ_QDST_FP4_E2M1 && p.b_format == ASCQ_QDST_FP4_E2M1;
     const bool six = p.a_format == ASCQ_QDST_FP4_E1M2 && p.b_format == ASCQ_QDST_FP4_E1M2;
     const double cus = device_compute_units();
-    MxPlan plan{0.0, 0.0, 1e30, 0};
     auto rounds = [&](double blocks) { return __builtin_ceil(blocks / cus); };
     const uint32_t rows = a8 && !b8 ? 32u : 64u;
     const double decode_rounds = rounds(static_cast<double>((p.m + rows - 1u) / rows) * ((p.n + 31u) / 32u));
     const double blocks = static_cast<double>((p.m + kMxBM - 1u) / kMxBM) * ((p.n + kMxBN - 1u) / kMxBN);
     if (six) {
         const double filled = blocks < cus ? blocks / cus : 1.0, store = p.n % 2u != 0 ? 16.5 : 0.0;
-        plan.decode = 1.7 + decode_rounds * (1.73 * p.k / 1024.0 + 3.6);
-        plan.tiles = 11.9 + 0.137e-6 * (static_cast<double>(p.m) + p.n) * p.k + rounds(blocks) * (0.6 * (1.0 + filled) * p.k / 128.0 + store);
-        return plan;
+        const double decode = 1.7 + decode_rounds * (1.73 * p.k / 1024.0 + 3.6);
+        const double tiles = 11.9 + 0.137e-6 * (static_cast<double>(p.m) + p.n) * p.k + rounds(blocks) * (0.6 * (1.0 + filled) * p.k / 128.0 + store);
+        return MxPlan{decode_ok && decode < tiles ? kMxDecode : kMxTiles, 0};
     }
-    // 8-bit pairs; e2m1 pairs; 8-bit a with e2m1 b
     const bool mixed = mx_ring_mixed(p);
-    const int kind = two4 ? 1 : mixed ? 2 : 0;
     const double k1024 = p.k / 1024.0, steps = p.k / (two4 ? 256.0 : 128.0);
-    if (!a8 && !b8 && !two4) {  // e1m2 beside e2m1
-        plan.decode = 4.0 + decode_rounds * 2.0 * k1024;
-    } else {
-        static constexpr double kDecode[3][3] = {{1.3, 1.60, 2.9}, {1.6, 0.83, 3.2}, {1.6, 0.84, 2.3}};
-        const double* const c = kDecode[two4 ? 1 : a8 && !b8 ? 2 : 0];
-        plan.decode = c[0] + decode_rounds * (c[1] * k1024 + c[2]);
-    }
-    const double widen_a = two4 || a8 ? 0.0 : static_cast<double>(p.m) * p.k / 6e6, widen_b = two4 || b8 ? 0.0 : static_cast<double>(p.n) * p.k / 6e6;
-    const double widen = widen_a + widen_b == 0.0 ? 0.0 : 5.0 + 1.9 * (widen_a + widen_b), filled = blocks < cus ? blocks / cus : 1.0;
-    plan.tiles = 8.0 + widen + rounds(blocks) * steps * (1.08 + (two4 ? 0.91 : 0.5) * filled) + 9.0 * (rounds(blocks) - 1.0);
+    // 8-bit pairs; e2m1 pairs; 8-bit a with e2m1 and with e1m2; 4-bit a with 8-bit b; e1m2 beside e2m1
+    static constexpr double kDecode[6][3] = {{1.3, 1.60, 2.9}, {1.6, 0.83, 3.2}, {1.6, 0.84, 2.3}, {1.5, 0.99, 2.7}, {1.25, 1.30, 2.7}, {1.4, 1.13, 3.75}};
+    const double* const c = kDecode[two4 ? 1 : a8 && b8 ? 0 : a8 ? (p.b_format == ASCQ_QDST_FP4_E2M1 ? 2 : 3) : b8 ? 4 : 5];
+    const double decode = c[0] + decode_rounds * (c[1] * k1024 + c[2]);
+    const double wide = two4 ? 0.0 : 1e-6 * p.k * ((a8 ? 0.0 : static_cast<double>(p.m)) + (b8 ? 0.0 : static_cast<double>(p.n)));  // millions of values
+    const double widen = wide == 0.0 ? 0.0 : 1.7 * ((a8 ? 0 : 1) + (b8 ? 0 : 1)) + 12.0 * (1.0 - __builtin_exp(wide / -13.0)) + 0.125 * wide;
+    const double filled = blocks < cus ? blocks / cus : 1.0;
+    const double tiles = 8.0 + widen + rounds(blocks) * steps * (1.08 + (two4 ? 0.91 : 0.5) * filled) + 9.0 * (rounds(blocks) - 1.0);
+    double ring = 1e30;
+    int shape = 0;
     if (mx_ring_supported(p)) {
         struct Shape {
             uint32_t bm, bn;
             double start, step, fill, round;
         };
-        static constexpr Shape kShapes[3][3] = {
+        static constexpr Shape kShapes[3][3] = {  // 8-bit pairs; e2m1 pairs; 8-bit a with e2m1 b
             {{64, 64, 3.8, 0.225, 0.04, 2.2}, {128, 64, 4.1, 0.27, 0.085, 2.5}, {128, 128, 4.7, 0.357, 0.155, 4.0}},
             {{64, 64, 3.8, 0.23, 0.068, 2.1}, {128, 64, 4.2, 0.29, 0.15, 2.5}, {128, 128, 4.7, 0.47, 0.215, 3.2}},
             {{64, 64, 3.8, 0.27, 0.10, 2.1}, {128, 64, 4.1, 0.45, 0.16, 2.4}, {128, 128, 5.0, 0.70, 0.245, 3.7}}};
         const double ring_steps = mixed ? p.k / 256.0 : steps;
         for (int i = 0; i < 3; ++i) {
-            const Shape& s = kShapes[kind][i];
-            const double tiles = static_cast<double>((p.m + s.bm - 1u) / s.bm) * ((p.n + s.bn - 1u) / s.bn);
-            const double whole = __builtin_floor(tiles / cus), rest = tiles / cus - whole;
-            const double us = s.start + (mixed ? 0.0 : widen) + s.round * (rounds(tiles) - 1.0) +
+            const Shape& s = kShapes[two4 ? 1 : mixed ? 2 : 0][i];
+            const double n_tiles = static_cast<double>((p.m + s.bm - 1u) / s.bm) * ((p.n + s.bn - 1u) / s.bn);
+            const double whole = __builtin_floor(n_tiles / cus), rest = n_tiles / cus - whole;
+            const double us = s.start + (mixed ? 0.0 : widen) + s.round * (rounds(n_tiles) - 1.0) +
                               ring_steps * (whole * (s.step + s.fill) + (rest > 0.0 ? s.step + s.fill * rest : 0.0));
-            if (us < plan.ring) {
-                plan.ring = us;
-                plan.shape = i;
+            if (us < ring) {
+                ring = us;
+                shape = i;
             }
         }
     }
-    return plan;
+    const double near = a8 ? 1.0 : 1.03;
+    if (decode_ok && decode < near * tiles && decode < near * ring) {
+        return MxPlan{kMxDecode, 0};
+    }
+    return MxPlan{1.04 * ring < tiles ? kMxRing : kMxTiles, shape};
 }
 
 int mx_validate(const ascq_mx_desc* d, const char* who)
@@ -731,8 +738,8 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
     const bool tile = mx_tile_shape_ok(d) && aligned16(a) && aligned16(b) && (reinterpret_cast<uintptr_t>(a_scale) & 7u) == 0 &&
                       (reinterpret_cast<uintptr_t>(b_scale) & 7u) == 0 &&
                       (need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned16(workspace)));
-    const MxPlan plan = tile ? mx_plan(p) : MxPlan{};
-    if (mx_decode_supported(p) && (!tile || (plan.decode < plan.tiles && plan.decode < plan.ring))) {
+    const MxPlan plan = tile ? mx_plan(p) : MxPlan{mx_decode_supported(p) ? kMxDecode : kMxTiles, 0};
+    if (plan.path == kMxDecode) {
         return launch_mx_decode(p, tile, st);
     }
     if (!tile) {
@@ -757,7 +764,7 @@ extern "C" int ascq_matmul_mx(const ascq_mx_desc* d, void* c, const void* a, con
         ws += rows * d->k;
         fmt = ASCQ_QDST_FP8_E4M3FN;
     };
-    const bool ring = plan.ring < plan.tiles;
+    const bool ring = plan.path == kMxRing;
     if (wa) {
         widen(p.a, fa, d->m);
     }

@@ -227,3 +227,16 @@ def test_mx_ring_tests_run_the_tiles_they_name(m, n, tile):
         for steps in (1, 2, 3, 6, 9, 17):
             k = steps * (256 if fa == mx_sizes.F2 else 128)
             assert mx_matmul(m, n, k, fa, fb, max(16, (k // 32 + 7) // 8 * 8)).kernel.startswith("mx_ring_kernel<%d, %d, " % tile)
+
+
+E4, F2, F1 = mx_sizes.E4, mx_sizes.F2, mx_sizes.F1
+
+
+# measured ahead by 8 % to six times
+@pytest.mark.parametrize("m,n,k,fa,fb,kernel", [(2005, 9032, 256, F1, F2, "mx_tile_kernel"), (3682, 2820, 256, F2, F1, "mx_tile_kernel"),
+                                                (971, 6737, 256, F1, F2, "mx_tile_kernel"), (66, 8240, 12032, F2, F1, "mx_decode_kernel"),
+                                                (511, 1228, 8960, F1, F2, "mx_decode_kernel"), (230, 14080, 6912, F2, F1, "mx_ring_kernel"),
+                                                (952, 558, 3328, F2, E4, "mx_decode_kernel"), (1411, 400, 3584, F2, E4, "mx_decode_kernel"),
+                                                (326, 7783, 2560, E4, F1, "mx_ring_kernel")])
+def test_mx_pairs_with_a_widened_operand_run_the_kernel_that_is_ahead(m, n, k, fa, fb, kernel):
+    assert mx_matmul(m, n, k, fa, fb, max(16, (k // 32 + 7) // 8 * 8), abi.BF16).name == kernel
