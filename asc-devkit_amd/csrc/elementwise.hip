@@ -551,7 +551,8 @@ __global__ __launch_bounds__(kBlock) void dynq_row_kernel(int8_t* __restrict__ q
     }
 }
 
-// Rows of fewer than 8 or more than 16384 columns: two passes over the row (the second one hits in L2).
+// Rows of fewer than 8 or more than 16384 columns, and few narrow ones off the vectors' width or alignment: two passes over the row (the second
+// one hits in L2).
 template <int kSrc>
 __global__ __launch_bounds__(kThreads) void dynq_generic_kernel(int8_t* __restrict__ q, float* __restrict__ ts,
                                                                 const void* __restrict__ x, uint32_t n, uint32_t ldq)
@@ -595,7 +596,10 @@ int launch_dynq(uint32_t m, uint32_t n, void* q, uint32_t ldq, void* ts, const v
     int8_t* qq = static_cast<int8_t*>(q);
     float* tt = static_cast<float*>(ts);
     const bool vec = (n % 8 == 0) && (ldq % 8 == 0) && aligned16(x) && ((reinterpret_cast<uintptr_t>(q) & 7u) == 0);
-    if (n < 8 || n > 16384) {
+    // Off the vectors' width or alignment: from 192 columns on, or many rows (800 random calls; us, two passes and vectors: 378 x 35 2.17 and
+    // 2.36, 487 x 60 2.24 and 2.42, 63 x 181 level, 9 x 362 1.09 times as fast, 1500 x 128 1.09 times, 8192 x 11 1.1 times).
+    const bool wide = n >= 192 || m >= 4096 || (n >= 64 && m >= 1024);
+    if (n < 8 || n > 16384 || (!vec && !wide)) {
         dynq_generic_kernel<kSrc><<<m, kThreads, 0, st>>>(qq, tt, x, n, ldq);
     } else if (vec) {
         launch_dynq_row<kSrc, false>(m, n, qq, ldq, tt, x, st);

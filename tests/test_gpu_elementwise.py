@@ -830,6 +830,20 @@ def test_antiquant_of_odd_widths_off_the_vector_alignment(n, int4, dst_dt, has_o
     assert room[0] == 0 and not room[1 + k * n:].any()
 
 
+@pytest.mark.parametrize("m,n", [(1023, 65), (1024, 65), (1030, 191), (4095, 9), (4096, 9), (4101, 63)])
+@pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16, abi.F32])
+def test_dynamic_quantiser_of_narrow_odd_rows(m, n, src_dt):
+    """Both sides of the numbers of rows from which narrow rows of an odd width come as vectors, the outputs one byte past a boundary."""
+    announce("dynamic quant, narrow", m, n, src_dt)
+    x, xd = src_array(np.random.default_rng(m + n), (m, n), src_dt, 3.0)
+    room = torch.full((m * n + 16,), 55, dtype=torch.int8, device=DEV)
+    q, ts = room[1:1 + m * n].view(m, n), torch.empty(m, dtype=torch.float32, device=DEV)
+    ops.dynamic_quant_per_token(xd, q, ts)
+    wq, wts = orc.dynamic_quant_per_token(src_dt, x)
+    assert np.array_equal(q.cpu().numpy(), wq) and np.array_equal(ts.cpu().numpy(), wts)
+    assert room[0] == 55 and (room[1 + m * n:] == 55).all()
+
+
 @pytest.mark.parametrize("n", [7, 9, 1025, 2049, 4099, 8191, 16383, 16385])
 @pytest.mark.parametrize("src_dt", [abi.F16, abi.BF16, abi.F32])
 def test_rows_of_odd_widths_quantise_nan_to_zero(n, src_dt):

@@ -79,6 +79,21 @@ def test_antiquant_of_odd_widths_is_vectors_where_wide_and_many(dst, per_tensor,
             assert launch.name == ("antiquant_vec_kernel" if n >= 192 and rows * n >= elements else "antiquant_scalar_kernel"), (rows, n)
 
 
+@pytest.mark.parametrize("rows,n,kernel", [(378, 35, "dynq_generic_kernel"), (63, 191, "dynq_generic_kernel"), (1023, 191, "dynq_generic_kernel"),
+                                           (1, 193, "dynq_row_kernel"), (1024, 65, "dynq_row_kernel"), (1024, 63, "dynq_generic_kernel"),
+                                           (4095, 9, "dynq_generic_kernel"), (4096, 9, "dynq_row_kernel"), (5, 7, "dynq_generic_kernel"),
+                                           (5000, 7, "dynq_generic_kernel"), (3, 16383, "dynq_row_kernel"), (5000, 16385, "dynq_generic_kernel")])
+def test_dynamic_quantiser_of_odd_widths_is_vectors_where_wide_or_many(rows, n, kernel):
+    launch, = route("ascq_dynamic_quant_per_token", abi.BF16, rows, n, DST, SCALE, SRC, None)
+    assert launch.name == kernel
+
+
+def test_dynamic_quantiser_of_whole_vectors_off_their_alignment_is_as_odd_widths():
+    for n, at, kernel in ((40, DST, "dynq_row_kernel"), (40, DST + 1, "dynq_generic_kernel"), (192, DST + 1, "dynq_row_kernel")):
+        launch, = route("ascq_dynamic_quant_per_token", abi.F16, 67, n, at, SCALE, SRC, None)
+        assert launch.name == kernel
+
+
 def half_matmul(entry, m, k, n, room=1 << 35, **kw):
     x, w, scale, offset, ws = 1 << 30, 1 << 36, 1 << 38, 1 << 39, 1 << 40
     if entry == "ascq_matmul_w8a16":
