@@ -196,12 +196,17 @@ static bool gemm_group_ring_supported(const GemmParams& p)
 // the tiles of matmul_w8a8_group.hip are ahead, which start a tile with less to wait for.  In us there and with 64 x 64, 64 x 128 and
 // 128 x 128 tiles: 8 groups, 195 rows, k = 2688, n = 1536 25.9 and 12.6, 16.1, 19.0; 16, 30, 3712, 1824 29.8 and 25.4, 21.0, 23.4;
 // 4, 907, 1024, 2080 14.6 and 19.4, 18.1, 12.9; 8, 472, 2304, 6784 32.2 and 46.0, 43.9, 36.5; -1: none of them.
+// Nor do few rows of few groups with a short k take the 64 x 128 tiles, whose ring costs more to fill than they have to do (us there and
+// here, 560 random calls: 2 groups, 2 rows, k = 128, n = 8736 5.6 and 7.4; 2, 11, 768, 11520 7.6 and 9.0; 4, 7, 640, 4512 7.7 and 8.6;
+// ahead again 2, 61, 1024, 13536 12.3 and 11.0, with FasterGelu 4, 40, 512, 4384 8.8 and 7.8, and from 5 groups on).
 int gemm_group_ring_shape(const GemmParams& p)
 {
     static constexpr uint32_t kTile[3][2] = {{64, 64}, {64, 128}, {128, 128}};
     for (int i = 0; i < 3; ++i) {
         if (group_ring_tiles(p, kTile[i][0], kTile[i][1]) <= device_compute_units()) {
-            return gemm_group_ring_supported(p) ? i : -1;
+            const bool few = i == 1 && p.groups <= 4u && p.m <= 64u && p.k < (p.groups <= 2u ? 1024u : 704u) &&
+                             p.epi.activation != ASCQ_MM_ACT_FASTER_GELU;
+            return gemm_group_ring_supported(p) && !few ? i : -1;
         }
     }
     return -1;

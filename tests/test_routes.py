@@ -196,9 +196,9 @@ def test_workspaces_too_small_for_the_weights_run_passes(kind, m, k, n):
         assert first.name in kernels
 
 
-def group_matmul(counts, k, n, nz=False, spare=0, out=abi.F16):
+def group_matmul(counts, k, n, nz=False, spare=0, out=abi.F16, act=abi.MM_ACT_NONE):
     mm = dict(m=sum(counts) + spare, n=n, k=k, out_dtype=out, quant_mode=abi.MM_QUANT_VECTOR, scale_format=abi.MM_SCALE_F32, has_tok_scale=1,
-              b_format=abi.MM_B_NZ if nz else abi.MM_B_ND)
+              activation=act, act_beta=1.0, b_format=abi.MM_B_NZ if nz else abi.MM_B_ND)
     d = ("GroupMatmulDesc", dict(mm=("MatmulDesc", mm), groups=len(counts), group_list_kind=abi.GROUP_LIST_COUNTS))
     launch, = route("ascq_group_matmul_w8a8", d, 1 << 42, 1 << 30, 1 << 36, None, 1 << 38, 1 << 39, 1 << 40, None)
     return launch
@@ -255,3 +255,12 @@ E4, F2, F1 = mx_sizes.E4, mx_sizes.F2, mx_sizes.F1
                                                 (326, 7783, 2560, E4, F1, "mx_ring_kernel")])
 def test_mx_pairs_with_a_widened_operand_run_the_kernel_that_is_ahead(m, n, k, fa, fb, kernel):
     assert mx_matmul(m, n, k, fa, fb, max(16, (k // 32 + 7) // 8 * 8), abi.BF16).name == kernel
+
+
+@pytest.mark.parametrize("counts,k,n,act,ring", [([1, 1], 128, 8736, abi.MM_ACT_SWIGLU, False), ([9, 2], 768, 11520, abi.MM_ACT_SWIGLU, False),
+                                                 ([3, 1, 2, 1], 640, 4512, abi.MM_ACT_SWIGLU, False), ([18, 2], 384, 10912, abi.MM_ACT_NONE, False),
+                                                 ([35, 26], 1024, 13536, abi.MM_ACT_SWIGLU, True), ([20, 10, 6, 4], 512, 4384, abi.MM_ACT_FASTER_GELU, True),
+                                                 ([10] * 8, 256, 2272, abi.MM_ACT_NONE, True), ([93, 80, 60, 49], 640, 2944, abi.MM_ACT_NONE, True)])
+def test_few_rows_of_few_groups_with_a_short_k_stay_off_the_ring(counts, k, n, act, ring):
+    launch = group_matmul(counts, k, n, out=abi.BF16, act=act)
+    assert launch.kernel.startswith("gemm_group_ring_kernel<64, 128, " if ring else "gemm_dma_group_kernel<")
