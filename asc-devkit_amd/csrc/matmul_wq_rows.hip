@@ -393,7 +393,11 @@ bool wq_rows_ahead(const WqParams& p, bool int4, bool sum, bool has_offset, doub
     // 5 % ahead, or the two are as good as each other.  int8 with up to 10 rows: 13 %, since the estimate is up to as much below
     // what these tiles take there (11 of 170 random calls were slower than in passes: 5 x 4736 x 8064 12.5 us in passes, 14.8
     // here, estimates 13.6 and 12.7)
-    if (us > (!int4 && p.m <= 10u ? 0.87 : 0.95) * other_us) {
+    // int4 above 120 us: 15 %.  Many rounds of a full chip take up to a fifth longer than estimated (570 random calls, 12 of them slower
+    // than on the large tiles, one with this: 179 x 10880 x 29824 157 us there, 189 here, estimates 175 and 166; 427 x 11776 x 12624 166
+    // and 198).
+    const double ahead = !int4 && p.m <= 10u ? 0.87 : int4 && us > 120.0 ? 0.85 : 0.95;
+    if (us > ahead * other_us) {
         return false;
     }
     WqParams q = p;

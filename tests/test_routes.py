@@ -127,6 +127,13 @@ def test_packed_int4_in_many_groups_stays_in_passes_with_the_fewest_rows(m, k, n
     assert first.name == ("w4a16_packed_kernel" if passes else "wq_rows_kernel")
 
 
+@pytest.mark.parametrize("m,k,n,group,whole_k", [(179, 10880, 29824, 128, False), (427, 11776, 12624, 64, False), (316, 7040, 25960, 128, False),
+                                                 (513, 9088, 13920, 128, False), (216, 14080, 8960, 128, True), (141, 8064, 19472, 128, True)])
+def test_long_int4_calls_stay_on_the_large_tiles_where_those_are_ahead(m, k, n, group, whole_k):
+    launch, = half_matmul("ascq_matmul_w4a16_packed", m, k, n, group_size=group)
+    assert launch.name == ("wq_rows_kernel" if whole_k else "wq_gemm_kernel")
+
+
 # ---- the sizes of the GPU tests run the kernels that those tests name
 def each(groups):
     return [(kernel, size) for kernel, members in groups.items() for size in members]
