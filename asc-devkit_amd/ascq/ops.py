@@ -598,6 +598,10 @@ def matmul_w8a16(y, x, w, offset=None, scale=None, workspace=None, trans_b=False
     scale / offset: f16 tensors of n elements (SetAntiQuantVector) or Python floats (SetAntiQuantScalar); offset None =
     MatmulConfig::hasAntiQuantOffset false.  mode: abi.W8A16_CHANNEL_SUM applies scale and offset once per output to
     fp32 sums (up to 4 rows on [n, k] weights; elsewhere the per-weight form runs).
+
+    workspace None: scratch is kept per size and stream; on [k, n] weights up to 128 MiB, or k * n bytes where that is more and
+    the call turns the weights round first (above 96 rows, and from 17 on where that is faster).  A tensor of the size that
+    the query answers for up to 16 rows is accepted as well and keeps such a call on passes over the weights.
     """
     m, k = x.shape
     n = y.shape[1]

@@ -8,8 +8,9 @@
 // to 16 RT activation rows through a two-slot LDS ring of its own: direct-to-LDS loads, one batch in flight while the
 // other is computed, no barrier before the final sum.  The activations travel in the same queue: they are re-read by
 // every workgroup from the L2, m / (16 S) of the weights' bytes, which is why more rows are cut into blocks of 64
-// only up to a few hundred rows (mx_decode_preferred).  n = k = 8192, 16 rows, with one lane per output element before:
-// e2m1 4830 -> 8.9 us a call (4.0 TB/s; the caller's Python is as long as the kernel), e4m3 3870 -> 16.3 us, fp8
+// only up to a few hundred rows (mx_plan).  n = k = 8192, 16 rows, with one lane per output element before:
+// e2m1 4830 -> 8.8 us a call (4.1 TB/s: a wavefront's share is four batches and two are on their way, so a third is asked
+// for when the first has landed; 3 us less host time per call left it where it was), e4m3 3870 -> 16.3 us, fp8
 // activations on e2m1 weights 4415 -> 14.8 us; 64 rows on the 256 x 256 tiles before: e2m1 42.4 -> 13.0 us, e4m3 77 ->
 // 19.5 us.  32 columns per workgroup (S = 2) give every compute unit one at n = 8192; narrower matrices take 16 (a unit then
 // streams half the bytes: n = 1024, k = 14336, e4m3, 9 against 14 us).

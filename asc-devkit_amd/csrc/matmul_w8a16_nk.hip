@@ -562,7 +562,6 @@ int launch_w8a16_nk(const void* x, const void* w, const void* scale, const void*
                     uint32_t k, bool has_offset, bool out_f32, uint32_t scale_bits, uint32_t offset_bits, hipStream_t st,
                     bool channel_sum);
 
-// Weights given as [k, n] and many rows: transposed once into the caller's workspace (k * n bytes), then the tile GEMM.
 // us of passes of 16 rows (51 random calls, nine tenths within 15 %): a launch, and per 1024 k a time that grows with the columns
 static double passes_estimate(uint32_t m, uint32_t n, uint32_t k)
 {
@@ -602,6 +601,7 @@ bool w8a16_kn_gemm_supported(uint32_t m, uint32_t n, uint32_t k, const void* x, 
     return w8a16_kn_transposed(m, n, k) && aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0;
 }
 
+// Weights given as [k, n]: transposed once into the caller's workspace (k * n bytes), then the kernels of the [n, k] form.
 int launch_w8a16_kn_via_transpose(const void* x, const void* w, const void* scale, const void* offset, void* y,
                                   uint32_t m, uint32_t n, uint32_t k, bool has_offset, bool out_f32, uint32_t scale_bits,
                                   uint32_t offset_bits, void* workspace, hipStream_t st)

@@ -647,7 +647,8 @@ int ascq_matmul_w8a16_workspace_size(const ascq_w8a16_desc* desc, size_t* bytes)
  * with one lane per output element.
  * Accuracy: exact products and fp32 sums, about 1e-7 from 64 bits (2-norm), but for an fp8 operand in a call that the tiles
  * could take (64 rows and columns and more, the conditions above): there the scaled matrix instruction aligns the
- * products of an instruction to the largest and drops what lies 2^13 below it, which leaves up to 1.3e-5 (2-norm) and
+ * products of an instruction to the largest and drops what lies 2^13 below it, which leaves up to 1.3e-5 (2-norm of normally
+ * distributed values; 4.6e-5 of uniform codes) and
  * single results off by up to 2.3e-4 of their terms' magnitudes.
  * ref: include/basic_api/kernel_operator_mm_intf.h:321-340 (MmadMx), examples/01_simd_cpp_api/03_basic_api/
  *      03_matrix_compute/mmad_mx/README.md:5,131-152 and scripts/gen_data.py:52-140 (layouts, golden),
