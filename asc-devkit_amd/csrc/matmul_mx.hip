@@ -573,7 +573,10 @@ inline bool mx_tile_shape_ok(const ascq_mx_desc* d)
         mx_six_bytes(d->m, d->n, d->k) > (static_cast<uint64_t>(d->m) + d->n) * d->k) {
         return false;
     }
-    return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u;
+    // 32-bit offsets: of scale bytes from the first row, of operands from a tile's first row
+    const uint64_t rows = d->m > d->n ? d->m : d->n;
+    return d->k % (four ? 256u : 128u) == 0 && d->scale_k % 8u == 0 && d->scale_k >= 16u && d->m >= 64u && d->n >= 64u &&
+           rows * d->scale_k < (1ull << 32) && (four ? d->k / 2u : d->k) <= (1u << 24);
 }
 
 // Which kernel runs a call of the tiles' shapes: that of matmul_mx_decode.hip, the 256 x 256 tiles, or the smaller ones of

@@ -638,7 +638,7 @@ int ascq_matmul_w8a16_workspace_size(const ascq_w8a16_desc* desc, size_t* bytes)
  * product rounded to the output type, compared at rtol = atol = 1e-3.
  * a_format / b_format: ASCQ_QDST_FP8_E4M3FN | ASCQ_QDST_FP8_E5M2 | ASCQ_QDST_FP4_E2M1 | ASCQ_QDST_FP4_E1M2.
  * Two 8-bit operands, or two e2m1 operands, with k % 128 == 0 (8-bit) / k % 256 == 0 (4-bit), 16-byte aligned a, b and
- * scale_k % 8 == 0, scale_k >= 16 run the scaled matrix instruction on tiles of 64 x 64 to 256 x 256 straight from the given buffers
+ * scale_k % 8 == 0, scale_k >= 16 (max(m, n) * scale_k below 2^32, rows of up to 2^24 bytes) run the scaled matrix instruction on tiles of 64 x 64 to 256 x 256 straight from the given buffers
  * (as do an 8-bit a and an e2m1 b with k % 256 == 0 where the smaller tiles take the call).  Other format pairs first widen their 4-bit operands in the workspace (two e1m2 operands to 6-bit e2m3 codes, anything else
  * to e4m3; both exact).  Few rows (always below 64, up to a few hundred where an estimate says so) and shapes outside
  * the tiles' run a weight-streaming kernel that takes every format pair as it lies, needs no workspace (one that the size

@@ -271,3 +271,20 @@ def test_mx_pairs_with_a_widened_operand_run_the_kernel_that_is_ahead(m, n, k, f
 def test_few_rows_of_few_groups_with_a_short_k_stay_off_the_ring(counts, k, n, act, ring):
     launch = group_matmul(counts, k, n, out=abi.BF16, act=act)
     assert launch.kernel.startswith("gemm_group_ring_kernel<64, 128, " if ring else "gemm_dma_group_kernel<")
+
+
+@pytest.mark.parametrize("fa,fb", [(E4, E4), (F2, F2), (E4, F2), (F2, F1)])
+def test_mx_rows_whose_offsets_pass_32_bits_leave_the_tiles(fa, fb):
+    """The tiles and the ring address scale bytes by 32 bits from a's or b's first row, operands from a tile's; the few-row kernel by 64."""
+    for m, n in ((128, 3000), (3000, 128), (700, 2999), (4100, 2344)):
+        rows = max(m, n)
+        last = (2 ** 32 - 1) // rows // 8 * 8            # the longest scale rows (in eights) that 32 bits reach
+        assert mx_matmul(m, n, 1024, fa, fb, 64).name != "mx_elementwise_kernel"
+        assert mx_matmul(m, n, 1024, fa, fb, last).kernel == mx_matmul(m, n, 1024, fa, fb, 64).kernel
+        launch = mx_matmul(m, n, 1024, fa, fb, last + 8)
+        assert launch.name == "mx_decode_kernel"
+        if fa == E4 == fb:
+            assert launch.args[4] == "false"             # as for any shape that the tiles do not take
+    row = 1 << (25 if fa == fb == F2 else 24)            # values of a row of 2^24 bytes, the longest that 256 rows of 32-bit offsets hold
+    assert mx_matmul(64, 4000, row, fa, fb, row // 32).name == "mx_tile_kernel"
+    assert mx_matmul(64, 4000, row + 256, fa, fb, row // 32 + 8).name == "mx_elementwise_kernel"
