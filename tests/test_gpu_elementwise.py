@@ -758,7 +758,7 @@ def test_quantisers_of_odd_widths_off_the_vector_alignment(n, src_dt, elements):
     """Widths on both sides of the vector's 8 columns and of the row kernels' limits, inputs and outputs one element past a
     16-byte boundary; the bytes around the outputs stay as they are.  Few rows, and (wide ones) as many as the vectors take."""
     if elements and n < 1023:
-        pytest.skip("narrow rows run one element per lane in any number")
+        pytest.skip("narrow rows run one element per lane in any number (the dynamic quantiser: a test of its own)")
     m = max(13, -(-elements // n))
     announce("quant odd widths", n, src_dt, m)
     rng = np.random.default_rng(n)
